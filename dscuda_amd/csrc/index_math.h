@@ -442,5 +442,27 @@ DSCUDA_HOST_DEVICE inline DecodeLayout decode_layout(int batch, int heads, int s
     return layout;
 }
 
+// The same for the kernels that take 32 * row_blocks rows (heads) per workgroup: slots hold the real heads only, one
+// bf16 row of `rank` values plus two floats per head, rounded up to 16 bytes, and the compute units are shared by the
+// head groups.
+DSCUDA_HOST_DEVICE inline DecodeLayout narrow_decode_layout(int batch, int heads, int splits, int compute_units,
+                                                            int row_blocks, int rank) {
+    DecodeLayout layout;
+    const int rows_per_group = 32 * row_blocks;
+    layout.head_groups = (heads + rows_per_group - 1) / rows_per_group;
+    layout.slot_floats = ((long long)heads * (rank / 2 + 2) + 3) / 4 * 4;
+    const long long workspace = (long long)batch * heads * splits * (rank + 2);
+    const long long fixed = (long long)batch * layout.slot_floats + plan_elements(batch, 0);
+    long long cutting = workspace >= fixed ? (workspace - fixed) / (layout.slot_floats + 1) : 0;
+    const int most = compute_units > layout.head_groups ? compute_units / layout.head_groups : 1;
+    if (cutting > most) cutting = most;
+    layout.whole_sequences = (splits <= 1 || cutting < 2) ? 1 : 0;
+    layout.workgroups = layout.whole_sequences ? batch : (int)cutting;
+    layout.slots = layout.whole_sequences ? 0 : (long long)layout.workgroups + batch;
+    layout.plan_offset = layout.slots * layout.slot_floats;
+    layout.plan_ints = plan_elements(batch, layout.workgroups);
+    return layout;
+}
+
 }  // namespace index_math
 }  // namespace dscuda

@@ -1,0 +1,362 @@
+// The shared 576-wide latent key stream in units of 32 keys: where a unit lies in memory (paged, contiguous, or
+// latent and rope parts in tensors of their own), the global -> LDS requests that fetch it, and the fragment reads
+// of a unit in LDS.  Used by the absorbed decode and prefill-forward kernels.
+#pragma once
+
+#include "hip_common.h"
+#include "index_math.h"
+
+namespace dscuda {
+namespace {
+
+constexpr int RANK = 512;
+constexpr int ROPE = 64;
+constexpr int WIDTH = RANK + ROPE;
+constexpr int BN = 64;                      // keys per tile, the grain of the decode work list
+constexpr int CHUNKS = WIDTH / 8;           // 72 16-byte chunks per key row
+constexpr int ROW_BYTES = CHUNKS * 16;      // 1152
+
+constexpr int UNIT = 32;
+constexpr int UNIT_BYTES = UNIT * ROW_BYTES;              // 36 KB
+constexpr int UNIT_SLOTS = 4;
+constexpr int LOAD_WAVES = 4;                             // waves that share the requests of a unit
+constexpr int UNIT_LOADS = UNIT * CHUNKS / (64 * LOAD_WAVES);   // 9 wave instructions of 1 KB per wave and unit
+static_assert(UNIT_LOADS * 64 * LOAD_WAVES == UNIT * CHUNKS, "unit loads must divide evenly");
+
+__device__ __forceinline__ int swizzle_of_row(int row) {
+    return index_math::tile_swizzle<ROW_BYTES>(row);
+}
+
+__device__ __forceinline__ int tiles_of(int length) {
+    return (max(length, 0) + BN - 1) / BN;
+}
+
+struct KeyStream {
+    const bf16_t* latent;      // token t at latent + t*latent_stride, 512 wide
+    const bf16_t* rope;        // token t at rope + t*rope_stride, 64 wide
+    size_t latent_stride;
+    size_t rope_stride;
+    const int* block_table;    // nullptr: tokens are stored contiguously
+    int page_size;
+};
+
+struct UnitSource {
+    const bf16_t* base;      // first row of the unit (contiguous form; split form: of its latent part)
+    const bf16_t* rope_base; // split form: first row of the unit's rope part
+    unsigned lds_base;       // LDS byte offset of this wave's 9 KB of the unit's slot
+    int key0;
+    int row_limit;           // rows above it repeat it (>= 0: the unit holds a visible token)
+    bool contiguous;         // the unit is one run of rows: no paging, or pages that hold whole units
+    bool split;              // no paging, latent and rope parts in tensors of their own, offsets that fit 32 bits
+    bool full;               // all 32 rows are visible tokens: the per-lane offsets are the same for every such unit
+    bool enabled;
+};
+
+// Hands out the sources of consecutive units of one sequence.  The decode cache is packed
+// (576-wide rows), so only paging decides the form.  When pages hold whole units, the ids of
+// 64 consecutive pages of the sequence sit in one register (lane l: page first_page + l) and a
+// unit finds its page with one lane read: a scalar load per unit would have its wait drain the
+// LDS queue as well, in the middle of the fragment stream.
+struct UnitCursor {
+    int unit;                // the unit handed out next
+    int page;                // its page (index into the sequence's block table) ...
+    int within;              // ... and its place inside that page, in units
+    int units_per_page;
+    int first_page;          // page whose id lane 0 of `ids` holds
+    int last_page;           // last page of the sequence with a visible token: no entry past it is read
+    int ids;
+    bool paged;
+    bool contiguous;
+    bool split;
+
+    // Waits for the ids on the spot (the empty asm statement is their first use): a wait left to the
+    // first lane read would sit on the path of every step and wait for the unit requests as well.
+    __device__ __forceinline__ void load_ids(const KeyStream& keys, int from) {
+        first_page = from;
+        ids = keys.block_table[min(from + fresh_lane_id(), last_page)];
+        asm volatile("" : "+v"(ids));
+    }
+
+    __device__ __forceinline__ void init(const KeyStream& keys, int first_unit, int last_token) {
+        paged = keys.block_table != nullptr;
+        contiguous = !paged || (keys.page_size % UNIT == 0);
+        split = false;
+        unit = __builtin_amdgcn_readfirstlane(first_unit);
+        page = within = units_per_page = first_page = last_page = ids = 0;
+        if (paged && contiguous) {
+            units_per_page = __builtin_amdgcn_readfirstlane(keys.page_size / UNIT);
+            page = __builtin_amdgcn_readfirstlane(first_unit / units_per_page);
+            within = __builtin_amdgcn_readfirstlane(first_unit - page * units_per_page);
+            last_page = __builtin_amdgcn_readfirstlane(last_token / keys.page_size);
+            load_ids(keys, page);
+        }
+    }
+
+    __device__ __forceinline__ UnitSource next(unsigned char* lds, const KeyStream& keys, int last_token, int wave,
+                                               int unit_end) {
+        UnitSource source;
+        source.contiguous = contiguous;
+        source.split = split;
+        source.enabled = unit < unit_end;
+        source.key0 = unit * UNIT;
+        source.row_limit = last_token - source.key0;
+        source.full = source.row_limit >= UNIT - 1;
+        source.lds_base = __builtin_amdgcn_readfirstlane(lds_offset_of(lds) + ((unsigned)unit % UNIT_SLOTS) * UNIT_BYTES +
+                                                         wave * (UNIT_LOADS * 1024));
+        source.base = keys.latent;
+        source.rope_base = keys.rope;
+        if (split) {
+            source.base = keys.latent + (size_t)source.key0 * keys.latent_stride;
+            source.rope_base = keys.rope + (size_t)source.key0 * keys.rope_stride;
+        }
+        if (source.enabled && contiguous) {
+            long long physical = source.key0;
+            if (paged) {
+                // enabled: the unit holds a visible token, so page <= last_page
+                if (page - first_page >= 64) load_ids(keys, page);
+                const int id = __builtin_amdgcn_readlane(ids, page - first_page);
+                physical = (long long)id * keys.page_size + within * UNIT;
+            }
+            source.base = keys.latent + physical * WIDTH;
+        }
+        ++unit;
+        if (paged && contiguous && ++within == units_per_page) {
+            within = 0;
+            ++page;
+        }
+        return source;
+    }
+};
+
+// Per-lane offsets of the nine loads of a full unit (no row past the end of the sequence).
+struct FullUnitOffsets {
+    unsigned of[UNIT_LOADS];
+
+    __device__ __forceinline__ void init(int wave, int lane) {
+#pragma unroll
+        for (int i = 0; i < UNIT_LOADS; ++i) {
+            of[i] = index_math::contiguous_load_offset<ROW_BYTES, UNIT / 4>(wave, i, lane, UNIT - 1);
+        }
+    }
+};
+
+// Load number i (0..8) of a contiguous unit; i is a constant after unrolling.
+__device__ __forceinline__ void issue_unit_load(const UnitSource& source, const FullUnitOffsets& offsets, int wave, int i,
+                                                int lane) {
+    const unsigned offset = source.full
+        ? offsets.of[i]
+        : index_math::contiguous_load_offset<ROW_BYTES, UNIT / 4>(wave, i, lane, source.row_limit);
+    direct_load_16_offset_streaming(source.base, offset, source.lds_base + i * 1024);   // the cache is read once per call
+}
+
+// Load I of a unit whose latent and rope parts lie in tensors of their own, unpaged (`split`): a wave instruction
+// covers at most two rows of the unit (compile-time boundary), and a lane's 16 bytes come from the one tensor or the
+// other.  Row strides stay below 2^24 elements (the caller saw to that).
+template <int I>
+__device__ __forceinline__ void issue_split_load(const UnitSource& source, const KeyStream& keys, int wave, int lane) {
+    constexpr int FIRST_ROW = (64 * I) / CHUNKS;                 // of the wave's eight rows: the row of lane 0
+    constexpr int BOUNDARY = CHUNKS * (FIRST_ROW + 1) - 64 * I;   // first lane of the next row (64 or more: none)
+    // what depends on the row is the same for all lanes of a row: two candidates, wave-uniform
+    const int row = (UNIT / 4) * wave + FIRST_ROW;
+    const int swizzle[2] = {swizzle_of_row(row), swizzle_of_row(row + 1)};
+    const unsigned row_here[2] = {(unsigned)min(row, source.row_limit), (unsigned)min(row + 1, source.row_limit)};
+    const bool second = BOUNDARY < 64 && lane >= BOUNDARY;
+    const int position = lane + (64 * I - CHUNKS * FIRST_ROW) - (second ? CHUNKS : 0);
+    const int chunk = position ^ (second ? swizzle[1] : swizzle[0]);
+    const bool rope = chunk >= RANK / 8;
+    // bytes from the first row of the unit's part in the lane's tensor (the bases of the source hold key0 * stride)
+    const unsigned row_bytes = __umul24(second ? row_here[1] : row_here[0],
+                                        rope ? 2u * (unsigned)keys.rope_stride : 2u * (unsigned)keys.latent_stride);
+    const unsigned bytes = row_bytes + 16u * (unsigned)chunk - (rope ? 2u * RANK : 0u);
+    const unsigned char* part = reinterpret_cast<const unsigned char*>(rope ? source.rope_base : source.base);
+    direct_load_16(part + bytes, source.lds_base + I * 1024);
+}
+
+// All nine loads of a unit at once: the first units of a walk, and every unit of the
+// general form (per-lane page lookup, or latent and rope parts in tensors of their own).
+__device__ __forceinline__ void issue_unit(const UnitSource& source, const FullUnitOffsets& offsets, const KeyStream& keys,
+                                           int wave) {
+    if (!source.enabled) return;
+    const int lane = fresh_lane_id();
+    if (source.contiguous) {
+#pragma unroll
+        for (int i = 0; i < UNIT_LOADS; ++i) issue_unit_load(source, offsets, wave, i, lane);
+        return;
+    }
+    if (source.split) {
+        unrolled<0, UNIT_LOADS>([&](auto tag) { issue_split_load<decltype(tag)::value>(source, keys, wave, lane); });
+        return;
+    }
+    const bool paged = keys.block_table != nullptr;
+#pragma unroll 1
+    for (int i = 0; i < UNIT_LOADS; ++i) {
+        const int slot = 64 * i + lane;
+        const int row = (UNIT / 4) * wave + slot / CHUNKS;
+        const int chunk = (slot % CHUNKS) ^ swizzle_of_row(row);
+        const int token = source.key0 + min(row, source.row_limit);
+        long long physical = token;
+        if (paged) {
+            const int page = keys.block_table[token / keys.page_size];
+            physical = (long long)page * keys.page_size + token % keys.page_size;
+        }
+        const bf16_t* address = chunk < RANK / 8 ? keys.latent + physical * keys.latent_stride + 8 * chunk
+                                                 : keys.rope + physical * keys.rope_stride + 8 * (chunk - RANK / 8);
+        direct_load_16(address, source.lds_base + i * 1024);
+    }
+}
+
+// Per-lane byte offsets of the fragment reads inside a unit (rows 0..31 of 1152 bytes).
+// K operand: row lane%32, 16-byte chunk 2*ks + g at position (2*ks + g) ^ f(row); the XOR
+// only mixes the low three bits, so four offsets plus (ks/4)*128 reach every k-step.
+// V^T operand through transposing reads: in a block of 16 lanes, lane s points at row
+// 4*g + s/4 (+8 for the second read), columns 4*(s%4)..+3 of the 16-column group
+// 16*(block%2); bit 2 of f moves a row's data by one 64-byte column block, which two
+// offsets per read (even / odd column block) turn back into immediates.
+struct UnitReads {
+    unsigned k[4];
+    unsigned v_first[2];
+    unsigned v_second[2];
+
+    __device__ __forceinline__ void init(int lane) {
+        const int lq = lane % 32;
+        const int g = lane / 32;
+        const int swz = swizzle_of_row(lq);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) k[j] = lq * ROW_BYTES + ((2 * j + g) ^ swz) * 16;
+        const int s16 = lane % 16;
+        const int block = lane / 16;
+        const int row1 = 4 * g + s16 / 4;
+        const int f1 = swizzle_of_row(row1);
+        const int chunk_low = (2 * (block % 2) + (s16 % 4) / 2) ^ (f1 & 3);
+        const int flip = 64 * ((row1 >> 1) & 1);
+        const int lane1 = row1 * ROW_BYTES + chunk_low * 16 + 8 * (s16 & 1);
+        const int lane2 = (row1 + 8) * ROW_BYTES + (chunk_low ^ 1) * 16 + 8 * (s16 & 1);
+        v_first[0] = lane1 + flip;
+        v_first[1] = lane1 - flip;
+        v_second[0] = lane2 + flip;
+        v_second[1] = lane2 - flip;
+    }
+};
+
+typedef short unit_s16x4 __attribute__((ext_vector_type(4)));
+typedef short unit_s16x8 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) unit_s16x4* unit_tr_pointer;
+
+template <int KS>
+__device__ __forceinline__ bf16x8 unit_key_fragment(const unsigned char* unit, const UnitReads& reads) {
+    return *reinterpret_cast<const bf16x8*>(unit + reads.k[KS % 4] + (KS / 4) * 128);
+}
+
+// 16-key step N (0, 1) of the unit, column block D (0..15)
+template <int N, int D>
+__device__ __forceinline__ bf16x8 unit_value_fragment(const unsigned char* unit, const UnitReads& reads) {
+    constexpr int CONSTANT = N * 16 * ROW_BYTES + D * 64;
+    const unit_s16x4 low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((unit_tr_pointer)(unit + reads.v_first[D % 2] + CONSTANT));
+    const unit_s16x4 high = __builtin_amdgcn_ds_read_tr16_b64_v4i16((unit_tr_pointer)(unit + reads.v_second[D % 2] + CONSTANT));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(low, high, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+// ---- decode: a workgroup's range of the work list -----------------------------------------------------------------
+
+using index_math::PLAN_HEADER;
+using index_math::PLAN_OVERHEAD;
+using index_math::PLAN_RANGES;
+using index_math::PLAN_TOTAL;
+using index_math::PLAN_WHOLE;
+using index_math::PLAN_WORKGROUPS;
+
+constexpr int SELF_PLAN_BATCH = 256;   // sequences a workgroup turns into a plan by itself
+
+struct DecodeRange {
+    const int* prefix;   // positions before each sequence, in memory (the caller's plan) or in LDS
+    int overhead;
+    int begin, end;      // positions of this workgroup's range; begin >= end: nothing to do
+    int sequence;        // first sequence that reaches past `begin`
+};
+
+// The plan comes from memory (own_workgroups == 0: the caller's, or one mla_decode_plan_kernel has just built), or,
+// for a batch that one workgroup scans in one go, is worked out here by every workgroup for itself, which saves the
+// call a kernel launch; `leave_plan`: this workgroup then also writes what the merge kernel reads of it.  Called by
+// all threads of a workgroup of at least SELF_PLAN_BATCH threads; the three arrays are in LDS.
+__device__ __forceinline__ DecodeRange decode_range(int* plan, const int* cache_lengths, int batch_size, int own_workgroups,
+                                                    int own_whole, int* own_prefix, int* own_lengths, int* own_wave_totals,
+                                                    int tid, int workgroup, bool leave_plan) {
+    DecodeRange range;
+    int total, ranges;
+    bool whole_sequences;
+    if (own_workgroups > 0) {
+        whole_sequences = own_whole != 0;
+        range.overhead = whole_sequences ? 0 : index_math::SEGMENT_OVERHEAD;
+        int value = 0;
+        if (tid < SELF_PLAN_BATCH) {
+            const int own_length = tid < batch_size ? cache_lengths[tid] : 0;
+            own_lengths[tid] = own_length;
+            value = tid < batch_size ? index_math::positions_of(tiles_of(own_length), range.overhead) : 0;
+#pragma unroll
+            for (int offset = 1; offset < 64; offset <<= 1) {
+                const int other = __shfl_up(value, offset);
+                if (tid % 64 >= offset) value += other;
+            }
+            if (tid % 64 == 63) own_wave_totals[tid / 64] = value;
+            if (tid == 0) own_prefix[0] = 0;
+        }
+        __syncthreads();
+        if (tid < batch_size) {
+            int before = 0;
+#pragma unroll
+            for (int w = 0; w < SELF_PLAN_BATCH / 64; ++w) {
+                if (w < tid / 64) before += own_wave_totals[w];
+            }
+            own_prefix[tid + 1] = before + value;
+        }
+        __syncthreads();
+        // what comes out of LDS is the same in every lane, which the compiler cannot know
+        total = __builtin_amdgcn_readfirstlane(own_prefix[batch_size]);
+        ranges = index_math::ranges_of(total, own_workgroups);
+        range.prefix = own_prefix;
+        if (leave_plan) {
+            if (tid == 0) {
+                plan[PLAN_TOTAL] = total;
+                plan[PLAN_WORKGROUPS] = own_workgroups;
+                plan[PLAN_OVERHEAD] = range.overhead;
+                plan[PLAN_WHOLE] = own_whole;
+                plan[PLAN_RANGES] = ranges;
+            }
+            if (tid <= batch_size) plan[index_math::plan_prefix_at() + tid] = own_prefix[tid];
+        }
+    } else {
+        total = plan[PLAN_TOTAL];
+        range.overhead = plan[PLAN_OVERHEAD];
+        whole_sequences = plan[PLAN_WHOLE] != 0;
+        ranges = plan[PLAN_RANGES];
+        range.prefix = plan + index_math::plan_prefix_at();
+    }
+
+    range.sequence = 0;
+    if (whole_sequences) {
+        range.begin = __builtin_amdgcn_readfirstlane(range.prefix[workgroup]);
+        range.end = __builtin_amdgcn_readfirstlane(range.prefix[workgroup + 1]);
+    } else {
+        range.begin = range.end = 0;
+        if (workgroup >= ranges) return range;
+        range.begin = index_math::range_begin_of(total, ranges, workgroup);
+        range.end = index_math::range_begin_of(total, ranges, workgroup + 1);
+    }
+    if (range.begin >= range.end) return range;
+    if (own_workgroups > 0 && !whole_sequences) {
+        int low = 0, high = batch_size;
+        while (low < high) {
+            const int mid = (low + high) / 2;
+            if (__builtin_amdgcn_readfirstlane(range.prefix[mid + 1]) <= range.begin) low = mid + 1; else high = mid;
+        }
+        range.sequence = low;
+    } else if (own_workgroups > 0) {
+        range.sequence = workgroup;
+    } else {
+        range.sequence = plan[index_math::plan_first_sequence_at(batch_size) + workgroup];
+    }
+    return range;
+}
+
+}  // namespace
+}  // namespace dscuda

@@ -51,6 +51,7 @@
 #include "attn_kernels.h"
 #include "hip_common.h"
 #include "index_math.h"
+#include "latent_stream.h"
 
 #include <algorithm>
 #include <cstdint>
@@ -60,36 +61,15 @@
 namespace dscuda {
 namespace {
 
-constexpr int RANK = 512;
-constexpr int ROPE = 64;
-constexpr int WIDTH = RANK + ROPE;
-constexpr int BN = 64;                      // keys per tile, the grain of the decode work list
 constexpr int ROWS = 128;                   // rows per workgroup
-constexpr int THREADS = 256;
-constexpr int CHUNKS = WIDTH / 8;           // 72 16-byte chunks per key row
-constexpr int ROW_BYTES = CHUNKS * 16;      // 1152
+constexpr int THREADS = 64 * LOAD_WAVES;
 constexpr int KSTEPS = WIDTH / 16;          // 36
 constexpr int DBLOCKS = RANK / 32;          // 16
 constexpr int EPILOGUE_PITCH = 1024 + 16;   // bytes per staged output row
 
-typedef const __attribute__((address_space(1))) void* global_pointer;
-
-__device__ __forceinline__ int swizzle_of_row(int row) {
-    return index_math::tile_swizzle<ROW_BYTES>(row);
-}
-
 __device__ __forceinline__ float uniform(float value) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, value)));
 }
-
-struct KeyStream {
-    const bf16_t* latent;      // token t at latent + t*latent_stride, 512 wide
-    const bf16_t* rope;        // token t at rope + t*rope_stride, 64 wide
-    size_t latent_stride;
-    size_t rope_stride;
-    const int* block_table;    // nullptr: tokens are stored contiguously
-    int page_size;
-};
 
 // Score-chain MFMAs with the accumulator held in ordinary vector registers.
 // The compiler's own MFMAs take accumulator-file destinations in a kernel this
@@ -253,228 +233,7 @@ __device__ __forceinline__ void reset(RowState& state) {
 // of the sequence repeat the last valid row and their scores are masked, so nothing
 // has to be cleared.
 
-constexpr int UNIT = 32;
-constexpr int UNIT_BYTES = UNIT * ROW_BYTES;              // 36 KB
-constexpr int UNIT_SLOTS = 4;
-constexpr int UNIT_LOADS = UNIT * CHUNKS / THREADS;       // 9 wave instructions of 1 KB per wave and unit
 constexpr int STREAM_RING = 6;                            // fragments read ahead of the MFMA that takes them
-static_assert(UNIT_LOADS * THREADS == UNIT * CHUNKS, "unit loads must divide evenly");
-
-struct UnitSource {
-    const bf16_t* base;      // first row of the unit (contiguous form; split form: of its latent part)
-    const bf16_t* rope_base; // split form: first row of the unit's rope part
-    unsigned lds_base;       // LDS byte offset of this wave's 9 KB of the unit's slot
-    int key0;
-    int row_limit;           // rows above it repeat it (>= 0: the unit holds a visible token)
-    bool contiguous;         // the unit is one run of rows: no paging, or pages that hold whole units
-    bool split;              // no paging, latent and rope parts in tensors of their own, offsets that fit 32 bits
-    bool full;               // all 32 rows are visible tokens: the per-lane offsets are the same for every such unit
-    bool enabled;
-};
-
-// Hands out the sources of consecutive units of one sequence.  The decode cache is packed
-// (576-wide rows), so only paging decides the form.  When pages hold whole units, the ids of
-// 64 consecutive pages of the sequence sit in one register (lane l: page first_page + l) and a
-// unit finds its page with one lane read: a scalar load per unit would have its wait drain the
-// LDS queue as well, in the middle of the fragment stream.
-struct UnitCursor {
-    int unit;                // the unit handed out next
-    int page;                // its page (index into the sequence's block table) ...
-    int within;              // ... and its place inside that page, in units
-    int units_per_page;
-    int first_page;          // page whose id lane 0 of `ids` holds
-    int last_page;           // last page of the sequence with a visible token: no entry past it is read
-    int ids;
-    bool paged;
-    bool contiguous;
-    bool split;
-
-    // Waits for the ids on the spot (the empty asm statement is their first use): a wait left to the
-    // first lane read would sit on the path of every step and wait for the unit requests as well.
-    __device__ __forceinline__ void load_ids(const KeyStream& keys, int from) {
-        first_page = from;
-        ids = keys.block_table[min(from + fresh_lane_id(), last_page)];
-        asm volatile("" : "+v"(ids));
-    }
-
-    __device__ __forceinline__ void init(const KeyStream& keys, int first_unit, int last_token) {
-        paged = keys.block_table != nullptr;
-        contiguous = !paged || (keys.page_size % UNIT == 0);
-        split = false;
-        unit = __builtin_amdgcn_readfirstlane(first_unit);
-        page = within = units_per_page = first_page = last_page = ids = 0;
-        if (paged && contiguous) {
-            units_per_page = __builtin_amdgcn_readfirstlane(keys.page_size / UNIT);
-            page = __builtin_amdgcn_readfirstlane(first_unit / units_per_page);
-            within = __builtin_amdgcn_readfirstlane(first_unit - page * units_per_page);
-            last_page = __builtin_amdgcn_readfirstlane(last_token / keys.page_size);
-            load_ids(keys, page);
-        }
-    }
-
-    __device__ __forceinline__ UnitSource next(unsigned char* lds, const KeyStream& keys, int last_token, int wave,
-                                               int unit_end) {
-        UnitSource source;
-        source.contiguous = contiguous;
-        source.split = split;
-        source.enabled = unit < unit_end;
-        source.key0 = unit * UNIT;
-        source.row_limit = last_token - source.key0;
-        source.full = source.row_limit >= UNIT - 1;
-        source.lds_base = __builtin_amdgcn_readfirstlane(lds_offset_of(lds) + ((unsigned)unit % UNIT_SLOTS) * UNIT_BYTES +
-                                                         wave * (UNIT_LOADS * 1024));
-        source.base = keys.latent;
-        source.rope_base = keys.rope;
-        if (split) {
-            source.base = keys.latent + (size_t)source.key0 * keys.latent_stride;
-            source.rope_base = keys.rope + (size_t)source.key0 * keys.rope_stride;
-        }
-        if (source.enabled && contiguous) {
-            long long physical = source.key0;
-            if (paged) {
-                // enabled: the unit holds a visible token, so page <= last_page
-                if (page - first_page >= 64) load_ids(keys, page);
-                const int id = __builtin_amdgcn_readlane(ids, page - first_page);
-                physical = (long long)id * keys.page_size + within * UNIT;
-            }
-            source.base = keys.latent + physical * WIDTH;
-        }
-        ++unit;
-        if (paged && contiguous && ++within == units_per_page) {
-            within = 0;
-            ++page;
-        }
-        return source;
-    }
-};
-
-// Per-lane offsets of the nine loads of a full unit (no row past the end of the sequence).
-struct FullUnitOffsets {
-    unsigned of[UNIT_LOADS];
-
-    __device__ __forceinline__ void init(int wave, int lane) {
-#pragma unroll
-        for (int i = 0; i < UNIT_LOADS; ++i) {
-            of[i] = index_math::contiguous_load_offset<ROW_BYTES, UNIT / 4>(wave, i, lane, UNIT - 1);
-        }
-    }
-};
-
-// Load number i (0..8) of a contiguous unit; i is a constant after unrolling.
-__device__ __forceinline__ void issue_unit_load(const UnitSource& source, const FullUnitOffsets& offsets, int wave, int i,
-                                                int lane) {
-    const unsigned offset = source.full
-        ? offsets.of[i]
-        : index_math::contiguous_load_offset<ROW_BYTES, UNIT / 4>(wave, i, lane, source.row_limit);
-    direct_load_16_offset_streaming(source.base, offset, source.lds_base + i * 1024);   // the cache is read once per call
-}
-
-// Load I of a unit whose latent and rope parts lie in tensors of their own, unpaged (`split`): a wave instruction
-// covers at most two rows of the unit (compile-time boundary), and a lane's 16 bytes come from the one tensor or the
-// other.  Row strides stay below 2^24 elements (the caller saw to that).
-template <int I>
-__device__ __forceinline__ void issue_split_load(const UnitSource& source, const KeyStream& keys, int wave, int lane) {
-    constexpr int FIRST_ROW = (64 * I) / CHUNKS;                 // of the wave's eight rows: the row of lane 0
-    constexpr int BOUNDARY = CHUNKS * (FIRST_ROW + 1) - 64 * I;   // first lane of the next row (64 or more: none)
-    // what depends on the row is the same for all lanes of a row: two candidates, wave-uniform
-    const int row = (UNIT / 4) * wave + FIRST_ROW;
-    const int swizzle[2] = {swizzle_of_row(row), swizzle_of_row(row + 1)};
-    const unsigned row_here[2] = {(unsigned)min(row, source.row_limit), (unsigned)min(row + 1, source.row_limit)};
-    const bool second = BOUNDARY < 64 && lane >= BOUNDARY;
-    const int position = lane + (64 * I - CHUNKS * FIRST_ROW) - (second ? CHUNKS : 0);
-    const int chunk = position ^ (second ? swizzle[1] : swizzle[0]);
-    const bool rope = chunk >= RANK / 8;
-    // bytes from the first row of the unit's part in the lane's tensor (the bases of the source hold key0 * stride)
-    const unsigned row_bytes = __umul24(second ? row_here[1] : row_here[0],
-                                        rope ? 2u * (unsigned)keys.rope_stride : 2u * (unsigned)keys.latent_stride);
-    const unsigned bytes = row_bytes + 16u * (unsigned)chunk - (rope ? 2u * RANK : 0u);
-    const unsigned char* part = reinterpret_cast<const unsigned char*>(rope ? source.rope_base : source.base);
-    direct_load_16(part + bytes, source.lds_base + I * 1024);
-}
-
-// All nine loads of a unit at once: the first units of a walk, and every unit of the
-// general form (per-lane page lookup, or latent and rope parts in tensors of their own).
-__device__ __forceinline__ void issue_unit(const UnitSource& source, const FullUnitOffsets& offsets, const KeyStream& keys,
-                                           int wave) {
-    if (!source.enabled) return;
-    const int lane = fresh_lane_id();
-    if (source.contiguous) {
-#pragma unroll
-        for (int i = 0; i < UNIT_LOADS; ++i) issue_unit_load(source, offsets, wave, i, lane);
-        return;
-    }
-    if (source.split) {
-        unrolled<0, UNIT_LOADS>([&](auto tag) { issue_split_load<decltype(tag)::value>(source, keys, wave, lane); });
-        return;
-    }
-    const bool paged = keys.block_table != nullptr;
-#pragma unroll 1
-    for (int i = 0; i < UNIT_LOADS; ++i) {
-        const int slot = 64 * i + lane;
-        const int row = (UNIT / 4) * wave + slot / CHUNKS;
-        const int chunk = (slot % CHUNKS) ^ swizzle_of_row(row);
-        const int token = source.key0 + min(row, source.row_limit);
-        long long physical = token;
-        if (paged) {
-            const int page = keys.block_table[token / keys.page_size];
-            physical = (long long)page * keys.page_size + token % keys.page_size;
-        }
-        const bf16_t* address = chunk < RANK / 8 ? keys.latent + physical * keys.latent_stride + 8 * chunk
-                                                 : keys.rope + physical * keys.rope_stride + 8 * (chunk - RANK / 8);
-        direct_load_16(address, source.lds_base + i * 1024);
-    }
-}
-
-// Per-lane byte offsets of the fragment reads inside a unit (rows 0..31 of 1152 bytes).
-// K operand: row lane%32, 16-byte chunk 2*ks + g at position (2*ks + g) ^ f(row); the XOR
-// only mixes the low three bits, so four offsets plus (ks/4)*128 reach every k-step.
-// V^T operand through transposing reads: in a block of 16 lanes, lane s points at row
-// 4*g + s/4 (+8 for the second read), columns 4*(s%4)..+3 of the 16-column group
-// 16*(block%2); bit 2 of f moves a row's data by one 64-byte column block, which two
-// offsets per read (even / odd column block) turn back into immediates.
-struct UnitReads {
-    unsigned k[4];
-    unsigned v_first[2];
-    unsigned v_second[2];
-
-    __device__ __forceinline__ void init(int lane) {
-        const int lq = lane % 32;
-        const int g = lane / 32;
-        const int swz = swizzle_of_row(lq);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) k[j] = lq * ROW_BYTES + ((2 * j + g) ^ swz) * 16;
-        const int s16 = lane % 16;
-        const int block = lane / 16;
-        const int row1 = 4 * g + s16 / 4;
-        const int f1 = swizzle_of_row(row1);
-        const int chunk_low = (2 * (block % 2) + (s16 % 4) / 2) ^ (f1 & 3);
-        const int flip = 64 * ((row1 >> 1) & 1);
-        const int lane1 = row1 * ROW_BYTES + chunk_low * 16 + 8 * (s16 & 1);
-        const int lane2 = (row1 + 8) * ROW_BYTES + (chunk_low ^ 1) * 16 + 8 * (s16 & 1);
-        v_first[0] = lane1 + flip;
-        v_first[1] = lane1 - flip;
-        v_second[0] = lane2 + flip;
-        v_second[1] = lane2 - flip;
-    }
-};
-
-typedef short unit_s16x4 __attribute__((ext_vector_type(4)));
-typedef short unit_s16x8 __attribute__((ext_vector_type(8)));
-typedef __attribute__((address_space(3))) unit_s16x4* unit_tr_pointer;
-
-template <int KS>
-__device__ __forceinline__ bf16x8 unit_key_fragment(const unsigned char* unit, const UnitReads& reads) {
-    return *reinterpret_cast<const bf16x8*>(unit + reads.k[KS % 4] + (KS / 4) * 128);
-}
-
-// 16-key step N (0, 1) of the unit, column block D (0..15)
-template <int N, int D>
-__device__ __forceinline__ bf16x8 unit_value_fragment(const unsigned char* unit, const UnitReads& reads) {
-    constexpr int CONSTANT = N * 16 * ROW_BYTES + D * 64;
-    const unit_s16x4 low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((unit_tr_pointer)(unit + reads.v_first[D % 2] + CONSTANT));
-    const unit_s16x4 high = __builtin_amdgcn_ds_read_tr16_b64_v4i16((unit_tr_pointer)(unit + reads.v_second[D % 2] + CONSTANT));
-    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(low, high, 0, 1, 2, 3, 4, 5, 6, 7));
-}
 
 // Scores of the unit at `unit` into `scores`, nothing overlapped (the first unit of a walk).
 __device__ __forceinline__ void unit_scores(f32x16& scores, const bf16x8 (&qf)[KSTEPS], const unsigned char* unit,
@@ -716,20 +475,9 @@ __device__ __forceinline__ void walk_units(RowState& state, const bf16_t* query_
     workgroup_barrier();   // the slots are free: the caller stages its results through them
 }
 
-__device__ __forceinline__ int tiles_of(int length) {
-    return (max(length, 0) + BN - 1) / BN;
-}
-
 // ----------------------------------------------------------------------------
 // decode
 // ----------------------------------------------------------------------------
-
-using index_math::PLAN_HEADER;
-using index_math::PLAN_OVERHEAD;
-using index_math::PLAN_RANGES;
-using index_math::PLAN_TOTAL;
-using index_math::PLAN_WHOLE;
-using index_math::PLAN_WORKGROUPS;
 
 // One workgroup turns the lengths into the plan (index_math.h): the prefix of positions
 // (tiles plus the per-sequence overhead when sequences are cut), the first sequence of
@@ -799,8 +547,6 @@ __global__ __launch_bounds__(THREADS) void mla_decode_plan_kernel(int* __restric
     }
 }
 
-constexpr int SELF_PLAN_BATCH = THREADS;   // sequences a workgroup turns into a plan by itself
-
 // The decode kernel: every workgroup walks its range of the work list (see index_math.h).
 //
 // Workspace: slot workgroup + sequence holds, for a segment that is only part of its
@@ -830,80 +576,12 @@ __global__ __launch_bounds__(THREADS) void mla_decode_split_kernel(
     const int head0 = head_group * ROWS;
     const float c = uniform(scale * LOG2E);
 
-    // The plan: read from memory (own_workgroups == 0: the caller's, or one mla_decode_plan_kernel has just built),
-    // or, for a batch that one workgroup scans in one go, worked out here by every workgroup for itself, which
-    // saves the call a kernel launch.  The first workgroup then also leaves what the merge kernel reads of it.
-    int total, overhead, ranges;
-    bool whole_sequences;
-    const int* prefix;
-    if (own_workgroups > 0) {
-        whole_sequences = own_whole != 0;
-        overhead = whole_sequences ? 0 : index_math::SEGMENT_OVERHEAD;
-        const int own_length = tid < batch_size ? cache_lengths[tid] : 0;
-        own_lengths[tid] = own_length;
-        int value = tid < batch_size ? index_math::positions_of(tiles_of(own_length), overhead) : 0;
-#pragma unroll
-        for (int offset = 1; offset < 64; offset <<= 1) {
-            const int other = __shfl_up(value, offset);
-            if (lane >= offset) value += other;
-        }
-        if (lane == 63) own_wave_totals[wave] = value;
-        if (tid == 0) own_prefix[0] = 0;
-        __syncthreads();
-        int before = 0;
-#pragma unroll
-        for (int w = 0; w < THREADS / 64; ++w) {
-            if (w < wave) before += own_wave_totals[w];
-        }
-        if (tid < batch_size) own_prefix[tid + 1] = before + value;
-        __syncthreads();
-        // what comes out of LDS is the same in every lane, which the compiler cannot know: say so, or everything
-        // computed from it (the base addresses of the unit requests among it) ends up in vector registers
-        total = __builtin_amdgcn_readfirstlane(own_prefix[batch_size]);
-        ranges = index_math::ranges_of(total, own_workgroups);
-        prefix = own_prefix;
-        if (blockIdx.x == 0 && blockIdx.y == 0) {
-            if (tid == 0) {
-                plan[PLAN_TOTAL] = total;
-                plan[PLAN_WORKGROUPS] = own_workgroups;
-                plan[PLAN_OVERHEAD] = overhead;
-                plan[PLAN_WHOLE] = own_whole;
-                plan[PLAN_RANGES] = ranges;
-            }
-            if (tid <= batch_size) plan[index_math::plan_prefix_at() + tid] = own_prefix[tid];
-        }
-    } else {
-        total = plan[PLAN_TOTAL];
-        overhead = plan[PLAN_OVERHEAD];
-        whole_sequences = plan[PLAN_WHOLE] != 0;
-        ranges = plan[PLAN_RANGES];
-        prefix = plan + index_math::plan_prefix_at();
-    }
-
-    int range_begin, range_end;
-    if (whole_sequences) {
-        range_begin = __builtin_amdgcn_readfirstlane(prefix[workgroup]);
-        range_end = __builtin_amdgcn_readfirstlane(prefix[workgroup + 1]);
-    } else {
-        if (workgroup >= ranges) return;
-        range_begin = index_math::range_begin_of(total, ranges, workgroup);
-        range_end = index_math::range_begin_of(total, ranges, workgroup + 1);
-    }
+    const DecodeRange range = decode_range(plan, cache_lengths, batch_size, own_workgroups, own_whole, own_prefix, own_lengths,
+                                           own_wave_totals, tid, workgroup, blockIdx.x == 0 && blockIdx.y == 0);
+    const int range_begin = range.begin, range_end = range.end, overhead = range.overhead;
+    const int* prefix = range.prefix;
     if (range_begin >= range_end) return;
-    int sequence;
-    if (own_workgroups > 0 && !whole_sequences) {
-        // first sequence whose positions reach past range_begin
-        int low = 0, high = batch_size;
-        while (low < high) {
-            const int mid = (low + high) / 2;
-            if (__builtin_amdgcn_readfirstlane(prefix[mid + 1]) <= range_begin) low = mid + 1; else high = mid;
-        }
-        sequence = low;
-    } else if (own_workgroups > 0) {
-        sequence = workgroup;
-    } else {
-        sequence = plan[index_math::plan_first_sequence_at(batch_size) + workgroup];
-    }
+    int sequence = range.sequence;
 
     const int head = head0 + 32 * wave + lq;
     const bool valid = head < heads;
@@ -1146,9 +824,46 @@ std::size_t mla_decode_plan_elements(int batch_size, int /*heads*/, int /*splits
     return static_cast<std::size_t>(index_math::plan_elements_bound(batch_size));
 }
 
+namespace {
+
+// Which kernel takes a decode call, and how its list is cut.  Depends on the batch, the head count and the splits
+// only, so that a plan built for them fits the call.
+struct DecodeChoice {
+    int row_blocks;   // of the kernels in mla_narrow.hip; 0: the 128-row kernel of this file
+    index_math::DecodeLayout layout;
+};
+
+// The line between the kernels (times of the whole call, 1024..8192 tokens a sequence unless stated, 8 splits):
+//   * 32 rows when one head group holds all heads (64 sequences, 16 heads: 69 us against 75 with 64 rows and 104 with
+//     128; 32 heads: 75 / 76 / 104), or when every range the partial-result slots allow finds a compute unit for each
+//     of its head groups anyway (4 sequences, 128 heads: 31 / 32 / 53; 1 sequence of 200 tokens: 13 / 14 / 21);
+//   * 64 rows up to 64 heads (64 sequences, 64 heads: 109 / 83 / 109) and beyond while sequences x head groups stay
+//     few: the 128-row kernel is then held back by its slots and its start (16 sequences, 128 heads: 63 / 50 / 64);
+//   * 128 rows otherwise (32 sequences, 128 heads: 101 / 78 / 79; 64 sequences: 183 / 136 / 117).
+constexpr int NARROW_SEQUENCE_GROUPS = 48;
+
+DecodeChoice decode_choice(int batch_size, int heads, int splits) {
+    DecodeChoice choice;
+    const long long groups32 = (heads + 31) / 32, groups64 = (heads + 63) / 64;
+    const long long ranges = (long long)batch_size * (2LL * splits - 1);
+    if (groups32 == 1 || groups32 * ranges <= compute_units()) {
+        choice.row_blocks = 1;
+    } else if (groups64 == 1 || batch_size * groups64 <= NARROW_SEQUENCE_GROUPS) {
+        choice.row_blocks = 2;
+    } else {
+        choice.row_blocks = 0;
+    }
+    choice.layout = choice.row_blocks == 0
+        ? index_math::decode_layout(batch_size, heads, splits, compute_units(), ROWS, RANK)
+        : index_math::narrow_decode_layout(batch_size, heads, splits, compute_units(), choice.row_blocks, RANK);
+    return choice;
+}
+
+}  // namespace
+
 void mla_decode_plan_dispatch(int* plan, const int* cache_lengths, int batch_size, int heads, int splits,
                               hipStream_t stream) {
-    const index_math::DecodeLayout layout = index_math::decode_layout(batch_size, heads, splits, compute_units(), ROWS, RANK);
+    const index_math::DecodeLayout layout = decode_choice(batch_size, heads, splits).layout;
     hipLaunchKernelGGL(mla_decode_plan_kernel, dim3(1), dim3(THREADS), 0, stream, plan, cache_lengths, batch_size,
                        layout.workgroups, layout.whole_sequences);
     HIP_CHECK(hipGetLastError());
@@ -1161,28 +876,36 @@ void mla_decode_dispatch(bf16_t* output, float* logsumexp, const bf16_t* query, 
     if ((reinterpret_cast<uintptr_t>(workspace) & 15) != 0) {
         throw std::invalid_argument("MLA decode requires a workspace aligned to 16 bytes");
     }
-    static hip_common::OncePerDevice prepared;
-    prepared.run([] { allow_large_lds(mla_decode_split_kernel); });
     // How the caller's B*H*splits*(C+2) floats are used: index_math::decode_layout.
-    const index_math::DecodeLayout layout = index_math::decode_layout(batch_size, heads, splits, compute_units(), ROWS, RANK);
-    int own_workgroups = 0;
+    const DecodeChoice choice = decode_choice(batch_size, heads, splits);
+    const index_math::DecodeLayout& layout = choice.layout;
+    bool own_plan = false;
     if (plan == nullptr) {
         // no plan from the caller: this call's own, behind the partial-result slots -- built by the decode kernel
         // itself when one workgroup can scan the batch, by the plan kernel otherwise
         plan = reinterpret_cast<int*>(workspace + layout.plan_offset);
         if (batch_size <= SELF_PLAN_BATCH) {
-            own_workgroups = layout.workgroups;
+            own_plan = true;
         } else {
             hipLaunchKernelGGL(mla_decode_plan_kernel, dim3(1), dim3(THREADS), 0, stream, plan, cache_lengths, batch_size,
                                layout.workgroups, layout.whole_sequences);
             HIP_CHECK(hipGetLastError());
         }
     }
+    if (choice.row_blocks != 0) {
+        mla_narrow_decode_launch(output, logsumexp, query, paged_kv_cache, block_table, cache_lengths, workspace, plan,
+                                 batch_size, heads, page_size, pages_per_sequence, choice.row_blocks, layout.workgroups,
+                                 layout.whole_sequences, layout.slot_floats, own_plan, scale, stream);
+        return;
+    }
+    static hip_common::OncePerDevice prepared;
+    prepared.run([] { allow_large_lds(mla_decode_split_kernel); });
     const int padded_rows = (heads + 31) / 32 * 32;
     const dim3 grid(layout.workgroups, layout.head_groups);
     hipLaunchKernelGGL(mla_decode_split_kernel, grid, dim3(THREADS), LDS_BYTES, stream, output, logsumexp, query,
                        paged_kv_cache, block_table, cache_lengths, workspace, plan, batch_size, heads, page_size,
-                       pages_per_sequence, layout.slot_floats, padded_rows, scale, own_workgroups, layout.whole_sequences);
+                       pages_per_sequence, layout.slot_floats, padded_rows, scale, own_plan ? layout.workgroups : 0,
+                       layout.whole_sequences);
     HIP_CHECK(hipGetLastError());
     if (!layout.whole_sequences) {
         hipLaunchKernelGGL(mla_decode_merge_kernel, dim3(MERGE_QUARTERS * (padded_rows / 32), batch_size), dim3(64), 0,
@@ -1195,13 +918,23 @@ void mla_decode_dispatch(bf16_t* output, float* logsumexp, const bf16_t* query, 
 void mla_absorbed_forward_dispatch(bf16_t* output, float* logsumexp, const bf16_t* query_latent,
                                    const bf16_t* query_rope, const bf16_t* kv_latent, const bf16_t* key_rope,
                                    int batch_size, int sequence_length, int heads, float scale, hipStream_t stream) {
-    static hip_common::OncePerDevice prepared;
-    prepared.run([] { allow_large_lds(mla_absorbed_forward_kernel); });
     const long long rows = (long long)sequence_length * heads;
     const long long row_blocks = (rows + ROWS - 1) / ROWS;
     if (row_blocks * batch_size > 0x7fffffffLL) {
         throw std::invalid_argument("MLA forward: batch*tokens*heads exceeds the grid limit");
     }
+    // 32 or 64 rows per workgroup while 128 rows leave compute units idle (whole layer of absorb, forward and
+    // un-absorb, 32 / 64 / 128 rows): 32 blocks (T = 512, H = 8) 42 / 45 / 61 us, 128 blocks 52 / 52 / 66, 243 blocks
+    // 236 / 168 / 241, 256 blocks 108 / 84 / 103, 391 blocks 113 / 95 / 92, 1024 blocks 374 / 284 / 268.
+    const long long blocks = row_blocks * batch_size;
+    const int narrow = 2 * blocks <= compute_units() ? 1 : 4 * blocks <= 5LL * compute_units() ? 2 : 0;
+    if (narrow != 0) {
+        mla_narrow_forward_launch(output, logsumexp, query_latent, query_rope, kv_latent, key_rope, batch_size,
+                                  sequence_length, heads, narrow, scale, stream);
+        return;
+    }
+    static hip_common::OncePerDevice prepared;
+    prepared.run([] { allow_large_lds(mla_absorbed_forward_kernel); });
     hipLaunchKernelGGL(mla_absorbed_forward_kernel, dim3((unsigned)(row_blocks * batch_size)), dim3(THREADS), LDS_BYTES,
                        stream, output, logsumexp, query_latent, query_rope, kv_latent, key_rope, sequence_length, heads,
                        (int)row_blocks, scale);

@@ -527,6 +527,23 @@ void check_decode_layout() {
             }
         }
     }
+    // the layout of the kernels with fewer rows per workgroup: the same workspace, slots of the real heads only
+    for (int compute_units : {1, 8, 256}) {
+        for (int batch = 1; batch <= 80; batch += 3) {
+            for (int heads : {1, 2, 16, 31, 33, 64, 65, 128, 160}) {
+                for (int splits : {1, 2, 3, 8, 33}) {
+                    for (int row_blocks : {1, 2}) {
+                        const DecodeLayout layout = narrow_decode_layout(batch, heads, splits, compute_units, row_blocks, RANK);
+                        const long long workspace = (long long)batch * heads * splits * (RANK + 2);
+                        EXPECT(layout.plan_offset + layout.plan_ints <= workspace, "narrow B %d H %d splits %d: past the workspace", batch, heads, splits);
+                        EXPECT(layout.slot_floats >= heads * (RANK / 2 + 2) && layout.slot_floats % 4 == 0, "narrow H %d", heads);
+                        EXPECT(layout.whole_sequences ? layout.workgroups == batch : layout.workgroups >= 2 && layout.slots == layout.workgroups + batch,
+                               "narrow B %d H %d splits %d", batch, heads, splits);
+                    }
+                }
+            }
+        }
+    }
     // the headline decode shape uses every compute unit
     const DecodeLayout headline = decode_layout(64, 128, 8, 256, ROWS, RANK);
     EXPECT(!headline.whole_sequences && headline.workgroups == 256, "B 64 H 128 splits 8: %d workgroups", headline.workgroups);

@@ -1,0 +1,95 @@
+"""The three forms of the absorbed decode and prefill forward (32, 64 and 128 rows per workgroup) at the edges of
+their row groups, key units and dispatch ranges, against the fp32 oracle; and the raised softmax reference in each."""
+
+import pytest
+import torch
+
+from dscuda_amd.harness import configs, ops
+from oracle import attention_oracle as oracle
+from tests.parity import announce, assert_close_bf16, assert_close_lse
+
+pytestmark = pytest.mark.gpu
+
+
+def assert_rounded(out, expected, expected_lse, values):
+    """Probabilities, partial rows and results are each rounded to bf16 once, by at most 2^-9 of a mean of |values|
+    that the softmax weights; the weights themselves carry the fp32 error of scores this large: 36 partial sums, the
+    scaling and the two log-sum-exp steps round by 2^-24 of the score each."""
+    largest = values.float().abs().max().item()
+    weights = 40 * 2 ** -24 * expected_lse.abs().max().item()
+    error = (out.cpu().float() - expected).abs()
+    worst, mean = error.max().item(), error.mean().item()
+    assert worst <= (3 * 2 ** -9 + weights) * largest and mean <= 6e-3
+
+
+@pytest.mark.parametrize("batch,heads,splits", [
+    (7, 1, 8), (7, 15, 8), (7, 17, 4), (7, 32, 8), (7, 32, 1),   # 32 rows, one head group
+    (7, 33, 8), (2, 65, 8), (7, 128, 1),                          # 32 rows, every range has its compute units
+    (14, 64, 8), (14, 47, 8), (14, 65, 8), (14, 100, 3),          # 64 rows
+    (28, 128, 8), (28, 97, 2),                                    # 128 rows
+])
+def test_decode_row_blocks(cuda, batch, heads, splits):
+    lengths = ([1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 128, 129, 200, 700] * 2)[:batch]
+    tokens = max(lengths)
+    g = torch.Generator().manual_seed(batch + heads)
+    query = (torch.randn(batch, 1, heads, 576, generator=g) * 0.25).bfloat16()
+    cache = (torch.randn(batch, tokens, 576, generator=g) * 0.25).bfloat16()
+    paged, table = configs.pack_cache(cache, 64)
+    lengths = torch.tensor(lengths, dtype=torch.int32)
+    scale = configs.c_float(576 ** -0.5)
+    announce("decode row blocks", dict(B=batch, H=heads, splits=splits))
+    out, lse = ops.mla_decode(query.to(cuda), paged.to(cuda), table.to(cuda), lengths.to(cuda), scale, splits=splits)
+    expected, expected_lse = oracle.mla_decode_unrounded(query, cache, lengths, scale)
+    assert_close_bf16("O", out, expected)
+    assert_close_lse("LSE", lse, expected_lse)
+
+
+@pytest.mark.parametrize("batch,heads", [(2, 40), (14, 64), (28, 128)])   # 32, 64 and 128 rows
+def test_decode_raised_reference(cuda, batch, heads):
+    """Keys late in the stream aligned with one head of each row group: scores thousands above the first keys'."""
+    tokens = 420
+    g = torch.Generator().manual_seed(31)
+    query = torch.randn(batch, 1, heads, 576, generator=g).bfloat16()
+    cache = (torch.randn(batch, tokens, 576, generator=g) * 0.05).bfloat16()
+    for first, last, head, factor in [(70, 72, 0, 1.0), (200, 201, heads - 1, 2.0), (300, 340, heads // 2, 4.0)]:
+        cache[:, first:last] = (query[:, 0, head:head + 1].float() * factor).bfloat16()
+    lengths = torch.tensor([tokens - 11 * (b % 9) for b in range(batch)], dtype=torch.int32)
+    paged, table = configs.pack_cache(cache, 64)
+    announce("decode raised reference", dict(B=batch, H=heads))
+    out, lse = ops.mla_decode(query.to(cuda), paged.to(cuda), table.to(cuda), lengths.to(cuda), 1.0, splits=2)
+    expected, expected_lse = oracle.mla_decode_unrounded(query, cache, lengths, 1.0)
+    assert expected_lse.max() > 500
+    assert_rounded(out, expected, expected_lse, cache)
+    assert ((lse.cpu() - expected_lse).abs() / expected_lse.abs().clamp_min(1)).max().item() <= 1e-5
+
+
+@pytest.mark.parametrize("batch,tokens,heads", [
+    (1, 32, 1), (1, 33, 1), (3, 63, 2), (1, 129, 31),   # 32 rows, last block of 1, 2, 30 and 31 rows among them
+    (1, 273, 63), (2, 129, 65), (1, 160, 127),          # 64 rows
+    (1, 345, 120),                                      # 128 rows
+])
+def test_forward_row_blocks(cuda, batch, tokens, heads):
+    ql, qr, c, kr, scale = configs.mla_absorbed_inputs(batch, tokens, heads, seed=tokens)
+    announce("forward row blocks", dict(B=batch, T=tokens, H=heads))
+    out, lse = ops.mla_forward(ql.to(cuda), qr.to(cuda), c.to(cuda), kr.to(cuda), scale)
+    expected, expected_lse = oracle.mla_forward_unrounded(ql, qr, c, kr, scale, oracle.causal_mask(tokens))
+    assert_close_bf16("O", out, expected, max_abs=8e-3)
+    assert_close_lse("LSE", lse, expected_lse, tol=1e-4)
+
+
+@pytest.mark.parametrize("tokens,heads", [(150, 64), (330, 128)])   # 64 and 128 rows
+def test_forward_raised_reference(cuda, tokens, heads):
+    g = torch.Generator().manual_seed(14)
+    direction = torch.randn(576, generator=g)
+    query = (direction[None, None, None, :] + 0.1 * torch.randn(1, tokens, heads, 576, generator=g)).bfloat16()
+    keys = (torch.randn(1, tokens, 576, generator=g) * 0.05).bfloat16()
+    for first, last, factor in [(50, 60, 1.0), (100, 130, 4.0)]:
+        keys[:, first:last] = (direction * factor).bfloat16()
+    ql, qr = query[..., :512].contiguous(), query[..., 512:].contiguous()
+    c, kr = keys[..., :512].contiguous(), keys[..., 512:].contiguous()
+    announce("forward raised reference", dict(T=tokens, H=heads))
+    out, lse = ops.mla_forward(ql.to(cuda), qr.to(cuda), c.to(cuda), kr.to(cuda), 1.0)
+    expected, expected_lse = oracle.mla_forward_unrounded(ql, qr, c, kr, 1.0, oracle.causal_mask(tokens))
+    assert expected_lse.max() > 500
+    assert_rounded(out, expected, expected_lse, c)
+    assert ((lse.cpu() - expected_lse).abs() / expected_lse.abs().clamp_min(1)).max().item() <= 1e-5
