@@ -1,17 +1,13 @@
 // Causal attention forward for gfx950: S^T = K Q^T and O^T = V^T P^T on bf16
 // MFMA 32x32x16 tiles, online softmax in fp32, natural-log LSE.
 //
-// One kernel template serves the flash-attention forward (D = 64 / 128, GQA)
-// and the per-head MLA prefill forward (d_qk = 128 nope + 64 rope = 192,
-// d_v = 128).  It takes the place of the reference's
+// Two kernels serve the flash-attention forward (D = 64 / 128, GQA) and the
+// per-head MLA prefill forward (d_qk = 128 nope + 64 rope = 192, d_v = 128):
+// split keys for short and medium problems, a persistent one for large ones.
+// They take the place of the reference's
 // flash_attention_forward_tensor_core_kernel
 // (kernels/attention/flash_attention/sm89_forward.cu:99-205); the tiling is
 // chosen for 64-lane waves and the 160 KB LDS, not taken from there.
-//
-// Work decomposition
-//   workgroup = NWAVES waves, each wave owns 32 query rows for the whole key
-//   loop (BM = 32*NWAVES queries per workgroup).  Keys are walked in tiles of
-//   BN = 64 from key 0 up to the diagonal.
 //
 // Transposed formulation
 //   Scores are produced as S^T (keys x queries): A = K tile (LDS), B = Q
@@ -24,11 +20,11 @@
 //
 // Tiles: global -> LDS without registers
 //   K and V tiles arrive by global_load_lds (16 bytes per lane, 1 KB of
-//   consecutive LDS per wave instruction), both row-major, two stages.  No
+//   consecutive LDS per wave instruction), both row-major.  No
 //   thread holds tile data in registers and nothing is written to LDS with
 //   store instructions.  With no padding possible inside the 1 KB a wave
 //   instruction fills, bank spread comes from a swizzle applied on the global
-//   side (which 16-byte chunk a lane fetches):
+//   side (which 16-byte chunk a lane fetches; in the persistent kernel, the other takes lds_tiles.h as it is):
 //     K  : chunk c of row r sits at position c ^ fK(r).  A fragment read is 16
 //          lanes x 16 B down a column of rows; fK(r) = (r>>1)&7 for rows that
 //          are 128 (mod 256) bytes long, r&15 for rows that are 0 (mod 256).
@@ -44,7 +40,9 @@
 #include "attn_kernels.h"
 #include "hip_common.h"
 #include "index_math.h"
+#include "lds_tiles.h"
 
+#include <algorithm>
 #include <cmath>
 #include <stdexcept>
 #include <string>
@@ -65,12 +63,8 @@ struct FwdConfig {
     static constexpr int V_CHUNKS = DV / 8;
     static constexpr int V_GROUPS = DV / 32;               // 64-byte column groups per row
     static constexpr int V_BYTES = BN * V_ROW;
-    static constexpr int STAGE_BYTES = K_BYTES + V_BYTES;
     static constexpr int K_LOADS_PER_WAVE = K_BYTES / 1024 / NWAVES;   // wave instructions
     static constexpr int V_LOADS_PER_WAVE = V_BYTES / 1024 / NWAVES;
-    static constexpr int O_PITCH = DV * 2 + 16;            // epilogue staging, bytes
-    static constexpr int O_BYTES = BM * O_PITCH;
-    static constexpr int LDS_BYTES = (2 * STAGE_BYTES > O_BYTES) ? 2 * STAGE_BYTES : O_BYTES;
     static_assert(K_BYTES % (1024 * NWAVES) == 0 && V_BYTES % (1024 * NWAVES) == 0,
                   "tile loads must divide evenly over the waves");
     static_assert(K_ROW % 128 == 0, "K rows must be a multiple of 128 bytes");
@@ -84,98 +78,129 @@ struct FwdConfig {
     }
 };
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef short s16x8 __attribute__((ext_vector_type(8)));
-typedef __attribute__((address_space(3))) s16x4* transposing_read_pointer;
+// ---------------------------------------------------------------------------
+// Split-key variant for short and medium problems.
+//
+// A workgroup of eight waves (two per SIMD) takes 32 * QG queries and walks the keys in tiles of 128; the eight waves
+// are QG query groups x KG key groups, a wave holds 32 queries and TILE / KG keys of every tile, with softmax statistics
+// and output sums of its own.  After the last tile the KG parts of a query meet in LDS: every wave hands the column
+// blocks it does not own to their owners, which scale the parts to the common maximum and add them up.
+// The walk of a workgroup is half (KG = 2) or a quarter (KG = 4) as many dependent rounds of scores, softmax and
+// output products as with one wave for all keys, and the two waves of a SIMD cover each other's latencies.
+// Queries arrive as a tile of their own (whole rows, then operand reads from LDS): loaded by the lanes that need them,
+// 16 bytes of 32 different rows per instruction and once per key group, they took longer than a tile of keys.
+//
+// What bounds it: a step of 128 queries and 128 keys (head size 128, stamps) takes 4000 cycles -- requests 600 to 850 (64
+// pieces of 1 KB at the 13 cycles the address unit takes for one), scores 1150 and output products 1170 for the two
+// waves of a SIMD (1024 of matrix time each), softmax 250 to 550, barrier -- and start and end of a workgroup some 8000.
+// Moving the requests into the product streams, setting the waves of a SIMD half a step apart, leaving the requests to
+// four of the waves, touching the keys ahead of time for the L2: each within 5 % of this order, or slower.
+// With one wave for all keys (128 queries, four waves) before: 8 heads of 512 tokens, 64 columns 12.0 -> 7.3 us; 32 x 8
+// heads of 2048 tokens, 128 columns 58 -> 41 us (830 TFLOP/s); 16 heads of 1000 tokens, 192 / 128 columns 31 -> 16 us.
+template <int DQK, int DV, int QG, int KG>
+struct SplitConfig {
+    static constexpr int TILE = 128;
+    static constexpr int WAVES = QG * KG;
+    static constexpr int THREADS = 64 * WAVES;
+    static constexpr int BN = TILE / KG;                   // keys per wave and tile
+    static constexpr int BM = 32 * QG;
+    static constexpr int K_ROW = DQK * 2;                  // bytes
+    static constexpr int K_BYTES = TILE * K_ROW;
+    static constexpr int V_ROW = DV * 2;
+    static constexpr int V_BYTES = TILE * V_ROW;
+    static constexpr int STAGE_BYTES = K_BYTES + V_BYTES;
+    static constexpr int DBLOCKS = DV / 32;
+    // after the walk: parts on their way to their owners (4 KB per 32 x 32 block), statistics, output rows
+    static constexpr int PART_BYTES = QG * DBLOCKS * (KG - 1) * 4096;
+    static constexpr int MAX_AT = PART_BYTES;              // [KG][BM]
+    static constexpr int SUM_AT = MAX_AT + KG * BM * 4;    // [KG][BM]
+    static constexpr int O_AT = SUM_AT + KG * BM * 4;
+    static constexpr int O_PITCH = DV * 2 + 16;
+    static constexpr int MERGE_BYTES = O_AT + BM * O_PITCH;
+    static constexpr int LDS_BYTES = 2 * STAGE_BYTES > MERGE_BYTES ? 2 * STAGE_BYTES : MERGE_BYTES;
+    static_assert(WAVES == 8 && BN % 32 == 0 && BM <= TILE && LDS_BYTES <= 160 * 1024, "");
 
-template <int DQK, int DV, int NWAVES>
-__global__ __launch_bounds__(64 * NWAVES) void attention_forward_kernel(
+    __device__ static constexpr int owner(int block) { return block * KG / DBLOCKS; }
+};
+
+template <int DQK, int DV, int QG, int KG>
+__global__ __launch_bounds__(64 * QG * KG) void attention_forward_split_kernel(
     bf16_t* __restrict__ output, float* __restrict__ logsumexp,
     const bf16_t* __restrict__ query, const bf16_t* __restrict__ key, const bf16_t* __restrict__ value,
-    int sequence_length, int query_heads, int key_value_heads, int query_blocks, float scale) {
-    using C = FwdConfig<DQK, DV, NWAVES>;
+    int sequence_length, int query_heads, int key_value_heads, index_math::SplitOrder order, float scale) {
+    using C = SplitConfig<DQK, DV, QG, KG>;
+    using KReads = TileReads<C::K_ROW>;
+    using VReads = TileReads<C::V_ROW>;
     constexpr int BN = C::BN;
+    constexpr int MB = BN / 32;
     constexpr int KSTEPS = DQK / 16;
-    constexpr int DBLOCKS = DV / 32;
+    constexpr int NSTEPS = BN / 16;
+    constexpr int DBLOCKS = C::DBLOCKS;
+    constexpr int QK_MFMAS = MB * KSTEPS;
+    constexpr int PV_MFMAS = NSTEPS * DBLOCKS;
+    constexpr int RING = QK_MFMAS >= 8 ? 8 : 4;            // fragments read ahead of the product that takes them
+    constexpr float LOWEST = -1e30f;   // below every score, finite: a key group may hold no visible key of a row
 
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int query_group = wave % QG;
+    const int key_group = wave / QG;
     const int lane = tid % 64;
     const int lq = lane % 32;
     const int g = lane / 32;
 
-    // (batch, head) groups are dealt across XCDs; inside a group the heaviest
-    // (last) query blocks are issued first.
-    int bh, qb_rank;
-    xcd_order(blockIdx.x, gridDim.x / query_blocks, query_blocks, bh, qb_rank);
-    const int qb = query_blocks - 1 - qb_rank;
-    const int b = bh / query_heads;
-    const int h = bh % query_heads;
-    const int hk = h / (query_heads / key_value_heads);
+    const index_math::SplitItem item = index_math::split_item(blockIdx.x, order);
+    const int h = item.head;
+    const int qb = item.query_block;
+    const int b = item.batch;
+    const int hk = item.key_value_head;
     const int S = sequence_length;
 
     const int q0 = qb * C::BM;
-    const int wave_q0 = q0 + 32 * wave;
+    const int wave_q0 = q0 + 32 * query_group;
     const int q_row = wave_q0 + lq;
-
-    const size_t q_stride = (size_t)query_heads * DQK;
+    const unsigned q_stride_bytes = (unsigned)query_heads * DQK * 2;
     const unsigned k_stride_bytes = (unsigned)key_value_heads * DQK * 2;
     const unsigned v_stride_bytes = (unsigned)key_value_heads * DV * 2;
-    const bf16_t* q_base = query + ((size_t)b * S * query_heads + h) * DQK;
     const unsigned char* k_base =
         reinterpret_cast<const unsigned char*>(key + ((size_t)b * S * key_value_heads + hk) * DQK);
     const unsigned char* v_base =
         reinterpret_cast<const unsigned char*>(value + ((size_t)b * S * key_value_heads + hk) * DV);
-
-    // ---- Q fragments (B operand: column = query lq, k = 16*ks + 8*g + j)
-    bf16x8 qf[KSTEPS];
-    {
-        const bool valid = q_row < S;
-        const bf16_t* row = q_base + (size_t)(valid ? q_row : 0) * q_stride + 8 * g;
-#pragma unroll
-        for (int ks = 0; ks < KSTEPS; ++ks) {
-            u32x4 bits = {0, 0, 0, 0};
-            if (valid) {
-                bits = *reinterpret_cast<const u32x4*>(row + 16 * ks);
-            }
-            qf[ks] = __builtin_bit_cast(bf16x8, bits);
-        }
-    }
-
-    const int last_key = min(S, q0 + C::BM) - 1;
-    const int tiles = last_key / BN + 1;
     const unsigned lds_base = lds_offset_of(lds);
 
-    // Requests this wave's share of tile `tile` into `stage`.  Rows past the end
-    // of the sequence are clamped to the last one: such keys are invisible to
-    // every stored query, the data only has to be finite.
-    auto request_tile = [&](int tile, int stage) {
-        const int key0 = tile * BN;
-        const int row_limit = S - 1 - key0;
-        const unsigned char* k_tile = k_base + (size_t)key0 * k_stride_bytes;
-        const unsigned char* v_tile = v_base + (size_t)key0 * v_stride_bytes;
-        const unsigned stage_base = lds_base + stage * C::STAGE_BYTES;
-#pragma unroll
-        for (int i = 0; i < C::K_LOADS_PER_WAVE; ++i) {
-            const int load = wave * C::K_LOADS_PER_WAVE + i;
-            const int slot = 64 * load + lane;
-            const int row = slot / C::K_CHUNKS;
-            const int chunk = (slot % C::K_CHUNKS) ^ C::k_swizzle(row);
-            const unsigned offset = (unsigned)min(row, row_limit) * k_stride_bytes + 16u * chunk;
-            direct_load_16_offset(k_tile, offset, stage_base + load * 1024);
-        }
-#pragma unroll
-        for (int i = 0; i < C::V_LOADS_PER_WAVE; ++i) {
-            const int load = wave * C::V_LOADS_PER_WAVE + i;
-            const int slot = 64 * load + lane;
-            const int row = slot / C::V_CHUNKS;
-            const int chunk = (slot % C::V_CHUNKS) ^ (C::v_flip(row) << 2);
-            const unsigned offset = (unsigned)min(row, row_limit) * v_stride_bytes + 16u * chunk;
-            direct_load_16_offset(v_tile, offset, stage_base + C::K_BYTES + load * 1024);
-        }
+    // Rows past the end of the sequence repeat the last one: such keys are invisible to every stored query.
+    TileRequests<C::K_ROW, C::WAVES, C::TILE> k_requests;
+    TileRequests<C::V_ROW, C::WAVES, C::TILE> v_requests;
+    k_requests.init(k_stride_bytes, wave, lane);
+    v_requests.init(v_stride_bytes, wave, lane);
+    auto request_tile = [&](int tile) {
+        const int key0 = tile * C::TILE;
+        const unsigned target = lds_base + (tile & 1) * C::STAGE_BYTES;
+        k_requests.request(k_base + (size_t)key0 * k_stride_bytes, k_stride_bytes, S - 1 - key0, target, wave);
+        v_requests.request(v_base + (size_t)key0 * v_stride_bytes, v_stride_bytes, S - 1 - key0, target + C::K_BYTES, wave);
     };
+
+    KReads k_reads;
+    VReads v_reads;
+    k_reads.init(lane);
+    v_reads.init(lane);
+
+    // The queries go where tile 1 will go, tile 0 to its own stage.
+    bf16x8 qf[KSTEPS];   // B operand: column = query lq, k = 16*ks + 8*g + j
+    {
+        TileRequests<C::K_ROW, C::WAVES, C::BM> q_requests;
+        q_requests.init(q_stride_bytes, wave, lane);
+        q_requests.request(reinterpret_cast<const unsigned char*>(query + (((size_t)b * S + q0) * query_heads + h) * DQK),
+                           q_stride_bytes, S - 1 - q0, lds_base + C::STAGE_BYTES, wave);
+        request_tile(0);
+        wait_vector_memory<TileRequests<C::K_ROW, C::WAVES, C::TILE>::LOADS + TileRequests<C::V_ROW, C::WAVES, C::TILE>::LOADS>();
+        workgroup_barrier();   // the query tile has landed
+        unsigned q_at[KReads::NAT];
+        rebase(q_at, k_reads.natural, C::STAGE_BYTES + query_group * 32 * C::K_ROW);
+        unrolled<0, KSTEPS>([&](auto tag) { qf[decltype(tag)::value] = natural_fragment<C::K_ROW, 0, decltype(tag)::value>(lds, q_at); });
+    }
 
     f32x16 o_acc[DBLOCKS];
 #pragma unroll
@@ -183,155 +208,177 @@ __global__ __launch_bounds__(64 * NWAVES) void attention_forward_kernel(
 #pragma unroll
         for (int i = 0; i < 16; ++i) o_acc[d][i] = 0.f;
     }
-    float row_max = -INFINITY;  // reference point of the exponent, raw score units
-    float row_sum = 0.f;        // this lane's share (its 32 keys per tile) of the normaliser
+    float row_max = LOWEST;    // reference point of the exponent, raw score units
+    float row_sum = 0.f;       // this lane's share of the normaliser
     const float c = scale * LOG2E;
 
-    // Per-lane pieces of the LDS read addresses.
-    const int k_swz = C::k_swizzle(lq);                        // rows lq and lq+32 share it
-    const int s16 = lane % 16;
-    const int v_row = 4 * g + s16 / 4;                          // + 16*n, + 8 for the second read
-    const int v_in_group = 32 * ((lane / 16) % 2) + 8 * (s16 % 4);
-    const int v_flip = C::v_flip(v_row);                        // rows v_row + 8*m share it
-
-    wait_vector_memory<0>();   // the query loads: no wait for them may remain inside the loop
-    request_tile(0, 0);
-
+    const int tiles = (min(S, q0 + C::BM) - 1) / C::TILE + 1;
     for (int tile = 0; tile < tiles; ++tile) {
-        const int stage = tile & 1;
         wait_vector_memory<0>();   // this wave's share of the tile has landed
-        workgroup_barrier();       // ... and everybody's; every wave has left the previous tile
-        if (tile + 1 < tiles) {
-            request_tile(tile + 1, stage ^ 1);
+        workgroup_barrier();       // ... and everybody's; every wave has left the previous tile (or its queries)
+        if (tile + 1 < tiles) request_tile(tile + 1);
+        const int key0 = tile * C::TILE + key_group * BN;
+        if (key0 > wave_q0 + 31) continue;   // every key of this wave's part is in its queries' future
+
+        const unsigned stage = (tile & 1) * C::STAGE_BYTES;
+        unsigned k_at[KReads::NAT], v_at[2][VReads::TR];
+        rebase(k_at, k_reads.natural, stage + key_group * BN * C::K_ROW);
+        rebase(v_at, v_reads.transposed, stage + C::K_BYTES + key_group * BN * C::V_ROW);
+        // fragment I of the stream: k-step I / MB of key block I % MB, then 16-key step and column block of V
+        auto fragment = [&](auto tag) -> bf16x8 {
+            constexpr int I = decltype(tag)::value;
+            if constexpr (I < QK_MFMAS) {
+                return natural_fragment<C::K_ROW, 32 * (I % MB), I / MB>(lds, k_at);
+            } else {
+                constexpr int J = I - QK_MFMAS;
+                return transposed_fragment<C::V_ROW, 16 * (J / DBLOCKS), J % DBLOCKS>(lds, v_at);
+            }
+        };
+
+        f32x16 s_acc[MB];
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s_acc[mb][i] = 0.f;
         }
-        const int key0 = tile * BN;
-        if (key0 <= wave_q0 + 31) {  // otherwise every key of the tile is in this wave's future
-            const unsigned char* k_lds = lds + stage * C::STAGE_BYTES;
-            const unsigned char* v_lds = k_lds + C::K_BYTES;
+        bf16x8 ring[RING];
+        static_assert(QK_MFMAS >= RING && PV_MFMAS >= RING, "the first V fragments are read behind the last K fragments");
+        unrolled<0, RING>([&](auto tag) { ring[decltype(tag)::value] = fragment(tag); });
+        unrolled<0, QK_MFMAS>([&](auto tag) {
+            constexpr int I = decltype(tag)::value;
+            s_acc[I % MB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[I % RING], qf[I / MB], s_acc[I % MB], 0, 0, 0);
+            ring[I % RING] = fragment(std::integral_constant<int, I + RING>{});
+            __builtin_amdgcn_sched_barrier(0);
+        });
 
-            f32x16 s_acc[2];
+        if (key0 + BN - 1 > wave_q0) {  // the part reaches past this wave's first query
 #pragma unroll
-            for (int mb = 0; mb < 2; ++mb) {
+            for (int mb = 0; mb < MB; ++mb) {
 #pragma unroll
-                for (int i = 0; i < 16; ++i) s_acc[mb][i] = 0.f;
-            }
-#pragma unroll
-            for (int ks = 0; ks < KSTEPS; ++ks) {
-                const int position = (2 * ks + g) ^ k_swz;
-#pragma unroll
-                for (int mb = 0; mb < 2; ++mb) {
-                    const bf16x8 a =
-                        *reinterpret_cast<const bf16x8*>(k_lds + (32 * mb + lq) * C::K_ROW + 16 * position);
-                    s_acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[ks], s_acc[mb], 0, 0, 0);
-                }
-            }
-
-            if (key0 + BN - 1 > wave_q0) {  // tile crosses this wave's diagonal
-#pragma unroll
-                for (int mb = 0; mb < 2; ++mb) {
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        const int k = key0 + 32 * mb + 8 * (i / 4) + 4 * g + (i % 4);
-                        if (k > q_row) s_acc[mb][i] = -INFINITY;
-                    }
-                }
-            }
-
-            float tile_max = s_acc[0][0];
-#pragma unroll
-            for (int mb = 0; mb < 2; ++mb) {
-#pragma unroll
-                for (int i = 0; i < 16; ++i) tile_max = fmaxf(tile_max, s_acc[mb][i]);
-            }
-            tile_max = half_wave_max(tile_max);
-
-            // The reference point only moves when some row's maximum grew by
-            // more than 2^8 in the exponent; until then probabilities may
-            // exceed one, which fp32 sums and bf16 operands hold without loss.
-            const float new_max = fmaxf(row_max, tile_max);
-            const bool grew = (new_max - row_max) * c > 8.0f;
-            if (__any(grew)) {
-                const float alpha = __builtin_amdgcn_exp2f((row_max - new_max) * c);
-                row_max = new_max;
-                row_sum *= alpha;
-#pragma unroll
-                for (int d = 0; d < DBLOCKS; ++d) {
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) o_acc[d][i] *= alpha;
-                }
-            }
-
-            const float offset = row_max * c;
-            bf16x8 pf[4];
-#pragma unroll
-            for (int n = 0; n < 4; ++n) {
-                u32x4 packed;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int i = 8 * (n % 2) + 2 * j;
-                    const float p0 = __builtin_amdgcn_exp2f(fmaf(s_acc[n / 2][i], c, -offset));
-                    const float p1 = __builtin_amdgcn_exp2f(fmaf(s_acc[n / 2][i + 1], c, -offset));
-                    row_sum += p0 + p1;
-                    packed[j] = pack_bf16(p0, p1);
-                }
-                pf[n] = __builtin_bit_cast(bf16x8, packed);
-            }
-
-            // V^T operand through transposing reads.  In a block of 16 lanes, lane s
-            // points at key row 16n + 4g + s/4 (+8 for the second read) and columns
-            // 4*(s%4)..+3 of the 16-column half (block%2) of column group d; the
-            // instruction hands lane i column i of the four rows.  Together: MFMA row
-            // lane%32, keys {4g..4g+3, 8+4g..8+4g+3} of the 16-key step, the k-order
-            // P^T carries from the C layout.
-#pragma unroll
-            for (int n = 0; n < 4; ++n) {
-#pragma unroll
-                for (int d = 0; d < DBLOCKS; ++d) {
-                    const unsigned char* first =
-                        v_lds + (16 * n + v_row) * C::V_ROW + 64 * (d ^ v_flip) + v_in_group;
-                    const s16x4 low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((transposing_read_pointer)first);
-                    const s16x4 high =
-                        __builtin_amdgcn_ds_read_tr16_b64_v4i16((transposing_read_pointer)(first + 8 * C::V_ROW));
-                    const s16x8 both = __builtin_shufflevector(low, high, 0, 1, 2, 3, 4, 5, 6, 7);
-                    o_acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, both), pf[n],
-                                                                       o_acc[d], 0, 0, 0);
+                for (int i = 0; i < 16; ++i) {
+                    const int k = key0 + 32 * mb + 8 * (i / 4) + 4 * g + (i % 4);
+                    if (k > q_row) s_acc[mb][i] = -INFINITY;
                 }
             }
         }
+        float tile_max = s_acc[0][0];
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) tile_max = fmaxf(tile_max, s_acc[mb][i]);
+        }
+        tile_max = half_wave_max(tile_max);
+        // The reference point only moves when some row's maximum grew by more than 2^8 in the exponent.
+        const float new_max = fmaxf(row_max, tile_max);
+        const bool grew = (new_max - row_max) * c > 8.0f;
+        if (__any(grew)) {
+            const float alpha = __builtin_amdgcn_exp2f((row_max - new_max) * c);
+            row_max = new_max;
+            row_sum *= alpha;
+#pragma unroll
+            for (int d = 0; d < DBLOCKS; ++d) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) o_acc[d][i] *= alpha;
+            }
+        }
+        const float offset = row_max * c;
+        bf16x8 pf[NSTEPS];
+#pragma unroll
+        for (int n = 0; n < NSTEPS; ++n) {
+            u32x4 packed;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int i = 8 * (n % 2) + 2 * j;
+                const float p0 = __builtin_amdgcn_exp2f(fmaf(s_acc[n / 2][i], c, -offset));
+                const float p1 = __builtin_amdgcn_exp2f(fmaf(s_acc[n / 2][i + 1], c, -offset));
+                row_sum += p0 + p1;
+                packed[j] = pack_bf16(p0, p1);
+            }
+            pf[n] = __builtin_bit_cast(bf16x8, packed);
+        }
+        unrolled<QK_MFMAS, QK_MFMAS + PV_MFMAS>([&](auto tag) {
+            constexpr int I = decltype(tag)::value;
+            constexpr int J = I - QK_MFMAS;
+            o_acc[J % DBLOCKS] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[I % RING], pf[J / DBLOCKS], o_acc[J % DBLOCKS], 0, 0, 0);
+            if constexpr (I + RING < QK_MFMAS + PV_MFMAS) ring[I % RING] = fragment(std::integral_constant<int, I + RING>{});
+            __builtin_amdgcn_sched_barrier(0);
+        });
     }
 
-    // ---- epilogue: normalise, stage O through LDS for 16-byte row stores
-    workgroup_barrier();   // every wave is done reading the tile stages
-    const float total = half_wave_sum(row_sum);
-    const float inverse = 1.0f / total;
-    if (g == 0 && q_row < S) {
-        logsumexp[((size_t)b * query_heads + h) * S + q_row] = row_max * scale + __logf(total);
+    // ---- the KG parts of a query: statistics and foreign blocks into LDS, then every owner puts its blocks together
+    float* maxima = reinterpret_cast<float*>(lds + C::MAX_AT);
+    float* sums = reinterpret_cast<float*>(lds + C::SUM_AT);
+    const int q_local = 32 * query_group + lq;
+    // part of a block: 16-byte pieces [i4][lane] as the registers hold them
+    auto part_of = [&](int block, int from) {
+        const int index = from < C::owner(block) ? from : from - 1;
+        return lds + ((query_group * DBLOCKS + block) * (KG - 1) + index) * 4096 + 16 * lane;
+    };
+    row_sum = half_wave_sum(row_sum);
+    workgroup_barrier();   // every wave is done with the tile stages
+    if (g == 0) {
+        maxima[key_group * C::BM + q_local] = row_max;
+        sums[key_group * C::BM + q_local] = row_sum;
     }
-    unsigned char* o_lds = lds + (32 * wave) * C::O_PITCH;
 #pragma unroll
     for (int d = 0; d < DBLOCKS; ++d) {
+        if (C::owner(d) != key_group) {
 #pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) {
-            u32x2 packed;
-            packed.x = pack_bf16(o_acc[d][4 * i4 + 0] * inverse, o_acc[d][4 * i4 + 1] * inverse);
-            packed.y = pack_bf16(o_acc[d][4 * i4 + 2] * inverse, o_acc[d][4 * i4 + 3] * inverse);
-            const int dv = 32 * d + 8 * i4 + 4 * g;
-            *reinterpret_cast<u32x2*>(o_lds + lq * C::O_PITCH + 2 * dv) = packed;
+            for (int i4 = 0; i4 < 4; ++i4) {
+                *reinterpret_cast<f32x4*>(part_of(d, key_group) + 1024 * i4) =
+                    f32x4{o_acc[d][4 * i4], o_acc[d][4 * i4 + 1], o_acc[d][4 * i4 + 2], o_acc[d][4 * i4 + 3]};
+            }
         }
     }
-    __syncthreads();
+    workgroup_barrier();
+    float highest = maxima[q_local];
+#pragma unroll
+    for (int k = 1; k < KG; ++k) highest = fmaxf(highest, maxima[k * C::BM + q_local]);
+    float weight[KG];
+    float total = 0.f;
+#pragma unroll
+    for (int k = 0; k < KG; ++k) {
+        weight[k] = __builtin_amdgcn_exp2f((maxima[k * C::BM + q_local] - highest) * c);
+        total = fmaf(sums[k * C::BM + q_local], weight[k], total);
+    }
+    if (key_group == 0 && g == 0 && q_row < S) {
+        logsumexp[((size_t)b * query_heads + h) * S + q_row] = highest * scale + __logf(total);
+    }
+    const float inverse = 1.0f / total;
+#pragma unroll
+    for (int k = 0; k < KG; ++k) weight[k] *= inverse;
+#pragma unroll
+    for (int d = 0; d < DBLOCKS; ++d) {
+        if (C::owner(d) == key_group) {
+#pragma unroll
+            for (int i4 = 0; i4 < 4; ++i4) {
+                f32x4 sum;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) sum[j] = o_acc[d][4 * i4 + j] * weight[C::owner(d)];
+#pragma unroll
+                for (int k = 0; k < KG; ++k) {
+                    if (k == C::owner(d)) continue;
+                    const f32x4 part = *reinterpret_cast<const f32x4*>(part_of(d, k) + 1024 * i4);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) sum[j] = fmaf(part[j], weight[k], sum[j]);
+                }
+                const u32x2 packed = {pack_bf16(sum[0], sum[1]), pack_bf16(sum[2], sum[3])};
+                *reinterpret_cast<u32x2*>(lds + C::O_AT + q_local * C::O_PITCH + 2 * (32 * d + 8 * i4 + 4 * g)) = packed;
+            }
+        }
+    }
+    workgroup_barrier();
     constexpr int ROW_CHUNKS = DV / 8;          // 16-byte chunks per output row
-    constexpr int ROWS_PER_PASS = 64 / ROW_CHUNKS;
     const size_t o_stride = (size_t)query_heads * DV;
     bf16_t* o_base = output + ((size_t)b * S * query_heads + h) * DV;
 #pragma unroll
-    for (int pass = 0; pass < 32 / ROWS_PER_PASS; ++pass) {
-        const int row = pass * ROWS_PER_PASS + lane / ROW_CHUNKS;
-        const int chunk = lane % ROW_CHUNKS;
-        const int q = wave_q0 + row;
-        if (q < S) {
-            const u32x4 bits = *reinterpret_cast<const u32x4*>(o_lds + row * C::O_PITCH + 16 * chunk);
-            *reinterpret_cast<u32x4*>(o_base + (size_t)q * o_stride + 8 * chunk) = bits;
+    for (int pass = 0; pass < C::BM * ROW_CHUNKS / C::THREADS; ++pass) {
+        const int piece = pass * C::THREADS + tid;
+        const int row = piece / ROW_CHUNKS;
+        const int chunk = piece % ROW_CHUNKS;
+        if (q0 + row < S) {
+            *reinterpret_cast<u32x4*>(o_base + (size_t)(q0 + row) * o_stride + 8 * chunk) =
+                *reinterpret_cast<const u32x4*>(lds + C::O_AT + row * C::O_PITCH + 16 * chunk);
         }
     }
 }
@@ -393,7 +440,7 @@ __global__ __launch_bounds__(512) void attention_forward_pingpong_kernel(
     bf16_t* __restrict__ output, float* __restrict__ logsumexp,
     const bf16_t* __restrict__ query, const bf16_t* __restrict__ key, const bf16_t* __restrict__ value,
     int sequence_length, int query_heads, int key_value_heads, int query_blocks, int batch_heads, int clusters,
-    float scale) {
+    int abreast, float scale) {
     using C = FwdConfig<DQK, DV, 8>;
     constexpr int BN = C::BN;
     constexpr int KSTEPS = DQK / 16;
@@ -420,6 +467,7 @@ __global__ __launch_bounds__(512) void attention_forward_pingpong_kernel(
     const int g = lane / 32;
     const int S = sequence_length;
 
+    __builtin_assume(abreast > 0);
     const int cluster = blockIdx.x % clusters;
     const int member = blockIdx.x / clusters;
     const int members = gridDim.x / clusters;
@@ -534,10 +582,10 @@ __global__ __launch_bounds__(512) void attention_forward_pingpong_kernel(
     };
 
     ForwardItem item, next_item;
-    if (!forward_item(0, member, members, cluster, clusters, cluster_heads, query_blocks, item)) {
+    if (!forward_item(0, member, members, cluster, clusters, cluster_heads, query_blocks, item, abreast)) {
         return;   // uniform over the workgroup
     }
-    bool has_next = forward_item(1, member, members, cluster, clusters, cluster_heads, query_blocks, next_item);
+    bool has_next = forward_item(1, member, members, cluster, clusters, cluster_heads, query_blocks, next_item, abreast);
 
     // ---- prologue of the first item: its queries and its tiles 0 and 1
     load_queries(item);
@@ -763,74 +811,78 @@ __global__ __launch_bounds__(512) void attention_forward_pingpong_kernel(
         }
         item = next_item;
         ++round;
-        has_next = forward_item(round + 1, member, members, cluster, clusters, cluster_heads, query_blocks, next_item);
+        has_next = forward_item(round + 1, member, members, cluster, clusters, cluster_heads, query_blocks, next_item, abreast);
     }
     if (group == 0) {
         workgroup_barrier();
     }
 }
 
-template <int DQK, int DV, int NWAVES>
-void launch_forward(bf16_t* output, float* logsumexp, const bf16_t* query, const bf16_t* key, const bf16_t* value,
-                    int batch_size, int sequence_length, int query_heads, int key_value_heads, float scale,
-                    hipStream_t stream) {
-    using C = FwdConfig<DQK, DV, NWAVES>;
+template <int DQK, int DV, int QG, int KG>
+void launch_forward_split(bf16_t* output, float* logsumexp, const bf16_t* query, const bf16_t* key, const bf16_t* value,
+                          int batch_size, int sequence_length, int query_heads, int key_value_heads, float scale,
+                          hipStream_t stream) {
+    using C = SplitConfig<DQK, DV, QG, KG>;
     const int query_blocks = (sequence_length + C::BM - 1) / C::BM;
-    const long long groups = (long long)batch_size * query_heads;
-    const long long grid = groups * query_blocks;
-    if (grid > 0x7fffffffLL) {
-        throw std::invalid_argument("attention forward: batch*heads*query_blocks exceeds the grid limit");
-    }
-    // per-lane byte offsets inside a key tile are 32-bit
-    if ((long long)key_value_heads * (DQK > DV ? DQK : DV) * 2 * C::BN > 0x7fffffffLL) {
-        throw std::invalid_argument("attention forward: key_value_heads * head size is too large");
-    }
-    auto kernel = attention_forward_kernel<DQK, DV, NWAVES>;
-    if (C::LDS_BYTES > 64 * 1024) {
-        static hip_common::OncePerDevice raised;
-        raised.run([&] {
-            HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS_BYTES));
-        });
-    }
-    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(C::THREADS), C::LDS_BYTES, stream, output, logsumexp, query,
-                       key, value, sequence_length, query_heads, key_value_heads, query_blocks, scale);
+    const long long grid = (long long)batch_size * query_heads * query_blocks;
+    auto kernel = attention_forward_split_kernel<DQK, DV, QG, KG>;
+    static hip_common::OncePerDevice raised;
+    raised.run([&] {
+        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS_BYTES));
+    });
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(C::THREADS), C::LDS_BYTES, stream, output, logsumexp, query, key,
+                       value, sequence_length, query_heads, key_value_heads,
+                       index_math::split_order(batch_size, query_heads, key_value_heads, query_blocks), scale);
     HIP_CHECK(hipGetLastError());
+}
+
+// How the persistent kernel would take a problem: its clusters and workgroups, and what index_math::forward_choice
+// makes of them.  Worked out once for the shape a thread asked about last (a few microseconds for a long sequence).
+struct PingPongPlan {
+    int clusters;
+    int grid;
+    index_math::ForwardChoice choice;
+};
+
+PingPongPlan pingpong_plan(long long batch_heads, int sequence_length) {
+    struct Memory {
+        long long batch_heads = 0;
+        int sequence_length = 0, compute_units = 0;
+        PingPongPlan plan = {};
+    };
+    thread_local Memory last;
+    const int compute_units = hip_common::compute_units_of_current_device();
+    if (last.batch_heads != batch_heads || last.sequence_length != sequence_length || last.compute_units != compute_units) {
+        // one workgroup per compute unit (the LDS footprint admits no second one)
+        PingPongPlan plan;
+        plan.clusters = (batch_heads % PingPong::CLUSTERS == 0 && compute_units >= PingPong::CLUSTERS) ? PingPong::CLUSTERS : 1;
+        const long long query_blocks = (sequence_length + 255) / 256;
+        const long long members = std::min<long long>(compute_units / plan.clusters, batch_heads / plan.clusters * query_blocks);
+        plan.grid = (int)(members * plan.clusters);
+        plan.choice = index_math::forward_choice((int)members, plan.clusters, (int)(batch_heads / plan.clusters), sequence_length);
+        last = Memory{batch_heads, sequence_length, compute_units, plan};
+    }
+    return last.plan;
 }
 
 template <int DQK, int DV>
 void launch_forward_pingpong(bf16_t* output, float* logsumexp, const bf16_t* query, const bf16_t* key,
                              const bf16_t* value, int batch_size, int sequence_length, int query_heads,
-                             int key_value_heads, float scale, hipStream_t stream) {
+                             int key_value_heads, const PingPongPlan& plan, float scale, hipStream_t stream) {
     using C = FwdConfig<DQK, DV, 8>;
     constexpr int LDS_BYTES = PingPong::K_SLOTS * C::K_BYTES + PingPong::V_SLOTS * C::V_BYTES + PingPong::O_BYTES;
     static_assert(LDS_BYTES <= 160 * 1024, "the tile slots and the output staging rows must fit the LDS");
     const int query_blocks = (sequence_length + C::BM - 1) / C::BM;
-    const long long batch_heads = (long long)batch_size * query_heads;
-    if (batch_heads * query_blocks > 0x7fffffffLL) {
-        throw std::invalid_argument("attention forward: batch*heads*query_blocks exceeds the item limit");
-    }
-    if ((long long)key_value_heads * (DQK > DV ? DQK : DV) * 2 * C::BN > 0x7fffffffLL) {
-        throw std::invalid_argument("attention forward: key_value_heads * head size is too large");
-    }
-    // one workgroup per compute unit (the LDS footprint admits no second one)
-    const int compute_units = hip_common::compute_units_of_current_device();
-    const int clusters = (batch_heads % PingPong::CLUSTERS == 0 && compute_units >= PingPong::CLUSTERS)
-                             ? PingPong::CLUSTERS : 1;
-    long long grid = compute_units / clusters * clusters;
-    const long long items_per_cluster = batch_heads / clusters * query_blocks;
-    if (grid / clusters > items_per_cluster) {
-        grid = items_per_cluster * clusters;
-    }
     auto kernel = attention_forward_pingpong_kernel<DQK, DV>;
     static hip_common::OncePerDevice raised;
     raised.run([&] {
         HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES));
     });
-    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(C::THREADS), LDS_BYTES, stream, output, logsumexp, query,
-                       key, value, sequence_length, query_heads, key_value_heads, query_blocks, (int)batch_heads,
-                       clusters, scale);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)plan.grid), dim3(C::THREADS), LDS_BYTES, stream, output, logsumexp, query,
+                       key, value, sequence_length, query_heads, key_value_heads, query_blocks, batch_size * query_heads,
+                       plan.clusters, plan.choice.abreast, scale);
     HIP_CHECK(hipGetLastError());
 }
 
@@ -840,28 +892,61 @@ void attention_forward_dispatch(bf16_t* output, float* logsumexp, const bf16_t* 
                                 const bf16_t* value, int batch_size, int sequence_length, int query_heads,
                                 int key_value_heads, int qk_head_size, int v_head_size, float scale,
                                 hipStream_t stream) {
-    // Few, large workgroups (256 queries) when there is enough work to fill the
-    // chip; 128-query workgroups otherwise so that short problems still spread.
-    const long long rows = (long long)batch_size * query_heads * sequence_length;
-    // the persistent kernel streams two tiles ahead across items: every item needs two tiles
-    const bool large = rows >= 256LL * 256 * 2 && sequence_length >= 128;
-#define DSCUDA_FWD_CASE(DQK, DV)                                                                                  \
-    if (qk_head_size == DQK && v_head_size == DV) {                                                               \
-        if constexpr (DV >= 128) {                                                                                \
-            if (large) {                                                                                          \
-                launch_forward_pingpong<DQK, DV>(output, logsumexp, query, key, value, batch_size,               \
-                                                 sequence_length, query_heads, key_value_heads, scale, stream);   \
-                return;                                                                                           \
-            }                                                                                                     \
-        }                                                                                                         \
-        launch_forward<DQK, DV, 4>(output, logsumexp, query, key, value, batch_size, sequence_length,             \
-                                   query_heads, key_value_heads, scale, stream);                                  \
-        return;                                                                                                   \
+    // Offsets of the lanes inside a tile of 128 rows (keys or queries) are 32-bit, items and workgroups are counted in ints.
+    const long long widest = 2LL * std::max(qk_head_size, v_head_size) * std::min(sequence_length, 128);
+    if (widest * std::max(query_heads, key_value_heads) > 0xffffffffLL) {
+        throw std::invalid_argument("attention forward: heads * head size is too large");
     }
+    const long long batch_heads = (long long)batch_size * query_heads;
+    const long long blocks64 = (sequence_length + 63LL) / 64, blocks128 = (sequence_length + 127LL) / 128;
+    if (batch_heads * blocks64 > 0x7fffffffLL) {
+        throw std::invalid_argument("attention forward: batch*heads*query_blocks exceeds the grid limit");
+    }
+    const int compute_units = hip_common::compute_units_of_current_device();
+#define DSCUDA_FWD_SPLIT(DQK, DV, QG, KG)                                                                          \
+    launch_forward_split<DQK, DV, QG, KG>(output, logsumexp, query, key, value, batch_size, sequence_length,       \
+                                          query_heads, key_value_heads, scale, stream)
+#define DSCUDA_FWD_CASE(DQK, DV)                                                                                   \
+    if (qk_head_size == DQK && v_head_size == DV) {                                                                \
+        if (persistent) {                                                                                          \
+            launch_forward_pingpong<DQK, DV>(output, logsumexp, query, key, value, batch_size, sequence_length,    \
+                                             query_heads, key_value_heads, plan, scale, stream);                   \
+        } else if (quarters) {                                                                                     \
+            DSCUDA_FWD_SPLIT(DQK, DV, 2, 4);                                                                       \
+        } else {                                                                                                   \
+            DSCUDA_FWD_SPLIT(DQK, DV, 4, 2);                                                                       \
+        }                                                                                                          \
+        return;                                                                                                    \
+    }
+    if (qk_head_size == 64 && v_head_size == 64) {
+        // 64 queries per workgroup at any size (128: 22.7 against 16.3 us for 8 heads of 2048 tokens, 203 against 205 us
+        // for 64 heads of 4352); with 64 columns the softmax outweighs the products, and the persistent kernel's phases
+        // do not come out even.
+        DSCUDA_FWD_SPLIT(64, 64, 2, 4);
+        return;
+    }
+    // Persistent kernel or split keys: the tiles of the busiest workgroup against the steps (128 queries x 128 keys, 1.1
+    // tiles each, start and end of a workgroup 2.5 more) of the mean or the longest one.  Both sides of the line, split
+    // against persistent: 32 heads of 5120 tokens 269 / 254 us, 128 heads of 1152 tokens 78 / 81, 64 of 2048 100 / 91,
+    // 32 of 3313 121 / 118 (estimated), 16 of 1000 21 / 41 (estimated).
+    const double mean_steps = (double)batch_heads * (0.5 * blocks128 * (blocks128 + 1) + 2.5 * blocks128) / compute_units;
+    const double split_cost = 1.1 * std::max(mean_steps, blocks128 + 2.5);
+    PingPongPlan plan = {};
+    bool persistent = false;
+    // the persistent kernel streams two tiles ahead across items: every item needs two tiles
+    if (sequence_length >= 128 && mean_steps > blocks128) {
+        plan = pingpong_plan(batch_heads, sequence_length);
+        persistent = plan.choice.cost <= split_cost;
+    }
+    // 64 queries instead of 128 while that finds idle compute units, for long sequences up to one workgroup of 128 per
+    // unit (64 / 128: 16 heads of 1000 tokens 16.3 / 20.6 us, 8 of 4096 47.5 / 57.6, 64 of 512 16.3 / 15.4, 32 of 1500
+    // 41.5 / 32.0).
+    const long long workgroups = batch_heads * blocks128;
+    const bool quarters = 2 * workgroups <= compute_units || (workgroups <= compute_units && sequence_length >= 1024);
     DSCUDA_FWD_CASE(192, 128)
     DSCUDA_FWD_CASE(128, 128)
-    DSCUDA_FWD_CASE(64, 64)
 #undef DSCUDA_FWD_CASE
+#undef DSCUDA_FWD_SPLIT
     throw std::invalid_argument("attention forward: unsupported head sizes (d_qk,d_v) = (" +
                                 std::to_string(qk_head_size) + "," + std::to_string(v_head_size) + ")");
 }

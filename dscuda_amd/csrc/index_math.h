@@ -148,23 +148,157 @@ struct ForwardItem {
 
 // Item `round` of workgroup `member` (of `members`) of a cluster that owns
 // `cluster_heads` (batch, head) pairs (pairs cluster, cluster + clusters, ...);
-// false past the end of the list.  Inside a cluster the items are laid out two
-// heads at a time (one if the count is odd), blocks from the heaviest (last) to
+// false past the end of the list.  Inside a cluster the items are laid out
+// `abreast` heads at a time (0: two, or one if the count is odd), blocks from the heaviest (last) to
 // the lightest, and cut into rounds of one item per workgroup; odd rounds are
 // handed out in reverse.
 DSCUDA_HOST_DEVICE inline bool forward_item(int round, int member, int members, int cluster, int clusters,
-                                            int cluster_heads, int query_blocks, ForwardItem& item) {
+                                            int cluster_heads, int query_blocks, ForwardItem& item, int abreast = 0) {
     const int position = (round & 1) ? members - 1 - member : member;
     const int index = round * members + position;
     if (index >= cluster_heads * query_blocks) {
         return false;
     }
-    const int interleave = (cluster_heads % 2 == 0) ? 2 : 1;
+    const int interleave = abreast > 0 ? abreast : (cluster_heads % 2 == 0) ? 2 : 1;
     const int group = index / (interleave * query_blocks);
     const int rest = index % (interleave * query_blocks);
     item.batch_head = cluster + clusters * (interleave * group + rest % interleave);
     item.query_block = query_blocks - 1 - rest / interleave;
     return true;
+}
+
+// Tiles (64 keys x 256 queries) of the busiest workgroup of a cluster, an item's start and end counted as three more.
+constexpr int FORWARD_ITEM_TILES = 3;
+
+inline int forward_makespan(int members, int clusters, int cluster_heads, int sequence_length, int abreast) {
+    const int query_blocks = (sequence_length + 255) / 256;
+    int longest = 0;
+    for (int member = 0; member < members; ++member) {
+        int tiles = 0;
+        ForwardItem item;
+        for (int round = 0; forward_item(round, member, members, 0, clusters, cluster_heads, query_blocks, item, abreast); ++round) {
+            const int end = (item.query_block + 1) * 256;
+            tiles += ((end < sequence_length ? end : sequence_length) + 63) / 64 + FORWARD_ITEM_TILES;
+        }
+        if (tiles > longest) longest = tiles;
+    }
+    return longest;
+}
+
+// How many heads a cluster takes abreast, and the cost of the launch in tiles.  Two at a time keep few keys live in the
+// L2; where the rounds then do not come out even (2.5 rounds of items: the busiest workgroup has 1.4 times the mean),
+// more heads sorted together do: 32 heads of 7168 tokens 570 -> 463 us, 128 heads of 1700 tokens 168 -> 147 us with all
+// of a cluster's heads abreast.  Each doubling costs some 1.5 % through the L2 (128 heads of 4096 tokens, already even:
+// 642 us with two, 652 with eight, 676 with sixteen).
+struct ForwardChoice {
+    int abreast;
+    double cost;
+};
+
+inline ForwardChoice forward_choice(int members, int clusters, int cluster_heads, int sequence_length) {
+    const long long query_blocks = (sequence_length + 255) / 256;
+    long long total = 0;   // of a head
+    for (long long block = 0; block < query_blocks; ++block) {
+        const long long end = (block + 1) * 256 < sequence_length ? (block + 1) * 256 : sequence_length;
+        total += (end + 63) / 64 + FORWARD_ITEM_TILES;
+    }
+    const double mean = (double)total * cluster_heads / members;
+    ForwardChoice best = {cluster_heads % 2 == 0 ? 2 : 1, 0.0};
+    best.cost = forward_makespan(members, clusters, cluster_heads, sequence_length, best.abreast);
+    double penalty = 1.0;
+    for (int abreast = 4; best.cost > 1.03 * mean && abreast / 2 < cluster_heads; abreast *= 2) {
+        penalty += 0.015;
+        const int heads = abreast < cluster_heads ? abreast : cluster_heads;
+        if (cluster_heads % heads != 0) continue;
+        const double cost = penalty * forward_makespan(members, clusters, cluster_heads, sequence_length, heads);
+        if (cost < best.cost) best = ForwardChoice{heads, cost};
+    }
+    return best;
+}
+
+// ---- work order of the split-key forward kernel ----------------------------------
+// Division by a constant the host knows, as a multiply and a shift (n < 2^31).
+struct FastDivision {
+    unsigned multiplier;
+    unsigned shift;
+    unsigned divisor;
+};
+
+inline FastDivision fast_division(unsigned divisor) {
+    FastDivision division;
+    division.divisor = divisor;
+    division.shift = 0;
+    while ((1ULL << division.shift) < divisor) ++division.shift;
+    division.multiplier = (unsigned)((((1ULL << division.shift) - divisor) << 32) / divisor + 1);
+    return division;
+}
+
+DSCUDA_HOST_DEVICE inline unsigned divide(unsigned n, const FastDivision& by) {
+    return (unsigned)(((((unsigned long long)n * by.multiplier) >> 32) + n) >> by.shift);
+}
+
+// Items (batch, query head, query block), numbered so that what runs at one time shares keys and ends together.
+// Workgroups go to the XCDs round-robin by linear id and every XCD has an L2 of its own, so the query heads that read
+// one key/value head stay on one XCD; with too few key/value heads for that, query heads are dealt to the XCDs one by
+// one; with too few of those there is no dealing.  An XCD takes a number of its groups together, the longest query
+// blocks of all of them first: all its groups while they make at most four rounds of its compute units (what decides
+// then is that no long block starts late), beyond that two rounds' worth at a time (what decides then is that few
+// heads' keys are live in the L2).
+struct SplitOrder {
+    FastDivision turn;       // items an XCD takes together
+    FastDivision abreast;    // (group, query head) pairs among them
+    FastDivision members;    // query heads of a group
+    FastDivision groups;     // groups per batch element
+    FastDivision sharing;    // query heads per key/value head
+    int clusters;
+    int together;            // groups an XCD takes together
+    int query_blocks;
+};
+
+inline SplitOrder split_order(int batch, int query_heads, int key_value_heads, int query_blocks) {
+    constexpr int XCDS = 8, UNITS = 32;
+    SplitOrder order;
+    const int sharing = query_heads / key_value_heads;
+    const bool by_group = (long long)batch * key_value_heads % XCDS == 0;
+    order.clusters = by_group || (long long)batch * query_heads % XCDS == 0 ? XCDS : 1;
+    const int members = by_group ? sharing : 1;
+    const long long groups = (long long)batch * query_heads / members / order.clusters;   // of an XCD
+    const long long inner = (long long)members * query_blocks;
+    long long together = groups;
+    if (order.clusters > 1 && groups * inner > 4 * UNITS) {
+        together = (2 * UNITS + inner - 1) / inner;
+        while (groups % together != 0) ++together;
+    }
+    order.together = (int)together;
+    order.turn = fast_division((unsigned)(together * inner));
+    order.abreast = fast_division((unsigned)(together * members));
+    order.members = fast_division((unsigned)members);
+    order.groups = fast_division((unsigned)(query_heads / members));
+    order.sharing = fast_division((unsigned)sharing);
+    order.query_blocks = query_blocks;
+    return order;
+}
+
+struct SplitItem {
+    int batch, head, key_value_head, query_block;
+};
+
+DSCUDA_HOST_DEVICE inline SplitItem split_item(unsigned linear, const SplitOrder& order) {
+    SplitItem item;
+    const unsigned slot = order.clusters > 1 ? linear / 8 : linear;
+    const unsigned turn = divide(slot, order.turn);
+    const unsigned rest = slot - turn * order.turn.divisor;
+    const unsigned rank = divide(rest, order.abreast);
+    const unsigned pair = rest - rank * order.abreast.divisor;
+    const unsigned group_of_turn = divide(pair, order.members);
+    const unsigned local = turn * (unsigned)order.together + group_of_turn;
+    const unsigned group = order.clusters > 1 ? linear % 8 + 8 * local : local;
+    const unsigned batch = divide(group, order.groups);
+    item.batch = (int)batch;
+    item.head = (int)((group - batch * order.groups.divisor) * order.members.divisor + pair - group_of_turn * order.members.divisor);
+    item.key_value_head = (int)divide((unsigned)item.head, order.sharing);
+    item.query_block = order.query_blocks - 1 - (int)rank;
+    return item;
 }
 
 // ---- decode: tile loads -------------------------------------------------------

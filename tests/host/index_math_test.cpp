@@ -551,7 +551,52 @@ void check_decode_layout() {
     EXPECT(decode_layout(5, 128, 1, 256, ROWS, RANK).whole_sequences == 1, "splits 1 must not cut");
 }
 
+// ---- split-key forward: division by multiplication, every (batch, head, block) exactly once with its key/value head;
+// persistent forward: any number of heads abreast covers every item once, and the choice is never worse than the default
+void check_split_order() {
+    for (unsigned divisor = 1; divisor < 2000; ++divisor) {
+        const FastDivision by = fast_division(divisor);
+        for (unsigned n : {0u, 1u, divisor - 1, divisor, divisor + 1, 7 * divisor - 1, 7 * divisor, 123456789u, 0x7ffffffeu, 0x7fffffffu}) {
+            EXPECT(divide(n, by) == n / divisor, "%u / %u", n, divisor);
+        }
+    }
+    for (int batch : {1, 2, 3, 8}) {
+        for (int kv : {1, 2, 3, 4, 8}) {
+            for (int sharing : {1, 2, 3, 8}) {
+                for (int blocks : {1, 2, 5, 17, 70}) {
+                    const SplitOrder order = split_order(batch, kv * sharing, kv, blocks);
+                    std::vector<int> seen(batch * kv * sharing * blocks, 0);
+                    for (int i = 0; i < (int)seen.size(); ++i) {
+                        const SplitItem item = split_item((unsigned)i, order);
+                        EXPECT(item.batch < batch && item.head < kv * sharing && item.query_block >= 0 && item.query_block < blocks &&
+                                   item.key_value_head == item.head / sharing, "B %d kv %d sharing %d item %d", batch, kv, sharing, i);
+                        ++seen[(item.batch * kv * sharing + item.head) * blocks + item.query_block];
+                    }
+                    for (int count : seen) EXPECT(count == 1, "B %d kv %d sharing %d blocks %d", batch, kv, sharing, blocks);
+                }
+            }
+        }
+    }
+    for (int heads : {1, 2, 3, 4, 6, 16}) {
+        for (int sequence : {128, 700, 1152, 4096, 5120}) {
+            const int blocks = (sequence + 255) / 256, members = std::min(32, heads * blocks);
+            const ForwardChoice choice = forward_choice(members, 8, heads, sequence);
+            EXPECT(heads % choice.abreast == 0, "%d heads, %d abreast", heads, choice.abreast);
+            EXPECT(choice.cost <= forward_makespan(members, 8, heads, sequence, 0), "%d heads of %d", heads, sequence);
+            std::vector<int> seen(heads * blocks, 0);
+            for (int member = 0; member < members; ++member) {
+                ForwardItem item;
+                for (int round = 0; forward_item(round, member, members, 3, 8, heads, blocks, item, choice.abreast); ++round) {
+                    ++seen[(item.batch_head - 3) / 8 * blocks + item.query_block];
+                }
+            }
+            for (int count : seen) EXPECT(count == 1, "%d heads of %d, %d abreast", heads, sequence, choice.abreast);
+        }
+    }
+}
+
 int main() {
+    check_split_order();
     check_swizzle<128>();
     check_swizzle<256>();
     check_swizzle<384>();

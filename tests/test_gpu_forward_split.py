@@ -1,0 +1,63 @@
+"""The split-key and the persistent forward at the edges of their tiles (32, 64 and 128 queries or keys), of their work
+order (head counts that are dealt to the XCDs by group, by head or not at all) and of the line between them."""
+
+import pytest
+import torch
+
+from dscuda_amd.harness import configs, ops
+from oracle import attention_oracle as oracle
+from tests.parity import announce, assert_close_bf16, assert_close_lse
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("batch,seq,heads", [
+    (1, 31, 1), (1, 32, 2), (3, 33, 1), (1, 63, 3), (1, 64, 8), (2, 65, 4), (1, 127, 5), (1, 128, 16), (1, 129, 3),
+    (1, 191, 2), (2, 193, 8), (1, 256, 3), (1, 320, 1),                      # 64 queries per workgroup
+    (1, 130, 70), (2, 129, 68), (1, 385, 40), (1, 257, 96),                  # 128
+    (1, 1024, 128), (1, 640, 160),                                           # persistent
+])
+def test_prefill_tile_edges(cuda, batch, seq, heads):
+    q, k, v, scale = configs.mla_prefill_inputs(batch, seq, heads, seed=seq)
+    announce("prefill tile edges", dict(B=batch, S=seq, H=heads))
+    out, lse = ops.mla_prefill_forward(q.to(cuda), k.to(cuda), v.to(cuda), scale)
+    sample = sorted({0, heads // 2, heads - 1})
+    expected, expected_lse = oracle.causal_attention_forward(q, k, v, scale, heads=sample)
+    assert_close_bf16("O", out[:, :, sample], expected)
+    assert_close_lse("LSE", lse[:, sample], expected_lse)
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("batch,tokens,kv_heads,sharing", [
+    (1, 192, 8, 3), (2, 64, 4, 1), (1, 128, 1, 8), (3, 320, 1, 5), (1, 448, 24, 4),
+])
+def test_flash_work_orders(cuda, batch, tokens, kv_heads, sharing, dim):
+    heads = kv_heads * sharing
+    q, k, v, scale = configs.flash_forward_inputs(batch, tokens, heads, kv_heads, dim, seed=tokens, factor=0.5)
+    announce("flash work orders", dict(B=batch, T=tokens, Hq=heads, Hkv=kv_heads, D=dim))
+    out, lse = ops.flash_forward(q.to(cuda), k.to(cuda), v.to(cuda), scale)
+    expected, expected_lse = oracle.causal_attention_forward(q, k, v, scale)
+    assert_close_bf16("O", out, expected)
+    assert_close_lse("LSE", lse, expected_lse)
+
+
+@pytest.mark.parametrize("heads", [2, 72])   # 64 and 128 queries per workgroup
+def test_parts_with_distant_maxima(cuda, heads):
+    """Scores that grow by thousands along the keys: the key groups of a workgroup end with maxima far apart, and rows
+    near a tile's start have no visible key in some of them."""
+    seq = 300
+    g = torch.Generator().manual_seed(3)
+    direction = torch.randn(192, generator=g)
+    q = (direction + 0.1 * torch.randn(1, seq, heads, 192, generator=g)).bfloat16()
+    growth = torch.linspace(0, 1, seq)[None, :, None, None]
+    k = (direction * growth + 0.05 * torch.randn(1, seq, heads, 192, generator=g)).bfloat16()
+    v = torch.randn(1, seq, heads, 128, generator=g).bfloat16()
+    announce("distant maxima", dict(H=heads))
+    out, lse = ops.mla_prefill_forward(q.to(cuda), k.to(cuda), v.to(cuda), 4.0)
+    expected, expected_lse = oracle.causal_attention_forward(q, k, v, 4.0)
+    assert expected_lse.max() > 500
+    # the weights carry the fp32 error of scores this large: twelve partial sums and the scaling, 2^-24 of the score each
+    weights = 16 * 2 ** -24 * expected_lse.abs().max().item()
+    largest = v.float().abs().max().item()
+    assert (out.cpu().float() - expected).abs().max().item() <= (2 * 2 ** -9 + weights) * largest
+    assert ((lse.cpu() - expected_lse).abs() / expected_lse.abs().clamp_min(1)).max().item() <= 1e-5
