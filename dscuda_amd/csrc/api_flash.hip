@@ -61,7 +61,8 @@ std::size_t flash_attention_backward_workspace_elements(int batch_size, int sequ
         query_heads % key_value_heads != 0 || (head_size != 64 && head_size != 128)) {
         return 0;
     }
-    return attention_backward_workspace_elements(batch_size, sequence_length, query_heads, key_value_heads);
+    return attention_backward_workspace_elements(batch_size, sequence_length, query_heads, key_value_heads, head_size,
+                                                 head_size);
 }
 
 void flash_attention_backward_set_workspace_limit(std::size_t bytes) {

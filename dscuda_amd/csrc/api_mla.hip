@@ -174,11 +174,11 @@ void mla_prefill_forward_cuda(__hip_bfloat16* output, float* logsumexp, const __
 }
 
 std::size_t mla_prefill_backward_workspace_elements(int batch_size, int sequence_length, int heads,
-                                                    int /*qk_head_size*/, int /*v_head_size*/) {
+                                                    int qk_head_size, int v_head_size) {
     if (batch_size <= 0 || sequence_length <= 0 || heads <= 0) {
         return 0;
     }
-    return attention_backward_workspace_elements(batch_size, sequence_length, heads, heads);
+    return attention_backward_workspace_elements(batch_size, sequence_length, heads, heads, qk_head_size, v_head_size);
 }
 
 void mla_prefill_backward_set_workspace_limit(std::size_t bytes) {

@@ -16,8 +16,11 @@
 //                    dV += P^T dO,  dK += dS^T Q
 //                and leaves dS (bf16, before the scale factor) in the workspace,
 //                one 16 KB block per (key block, query tile)
+//                Few pairs would leave compute units idle: their walks are cut into
+//                parts whose fp32 sums go to the workspace
 //   dQ           the separate accumulation pass: a plain product dQ = scale * dS K
-//                over the stored dS blocks, nothing is recomputed
+//                over the stored dS blocks, nothing is recomputed.  Workgroups of
+//                the same launch add up the parts of cut walks, in order
 //
 // Operand feeds.  Q and dO tiles arrive by global_load_lds and are stored once,
 // row-major.  Both orientations are read from that one copy: 16-byte row reads
@@ -93,15 +96,16 @@ __device__ __forceinline__ void clear(f32x16& value) {
 
 // ---- statistics ---------------------------------------------------------------
 
-// One 16-lane group per (b, s, h) row of the sequence padded to whole query tiles.
+// One group of DV / 8 lanes per (b, s, h) row of the sequence padded to whole query tiles.
 template <int DV>
 __global__ __launch_bounds__(256) void attention_backward_statistics_kernel(
     float* __restrict__ statistics, const bf16_t* __restrict__ output_gradient, const bf16_t* __restrict__ output,
     const float* __restrict__ logsumexp, int batch_size, int sequence_length, int heads, int query_tiles) {
     const long long padded = (long long)query_tiles * QTILE;
     const long long rows = (long long)batch_size * padded * heads;
-    const long long row = (long long)blockIdx.x * 16 + threadIdx.x / 16;
-    const int part = threadIdx.x % 16;
+    constexpr int LANES = DV / 8;
+    const long long row = (long long)blockIdx.x * (256 / LANES) + threadIdx.x / LANES;
+    const int part = threadIdx.x % LANES;
     if (row >= rows) {
         return;
     }
@@ -112,20 +116,17 @@ __global__ __launch_bounds__(256) void attention_backward_statistics_kernel(
     float lse2 = INFINITY;
     if (s < sequence_length) {
         const long long source = ((b * sequence_length + s) * heads + h) * DV;
+        const u32x4 x = *reinterpret_cast<const u32x4*>(output_gradient + source + part * 8);
+        const u32x4 y = *reinterpret_cast<const u32x4*>(output + source + part * 8);
 #pragma unroll
-        for (int c = part * 8; c < DV; c += 128) {
-            const u32x4 x = *reinterpret_cast<const u32x4*>(output_gradient + source + c);
-            const u32x4 y = *reinterpret_cast<const u32x4*>(output + source + c);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                sum += bf16_bits_to_float(x[j] & 0xffffu) * bf16_bits_to_float(y[j] & 0xffffu);
-                sum += bf16_bits_to_float(x[j] >> 16) * bf16_bits_to_float(y[j] >> 16);
-            }
+        for (int j = 0; j < 4; ++j) {
+            sum += bf16_bits_to_float(x[j] & 0xffffu) * bf16_bits_to_float(y[j] & 0xffffu);
+            sum += bf16_bits_to_float(x[j] >> 16) * bf16_bits_to_float(y[j] >> 16);
         }
         lse2 = logsumexp[(b * heads + h) * sequence_length + s] * LOG2E;
     }
 #pragma unroll
-    for (int offset = 1; offset < 16; offset <<= 1) sum += __shfl_xor(sum, offset);
+    for (int offset = 1; offset < LANES; offset <<= 1) sum += __shfl_xor(sum, offset);
     if (part == 0) {
         float* target = statistics + ((b * heads + h) * query_tiles + s / QTILE) * STAT_FLOATS + s % QTILE;
         target[0] = lse2;
@@ -156,6 +157,43 @@ __global__ __launch_bounds__(256) void attention_backward_statistics_kernel(
 
 constexpr int KV_THREADS = 512;
 
+// Which part of which key block's walk is workgroup `item` of a pair.  A lane holds the number of parts of one key
+// block: 64 of them at a time instead of a chain of divisions.
+__device__ __forceinline__ void locate_part(int item, int key_blocks, int query_tiles, int sharing, int part_steps,
+                                            int lane, int& kb, int& part) {
+    int before = 0;   // parts of the blocks ahead of `first`
+    for (int first = 0; first < key_blocks; first += 64) {
+        const int block = first + lane;
+        const int parts =
+            block < key_blocks ? index_math::walk_parts((query_tiles - 2 * block) * sharing, part_steps) : 0;
+        int end = before + parts;
+#pragma unroll
+        for (int distance = 1; distance < 64; distance <<= 1) {
+            const int below = __shfl_up(end - before, distance);
+            if (lane >= distance) end += below;
+        }
+        const unsigned long long holds = __ballot(end > item);
+        if (holds != 0) {
+            const int found = __builtin_ctzll(holds);
+            kb = first + found;
+            part = item - (__builtin_amdgcn_readlane(end, found) - __builtin_amdgcn_readlane(parts, found));
+            return;
+        }
+        before = __builtin_amdgcn_readlane(end, 63);
+    }
+}
+
+// Accumulators of 32 keys, as the MFMA leaves them, to rows of COLUMNS floats: 128 bytes of two rows an instruction.
+template <int BLOCKS, int COLUMNS>
+__device__ __forceinline__ void store_partial(float* rows, const f32x16 (&sums)[BLOCKS], int lq, int g) {
+    float* target = rows + 4 * g * COLUMNS + lq;
+#pragma unroll
+    for (int d = 0; d < BLOCKS; ++d) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) target[(8 * (i / 4) + i % 4) * COLUMNS + 32 * d] = sums[d][i];
+    }
+}
+
 template <int DQK, int DV>
 struct KeyValueGradConfig {
     static constexpr int Q_ROW = 2 * DQK;
@@ -177,9 +215,10 @@ struct KeyValueGradConfig {
 template <int DQK, int DV>
 __global__ __launch_bounds__(KV_THREADS) void attention_key_value_gradient_kernel(
     bf16_t* __restrict__ key_gradient, bf16_t* __restrict__ value_gradient, unsigned char* __restrict__ ds_blocks,
-    const float* __restrict__ statistics, const bf16_t* __restrict__ output_gradient,
+    float* __restrict__ partial_sums, const float* __restrict__ statistics, const bf16_t* __restrict__ output_gradient,
     const bf16_t* __restrict__ query, const bf16_t* __restrict__ key, const bf16_t* __restrict__ value,
-    int sequence_length, int heads, int kv_heads, int key_blocks, int query_tiles, int first_pair, float scale) {
+    int sequence_length, int heads, int kv_heads, int key_blocks, int query_tiles, int first_pair, int part_steps,
+    int items, float scale) {
     using C = KeyValueGradConfig<DQK, DV>;
     constexpr int QK_STEPS = DQK / 16;
     constexpr int V_STEPS = DV / 16;
@@ -205,20 +244,23 @@ __global__ __launch_bounds__(KV_THREADS) void attention_key_value_gradient_kerne
     // Every key block walks the tiles from the last one down to its diagonal: blocks
     // started together then read the same tile at the same time, and one fetch from
     // memory serves them all.
-    int bh, kb;
+    //
+    // A pair is `items` workgroups: its key blocks, or, where part_steps is not zero, the
+    // parts their walks are cut into (choose_walk_cut), those of key block 0 first.
+    int bh, item;
     {
         constexpr int XCDS = 8;
-        const int pairs = gridDim.x / key_blocks;
+        const int pairs = gridDim.x / items;
         if (pairs % XCDS == 0) {
             const int slot = blockIdx.x / XCDS;
-            bh = blockIdx.x % XCDS + XCDS * (slot / key_blocks);
-            kb = slot % key_blocks;
+            bh = blockIdx.x % XCDS + XCDS * (slot / items);
+            item = slot % items;
         } else {
-            bh = blockIdx.x / key_blocks;
-            kb = blockIdx.x % key_blocks;
+            bh = blockIdx.x / items;
+            item = blockIdx.x % items;
         }
     }
-    // The launch covers the (batch, key/value head) pairs first_pair .. first_pair + gridDim.x / key_blocks - 1.
+    // The launch covers the (batch, key/value head) pairs first_pair .. first_pair + gridDim.x / items - 1.
     // `heads` query heads share `kv_heads` key/value heads: query heads h * sharing .. + sharing - 1 read key/value
     // head h, and this workgroup walks the query tiles of each of them in turn, all into the same dK / dV
     // accumulators.  The dS blocks of member m of pair first_pair + i sit at position i * sharing + m of the
@@ -229,6 +271,8 @@ __global__ __launch_bounds__(KV_THREADS) void attention_key_value_gradient_kerne
     const int b = bh / kv_heads;
     const int h = bh % kv_heads;          // key/value head
     const int first_query_head = h * sharing;
+    int kb = item, part = 0;
+    if (part_steps > 0) locate_part(item, key_blocks, query_tiles, sharing, part_steps, lane, kb, part);
     const int k0 = kb * KBLOCK;
     const int group_k0 = k0 + 32 * group;
     const int key_row = group_k0 + lq;
@@ -245,9 +289,23 @@ __global__ __launch_bounds__(KV_THREADS) void attention_key_value_gradient_kerne
     const float* stat_base = statistics + ((size_t)b * heads + first_query_head) * query_tiles * STAT_FLOATS;
     const unsigned lds_base = lds_offset_of(lds);
 
-    // Step `index` of the walk works on tile query_tiles - 1 - index % tiles of member index / tiles.
+    // Step i of a key block's walk works on tile query_tiles - 1 - i % tiles of member i / tiles.  This workgroup's
+    // steps are counted from 0 (`index`); the first is step `local` first_local of member first_member.
     const int tiles = query_tiles - 2 * kb;   // >= 1, per member
-    const int steps = tiles * sharing;
+    int steps = tiles * sharing;
+    int first_member = 0, first_local = 0;
+    bool whole = true;
+    if (part_steps > 0) {
+        const int parts = index_math::walk_parts(steps, part_steps);
+        const int begin = index_math::part_begin(steps, parts, part);
+        steps = index_math::part_begin(steps, parts, part + 1) - begin;
+        first_member = begin / tiles;
+        first_local = begin % tiles;
+        whole = parts == 1;
+    }
+    // the sums of a part leave as they are, 128 rows of dK | dV columns; attention_query_gradient_kernel adds them up
+    constexpr int PARTIAL_COLUMNS = DQK + DV;
+    float* partial = partial_sums + ((size_t)local_pair * items + item) * (KBLOCK * PARTIAL_COLUMNS);
 
     // Tiles are requested by the four value waves, each the same number of loads per
     // tile: a value wave then knows that all but its last REQUEST_LOADS loads have
@@ -286,9 +344,9 @@ __global__ __launch_bounds__(KV_THREADS) void attention_key_value_gradient_kerne
 
     if (!key_wave) {
         // ================= value wave: S, P, dV =================
-        request_tile(0, 0, 0);
+        request_tile(0, first_member, first_local);
         if (steps > 1) {
-            if (tiles > 1) request_tile(1, 0, 1); else request_tile(1, 1, 0);
+            if (first_local + 1 < tiles) request_tile(1, first_member, first_local + 1); else request_tile(1, first_member + 1, 0);
         }
         const bf16_t* k_base = key + ((size_t)b * S * kv_heads + h) * DQK;
         bf16x8 kf[QK_STEPS];   // B operand: column = key lq
@@ -415,16 +473,21 @@ __global__ __launch_bounds__(KV_THREADS) void attention_key_value_gradient_kerne
         wait_vector_memory<0>();
         workgroup_barrier();
         score_stream(0);
-        for (int member = 0, index = 0; member < sharing; ++member) {
-            for (int local = 0; local < tiles - 2; ++local, ++index) {
+        for (int member = first_member, local = first_local, index = 0; index < steps; ++member, local = 0) {
+            const int last = min(tiles, local + steps - index);   // of this member's tiles
+            for (; local < min(tiles - 2, last); ++local, ++index) {
                 value_tile(std::false_type{}, index, member, local);
             }
-            for (int local = max(tiles - 2, 0); local < tiles; ++local, ++index) {
+            for (; local < last; ++local, ++index) {
                 value_tile(std::true_type{}, index, member, local);
             }
         }
 
         // ---- epilogue: lane holds column 32*d + lq and keys 8*(i/4) + 4*g + i%4
+        if (!whole) {
+            store_partial<DV_BLOCKS, PARTIAL_COLUMNS>(partial + 32 * group * PARTIAL_COLUMNS + DQK, dv_acc, lq, g);
+            return;
+        }
         __syncthreads();
         unsigned char* dv_lds = lds + group * 32 * (C::DK_PITCH + C::DV_PITCH) + 32 * C::DK_PITCH;
 #pragma unroll
@@ -476,7 +539,7 @@ __global__ __launch_bounds__(KV_THREADS) void attention_key_value_gradient_kerne
         wait_vector_memory<0>();   // the V rows
         workgroup_barrier();       // tile 0 has landed
 
-        for (int index = 0, member = 0, local = 0; index < steps; ++index, ++local) {
+        for (int index = 0, member = first_member, local = first_local; index < steps; ++index, ++local) {
             if (local == tiles) {
                 local = 0;
                 ++member;
@@ -555,6 +618,10 @@ __global__ __launch_bounds__(KV_THREADS) void attention_key_value_gradient_kerne
         }
 
         // ---- epilogue: lane holds column 32*d + lq and keys 8*(i/4) + 4*g + i%4
+        if (!whole) {
+            store_partial<DK_BLOCKS, PARTIAL_COLUMNS>(partial + 32 * group * PARTIAL_COLUMNS, dk_acc, lq, g);
+            return;
+        }
         __syncthreads();
         unsigned char* dk_lds = lds + group * 32 * (C::DK_PITCH + C::DV_PITCH);
 #pragma unroll
@@ -604,13 +671,79 @@ struct QueryGradConfig {
 // waits for the older of its two requests in flight.
 constexpr int DQ_THREADS = 512;
 
-template <int DQK>
+// The partial dK and dV sums of a launch whose walks were cut, and where they go.
+struct PartialSums {
+    const float* sums;        // [pair][item][128 keys][dK columns | dV columns]
+    bf16_t* key_gradient;
+    bf16_t* value_gradient;
+    int items;                // per pair
+    int cut_blocks;           // key blocks 0 .. cut_blocks - 1 have more than one part
+    int part_steps;
+    int first_pair;           // (batch, key/value head) pair of the first partial sums
+};
+
+// Adds up the parts of dK and dV, in order, and rounds once.  A workgroup takes 512 groups of four columns of one
+// (pair, key block); reads and writes are whole cache lines.
+template <int DQK, int DV>
+__device__ __forceinline__ void add_partial_sums(const PartialSums& partial, int workgroup, int sequence_length,
+                                                 int kv_heads, int query_tiles, int sharing, float scale) {
+    constexpr int COLUMNS = DQK + DV;
+    constexpr int QUADS = COLUMNS / 4;
+    constexpr int PIECES = KBLOCK * QUADS / DQ_THREADS;
+    const int piece = workgroup % PIECES;
+    const int kb = workgroup / PIECES % partial.cut_blocks;
+    const int pair = workgroup / PIECES / partial.cut_blocks;
+    const int parts = index_math::walk_parts((query_tiles - 2 * kb) * sharing, partial.part_steps);
+    // items ahead of this key block's
+    int ahead = 0;
+    for (int block = threadIdx.x % 64; block < kb; block += 64) {
+        ahead += index_math::walk_parts((query_tiles - 2 * block) * sharing, partial.part_steps);
+    }
+#pragma unroll
+    for (int distance = 1; distance < 64; distance <<= 1) ahead += __shfl_xor(ahead, distance);
+
+    const int quad = piece * DQ_THREADS + threadIdx.x;
+    const int row = quad / QUADS;
+    const int column = 4 * (quad % QUADS);
+    const int key_row = kb * KBLOCK + row;
+    if (key_row >= sequence_length) {
+        return;
+    }
+    const float* source = partial.sums + (((size_t)pair * partial.items + ahead) * KBLOCK + row) * COLUMNS + column;
+    f32x4 sum = *reinterpret_cast<const f32x4*>(source);
+#pragma unroll 4
+    for (int part = 1; part < parts; ++part) {
+        sum += *reinterpret_cast<const f32x4*>(source + (size_t)part * (KBLOCK * COLUMNS));
+    }
+    const int bh = partial.first_pair + pair;
+    const size_t token = ((size_t)(bh / kv_heads) * sequence_length + key_row) * kv_heads + bh % kv_heads;
+    bf16_t* target;
+    if (column < DQK) {
+        sum *= scale;
+        target = partial.key_gradient + token * DQK + column;
+    } else {
+        target = partial.value_gradient + token * DV + (column - DQK);
+    }
+    u32x2 packed;
+    packed.x = pack_bf16(sum[0], sum[1]);
+    packed.y = pack_bf16(sum[2], sum[3]);
+    *reinterpret_cast<u32x2*>(target) = packed;
+}
+
+template <int DQK, int DV>
 __global__ __launch_bounds__(DQ_THREADS) void attention_query_gradient_kernel(
     bf16_t* __restrict__ query_gradient, const unsigned char* __restrict__ ds_blocks, const bf16_t* __restrict__ key,
     int sequence_length, int heads, int kv_heads, int query_blocks, int key_blocks, int query_tiles, int first_pair,
-    float scale) {
+    int workgroups, float scale, PartialSums partial) {
     using C = QueryGradConfig<DQK>;
     constexpr int WAVES = DQ_THREADS / 64;
+
+    // Workgroups past the query blocks add up the parts of dK and dV: independent of dQ, and a launch less.
+    if ((int)blockIdx.x >= workgroups) {
+        add_partial_sums<DQK, DV>(partial, blockIdx.x - workgroups, sequence_length, kv_heads, query_tiles,
+                                  heads / kv_heads, scale);
+        return;
+    }
 
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
 
@@ -622,10 +755,10 @@ __global__ __launch_bounds__(DQ_THREADS) void attention_query_gradient_kernel(
     const int S = sequence_length;
 
     int bh, rank;
-    xcd_order(blockIdx.x, gridDim.x / query_blocks, query_blocks, bh, rank);
+    xcd_order(blockIdx.x, workgroups / query_blocks, query_blocks, bh, rank);
     // the heads in the reverse of the order in which the first pass wrote their dS blocks: what it wrote last is
     // still in the memory-side cache
-    bh = gridDim.x / query_blocks - 1 - bh;
+    bh = workgroups / query_blocks - 1 - bh;
     const int jb = query_blocks - 1 - rank;   // heaviest (last) query blocks first
     const int local_pair = bh;                // position of this pair's dS blocks in the workspace
     bh += first_pair;
@@ -864,9 +997,12 @@ struct BackwardShape {
     long long pairs_per_launch;
     long long statistics_floats;   // every (batch, query head)
     long long ds_floats;           // one chunk of pairs, `sharing` query heads each
+    index_math::WalkCut cut;       // of the key blocks' walks
+    long long partial_floats;      // one chunk of pairs; 0 if no walk is cut
 };
 
-BackwardShape backward_shape(int batch_size, int sequence_length, int heads, int kv_heads) {
+BackwardShape backward_shape(int batch_size, int sequence_length, int heads, int kv_heads, int qk_head_size,
+                             int v_head_size) {
     BackwardShape shape;
     shape.key_blocks = (sequence_length + KBLOCK - 1) / KBLOCK;
     shape.query_tiles = (sequence_length + QTILE - 1) / QTILE;
@@ -880,6 +1016,17 @@ BackwardShape backward_shape(int batch_size, int sequence_length, int heads, int
     if (chunk < 1) chunk = 1;
     shape.pairs_per_launch = chunk < shape.pairs ? chunk : shape.pairs;
     shape.ds_floats = shape.pairs_per_launch * shape.sharing * ds_block_count(shape.key_blocks, shape.query_tiles) * DS_BLOCK_FLOATS;
+    // two workgroups of the first pass share a compute unit where their stages leave room in LDS
+    const int per_unit = 1;
+    shape.cut = index_math::choose_walk_cut(shape.pairs_per_launch, shape.key_blocks, shape.query_tiles, shape.sharing,
+                                            256 * per_unit);
+    shape.partial_floats = shape.cut.part_steps > 0
+        ? shape.pairs_per_launch * shape.cut.items * KBLOCK * (qk_head_size + v_head_size) : 0;
+    // the sums of the parts stay inside a budget that the caller has set
+    if (ds_budget_override.load(std::memory_order_relaxed) > 0 && 4 * (shape.ds_floats + shape.partial_floats) > ds_budget_bytes()) {
+        shape.cut = index_math::WalkCut{0, shape.key_blocks, 0};
+        shape.partial_floats = 0;
+    }
     return shape;
 }
 
@@ -890,10 +1037,11 @@ void launch_backward(bf16_t* query_gradient, bf16_t* key_gradient, bf16_t* value
                      int sequence_length, int heads, int kv_heads, float scale, hipStream_t stream) {
     using KC = KeyValueGradConfig<DQK, DV>;
     using QC = QueryGradConfig<DQK>;
-    const BackwardShape shape = backward_shape(batch_size, sequence_length, heads, kv_heads);
+    const BackwardShape shape = backward_shape(batch_size, sequence_length, heads, kv_heads, DQK, DV);
     const long long groups = (long long)batch_size * heads;
     const long long padded_rows = groups * shape.query_tiles * QTILE;
-    if ((padded_rows + 15) / 16 > 0x7fffffffLL || groups * shape.key_blocks > 0x7fffffffLL) {
+    constexpr int STATISTICS_ROWS = 256 / (DV / 8);   // per workgroup; padded_rows is a multiple of it
+    if (padded_rows / STATISTICS_ROWS > 0x7fffffffLL || groups * shape.key_blocks > 0x7fffffffLL) {
         throw std::invalid_argument("attention backward: problem exceeds the grid limit");
     }
     // per-lane byte offsets inside a tile are 32-bit
@@ -902,28 +1050,34 @@ void launch_backward(bf16_t* query_gradient, bf16_t* key_gradient, bf16_t* value
     }
     float* statistics = workspace;
     unsigned char* ds_blocks = reinterpret_cast<unsigned char*>(workspace + shape.statistics_floats);
+    float* partial_sums = workspace + shape.statistics_floats + shape.ds_floats;
     static hip_common::OncePerDevice prepared;
     prepared.run([] {
         raise_lds_limit(attention_key_value_gradient_kernel<DQK, DV>, KC::LDS_BYTES);
-        raise_lds_limit(attention_query_gradient_kernel<DQK>, QC::LDS_BYTES);
+        raise_lds_limit(attention_query_gradient_kernel<DQK, DV>, QC::LDS_BYTES);
     });
-    hipLaunchKernelGGL((attention_backward_statistics_kernel<DV>), dim3((unsigned)((padded_rows + 15) / 16)), dim3(256),
-                       0, stream, statistics, output_gradient, output, logsumexp, batch_size, sequence_length, heads,
+    hipLaunchKernelGGL((attention_backward_statistics_kernel<DV>), dim3((unsigned)(padded_rows / STATISTICS_ROWS)),
+                       dim3(256), 0, stream, statistics, output_gradient, output, logsumexp, batch_size, sequence_length, heads,
                        shape.query_tiles);
     HIP_CHECK(hipGetLastError());
     for (long long first = 0; first < shape.pairs; first += shape.pairs_per_launch) {
         const long long count = std::min(shape.pairs_per_launch, shape.pairs - first);
-        hipLaunchKernelGGL((attention_key_value_gradient_kernel<DQK, DV>), dim3((unsigned)(count * shape.key_blocks)),
-                           dim3(KV_THREADS), KC::LDS_BYTES, stream, key_gradient, value_gradient, ds_blocks, statistics,
-                           output_gradient, query, key, value, sequence_length, heads, kv_heads, shape.key_blocks,
-                           shape.query_tiles, (int)first, scale);
+        hipLaunchKernelGGL((attention_key_value_gradient_kernel<DQK, DV>), dim3((unsigned)(count * shape.cut.items)),
+                           dim3(KV_THREADS), KC::LDS_BYTES, stream, key_gradient, value_gradient, ds_blocks, partial_sums,
+                           statistics, output_gradient, query, key, value, sequence_length, heads, kv_heads,
+                           shape.key_blocks, shape.query_tiles, (int)first, shape.cut.part_steps, shape.cut.items, scale);
         HIP_CHECK(hipGetLastError());
         // the next chunk's first pass overwrites the dS blocks: it follows this pass in the stream.  The query
         // heads of the chunk's pairs are consecutive: count * sharing of them from first * sharing on.
-        hipLaunchKernelGGL((attention_query_gradient_kernel<DQK>),
-                           dim3((unsigned)(count * shape.sharing * shape.query_blocks)), dim3(DQ_THREADS), QC::LDS_BYTES,
-                           stream, query_gradient, ds_blocks, key, sequence_length, heads, kv_heads, shape.query_blocks,
-                           shape.key_blocks, shape.query_tiles, (int)(first * shape.sharing), scale);
+        constexpr int PIECES = KBLOCK * (DQK + DV) / 4 / DQ_THREADS;
+        const long long workgroups = count * shape.sharing * shape.query_blocks;
+        const PartialSums partial = {partial_sums, key_gradient, value_gradient, shape.cut.items, shape.cut.cut_blocks,
+                                     shape.cut.part_steps, (int)first};
+        hipLaunchKernelGGL((attention_query_gradient_kernel<DQK, DV>),
+                           dim3((unsigned)(workgroups + count * shape.cut.cut_blocks * PIECES)), dim3(DQ_THREADS),
+                           QC::LDS_BYTES, stream, query_gradient, ds_blocks, key, sequence_length, heads, kv_heads,
+                           shape.query_blocks, shape.key_blocks, shape.query_tiles, (int)(first * shape.sharing),
+                           (int)workgroups, scale, partial);
         HIP_CHECK(hipGetLastError());
     }
 }
@@ -934,12 +1088,19 @@ void attention_backward_set_workspace_limit(std::size_t bytes) {
     ds_budget_override.store(bytes > (std::size_t)1 << 62 ? 1LL << 62 : (long long)bytes, std::memory_order_relaxed);
 }
 
-std::size_t attention_backward_workspace_elements(int batch_size, int sequence_length, int heads, int kv_heads) {
+std::size_t attention_backward_workspace_elements(int batch_size, int sequence_length, int heads, int kv_heads,
+                                                  int qk_head_size, int v_head_size) {
     if (kv_heads <= 0 || heads % kv_heads != 0) {
         throw std::invalid_argument("attention backward: query heads must be a positive multiple of key/value heads");
     }
-    const BackwardShape shape = backward_shape(batch_size, sequence_length, heads, kv_heads);
-    return static_cast<std::size_t>(shape.statistics_floats + shape.ds_floats);
+    auto elements = [&](int qk, int v) {
+        const BackwardShape shape = backward_shape(batch_size, sequence_length, heads, kv_heads, qk, v);
+        return static_cast<std::size_t>(shape.statistics_floats + shape.ds_floats + shape.partial_floats);
+    };
+    if ((qk_head_size == 192 && v_head_size == 128) || (qk_head_size == v_head_size && (v_head_size == 64 || v_head_size == 128))) {
+        return elements(qk_head_size, v_head_size);
+    }
+    return std::max({elements(192, 128), elements(128, 128), elements(64, 64)});   // enough whichever geometry follows
 }
 
 void attention_backward_dispatch(bf16_t* query_gradient, bf16_t* key_gradient, bf16_t* value_gradient,

@@ -21,8 +21,10 @@ void attention_forward_dispatch(__hip_bfloat16* output, float* logsumexp, const 
 
 // attn_bwd.hip -- recompute backward of the above for Hq == Hkv.  The fp32
 // workspace (attention_backward_workspace_elements floats) holds the per-row
-// statistics and the bf16 dS blocks handed from the dK/dV kernel to the dQ pass.
-std::size_t attention_backward_workspace_elements(int batch_size, int sequence_length, int heads, int kv_heads);
+// statistics, the bf16 dS blocks handed from the dK/dV kernel to the dQ pass and,
+// where the dK/dV walks are cut, the fp32 sums of their parts.
+std::size_t attention_backward_workspace_elements(int batch_size, int sequence_length, int heads, int kv_heads,
+                                                  int qk_head_size, int v_head_size);
 
 // Bytes the dS blocks of one chunk of (batch, key/value head) pairs may take (0: the built-in 3 GiB); process-wide.
 void attention_backward_set_workspace_limit(std::size_t bytes);

@@ -41,6 +41,79 @@ DSCUDA_HOST_DEVICE inline long long ds_block_count(int key_blocks, int query_til
     return (long long)key_blocks * query_tiles - (long long)key_blocks * (key_blocks - 1);
 }
 
+// ---- cut of the key blocks' walks (backward) -----------------------------------
+// Key block kb of a (batch, key/value head) pair is walked in (query_tiles - 2 * kb) * sharing steps, one query tile of
+// one query head each.  A walk may be cut into parts of at most part_steps steps, equal to within one, each a workgroup
+// of its own.
+DSCUDA_HOST_DEVICE inline int walk_parts(int steps, int part_steps) {
+    return (int)(((unsigned)steps + (unsigned)part_steps - 1) / (unsigned)part_steps);
+}
+
+// First step of part `part` (part == parts: the end of the walk).
+DSCUDA_HOST_DEVICE inline int part_begin(int steps, int parts, int part) {
+    const unsigned each = (unsigned)steps / (unsigned)parts, more = (unsigned)steps % (unsigned)parts;
+    return (int)(each * (unsigned)part + ((unsigned)part < more ? (unsigned)part : more));
+}
+
+struct WalkCut {
+    int part_steps;   // 0: no walk is cut
+    int items;        // workgroups per pair
+    int cut_blocks;   // key blocks 0 .. cut_blocks - 1 have more than one part
+};
+
+inline long long walk_items(int key_blocks, int query_tiles, int sharing, int part_steps) {
+    long long items = 0;
+    for (int kb = 0; kb < key_blocks; ++kb) items += walk_parts((query_tiles - 2 * kb) * sharing, part_steps);
+    return items;
+}
+
+// The cut for a launch of `pairs` pairs on `slots` workgroups at a time.  Costs are in steps of one workgroup.  A
+// workgroup costs ITEM_STEPS besides its own (rows and first tile, the sums' way out, and for a part its share of the
+// addition); one round of workgroups ends with the longest, several rounds some way into the last one: parts are alike
+// and end together or not at all (half a part), whole walks start longest first and even out (a quarter of the
+// longest).  Candidates: the shortest parts that still run as one round, and several rounds of parts of 1/2 .. 1/6 of
+// the mean load.  Measured, whole walks -> cut (us for forward and backward): 128/128 columns, T=4096, 8 heads on 1:
+// 908 -> 187 (32 walks of up to 512 steps); T=8192, 16 on 4: 1316 -> 1128 (256 walks, several rounds); 192/128 columns,
+// T=4096, 4 heads: 224 -> 160, T=1000, 16 heads: 75 -> 64 (parts of 6).  Forced cuts of launches that the rule leaves
+// whole: T=2000, 32 heads 235 -> 241 (parts of 24); T=8192, 8 heads 640 -> 686 (64); T=6000, 32 heads 1464 -> 1541.
+// Walks below 12 steps stay whole: T=500, 8 heads 46 -> 45 with parts of 6.
+inline WalkCut choose_walk_cut(long long pairs, int key_blocks, int query_tiles, int sharing, int slots) {
+    constexpr int MIN_PART = 6;
+    constexpr double ITEM_STEPS = 6;
+    constexpr double GAIN = 0.9;   // of the cost of whole walks: what a cut has to stay below
+    const WalkCut whole = {0, key_blocks, 0};
+    const int longest = query_tiles * sharing;
+    if (longest < 2 * MIN_PART || pairs * key_blocks >= 4LL * slots) return whole;
+    const double mean = (double)pairs * key_blocks * (query_tiles - key_blocks + 1) * sharing / slots;
+    auto cost = [&](long long items, int part, double tail) {
+        return items * pairs <= slots ? part + ITEM_STEPS : mean + items * pairs * ITEM_STEPS / slots + tail * part;
+    };
+    const double uncut = cost(key_blocks, longest, 0.25);
+    double best = GAIN * (uncut > longest ? uncut : longest);
+    int part_steps = 0;
+    auto consider = [&](int part) {
+        if (part < MIN_PART || part >= longest) return;
+        const double value = cost(walk_items(key_blocks, query_tiles, sharing, part), part, 0.5);
+        if (value < best) {
+            best = value;
+            part_steps = part;
+        }
+    };
+    for (int rounds = 2; rounds <= 6; ++rounds) consider((int)(mean / rounds));
+    if (pairs * key_blocks <= slots) {
+        int low = MIN_PART, high = longest;   // walk_items falls with the length of a part
+        while (low < high) {
+            const int middle = (low + high) / 2;
+            if (pairs * walk_items(key_blocks, query_tiles, sharing, middle) <= slots) high = middle; else low = middle + 1;
+        }
+        consider(low);
+    }
+    if (part_steps == 0) return whole;
+    WalkCut cut = {part_steps, (int)walk_items(key_blocks, query_tiles, sharing, part_steps), 0};
+    while (cut.cut_blocks < key_blocks && (query_tiles - 2 * cut.cut_blocks) * sharing > part_steps) ++cut.cut_blocks;
+    return cut;
+}
+
 // ---- tile requests of the backward kernels ------------------------------------
 // One wave's share of the global -> LDS requests of a [ROWS][ROW_BYTES] tile that
 // WAVES waves fetch together.  LDS slot 64*load + lane (16 bytes each) holds chunk

@@ -34,7 +34,8 @@ void flash_attention_forward_cuda(
 
 // FP32 elements of workspace the backward needs (row statistics of every query head plus
 // the BF16 dS blocks one pass hands to the other, for as many (batch, key/value head)
-// pairs as one pass covers).  0 for shapes the backward rejects.
+// pairs as one pass covers, and the fp32 sums of dK and dV of the parts a key block's walk
+// over the queries is cut into where the pairs alone would leave compute units idle).  0 for shapes the backward rejects.
 std::size_t flash_attention_backward_workspace_elements(
     int batch_size,
     int sequence_length,

@@ -229,7 +229,9 @@ void mla_prefill_forward_cuda(
 // query-gradient pass, 16 KB per causal (128-key block, 64-query tile) pair --
 // about S*S bytes per (batch, head), for as many (batch, head) pairs at a time as
 // fit 3 GiB (at least one): the two passes run over the pairs in chunks that share
-// that set of blocks.  0 for non-positive sizes.
+// that set of blocks.  Where the pairs alone would leave compute units idle the walk
+// over the queries of a key block is cut into parts, and their fp32 sums of dK and dV
+// (160 KB a part for 192/128 columns, some 260 parts) follow.  0 for non-positive sizes.
 std::size_t mla_prefill_backward_workspace_elements(
     int batch_size,
     int sequence_length,

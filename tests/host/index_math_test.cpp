@@ -595,7 +595,49 @@ void check_split_order() {
     }
 }
 
+// ---- cut of the backward's walks: every step in one part, parts equal to within one and no longer than asked for
+void check_walk_cut() {
+    for (int slots : {256, 8}) {
+        for (long long pairs : {1, 2, 5, 8, 16, 33, 128}) {
+            for (int sharing : {1, 2, 3, 8}) {
+                for (int tiles : {1, 2, 5, 6, 7, 11, 12, 13, 16, 31, 64, 129, 256}) {
+                    const int blocks = (tiles + 1) / 2;
+                    const WalkCut cut = choose_walk_cut(pairs, blocks, tiles, sharing, slots);
+                    if (cut.part_steps == 0) {
+                        EXPECT(cut.items == blocks && cut.cut_blocks == 0, "pairs %lld tiles %d sharing %d", pairs, tiles, sharing);
+                        continue;
+                    }
+                    EXPECT(tiles * sharing >= 12 && cut.part_steps >= 6, "pairs %lld tiles %d sharing %d", pairs, tiles, sharing);
+                    int items = 0;
+                    for (int kb = 0; kb < blocks; ++kb) {
+                        const int steps = (tiles - 2 * kb) * sharing;
+                        const int parts = walk_parts(steps, cut.part_steps);
+                        EXPECT((parts > 1) == (kb < cut.cut_blocks), "tiles %d sharing %d block %d", tiles, sharing, kb);
+                        EXPECT(part_begin(steps, parts, 0) == 0 && part_begin(steps, parts, parts) == steps, "steps %d parts %d", steps, parts);
+                        for (int part = 0; part < parts; ++part) {
+                            const int length = part_begin(steps, parts, part + 1) - part_begin(steps, parts, part);
+                            EXPECT(length >= steps / parts && length <= (steps + parts - 1) / parts && length >= 1 &&
+                                   length <= cut.part_steps, "steps %d part %d of %d: %d", steps, part, parts, length);
+                        }
+                        items += parts;
+                    }
+                    EXPECT(items == cut.items, "tiles %d sharing %d: %d items, %d counted", tiles, sharing, cut.items, items);
+                }
+            }
+        }
+    }
+    // launches whose whole walks were measured faster stay whole, those that were measured slower are cut
+    EXPECT(choose_walk_cut(32, 16, 32, 1, 256).part_steps == 0, "T=2000, 32 heads");
+    EXPECT(choose_walk_cut(8, 64, 128, 1, 256).part_steps == 0, "T=8192, 8 heads");
+    EXPECT(choose_walk_cut(128, 32, 64, 1, 256).part_steps == 0, "T=4096, 128 heads");
+    EXPECT(choose_walk_cut(24, 5, 10, 1, 256).part_steps == 0, "walks of ten steps");
+    EXPECT(choose_walk_cut(16, 8, 16, 1, 256).part_steps == 6, "T=1000, 16 heads");
+    EXPECT(choose_walk_cut(8, 9, 17, 4, 256).part_steps > 0, "T=1088, 2 x 16 heads on 4");
+    EXPECT(choose_walk_cut(4, 64, 128, 4, 256).part_steps > 0, "T=8192, 16 heads on 4");
+}
+
 int main() {
+    check_walk_cut();
     check_split_order();
     check_swizzle<128>();
     check_swizzle<256>();
