@@ -269,6 +269,145 @@ __global__ __launch_bounds__(THREADS) void mla_unabsorb_output_kernel(bf16_t* __
     }
 }
 
+// ---- few tokens ---------------------------------------------------------------------
+// A decode step has a handful of tokens per head: the kernels above would put a head on one compute unit, which then
+// waits for 128 KB of weight before its first product.  Here a workgroup takes a quarter of a head's weight and 32
+// tokens, and every load of a thread is in flight at once: one round trip to memory, eight MFMAs a wave.  16 tokens of
+// 16 heads: absorb 7.6 -> 3.2 us, un-absorb 6.6 -> 3.7.
+//
+// Every 32 tokens fetch the weight again, so the kernels above win once (token tiles) x heads is large.  Absorb at 256
+// tiles 8.0-8.2 against 9.3-11.6 us (64 tokens of 128 heads, 512 of 16), at 512 tiles 13.4 against 13.2-13.9.
+// Un-absorb, whose weight rows come as 32 bytes of 32 rows an instruction, at 128 tiles 5.1-5.8 against 6.7-9.7 us
+// (16 tokens of 128 heads, 128 of 32), at 256 tiles 10.2-12.8 against 8.1-9.8.
+constexpr long long ABSORB_FEW_TILES = 256;
+constexpr long long UNABSORB_FEW_TILES = 128;
+
+constexpr int SLICE = RANK / 4;                    // output columns of an absorb workgroup
+constexpr int SLICE_PITCH = 2 * SLICE + 16;        // bytes; 16 modulo 256 as above
+constexpr int SLICE_BYTES = HEAD * SLICE_PITCH;
+constexpr int FEW_LDS_BYTES = SLICE_BYTES + TILE * SLICE_PITCH;
+
+// q_latent = q_nope W_UK: blockIdx.x = 4 * head + quarter of the columns, blockIdx.y = 32 tokens; a wave per 32 columns
+__global__ __launch_bounds__(THREADS) void mla_absorb_query_few_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
+                                                                       const bf16_t* __restrict__ weight, long long tokens,
+                                                                       Strides strides) {
+    constexpr int KSTEPS = HEAD / 16;
+    constexpr int PIECES = HEAD * SLICE / 8 / THREADS;   // 16-byte pieces of the weight slice per thread
+    __shared__ __attribute__((aligned(16))) unsigned char lds[FEW_LDS_BYTES];
+    const int tid = threadIdx.x;
+    const int wave = tid / 64;
+    const int lane = tid % 64;
+    const int lq = lane % 32;
+    const int g = lane / 32;
+    const int head = blockIdx.x / 4;
+    const int column0 = blockIdx.x % 4 * SLICE;
+    const long long tile0 = (long long)blockIdx.y * TILE;
+
+    u32x4 rows[KSTEPS], pieces[PIECES];
+    const bf16_t* x_head = x + head * strides.x_head;
+    fetch_token_row(rows, x_head + min(tile0 + lq, tokens - 1) * strides.x_token, tile0 + lq < tokens, g);
+    const bf16_t* slice = weight + head * strides.w_head + column0;
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) {
+        const int piece = tid + j * THREADS;
+        pieces[j] = *reinterpret_cast<const u32x4*>(slice + piece / (SLICE / 8) * RANK + 8 * (piece % (SLICE / 8)));
+    }
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) {
+        const int piece = tid + j * THREADS;
+        *reinterpret_cast<u32x4*>(lds + piece / (SLICE / 8) * SLICE_PITCH + 16 * (piece % (SLICE / 8))) = pieces[j];
+    }
+    __syncthreads();
+
+    // operands as in mla_absorb_query_kernel
+    const int s = lane % 16;
+    const int half = (lane / 16) % 2;
+    const unsigned char* at = lds + (4 * g + s / 4) * SLICE_PITCH + 32 * half + 8 * (s % 4) + 64 * wave;
+    f32x16 acc;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks) {
+        const auto first_pair = __builtin_amdgcn_permlane32_swap(rows[ks][0], rows[ks][2], false, false);
+        const auto second_pair = __builtin_amdgcn_permlane32_swap(rows[ks][1], rows[ks][3], false, false);
+        const bf16x8 xf = __builtin_bit_cast(bf16x8, u32x4{first_pair[0], second_pair[0], first_pair[1], second_pair[1]});
+        const s16x4 low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((transposing_read_pointer)(at + 16 * ks * SLICE_PITCH));
+        const s16x4 high = __builtin_amdgcn_ds_read_tr16_b64_v4i16((transposing_read_pointer)(at + (16 * ks + 8) * SLICE_PITCH));
+        const bf16x8 wf = __builtin_bit_cast(bf16x8, __builtin_shufflevector(low, high, 0, 1, 2, 3, 4, 5, 6, 7));
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf, xf, acc, 0, 0, 0);
+    }
+    // lane holds token lq and columns 32*wave + 8*i4 + 4*g .. +3: rows of 256 bytes through LDS
+    unsigned char* out_rows = lds + SLICE_BYTES;
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) {
+        u32x2 packed;
+        packed.x = pack_bf16(acc[4 * i4 + 0], acc[4 * i4 + 1]);
+        packed.y = pack_bf16(acc[4 * i4 + 2], acc[4 * i4 + 3]);
+        *reinterpret_cast<u32x2*>(out_rows + lq * SLICE_PITCH + 64 * wave + 16 * i4 + 8 * g) = packed;
+    }
+    __syncthreads();
+    for (int piece = tid; piece < TILE * SLICE / 8; piece += THREADS) {
+        const int row = piece / (SLICE / 8);
+        const int chunk = piece % (SLICE / 8);
+        if (tile0 + row < tokens) {
+            *reinterpret_cast<u32x4*>(y + head * strides.y_head + (tile0 + row) * strides.y_token + column0 + 8 * chunk) =
+                *reinterpret_cast<const u32x4*>(out_rows + row * SLICE_PITCH + 16 * chunk);
+        }
+    }
+}
+
+// out = o_latent W_UV^T: blockIdx.x = 4 * head + 32 of the weight's rows, blockIdx.y = 32 tokens; each wave contracts a
+// quarter of the latent columns, weight rows straight from memory, and the quarters are added in order
+__global__ __launch_bounds__(THREADS) void mla_unabsorb_output_few_kernel(bf16_t* __restrict__ y,
+                                                                          const bf16_t* __restrict__ x,
+                                                                          const bf16_t* __restrict__ weight,
+                                                                          long long tokens, Strides strides) {
+    constexpr int WAVES = THREADS / 64;
+    constexpr int COLUMNS = RANK / WAVES;
+    constexpr int KSTEPS = COLUMNS / 16;
+    constexpr int SUM_PITCH = TILE + 4;   // floats per token
+    __shared__ __attribute__((aligned(16))) float sums[WAVES][TILE * SUM_PITCH];
+    const int tid = threadIdx.x;
+    const int wave = tid / 64;
+    const int lane = tid % 64;
+    const int lq = lane % 32;
+    const int g = lane / 32;
+    const int head = blockIdx.x / 4;
+    const int row0 = blockIdx.x % 4 * TILE;
+    const long long tile0 = (long long)blockIdx.y * TILE;
+
+    u32x4 rows[KSTEPS], weights[KSTEPS];
+    fetch_token_row(weights, weight + head * strides.w_head + (row0 + lq) * RANK + COLUMNS * wave, true, g);
+    fetch_token_row(rows, x + head * strides.x_head + min(tile0 + lq, tokens - 1) * strides.x_token + COLUMNS * wave,
+                    tile0 + lq < tokens, g);
+    f32x16 acc;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks) {
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, weights[ks]),
+                                                      __builtin_bit_cast(bf16x8, rows[ks]), acc, 0, 0, 0);
+    }
+    // lane holds token lq and weight rows 8*i4 + 4*g .. +3
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) {
+        *reinterpret_cast<f32x4*>(&sums[wave][lq * SUM_PITCH + 8 * i4 + 4 * g]) =
+            f32x4{acc[4 * i4], acc[4 * i4 + 1], acc[4 * i4 + 2], acc[4 * i4 + 3]};
+    }
+    __syncthreads();
+    const int token = tid / 8;
+    const int column = 4 * (tid % 8);
+    f32x4 sum = *reinterpret_cast<const f32x4*>(&sums[0][token * SUM_PITCH + column]);
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) sum += *reinterpret_cast<const f32x4*>(&sums[w][token * SUM_PITCH + column]);
+    if (tile0 + token < tokens) {
+        u32x2 packed;
+        packed.x = pack_bf16(sum[0], sum[1]);
+        packed.y = pack_bf16(sum[2], sum[3]);
+        *reinterpret_cast<u32x2*>(y + head * strides.y_head + (tile0 + token) * strides.y_token + row0 + column) = packed;
+    }
+}
+
 void check(bool condition, const char* message) {
     if (!condition) throw std::invalid_argument(message);
 }
@@ -281,10 +420,17 @@ int compute_units() {
 // workgroup stages the head's weight first, which costs it about as long as 128 tokens.  The number of chunks is
 // the one with the shortest schedule: rounds of workgroups over the compute units times the cost of a workgroup
 // (4096 tokens x 128 heads on 256 compute units: two chunks, one round, 138 / 171 us against 145 / 178 us with four).
-template <typename Kernel>
-void launch(Kernel kernel, bf16_t* y, const bf16_t* x, const bf16_t* weight, long long tokens, int heads,
+template <typename Kernel, typename FewKernel>
+void launch(Kernel kernel, FewKernel few_kernel, long long few_tiles, bf16_t* y, const bf16_t* x, const bf16_t* weight, long long tokens, int heads,
             const Strides& strides, hipStream_t stream) {
     check(heads <= 65535, "MLA projection: more heads than the grid allows");
+    const long long tiles = (tokens + TILE - 1) / TILE;
+    if (tiles * heads <= few_tiles) {
+        hipLaunchKernelGGL(few_kernel, dim3((unsigned)(4 * heads), (unsigned)tiles), dim3(THREADS), 0, stream, y, x, weight,
+                           tokens, strides);
+        HIP_CHECK(hipGetLastError());
+        return;
+    }
     constexpr long long STAGING_TOKENS = 4 * TILE;
     const long long units = std::max(1, compute_units());
     const long long most = (tokens + 4 * TILE - 1) / (4 * TILE);
@@ -335,7 +481,7 @@ void mla_absorb_query_dispatch(bf16_t* query_latent, const bf16_t* query_nope, c
         HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(mla_absorb_query_kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES));
     });
-    launch(mla_absorb_query_kernel, query_latent, query_nope, weight, tokens, heads, strides, stream);
+    launch(mla_absorb_query_kernel, mla_absorb_query_few_kernel, ABSORB_FEW_TILES, query_latent, query_nope, weight, tokens, heads, strides, stream);
 }
 
 void mla_unabsorb_output_dispatch(bf16_t* output, const bf16_t* output_latent, const bf16_t* weight, long long tokens,
@@ -350,7 +496,7 @@ void mla_unabsorb_output_dispatch(bf16_t* output, const bf16_t* output_latent, c
         HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(mla_unabsorb_output_kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES));
     });
-    launch(mla_unabsorb_output_kernel, output, output_latent, weight, tokens, heads, strides, stream);
+    launch(mla_unabsorb_output_kernel, mla_unabsorb_output_few_kernel, UNABSORB_FEW_TILES, output, output_latent, weight, tokens, heads, strides, stream);
 }
 
 }  // namespace dscuda

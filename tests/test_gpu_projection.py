@@ -49,6 +49,27 @@ def test_unabsorb_output(cuda, batch, seq, heads):
     assert_close_bf16("output", out.cpu(), expected)
 
 
+@pytest.mark.parametrize("tokens,heads", [(32, 2), (33, 5), (64, 128), (65, 128), (32, 128), (33, 128), (512, 16), (513, 16),
+                                          (1, 257)])
+def test_projections_on_either_side_of_the_token_rule(cuda, tokens, heads):
+    """Whole and just exceeded token tiles at the largest (token tiles) x heads of the kernels for few tokens: 256 for
+    the absorb, 128 for the un-absorb.  Weights are slices of wkv_b, rows slices of wider tensors."""
+    wkv_b, g = _weights(heads, 53)
+    device_weights = wkv_b.to(cuda)
+    query = (torch.randn(1, tokens, heads, 192, generator=g) * 0.5).bfloat16()
+    latent = (torch.randn(1, tokens, heads, 576, generator=g) * 0.5).bfloat16()
+    announce("mla projections, token rule", dict(T=tokens, H=heads))
+    packed = torch.full((1, tokens + 1, heads, 576), 7.0, device=cuda, dtype=torch.bfloat16)
+    ops.mla_absorb_query(query.to(cuda)[..., :128], device_weights[:, :128], out=packed[:, :tokens, :, :512])
+    result = torch.full((1, tokens + 1, heads, 136), 7.0, device=cuda, dtype=torch.bfloat16)
+    ops.mla_unabsorb_output(latent.to(cuda)[..., :512], device_weights[:, 128:], out=result[:, :tokens, :, :128])
+    torch.cuda.synchronize()
+    assert_close_bf16("q_latent", packed[:, :tokens, :, :512].cpu(), oracle.absorb_query(query[..., :128], wkv_b[:, :128]))
+    assert_close_bf16("output", result[:, :tokens, :, :128].cpu(), oracle.unabsorb_output(latent[..., :512], wkv_b[:, 128:]))
+    assert (packed[:, tokens:].float() == 7.0).all() and (packed[..., 512:].float() == 7.0).all()
+    assert (result[:, tokens:].float() == 7.0).all() and (result[..., 128:].float() == 7.0).all()
+
+
 def test_projections_compose_with_decode(cuda):
     """An absorbed decode step between the two projections equals per-head attention over the expanded keys and
     values (the identity that makes absorption valid), within bf16 rounding of the intermediate tensors."""
