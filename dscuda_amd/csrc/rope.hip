@@ -14,10 +14,14 @@
 // fp32 without fusing, the result rounded to bf16: the same sequence of roundings as
 // forming the rotation with fp32 tensors on the host.
 //
-// Layout on the chip: one wave per (batch, position).  A lane owns pair lane % (rope/2)
-// and computes its sine and cosine once; the 64 / (rope/2) groups of lanes then walk the
-// heads in turn, so every access of a group is one contiguous run of 2 * rope bytes.
-// The kernel moves 4 * rope bytes per (b, s, h) and is bound by memory.
+// Layout on the chip: one wave per (batch, position) and slice of the heads.  A lane owns
+// pair lane % (rope/2) and computes its sine and cosine once; the 64 / (rope/2) groups of
+// lanes then walk the heads, so every access of a group is one contiguous run of
+// 2 * rope bytes.  The kernel moves 4 * rope bytes per (b, s, h) and is bound by memory:
+// BATCH heads of a group are fetched before the first is stored (in place, so the loads
+// would otherwise wait for the stores, a round trip per head), and where the rows alone
+// leave the chip idle the heads are sliced so that one batch covers a wave.  64 rows of
+// 128 heads 11.9 -> 3.5 us, 1024 rows 14.4 -> 9.4, 4096 rows 29.3 -> 23.8 (5.6 TB/s).
 
 #include "attn_kernels.h"
 #include "hip_common.h"
@@ -32,10 +36,11 @@ namespace {
 
 constexpr int ROPE_THREADS = 256;
 constexpr int ROPE_ROWS = ROPE_THREADS / 64;   // (batch, position) rows per workgroup
+constexpr int BATCH = 8;                       // heads a group of lanes has in flight
 
 __global__ __launch_bounds__(ROPE_THREADS) void rope_apply_kernel(bf16_t* __restrict__ tensor,
                                                                   const int* __restrict__ positions, long long rows,
-                                                                  int sequence_length, int heads, int width,
+                                                                  int sequence_length, int heads, int slice, int width,
                                                                   int rope_offset, int rope, double log2_theta) {
     const long long row = (long long)blockIdx.x * ROPE_ROWS + threadIdx.x / 64;
     if (row >= rows) return;
@@ -52,14 +57,21 @@ __global__ __launch_bounds__(ROPE_THREADS) void rope_apply_kernel(bf16_t* __rest
     const float cosine = (float)cos(angle);
     const float sine = (float)sin(angle);
     unsigned* base = reinterpret_cast<unsigned*>(tensor + (size_t)row * heads * width + rope_offset) + pair;
-    for (int h = group; h < heads; h += groups) {
-        unsigned* target = base + (size_t)h * (width / 2);
-        const unsigned bits = *target;
-        const float even = __uint_as_float(bits << 16);
-        const float odd = __uint_as_float(bits & 0xffff0000u);
-        const float rotated_even = __fsub_rn(__fmul_rn(even, cosine), __fmul_rn(odd, sine));
-        const float rotated_odd = __fadd_rn(__fmul_rn(even, sine), __fmul_rn(odd, cosine));
-        *target = pack_bf16(rotated_even, rotated_odd);
+    const int end = min(heads, (int)(blockIdx.y + 1) * slice);
+    for (int first = blockIdx.y * slice + group; first < end; first += groups * BATCH) {
+        unsigned bits[BATCH];
+#pragma unroll
+        for (int j = 0; j < BATCH; ++j) {
+            bits[j] = base[(size_t)min(first + j * groups, end - 1) * (width / 2)];
+        }
+#pragma unroll
+        for (int j = 0; j < BATCH; ++j) {
+            const float even = __uint_as_float(bits[j] << 16);
+            const float odd = __uint_as_float(bits[j] & 0xffff0000u);
+            const float rotated_even = __fsub_rn(__fmul_rn(even, cosine), __fmul_rn(odd, sine));
+            const float rotated_odd = __fadd_rn(__fmul_rn(even, sine), __fmul_rn(odd, cosine));
+            if (first + j * groups < end) base[(size_t)(first + j * groups) * (width / 2)] = pack_bf16(rotated_even, rotated_odd);
+        }
     }
 }
 
@@ -92,8 +104,13 @@ void rope_apply_dispatch(bf16_t* tensor, const int* positions, int batch_size, i
     if (blocks > 0x7fffffffLL) {
         throw std::invalid_argument("rope: batch * sequence length exceeds the grid limit");
     }
-    hipLaunchKernelGGL(rope_apply_kernel, dim3((unsigned)blocks), dim3(ROPE_THREADS), 0, stream, tensor, positions, rows,
-                       sequence_length, heads, width, rope_offset, rope_size, std::log2((double)theta));
+    // below four workgroups per compute unit the heads are sliced, one batch of every group of lanes a slice
+    const int batch_heads = 64 / (rope_size / 2) * BATCH;
+    const int slice = blocks < 4LL * hip_common::compute_units_of_current_device() && (heads - 1) / batch_heads < 65535
+        ? batch_heads : heads;
+    const unsigned slices = (unsigned)((heads + (long long)slice - 1) / slice);
+    hipLaunchKernelGGL(rope_apply_kernel, dim3((unsigned)blocks, slices), dim3(ROPE_THREADS), 0, stream, tensor, positions,
+                       rows, sequence_length, heads, slice, width, rope_offset, rope_size, std::log2((double)theta));
     HIP_CHECK(hipGetLastError());
 }
 

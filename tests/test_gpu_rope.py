@@ -82,3 +82,22 @@ def test_rope_rejects_bad_slices(cuda):
     for offset, size in ((0, 48), (1, 32), (48, 32), (0, 0)):
         with pytest.raises(RuntimeError):
             ops.rope_apply(x, offset, size)
+
+
+@pytest.mark.parametrize("shape,size", [
+    ((5, 1, 128, 64), 64),      # few rows: eight slices of 16 heads
+    ((3, 2, 35, 64), 64),       # the last slice holds three heads, of a group of lanes two or one
+    ((1, 4, 9, 128), 128),      # one pair per lane: batches of eight heads, the last slice holds one
+    ((1, 4100, 19, 8), 8),      # many rows: the heads in one slice, 16 groups of lanes
+    ((1, 4100, 18, 64), 64),    # ... and a second batch of two heads
+])
+def test_rope_slices_of_heads(cuda, shape, size):
+    announce("rope, slices of heads", dict(shape=shape, size=size))
+    x = (torch.randn(shape, generator=torch.Generator().manual_seed(80)) * 0.5).bfloat16()
+    guarded = torch.full((x.numel() + 64,), 7.0, device=cuda, dtype=torch.bfloat16)
+    tensor = guarded[:x.numel()].view(shape)
+    tensor.copy_(x.to(cuda))
+    ops.rope_apply(tensor, 0, size)
+    torch.cuda.synchronize()
+    _compare(tensor, _expected(x, 0, size))
+    assert (guarded[x.numel():].float() == 7.0).all()
