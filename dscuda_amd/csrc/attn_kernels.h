@@ -70,6 +70,15 @@ void mla_absorbed_backward_dispatch(__hip_bfloat16* query_latent_gradient, __hip
                                     const __hip_bfloat16* key_rope, int batch_size, int sequence_length, int heads,
                                     float scale, hipStream_t stream);
 
+// mla_absorbed_short.hip -- the launches after the row statistics for at most 512 tokens (delta of a row in the first
+// four bytes of its rope query gradient); the query gradients are 16-byte aligned.
+void mla_absorbed_short_backward_launch(__hip_bfloat16* query_latent_gradient, __hip_bfloat16* query_rope_gradient,
+                                        __hip_bfloat16* kv_latent_gradient, __hip_bfloat16* key_rope_gradient,
+                                        const __hip_bfloat16* output_gradient, const float* logsumexp,
+                                        const __hip_bfloat16* query_latent, const __hip_bfloat16* query_rope,
+                                        const __hip_bfloat16* kv_latent, const __hip_bfloat16* key_rope, int batch_size,
+                                        int sequence_length, int heads, float scale, hipStream_t stream);
+
 // > 0: the key-gradient pass cuts its work by intervals of that many row tiles at any size; 0: its own choice.
 void mla_absorbed_backward_set_key_interval_tiles(int tiles);
 

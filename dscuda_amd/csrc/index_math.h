@@ -579,6 +579,35 @@ DSCUDA_HOST_DEVICE inline long long key_gradient_ranges(long long total, long lo
     return (longest < row_tiles || blocks > compute_units) ? ranges : 0;
 }
 
+// ---- absorbed backward of short sequences: where P is kept ------------------------
+// Row `row` = token * heads + head of a batch element with `blocks` blocks of 32 tokens (the last one possibly short)
+// keeps dS of key block b (32 keys, 64 bytes) in chunk b of its own 16 chunks of the latent query gradient, b = 0 ..
+// its token block.  P of key block b: for a row of token block i < blocks - 1 in chunk kept_chunk of row kept_row, a
+// row of block blocks - 2 - i, behind that row's dS; for a row of the last block in the rope query gradient (one
+// chunk a row) of row kept_row, a row of block b.
+constexpr int SHORT_TOKENS = 512;
+
+// Which calls keep P and dS instead of partial key gradients.  More tokens do not fit.  The key-gradient launch walks
+// all rows of a batch element per 32 keys x 32 columns, so many rows, or many heads on few keys, are better off with
+// the other kernels.  Forward and backward, partial results -> kept (us): 512 tokens x 8 heads 106 -> 71, 300 x 4
+// 106 -> 46, 350 x 16 82 -> 70, 128 x 32 56 -> 49, 3 x 500 x 4 142 -> 81, 8 x 500 x 4 169 -> 152; left to the others:
+// 200 x 32 67 -> 66, 480 x 16 96 -> 98, 100 x 64 56 -> 58, 32 x 128 45 -> 50, 4 x 512 x 8 133 -> 138.
+DSCUDA_HOST_DEVICE inline bool short_backward(long long batch, int tokens, int heads) {
+    const long long rows = (long long)tokens * heads;
+    return tokens <= SHORT_TOKENS && heads <= 32 && rows <= 6000 && rows * batch <= 16000;
+}
+
+DSCUDA_HOST_DEVICE inline bool kept_in_rope(int token_block, int blocks) { return token_block == blocks - 1; }
+
+DSCUDA_HOST_DEVICE inline int kept_row(int row, int token_block, int key_block, int blocks, int heads) {
+    const int block = kept_in_rope(token_block, blocks) ? key_block : blocks - 2 - token_block;
+    return row + (block - token_block) * 32 * heads;
+}
+
+DSCUDA_HOST_DEVICE inline int kept_chunk(int token_block, int key_block, int blocks) {
+    return blocks - 1 - token_block + key_block;
+}
+
 // ---- decode: the plan and how a call uses the caller's workspace ---------------
 // The plan is what a decode call needs to know about the lengths of its batch
 // before any workgroup starts: an int table

@@ -39,6 +39,8 @@
 //                     token of those rows.  Every wave forms one quadrant of S^T and
 //                     dP^T of the tile, the quadrants of dS^T meet in LDS, and every
 //                     wave accumulates dQ^T for its own share of the 18 column blocks.
+// Short sequences with few rows (index_math::short_backward), whose query-gradient buffers have room for few partial
+// results, take three other launches after the row statistics (mla_absorbed_short.hip).
 #include "attn_kernels.h"
 #include "hip_common.h"
 #include "index_math.h"
@@ -1535,6 +1537,12 @@ void mla_absorbed_backward_dispatch(bf16_t* query_latent_gradient, bf16_t* query
     hipLaunchKernelGGL(mla_absorbed_row_statistics_kernel, dim3((unsigned)(row_blocks * batch_size)), dim3(THREADS), 0,
                        stream, delta, output_gradient, output, rows * batch_size);
     HIP_CHECK(hipGetLastError());
+    if (forced == 0 && index_math::short_backward(batch_size, sequence_length, heads)) {
+        mla_absorbed_short_backward_launch(query_latent_gradient, query_rope_gradient, kv_latent_gradient, key_rope_gradient,
+                                           output_gradient, logsumexp, query_latent, query_rope, kv_latent, key_rope,
+                                           batch_size, sequence_length, heads, scale, stream);
+        return;
+    }
     if (interval_length > 0) {
         hipLaunchKernelGGL(mla_absorbed_key_pair_gradient_kernel, dim3((unsigned)grid), dim3(THREADS),
                            KeyPairLayout::LDS_BYTES, stream, kv_latent_gradient, key_rope_gradient, partial_slots, delta,

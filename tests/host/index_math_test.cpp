@@ -636,7 +636,34 @@ void check_walk_cut() {
     EXPECT(choose_walk_cut(4, 64, 128, 4, 256).part_steps > 0, "T=8192, 16 heads on 4");
 }
 
+// ---- kept P and dS of the short absorbed backward: every chunk has a place of its own inside rows that exist
+void check_kept_scores() {
+    for (int heads : {1, 2, 3}) {
+        for (int tokens = 1; tokens <= SHORT_TOKENS; tokens += tokens % 32 < 2 || tokens % 32 > 29 ? 1 : 7) {
+            const int blocks = (tokens + 31) / 32, rows = tokens * heads;
+            std::vector<char> latent(16 * rows, 0), rope(rows, 0);
+            for (int row = 0; row < rows; ++row) {
+                const int own = row / heads / 32;
+                for (int block = 0; block <= own; ++block) {
+                    EXPECT(++latent[16 * row + block] == 1, "tokens %d row %d block %d: dS", tokens, row, block);
+                    const int at = kept_row(row, own, block, blocks, heads);
+                    EXPECT(at >= 0 && at < rows, "tokens %d row %d block %d: row %d", tokens, row, block, at);
+                    if (at < 0 || at >= rows) continue;
+                    if (kept_in_rope(own, blocks)) {
+                        EXPECT(++rope[at] == 1, "tokens %d row %d block %d: P", tokens, row, block);
+                    } else {
+                        const int chunk = kept_chunk(own, block, blocks);
+                        EXPECT(chunk >= 0 && chunk < 16, "tokens %d row %d block %d: chunk %d", tokens, row, block, chunk);
+                        if (chunk >= 0 && chunk < 16) EXPECT(++latent[16 * at + chunk] == 1, "tokens %d row %d block %d: P", tokens, row, block);
+                    }
+                }
+            }
+        }
+    }
+}
+
 int main() {
+    check_kept_scores();
     check_walk_cut();
     check_split_order();
     check_swizzle<128>();
