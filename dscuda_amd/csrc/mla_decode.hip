@@ -649,49 +649,81 @@ __global__ __launch_bounds__(THREADS) void mla_decode_split_kernel(
 }
 
 // Merge the parts of every sequence that was cut by a range boundary.  One wave per
-// (sequence, wave of 32 heads, quarter of the 512 columns): it reads its share of every
+// (sequence, wave of 32 heads, eighth of the 512 columns): it reads its share of every
 // part in the order the registers of the split kernel held it (same lane numbering),
 // so lane l ends up with head l % 32 and, per column block d, the columns
 // output_column(d, i4, l / 32) + 0..3; the results go through LDS to leave as 16-byte
-// pieces of output rows.
-constexpr int MERGE_QUARTERS = 4;
-constexpr int MERGE_PIECES = PARTIAL_PIECES / MERGE_QUARTERS;       // 8 pieces of 16 bytes per lane and part
-constexpr int MERGE_COLUMNS = RANK / MERGE_QUARTERS;                // 128
-constexpr int MERGE_PITCH = MERGE_COLUMNS * 2 + 16;                  // bytes per staged row
+// pieces of output rows.  Bound by round trips to partial results that another XCD wrote:
+// statistics and pieces of MERGE_AHEAD parts (more than most sequences have) are asked for
+// at once, before the first of them is needed.  One part after the other, a quarter of the columns per
+// wave, took 13.2 us for 64 sequences x 128 heads (five parts each, 40 MB); so 10.3 us.  Whole
+// calls: that 119.4 -> 116.6 us, 32 x 128 78.6 -> 73.8, 28 x 128 x 200..1000 tokens 38.1 -> 33.6,
+// 4 x 1024 98.9 -> 93.1.
+constexpr int MERGE_SLICES = 8;
+constexpr int MERGE_PIECES = PARTIAL_PIECES / MERGE_SLICES;         // 4 pieces of 16 bytes per lane and part
+constexpr int MERGE_COLUMNS = RANK / MERGE_SLICES;                  // 64
+constexpr int MERGE_PITCH = MERGE_COLUMNS * 2 + 16;                 // bytes per staged row
+constexpr int MERGE_AHEAD = 8;
 
 __global__ __launch_bounds__(64) void mla_decode_merge_kernel(bf16_t* __restrict__ output, float* __restrict__ logsumexp,
-                                                              const float* __restrict__ workspace, int* __restrict__ plan,
-                                                              int batch_size, int heads, long long slot_floats,
-                                                              int padded_rows) {
+                                                              const float* __restrict__ workspace,
+                                                              const int* __restrict__ plan, int heads,
+                                                              long long slot_floats, int padded_rows) {
     __shared__ __attribute__((aligned(16))) unsigned char staging[32 * MERGE_PITCH];
     const int lane = threadIdx.x;
     const int lq = lane % 32;
     const int g = lane / 32;
-    const int quarter = blockIdx.x % MERGE_QUARTERS;
-    const int wave_block = blockIdx.x / MERGE_QUARTERS;   // 32 heads, numbered over all head groups
+    const int slice = blockIdx.x % MERGE_SLICES;
+    const int wave_block = blockIdx.x / MERGE_SLICES;     // 32 heads, numbered over all head groups
     const int sequence = blockIdx.y;
 
     const int total = plan[PLAN_TOTAL];
-    const int workgroups = plan[PLAN_WORKGROUPS];
     const int overhead = plan[PLAN_OVERHEAD];
+    const int ranges = plan[PLAN_RANGES];
     const int* prefix = plan + index_math::plan_prefix_at();
     const int sequence_begin = prefix[sequence];
     const int sequence_end = prefix[sequence + 1];
+    asm volatile("" ::"s"(total), "s"(overhead), "s"(ranges), "s"(sequence_end));   // one round trip, not two
     if (sequence_end <= sequence_begin) return;   // no tiles: nothing was computed for it
     int first, last;
-    index_math::ranges_of_sequence(total, plan[PLAN_RANGES], sequence_begin, sequence_end - sequence_begin, overhead, first, last);
+    index_math::ranges_of_sequence(total, ranges, sequence_begin, sequence_end - sequence_begin, overhead, first, last);
     if (first == last) return;                    // finished in place by the split kernel
 
     const int head = 32 * wave_block + lq;
-    const bool valid = head < heads;
-    const size_t stats_offset = (size_t)padded_rows * (RANK / 2);
-    const size_t pieces_offset = (size_t)wave_block * PARTIAL_WAVE_BYTES + (size_t)(quarter * MERGE_PIECES * 64 + lane) * 16;
+    const int parts = last - first + 1;
+    const float* slots = workspace + ((size_t)first + sequence) * slot_floats;
+    // lanes past the last head repeat its statistics; what they merge is not stored
+    const float* statistics = slots + (size_t)padded_rows * (RANK / 2) + 2 * min(head, heads - 1);
+    const unsigned char* pieces = reinterpret_cast<const unsigned char*>(slots) + (size_t)wave_block * PARTIAL_WAVE_BYTES +
+        (size_t)(slice * MERGE_PIECES * 64 + lane) * 16;
 
+    float part_reference[MERGE_AHEAD], part_sum[MERGE_AHEAD];
+    u32x4 bits[MERGE_AHEAD][MERGE_PIECES];
+    auto request = [&](int base) {
+#pragma unroll
+        for (int i = 0; i < MERGE_AHEAD; ++i) {
+            if (base + i < parts) {
+                part_reference[i] = statistics[(size_t)(base + i) * slot_floats];
+                part_sum[i] = statistics[(size_t)(base + i) * slot_floats + 1];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < MERGE_AHEAD; ++i) {
+            if (base + i < parts) {
+#pragma unroll
+                for (int j = 0; j < MERGE_PIECES; ++j) {
+                    bits[i][j] = *reinterpret_cast<const u32x4*>(pieces + (size_t)(base + i) * slot_floats * 4 + j * 1024);
+                }
+            }
+        }
+    };
+    request(0);
     float reference = -INFINITY;
-    for (int w = first; w <= last; ++w) {
-        const float* part = workspace + ((size_t)w + sequence) * slot_floats;
-        if (valid) reference = fmaxf(reference, part[stats_offset + 2 * head]);
+#pragma unroll
+    for (int i = 0; i < MERGE_AHEAD; ++i) {
+        if (i < parts) reference = fmaxf(reference, part_reference[i]);
     }
+    for (int part = MERGE_AHEAD; part < parts; ++part) reference = fmaxf(reference, statistics[(size_t)part * slot_floats]);
     float normaliser = 0.f;
     float sums[MERGE_PIECES][8];
 #pragma unroll
@@ -699,26 +731,26 @@ __global__ __launch_bounds__(64) void mla_decode_merge_kernel(bf16_t* __restrict
 #pragma unroll
         for (int k = 0; k < 8; ++k) sums[j][k] = 0.f;
     }
-    for (int w = first; w <= last; ++w) {
-        const float* part = workspace + ((size_t)w + sequence) * slot_floats;
-        float weight = 0.f;
-        if (valid) {
-            weight = __builtin_amdgcn_exp2f(part[stats_offset + 2 * head] - reference);
-            normaliser = fmaf(weight, part[stats_offset + 2 * head + 1], normaliser);
-        }
-        const unsigned char* pieces = reinterpret_cast<const unsigned char*>(part) + pieces_offset;
+    for (int base = 0; base < parts; base += MERGE_AHEAD) {
+        if (base > 0) request(base);
 #pragma unroll
-        for (int j = 0; j < MERGE_PIECES; ++j) {
-            const u32x4 bits = *reinterpret_cast<const u32x4*>(pieces + j * 1024);
+        for (int i = 0; i < MERGE_AHEAD; ++i) {
+            if (base + i < parts) {
+                const float weight = __builtin_amdgcn_exp2f(part_reference[i] - reference);
+                normaliser = fmaf(weight, part_sum[i], normaliser);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                sums[j][2 * k] = fmaf(weight, __uint_as_float(bits[k] << 16), sums[j][2 * k]);
-                sums[j][2 * k + 1] = fmaf(weight, __uint_as_float(bits[k] & 0xffff0000u), sums[j][2 * k + 1]);
+                for (int j = 0; j < MERGE_PIECES; ++j) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        sums[j][2 * k] = fmaf(weight, __uint_as_float(bits[i][j][k] << 16), sums[j][2 * k]);
+                        sums[j][2 * k + 1] = fmaf(weight, __uint_as_float(bits[i][j][k] & 0xffff0000u), sums[j][2 * k + 1]);
+                    }
+                }
             }
         }
     }
-    const float inverse = valid ? 1.0f / normaliser : 0.f;
-    // piece j of the quarter is registers 8*(j%2) .. +7 of column block d = 4*quarter + j/2: two runs of
+    const float inverse = 1.0f / normaliser;
+    // piece j of the slice is registers 8*(j%2) .. +7 of column block d = 2*slice + j/2: two runs of
     // four columns, output_column(d, 2*(j%2), g) and output_column(d, 2*(j%2) + 1, g)
 #pragma unroll
     for (int j = 0; j < MERGE_PIECES; ++j) {
@@ -727,22 +759,22 @@ __global__ __launch_bounds__(64) void mla_decode_merge_kernel(bf16_t* __restrict
             u32x2 packed;
             packed.x = pack_bf16(sums[j][4 * run] * inverse, sums[j][4 * run + 1] * inverse);
             packed.y = pack_bf16(sums[j][4 * run + 2] * inverse, sums[j][4 * run + 3] * inverse);
-            const int column = output_column(j / 2, 2 * (j % 2) + run, g);   // within the quarter's 128 columns
+            const int column = output_column(j / 2, 2 * (j % 2) + run, g);   // within the slice's 64 columns
             *reinterpret_cast<u32x2*>(staging + lq * MERGE_PITCH + 2 * column) = packed;
         }
     }
     __syncthreads();
-    // 32 rows x 256 bytes: 16 lanes per row, four rows per pass
+    // 32 rows x 128 bytes: 8 lanes per row, eight rows per pass
 #pragma unroll
-    for (int pass = 0; pass < 8; ++pass) {
-        const int r = 4 * pass + lane / 16;
+    for (int pass = 0; pass < 4; ++pass) {
+        const int r = 8 * pass + lane / 8;
         const int h = 32 * wave_block + r;
         if (h < heads) {
-            const u32x4 bits = *reinterpret_cast<const u32x4*>(staging + r * MERGE_PITCH + 16 * (lane % 16));
-            *reinterpret_cast<u32x4*>(output + ((size_t)sequence * heads + h) * RANK + quarter * MERGE_COLUMNS + 8 * (lane % 16)) = bits;
+            const u32x4 row_bits = *reinterpret_cast<const u32x4*>(staging + r * MERGE_PITCH + 16 * (lane % 8));
+            *reinterpret_cast<u32x4*>(output + ((size_t)sequence * heads + h) * RANK + slice * MERGE_COLUMNS + 8 * (lane % 8)) = row_bits;
         }
     }
-    if (quarter == 0 && valid && g == 0) {
+    if (slice == 0 && head < heads && g == 0) {
         logsumexp[(size_t)sequence * heads + head] = (reference + __builtin_amdgcn_logf(normaliser)) * LN2;
     }
 }
@@ -908,9 +940,8 @@ void mla_decode_dispatch(bf16_t* output, float* logsumexp, const bf16_t* query, 
                        layout.whole_sequences);
     HIP_CHECK(hipGetLastError());
     if (!layout.whole_sequences) {
-        hipLaunchKernelGGL(mla_decode_merge_kernel, dim3(MERGE_QUARTERS * (padded_rows / 32), batch_size), dim3(64), 0,
-                           stream, output, logsumexp, workspace, plan, batch_size, heads, layout.slot_floats,
-                           padded_rows);
+        hipLaunchKernelGGL(mla_decode_merge_kernel, dim3(MERGE_SLICES * (padded_rows / 32), batch_size), dim3(64), 0,
+                           stream, output, logsumexp, workspace, plan, heads, layout.slot_floats, padded_rows);
         HIP_CHECK(hipGetLastError());
     }
 }
