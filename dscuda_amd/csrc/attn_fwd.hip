@@ -161,7 +161,6 @@ __global__ __launch_bounds__(64 * QG * KG) void attention_forward_split_kernel(
     const int q0 = qb * C::BM;
     const int wave_q0 = q0 + 32 * query_group;
     const int q_row = wave_q0 + lq;
-    const unsigned q_stride_bytes = (unsigned)query_heads * DQK * 2;
     const unsigned k_stride_bytes = (unsigned)key_value_heads * DQK * 2;
     const unsigned v_stride_bytes = (unsigned)key_value_heads * DV * 2;
     const unsigned char* k_base =
@@ -190,10 +189,16 @@ __global__ __launch_bounds__(64 * QG * KG) void attention_forward_split_kernel(
     // The queries go where tile 1 will go, tile 0 to its own stage.
     bf16x8 qf[KSTEPS];   // B operand: column = query lq, k = 16*ks + 8*g + j
     {
-        TileRequests<C::K_ROW, C::WAVES, C::BM> q_requests;
-        q_requests.init(q_stride_bytes, wave, lane);
-        q_requests.request(reinterpret_cast<const unsigned char*>(query + (((size_t)b * S + q0) * query_heads + h) * DQK),
-                           q_stride_bytes, S - 1 - q0, lds_base + C::STAGE_BYTES, wave);
+        using Requests = TileRequests<C::K_ROW, C::WAVES, C::BM>;
+        const unsigned char* q_base = reinterpret_cast<const unsigned char*>(query + (((size_t)b * S + q0) * query_heads + h) * DQK);
+        if ((unsigned)query_heads <= 0xffffffffu / (C::BM * C::K_ROW)) {
+            const unsigned q_stride_bytes = (unsigned)query_heads * DQK * 2;
+            Requests q_requests;
+            q_requests.init(q_stride_bytes, wave, lane);
+            q_requests.request(q_base, q_stride_bytes, S - 1 - q0, lds_base + C::STAGE_BYTES, wave);
+        } else {   // rows of one tile more than 4 GiB apart
+            Requests::request_far(q_base, (size_t)query_heads * DQK * 2, S - 1 - q0, lds_base + C::STAGE_BYTES, wave);
+        }
         request_tile(0);
         wait_vector_memory<TileRequests<C::K_ROW, C::WAVES, C::TILE>::LOADS + TileRequests<C::V_ROW, C::WAVES, C::TILE>::LOADS>();
         workgroup_barrier();   // the query tile has landed
@@ -892,10 +897,9 @@ void attention_forward_dispatch(bf16_t* output, float* logsumexp, const bf16_t* 
                                 const bf16_t* value, int batch_size, int sequence_length, int query_heads,
                                 int key_value_heads, int qk_head_size, int v_head_size, float scale,
                                 hipStream_t stream) {
-    // Offsets of the lanes inside a tile of 128 rows (keys or queries) are 32-bit, items and workgroups are counted in ints.
-    const long long widest = 2LL * std::max(qk_head_size, v_head_size) * std::min(sequence_length, 128);
-    if (widest * std::max(query_heads, key_value_heads) > 0xffffffffLL) {
-        throw std::invalid_argument("attention forward: heads * head size is too large");
+    // Offsets of the lanes inside a tile of 128 keys are 32-bit; items and workgroups are counted in ints.
+    if (2LL * std::max(qk_head_size, v_head_size) * key_value_heads * 64 > 0x7fffffffLL) {
+        throw std::invalid_argument("attention forward: key_value_heads * head size is too large");
     }
     const long long batch_heads = (long long)batch_size * query_heads;
     const long long blocks64 = (sequence_length + 63LL) / 64, blocks128 = (sequence_length + 127LL) / 128;

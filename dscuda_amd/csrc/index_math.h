@@ -139,11 +139,13 @@ struct TileRequestMath {
 
     // general form: byte offset of lane `lane` of load `load` from the tile's first row; rows past
     // `row_limit` repeat that row
+    DSCUDA_HOST_DEVICE static int row_of(int load, int lane) { return (64 * load + lane) / CHUNKS; }
+    DSCUDA_HOST_DEVICE static int chunk_of(int load, int lane) {
+        return ((64 * load + lane) % CHUNKS) ^ tile_swizzle<ROW_BYTES>(row_of(load, lane));
+    }
     DSCUDA_HOST_DEVICE static unsigned offset_of(int load, int lane, unsigned row_stride, int row_limit) {
-        const int slot = 64 * load + lane;
-        const int row = slot / CHUNKS;
-        const int chunk = (slot % CHUNKS) ^ tile_swizzle<ROW_BYTES>(row);
-        return (unsigned)(row_limit < row ? row_limit : row) * row_stride + 16u * chunk;
+        const int row = row_of(load, lane);
+        return (unsigned)(row_limit < row ? row_limit : row) * row_stride + 16u * chunk_of(load, lane);
     }
     // fast form, full tiles only: per-lane base of residue r (computed once per kernel) ...
     DSCUDA_HOST_DEVICE static unsigned base_of(int r, int lane, unsigned row_stride, int wave) {

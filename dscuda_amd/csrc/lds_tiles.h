@@ -54,6 +54,18 @@ struct TileRequests {
             }
         }
     }
+    // The same for a row stride whose tile may span more than 32 bits of address, a 64-bit address per lane and load:
+    // for tiles that are loaded once.
+    static __device__ __forceinline__ void request_far(const unsigned char* tile, size_t row_stride, int row_limit,
+                                                       unsigned lds_target, int wave) {
+        const int lane = fresh_lane_id();
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            const int load = wave * LOADS + i;
+            direct_load_16(tile + (size_t)min(Math::row_of(load, lane), row_limit) * row_stride + 16 * Math::chunk_of(load, lane),
+                           lds_target + load * 1024);
+        }
+    }
 };
 
 // Per-lane byte offsets of the fragment reads of a row-major swizzled tile

@@ -61,3 +61,21 @@ def test_parts_with_distant_maxima(cuda, heads):
     largest = v.float().abs().max().item()
     assert (out.cpu().float() - expected).abs().max().item() <= (2 * 2 ** -9 + weights) * largest
     assert ((lse.cpu() - expected_lse).abs() / expected_lse.abs().clamp_min(1)).max().item() <= 1e-5
+
+
+@pytest.mark.parametrize("seq,heads,dim", [(64, 600000, 64), (128, 140000, 128), (192, 280000, 128)])
+def test_query_rows_four_gigabytes_apart(cuda, seq, heads, dim):
+    """One key/value head for so many query heads that the last query row of a tile (64 rows, 128, and a last one of 64)
+    lies more than 4 GiB behind its first."""
+    rows = 128 if seq == 128 else 64
+    assert (rows - 1) * heads * dim * 2 > 2 ** 32
+    g = torch.Generator(device=cuda).manual_seed(5)
+    q = torch.empty(1, seq, heads, dim, device=cuda, dtype=torch.bfloat16).normal_(0, 0.5, generator=g)
+    k, v = (torch.empty(1, seq, 1, dim, device=cuda, dtype=torch.bfloat16).normal_(0, 0.5, generator=g) for _ in range(2))
+    scale = configs.c_float(dim ** -0.5)
+    announce("query rows far apart", dict(S=seq, Hq=heads, D=dim))
+    out, lse = ops.flash_forward(q, k, v, scale)
+    sample = [0, heads // 2, heads - 1]
+    expected, expected_lse = oracle.causal_attention_forward(q[:, :, sample].cpu(), k.cpu(), v.cpu(), scale)
+    assert_close_bf16("O", out[:, :, sample], expected)
+    assert_close_lse("LSE", lse[:, sample], expected_lse)
