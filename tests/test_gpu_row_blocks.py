@@ -93,3 +93,20 @@ def test_forward_raised_reference(cuda, tokens, heads):
     assert expected_lse.max() > 500
     assert_rounded(out, expected, expected_lse, c)
     assert ((lse.cpu() - expected_lse).abs() / expected_lse.abs().clamp_min(1)).max().item() <= 1e-5
+
+
+@pytest.mark.parametrize("parts", [2, 15, 16, 17, 32, 33, 63, 64, 65, 81, 128])
+def test_decode_merge_of_many_parts(cuda, parts):
+    """One sequence cut into as many parts as it has tiles: rows are merged 16 parts, statistics 64 parts at a time."""
+    heads, tokens = 3, 64 * parts - 5
+    g = torch.Generator().manual_seed(parts)
+    query = (torch.randn(1, 1, heads, 576, generator=g) * 0.25).bfloat16()
+    cache = (torch.randn(1, tokens, 576, generator=g) * 0.25).bfloat16()
+    paged, table = configs.pack_cache(cache, 64)
+    lengths = torch.tensor([tokens], dtype=torch.int32)
+    scale = configs.c_float(576 ** -0.5)
+    announce("decode, merge of many parts", dict(T=tokens, H=heads))
+    out, lse = ops.mla_decode(query.to(cuda), paged.to(cuda), table.to(cuda), lengths.to(cuda), scale, splits=128)
+    expected, expected_lse = oracle.mla_decode_unrounded(query, cache, lengths, scale)
+    assert_close_bf16("O", out, expected)
+    assert_close_lse("LSE", lse, expected_lse)
