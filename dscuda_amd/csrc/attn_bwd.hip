@@ -1016,10 +1016,8 @@ BackwardShape backward_shape(int batch_size, int sequence_length, int heads, int
     if (chunk < 1) chunk = 1;
     shape.pairs_per_launch = chunk < shape.pairs ? chunk : shape.pairs;
     shape.ds_floats = shape.pairs_per_launch * shape.sharing * ds_block_count(shape.key_blocks, shape.query_tiles) * DS_BLOCK_FLOATS;
-    // two workgroups of the first pass share a compute unit where their stages leave room in LDS
-    const int per_unit = 1;
-    shape.cut = index_math::choose_walk_cut(shape.pairs_per_launch, shape.key_blocks, shape.query_tiles, shape.sharing,
-                                            256 * per_unit);
+    // one workgroup of the first pass per compute unit (the workspace's size is asked for without a device: 256 units)
+    shape.cut = index_math::choose_walk_cut(shape.pairs_per_launch, shape.key_blocks, shape.query_tiles, shape.sharing, 256);
     shape.partial_floats = shape.cut.part_steps > 0
         ? shape.pairs_per_launch * shape.cut.items * KBLOCK * (qk_head_size + v_head_size) : 0;
     // the sums of the parts stay inside a budget that the caller has set
