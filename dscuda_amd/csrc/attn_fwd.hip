@@ -929,12 +929,15 @@ void attention_forward_dispatch(bf16_t* output, float* logsumexp, const bf16_t* 
         DSCUDA_FWD_SPLIT(64, 64, 2, 4);
         return;
     }
-    // Persistent kernel or split keys: the tiles of the busiest workgroup against the steps (128 queries x 128 keys, 1.1
-    // tiles each, start and end of a workgroup 2.5 more) of the mean or the longest one.  Both sides of the line, split
-    // against persistent: 32 heads of 5120 tokens 269 / 254 us, 128 heads of 1152 tokens 78 / 81, 64 of 2048 100 / 91,
-    // 32 of 3313 121 / 118 (estimated), 16 of 1000 21 / 41 (estimated).
+    // Persistent kernel or split keys: the tiles of the busiest workgroup against the steps (128 queries x 128 keys, 1.15
+    // tiles each, start and end of a workgroup 2.5 more) of the mean or the longest one.  Measured with either kernel
+    // forced, split / persistent in us, 192/128 columns: 16 heads of 1000 tokens 15.5 / 31.6, 128 of 1152 75.6 / 78.3,
+    // 32 of 3313 120 / 109, 64 of 2048 97 / 90, 128 of 1700 157 / 144.  Where the two costs are within 5 %: 16 of 6573
+    // 232 / 217, 40 of 5137 352 / 334, 32 of 5137 284 / 271, 48 of 3545 205 / 198, 128 of 2154 235 / 227, but 64 of 1301
+    // 53 / 55 and 96 of 2154 165 / 167; 128/128 columns: 40 of 5120 274 / 256, 32 of 5120 220 / 211, but 96 of 1664
+    // 86 / 89.
     const double mean_steps = (double)batch_heads * (0.5 * blocks128 * (blocks128 + 1) + 2.5 * blocks128) / compute_units;
-    const double split_cost = 1.1 * std::max(mean_steps, blocks128 + 2.5);
+    const double split_cost = 1.15 * std::max(mean_steps, blocks128 + 2.5);
     PingPongPlan plan = {};
     bool persistent = false;
     // the persistent kernel streams two tiles ahead across items: every item needs two tiles
