@@ -139,7 +139,6 @@ __global__ __launch_bounds__(64 * QG * KG) void attention_forward_split_kernel(
     constexpr int QK_MFMAS = MB * KSTEPS;
     constexpr int PV_MFMAS = NSTEPS * DBLOCKS;
     constexpr int RING = QK_MFMAS >= 8 ? 8 : 4;            // fragments read ahead of the product that takes them
-    constexpr float LOWEST = -1e30f;   // below every score, finite: a key group may hold no visible key of a row
 
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
 
@@ -213,7 +212,9 @@ __global__ __launch_bounds__(64 * QG * KG) void attention_forward_split_kernel(
 #pragma unroll
         for (int i = 0; i < 16; ++i) o_acc[d][i] = 0.f;
     }
-    float row_max = LOWEST;    // reference point of the exponent, raw score units
+    // Reference point of the exponent, raw score units.  Parts and query groups start at multiples of 32, so a part that
+    // is walked shows every row a key and leaves a number here; -inf stays only with a key group that walked none.
+    float row_max = -INFINITY;
     float row_sum = 0.f;       // this lane's share of the normaliser
     const float c = scale * LOG2E;
 

@@ -63,6 +63,28 @@ def test_parts_with_distant_maxima(cuda, heads):
     assert ((lse.cpu() - expected_lse).abs() / expected_lse.abs().clamp_min(1)).max().item() <= 1e-5
 
 
+@pytest.mark.parametrize("heads", [2, 72])   # 64 and 128 queries per workgroup
+def test_scores_far_below_zero_under_a_small_scale(cuda, heads):
+    """Raw scores of -4e33 under a scale that brings them to some -400: the running maximum has to start below every
+    score, and key groups that a row's queries never reach must not count."""
+    seq = 200
+    g = torch.Generator().manual_seed(4)
+    randn = lambda dim: torch.randn(1, seq, heads, dim, generator=g)
+    q = (2.0 ** 52 * (1 + 0.05 * randn(192))).bfloat16()
+    k = (-2.0 ** 52 * (1 + 0.05 * randn(192))).bfloat16()
+    v = randn(128).bfloat16()
+    scale = configs.c_float(1e-31)
+    announce("scores far below zero", dict(H=heads))
+    out, lse = ops.mla_prefill_forward(q.to(cuda), k.to(cuda), v.to(cuda), scale)
+    expected, expected_lse = oracle.causal_attention_forward(q, k, v, scale)
+    assert expected_lse.max() < -300
+    # the weights carry the fp32 error of the scores: twelve partial sums and the scaling, 2^-24 of the score each
+    weights = 16 * 2 ** -24 * expected_lse.abs().max().item()
+    largest = v.float().abs().max().item()
+    assert (out.cpu().float() - expected).abs().max().item() <= (2 * 2 ** -9 + weights) * largest
+    assert ((lse.cpu() - expected_lse).abs() / expected_lse.abs()).max().item() <= 1e-5
+
+
 @pytest.mark.parametrize("seq,heads,dim", [(64, 600000, 64), (128, 140000, 128), (192, 280000, 128)])
 def test_query_rows_four_gigabytes_apart(cuda, seq, heads, dim):
     """One key/value head for so many query heads that the last query row of a tile (64 rows, 128, and a last one of 64)
