@@ -9,6 +9,8 @@
 
 #include <cstddef>
 
+#include "index_math.h"
+
 namespace dscuda {
 
 // attn_fwd.hip -- causal forward, per-head K/V (flash attention and MLA prefill).
@@ -97,13 +99,13 @@ void mla_decode_dispatch(__hip_bfloat16* output, float* logsumexp, const __hip_b
                          int pages_per_sequence, int splits, float scale, hipStream_t stream);
 
 // mla_narrow.hip -- the same two operations with 32 * row_blocks (row_blocks 1 or 2) rows per workgroup, for work that
-// leaves most of the chip idle at 128 rows; the dispatch functions above choose.  The decode arguments are those of
+// leaves most of the chip idle at 128 rows; the dispatch functions above choose.  `layout` is that of
 // index_math::narrow_decode_layout; `own_plan`: the kernel works the plan out itself and leaves it at `plan`.
 void mla_narrow_decode_launch(__hip_bfloat16* output, float* logsumexp, const __hip_bfloat16* query,
                               const __hip_bfloat16* paged_kv_cache, const int* block_table, const int* cache_lengths,
                               float* workspace, int* plan, int batch_size, int heads, int page_size,
-                              int pages_per_sequence, int row_blocks, int workgroups, int whole_sequences,
-                              long long slot_floats, bool own_plan, float scale, hipStream_t stream);
+                              int pages_per_sequence, int row_blocks, const index_math::DecodeLayout& layout,
+                              bool own_plan, float scale, hipStream_t stream);
 
 void mla_narrow_forward_launch(__hip_bfloat16* output, float* logsumexp, const __hip_bfloat16* query_latent,
                                const __hip_bfloat16* query_rope, const __hip_bfloat16* kv_latent,

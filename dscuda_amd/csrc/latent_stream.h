@@ -259,10 +259,13 @@ __device__ __forceinline__ bf16x8 unit_value_fragment(const unsigned char* unit,
 // ---- decode: a workgroup's range of the work list -----------------------------------------------------------------
 
 using index_math::PLAN_HEADER;
+using index_math::PLAN_MODE;
 using index_math::PLAN_OVERHEAD;
+using index_math::PLAN_PARTS;
 using index_math::PLAN_RANGES;
 using index_math::PLAN_TOTAL;
 using index_math::PLAN_WHOLE;
+using index_math::PLAN_WIDE_PARTS;
 using index_math::PLAN_WORKGROUPS;
 
 constexpr int SELF_PLAN_BATCH = 256;   // sequences a workgroup turns into a plan by itself
@@ -272,32 +275,80 @@ struct DecodeRange {
     int overhead;
     int begin, end;      // positions of this workgroup's range; begin >= end: nothing to do
     int sequence;        // first sequence that reaches past `begin`
+    bool wide;           // parts of cut sequences are kept in fp32
 };
 
-// The plan comes from memory (own_workgroups == 0: the caller's, or one mla_decode_plan_kernel has just built), or,
+// How a call cuts its list (index_math::DecodeLayout).
+struct DecodeCut {
+    int workgroups;
+    int whole_sequences;
+    int reference_ranges;
+    int wide_ranges;
+};
+
+__device__ __forceinline__ int plan_mode(const DecodeCut& cut, bool wide) {
+    return cut.whole_sequences ? PLAN_WHOLE : wide ? PLAN_WIDE_PARTS : PLAN_PARTS;
+}
+
+// The ranges `total` positions are cut into, and whether with fp32 parts.  Called by all threads of a workgroup;
+// `prefix`: positions before each of the batch's sequences, visible to all of them; `fewest`: at most the positions of any
+// sequence that has some.  A run of as many tiles as the longest range has positions holds a boundary: where that settles
+// it for the shortest sequence, no sequence is looked at (64-bit divisions and a barrier, 0.7 us of a call).
+__device__ __forceinline__ int choose_ranges(const DecodeCut& cut, const int* prefix, int batch_size, int total, int fewest,
+                                             int overhead, int tid, int threads, bool& wide) {
+    wide = false;
+    if (cut.reference_ranges > 0 && total > 0) {
+        const int reference = index_math::ranges_of(total, cut.reference_ranges);
+        if (fewest - overhead - 1 < (total + reference - 1) / reference) {
+            int all_cut = 1;
+            for (int s = tid; s < batch_size; s += threads) {
+                const int before = prefix[s], positions = prefix[s + 1] - before;
+                if (positions > 0 && !index_math::sequence_is_cut(total, reference, before, positions, overhead)) all_cut = 0;
+            }
+            if (__syncthreads_and(all_cut) == 0) {
+                wide = cut.wide_ranges > 0;
+                return wide ? index_math::ranges_of(total, cut.wide_ranges) : reference;
+            }
+        }
+    }
+    return index_math::ranges_of(total, cut.workgroups);
+}
+
+__device__ __forceinline__ int wave_min(int value) {
+#pragma unroll
+    for (int offset = 1; offset < 64; offset <<= 1) value = min(value, __shfl_xor(value, offset));
+    return value;
+}
+
+// The plan comes from memory (own_plan false: the caller's, or one mla_decode_plan_kernel has just built), or,
 // for a batch that one workgroup scans in one go, is worked out here by every workgroup for itself, which saves the
 // call a kernel launch; `leave_plan`: this workgroup then also writes what the merge kernel reads of it.  Called by
-// all threads of a workgroup of at least SELF_PLAN_BATCH threads; the three arrays are in LDS.
-__device__ __forceinline__ DecodeRange decode_range(int* plan, const int* cache_lengths, int batch_size, int own_workgroups,
-                                                    int own_whole, int* own_prefix, int* own_lengths, int* own_wave_totals,
-                                                    int tid, int workgroup, bool leave_plan) {
+// all threads of a workgroup of at least SELF_PLAN_BATCH threads; the three arrays (own_wave_totals: two ints per 64
+// sequences) are in LDS.
+__device__ __forceinline__ DecodeRange decode_range(int* plan, const int* cache_lengths, int batch_size, bool own_plan,
+                                                    const DecodeCut& cut, int* own_prefix, int* own_lengths,
+                                                    int* own_wave_totals, int tid, int threads, int workgroup, bool leave_plan) {
     DecodeRange range;
     int total, ranges;
     bool whole_sequences;
-    if (own_workgroups > 0) {
-        whole_sequences = own_whole != 0;
+    if (own_plan) {
+        whole_sequences = cut.whole_sequences != 0;
         range.overhead = whole_sequences ? 0 : index_math::SEGMENT_OVERHEAD;
         int value = 0;
         if (tid < SELF_PLAN_BATCH) {
             const int own_length = tid < batch_size ? cache_lengths[tid] : 0;
             own_lengths[tid] = own_length;
             value = tid < batch_size ? index_math::positions_of(tiles_of(own_length), range.overhead) : 0;
+            const int fewest = cut.reference_ranges > 0 ? wave_min(value > 0 ? value : 0x7fffffff) : 0;
 #pragma unroll
             for (int offset = 1; offset < 64; offset <<= 1) {
                 const int other = __shfl_up(value, offset);
                 if (tid % 64 >= offset) value += other;
             }
-            if (tid % 64 == 63) own_wave_totals[tid / 64] = value;
+            if (tid % 64 == 63) {
+                own_wave_totals[tid / 64] = value;
+                own_wave_totals[SELF_PLAN_BATCH / 64 + tid / 64] = fewest;
+            }
             if (tid == 0) own_prefix[0] = 0;
         }
         __syncthreads();
@@ -312,14 +363,18 @@ __device__ __forceinline__ DecodeRange decode_range(int* plan, const int* cache_
         __syncthreads();
         // what comes out of LDS is the same in every lane, which the compiler cannot know
         total = __builtin_amdgcn_readfirstlane(own_prefix[batch_size]);
-        ranges = index_math::ranges_of(total, own_workgroups);
+        int fewest = own_wave_totals[SELF_PLAN_BATCH / 64];
+#pragma unroll
+        for (int w = 1; w < SELF_PLAN_BATCH / 64; ++w) fewest = min(fewest, own_wave_totals[SELF_PLAN_BATCH / 64 + w]);
+        fewest = __builtin_amdgcn_readfirstlane(fewest);
+        ranges = choose_ranges(cut, own_prefix, batch_size, total, fewest, range.overhead, tid, threads, range.wide);
         range.prefix = own_prefix;
         if (leave_plan) {
             if (tid == 0) {
                 plan[PLAN_TOTAL] = total;
-                plan[PLAN_WORKGROUPS] = own_workgroups;
+                plan[PLAN_WORKGROUPS] = cut.workgroups;
                 plan[PLAN_OVERHEAD] = range.overhead;
-                plan[PLAN_WHOLE] = own_whole;
+                plan[PLAN_MODE] = plan_mode(cut, range.wide);
                 plan[PLAN_RANGES] = ranges;
             }
             if (tid <= batch_size) plan[index_math::plan_prefix_at() + tid] = own_prefix[tid];
@@ -327,7 +382,8 @@ __device__ __forceinline__ DecodeRange decode_range(int* plan, const int* cache_
     } else {
         total = plan[PLAN_TOTAL];
         range.overhead = plan[PLAN_OVERHEAD];
-        whole_sequences = plan[PLAN_WHOLE] != 0;
+        whole_sequences = plan[PLAN_MODE] == PLAN_WHOLE;
+        range.wide = plan[PLAN_MODE] == PLAN_WIDE_PARTS;
         ranges = plan[PLAN_RANGES];
         range.prefix = plan + index_math::plan_prefix_at();
     }
@@ -343,14 +399,14 @@ __device__ __forceinline__ DecodeRange decode_range(int* plan, const int* cache_
         range.end = index_math::range_begin_of(total, ranges, workgroup + 1);
     }
     if (range.begin >= range.end) return range;
-    if (own_workgroups > 0 && !whole_sequences) {
+    if (own_plan && !whole_sequences) {
         int low = 0, high = batch_size;
         while (low < high) {
             const int mid = (low + high) / 2;
             if (__builtin_amdgcn_readfirstlane(range.prefix[mid + 1]) <= range.begin) low = mid + 1; else high = mid;
         }
         range.sequence = low;
-    } else if (own_workgroups > 0) {
+    } else if (own_plan) {
         range.sequence = workgroup;
     } else {
         range.sequence = plan[index_math::plan_first_sequence_at(batch_size) + workgroup];

@@ -485,7 +485,7 @@ __device__ __forceinline__ void walk_units(RowState& state, const bf16_t* query_
 // THREADS lengths.
 __global__ __launch_bounds__(THREADS) void mla_decode_plan_kernel(int* __restrict__ plan,
                                                                   const int* __restrict__ cache_lengths, int batch_size,
-                                                                  int workgroups, int whole_sequences) {
+                                                                  DecodeCut cut) {
     __shared__ int wave_totals[THREADS / 64];
     const int tid = threadIdx.x;
     const int lane = tid % 64;
@@ -493,6 +493,8 @@ __global__ __launch_bounds__(THREADS) void mla_decode_plan_kernel(int* __restric
     int* prefix = plan + index_math::plan_prefix_at();
     int* first_sequence = plan + index_math::plan_first_sequence_at(batch_size);
 
+    const int workgroups = cut.workgroups;
+    const bool whole_sequences = cut.whole_sequences != 0;
     const int overhead = whole_sequences ? 0 : index_math::SEGMENT_OVERHEAD;
     int carry = 0;
     if (tid == 0) prefix[0] = 0;
@@ -518,15 +520,16 @@ __global__ __launch_bounds__(THREADS) void mla_decode_plan_kernel(int* __restric
         __syncthreads();
     }
     const int total = carry;
-    const int ranges = index_math::ranges_of(total, workgroups);
+    __syncthreads();   // the prefix written above is read back below
+    bool wide;
+    const int ranges = choose_ranges(cut, prefix, batch_size, total, 0, overhead, tid, THREADS, wide);
     if (tid == 0) {
         plan[PLAN_TOTAL] = total;
         plan[PLAN_WORKGROUPS] = workgroups;
         plan[PLAN_OVERHEAD] = overhead;
         plan[PLAN_RANGES] = ranges;
-        plan[PLAN_WHOLE] = whole_sequences;
+        plan[PLAN_MODE] = plan_mode(cut, wide);
     }
-    __syncthreads();   // the prefix written above is read back below
     for (int w = tid; w < workgroups; w += THREADS) {
         int sequence = w;
         if (!whole_sequences) {
@@ -556,12 +559,12 @@ __global__ __launch_bounds__(THREADS) void mla_decode_split_kernel(
     bf16_t* __restrict__ output, float* __restrict__ logsumexp, const bf16_t* __restrict__ query,
     const bf16_t* __restrict__ paged_kv_cache, const int* __restrict__ block_table,
     const int* __restrict__ cache_lengths, float* __restrict__ workspace, int* __restrict__ plan, int batch_size,
-    int heads, int page_size, int pages_per_sequence, long long slot_floats, int padded_rows, float scale,
-    int own_workgroups, int own_whole) {
+    int heads, int page_size, int pages_per_sequence, long long slot_floats, int padded_rows, float scale, bool own_plan,
+    DecodeCut cut) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     __shared__ int own_prefix[SELF_PLAN_BATCH + 1];
     __shared__ int own_lengths[SELF_PLAN_BATCH];   // saves the walk a round trip to memory for its sequence's length
-    __shared__ int own_wave_totals[THREADS / 64];
+    __shared__ int own_wave_totals[2 * SELF_PLAN_BATCH / 64];
 
     const int tid = threadIdx.x;
     const int lane = tid % 64;
@@ -576,8 +579,8 @@ __global__ __launch_bounds__(THREADS) void mla_decode_split_kernel(
     const int head0 = head_group * ROWS;
     const float c = uniform(scale * LOG2E);
 
-    const DecodeRange range = decode_range(plan, cache_lengths, batch_size, own_workgroups, own_whole, own_prefix, own_lengths,
-                                           own_wave_totals, tid, workgroup, blockIdx.x == 0 && blockIdx.y == 0);
+    const DecodeRange range = decode_range(plan, cache_lengths, batch_size, own_plan, cut, own_prefix, own_lengths,
+                                           own_wave_totals, tid, THREADS, workgroup, blockIdx.x == 0 && blockIdx.y == 0);
     const int range_begin = range.begin, range_end = range.end, overhead = range.overhead;
     const int* prefix = range.prefix;
     if (range_begin >= range_end) return;
@@ -609,7 +612,7 @@ __global__ __launch_bounds__(THREADS) void mla_decode_split_kernel(
             ++sequence;
             continue;
         }
-        const int tokens = own_workgroups > 0 ? __builtin_amdgcn_readfirstlane(own_lengths[sequence]) : cache_lengths[sequence];
+        const int tokens = own_plan ? __builtin_amdgcn_readfirstlane(own_lengths[sequence]) : cache_lengths[sequence];
         const bool whole = tile_begin == 0 && tile_end == sequence_end - sequence_begin - overhead;
         const bf16_t* query_row = query + ((size_t)sequence * heads + row) * WIDTH;
 
@@ -891,13 +894,17 @@ DecodeChoice decode_choice(int batch_size, int heads, int splits) {
     return choice;
 }
 
+DecodeCut cut_of(const index_math::DecodeLayout& layout) {
+    return DecodeCut{layout.workgroups, layout.whole_sequences, layout.reference_ranges, layout.wide_ranges};
+}
+
 }  // namespace
 
 void mla_decode_plan_dispatch(int* plan, const int* cache_lengths, int batch_size, int heads, int splits,
                               hipStream_t stream) {
     const index_math::DecodeLayout layout = decode_choice(batch_size, heads, splits).layout;
     hipLaunchKernelGGL(mla_decode_plan_kernel, dim3(1), dim3(THREADS), 0, stream, plan, cache_lengths, batch_size,
-                       layout.workgroups, layout.whole_sequences);
+                       cut_of(layout));
     HIP_CHECK(hipGetLastError());
 }
 
@@ -920,14 +927,14 @@ void mla_decode_dispatch(bf16_t* output, float* logsumexp, const bf16_t* query, 
             own_plan = true;
         } else {
             hipLaunchKernelGGL(mla_decode_plan_kernel, dim3(1), dim3(THREADS), 0, stream, plan, cache_lengths, batch_size,
-                               layout.workgroups, layout.whole_sequences);
+                               cut_of(layout));
             HIP_CHECK(hipGetLastError());
         }
     }
     if (choice.row_blocks != 0) {
         mla_narrow_decode_launch(output, logsumexp, query, paged_kv_cache, block_table, cache_lengths, workspace, plan,
-                                 batch_size, heads, page_size, pages_per_sequence, choice.row_blocks, layout.workgroups,
-                                 layout.whole_sequences, layout.slot_floats, own_plan, scale, stream);
+                                 batch_size, heads, page_size, pages_per_sequence, choice.row_blocks, layout, own_plan, scale,
+                                 stream);
         return;
     }
     static hip_common::OncePerDevice prepared;
@@ -936,8 +943,7 @@ void mla_decode_dispatch(bf16_t* output, float* logsumexp, const bf16_t* query, 
     const dim3 grid(layout.workgroups, layout.head_groups);
     hipLaunchKernelGGL(mla_decode_split_kernel, grid, dim3(THREADS), LDS_BYTES, stream, output, logsumexp, query,
                        paged_kv_cache, block_table, cache_lengths, workspace, plan, batch_size, heads, page_size,
-                       pages_per_sequence, layout.slot_floats, padded_rows, scale, own_plan ? layout.workgroups : 0,
-                       layout.whole_sequences);
+                       pages_per_sequence, layout.slot_floats, padded_rows, scale, own_plan, cut_of(layout));
     HIP_CHECK(hipGetLastError());
     if (!layout.whole_sequences) {
         hipLaunchKernelGGL(mla_decode_merge_kernel, dim3(MERGE_SLICES * (padded_rows / 32), batch_size), dim3(64), 0,

@@ -40,7 +40,8 @@ namespace {
 constexpr int NARROW_THREADS = 512;
 constexpr int SCORE_STEPS = WIDTH / 32;       // 18
 constexpr int OUT_BLOCKS = RANK / 32 / 4;     // 32-column blocks of an output wave: 4
-constexpr int STAGE_PITCH = 2 * RANK + 16;    // bytes per staged output row
+constexpr int STAGE_PITCH = 2 * RANK + 16;    // bytes per staged output row ...
+constexpr int WIDE_PITCH = 4 * RANK + 16;     // ... and per fp32 row of a part
 constexpr int SCORE_RING = 6;                 // key fragments read ahead of the product that takes them
 constexpr int VALUE_RING = 4;
 
@@ -59,7 +60,7 @@ struct NarrowLayout {
     static constexpr int SUM_AT = FACTOR_AT + ROWS * 4;                 // [2][ROWS]
     static constexpr int FLAG_AT = SUM_AT + 2 * ROWS * 4;               // [2]
     static constexpr int LDS_BYTES = FLAG_AT + 16;
-    static_assert(ROWS * STAGE_PITCH <= UNIT_SLOTS * UNIT_BYTES, "the staged rows take the place of the units");
+    static_assert(ROWS * WIDE_PITCH <= UNIT_SLOTS * UNIT_BYTES, "the staged rows take the place of the units");
 };
 
 typedef short narrow_s16x4 __attribute__((ext_vector_type(4)));
@@ -83,13 +84,14 @@ struct NarrowRow {
 };
 
 // One walk over tiles [tile_begin, tile_end) of one key stream for ROWS rows.  On return the
-// staged rows lie in LDS at row * STAGE_PITCH (bf16, normalised if `normalise`), `reference`
-// and `total` are set in the lanes of the score waves (of row 16 * group + lane % 16), all
-// waves have passed a barrier, and the caller owes one more before the next walk.
+// staged rows lie in LDS at row * STAGE_PITCH (bf16, normalised if `normalise`) or, if `wide`,
+// at row * WIDE_PITCH (fp32, not normalised), `reference` and `total` are set in the lanes of the
+// score waves (of row 16 * group + lane % 16), all waves have passed a barrier, and the caller
+// owes one more before the next walk.
 template <int RB, bool PREFILL>
 __device__ __forceinline__ void narrow_walk(const NarrowRow& row, unsigned char* lds, const KeyStream& keys, int tile_begin,
-                                            int tile_end, int tokens, float c, bool normalise, int wave, float& reference,
-                                            float& total) {
+                                            int tile_end, int tokens, float c, bool normalise, bool wide, int wave,
+                                            float& reference, float& total) {
     using L = NarrowLayout<RB>;
     constexpr int ROWS = L::ROWS;
     const int last_token = tokens - 1;
@@ -326,6 +328,18 @@ __device__ __forceinline__ void narrow_walk(const NarrowRow& row, unsigned char*
             if (normalise) {
                 inverse = 1.0f / (RB == 1 ? sums[32 * b + lq] + sums[ROWS + 32 * b + lq] : sums[32 * b + lq]);
             }
+            if (wide) {
+                unsigned char* row_parts = lds + (32 * b + lq) * WIDE_PITCH + 4 * (128 * v + 4 * g);
+#pragma unroll
+                for (int d = 0; d < OUT_BLOCKS; ++d) {
+#pragma unroll
+                    for (int i4 = 0; i4 < 4; ++i4) {
+                        *reinterpret_cast<f32x4*>(row_parts + 4 * (32 * d + 8 * i4)) =
+                            f32x4{out[d][b][4 * i4], out[d][b][4 * i4 + 1], out[d][b][4 * i4 + 2], out[d][b][4 * i4 + 3]};
+                    }
+                }
+                continue;
+            }
             unsigned char* staged = lds + (32 * b + lq) * STAGE_PITCH + 2 * (128 * v + 4 * g);
 #pragma unroll
             for (int d = 0; d < OUT_BLOCKS; ++d) {
@@ -356,24 +370,42 @@ __device__ __forceinline__ void store_staged_rows(const unsigned char* lds, int 
     }
 }
 
+// The same for fp32 rows, two instructions a row.
+template <int ROWS, typename RowPointer>
+__device__ __forceinline__ void store_wide_rows(const unsigned char* lds, int wave, RowPointer destination) {
+    const int lane = fresh_lane_id();
+#pragma unroll
+    for (int i = 0; i < ROWS / 8; ++i) {
+        const int row = 8 * i + wave;
+        float* to = destination(row);
+        if (to != nullptr) {
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+                *reinterpret_cast<f32x4*>(to + 256 * half + 4 * lane) =
+                    *reinterpret_cast<const f32x4*>(lds + row * WIDE_PITCH + 1024 * half + 16 * lane);
+            }
+        }
+    }
+}
+
 // ----------------------------------------------------------------------------
 // decode
 // ----------------------------------------------------------------------------
 
-// A partial result lies in slot range + sequence of the workspace (index_math.h): one bf16 row
-// of 512 per head, then (reference, sum) per head.
+// A partial result lies in slot range + sequence of the workspace (index_math.h): one row of 512 per head, bf16 or, in
+// a wide plan, fp32, then (reference, sum) per head.
 template <int RB>
 __global__ __launch_bounds__(NARROW_THREADS) void mla_narrow_decode_kernel(
     bf16_t* __restrict__ output, float* __restrict__ logsumexp, const bf16_t* __restrict__ query,
     const bf16_t* __restrict__ paged_kv_cache, const int* __restrict__ block_table,
     const int* __restrict__ cache_lengths, float* __restrict__ workspace, int* __restrict__ plan, int batch_size,
-    int heads, int page_size, int pages_per_sequence, long long slot_floats, float scale, int own_workgroups,
-    int own_whole) {
+    int heads, int page_size, int pages_per_sequence, long long slot_floats, long long wide_slot_floats, float scale,
+    bool own_plan, DecodeCut cut) {
     using L = NarrowLayout<RB>;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     __shared__ int own_prefix[SELF_PLAN_BATCH + 1];
     __shared__ int own_lengths[SELF_PLAN_BATCH];
-    __shared__ int own_wave_totals[SELF_PLAN_BATCH / 64];
+    __shared__ int own_wave_totals[2 * SELF_PLAN_BATCH / 64];
 
     const int tid = threadIdx.x;
     const int lane = tid % 64;
@@ -383,8 +415,8 @@ __global__ __launch_bounds__(NARROW_THREADS) void mla_narrow_decode_kernel(
     const float c = scale * LOG2E;
 
     if (tid < 2) *reinterpret_cast<volatile int*>(lds + L::FLAG_AT + 4 * tid) = 0;
-    const DecodeRange range = decode_range(plan, cache_lengths, batch_size, own_workgroups, own_whole, own_prefix, own_lengths,
-                                           own_wave_totals, tid, workgroup, blockIdx.x == 0 && blockIdx.y == 0);
+    const DecodeRange range = decode_range(plan, cache_lengths, batch_size, own_plan, cut, own_prefix, own_lengths,
+                                           own_wave_totals, tid, NARROW_THREADS, workgroup, blockIdx.x == 0 && blockIdx.y == 0);
     if (range.begin >= range.end) return;
 
     int sequence = range.sequence;
@@ -404,7 +436,7 @@ __global__ __launch_bounds__(NARROW_THREADS) void mla_narrow_decode_kernel(
             ++sequence;
             continue;
         }
-        const int tokens = __builtin_amdgcn_readfirstlane(own_workgroups > 0 ? own_lengths[sequence] : cache_lengths[sequence]);
+        const int tokens = __builtin_amdgcn_readfirstlane(own_plan ? own_lengths[sequence] : cache_lengths[sequence]);
         const bool whole = tile_begin == 0 && tile_end == sequence_end - sequence_begin - range.overhead;
 
         KeyStream keys;
@@ -421,7 +453,8 @@ __global__ __launch_bounds__(NARROW_THREADS) void mla_narrow_decode_kernel(
         row.rope = row.latent + RANK;
         row.visible = tokens;
         float reference = 0.f, total = 1.f;
-        narrow_walk<RB, false>(row, lds, keys, tile_begin, tile_end, tokens, c, whole, wave, reference, total);
+        narrow_walk<RB, false>(row, lds, keys, tile_begin, tile_end, tokens, c, whole, !whole && range.wide, wave, reference,
+                               total);
 
         const bool writer = wave < (RB == 1 ? 2 : 4) && lane < 16 && row.valid;
         if (whole) {
@@ -430,14 +463,21 @@ __global__ __launch_bounds__(NARROW_THREADS) void mla_narrow_decode_kernel(
                 return head0 + r < heads ? output + ((size_t)sequence * heads + head0 + r) * RANK : nullptr;
             });
         } else {
-            float* slot = workspace + ((size_t)workgroup + sequence) * slot_floats;
+            float* slot = workspace + ((size_t)workgroup + sequence) * (range.wide ? wide_slot_floats : slot_floats);
             if (writer) {
-                slot[(size_t)heads * (RANK / 2) + 2 * head] = reference;
-                slot[(size_t)heads * (RANK / 2) + 2 * head + 1] = total;
+                float* statistics = slot + (size_t)heads * (range.wide ? RANK : RANK / 2) + 2 * head;
+                statistics[0] = reference;
+                statistics[1] = total;
             }
-            store_staged_rows<L::ROWS>(lds, wave, [&](int r) -> bf16_t* {
-                return head0 + r < heads ? reinterpret_cast<bf16_t*>(slot) + (size_t)(head0 + r) * RANK : nullptr;
-            });
+            if (range.wide) {
+                store_wide_rows<L::ROWS>(lds, wave, [&](int r) -> float* {
+                    return head0 + r < heads ? slot + (size_t)(head0 + r) * RANK : nullptr;
+                });
+            } else {
+                store_staged_rows<L::ROWS>(lds, wave, [&](int r) -> bf16_t* {
+                    return head0 + r < heads ? reinterpret_cast<bf16_t*>(slot) + (size_t)(head0 + r) * RANK : nullptr;
+                });
+            }
         }
         workgroup_barrier();   // the staged rows have been read: the next segment's units may come
         position = segment_end;
@@ -447,41 +487,37 @@ __global__ __launch_bounds__(NARROW_THREADS) void mla_narrow_decode_kernel(
 
 // Merge of the parts of every sequence that a range boundary cut: a wave per (sequence, head),
 // eight columns per lane.  The statistics of 64 parts (a lane each) and the rows of the first
-// MERGE_AHEAD come in one round trip, further rows MERGE_AHEAD at a time.  Against statistics first and
-// rows four at a time, whole calls: 64 sequences x 16 heads x 1024..8192 tokens 71.3 -> 68.7 us, 16 x 128 50.4 -> 48.8,
-// 8 x 8 x 3336 19.7 -> 18.9, one of 200 tokens x 128 heads 12.7 -> 12.0.
+// AHEAD come in one round trip, further rows AHEAD at a time (sixteen bf16 rows or eight fp32
+// rows: 64 registers).  Against statistics first and rows four at a time, whole calls: 64 sequences
+// x 16 heads x 1024..8192 tokens 71.3 -> 68.7 us, 16 x 128 50.4 -> 48.8, 8 x 8 x 3336 19.7 -> 18.9,
+// one of 200 tokens x 128 heads 12.7 -> 12.0.
 constexpr int MERGE_WAVES = 4;
-constexpr int MERGE_AHEAD = 16;
-static_assert(64 % MERGE_AHEAD == 0, "the statistics change between two requests of rows");
 
-__global__ __launch_bounds__(64 * MERGE_WAVES) void mla_narrow_merge_kernel(
-    bf16_t* __restrict__ output, float* __restrict__ logsumexp, const float* __restrict__ workspace,
-    const int* __restrict__ plan, int batch_size, int heads, long long slot_floats) {
-    const int lane = threadIdx.x % 64;
-    const int head = blockIdx.x * MERGE_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-    const int sequence = blockIdx.y;
-    if (head >= heads) return;
-    const int total = plan[PLAN_TOTAL];
-    const int overhead = plan[PLAN_OVERHEAD];
-    const int ranges = plan[PLAN_RANGES];
-    const int* prefix = plan + index_math::plan_prefix_at();
-    const int sequence_begin = prefix[sequence];
-    const int sequence_end = prefix[sequence + 1];
-    asm volatile("" ::"s"(total), "s"(overhead), "s"(ranges), "s"(sequence_end));   // one round trip, not two
-    if (sequence_end <= sequence_begin) return;   // no tiles: nothing was computed for it
-    int first, last;
-    index_math::ranges_of_sequence(total, ranges, sequence_begin, sequence_end - sequence_begin, overhead, first, last);
-    if (first == last) return;                    // finished in place
+struct MergedRow {
+    float sums[8];       // not normalised
+    float highest;       // reference of the sums
+    float normaliser;
+};
 
-    const float* slots = workspace + ((size_t)first + sequence) * slot_floats;
-    const size_t stats_offset = (size_t)heads * (RANK / 2) + 2 * head;
-    const int parts = last - first + 1;
-    const bf16_t* rows = reinterpret_cast<const bf16_t*>(slots) + (size_t)head * RANK + 8 * lane;
-    u32x4 bits[MERGE_AHEAD];
+template <bool WIDE>
+__device__ __forceinline__ MergedRow merge_parts(const float* slots, long long slot_floats, int parts, int heads, int head,
+                                                 int lane) {
+    constexpr int AHEAD = WIDE ? 8 : 16;
+    constexpr int PIECES = WIDE ? 2 : 1;   // of 16 bytes per lane and row
+    static_assert(64 % AHEAD == 0, "the statistics change between two requests of rows");
+    const size_t stats_offset = (size_t)heads * (WIDE ? RANK : RANK / 2) + 2 * head;
+    // the lane's eight columns of part 0
+    const float* rows = slots + (WIDE ? (size_t)head * RANK + 8 * lane : (size_t)head * (RANK / 2) + 4 * lane);
+    u32x4 bits[AHEAD][PIECES];
     auto request = [&](int part) {
 #pragma unroll
-        for (int i = 0; i < MERGE_AHEAD; ++i) {
-            if (part + i < parts) bits[i] = *reinterpret_cast<const u32x4*>(rows + (part + i) * (2 * slot_floats));
+        for (int i = 0; i < AHEAD; ++i) {
+            if (part + i < parts) {
+#pragma unroll
+                for (int j = 0; j < PIECES; ++j) {
+                    bits[i][j] = *reinterpret_cast<const u32x4*>(rows + (part + i) * slot_floats + 4 * j);
+                }
+            }
         }
     };
     // lane: statistics of part base + lane; those of the first 64 parts stay in registers
@@ -495,6 +531,7 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void mla_narrow_merge_kernel(
             lane_sum = stats[1];
         }
     };
+    MergedRow row;
     float highest = -INFINITY;
     for (int base = 64; base < parts; base += 64) {
         load_statistics(base);
@@ -506,11 +543,10 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void mla_narrow_merge_kernel(
 #pragma unroll
     for (int offset = 1; offset < 64; offset <<= 1) highest = fmaxf(highest, __shfl_xor(highest, offset));
     float normaliser = 0.f;
-    float sums[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) sums[k] = 0.f;
+    for (int k = 0; k < 8; ++k) row.sums[k] = 0.f;
     float weight = 0.f;
-    for (int part = 0; part < parts; part += MERGE_AHEAD) {
+    for (int part = 0; part < parts; part += AHEAD) {
         if (part > 0) request(part);
         if (part % 64 == 0) {
             if (part > 0) load_statistics(part);
@@ -518,25 +554,60 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void mla_narrow_merge_kernel(
             normaliser = fmaf(weight, lane_sum, normaliser);
         }
 #pragma unroll
-        for (int i = 0; i < MERGE_AHEAD; ++i) {
+        for (int i = 0; i < AHEAD; ++i) {
             if (part + i < parts) {
                 const float w = __shfl(weight, (part + i) % 64);
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
-                    sums[2 * k] = fmaf(w, __uint_as_float(bits[i][k] << 16), sums[2 * k]);
-                    sums[2 * k + 1] = fmaf(w, __uint_as_float(bits[i][k] & 0xffff0000u), sums[2 * k + 1]);
+                    if constexpr (WIDE) {
+                        row.sums[k] = fmaf(w, __uint_as_float(bits[i][0][k]), row.sums[k]);
+                        row.sums[4 + k] = fmaf(w, __uint_as_float(bits[i][1][k]), row.sums[4 + k]);
+                    } else {
+                        row.sums[2 * k] = fmaf(w, __uint_as_float(bits[i][0][k] << 16), row.sums[2 * k]);
+                        row.sums[2 * k + 1] = fmaf(w, __uint_as_float(bits[i][0][k] & 0xffff0000u), row.sums[2 * k + 1]);
+                    }
                 }
             }
         }
     }
 #pragma unroll
     for (int offset = 1; offset < 64; offset <<= 1) normaliser += __shfl_xor(normaliser, offset);
-    const float inverse = 1.0f / normaliser;
+    row.highest = highest;
+    row.normaliser = normaliser;
+    return row;
+}
+
+__global__ __launch_bounds__(64 * MERGE_WAVES) void mla_narrow_merge_kernel(
+    bf16_t* __restrict__ output, float* __restrict__ logsumexp, const float* __restrict__ workspace,
+    const int* __restrict__ plan, int batch_size, int heads, long long slot_floats, long long wide_slot_floats) {
+    const int lane = threadIdx.x % 64;
+    const int head = blockIdx.x * MERGE_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const int sequence = blockIdx.y;
+    if (head >= heads) return;
+    const int total = plan[PLAN_TOTAL];
+    const int overhead = plan[PLAN_OVERHEAD];
+    const int ranges = plan[PLAN_RANGES];
+    const int mode = plan[PLAN_MODE];
+    const int* prefix = plan + index_math::plan_prefix_at();
+    const int sequence_begin = prefix[sequence];
+    const int sequence_end = prefix[sequence + 1];
+    asm volatile("" ::"s"(total), "s"(overhead), "s"(ranges), "s"(mode), "s"(sequence_end));   // one round trip, not two
+    if (sequence_end <= sequence_begin) return;   // no tiles: nothing was computed for it
+    int first, last;
+    index_math::ranges_of_sequence(total, ranges, sequence_begin, sequence_end - sequence_begin, overhead, first, last);
+    if (first == last) return;                    // finished in place
+
+    const size_t slot = (size_t)first + sequence;
+    const int parts = last - first + 1;
+    const MergedRow row = mode == PLAN_WIDE_PARTS
+        ? merge_parts<true>(workspace + slot * wide_slot_floats, wide_slot_floats, parts, heads, head, lane)
+        : merge_parts<false>(workspace + slot * slot_floats, slot_floats, parts, heads, head, lane);
+    const float inverse = 1.0f / row.normaliser;
     u32x4 packed;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) packed[k] = pack_bf16(sums[2 * k] * inverse, sums[2 * k + 1] * inverse);
+    for (int k = 0; k < 4; ++k) packed[k] = pack_bf16(row.sums[2 * k] * inverse, row.sums[2 * k + 1] * inverse);
     *reinterpret_cast<u32x4*>(output + ((size_t)sequence * heads + head) * RANK + 8 * lane) = packed;
-    if (lane == 0) logsumexp[(size_t)sequence * heads + head] = (highest + __builtin_amdgcn_logf(normaliser)) * LN2;
+    if (lane == 0) logsumexp[(size_t)sequence * heads + head] = (row.highest + __builtin_amdgcn_logf(row.normaliser)) * LN2;
 }
 
 // ----------------------------------------------------------------------------
@@ -580,7 +651,7 @@ __global__ __launch_bounds__(NARROW_THREADS) void mla_narrow_forward_kernel(
     row.rope = query_rope + global_row * ROPE;
     row.visible = row.valid ? token + 1 : visible;
     float reference = 0.f, total = 1.f;
-    narrow_walk<RB, true>(row, lds, keys, 0, tiles_of(visible), visible, c, true, wave, reference, total);
+    narrow_walk<RB, true>(row, lds, keys, 0, tiles_of(visible), visible, c, true, false, wave, reference, total);
 
     if (wave < (RB == 1 ? 2 : 4) && lane < 16 && row.valid) {
         logsumexp[((size_t)batch * heads + (int)(at % heads)) * sequence_length + token] =
@@ -612,15 +683,15 @@ void prepare_narrow() {
 void mla_narrow_decode_launch(bf16_t* output, float* logsumexp, const bf16_t* query, const bf16_t* paged_kv_cache,
                               const int* block_table, const int* cache_lengths, float* workspace, int* plan,
                               int batch_size, int heads, int page_size, int pages_per_sequence, int row_blocks,
-                              int workgroups, int whole_sequences, long long slot_floats, bool own_plan, float scale,
-                              hipStream_t stream) {
+                              const index_math::DecodeLayout& layout, bool own_plan, float scale, hipStream_t stream) {
     prepare_narrow();
     const int rows = 32 * row_blocks;
-    const dim3 grid(workgroups, (heads + rows - 1) / rows);
+    const dim3 grid(layout.workgroups, (heads + rows - 1) / rows);
+    const DecodeCut cut = {layout.workgroups, layout.whole_sequences, layout.reference_ranges, layout.wide_ranges};
     auto launch = [&](auto kernel, int lds_bytes) {
         hipLaunchKernelGGL(kernel, grid, dim3(NARROW_THREADS), lds_bytes, stream, output, logsumexp, query, paged_kv_cache,
                            block_table, cache_lengths, workspace, plan, batch_size, heads, page_size, pages_per_sequence,
-                           slot_floats, scale, own_plan ? workgroups : 0, whole_sequences);
+                           layout.slot_floats, layout.wide_slot_floats, scale, own_plan, cut);
         HIP_CHECK(hipGetLastError());
     };
     if (row_blocks == 1) {
@@ -628,10 +699,10 @@ void mla_narrow_decode_launch(bf16_t* output, float* logsumexp, const bf16_t* qu
     } else {
         launch(mla_narrow_decode_kernel<2>, NarrowLayout<2>::LDS_BYTES);
     }
-    if (!whole_sequences) {
+    if (!layout.whole_sequences) {
         hipLaunchKernelGGL(mla_narrow_merge_kernel, dim3((heads + MERGE_WAVES - 1) / MERGE_WAVES, batch_size),
                            dim3(64 * MERGE_WAVES), 0, stream, output, logsumexp, workspace, plan, batch_size, heads,
-                           slot_floats);
+                           layout.slot_floats, layout.wide_slot_floats);
         HIP_CHECK(hipGetLastError());
     }
 }

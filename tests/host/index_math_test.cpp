@@ -539,6 +539,22 @@ void check_decode_layout() {
                         EXPECT(layout.slot_floats >= heads * (RANK / 2 + 2) && layout.slot_floats % 4 == 0, "narrow H %d", heads);
                         EXPECT(layout.whole_sequences ? layout.workgroups == batch : layout.workgroups >= 2 && layout.slots == layout.workgroups + batch,
                                "narrow B %d H %d splits %d", batch, heads, splits);
+                        // never more ranges with bf16 parts than the padded slots of decode_layout allow, unless the
+                        // fallback with fp32 parts is there for the sequences that those leave whole
+                        const DecodeLayout padded = decode_layout(batch, heads, splits, compute_units, ROWS, RANK);
+                        const int reference = padded.whole_sequences ? 1 : padded.workgroups;
+                        if (layout.whole_sequences || layout.workgroups <= reference) {
+                            EXPECT(layout.reference_ranges == 0, "narrow B %d H %d splits %d", batch, heads, splits);
+                            continue;
+                        }
+                        EXPECT(layout.reference_ranges == reference && layout.wide_ranges <= layout.workgroups &&
+                                   (layout.wide_ranges == 0 || layout.wide_ranges >= reference),
+                               "narrow B %d H %d splits %d", batch, heads, splits);
+                        EXPECT(layout.wide_slot_floats >= heads * (RANK + 2) && layout.wide_slot_floats % 4 == 0, "narrow H %d", heads);
+                        // in front of the plan; a single range leaves no parts
+                        EXPECT(layout.wide_ranges <= 1 || (layout.wide_ranges + batch) * layout.wide_slot_floats <= layout.plan_offset,
+                               "narrow B %d H %d splits %d: fp32 slots reach the plan", batch, heads, splits);
+                        EXPECT(layout.slots * layout.slot_floats <= layout.plan_offset, "narrow B %d H %d splits %d", batch, heads, splits);
                     }
                 }
             }

@@ -110,3 +110,31 @@ def test_decode_merge_of_many_parts(cuda, parts):
     expected, expected_lse = oracle.mla_decode_unrounded(query, cache, lengths, scale)
     assert_close_bf16("O", out, expected)
     assert_close_lse("LSE", lse, expected_lse)
+
+
+@pytest.mark.parametrize("batch,heads,splits,low,high", [
+    (1, 8, 8, 400, 400), (5, 8, 8, 33, 271), (3, 40, 8, 60, 300),   # more ranges than padded slots would allow
+    (8, 16, 2, 300, 2000), (2, 24, 2, 300, 300),
+    (300, 4, 2, 64, 200),                                            # the plan kernel
+])
+def test_sequences_that_fewer_ranges_leave_whole_are_rounded_once(cuda, batch, heads, splits, low, high):
+    """Probabilities and results are rounded to bf16, parts of these sequences are not.  A rounding errs evenly within
+    half a step of 2^-7 of the power of two below a value: 2^-7 / sqrt(12) over a root mean square of 1.36 (such powers)
+    is 1.66e-3 in the 2-norm.  Two independent ones make 2.35e-3, a third one, of the parts, 2.88e-3."""
+    g = torch.Generator().manual_seed(batch + heads)
+    lengths = torch.linspace(low, high, batch).int()
+    tokens = int(lengths.max())
+    query = (torch.randn(batch, 1, heads, 576, generator=g) * 0.5).bfloat16()
+    cache = (torch.randn(batch, tokens, 576, generator=g) * 0.5).bfloat16()
+    paged, table = configs.pack_cache(cache, 64)
+    scale = configs.c_float(192 ** -0.5)
+    announce("decode, parts in fp32", dict(B=batch, H=heads, splits=splits, lengths=(low, high)))
+    on_gpu = [x.to(cuda) for x in (query, paged, table, lengths)]
+    out, lse = ops.mla_decode(*on_gpu, scale, splits=splits)
+    plan = ops.mla_decode_plan(on_gpu[3], heads, splits)
+    planned, planned_lse = ops.mla_decode_planned(*on_gpu, plan, scale, splits=splits)
+    assert torch.equal(out, planned) and torch.equal(lse, planned_lse)
+    expected, expected_lse = oracle.mla_decode_unrounded(query.double(), cache.double(), lengths, scale)
+    error = (out.cpu().double() - expected).norm() / expected.norm()
+    assert error.item() <= 2.6e-3
+    assert_close_lse("LSE", lse, expected_lse)
