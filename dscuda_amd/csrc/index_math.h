@@ -610,6 +610,27 @@ DSCUDA_HOST_DEVICE inline int kept_chunk(int token_block, int key_block, int blo
     return blocks - 1 - token_block + key_block;
 }
 
+// ---- projections: do results lie over inputs ---------------------------------------
+// Rows of `width` elements, `tokens` x `heads` of them.
+struct ProjectionRows {
+    long long token_stride, head_stride;   // in elements
+    int width;
+
+    DSCUDA_HOST_DEVICE long long extent(long long tokens, int heads) const {
+        return (tokens - 1) * token_stride + (heads - 1) * head_stride + width;
+    }
+};
+
+// Whether no element of `y`, whose first row starts `offset` elements behind the first row of `x`, is one of `x`: apart in
+// memory, or different columns of the same rows.  False where that is not plain to see.
+DSCUDA_HOST_DEVICE inline bool rows_apart(const ProjectionRows& x, const ProjectionRows& y, long long offset,
+                                          long long tokens, int heads) {
+    if (offset >= x.extent(tokens, heads) || -offset >= y.extent(tokens, heads)) return true;
+    if (x.token_stride != y.token_stride || x.head_stride != y.head_stride || x.token_stride % x.head_stride != 0) return false;
+    const long long column = (offset % x.head_stride + x.head_stride) % x.head_stride;
+    return column >= x.width && column + y.width <= x.head_stride;
+}
+
 // ---- decode: the plan and how a call uses the caller's workspace ---------------
 // The plan is what a decode call needs to know about the lengths of its batch
 // before any workgroup starts: an int table

@@ -26,6 +26,7 @@
 
 #include "attn_kernels.h"
 #include "hip_common.h"
+#include "index_math.h"
 
 #include <algorithm>
 #include <cstdint>
@@ -422,10 +423,13 @@ int compute_units() {
 // (4096 tokens x 128 heads on 256 compute units: two chunks, one round, 138 / 171 us against 145 / 178 us with four).
 template <typename Kernel, typename FewKernel>
 void launch(Kernel kernel, FewKernel few_kernel, long long few_tiles, bf16_t* y, const bf16_t* x, const bf16_t* weight, long long tokens, int heads,
-            const Strides& strides, hipStream_t stream) {
+            const Strides& strides, int x_width, int y_width, hipStream_t stream) {
     check(heads <= 65535, "MLA projection: more heads than the grid allows");
     const long long tiles = (tokens + TILE - 1) / TILE;
-    if (tiles * heads <= few_tiles) {
+    const long long offset = ((long long)reinterpret_cast<uintptr_t>(y) - (long long)reinterpret_cast<uintptr_t>(x)) / 2;
+    const bool apart = index_math::rows_apart({strides.x_token, strides.x_head, x_width}, {strides.y_token, strides.y_head, y_width},
+                                              offset, tokens, heads);
+    if (apart && tiles * heads <= few_tiles) {
         hipLaunchKernelGGL(few_kernel, dim3((unsigned)(4 * heads), (unsigned)tiles), dim3(THREADS), 0, stream, y, x, weight,
                            tokens, strides);
         HIP_CHECK(hipGetLastError());
@@ -481,7 +485,8 @@ void mla_absorb_query_dispatch(bf16_t* query_latent, const bf16_t* query_nope, c
         HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(mla_absorb_query_kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES));
     });
-    launch(mla_absorb_query_kernel, mla_absorb_query_few_kernel, ABSORB_FEW_TILES, query_latent, query_nope, weight, tokens, heads, strides, stream);
+    launch(mla_absorb_query_kernel, mla_absorb_query_few_kernel, ABSORB_FEW_TILES, query_latent, query_nope, weight, tokens, heads, strides, HEAD,
+           RANK, stream);
 }
 
 void mla_unabsorb_output_dispatch(bf16_t* output, const bf16_t* output_latent, const bf16_t* weight, long long tokens,
@@ -496,7 +501,8 @@ void mla_unabsorb_output_dispatch(bf16_t* output, const bf16_t* output_latent, c
         HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(mla_unabsorb_output_kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES));
     });
-    launch(mla_unabsorb_output_kernel, mla_unabsorb_output_few_kernel, UNABSORB_FEW_TILES, output, output_latent, weight, tokens, heads, strides, stream);
+    launch(mla_unabsorb_output_kernel, mla_unabsorb_output_few_kernel, UNABSORB_FEW_TILES, output, output_latent, weight, tokens, heads, strides,
+           RANK, HEAD, stream);
 }
 
 }  // namespace dscuda

@@ -298,7 +298,8 @@ void rope_apply_cuda(
 // tensor lies at base + t * token_stride + h * head_stride (elements), so the absorb can read the nope
 // columns of a [B,S,H,192] query and write the latent columns of the packed [B,S,H,576] decode query
 // directly.  BF16 in and out, FP32 accumulation.  All tensors aligned to 16 bytes, all strides multiples
-// of 8 elements.
+// of 8 elements.  The result of a token and head may lie over its own input row (equal strides), over no
+// other row.
 void mla_absorb_query_cuda(
     __hip_bfloat16* query_latent,
     const __hip_bfloat16* query_nope,

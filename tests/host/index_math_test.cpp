@@ -567,6 +567,43 @@ void check_decode_layout() {
     EXPECT(decode_layout(5, 128, 1, 256, ROWS, RANK).whole_sequences == 1, "splits 1 must not cut");
 }
 
+// ---- projections: rows_apart never calls rows that share an element apart, and sees what is apart in the usual layouts
+void check_rows_apart() {
+    const long long strides[][2] = {{8, 8}, {24, 8}, {24, 12}, {30, 12}, {40, 8}};
+    for (long long tokens : {1, 2, 5}) {
+        for (int heads : {1, 2, 3}) {
+            for (auto& xs : strides) {
+                for (auto& ys : strides) {
+                    for (int x_width : {2, 8}) {
+                        for (int y_width : {2, 8}) {
+                            const ProjectionRows x = {xs[0], xs[1], x_width}, y = {ys[0], ys[1], y_width};
+                            for (long long offset = -250; offset <= 250; ++offset) {
+                                std::set<long long> elements;
+                                for (long long t = 0; t < tokens; ++t) {
+                                    for (int h = 0; h < heads; ++h) {
+                                        for (int c = 0; c < x_width; ++c) elements.insert(t * xs[0] + h * xs[1] + c);
+                                    }
+                                }
+                                bool shared = false;
+                                for (long long t = 0; t < tokens; ++t) {
+                                    for (int h = 0; h < heads; ++h) {
+                                        for (int c = 0; c < y_width; ++c) shared |= elements.count(offset + t * ys[0] + h * ys[1] + c) != 0;
+                                    }
+                                }
+                                EXPECT(!(shared && rows_apart(x, y, offset, tokens, heads)), "offset %lld of rows %d and %d", offset, x_width, y_width);
+                            }
+                        }
+                    }
+                }
+            }
+        }
+    }
+    const ProjectionRows nope = {16 * 704, 704, 128}, latent = {16 * 704, 704, 512};   // one buffer, nope | rope | latent
+    EXPECT(rows_apart(nope, latent, 192, 33, 16) && rows_apart(latent, nope, -192, 33, 16), "columns of one buffer");
+    EXPECT(!rows_apart(nope, latent, 0, 1, 1) && !rows_apart(nope, latent, 64, 4, 16), "a result over its input");
+    EXPECT(rows_apart(nope, latent, 33 * 16 * 704, 33, 16), "one buffer behind the other");
+}
+
 // ---- split-key forward: division by multiplication, every (batch, head, block) exactly once with its key/value head;
 // persistent forward: any number of heads abreast covers every item once, and the choice is never worse than the default
 void check_split_order() {
@@ -708,6 +745,7 @@ int main() {
     check_key_interval_choice();
     check_decode_ranges();
     check_decode_layout();
+    check_rows_apart();
     if (failures) {
         std::printf("%d check(s) failed\n", failures);
         return 1;

@@ -70,6 +70,28 @@ def test_projections_on_either_side_of_the_token_rule(cuda, tokens, heads):
     assert (result[:, tokens:].float() == 7.0).all() and (result[..., 128:].float() == 7.0).all()
 
 
+@pytest.mark.parametrize("tokens,heads", [(1, 128), (33, 7), (200, 3)])
+def test_projections_over_their_own_inputs(cuda, tokens, heads):
+    """The absorbed query over its nope columns, the output over the latent columns it comes from, and both beside them."""
+    wkv_b, g = _weights(heads, 59)
+    device_weights = wkv_b.to(cuda)
+    rows = (torch.randn(1, tokens, heads, 704, generator=g) * 0.5).bfloat16()
+    expected = oracle.absorb_query(rows[..., :128], wkv_b[:, :128])
+    expected_output = oracle.unabsorb_output(rows[..., :512], wkv_b[:, 128:])
+    announce("mla projections in place", dict(T=tokens, H=heads))
+    for _ in range(10):
+        over, beside = rows.to(cuda), rows.to(cuda)
+        ops.mla_absorb_query(over[..., :128], device_weights[:, :128], out=over[..., :512])
+        ops.mla_absorb_query(beside[..., :128], device_weights[:, :128], out=beside[..., 192:])
+        assert_close_bf16("over", over[..., :512].cpu(), expected)
+        assert_close_bf16("beside", beside[..., 192:].cpu(), expected)
+        over, beside = rows.to(cuda), rows.to(cuda)
+        ops.mla_unabsorb_output(over[..., :512], device_weights[:, 128:], out=over[..., 256:384])
+        ops.mla_unabsorb_output(beside[..., :512], device_weights[:, 128:], out=beside[..., 512:640])
+        assert_close_bf16("over", over[..., 256:384].cpu(), expected_output)
+        assert_close_bf16("beside", beside[..., 512:640].cpu(), expected_output)
+
+
 def test_projections_compose_with_decode(cuda):
     """An absorbed decode step between the two projections equals per-head attention over the expanded keys and
     values (the identity that makes absorption valid), within bf16 rounding of the intermediate tensors."""
