@@ -1,9 +1,11 @@
 // Causal attention forward for gfx950: S^T = K Q^T and O^T = V^T P^T on bf16
 // MFMA 32x32x16 tiles, online softmax in fp32, natural-log LSE.
 //
-// Two kernels serve the flash-attention forward (D = 64 / 128, GQA) and the
+// Three kernels serve the flash-attention forward (D = 64 / 128, GQA) and the
 // per-head MLA prefill forward (d_qk = 128 nope + 64 rope = 192, d_v = 128):
-// split keys for short and medium problems, a persistent one for large ones.
+// split keys for short and medium problems, a persistent one for large ones,
+// and small independent workgroups (four waves) for many heads of 64 columns or
+// of one tile of keys.
 // They take the place of the reference's
 // flash_attention_forward_tensor_core_kernel
 // (kernels/attention/flash_attention/sm89_forward.cu:99-205); the tiling is
@@ -24,7 +26,8 @@
 //   thread holds tile data in registers and nothing is written to LDS with
 //   store instructions.  With no padding possible inside the 1 KB a wave
 //   instruction fills, bank spread comes from a swizzle applied on the global
-//   side (which 16-byte chunk a lane fetches; in the persistent kernel, the other takes lds_tiles.h as it is):
+//   side: which 16-byte chunk a lane fetches.  The split-key kernel takes that of
+//   lds_tiles.h, the others
 //     K  : chunk c of row r sits at position c ^ fK(r).  A fragment read is 16
 //          lanes x 16 B down a column of rows; fK(r) = (r>>1)&7 for rows that
 //          are 128 (mod 256) bytes long, r&15 for rows that are 0 (mod 256).
@@ -63,8 +66,13 @@ struct FwdConfig {
     static constexpr int V_CHUNKS = DV / 8;
     static constexpr int V_GROUPS = DV / 32;               // 64-byte column groups per row
     static constexpr int V_BYTES = BN * V_ROW;
+    static constexpr int STAGE_BYTES = K_BYTES + V_BYTES;
     static constexpr int K_LOADS_PER_WAVE = K_BYTES / 1024 / NWAVES;   // wave instructions
     static constexpr int V_LOADS_PER_WAVE = V_BYTES / 1024 / NWAVES;
+    // four-wave kernel: two stages, then the output rows in their place
+    static constexpr int O_PITCH = DV * 2 + 16;            // bytes
+    static constexpr int O_BYTES = BM * O_PITCH;
+    static constexpr int LDS_BYTES = (2 * STAGE_BYTES > O_BYTES) ? 2 * STAGE_BYTES : O_BYTES;
     static_assert(K_BYTES % (1024 * NWAVES) == 0 && V_BYTES % (1024 * NWAVES) == 0,
                   "tile loads must divide evenly over the waves");
     static_assert(K_ROW % 128 == 0, "K rows must be a multiple of 128 bytes");
@@ -77,6 +85,265 @@ struct FwdConfig {
         return V_GROUPS == 4 ? (row & 3) : ((row >> 1) & 1);
     }
 };
+
+// ---------------------------------------------------------------------------
+// Four waves, 128 queries.
+//
+// Each wave owns 32 query rows for the whole key loop; keys are walked in tiles of 64 from key 0 up to the diagonal, two
+// stages.  A walk is one dependent chain of scores, softmax and output products per tile, twice to four times as long as
+// in the split-key kernel, but a workgroup of 64 columns takes 32 KB of LDS and a quarter of the waves of a compute unit:
+// with enough of them the others cover each chain, no output part crosses LDS, and start and end of a workgroup, 8000
+// cycles there, are cheap.  Bound by issue (matrix, softmax and LDS reads of two to four workgroups a unit).
+// Split keys -> four waves (us): 64 columns, 2048 heads of 128 tokens 35.9 -> 26.3, of 1024 tokens 592 -> 486; 512 heads
+// of 2048 tokens 463 -> 418; one tile of keys: 2048 heads of 64 tokens, 64 columns 18.1 -> 15.9, 192/128 columns
+// 51.7 -> 48.8, of one token 45.3 -> 34.2.
+template <int DQK, int DV, int NWAVES>
+__global__ __launch_bounds__(64 * NWAVES) void attention_forward_kernel(
+    bf16_t* __restrict__ output, float* __restrict__ logsumexp,
+    const bf16_t* __restrict__ query, const bf16_t* __restrict__ key, const bf16_t* __restrict__ value,
+    int sequence_length, int query_heads, int key_value_heads, int query_blocks, float scale) {
+    using C = FwdConfig<DQK, DV, NWAVES>;
+    constexpr int BN = C::BN;
+    constexpr int KSTEPS = DQK / 16;
+    constexpr int DBLOCKS = DV / 32;
+
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int lane = tid % 64;
+    const int lq = lane % 32;
+    const int g = lane / 32;
+
+    // (batch, head) groups are dealt across XCDs; inside a group the heaviest
+    // (last) query blocks are issued first.
+    int bh, qb_rank;
+    xcd_order(blockIdx.x, gridDim.x / query_blocks, query_blocks, bh, qb_rank);
+    const int qb = query_blocks - 1 - qb_rank;
+    const int b = bh / query_heads;
+    const int h = bh % query_heads;
+    const int hk = h / (query_heads / key_value_heads);
+    const int S = sequence_length;
+
+    const int q0 = qb * C::BM;
+    const int wave_q0 = q0 + 32 * wave;
+    const int q_row = wave_q0 + lq;
+
+    const size_t q_stride = (size_t)query_heads * DQK;
+    const unsigned k_stride_bytes = (unsigned)key_value_heads * DQK * 2;
+    const unsigned v_stride_bytes = (unsigned)key_value_heads * DV * 2;
+    const bf16_t* q_base = query + ((size_t)b * S * query_heads + h) * DQK;
+    const unsigned char* k_base =
+        reinterpret_cast<const unsigned char*>(key + ((size_t)b * S * key_value_heads + hk) * DQK);
+    const unsigned char* v_base =
+        reinterpret_cast<const unsigned char*>(value + ((size_t)b * S * key_value_heads + hk) * DV);
+
+    // ---- Q fragments (B operand: column = query lq, k = 16*ks + 8*g + j)
+    bf16x8 qf[KSTEPS];
+    {
+        const bool valid = q_row < S;
+        const bf16_t* row = q_base + (size_t)(valid ? q_row : 0) * q_stride + 8 * g;
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ++ks) {
+            u32x4 bits = {0, 0, 0, 0};
+            if (valid) {
+                bits = *reinterpret_cast<const u32x4*>(row + 16 * ks);
+            }
+            qf[ks] = __builtin_bit_cast(bf16x8, bits);
+        }
+    }
+
+    const int last_key = min(S, q0 + C::BM) - 1;
+    const int tiles = last_key / BN + 1;
+    const unsigned lds_base = lds_offset_of(lds);
+
+    // Requests this wave's share of tile `tile` into `stage`.  Rows past the end
+    // of the sequence are clamped to the last one: such keys are invisible to
+    // every stored query, the data only has to be finite.
+    auto request_tile = [&](int tile, int stage) {
+        const int key0 = tile * BN;
+        const int row_limit = S - 1 - key0;
+        const unsigned char* k_tile = k_base + (size_t)key0 * k_stride_bytes;
+        const unsigned char* v_tile = v_base + (size_t)key0 * v_stride_bytes;
+        const unsigned stage_base = lds_base + stage * C::STAGE_BYTES;
+#pragma unroll
+        for (int i = 0; i < C::K_LOADS_PER_WAVE; ++i) {
+            const int load = wave * C::K_LOADS_PER_WAVE + i;
+            const int slot = 64 * load + lane;
+            const int row = slot / C::K_CHUNKS;
+            const int chunk = (slot % C::K_CHUNKS) ^ C::k_swizzle(row);
+            const unsigned offset = (unsigned)min(row, row_limit) * k_stride_bytes + 16u * chunk;
+            direct_load_16_offset(k_tile, offset, stage_base + load * 1024);
+        }
+#pragma unroll
+        for (int i = 0; i < C::V_LOADS_PER_WAVE; ++i) {
+            const int load = wave * C::V_LOADS_PER_WAVE + i;
+            const int slot = 64 * load + lane;
+            const int row = slot / C::V_CHUNKS;
+            const int chunk = (slot % C::V_CHUNKS) ^ (C::v_flip(row) << 2);
+            const unsigned offset = (unsigned)min(row, row_limit) * v_stride_bytes + 16u * chunk;
+            direct_load_16_offset(v_tile, offset, stage_base + C::K_BYTES + load * 1024);
+        }
+    };
+
+    f32x16 o_acc[DBLOCKS];
+#pragma unroll
+    for (int d = 0; d < DBLOCKS; ++d) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o_acc[d][i] = 0.f;
+    }
+    float row_max = -INFINITY;  // reference point of the exponent, raw score units
+    float row_sum = 0.f;        // this lane's share (its 32 keys per tile) of the normaliser
+    const float c = scale * LOG2E;
+
+    // Per-lane pieces of the LDS read addresses.
+    const int k_swz = C::k_swizzle(lq);                        // rows lq and lq+32 share it
+    const int s16 = lane % 16;
+    const int v_row = 4 * g + s16 / 4;                          // + 16*n, + 8 for the second read
+    const int v_in_group = 32 * ((lane / 16) % 2) + 8 * (s16 % 4);
+    const int v_flip = C::v_flip(v_row);                        // rows v_row + 8*m share it
+
+    wait_vector_memory<0>();   // the query loads: no wait for them may remain inside the loop
+    request_tile(0, 0);
+
+    for (int tile = 0; tile < tiles; ++tile) {
+        const int stage = tile & 1;
+        wait_vector_memory<0>();   // this wave's share of the tile has landed
+        workgroup_barrier();       // ... and everybody's; every wave has left the previous tile
+        if (tile + 1 < tiles) {
+            request_tile(tile + 1, stage ^ 1);
+        }
+        const int key0 = tile * BN;
+        if (key0 <= wave_q0 + 31) {  // otherwise every key of the tile is in this wave's future
+            const unsigned char* k_lds = lds + stage * C::STAGE_BYTES;
+            const unsigned char* v_lds = k_lds + C::K_BYTES;
+
+            f32x16 s_acc[2];
+#pragma unroll
+            for (int mb = 0; mb < 2; ++mb) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) s_acc[mb][i] = 0.f;
+            }
+#pragma unroll
+            for (int ks = 0; ks < KSTEPS; ++ks) {
+                const int position = (2 * ks + g) ^ k_swz;
+#pragma unroll
+                for (int mb = 0; mb < 2; ++mb) {
+                    const bf16x8 a =
+                        *reinterpret_cast<const bf16x8*>(k_lds + (32 * mb + lq) * C::K_ROW + 16 * position);
+                    s_acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[ks], s_acc[mb], 0, 0, 0);
+                }
+            }
+
+            if (key0 + BN - 1 > wave_q0) {  // tile crosses this wave's diagonal
+#pragma unroll
+                for (int mb = 0; mb < 2; ++mb) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        const int k = key0 + 32 * mb + 8 * (i / 4) + 4 * g + (i % 4);
+                        if (k > q_row) s_acc[mb][i] = -INFINITY;
+                    }
+                }
+            }
+
+            float tile_max = s_acc[0][0];
+#pragma unroll
+            for (int mb = 0; mb < 2; ++mb) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) tile_max = fmaxf(tile_max, s_acc[mb][i]);
+            }
+            tile_max = half_wave_max(tile_max);
+
+            // The reference point only moves when some row's maximum grew by
+            // more than 2^8 in the exponent; until then probabilities may
+            // exceed one, which fp32 sums and bf16 operands hold without loss.
+            const float new_max = fmaxf(row_max, tile_max);
+            const bool grew = (new_max - row_max) * c > 8.0f;
+            if (__any(grew)) {
+                const float alpha = __builtin_amdgcn_exp2f((row_max - new_max) * c);
+                row_max = new_max;
+                row_sum *= alpha;
+#pragma unroll
+                for (int d = 0; d < DBLOCKS; ++d) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) o_acc[d][i] *= alpha;
+                }
+            }
+
+            const float offset = row_max * c;
+            bf16x8 pf[4];
+#pragma unroll
+            for (int n = 0; n < 4; ++n) {
+                u32x4 packed;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int i = 8 * (n % 2) + 2 * j;
+                    const float p0 = __builtin_amdgcn_exp2f(fmaf(s_acc[n / 2][i], c, -offset));
+                    const float p1 = __builtin_amdgcn_exp2f(fmaf(s_acc[n / 2][i + 1], c, -offset));
+                    row_sum += p0 + p1;
+                    packed[j] = pack_bf16(p0, p1);
+                }
+                pf[n] = __builtin_bit_cast(bf16x8, packed);
+            }
+
+            // V^T operand through transposing reads.  In a block of 16 lanes, lane s
+            // points at key row 16n + 4g + s/4 (+8 for the second read) and columns
+            // 4*(s%4)..+3 of the 16-column half (block%2) of column group d; the
+            // instruction hands lane i column i of the four rows.  Together: MFMA row
+            // lane%32, keys {4g..4g+3, 8+4g..8+4g+3} of the 16-key step, the k-order
+            // P^T carries from the C layout.
+#pragma unroll
+            for (int n = 0; n < 4; ++n) {
+#pragma unroll
+                for (int d = 0; d < DBLOCKS; ++d) {
+                    const unsigned char* first =
+                        v_lds + (16 * n + v_row) * C::V_ROW + 64 * (d ^ v_flip) + v_in_group;
+                    const s16x4 low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((transposing_read_pointer)first);
+                    const s16x4 high =
+                        __builtin_amdgcn_ds_read_tr16_b64_v4i16((transposing_read_pointer)(first + 8 * C::V_ROW));
+                    const s16x8 both = __builtin_shufflevector(low, high, 0, 1, 2, 3, 4, 5, 6, 7);
+                    o_acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, both), pf[n],
+                                                                       o_acc[d], 0, 0, 0);
+                }
+            }
+        }
+    }
+
+    // ---- epilogue: normalise, stage O through LDS for 16-byte row stores
+    workgroup_barrier();   // every wave is done reading the tile stages
+    const float total = half_wave_sum(row_sum);
+    const float inverse = 1.0f / total;
+    if (g == 0 && q_row < S) {
+        logsumexp[((size_t)b * query_heads + h) * S + q_row] = row_max * scale + __logf(total);
+    }
+    unsigned char* o_lds = lds + (32 * wave) * C::O_PITCH;
+#pragma unroll
+    for (int d = 0; d < DBLOCKS; ++d) {
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+            u32x2 packed;
+            packed.x = pack_bf16(o_acc[d][4 * i4 + 0] * inverse, o_acc[d][4 * i4 + 1] * inverse);
+            packed.y = pack_bf16(o_acc[d][4 * i4 + 2] * inverse, o_acc[d][4 * i4 + 3] * inverse);
+            const int dv = 32 * d + 8 * i4 + 4 * g;
+            *reinterpret_cast<u32x2*>(o_lds + lq * C::O_PITCH + 2 * dv) = packed;
+        }
+    }
+    __syncthreads();
+    constexpr int ROW_CHUNKS = DV / 8;          // 16-byte chunks per output row
+    constexpr int ROWS_PER_PASS = 64 / ROW_CHUNKS;
+    const size_t o_stride = (size_t)query_heads * DV;
+    bf16_t* o_base = output + ((size_t)b * S * query_heads + h) * DV;
+#pragma unroll
+    for (int pass = 0; pass < 32 / ROWS_PER_PASS; ++pass) {
+        const int row = pass * ROWS_PER_PASS + lane / ROW_CHUNKS;
+        const int chunk = lane % ROW_CHUNKS;
+        const int q = wave_q0 + row;
+        if (q < S) {
+            const u32x4 bits = *reinterpret_cast<const u32x4*>(o_lds + row * C::O_PITCH + 16 * chunk);
+            *reinterpret_cast<u32x4*>(o_base + (size_t)q * o_stride + 8 * chunk) = bits;
+        }
+    }
+}
 
 // ---------------------------------------------------------------------------
 // Split-key variant for short and medium problems.
@@ -824,6 +1091,26 @@ __global__ __launch_bounds__(512) void attention_forward_pingpong_kernel(
     }
 }
 
+template <int DQK, int DV>
+void launch_forward_four_waves(bf16_t* output, float* logsumexp, const bf16_t* query, const bf16_t* key, const bf16_t* value,
+                               int batch_size, int sequence_length, int query_heads, int key_value_heads, float scale,
+                               hipStream_t stream) {
+    using C = FwdConfig<DQK, DV, 4>;
+    const int query_blocks = (sequence_length + C::BM - 1) / C::BM;
+    auto kernel = attention_forward_kernel<DQK, DV, 4>;
+    if (C::LDS_BYTES > 64 * 1024) {
+        static hip_common::OncePerDevice raised;
+        raised.run([&] {
+            HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS_BYTES));
+        });
+    }
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((long long)batch_size * query_heads * query_blocks)), dim3(C::THREADS),
+                       C::LDS_BYTES, stream, output, logsumexp, query, key, value, sequence_length, query_heads,
+                       key_value_heads, query_blocks, scale);
+    HIP_CHECK(hipGetLastError());
+}
+
 template <int DQK, int DV, int QG, int KG>
 void launch_forward_split(bf16_t* output, float* logsumexp, const bf16_t* query, const bf16_t* key, const bf16_t* value,
                           int batch_size, int sequence_length, int query_heads, int key_value_heads, float scale,
@@ -911,9 +1198,14 @@ void attention_forward_dispatch(bf16_t* output, float* logsumexp, const bf16_t* 
 #define DSCUDA_FWD_SPLIT(DQK, DV, QG, KG)                                                                          \
     launch_forward_split<DQK, DV, QG, KG>(output, logsumexp, query, key, value, batch_size, sequence_length,       \
                                           query_heads, key_value_heads, scale, stream)
+#define DSCUDA_FWD_FOUR_WAVES(DQK, DV)                                                                             \
+    launch_forward_four_waves<DQK, DV>(output, logsumexp, query, key, value, batch_size, sequence_length,          \
+                                       query_heads, key_value_heads, scale, stream)
 #define DSCUDA_FWD_CASE(DQK, DV)                                                                                   \
     if (qk_head_size == DQK && v_head_size == DV) {                                                                \
-        if (persistent) {                                                                                          \
+        if (one_tile) {                                                                                            \
+            DSCUDA_FWD_FOUR_WAVES(DQK, DV);                                                                        \
+        } else if (persistent) {                                                                                          \
             launch_forward_pingpong<DQK, DV>(output, logsumexp, query, key, value, batch_size, sequence_length,    \
                                              query_heads, key_value_heads, plan, scale, stream);                   \
         } else if (quarters) {                                                                                     \
@@ -923,11 +1215,28 @@ void attention_forward_dispatch(bf16_t* output, float* logsumexp, const bf16_t* 
         }                                                                                                          \
         return;                                                                                                    \
     }
+    // One tile of keys: the split-key kernel's tiles of 128 keys are half repeated rows, which half a compute unit's worth
+    // of heads and more have to wait for (split / four waves: 64 heads 6.3 / 6.4 us, 256 heads 7.1 / 6.3, 512 heads of 192
+    // columns 12.6 / 14.6).
+    const bool one_tile = sequence_length <= 64 && 2 * batch_heads >= compute_units;
     if (qk_head_size == 64 && v_head_size == 64) {
-        // 64 queries per workgroup at any size (128: 22.7 against 16.3 us for 8 heads of 2048 tokens, 203 against 205 us
-        // for 64 heads of 4352); with 64 columns the softmax outweighs the products, and the persistent kernel's phases
-        // do not come out even.
-        DSCUDA_FWD_SPLIT(64, 64, 2, 4);
+        // With 64 columns the softmax outweighs the products, and the persistent kernel's phases do not come out even.  Four
+        // waves from one and a half heads per compute unit on (split / four waves, of 1024 tokens, in us: 128 heads equal,
+        // 256 heads 66.3 / 67.3, 384 heads 4 % less, 512 heads 132 / 121; of 512 tokens: 64 heads 8.0 / 11.9, 256 heads
+        // 24.6 / 26.9, 512 heads 46.2 / 43.6), from one head per unit on for long sequences (256 heads of 2048 tokens
+        // 213 / 206, of 4608 972 / 931), and at seven eighths to one head per unit where full rounds of workgroups of 64
+        // queries (two a unit) are followed by a short one (256 heads of 192 tokens 9.2 / 8.6, of 384 tokens 18.1 / 16.1; of
+        // 128 and 448 tokens 3 and 17 % more).
+        const bool heads_enough = 2 * batch_heads >= 3LL * compute_units || (batch_heads >= compute_units && sequence_length >= 2048);
+        const bool uneven = 8 * batch_heads >= 7LL * compute_units && batch_heads <= compute_units && sequence_length > 128 &&
+            sequence_length <= 384;
+        if (one_tile || heads_enough || uneven) {
+            DSCUDA_FWD_FOUR_WAVES(64, 64);
+        } else {
+            // 64 queries per workgroup (128: 22.7 against 16.3 us for 8 heads of 2048 tokens, 203 against 205 us for 64
+            // heads of 4352)
+            DSCUDA_FWD_SPLIT(64, 64, 2, 4);
+        }
         return;
     }
     // Persistent kernel or split keys: the tiles of the busiest workgroup against the steps (128 queries x 128 keys, 1.15
@@ -954,6 +1263,7 @@ void attention_forward_dispatch(bf16_t* output, float* logsumexp, const bf16_t* 
     DSCUDA_FWD_CASE(192, 128)
     DSCUDA_FWD_CASE(128, 128)
 #undef DSCUDA_FWD_CASE
+#undef DSCUDA_FWD_FOUR_WAVES
 #undef DSCUDA_FWD_SPLIT
     throw std::invalid_argument("attention forward: unsupported head sizes (d_qk,d_v) = (" +
                                 std::to_string(qk_head_size) + "," + std::to_string(v_head_size) + ")");

@@ -41,6 +41,37 @@ def test_flash_work_orders(cuda, batch, tokens, kv_heads, sharing, dim):
     assert_close_lse("LSE", lse, expected_lse)
 
 
+@pytest.mark.parametrize("batch,tokens,heads,kv_heads", [
+    (3, 64, 128, 128), (4, 192, 96, 32), (24, 128, 16, 16), (2, 192, 128, 16), (1, 320, 224, 56), (1, 384, 256, 64),
+    (1, 448, 384, 48), (1, 2112, 256, 2),   # four waves
+    (2, 448, 128, 32), (1, 128, 256, 64), (1, 192, 223, 223), (1, 64, 127, 127),   # the other side of the rule
+])
+def test_flash_64_columns_many_heads(cuda, batch, tokens, heads, kv_heads):
+    q, k, v, scale = configs.flash_forward_inputs(batch, tokens, heads, kv_heads, 64, seed=tokens, factor=0.5)
+    announce("flash, many heads", dict(B=batch, T=tokens, Hq=heads, Hkv=kv_heads))
+    out, lse = ops.flash_forward(q.to(cuda), k.to(cuda), v.to(cuda), scale)
+    sample = sorted({0, heads // 2, heads - 1})
+    group = heads // kv_heads
+    own = [h // group for h in sample]
+    expected, expected_lse = oracle.causal_attention_forward(q[:, :, sample], k[:, :, own], v[:, :, own], scale)
+    assert_close_bf16("O", out[:, :, sample], expected)
+    assert_close_lse("LSE", lse[:, sample], expected_lse)
+
+
+@pytest.mark.parametrize("dqk", [192, 128])
+@pytest.mark.parametrize("batch,seq,heads", [(1, 1, 128), (3, 31, 130), (2, 33, 64), (9, 64, 16), (2, 65, 64), (1, 64, 127)])
+def test_one_tile_of_keys(cuda, batch, seq, heads, dqk):
+    g = torch.Generator().manual_seed(seq)
+    randn = lambda dim: (torch.randn(batch, seq, heads, dim, generator=g) * 0.5).bfloat16()
+    q, k, v = randn(dqk), randn(dqk), randn(128)
+    scale = configs.c_float(dqk ** -0.5)
+    announce("one tile of keys", dict(B=batch, S=seq, H=heads, dqk=dqk))
+    out, lse = ops.mla_prefill_forward(q.to(cuda), k.to(cuda), v.to(cuda), scale)
+    expected, expected_lse = oracle.causal_attention_forward(q, k, v, scale)
+    assert_close_bf16("O", out, expected)
+    assert_close_lse("LSE", lse, expected_lse)
+
+
 @pytest.mark.parametrize("heads", [2, 72])   # 64 and 128 queries per workgroup
 def test_parts_with_distant_maxima(cuda, heads):
     """Scores that grow by thousands along the keys: the key groups of a workgroup end with maxima far apart, and rows
