@@ -722,8 +722,9 @@ DSCUDA_HOST_DEVICE inline DecodeLayout decode_layout(int batch, int heads, int s
 // (relative error against fp64 of one sequence of 400 tokens, 8 heads: 2.4e-3 whole, 2.8e-3 in parts).  So bf16 parts are
 // for batches all of whose sequences the ranges of decode_layout (`reference_ranges`) cut as well; any other batch is
 // cut into `wide_ranges` ranges with fp32 parts, for which slots of twice the size leave room, or as decode_layout would
-// (wide_ranges 0) if that makes more ranges.  us with bf16 parts throughout -> so, eight heads, 8 splits: eight sequences
-// of 1024..8192 tokens 24.7 -> 35.1, 1 of 400 11.0 -> 13.4; 16 heads, 2 splits, eight of 1024..8192 62.8 -> 178.
+// (wide_ranges 0) if that makes more ranges; a workgroup per sequence where decode_layout has that and the ranges would be
+// fewer than the sequences (ranges / workgroups: two sequences of 13 tokens, 16 heads, 2 splits 16.6 / 7.3 us).  us with bf16 parts throughout -> so, eight heads, 8 splits: eight sequences
+// of 1024..8192 tokens 24.7 -> 35.1, 1 of 400 11.0 -> 13.4; 16 heads, 2 splits, eight of 1024..8192 62.8 -> 171.
 DSCUDA_HOST_DEVICE inline DecodeLayout narrow_decode_layout(int batch, int heads, int splits, int compute_units,
                                                             int row_blocks, int rank) {
     DecodeLayout layout;
@@ -750,6 +751,14 @@ DSCUDA_HOST_DEVICE inline DecodeLayout narrow_decode_layout(int batch, int heads
         long long wide = (workspace - layout.plan_ints) / layout.wide_slot_floats - batch;
         if (wide > layout.workgroups) wide = layout.workgroups;
         if (wide < 1) wide = 1;   // a single range cuts nothing and needs no slot
+        if (reference.whole_sequences && wide < batch) {   // decode_layout runs every sequence on its own: not fewer at a time
+            layout.whole_sequences = 1;
+            layout.workgroups = batch;
+            layout.slots = layout.plan_offset = 0;
+            layout.plan_ints = plan_elements(batch, batch);
+            layout.reference_ranges = 0;
+            return layout;
+        }
         if (wide >= reference_ranges) {
             layout.wide_ranges = (int)wide;
             const long long wide_end = wide > 1 ? (wide + batch) * layout.wide_slot_floats : 0;

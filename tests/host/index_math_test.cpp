@@ -543,6 +543,9 @@ void check_decode_layout() {
                         // fallback with fp32 parts is there for the sequences that those leave whole
                         const DecodeLayout padded = decode_layout(batch, heads, splits, compute_units, ROWS, RANK);
                         const int reference = padded.whole_sequences ? 1 : padded.workgroups;
+                        // where that layout takes a workgroup per sequence, never fewer ranges than sequences
+                        EXPECT(!padded.whole_sequences || layout.whole_sequences || layout.wide_ranges >= batch,
+                               "narrow B %d H %d splits %d: %d ranges", batch, heads, splits, layout.wide_ranges);
                         if (layout.whole_sequences || layout.workgroups <= reference) {
                             EXPECT(layout.reference_ranges == 0, "narrow B %d H %d splits %d", batch, heads, splits);
                             continue;
