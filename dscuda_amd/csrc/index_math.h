@@ -768,6 +768,52 @@ DSCUDA_HOST_DEVICE inline DecodeLayout narrow_decode_layout(int batch, int heads
     return layout;
 }
 
+// Which kernel takes a decode call, and how its list is cut.
+struct DecodeForm {
+    int row_blocks;   // 32 * row_blocks rows per workgroup; 0: 128 rows
+    DecodeLayout layout;
+};
+
+constexpr int DECODE_ROWS = 128;
+constexpr int NARROW_SEQUENCE_GROUPS = 48;
+
+// Depends on the batch, the head count and the splits only, so that a plan built for them fits the call.  The line
+// between the kernels (times of the whole call, 1024..8192 tokens a sequence unless stated, 8 splits):
+//   * 32 rows when one head group holds all heads (64 sequences, 16 heads: 69 us against 75 with 64 rows and 104 with
+//     128; 32 heads: 75 / 76 / 104), or when every range the partial-result slots allow finds a compute unit for each
+//     of its head groups anyway (4 sequences, 128 heads: 31 / 32 / 53; 1 sequence of 200 tokens: 13 / 14 / 21);
+//   * 64 rows up to 64 heads (64 sequences, 64 heads: 109 / 83 / 109) and beyond while sequences x head groups stay
+//     few: the 128-row kernel is then held back by its slots and its start (16 sequences, 128 heads: 63 / 50 / 64);
+//   * 128 rows otherwise (32 sequences, 128 heads: 101 / 78 / 79; 64 sequences: 183 / 136 / 117).
+inline DecodeForm decode_form(int batch, int heads, int splits, int compute_units, int rank) {
+    const long long groups32 = (heads + 31) / 32, groups64 = (heads + 63) / 64;
+    const long long ranges = (long long)batch * (2LL * splits - 1);
+    DecodeForm form;
+    if (groups32 == 1 || groups32 * ranges <= compute_units) {
+        form.row_blocks = 1;
+    } else if (groups64 == 1 || batch * groups64 <= NARROW_SEQUENCE_GROUPS) {
+        form.row_blocks = 2;
+    } else {
+        form.row_blocks = 0;
+    }
+    form.layout = form.row_blocks == 0 ? decode_layout(batch, heads, splits, compute_units, DECODE_ROWS, rank)
+                                       : narrow_decode_layout(batch, heads, splits, compute_units, form.row_blocks, rank);
+    return form;
+}
+
+// The form a call with `page_size` tokens a page takes.  Pages that do not hold whole units of 32 keys are looked up key
+// by key, nine round trips a unit that bound the call, and head groups of 64 each do so for the whole cache.  Where
+// 128 rows make more ranges than those groups have, they take over (64 / 128 rows, pages of one token: 20 sequences of
+// 14913 tokens, 128 heads, 32 splits 446 / 284 us, 19 of 18668, 96 heads 519 / 332; of 48 tokens: 16 of 16051, 96 heads
+// 360 / 237).  A plan built for the other form serves: its positions are the same, the ranges are counted anew.
+inline DecodeForm decode_form_of_call(int batch, int heads, int splits, int page_size, int compute_units, int rank) {
+    const DecodeForm form = decode_form(batch, heads, splits, compute_units, rank);
+    if (form.row_blocks != 2 || page_size % 32 == 0 || form.layout.whole_sequences) return form;
+    const DecodeForm wide = {0, decode_layout(batch, heads, splits, compute_units, DECODE_ROWS, rank)};
+    return wide.layout.head_groups < form.layout.head_groups && !wide.layout.whole_sequences &&
+            wide.layout.workgroups > form.layout.workgroups ? wide : form;
+}
+
 // Whether `ranges` ranges cut the sequence with `positions` positions from `before` on.
 DSCUDA_HOST_DEVICE inline bool sequence_is_cut(int total, int ranges, int before, int positions, int overhead) {
     int first, last;

@@ -322,11 +322,12 @@ __device__ __forceinline__ int wave_min(int value) {
 
 // The plan comes from memory (own_plan false: the caller's, or one mla_decode_plan_kernel has just built), or,
 // for a batch that one workgroup scans in one go, is worked out here by every workgroup for itself, which saves the
-// call a kernel launch; `leave_plan`: this workgroup then also writes what the merge kernel reads of it.  Called by
+// call a kernel launch; `leave_plan`: this workgroup then also writes what the merge kernel reads of it.  `recut`: the
+// plan in memory was built for other ranges; its positions hold, the ranges are those of `cut`.  Called by
 // all threads of a workgroup of at least SELF_PLAN_BATCH threads; the three arrays (own_wave_totals: two ints per 64
 // sequences) are in LDS.
 __device__ __forceinline__ DecodeRange decode_range(int* plan, const int* cache_lengths, int batch_size, bool own_plan,
-                                                    const DecodeCut& cut, int* own_prefix, int* own_lengths,
+                                                    bool recut, const DecodeCut& cut, int* own_prefix, int* own_lengths,
                                                     int* own_wave_totals, int tid, int threads, int workgroup, bool leave_plan) {
     DecodeRange range;
     int total, ranges;
@@ -384,7 +385,7 @@ __device__ __forceinline__ DecodeRange decode_range(int* plan, const int* cache_
         range.overhead = plan[PLAN_OVERHEAD];
         whole_sequences = plan[PLAN_MODE] == PLAN_WHOLE;
         range.wide = plan[PLAN_MODE] == PLAN_WIDE_PARTS;
-        ranges = plan[PLAN_RANGES];
+        ranges = recut ? index_math::ranges_of(total, cut.workgroups) : plan[PLAN_RANGES];
         range.prefix = plan + index_math::plan_prefix_at();
     }
 
@@ -408,6 +409,11 @@ __device__ __forceinline__ DecodeRange decode_range(int* plan, const int* cache_
         range.sequence = low;
     } else if (own_plan) {
         range.sequence = workgroup;
+    } else if (recut) {
+        for (int first = 0; first < batch_size; first += 64) {   // sequences that end before the range
+            const int s = first + tid % 64;
+            range.sequence += __builtin_popcountll(__ballot(s < batch_size && range.prefix[min(s, batch_size - 1) + 1] <= range.begin));
+        }
     } else {
         range.sequence = plan[index_math::plan_first_sequence_at(batch_size) + workgroup];
     }

@@ -61,7 +61,7 @@
 namespace dscuda {
 namespace {
 
-constexpr int ROWS = 128;                   // rows per workgroup
+constexpr int ROWS = index_math::DECODE_ROWS;   // rows per workgroup
 constexpr int THREADS = 64 * LOAD_WAVES;
 constexpr int KSTEPS = WIDTH / 16;          // 36
 constexpr int DBLOCKS = RANK / 32;          // 16
@@ -560,7 +560,7 @@ __global__ __launch_bounds__(THREADS) void mla_decode_split_kernel(
     const bf16_t* __restrict__ paged_kv_cache, const int* __restrict__ block_table,
     const int* __restrict__ cache_lengths, float* __restrict__ workspace, int* __restrict__ plan, int batch_size,
     int heads, int page_size, int pages_per_sequence, long long slot_floats, int padded_rows, float scale, bool own_plan,
-    DecodeCut cut) {
+    bool recut, DecodeCut cut) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     __shared__ int own_prefix[SELF_PLAN_BATCH + 1];
     __shared__ int own_lengths[SELF_PLAN_BATCH];   // saves the walk a round trip to memory for its sequence's length
@@ -579,7 +579,7 @@ __global__ __launch_bounds__(THREADS) void mla_decode_split_kernel(
     const int head0 = head_group * ROWS;
     const float c = uniform(scale * LOG2E);
 
-    const DecodeRange range = decode_range(plan, cache_lengths, batch_size, own_plan, cut, own_prefix, own_lengths,
+    const DecodeRange range = decode_range(plan, cache_lengths, batch_size, own_plan, recut, cut, own_prefix, own_lengths,
                                            own_wave_totals, tid, THREADS, workgroup, blockIdx.x == 0 && blockIdx.y == 0);
     const int range_begin = range.begin, range_end = range.end, overhead = range.overhead;
     const int* prefix = range.prefix;
@@ -671,7 +671,8 @@ constexpr int MERGE_AHEAD = 8;
 __global__ __launch_bounds__(64) void mla_decode_merge_kernel(bf16_t* __restrict__ output, float* __restrict__ logsumexp,
                                                               const float* __restrict__ workspace,
                                                               const int* __restrict__ plan, int heads,
-                                                              long long slot_floats, int padded_rows) {
+                                                              long long slot_floats, int padded_rows,
+                                                              int recut_workgroups) {
     __shared__ __attribute__((aligned(16))) unsigned char staging[32 * MERGE_PITCH];
     const int lane = threadIdx.x;
     const int lq = lane % 32;
@@ -682,11 +683,12 @@ __global__ __launch_bounds__(64) void mla_decode_merge_kernel(bf16_t* __restrict
 
     const int total = plan[PLAN_TOTAL];
     const int overhead = plan[PLAN_OVERHEAD];
-    const int ranges = plan[PLAN_RANGES];
+    const int plan_ranges = plan[PLAN_RANGES];
     const int* prefix = plan + index_math::plan_prefix_at();
     const int sequence_begin = prefix[sequence];
     const int sequence_end = prefix[sequence + 1];
-    asm volatile("" ::"s"(total), "s"(overhead), "s"(ranges), "s"(sequence_end));   // one round trip, not two
+    asm volatile("" ::"s"(total), "s"(overhead), "s"(plan_ranges), "s"(sequence_end));   // one round trip, not two
+    const int ranges = recut_workgroups > 0 ? index_math::ranges_of(total, recut_workgroups) : plan_ranges;
     if (sequence_end <= sequence_begin) return;   // no tiles: nothing was computed for it
     int first, last;
     index_math::ranges_of_sequence(total, ranges, sequence_begin, sequence_end - sequence_begin, overhead, first, last);
@@ -861,39 +863,6 @@ std::size_t mla_decode_plan_elements(int batch_size, int /*heads*/, int /*splits
 
 namespace {
 
-// Which kernel takes a decode call, and how its list is cut.  Depends on the batch, the head count and the splits
-// only, so that a plan built for them fits the call.
-struct DecodeChoice {
-    int row_blocks;   // of the kernels in mla_narrow.hip; 0: the 128-row kernel of this file
-    index_math::DecodeLayout layout;
-};
-
-// The line between the kernels (times of the whole call, 1024..8192 tokens a sequence unless stated, 8 splits):
-//   * 32 rows when one head group holds all heads (64 sequences, 16 heads: 69 us against 75 with 64 rows and 104 with
-//     128; 32 heads: 75 / 76 / 104), or when every range the partial-result slots allow finds a compute unit for each
-//     of its head groups anyway (4 sequences, 128 heads: 31 / 32 / 53; 1 sequence of 200 tokens: 13 / 14 / 21);
-//   * 64 rows up to 64 heads (64 sequences, 64 heads: 109 / 83 / 109) and beyond while sequences x head groups stay
-//     few: the 128-row kernel is then held back by its slots and its start (16 sequences, 128 heads: 63 / 50 / 64);
-//   * 128 rows otherwise (32 sequences, 128 heads: 101 / 78 / 79; 64 sequences: 183 / 136 / 117).
-constexpr int NARROW_SEQUENCE_GROUPS = 48;
-
-DecodeChoice decode_choice(int batch_size, int heads, int splits) {
-    DecodeChoice choice;
-    const long long groups32 = (heads + 31) / 32, groups64 = (heads + 63) / 64;
-    const long long ranges = (long long)batch_size * (2LL * splits - 1);
-    if (groups32 == 1 || groups32 * ranges <= compute_units()) {
-        choice.row_blocks = 1;
-    } else if (groups64 == 1 || batch_size * groups64 <= NARROW_SEQUENCE_GROUPS) {
-        choice.row_blocks = 2;
-    } else {
-        choice.row_blocks = 0;
-    }
-    choice.layout = choice.row_blocks == 0
-        ? index_math::decode_layout(batch_size, heads, splits, compute_units(), ROWS, RANK)
-        : index_math::narrow_decode_layout(batch_size, heads, splits, compute_units(), choice.row_blocks, RANK);
-    return choice;
-}
-
 DecodeCut cut_of(const index_math::DecodeLayout& layout) {
     return DecodeCut{layout.workgroups, layout.whole_sequences, layout.reference_ranges, layout.wide_ranges};
 }
@@ -902,7 +871,7 @@ DecodeCut cut_of(const index_math::DecodeLayout& layout) {
 
 void mla_decode_plan_dispatch(int* plan, const int* cache_lengths, int batch_size, int heads, int splits,
                               hipStream_t stream) {
-    const index_math::DecodeLayout layout = decode_choice(batch_size, heads, splits).layout;
+    const index_math::DecodeLayout layout = index_math::decode_form(batch_size, heads, splits, compute_units(), RANK).layout;
     hipLaunchKernelGGL(mla_decode_plan_kernel, dim3(1), dim3(THREADS), 0, stream, plan, cache_lengths, batch_size,
                        cut_of(layout));
     HIP_CHECK(hipGetLastError());
@@ -916,8 +885,9 @@ void mla_decode_dispatch(bf16_t* output, float* logsumexp, const bf16_t* query, 
         throw std::invalid_argument("MLA decode requires a workspace aligned to 16 bytes");
     }
     // How the caller's B*H*splits*(C+2) floats are used: index_math::decode_layout.
-    const DecodeChoice choice = decode_choice(batch_size, heads, splits);
-    const index_math::DecodeLayout& layout = choice.layout;
+    const index_math::DecodeForm form =
+        index_math::decode_form_of_call(batch_size, heads, splits, page_size, compute_units(), RANK);
+    const index_math::DecodeLayout& layout = form.layout;
     bool own_plan = false;
     if (plan == nullptr) {
         // no plan from the caller: this call's own, behind the partial-result slots -- built by the decode kernel
@@ -931,23 +901,26 @@ void mla_decode_dispatch(bf16_t* output, float* logsumexp, const bf16_t* query, 
             HIP_CHECK(hipGetLastError());
         }
     }
-    if (choice.row_blocks != 0) {
+    if (form.row_blocks != 0) {
         mla_narrow_decode_launch(output, logsumexp, query, paged_kv_cache, block_table, cache_lengths, workspace, plan,
-                                 batch_size, heads, page_size, pages_per_sequence, choice.row_blocks, layout, own_plan, scale,
+                                 batch_size, heads, page_size, pages_per_sequence, form.row_blocks, layout, own_plan, scale,
                                  stream);
         return;
     }
     static hip_common::OncePerDevice prepared;
     prepared.run([] { allow_large_lds(mla_decode_split_kernel); });
+    // a plan built for the other form counts other ranges
+    const bool recut = !own_plan && index_math::decode_form(batch_size, heads, splits, compute_units(), RANK).row_blocks != 0;
     const int padded_rows = (heads + 31) / 32 * 32;
     const dim3 grid(layout.workgroups, layout.head_groups);
     hipLaunchKernelGGL(mla_decode_split_kernel, grid, dim3(THREADS), LDS_BYTES, stream, output, logsumexp, query,
                        paged_kv_cache, block_table, cache_lengths, workspace, plan, batch_size, heads, page_size,
-                       pages_per_sequence, layout.slot_floats, padded_rows, scale, own_plan, cut_of(layout));
+                       pages_per_sequence, layout.slot_floats, padded_rows, scale, own_plan, recut, cut_of(layout));
     HIP_CHECK(hipGetLastError());
     if (!layout.whole_sequences) {
         hipLaunchKernelGGL(mla_decode_merge_kernel, dim3(MERGE_SLICES * (padded_rows / 32), batch_size), dim3(64), 0,
-                           stream, output, logsumexp, workspace, plan, heads, layout.slot_floats, padded_rows);
+                           stream, output, logsumexp, workspace, plan, heads, layout.slot_floats, padded_rows,
+                           recut ? layout.workgroups : 0);
         HIP_CHECK(hipGetLastError());
     }
 }

@@ -415,7 +415,7 @@ __global__ __launch_bounds__(NARROW_THREADS) void mla_narrow_decode_kernel(
     const float c = scale * LOG2E;
 
     if (tid < 2) *reinterpret_cast<volatile int*>(lds + L::FLAG_AT + 4 * tid) = 0;
-    const DecodeRange range = decode_range(plan, cache_lengths, batch_size, own_plan, cut, own_prefix, own_lengths,
+    const DecodeRange range = decode_range(plan, cache_lengths, batch_size, own_plan, false, cut, own_prefix, own_lengths,
                                            own_wave_totals, tid, NARROW_THREADS, workgroup, blockIdx.x == 0 && blockIdx.y == 0);
     if (range.begin >= range.end) return;
 

@@ -568,6 +568,26 @@ void check_decode_layout() {
     EXPECT(!headline.whole_sequences && headline.workgroups == 256, "B 64 H 128 splits 8: %d workgroups", headline.workgroups);
     // splits = 1 never cuts
     EXPECT(decode_layout(5, 128, 1, 256, ROWS, RANK).whole_sequences == 1, "splits 1 must not cut");
+    // A call takes another form than its plan only where it then reads the cache fewer times with more ranges, and never
+    // where the plan's positions would differ.
+    int moved = 0;
+    for (int batch = 1; batch <= 80; ++batch) {
+        for (int heads : {1, 16, 33, 64, 65, 96, 128, 160, 300}) {
+            for (int splits : {1, 2, 4, 8, 32}) {
+                const DecodeForm plan = decode_form(batch, heads, splits, 256, RANK);
+                for (int page : {1, 8, 16, 32, 48, 64, 128}) {
+                    const DecodeForm call = decode_form_of_call(batch, heads, splits, page, 256, RANK);
+                    if (page % 32 == 0) EXPECT(call.row_blocks == plan.row_blocks, "page %d B %d H %d splits %d", page, batch, heads, splits);
+                    if (call.row_blocks == plan.row_blocks) continue;
+                    ++moved;
+                    EXPECT(plan.row_blocks == 2 && call.row_blocks == 0 && call.layout.whole_sequences == 0 && plan.layout.whole_sequences == 0 &&
+                               call.layout.head_groups < plan.layout.head_groups && call.layout.workgroups > plan.layout.workgroups,
+                           "page %d B %d H %d splits %d", page, batch, heads, splits);
+                }
+            }
+        }
+    }
+    EXPECT(moved > 0 && decode_form_of_call(20, 128, 32, 1, 256, RANK).row_blocks == 0, "pages of one token, 128 heads");
 }
 
 // ---- projections: rows_apart never calls rows that share an element apart, and sees what is apart in the usual layouts

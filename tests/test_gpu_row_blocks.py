@@ -6,6 +6,7 @@ import torch
 
 from dscuda_amd.harness import configs, ops
 from oracle import attention_oracle as oracle
+from tests.dispatch_rules import rules
 from tests.parity import announce, assert_close_bf16, assert_close_lse
 
 pytestmark = pytest.mark.gpu
@@ -138,3 +139,28 @@ def test_sequences_that_fewer_ranges_leave_whole_are_rounded_once(cuda, batch, h
     error = (out.cpu().double() - expected).norm() / expected.norm()
     assert error.item() <= 2.6e-3
     assert_close_lse("LSE", lse, expected_lse)
+
+
+@pytest.mark.parametrize("batch,heads,splits,page,high", [
+    (20, 128, 8, 16, 600), (16, 96, 32, 1, 300), (17, 65, 8, 48, 2000),
+])
+def test_decode_pages_that_hold_no_whole_units(cuda, batch, heads, splits, page, high):
+    """Calls whose plan is made for 64 rows but whose pages are looked up key by key run 128 rows over the plan's
+    positions: the same ranges, and so the same bits, as without a plan."""
+    units = torch.cuda.get_device_properties(cuda).multi_processor_count
+    assert rules().plan_rows(batch, heads, splits, units) == 2 and rules().call_rows(batch, heads, splits, page, units) == 0
+    g = torch.Generator().manual_seed(batch)
+    lengths = torch.linspace(1, high, batch).int()
+    query = (torch.randn(batch, 1, heads, 576, generator=g) * 0.25).bfloat16()
+    cache = (torch.randn(batch, high, 576, generator=g) * 0.25).bfloat16()
+    paged, table = configs.pack_cache(cache, page)
+    scale = configs.c_float(576 ** -0.5)
+    announce("decode, pages looked up", dict(B=batch, H=heads, splits=splits, page=page))
+    on_gpu = [x.to(cuda) for x in (query, paged, table, lengths)]
+    expected, expected_lse = oracle.mla_decode_unrounded(query, cache, lengths, scale)
+    out, lse = ops.mla_decode(*on_gpu, scale, splits=splits)
+    assert_close_bf16("O", out, expected)
+    assert_close_lse("LSE", lse, expected_lse)
+    plan = ops.mla_decode_plan(on_gpu[3], heads, splits)
+    planned, planned_lse = ops.mla_decode_planned(*on_gpu, plan, scale, splits=splits)
+    assert torch.equal(out, planned) and torch.equal(lse, planned_lse)
