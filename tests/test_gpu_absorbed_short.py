@@ -6,6 +6,7 @@ import torch
 
 from dscuda_amd.harness import configs, ops
 from oracle import attention_oracle as oracle
+from tests.dispatch_rules import rules
 from tests.parity import announce, assert_close_bf16
 
 pytestmark = pytest.mark.gpu
@@ -40,3 +41,20 @@ def test_absorbed_backward_of_short_sequences(cuda, batch, tokens, heads):
     for name, first, second, reference in zip(("dq_latent", "dq_rope", "dlatent", "dk_rope"), *runs, expected):
         assert torch.equal(first, second)
         assert_close_bf16(name, first.cpu(), reference)
+
+
+@pytest.mark.parametrize("batch,tokens,heads,kept", [
+    (1, 33, 1, True), (1, 3, 11, True), (2, 2, 17, True), (9, 384, 1, True), (2, 219, 20, True),
+    (1, 1, 32, False), (13, 4, 8, False), (10, 353, 2, False), (2, 224, 20, False), (2, 160, 32, False),
+])
+def test_which_calls_keep_their_scores(cuda, batch, tokens, heads, kept):
+    assert bool(rules().keeps_scores(batch, tokens, heads)) == kept
+    test_absorbed_backward_of_short_sequences(cuda, batch, tokens, heads)
+
+
+@pytest.mark.parametrize("batch,tokens,heads", [(1, 1, 1), (3, 9, 2), (1, 513, 1), (2, 700, 3), (1, 1024, 2)])
+def test_absorbed_backward_of_whole_key_blocks(cuda, batch, tokens, heads):
+    """Calls whose query gradients have no room for partial results: a workgroup walks all rows of its key block."""
+    units = torch.cuda.get_device_properties(cuda).multi_processor_count
+    assert not rules().keeps_scores(batch, tokens, heads) and rules().backward_ranges(batch, tokens, heads, units) == 0
+    test_absorbed_backward_of_short_sequences(cuda, batch, tokens, heads)
