@@ -84,6 +84,13 @@ GATES = {
 
 Case = collections.namedtuple("Case", "stem label command counter_command kernels")
 
+# Parts of the names of the kernels that an operation may launch, whichever of them a shape takes
+FORWARD_KERNELS = ["attention_forward"]
+BACKWARD_KERNELS = ["attention_backward", "attention_key_value", "attention_query"]
+DECODE_KERNELS = ["mla_decode", "mla_narrow_decode", "mla_narrow_merge"]
+ABSORBED_KERNELS = ["mla_absorbed", "mla_narrow_forward", "mla_short"]
+PROJECTION_KERNELS = ["mla_absorb_query", "mla_unabsorb_output"]
+
 
 def _python_case(workload, steps, counter_steps, *extra):
     base = [sys.executable, str(CASE_SCRIPT), workload, *map(str, extra)]
@@ -106,28 +113,28 @@ def metric_cases(suite):
         cases.append(Case(stem, label, command, counter_command, kernels))
 
     add("mla_prefill_forward_S4096_H128", "MLA prefill forward B=1 S=4096 H=128 192/128", "forward", 160, 60,
-        ["attention_forward"])
+        FORWARD_KERNELS)
     add("mla_prefill_backward_S4096_H128", "MLA prefill backward B=1 S=4096 H=128 192/128", "backward", 80, 30,
-        ["attention_backward", "attention_key_value", "attention_query"])
+        BACKWARD_KERNELS)
     add("mla_decode_B64_H128", "absorbed MLA decode B=64 H=128 lengths U[1024,8192] seed 3", "decode", 300, 100,
-        ["mla_decode"])
-    add("flash_forward_S512_H8_D64", "flash forward B=1 H=8 S=512 D=64", "flash", 300, 100, ["attention_forward"])
+        DECODE_KERNELS)
+    add("flash_forward_S512_H8_D64", "flash forward B=1 H=8 S=512 D=64", "flash", 300, 100, FORWARD_KERNELS)
     add("mla_absorbed_T4096_H128", "absorbed MLA prefill forward + backward (dscuda_mla_forward / _backward) B=1 T=4096 H=128",
-        "absorbed", 6, 3, ["mla_absorbed"])
+        "absorbed", 6, 3, ABSORBED_KERNELS)
     add("mla_projection_T4096_H128", "W_UK absorb and W_UV un-absorb of 4096 tokens x 128 heads", "projection", 60, 20,
-        ["mla_absorb_query", "mla_unabsorb_output"])
+        PROJECTION_KERNELS)
     if suite == "full":
         add("mla_prefill_forward_S16384_H128", "MLA prefill forward B=1 S=16384 H=128 192/128", "forward", 16, 8,
-            ["attention_forward"], "--seq", 16384)
+            FORWARD_KERNELS, "--seq", 16384)
         add("mla_prefill_backward_S16384_H128", "MLA prefill backward B=1 S=16384 H=128 192/128", "backward", 8, 4,
-            ["attention_backward", "attention_key_value", "attention_query"], "--seq", 16384)
+            BACKWARD_KERNELS, "--seq", 16384)
         # the same launches on all-zero inputs: same instruction streams, operands that do not toggle
         add("mla_prefill_forward_S4096_H128_zero_inputs", "MLA prefill forward B=1 S=4096 H=128 192/128, all inputs zero",
-            "forward", 160, 60, ["attention_forward"], "--data", "zero")
+            "forward", 160, 60, FORWARD_KERNELS, "--data", "zero")
         add("mla_prefill_backward_S4096_H128_zero_inputs", "MLA prefill backward B=1 S=4096 H=128 192/128, all inputs zero",
-            "backward", 80, 30, ["attention_backward", "attention_key_value", "attention_query"], "--data", "zero")
+            "backward", 80, 30, BACKWARD_KERNELS, "--data", "zero")
         add("mla_decode_B64_H128_zero_inputs", "absorbed MLA decode B=64 H=128 lengths U[1024,8192] seed 3, query and cache zero",
-            "decode", 300, 100, ["mla_decode"], "--data", "zero")
+            "decode", 300, 100, DECODE_KERNELS, "--data", "zero")
     return cases
 
 
@@ -137,10 +144,10 @@ def mla_cases(suite):
     for sequence in ((128,) if suite == "quick" else (128, 256, 512)):
         command = [str(BUILD / "benchmark_mla"), "1", str(sequence), "8", "512", "64"]
         cases.append(Case(f"mla_T{sequence}_forward_backward", f"B=1,T={sequence},H=8,D=512,R=64/custom/forward_backward",
-                          command, command, ["mla_absorbed"]))
+                          command, command, ABSORBED_KERNELS))
         command = [str(BUILD / "benchmark_mla_decode"), "2", str(sequence), "16", "512", "64", "8"]
         cases.append(Case(f"mla_KV{sequence}_decode", f"B=2,KV={sequence},H=16,D=512,R=64/custom/decode", command, command,
-                          ["mla_decode"]))
+                          DECODE_KERNELS))
     return cases
 
 
@@ -152,7 +159,7 @@ def flash_cases(suite):
         command = [str(BUILD / "benchmark_flash_attention"), *map(str, (batch, sequence, heads, dimension)), "forward"]
         cases.append(Case(f"flash_B{batch}_T{sequence}_H{heads}_D{dimension}_forward",
                           f"B={batch},T={sequence},H={heads},D={dimension}/custom/forward", command, command,
-                          ["attention_forward"]))
+                          FORWARD_KERNELS))
     return cases
 
 

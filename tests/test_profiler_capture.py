@@ -3,6 +3,7 @@ files (calibration by the copy case, settled durations, matrix-pipe utilisation 
 the pass definitions against the hardware's counter-block limits, and the raw-dump comparator."""
 
 import csv
+import re
 
 import numpy as np
 
@@ -109,6 +110,31 @@ def test_program_follows_the_separator_directly():
             command = capture.rocprof_command("fetch", "/tmp/x", case.counter_command)
             program = command[command.index("--") + 1]
             assert program.endswith(("python3", "python")) or "/build/benchmark_" in program, program
+
+
+def test_every_kernel_of_an_operation_is_kept():
+    """A table that leaves out the kernels a shape was moved to states the rest as the whole."""
+    operation_of = {"attn_fwd": lambda name: "forward", "attn_bwd": lambda name: "backward",
+                    "mla_decode": lambda name: "absorbed" if "forward" in name else "decode",
+                    "mla_narrow": lambda name: "absorbed" if "forward" in name else "decode",
+                    "mla_absorbed": lambda name: "absorbed", "mla_absorbed_short": lambda name: "absorbed",
+                    "mla_projection": lambda name: "projection"}
+    launched = {}
+    for file, operation in operation_of.items():
+        text = (capture.ROOT / "dscuda_amd" / "csrc" / f"{file}.hip").read_text()
+        names = re.findall(r"__global__[^;{]*?void\s+(\w+)\(", text)
+        assert names, file
+        for name in names:
+            launched.setdefault(operation(name), set()).add(name)
+    kept = {"forward": ["mla_prefill_forward_S4096_H128", "flash_forward_S512_H8_D64", "flash_B2_T512_H8_D128_forward"],
+            "backward": ["mla_prefill_backward_S4096_H128"], "decode": ["mla_decode_B64_H128", "mla_KV128_decode"],
+            "absorbed": ["mla_absorbed_T4096_H128", "mla_T128_forward_backward"],
+            "projection": ["mla_projection_T4096_H128"]}
+    cases = {case.stem: case for family in capture.FAMILIES.values() for case in family("full")}
+    for operation, stems in kept.items():
+        for stem in stems:
+            lost = [name for name in launched[operation] if not any(part in name for part in cases[stem].kernels)]
+            assert not lost, (stem, lost)
 
 
 def test_dump_comparator(tmp_path):
