@@ -7,6 +7,9 @@
 // fast path == general path).
 #pragma once
 
+#include <algorithm>
+#include <vector>
+
 #if defined(__HIPCC__)
 #define DSCUDA_HOST_DEVICE __host__ __device__
 #else
@@ -245,19 +248,27 @@ DSCUDA_HOST_DEVICE inline bool forward_item(int round, int member, int members, 
 // Tiles (64 keys x 256 queries) of the busiest workgroup of a cluster, an item's start and end counted as three more.
 constexpr int FORWARD_ITEM_TILES = 3;
 
-inline int forward_makespan(int members, int clusters, int cluster_heads, int sequence_length, int abreast) {
+// One pass over the items in the order of forward_item: the rounds run through the workgroups there and back.
+inline int forward_makespan(int members, int /* clusters: all alike */, int cluster_heads, int sequence_length, int abreast) {
     const int query_blocks = (sequence_length + 255) / 256;
-    int longest = 0;
-    for (int member = 0; member < members; ++member) {
-        int tiles = 0;
-        ForwardItem item;
-        for (int round = 0; forward_item(round, member, members, 0, clusters, cluster_heads, query_blocks, item, abreast); ++round) {
-            const int end = (item.query_block + 1) * 256;
-            tiles += ((end < sequence_length ? end : sequence_length) + 63) / 64 + FORWARD_ITEM_TILES;
+    const int interleave = abreast > 0 ? abreast : (cluster_heads % 2 == 0) ? 2 : 1;
+    std::vector<int> loads(members, 0);
+    int position = 0, direction = 1;
+    for (int group = 0; group < cluster_heads; group += interleave) {
+        for (int block = query_blocks - 1; block >= 0; --block) {
+            const int end = (block + 1) * 256;
+            const int tiles = ((end < sequence_length ? end : sequence_length) + 63) / 64 + FORWARD_ITEM_TILES;
+            for (int item = 0; item < interleave; ++item) {
+                loads[position] += tiles;
+                position += direction;
+                if (position == members || position < 0) {
+                    direction = -direction;
+                    position += direction;
+                }
+            }
         }
-        if (tiles > longest) longest = tiles;
     }
-    return longest;
+    return *std::max_element(loads.begin(), loads.end());
 }
 
 // How many heads a cluster takes abreast, and the cost of the launch in tiles.  Two at a time keep few keys live in the

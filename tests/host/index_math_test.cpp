@@ -671,6 +671,31 @@ void check_split_order() {
     }
 }
 
+// ---- persistent forward: the makespan is that of the items as the workgroups take them
+void check_forward_makespan() {
+    for (int heads : {1, 2, 3, 4, 7, 12, 33}) {
+        for (int sequence : {128, 257, 1000, 4096, 7168}) {
+            for (int limit : {1, 2, 32, 256}) {
+                const int blocks = (sequence + 255) / 256, members = std::min(limit, heads * blocks);
+                for (int abreast : {0, 1, 2, 4, heads}) {
+                    if (abreast > 0 && heads % abreast != 0) continue;
+                    int longest = 0;
+                    for (int member = 0; member < members; ++member) {
+                        int tiles = 0;
+                        ForwardItem item;
+                        for (int round = 0; forward_item(round, member, members, 0, 8, heads, blocks, item, abreast); ++round) {
+                            tiles += (std::min((item.query_block + 1) * 256, sequence) + 63) / 64 + FORWARD_ITEM_TILES;
+                        }
+                        longest = std::max(longest, tiles);
+                    }
+                    EXPECT(forward_makespan(members, 8, heads, sequence, abreast) == longest, "%d heads of %d, %d workgroups, %d abreast",
+                           heads, sequence, members, abreast);
+                }
+            }
+        }
+    }
+}
+
 // ---- cut of the backward's walks: every step in one part, parts equal to within one and no longer than asked for
 void check_walk_cut() {
     for (int slots : {256, 8}) {
@@ -742,6 +767,7 @@ int main() {
     check_kept_scores();
     check_walk_cut();
     check_split_order();
+    check_forward_makespan();
     check_swizzle<128>();
     check_swizzle<256>();
     check_swizzle<384>();
