@@ -73,12 +73,17 @@ def pointers(tensors):
     return [x.data_ptr() for x in tensors]
 
 
+# the current stream's handle without a Stream object, in a torch that has these two
+_current_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def stream():
     """Raw handle of torch's current stream (benchmarks/common.py:39-40).  The Stream object that
     torch.cuda.current_stream() makes costs 2.9 us a call on the host, the handle alone 0.2 us."""
-    if not torch.cuda.is_initialized():
+    if _current_raw_stream is None or _current_device is None or not torch.cuda.is_initialized():
         return torch.cuda.current_stream().cuda_stream
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return _current_raw_stream(_current_device())
 
 
 def c_float(value: float) -> float:

@@ -7,10 +7,12 @@ import json
 import subprocess
 import sys
 from pathlib import Path
+from types import SimpleNamespace
 
 import pytest
+import torch
 
-from dscuda_amd.harness import catalogue, configs, replay, tables
+from dscuda_amd.harness import catalogue, common, configs, replay, tables
 
 ROOT = Path(__file__).resolve().parents[1]
 
@@ -210,3 +212,13 @@ def test_bound_workloads_compare_with_per_output_tolerances():
     with pytest.raises(AssertionError):
         bound.verify("custom", (torch.zeros(4),))
     catalogue.Bound(workload, {}).verify("custom", (torch.ones(1),))   # nothing to compare with: nothing to fail
+
+
+# ---- operators' stream -------------------------------------------------------------------------------------------
+
+@pytest.mark.parametrize("missing", ["_current_raw_stream", "_current_device"])
+def test_stream_without_the_raw_handle_of_this_torch(monkeypatch, missing):
+    monkeypatch.setattr(common, missing, None)
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: SimpleNamespace(cuda_stream=77))
+    assert common.stream() == 77
