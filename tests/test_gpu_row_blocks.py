@@ -164,3 +164,34 @@ def test_decode_pages_that_hold_no_whole_units(cuda, batch, heads, splits, page,
     plan = ops.mla_decode_plan(on_gpu[3], heads, splits)
     planned, planned_lse = ops.mla_decode_planned(*on_gpu, plan, scale, splits=splits)
     assert torch.equal(out, planned) and torch.equal(lse, planned_lse)
+
+
+@pytest.mark.parametrize("batch,heads,splits,page,high", [
+    (28, 128, 8, 64, 400), (70, 128, 1, 64, 200),      # parts, and a workgroup per sequence
+    (260, 128, 8, 64, 130), (260, 128, 1, 64, 90),     # the plan kernel
+    (28, 128, 8, 16, 300), (28, 128, 8, 48, 300),      # pages looked up key by key
+    (28, 128, 8, 32, 2500),                            # page ids of two loads
+    (25, 160, 8, 64, 300), (40, 200, 1, 16, 150),      # a second head group
+])
+def test_decode_of_128_rows(cuda, batch, heads, splits, page, high):
+    """The 128-row form with its own plan and with the caller's, whose ranges are the same.  One sequence is empty: it
+    owns no key and no result."""
+    units = torch.cuda.get_device_properties(cuda).multi_processor_count
+    assert rules().plan_rows(batch, heads, splits, units) == 0 and rules().call_rows(batch, heads, splits, page, units) == 0
+    g = torch.Generator().manual_seed(batch + heads + page)
+    lengths = torch.linspace(1, high, batch).int()
+    lengths[batch // 3] = 0
+    query = (torch.randn(batch, 1, heads, 576, generator=g) * 0.25).bfloat16()
+    cache = (torch.randn(batch, high, 576, generator=g) * 0.25).bfloat16()
+    paged, table = configs.pack_cache(cache, page)
+    scale = configs.c_float(576 ** -0.5)
+    announce("decode of 128 rows", dict(B=batch, H=heads, splits=splits, page=page, tokens=high))
+    on_gpu = [x.to(cuda) for x in (query, paged, table, lengths)]
+    out, lse = ops.mla_decode(*on_gpu, scale, splits=splits)
+    plan = ops.mla_decode_plan(on_gpu[3], heads, splits)
+    planned, planned_lse = ops.mla_decode_planned(*on_gpu, plan, scale, splits=splits)
+    some = (lengths > 0).nonzero().flatten()
+    expected, expected_lse = oracle.mla_decode_unrounded(query[some], cache[some], lengths[some], scale)
+    assert_close_bf16("O", out.cpu()[some], expected)
+    assert_close_lse("LSE", lse.cpu()[some], expected_lse)
+    assert torch.equal(out.cpu()[some], planned.cpu()[some]) and torch.equal(lse.cpu()[some], planned_lse.cpu()[some])
