@@ -688,10 +688,11 @@ __global__ __launch_bounds__(64 * QG * KG) void attention_forward_split_kernel(
 // Work order.  Workgroup w belongs to cluster w % 8 (workgroups are dealt
 // round-robin to the 8 XCDs, each with its own L2) and the (batch, head) pairs
 // are dealt to the clusters the same way.  Inside a cluster the items are laid
-// out two heads at a time, blocks from the heaviest (last) to the lightest, and
-// cut into rounds of one item per workgroup; odd rounds are handed out in
-// reverse, so a workgroup's heavy and light blocks add up to the same total
-// while the cluster works on two heads at any time.
+// out `abreast` heads at a time (index_math::forward_choice: two where that comes
+// out even), blocks from the heaviest (last) to the lightest, and cut into rounds
+// of one item per workgroup; odd rounds are handed out in reverse, so a
+// workgroup's heavy and light blocks add up to the same total while the cluster
+// works on few heads at any time.
 struct PingPong {
     static constexpr int K_SLOTS = 3;
     static constexpr int V_SLOTS = 4;

@@ -146,7 +146,7 @@ __device__ __forceinline__ void issue_unit_load(const UnitSource& source, const 
     const unsigned offset = source.full
         ? offsets.of[i]
         : index_math::contiguous_load_offset<ROW_BYTES, UNIT / 4>(wave, i, lane, source.row_limit);
-    direct_load_16_offset_streaming(source.base, offset, source.lds_base + i * 1024);   // the cache is read once per call
+    direct_load_16_offset_streaming(source.base, offset, source.lds_base + i * 1024);   // each head group reads the cache once
 }
 
 // Load I of a unit whose latent and rope parts lie in tensors of their own, unpaged (`split`): a wave instruction
@@ -239,7 +239,6 @@ struct UnitReads {
 };
 
 typedef short unit_s16x4 __attribute__((ext_vector_type(4)));
-typedef short unit_s16x8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) unit_s16x4* unit_tr_pointer;
 
 template <int KS>

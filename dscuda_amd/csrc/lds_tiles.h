@@ -29,12 +29,6 @@ struct TileRequests {
 #pragma unroll
         for (int r = 0; r < PERIOD; ++r) base[r] = Math::base_of(r, lane, row_stride, wave);
     }
-    // load I of this wave's share of a full tile
-    template <int I>
-    __device__ __forceinline__ void request_full(const unsigned char* tile, unsigned row_stride, unsigned lds_target, int wave) const {
-        direct_load_16_offset(tile + (size_t)(Math::rows_before(0, wave) + Math::rows_before(I, 0)) * row_stride,
-                              Math::lane_part(base[I % PERIOD], I), lds_target + (wave * LOADS + I) * 1024);
-    }
     // `tile` = address of the tile's first row (uniform)
     __device__ __forceinline__ void request(const unsigned char* tile, unsigned row_stride, int row_limit,
                                             unsigned lds_target, int wave) const {

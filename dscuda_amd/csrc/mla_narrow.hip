@@ -63,8 +63,6 @@ struct NarrowLayout {
     static_assert(ROWS * WIDE_PITCH <= UNIT_SLOTS * UNIT_BYTES, "the staged rows take the place of the units");
 };
 
-typedef short narrow_s16x4 __attribute__((ext_vector_type(4)));
-
 __device__ __forceinline__ float quarter_max(float value) {   // over the lanes l, l ^ 16, l ^ 32, l ^ 48
     value = fmaxf(value, __shfl_xor(value, 16));
     return half_wave_max(value);

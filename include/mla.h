@@ -231,7 +231,10 @@ void mla_prefill_forward_cuda(
 // fit 3 GiB (at least one): the two passes run over the pairs in chunks that share
 // that set of blocks.  Where the pairs alone would leave compute units idle the walk
 // over the queries of a key block is cut into parts, and their fp32 sums of dK and dV
-// (160 KB a part for 192/128 columns, some 260 parts) follow.  0 for non-positive sizes.
+// follow: 160 KB a part for 192/128 columns, some 260 parts where they run as one round,
+// up to 1800 (0.3 GB) where several rounds of parts even out long walks.  They come on
+// top of the 3 GiB; under a limit that the caller has set, walks are cut only if the sums
+// fit beside the dS blocks.  0 for non-positive sizes.
 std::size_t mla_prefill_backward_workspace_elements(
     int batch_size,
     int sequence_length,
