@@ -999,6 +999,7 @@ struct BackwardShape {
     long long ds_floats;           // one chunk of pairs, `sharing` query heads each
     index_math::WalkCut cut;       // of the key blocks' walks
     long long partial_floats;      // one chunk of pairs; 0 if no walk is cut
+    long long workspace_floats;    // >= the sum of the three
 };
 
 BackwardShape backward_shape(int batch_size, int sequence_length, int heads, int kv_heads, int qk_head_size,
@@ -1017,14 +1018,21 @@ BackwardShape backward_shape(int batch_size, int sequence_length, int heads, int
     shape.pairs_per_launch = chunk < shape.pairs ? chunk : shape.pairs;
     shape.ds_floats = shape.pairs_per_launch * shape.sharing * ds_block_count(shape.key_blocks, shape.query_tiles) * DS_BLOCK_FLOATS;
     // one workgroup of the first pass per compute unit (the workspace's size is asked for without a device: 256 units)
-    shape.cut = index_math::choose_walk_cut(shape.pairs_per_launch, shape.key_blocks, shape.query_tiles, shape.sharing, 256);
-    shape.partial_floats = shape.cut.part_steps > 0
-        ? shape.pairs_per_launch * shape.cut.items * KBLOCK * (qk_head_size + v_head_size) : 0;
+    constexpr int SLOTS = 256;
+    const long long part_floats = KBLOCK * (qk_head_size + v_head_size);
+    shape.cut = index_math::choose_walk_cut(shape.pairs_per_launch, shape.key_blocks, shape.query_tiles, shape.sharing, SLOTS);
+    shape.partial_floats = shape.cut.part_steps > 0 ? shape.pairs_per_launch * shape.cut.items * part_floats : 0;
+    index_math::WalkCutRoom room = index_math::walk_cut_room(shape.pairs_per_launch, shape.key_blocks, shape.query_tiles,
+                                                             shape.sharing, SLOTS, DS_BLOCK_FLOATS);
     // the sums of the parts stay inside a budget that the caller has set
-    if (ds_budget_override.load(std::memory_order_relaxed) > 0 && 4 * (shape.ds_floats + shape.partial_floats) > ds_budget_bytes()) {
+    if (ds_budget_override.load(std::memory_order_relaxed) > 0) room.floats = std::min(room.floats, ds_budget_bytes() / 4);
+    if (shape.partial_floats > room.parts * part_floats || shape.ds_floats + shape.partial_floats > room.floats) {
         shape.cut = index_math::WalkCut{0, shape.key_blocks, 0};
         shape.partial_floats = 0;
     }
+    // room for the sums of shorter calls with as many pairs or fewer, too
+    shape.workspace_floats = shape.statistics_floats +
+        std::max(shape.ds_floats, std::min(shape.ds_floats + room.parts * part_floats, room.floats));
     return shape;
 }
 
@@ -1092,8 +1100,7 @@ std::size_t attention_backward_workspace_elements(int batch_size, int sequence_l
         throw std::invalid_argument("attention backward: query heads must be a positive multiple of key/value heads");
     }
     auto elements = [&](int qk, int v) {
-        const BackwardShape shape = backward_shape(batch_size, sequence_length, heads, kv_heads, qk, v);
-        return static_cast<std::size_t>(shape.statistics_floats + shape.ds_floats + shape.partial_floats);
+        return static_cast<std::size_t>(backward_shape(batch_size, sequence_length, heads, kv_heads, qk, v).workspace_floats);
     };
     if ((qk_head_size == 192 && v_head_size == 128) || (qk_head_size == v_head_size && (v_head_size == 64 || v_head_size == 128))) {
         return elements(qk_head_size, v_head_size);

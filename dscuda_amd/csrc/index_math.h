@@ -117,6 +117,24 @@ inline WalkCut choose_walk_cut(long long pairs, int key_blocks, int query_tiles,
     return cut;
 }
 
+// What a cut may ask of the workspace: at most `parts` parts, and `floats` floats for their sums and the dS blocks
+// (`block_floats` each, one per step) together.  Both grow with every argument, as the dS blocks do, so that a workspace
+// asked for the longest sequence and the most heads of a program also holds the sums of shorter calls that are cut where
+// those are not.  No cut of choose_walk_cut comes near them (1827 parts and 1.33 blocks per slot and step of the longest
+// walk at most, up to 40000 tokens and 32 heads sharing).
+struct WalkCutRoom {
+    long long parts;
+    long long floats;
+};
+
+inline WalkCutRoom walk_cut_room(long long pairs, int key_blocks, int query_tiles, int sharing, int slots, long long block_floats) {
+    constexpr int MIN_PART = 6;
+    const long long longest = (long long)query_tiles * sharing;
+    if (longest < 2 * MIN_PART) return WalkCutRoom{0, 0};
+    const long long steps = pairs * sharing * ds_block_count(key_blocks, query_tiles);
+    return WalkCutRoom{std::min(8LL * slots, steps / MIN_PART + pairs * key_blocks), 11 * slots * longest * block_floats / 8};
+}
+
 // ---- tile requests of the backward kernels ------------------------------------
 // One wave's share of the global -> LDS requests of a [ROWS][ROW_BYTES] tile that
 // WAVES waves fetch together.  LDS slot 64*load + lane (16 bytes each) holds chunk

@@ -37,7 +37,9 @@ void flash_attention_forward_cuda(
 // pairs as one pass covers, and the fp32 sums of dK and dV of the parts a key block's walk
 // over the queries is cut into where the pairs alone would leave compute units idle: 128 KB
 // a part for 128 columns, up to 1800 parts, on top of the 3 GiB that the dS blocks may take;
-// under a limit that the caller has set, walks are cut only if both fit).  0 for shapes the
+// under a limit that the caller has set, walks are cut only if both fit).  While the dS
+// blocks fit one pass, a workspace for the longest sequence and the largest batch of a
+// program holds what shorter and smaller calls with the same heads need.  0 for shapes the
 // backward rejects.
 std::size_t flash_attention_backward_workspace_elements(
     int batch_size,

@@ -234,7 +234,9 @@ void mla_prefill_forward_cuda(
 // follow: 160 KB a part for 192/128 columns, some 260 parts where they run as one round,
 // up to 1800 (0.3 GB) where several rounds of parts even out long walks.  They come on
 // top of the 3 GiB; under a limit that the caller has set, walks are cut only if the sums
-// fit beside the dS blocks.  0 for non-positive sizes.
+// fit beside the dS blocks.  While the dS blocks fit one pass, a workspace for the longest
+// sequence, the largest batch and the most heads of a program holds what smaller calls
+// need.  0 for non-positive sizes.
 std::size_t mla_prefill_backward_workspace_elements(
     int batch_size,
     int sequence_length,

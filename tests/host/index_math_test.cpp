@@ -737,6 +737,34 @@ void check_walk_cut() {
     EXPECT(choose_walk_cut(4, 64, 128, 4, 256).part_steps > 0, "T=8192, 16 heads on 4");
 }
 
+// ---- room for the sums of cut walks: holds every cut, and grows with tokens, pairs and heads sharing
+void check_walk_cut_room() {
+    constexpr int SLOTS = 256;
+    constexpr long long BLOCK = 4096;
+    for (int columns : {320, 256, 128}) {
+        const long long part_floats = 128 * columns;
+        for (int sharing : {1, 2, 4, 8, 32}) {
+            for (int tiles = 1; tiles <= 512; tiles += tiles < 64 ? 1 : 13) {
+                const int blocks = (tiles + 1) / 2;
+                for (long long pairs = 1; pairs * blocks <= 4 * SLOTS && pairs <= 128; ++pairs) {
+                    const WalkCutRoom room = walk_cut_room(pairs, blocks, tiles, sharing, SLOTS, BLOCK);
+                    const long long ds = pairs * sharing * ds_block_count(blocks, tiles) * BLOCK;
+                    const WalkCut cut = choose_walk_cut(pairs, blocks, tiles, sharing, SLOTS);
+                    const WalkCutRoom longer = walk_cut_room(pairs, (tiles + 2) / 2, tiles + 1, sharing, SLOTS, BLOCK);
+                    const WalkCutRoom more = walk_cut_room(pairs + 1, blocks, tiles, sharing, SLOTS, BLOCK);
+                    const WalkCutRoom shared = walk_cut_room(pairs, blocks, tiles, sharing + 1, SLOTS, BLOCK);
+                    for (const WalkCutRoom& other : {longer, more, shared}) {
+                        EXPECT(other.parts >= room.parts && other.floats >= room.floats, "pairs %lld tiles %d sharing %d", pairs, tiles, sharing);
+                    }
+                    if (cut.part_steps == 0 || 4 * ds > 3LL << 30) continue;
+                    EXPECT(pairs * cut.items <= room.parts && ds + pairs * cut.items * part_floats <= room.floats,
+                           "pairs %lld tiles %d sharing %d: %lld parts of %lld", pairs, tiles, sharing, pairs * cut.items, room.parts);
+                }
+            }
+        }
+    }
+}
+
 // ---- kept P and dS of the short absorbed backward: every chunk has a place of its own inside rows that exist
 void check_kept_scores() {
     for (int heads : {1, 2, 3}) {
@@ -766,6 +794,7 @@ void check_kept_scores() {
 int main() {
     check_kept_scores();
     check_walk_cut();
+    check_walk_cut_room();
     check_split_order();
     check_forward_makespan();
     check_swizzle<128>();

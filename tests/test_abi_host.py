@@ -54,6 +54,23 @@ def test_workspace_elements_match_the_reference_formula():
     assert prefill(0, 65, 3, 192, 128) == 0
 
 
+def test_a_backward_workspace_serves_smaller_calls():
+    """One workspace for the longest sequence and the most heads of a program: the sums of walks that are cut in a
+    shorter call, where those of the longest are not, must lie inside it."""
+    prefill = bind(library("mla"), "dscuda_mla_prefill_backward_workspace_elements", [I] * 5, ctypes.c_size_t)
+    flash = bind(library("flash_attention"), "dscuda_flash_backward_workspace_elements", [I] * 5, ctypes.c_size_t)
+    for dqk, dv in ((192, 128), (64, 64)):
+        sizes = {(heads, seq): prefill(1, seq, heads, dqk, dv) for heads in range(1, 41) for seq in range(32, 4352, 96)}
+        for (heads, seq), elements in sizes.items():
+            assert elements <= sizes.get((heads, seq + 96), elements), (heads, seq)
+            assert elements <= sizes.get((heads + 1, seq), elements), (heads, seq)
+    for query_heads, kv_heads in ((8, 1), (16, 4), (32, 32)):
+        sizes = {(batch, seq): flash(batch, seq, query_heads, kv_heads, 128) for batch in range(1, 9) for seq in range(64, 3136, 64)}
+        for (batch, seq), elements in sizes.items():
+            assert elements <= sizes.get((batch, seq + 64), elements), (query_heads, kv_heads, batch, seq)
+            assert elements <= sizes.get((batch + 1, seq), elements), (query_heads, kv_heads, batch, seq)
+
+
 def test_size_queries_need_no_device():
     """Every size query is arithmetic on its integer arguments (benchmarks/bindings/mla_bridge.cu:53-56 is): on a host
     without a GPU it returns, in a process of its own so that an exception let through the C boundary shows up as a
