@@ -65,15 +65,6 @@ __device__ __forceinline__ void direct_load_4_offset(const void* uniform_base, u
                  : "memory", "m0");
 }
 
-// f(integral_constant<int, BEGIN>) ... f(integral_constant<int, END - 1>)
-template <int BEGIN, int END, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (BEGIN < END) {
-        f(std::integral_constant<int, BEGIN>{});
-        static_for<BEGIN + 1, END>(f);
-    }
-}
-
 // Registers of an operand that stays with the wave: row `row` of a [.][D] matrix.
 template <int D>
 __device__ __forceinline__ void load_row_fragments(bf16x8 (&fragments)[D / 16], const bf16_t* base, size_t row_stride,
@@ -377,8 +368,8 @@ __global__ __launch_bounds__(KV_THREADS) void attention_key_value_gradient_kerne
             unsigned q_at[TileReads<C::Q_ROW>::NAT];
             rebase(q_at, q_reads.natural, stage);
             const unsigned stats_at = opaque(stage + C::Q_BYTES + C::O_BYTES + 16 * g);
-            static_for<0, RING>([&](auto k_tag) { ring[decltype(k_tag)::value] = s_fragment(q_at, k_tag); });
-            static_for<0, S_MFMAS>([&](auto k_tag) {
+            unrolled<0, RING>([&](auto k_tag) { ring[decltype(k_tag)::value] = s_fragment(q_at, k_tag); });
+            unrolled<0, S_MFMAS>([&](auto k_tag) {
                 constexpr int K = decltype(k_tag)::value;
                 constexpr int KS = K / 2;
                 s_acc[K % 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[K % RING], kf[KS],
@@ -416,9 +407,9 @@ __global__ __launch_bounds__(KV_THREADS) void attention_key_value_gradient_kerne
             // local index below `threshold` lies before this lane's key.
             u32x4 pf[2][2];
             const int threshold = key_row - 4 * g - (query_tiles - 1 - local) * QTILE;
-            static_for<0, 2>([&](auto qb_tag) {
+            unrolled<0, 2>([&](auto qb_tag) {
                 constexpr int QB = decltype(qb_tag)::value;
-                static_for<0, 4>([&](auto i4_tag) {
+                unrolled<0, 4>([&](auto i4_tag) {
                     constexpr int I4 = decltype(i4_tag)::value;
                     float p[4];
 #pragma unroll
@@ -436,7 +427,7 @@ __global__ __launch_bounds__(KV_THREADS) void attention_key_value_gradient_kerne
                 });
             });
             // hand P to the key wave
-            static_for<0, 4>([&](auto piece_tag) {
+            unrolled<0, 4>([&](auto piece_tag) {
                 constexpr int PIECE = decltype(piece_tag)::value;
                 *reinterpret_cast<u32x4*>(lds + handover + PIECE * 1024) = pf[PIECE / 2][PIECE % 2];
             });
@@ -453,8 +444,8 @@ __global__ __launch_bounds__(KV_THREADS) void attention_key_value_gradient_kerne
             const unsigned stage = (index % 3) * C::STAGE_BYTES;
             unsigned o_at[2][TileReads<C::O_ROW>::TR];
             rebase(o_at, o_reads.transposed, stage + C::Q_BYTES);
-            static_for<0, RING>([&](auto k_tag) { ring[decltype(k_tag)::value] = dv_fragment(o_at, k_tag); });
-            static_for<0, DV_MFMAS>([&](auto k_tag) {
+            unrolled<0, RING>([&](auto k_tag) { ring[decltype(k_tag)::value] = dv_fragment(o_at, k_tag); });
+            unrolled<0, DV_MFMAS>([&](auto k_tag) {
                 constexpr int K = decltype(k_tag)::value;
                 constexpr int STEP = K / DV_BLOCKS;   // 16-query step
                 constexpr int D = K % DV_BLOCKS;
@@ -554,9 +545,9 @@ __global__ __launch_bounds__(KV_THREADS) void attention_key_value_gradient_kerne
             // tile's delta values ahead
             f32x16 dp_acc[2];
             f32x4 delta4[2][4];   // queries 32*qb + 8*i4 + 4*g + (0..3)
-            static_for<0, RING>([&](auto k_tag) { ring[decltype(k_tag)::value] = dp_fragment(o_at, k_tag); });
+            unrolled<0, RING>([&](auto k_tag) { ring[decltype(k_tag)::value] = dp_fragment(o_at, k_tag); });
             rebase(q_at, q_reads.transposed, stage);
-            static_for<0, DP_MFMAS>([&](auto k_tag) {
+            unrolled<0, DP_MFMAS>([&](auto k_tag) {
                 constexpr int K = decltype(k_tag)::value;
                 constexpr int KS = K / 2;
                 dp_acc[K % 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[K % RING], vf[KS],
@@ -576,18 +567,18 @@ __global__ __launch_bounds__(KV_THREADS) void attention_key_value_gradient_kerne
 
             // dS = P (dP - delta): lane holds key lq and queries 32*qb + 8*i4 + 4*g + e
             u32x4 packed[4];      // pieces (query half, 16-query step)
-            static_for<0, 4>([&](auto piece_tag) {
+            unrolled<0, 4>([&](auto piece_tag) {
                 constexpr int PIECE = decltype(piece_tag)::value;
                 packed[PIECE] = *reinterpret_cast<const u32x4*>(lds + handover + PIECE * 1024);
             });
             unsigned char* block = ds_group + member * ds_head_bytes +
                 (size_t)ds_block_index(kb, query_tiles - 1 - local, query_tiles) * DS_BLOCK_BYTES;
             u32x4 dsf[2][2];
-            static_for<0, 4>([&](auto piece_tag) {
+            unrolled<0, 4>([&](auto piece_tag) {
                 constexpr int PIECE = decltype(piece_tag)::value;
                 constexpr int QB = PIECE / 2;
                 constexpr int N = PIECE % 2;
-                static_for<0, 2>([&](auto half_tag) {
+                unrolled<0, 2>([&](auto half_tag) {
                     constexpr int HALF = decltype(half_tag)::value;
                     constexpr int I4 = 2 * N + HALF;
                     float ds[4];
@@ -604,7 +595,7 @@ __global__ __launch_bounds__(KV_THREADS) void attention_key_value_gradient_kerne
                 __builtin_nontemporal_store(dsf[QB][N], reinterpret_cast<u32x4*>(block + (ds_slot[N] + QB * 2048)));
             });
             // dK += dS^T Q
-            static_for<0, DK_MFMAS>([&](auto k_tag) {
+            unrolled<0, DK_MFMAS>([&](auto k_tag) {
                 constexpr int K = decltype(k_tag)::value;
                 constexpr int STEP = K / DK_BLOCKS;
                 constexpr int D = K % DK_BLOCKS;

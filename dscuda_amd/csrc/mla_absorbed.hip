@@ -143,20 +143,11 @@ __device__ __forceinline__ void clear(f32x16& value) {
     for (int i = 0; i < 16; ++i) value[i] = 0.f;
 }
 
-// f(integral_constant<int, BEGIN>) ... f(integral_constant<int, END - 1>)
-template <int BEGIN, int END, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (BEGIN < END) {
-        f(std::integral_constant<int, BEGIN>{});
-        static_for<BEGIN + 1, END>(f);
-    }
-}
-
 // COUNT MFMAs, each fed by one LDS fragment read AHEAD steps before its use: with one wave per SIMD nothing
 // else hides the latency of the reads.  `ring` holds fragments 0 .. AHEAD-1 on entry.
 template <int COUNT, int AHEAD, typename Fragment, typename Multiply>
 __device__ __forceinline__ void fragment_stream(bf16x8 (&ring)[AHEAD], Fragment&& fragment, Multiply&& multiply) {
-    static_for<0, COUNT>([&](auto tag) {
+    unrolled<0, COUNT>([&](auto tag) {
         constexpr int I = decltype(tag)::value;
         multiply(tag, ring[I % AHEAD]);
         if constexpr (I + AHEAD < COUNT) ring[I % AHEAD] = fragment(std::integral_constant<int, I + AHEAD>{});
@@ -166,7 +157,7 @@ __device__ __forceinline__ void fragment_stream(bf16x8 (&ring)[AHEAD], Fragment&
 
 template <int AHEAD, typename Fragment>
 __device__ __forceinline__ void fill_ring(bf16x8 (&ring)[AHEAD], Fragment&& fragment) {
-    static_for<0, AHEAD>([&](auto tag) { ring[decltype(tag)::value] = fragment(tag); });
+    unrolled<0, AHEAD>([&](auto tag) { ring[decltype(tag)::value] = fragment(tag); });
 }
 
 // The score products of a 32 x 32 tile are split over the four waves: each forms one 16 x 16 quadrant (16x16x32
@@ -484,7 +475,7 @@ __device__ __forceinline__ void query_gradient_walk(
                 if (any) dsf[t][n] = exchange_fragment(exchange + t * EXCHANGE_BYTES, lq, g, n);
             }
         }
-        static_for<0, 2 * HELD>([&](auto tag) {
+        unrolled<0, 2 * HELD>([&](auto tag) {
             constexpr int I = decltype(tag)::value;
             constexpr int N = I / HELD;
             constexpr int F = I % HELD;
@@ -506,7 +497,7 @@ __device__ __forceinline__ void query_gradient_walk(
     // t + 1 arrives in the other buffer; past the last tile the last one is requested again, into a buffer nobody
     // reads, which keeps the streams free of branches.  One more step lets the gradient waves catch up.
     begin_requests(0, 0);
-    static_for<0, REQUESTS>(request);
+    unrolled<0, REQUESTS>(request);
     wait_vector_memory<0>();
     workgroup_barrier();
     for (int tile = 0; tile <= tiles; ++tile) {
@@ -859,7 +850,7 @@ __device__ __forceinline__ void key_gradient_walk(
                     dsf[n] = exchange_fragment(exchange + EXCHANGE_BYTES, lq, g, n);
                 }
             }
-            static_for<0, 2 * PER_STEP>([&](auto tag) {
+            unrolled<0, 2 * PER_STEP>([&](auto tag) {
                 constexpr int I = decltype(tag)::value;
                 constexpr int N = I / PER_STEP;
                 constexpr int F = I % PER_STEP;
@@ -885,7 +876,7 @@ __device__ __forceinline__ void key_gradient_walk(
         // t + 1 arrives in the other buffer.  One more step after the last tile lets the gradient waves catch up.
         // Every step ends with a barrier behind all LDS reads, so the buffers are free when a segment begins.
         begin_requests(first_tile, 0);
-        static_for<0, REQUESTS>(request);
+        unrolled<0, REQUESTS>(request);
         wait_vector_memory<0>();
         place_statistics(0);
         workgroup_barrier();
@@ -1244,7 +1235,7 @@ __device__ __forceinline__ void key_pair_walk(
                 }
             }
         }
-        static_for<0, 2 * PER_STEP>([&](auto tag) {
+        unrolled<0, 2 * PER_STEP>([&](auto tag) {
             constexpr int I = decltype(tag)::value;
             constexpr int N = I / PER_STEP;
             constexpr int F = I % PER_STEP;
@@ -1273,7 +1264,7 @@ __device__ __forceinline__ void key_pair_walk(
     // Step t: tile t is in buffer t % 2 (scored there, and picked up by the gradient waves for step t + 1), tile
     // t + 1 arrives in the other buffer.  One more step after the last tile lets the gradient waves catch up.
     begin_requests(first_tile, 0);
-    static_for<0, REQUESTS>(request);
+    unrolled<0, REQUESTS>(request);
     wait_vector_memory<0>();
     place_statistics(0);
     workgroup_barrier();

@@ -49,14 +49,6 @@ constexpr int AHEAD = 6;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4* transposing_read_pointer;
 
-template <int BEGIN, int END, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (BEGIN < END) {
-        f(std::integral_constant<int, BEGIN>{});
-        static_for<BEGIN + 1, END>(f);
-    }
-}
-
 // W[h] ([128][512], `weight`) -> LDS, 16-byte pieces
 // (sixteen loads in flight per thread and round trip: one at a time, the 32 round trips of a thread's share were a
 // third of the kernel's time)
@@ -192,8 +184,8 @@ __global__ __launch_bounds__(THREADS) void mla_absorb_query_kernel(bf16_t* __res
             for (int i = 0; i < 16; ++i) acc[b][i] = 0.f;
         }
         bf16x8 ring[AHEAD];
-        static_for<0, AHEAD>([&](auto tag) { ring[decltype(tag)::value] = weight_fragment(tag); });
-        static_for<0, KSTEPS * BLOCKS>([&](auto tag) {
+        unrolled<0, AHEAD>([&](auto tag) { ring[decltype(tag)::value] = weight_fragment(tag); });
+        unrolled<0, KSTEPS * BLOCKS>([&](auto tag) {
             constexpr int I = decltype(tag)::value;
             acc[I % BLOCKS] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[I % AHEAD], xf[I / BLOCKS], acc[I % BLOCKS], 0, 0, 0);
             if constexpr (I + AHEAD < KSTEPS * BLOCKS) {
@@ -253,8 +245,8 @@ __global__ __launch_bounds__(THREADS) void mla_unabsorb_output_kernel(bf16_t* __
             for (int i = 0; i < 16; ++i) acc[b][i] = 0.f;
         }
         bf16x8 ring[AHEAD];
-        static_for<0, AHEAD>([&](auto tag) { ring[decltype(tag)::value] = weight_fragment(tag); });
-        static_for<0, KSTEPS * BLOCKS>([&](auto tag) {
+        unrolled<0, AHEAD>([&](auto tag) { ring[decltype(tag)::value] = weight_fragment(tag); });
+        unrolled<0, KSTEPS * BLOCKS>([&](auto tag) {
             constexpr int I = decltype(tag)::value;
             acc[I % BLOCKS] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[I % AHEAD], xf[I / BLOCKS], acc[I % BLOCKS], 0, 0, 0);
             if constexpr (I + AHEAD < KSTEPS * BLOCKS) {
