@@ -24,6 +24,9 @@ extern "C" int backward_ranges(int batch, int tokens, int heads, int compute_uni
     return (int)key_gradient_ranges(visits.per_batch() * batch, (long long)visits.key_blocks * batch, visits.row_tiles,
                                     (long long)tokens * heads * batch * 1024, compute_units);
 }
+extern "C" int walks_are_cut(int pairs, int tokens, int sharing) {
+    return choose_walk_cut(pairs, (tokens + 127) / 128, (tokens + 63) / 64, sharing, 256).part_steps > 0;
+}
 extern "C" int keeps_scores(int batch, int tokens, int heads) { return short_backward(batch, tokens, heads); }
 """
 

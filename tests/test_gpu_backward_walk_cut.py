@@ -6,6 +6,7 @@ import torch
 
 from dscuda_amd.harness import configs, ops
 from oracle import attention_oracle as oracle
+from tests.dispatch_rules import rules
 from tests.parity import announce, assert_close_bf16
 
 pytestmark = pytest.mark.gpu
@@ -32,9 +33,10 @@ def test_cut_walks(cuda, batch, seq, q_heads, kv_heads, dqk, dv):
         workspace = ops.flash_backward_workspace(batch, seq, q_heads, kv_heads, dqk)
     else:
         workspace = ops.mla_prefill_backward_workspace(batch, seq, q_heads, dqk, dv)
+    assert rules().walks_are_cut(batch * kv_heads, seq, q_heads // kv_heads)
     key_blocks, tiles = (seq + 127) // 128, (seq + 63) // 64
     blocks = sum(tiles - 2 * kb for kb in range(key_blocks))
-    assert workspace.numel() > batch * q_heads * (tiles * 128 + blocks * 4096)   # room for partial sums: the walks are cut
+    assert workspace.numel() > batch * q_heads * (tiles * 128 + blocks * 4096)   # room for partial sums
     workspace.fill_(float("nan"))
     runs = []
     for _ in range(2):
