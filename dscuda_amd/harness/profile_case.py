@@ -12,7 +12,8 @@ Workloads: forward / backward (B=1, S, H=128, 192|128), decode (B=64, H=128,
 lengths ~ U[1024, 8192] seed 3), flash (B=1, H=8, S=512, D=64), absorbed (the
 reference's own prefill entry points, forward then backward, B=1, T=S, H heads,
 512 latent + 64 rope), projection (the W_UK absorb and W_UV un-absorb of S tokens x
-H heads), copy (a plain 16-byte-per-lane copy of 1 GiB, the calibration kernel for
+H heads), rope (the rotary embedding of the rope columns of S query rows x H heads, in
+place), copy (a plain 16-byte-per-lane copy of 1 GiB, the calibration kernel for
 FETCH_SIZE / WRITE_SIZE).  ``--data zero`` fills every input with zeros: the kernels
 execute the same instructions, only the operands stop toggling, which separates what a
 workload loses to the chip's power limit (the clock it is given) from what its schedule loses.
@@ -31,7 +32,7 @@ if str(ROOT) not in sys.path:
 
 def main():
     parser = argparse.ArgumentParser(description=__doc__)
-    parser.add_argument("workload", choices=("forward", "backward", "decode", "flash", "absorbed", "projection", "copy"))
+    parser.add_argument("workload", choices=("forward", "backward", "decode", "flash", "absorbed", "projection", "rope", "copy"))
     parser.add_argument("--steps", type=int, default=3)
     parser.add_argument("--seq", type=int, default=4096)
     parser.add_argument("--heads", type=int, default=128)
@@ -100,6 +101,9 @@ def main():
         def call():
             ops.mla_absorb_query(q_nope, wkv_b[:, :128], out=q_latent)
             ops.mla_unabsorb_output(o_latent, wkv_b[:, 128:], out=o)
+    elif args.workload == "rope":
+        tensor = randn((1, args.seq, args.heads, 192), 0.5)
+        call = lambda: ops.rope_apply(tensor, rope_offset=128)
     elif args.workload == "flash":
         q, k, v = randn((1, 512, 8, 64), 1.0), randn((1, 512, 8, 64), 1.0), randn((1, 512, 8, 64), 1.0)
         out, lse = torch.empty_like(q), torch.empty(1, 8, 512, device=device)

@@ -90,6 +90,7 @@ BACKWARD_KERNELS = ["attention_backward", "attention_key_value", "attention_quer
 DECODE_KERNELS = ["mla_decode", "mla_narrow_decode", "mla_narrow_merge"]
 ABSORBED_KERNELS = ["mla_absorbed", "mla_narrow_forward", "mla_short"]
 PROJECTION_KERNELS = ["mla_absorb_query", "mla_unabsorb_output"]
+ROPE_KERNELS = ["rope_apply"]
 
 
 def _python_case(workload, steps, counter_steps, *extra):
@@ -135,6 +136,17 @@ def metric_cases(suite):
             "backward", 80, 30, BACKWARD_KERNELS, "--data", "zero")
         add("mla_decode_B64_H128_zero_inputs", "absorbed MLA decode B=64 H=128 lengths U[1024,8192] seed 3, query and cache zero",
             "decode", 300, 100, DECODE_KERNELS, "--data", "zero")
+        # few heads or tokens: cut walks, kept scores, 32 rows per workgroup, a quarter of a head's weight
+        add("mla_prefill_backward_S1000_H16", "MLA prefill backward B=1 S=1000 H=16 192/128", "backward", 300, 100,
+            BACKWARD_KERNELS, "--seq", 1000, "--heads", 16)
+        add("mla_absorbed_T512_H8", "absorbed MLA prefill forward + backward B=1 T=512 H=8", "absorbed", 300, 100,
+            ABSORBED_KERNELS, "--seq", 512, "--heads", 8)
+        add("mla_decode_B64_H16", "absorbed MLA decode B=64 H=16 lengths U[1024,8192] seed 3", "decode", 300, 100,
+            DECODE_KERNELS, "--heads", 16)
+        add("mla_projection_T16_H16", "W_UK absorb and W_UV un-absorb of 16 tokens x 16 heads", "projection", 300, 100,
+            PROJECTION_KERNELS, "--seq", 16, "--heads", 16)
+        add("rope_T4096_H128", "rotary embedding of 4096 tokens x 128 heads, columns 128..191 of 192", "rope", 300, 100,
+            ROPE_KERNELS)
     return cases
 
 
