@@ -18,8 +18,9 @@
 // A 128-row workgroup takes 4000 a unit, so 32 rows win while the chip has idle compute
 // units, 64 rows where the key stream (one 36 KB unit per workgroup) is the bound and 128
 // where everything is busy.  Measured, 128-row kernels -> these: decode of 16 sequences
-// x 16 heads x 1024..4096 tokens 44 -> 22 us, 64 x 16 x 1024..8192 104 -> 69 us (5.5 TB/s),
-// 16 x 128 x 1024..8192 64 -> 50 us; prefill T = 512, H = 8 39 -> 19 us.
+// x 16 heads x 1024..4096 tokens 44 -> 22 us, 64 x 16 x 1024..8192 104 -> 69 us (384 MB at
+// 5.7 TB/s under the profiler), 16 x 128 x 1024..8192 64 -> 47 us; prefill T = 512, H = 8
+// 39 -> 19 us.
 //
 // Softmax reference.  As in mla_decode.hip the exponentials are taken against the first
 // unit's maximum plus a head room, and the reference is raised when a row outruns it (next to
