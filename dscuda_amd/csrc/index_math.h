@@ -757,8 +757,9 @@ DSCUDA_HOST_DEVICE inline DecodeLayout decode_layout(int batch, int heads, int s
 // for batches all of whose sequences the ranges of decode_layout (`reference_ranges`) cut as well; any other batch is
 // cut into `wide_ranges` ranges with fp32 parts, for which slots of twice the size leave room, or as decode_layout would
 // (wide_ranges 0) if that makes more ranges; a workgroup per sequence where decode_layout has that and the ranges would be
-// fewer than the sequences (ranges / workgroups: two sequences of 13 tokens, 16 heads, 2 splits 16.6 / 7.3 us).  us with bf16 parts throughout -> so, eight heads, 8 splits: eight sequences
-// of 1024..8192 tokens 24.7 -> 35.1, 1 of 400 11.0 -> 13.4; 16 heads, 2 splits, eight of 1024..8192 62.8 -> 171.
+// fewer than the sequences (ranges / workgroups: two sequences of 13 tokens, 16 heads, 2 splits 16.6 / 7.3 us).  bf16 parts
+// throughout -> so, us: eight heads, 8 splits, eight sequences of 1024..8192 tokens 24.7 -> 35.1, 1 of 400 11.0 -> 13.4;
+// 16 heads, 2 splits, eight of 1024..8192 62.8 -> 171.
 DSCUDA_HOST_DEVICE inline DecodeLayout narrow_decode_layout(int batch, int heads, int splits, int compute_units,
                                                             int row_blocks, int rank) {
     DecodeLayout layout;

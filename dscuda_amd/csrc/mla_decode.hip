@@ -659,9 +659,9 @@ __global__ __launch_bounds__(THREADS) void mla_decode_split_kernel(
 // pieces of output rows.  Bound by round trips to partial results that another XCD wrote:
 // statistics and pieces of MERGE_AHEAD parts (more than most sequences have) are asked for
 // at once, before the first of them is needed.  One part after the other, a quarter of the columns per
-// wave, took 13.2 us for 64 sequences x 128 heads (five parts each, 40 MB); so 10.3 us.  Whole
-// calls: that 119.4 -> 116.6 us, 32 x 128 78.6 -> 73.8, 28 x 128 x 200..1000 tokens 38.1 -> 33.6,
-// 4 x 1024 98.9 -> 93.1.
+// wave, took 12.4 us for 64 sequences x 128 heads (five parts each, 40 MB) under the profiler; so
+// 10.0 us.  Whole calls: that 119 -> 117 us (boxes differ by as much, both sides in turn), 32 x 128
+// 78.6 -> 73.8, 28 x 128 x 200..1000 tokens 38.1 -> 33.6, 4 x 1024 98.9 -> 93.1.
 constexpr int MERGE_SLICES = 8;
 constexpr int MERGE_PIECES = PARTIAL_PIECES / MERGE_SLICES;         // 4 pieces of 16 bytes per lane and part
 constexpr int MERGE_COLUMNS = RANK / MERGE_SLICES;                  // 64

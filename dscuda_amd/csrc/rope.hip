@@ -20,9 +20,10 @@
 // 2 * rope bytes.  The kernel moves 4 * rope bytes per (b, s, h) and is bound by memory:
 // BATCH heads of a group are fetched before the first is stored (in place, so the loads
 // would otherwise wait for the stores, a round trip per head), and where the rows alone
-// leave the chip idle the heads are sliced so that one batch covers a wave.  64 rows of
-// 128 heads 11.9 -> 3.5 us, 1024 rows 14.4 -> 9.4, 4096 rows 29.3 -> 23.8 (134 MB at 5.7 TB/s
-// under the profiler).
+// leave the chip idle the heads are sliced so that one batch covers a wave.  The last batch
+// asks for its own heads only (repeating the last head instead: 60 x 804 rows of 17 heads
+// 40.1 us, so 34.1).  64 rows of 128 heads 11.9 -> 3.5 us, 1024 rows 14.4 -> 8.0, 4096 rows
+// 28.9 -> 22.6 (134 MB at 6 TB/s).
 
 #include "attn_kernels.h"
 #include "hip_common.h"
@@ -37,8 +38,9 @@ namespace {
 
 constexpr int ROPE_THREADS = 256;
 constexpr int ROPE_ROWS = ROPE_THREADS / 64;   // (batch, position) rows per workgroup
-constexpr int BATCH = 8;                       // heads a group of lanes has in flight
 
+// BATCH: heads a group of lanes has in flight
+template <int BATCH>
 __global__ __launch_bounds__(ROPE_THREADS) void rope_apply_kernel(bf16_t* __restrict__ tensor,
                                                                   const int* __restrict__ positions, long long rows,
                                                                   int sequence_length, int heads, int slice, int width,
@@ -59,19 +61,29 @@ __global__ __launch_bounds__(ROPE_THREADS) void rope_apply_kernel(bf16_t* __rest
     const float sine = (float)sin(angle);
     unsigned* base = reinterpret_cast<unsigned*>(tensor + (size_t)row * heads * width + rope_offset) + pair;
     const int end = min(heads, (int)(blockIdx.y + 1) * slice);
+    auto rotate = [&](int h, unsigned bits) {
+        const float even = __uint_as_float(bits << 16);
+        const float odd = __uint_as_float(bits & 0xffff0000u);
+        const float rotated_even = __fsub_rn(__fmul_rn(even, cosine), __fmul_rn(odd, sine));
+        const float rotated_odd = __fadd_rn(__fmul_rn(even, sine), __fmul_rn(odd, cosine));
+        base[(size_t)h * (width / 2)] = pack_bf16(rotated_even, rotated_odd);
+    };
     for (int first = blockIdx.y * slice + group; first < end; first += groups * BATCH) {
         unsigned bits[BATCH];
+        if (first + (BATCH - 1) * groups < end) {
 #pragma unroll
-        for (int j = 0; j < BATCH; ++j) {
-            bits[j] = base[(size_t)min(first + j * groups, end - 1) * (width / 2)];
-        }
+            for (int j = 0; j < BATCH; ++j) bits[j] = base[(size_t)(first + j * groups) * (width / 2)];
 #pragma unroll
-        for (int j = 0; j < BATCH; ++j) {
-            const float even = __uint_as_float(bits[j] << 16);
-            const float odd = __uint_as_float(bits[j] & 0xffff0000u);
-            const float rotated_even = __fsub_rn(__fmul_rn(even, cosine), __fmul_rn(odd, sine));
-            const float rotated_odd = __fadd_rn(__fmul_rn(even, sine), __fmul_rn(odd, cosine));
-            if (first + j * groups < end) base[(size_t)(first + j * groups) * (width / 2)] = pack_bf16(rotated_even, rotated_odd);
+            for (int j = 0; j < BATCH; ++j) rotate(first + j * groups, bits[j]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < BATCH; ++j) {
+                if (first + j * groups < end) bits[j] = base[(size_t)(first + j * groups) * (width / 2)];
+            }
+#pragma unroll
+            for (int j = 0; j < BATCH; ++j) {
+                if (first + j * groups < end) rotate(first + j * groups, bits[j]);
+            }
         }
     }
 }
@@ -106,12 +118,18 @@ void rope_apply_dispatch(bf16_t* tensor, const int* positions, int batch_size, i
         throw std::invalid_argument("rope: batch * sequence length exceeds the grid limit");
     }
     // below four workgroups per compute unit the heads are sliced, one batch of every group of lanes a slice
-    const int batch_heads = 64 / (rope_size / 2) * BATCH;
-    const int slice = blocks < 4LL * hip_common::compute_units_of_current_device() && (heads - 1) / batch_heads < 65535
-        ? batch_heads : heads;
+    constexpr int BATCH = 8;
+    const int groups = 64 / (rope_size / 2);
+    const int batch_heads = groups * BATCH;
+    const bool sliced = blocks < 4LL * hip_common::compute_units_of_current_device() && (heads - 1) / batch_heads < 65535;
+    const int slice = sliced ? batch_heads : heads;
     const unsigned slices = (unsigned)((heads + (long long)slice - 1) / slice);
-    hipLaunchKernelGGL(rope_apply_kernel, dim3((unsigned)blocks, slices), dim3(ROPE_THREADS), 0, stream, tensor, positions,
-                       rows, sequence_length, heads, slice, width, rope_offset, rope_size, std::log2((double)theta));
+    // One head at a time where rows abound and a group of lanes has few heads: the rows cover the round trips, and the
+    // comparisons of a batch are time (eight in flight / one, us: 204845 rows of one head 87.7 / 81.7, 16384 rows of one
+    // 9.1 / 8.5, of two 9.6 / 8.9, 35742 rows of four 21.3 / 20.4; 16000 rows of eight 11.4 / 11.9).
+    const auto kernel = !sliced && heads < 4 * groups ? rope_apply_kernel<1> : rope_apply_kernel<BATCH>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks, slices), dim3(ROPE_THREADS), 0, stream, tensor, positions, rows,
+                       sequence_length, heads, slice, width, rope_offset, rope_size, std::log2((double)theta));
     HIP_CHECK(hipGetLastError());
 }
 

@@ -90,6 +90,9 @@ def test_rope_rejects_bad_slices(cuda):
     ((1, 4, 9, 128), 128),      # one pair per lane: batches of eight heads, the last slice holds one
     ((1, 4100, 19, 8), 8),      # many rows: the heads in one slice, 16 groups of lanes
     ((1, 4100, 18, 64), 64),    # ... and a second batch of two heads
+    ((1, 4100, 7, 64), 64),     # many rows of few heads: one at a time, the last group of lanes one less
+    ((1, 4100, 8, 64), 64),     # ... and the first count that goes by batches, a part of one
+    ((1, 4100, 16, 64), 64),    # ... and a whole one
 ])
 def test_rope_slices_of_heads(cuda, shape, size):
     announce("rope, slices of heads", dict(shape=shape, size=size))
