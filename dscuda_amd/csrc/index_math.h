@@ -621,14 +621,17 @@ constexpr int SHORT_TOKENS = 512;
 // Which calls keep P and dS instead of partial key gradients.  More tokens do not fit.  The key-gradient launch walks
 // all rows of a batch element per 32 keys x 32 columns, so many rows, or many heads on few keys, are better off with
 // the other kernels; so are calls whose key blocks alone occupy half the chip there, and those with one row tile a batch
-// element, where one launch more is what counts.  Forward and backward, partial results -> kept (us): 512 tokens x 8
-// heads 106 -> 71, 300 x 4 106 -> 46, 350 x 16 82 -> 70, 128 x 32 56 -> 49, 3 x 500 x 4 142 -> 81, 8 x 500 x 4 169 -> 152.
-// Backward alone, kept / partial results, of calls left to the others: 200 x 32 and 480 x 16 equal, 4 x 512 x 8 1.04,
-// 2 x 174 x 32 1.06, 2 x 278 x 20 1.13, 3 x 302 x 16 1.10, 14 x 337 x 3 1.15, 13 x 359 x 2 1.11, 13 x 4 x 1 1.31; of calls
-// that keep them: 2 x 219 x 20 0.92, 4 x 113 x 20 0.81, 8 x 338 x 3 0.84, 9 x 301 x 3 0.87, 1 x 3 x 16 0.93.
+// element or with batch elements enough to fill the chip, where one launch more is what counts.  Forward and backward,
+// partial results -> kept (us): 512 tokens x 8 heads 106 -> 71, 300 x 4 106 -> 46, 350 x 16 82 -> 70, 128 x 32 56 -> 49,
+// 3 x 500 x 4 142 -> 81, 8 x 500 x 4 169 -> 152.  Backward alone, kept / partial results, of calls left to the others:
+// 200 x 32 and 480 x 16 equal, 4 x 512 x 8 1.04, 2 x 174 x 32 1.06, 2 x 278 x 20 1.13, 3 x 302 x 16 1.10, 14 x 337 x 3 1.15,
+// 13 x 359 x 2 1.11, 13 x 4 x 1 1.31, 64 x 2 x 20 1.41, 24 x 2 x 17 1.14, 16 x 4 x 9 1.05, 64 x 8 x 8 1.25, 64 x 48 x 4 1.17,
+// 24 x 100 x 1 1.11; of calls that keep them: 2 x 219 x 20 0.92, 4 x 113 x 20 0.81, 8 x 338 x 3 0.84, 9 x 301 x 3 0.87,
+// 1 x 3 x 16 0.93, 8 x 4 x 9 0.97, 32 x 16 x 8 0.91, 32 x 64 x 4 0.91, 16 x 100 x 1 1.00.
 DSCUDA_HOST_DEVICE inline bool short_backward(long long batch, int tokens, int heads) {
     const long long rows = (long long)tokens * heads;
     if (tokens > SHORT_TOKENS || heads > 32 || rows > 6000 || rows * batch > 16000 || rows <= 32) return false;
+    if (batch > (rows < 64 ? 12 : heads == 1 ? 16 : 32)) return false;
     if (heads <= 3) return batch * ((tokens + 31) / 32) <= 110;
     return heads < 16 || rows * batch * tokens <= (heads <= 20 ? 2000000 : 1600000);
 }

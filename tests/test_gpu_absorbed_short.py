@@ -45,6 +45,7 @@ def test_absorbed_backward_of_short_sequences(cuda, batch, tokens, heads):
 
 @pytest.mark.parametrize("batch,tokens,heads,kept", [
     (1, 33, 1, True), (1, 3, 11, True), (2, 2, 17, True), (9, 384, 1, True), (2, 219, 20, True),
+    (12, 2, 17, True), (32, 16, 4, True), (16, 100, 1, True), (13, 2, 17, False), (33, 16, 4, False), (17, 100, 1, False),
     (1, 1, 32, False), (13, 4, 8, False), (10, 353, 2, False), (2, 224, 20, False), (2, 160, 32, False),
 ])
 def test_which_calls_keep_their_scores(cuda, batch, tokens, heads, kept):
