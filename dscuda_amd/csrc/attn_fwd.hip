@@ -1248,21 +1248,18 @@ void attention_forward_dispatch(bf16_t* output, float* logsumexp, const bf16_t* 
         }
         return;
     }
-    // Persistent kernel or split keys: the tiles of the busiest workgroup against the steps (128 queries x 128 keys, 1.15
-    // tiles each, start and end of a workgroup 2.5 more) of the mean or the longest one.  Measured with either kernel
+    // Persistent kernel or split keys: the tiles of the busiest workgroup against index_math::split_forward_cost.  Measured with either kernel
     // forced, split / persistent in us, 192/128 columns: 16 heads of 1000 tokens 15.5 / 31.6, 128 of 1152 75.6 / 78.3,
     // 32 of 3313 120 / 109, 64 of 2048 97 / 90, 128 of 1700 157 / 144.  Where the two costs are within 5 %: 16 of 6573
     // 232 / 217, 40 of 5137 352 / 334, 32 of 5137 284 / 271, 48 of 3545 205 / 198, 128 of 2154 235 / 227, but 64 of 1301
     // 53 / 55 and 96 of 2154 165 / 167; 128/128 columns: 40 of 5120 274 / 256, 32 of 5120 220 / 211, but 96 of 1664
     // 86 / 89.
-    const double mean_steps = (double)batch_heads * (0.5 * blocks128 * (blocks128 + 1) + 2.5 * blocks128) / compute_units;
-    const double split_cost = 1.15 * std::max(mean_steps, blocks128 + 2.5);
     PingPongPlan plan = {};
     bool persistent = false;
     // the persistent kernel streams two tiles ahead across items: every item needs two tiles
-    if (sequence_length >= 128 && mean_steps > blocks128) {
+    if (sequence_length >= 128 && index_math::split_forward_steps(batch_heads, sequence_length, compute_units) > blocks128) {
         plan = pingpong_plan(batch_heads, sequence_length);
-        persistent = plan.choice.cost <= split_cost;
+        persistent = plan.choice.cost <= index_math::split_forward_cost(batch_heads, sequence_length, compute_units);
     }
     // 64 queries instead of 128 while that finds idle compute units, for long sequences up to one workgroup of 128 per
     // unit (64 / 128: 16 heads of 1000 tokens 16.3 / 20.6 us, 8 of 4096 47.5 / 57.6, 64 of 512 16.3 / 15.4, 32 of 1500

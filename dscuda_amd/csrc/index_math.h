@@ -293,7 +293,8 @@ inline int forward_makespan(int members, int /* clusters: all alike */, int clus
 // L2; where the rounds then do not come out even (2.5 rounds of items: the busiest workgroup has 1.4 times the mean),
 // more heads sorted together do: 32 heads of 7168 tokens 570 -> 463 us, 128 heads of 1700 tokens 168 -> 147 us with all
 // of a cluster's heads abreast.  Each doubling costs some 1.5 % through the L2 (128 heads of 4096 tokens, already even:
-// 642 us with two, 652 with eight, 676 with sixteen).
+// 642 us with two, 652 with eight, 676 with sixteen), and more than that for short sequences, so a gain of less than 3 %
+// is none (256 heads of 800 tokens, a gain of 0.1 %: 101.6 us with two, 106.5 with 32; 221 of 3700 1095 / 1137).
 struct ForwardChoice {
     int abreast;
     double cost;
@@ -309,15 +310,32 @@ inline ForwardChoice forward_choice(int members, int clusters, int cluster_heads
     const double mean = (double)total * cluster_heads / members;
     ForwardChoice best = {cluster_heads % 2 == 0 ? 2 : 1, 0.0};
     best.cost = forward_makespan(members, clusters, cluster_heads, sequence_length, best.abreast);
+    const double worth = 0.97 * best.cost;
     double penalty = 1.0;
     for (int abreast = 4; best.cost > 1.03 * mean && abreast / 2 < cluster_heads; abreast *= 2) {
         penalty += 0.015;
         const int heads = abreast < cluster_heads ? abreast : cluster_heads;
         if (cluster_heads % heads != 0) continue;
         const double cost = penalty * forward_makespan(members, clusters, cluster_heads, sequence_length, heads);
-        if (cost < best.cost) best = ForwardChoice{heads, cost};
+        if (cost < best.cost && cost < worth) best = ForwardChoice{heads, cost};
     }
     return best;
+}
+
+// The cost of the split-key kernel with 128 queries a workgroup in the same tiles: steps (128 queries x 128 keys, start and
+// end of a workgroup 2.5 more) of the mean or the longest workgroup, 1.15 tiles each.  Where the heads cannot be dealt to
+// the XCDs every L2 reads every head's keys, and a workgroup of 128 queries fetches each key twice as often as one of 256:
+// 1.17 times that (1.15 tiles throughout -> so, us, 192/128 columns: 171 heads of 1000 tokens 102 -> 92, 195 of 1300
+// 194 -> 169, 156 of 1800 258 -> 226, 67 of 2500 183 -> 153, 300 of 3700 2057 -> 1588; 128/128: 171 of 768 67 -> 54).
+inline double split_forward_steps(long long batch_heads, int sequence_length, int compute_units) {
+    const long long blocks = (sequence_length + 127LL) / 128;
+    return (double)batch_heads * (0.5 * blocks * (blocks + 1) + 2.5 * blocks) / compute_units;
+}
+
+inline double split_forward_cost(long long batch_heads, int sequence_length, int compute_units) {
+    const double step_tiles = batch_heads % 8 == 0 ? 1.15 : 1.15 * 1.17;
+    return step_tiles * std::max(split_forward_steps(batch_heads, sequence_length, compute_units),
+                                 (sequence_length + 127LL) / 128 + 2.5);
 }
 
 // ---- work order of the split-key forward kernel ----------------------------------

@@ -8,6 +8,8 @@
 #include <cstdlib>
 #include <set>
 #include <utility>
+#include <tuple>
+#include <utility>
 #include <vector>
 
 using namespace dscuda::index_math;
@@ -652,6 +654,18 @@ void check_split_order() {
                 }
             }
         }
+    }
+    // persistent or split keys, by what was measured: heads that no XCD order deals out, and those that one does
+    for (const auto& [heads, sequence, persistent] : {std::tuple{171, 1000, true}, {195, 1300, true}, {156, 1800, true},
+                                                      {300, 3700, true}, {67, 1000, false}, {130, 800, false},
+                                                      {136, 1000, false}, {128, 1152, false}, {128, 2048, true}}) {
+        const int clusters = heads % 8 == 0 ? 8 : 1;
+        const ForwardChoice choice = forward_choice(256 / clusters, clusters, heads / clusters, sequence);
+        EXPECT((choice.cost <= split_forward_cost(heads, sequence, 256)) == persistent, "%d heads of %d", heads, sequence);
+    }
+    for (const auto& [heads, sequence] : {std::pair{256, 800}, {221, 3700}}) {   // next to nothing to gain from more abreast
+        const int clusters = heads % 8 == 0 ? 8 : 1;
+        EXPECT(forward_choice(256 / clusters, clusters, heads / clusters, sequence).abreast <= 2, "%d heads of %d", heads, sequence);
     }
     for (int heads : {1, 2, 3, 4, 6, 16}) {
         for (int sequence : {128, 700, 1152, 4096, 5120}) {
