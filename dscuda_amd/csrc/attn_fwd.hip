@@ -418,6 +418,7 @@ __global__ __launch_bounds__(64 * QG * KG) void attention_forward_split_kernel(
     const int g = lane / 32;
 
     const index_math::SplitItem item = index_math::split_item(blockIdx.x, order);
+    if (item.batch >= order.batch) return;   // a slot of the last turn without a head
     const int h = item.head;
     const int qb = item.query_block;
     const int b = item.batch;
@@ -1118,16 +1119,19 @@ void launch_forward_split(bf16_t* output, float* logsumexp, const bf16_t* query,
                           hipStream_t stream) {
     using C = SplitConfig<DQK, DV, QG, KG>;
     const int query_blocks = (sequence_length + C::BM - 1) / C::BM;
-    const long long grid = (long long)batch_size * query_heads * query_blocks;
+    const long long batch_heads = (long long)batch_size * query_heads;
+    // 64 columns: for 128 the dispatch below has the persistent kernel there
+    const bool spread = DV == 64 && index_math::split_spreads(batch_heads, sequence_length) &&
+        (batch_heads + 7) * query_blocks <= 0x7fffffffLL;
+    const index_math::SplitOrder order = index_math::split_order(batch_size, query_heads, key_value_heads, query_blocks, spread);
     auto kernel = attention_forward_split_kernel<DQK, DV, QG, KG>;
     static hip_common::OncePerDevice raised;
     raised.run([&] {
         HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS_BYTES));
     });
-    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(C::THREADS), C::LDS_BYTES, stream, output, logsumexp, query, key,
-                       value, sequence_length, query_heads, key_value_heads,
-                       index_math::split_order(batch_size, query_heads, key_value_heads, query_blocks), scale);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)order.workgroups), dim3(C::THREADS), C::LDS_BYTES, stream, output, logsumexp,
+                       query, key, value, sequence_length, query_heads, key_value_heads, order, scale);
     HIP_CHECK(hipGetLastError());
 }
 

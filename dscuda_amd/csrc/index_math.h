@@ -375,16 +375,28 @@ struct SplitOrder {
     int clusters;
     int together;            // groups an XCD takes together
     int query_blocks;
+    int batch;
+    long long workgroups;    // of the launch; items with a batch index past the last one are nobody's
 };
 
-inline SplitOrder split_order(int batch, int query_heads, int key_value_heads, int query_blocks) {
+// Whether heads that are no multiple of eight are dealt to the XCDs all the same, the last turn to some of them only.
+// Undealt, every L2 reads every head's keys, which is slow as soon as they do not fit (64 columns, four waves with the heads
+// in turn / undealt / so, us: 221 heads of 448 tokens 25 / 25 / 20, 67 of 1728 66 / 65 / 46, 115 of 2368 145 / 193 / 124, 189 of
+// 3392 425 / 628 / 391, 250 of 5952 1620 / 2490 / 1467); with few heads the idle slots of the last turn, at most seven
+// heads, would weigh more.
+inline bool split_spreads(long long batch_heads, int sequence_length) {
+    return batch_heads % 8 != 0 && batch_heads >= 64 && batch_heads * sequence_length >= 50000;
+}
+
+inline SplitOrder split_order(int batch, int query_heads, int key_value_heads, int query_blocks, bool spread = false) {
     constexpr int XCDS = 8, UNITS = 32;
     SplitOrder order;
+    order.batch = batch;
     const int sharing = query_heads / key_value_heads;
     const bool by_group = (long long)batch * key_value_heads % XCDS == 0;
-    order.clusters = by_group || (long long)batch * query_heads % XCDS == 0 ? XCDS : 1;
+    order.clusters = by_group || spread || (long long)batch * query_heads % XCDS == 0 ? XCDS : 1;
     const int members = by_group ? sharing : 1;
-    const long long groups = (long long)batch * query_heads / members / order.clusters;   // of an XCD
+    const long long groups = ((long long)batch * query_heads / members + order.clusters - 1) / order.clusters;   // of an XCD
     const long long inner = (long long)members * query_blocks;
     long long together = groups;
     if (order.clusters > 1 && groups * inner > 4 * UNITS) {
@@ -392,6 +404,7 @@ inline SplitOrder split_order(int batch, int query_heads, int key_value_heads, i
         while (groups % together != 0) ++together;
     }
     order.together = (int)together;
+    order.workgroups = order.clusters * groups * inner;
     order.turn = fast_division((unsigned)(together * inner));
     order.abreast = fast_division((unsigned)(together * members));
     order.members = fast_division((unsigned)members);

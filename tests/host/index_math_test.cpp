@@ -642,15 +642,21 @@ void check_split_order() {
         for (int kv : {1, 2, 3, 4, 8}) {
             for (int sharing : {1, 2, 3, 8}) {
                 for (int blocks : {1, 2, 5, 17, 70}) {
-                    const SplitOrder order = split_order(batch, kv * sharing, kv, blocks);
+                  for (bool spread : {false, true}) {
+                    const SplitOrder order = split_order(batch, kv * sharing, kv, blocks, spread);
                     std::vector<int> seen(batch * kv * sharing * blocks, 0);
-                    for (int i = 0; i < (int)seen.size(); ++i) {
+                    EXPECT(order.workgroups >= (long long)seen.size() && order.workgroups < (long long)seen.size() + 8 * sharing * blocks,
+                           "B %d kv %d sharing %d blocks %d", batch, kv, sharing, blocks);
+                    EXPECT(spread || order.workgroups == (long long)seen.size(), "B %d kv %d sharing %d", batch, kv, sharing);
+                    for (int i = 0; i < (int)order.workgroups; ++i) {
                         const SplitItem item = split_item((unsigned)i, order);
+                        if (item.batch >= batch) continue;
                         EXPECT(item.batch < batch && item.head < kv * sharing && item.query_block >= 0 && item.query_block < blocks &&
                                    item.key_value_head == item.head / sharing, "B %d kv %d sharing %d item %d", batch, kv, sharing, i);
                         ++seen[(item.batch * kv * sharing + item.head) * blocks + item.query_block];
                     }
                     for (int count : seen) EXPECT(count == 1, "B %d kv %d sharing %d blocks %d", batch, kv, sharing, blocks);
+                  }
                 }
             }
         }

@@ -45,6 +45,7 @@ def test_flash_work_orders(cuda, batch, tokens, kv_heads, sharing, dim):
     (3, 64, 128, 128), (4, 192, 96, 32), (24, 128, 16, 16), (2, 192, 128, 16), (1, 320, 224, 56), (1, 384, 256, 64),
     (1, 448, 384, 48), (1, 2112, 256, 2),   # four waves
     (2, 448, 128, 32), (1, 128, 256, 64), (1, 192, 223, 223), (1, 64, 127, 127),   # the other side of the rule
+    (1, 1280, 67, 67), (3, 896, 33, 11), (1, 576, 155, 31),   # heads dealt to the XCDs with slots left over
 ])
 def test_flash_64_columns_many_heads(cuda, batch, tokens, heads, kv_heads):
     q, k, v, scale = configs.flash_forward_inputs(batch, tokens, heads, kv_heads, 64, seed=tokens, factor=0.5)
