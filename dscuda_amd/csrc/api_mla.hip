@@ -85,7 +85,28 @@ void mla_compressed_attention_backward_cuda(
     check_positive("MLA backward", batch_size, sequence_length, heads);
     mla_absorbed_backward_dispatch(query_latent_gradient, query_rope_gradient, kv_latent_gradient, key_rope_gradient,
                                    output_gradient, output, logsumexp, query_latent, query_rope, kv_latent, key_rope,
-                                   batch_size, sequence_length, heads, scale, stream);
+                                   nullptr, 0, batch_size, sequence_length, heads, scale, stream);
+}
+
+std::size_t mla_backward_workspace_elements(int batch_size, int sequence_length, int heads, int kv_rank, int rope_size) {
+    if (batch_size <= 0 || sequence_length <= 0 || heads <= 0 || kv_rank != MLA_KV_RANK || rope_size != MLA_ROPE_SIZE) {
+        return 0;
+    }
+    return mla_absorbed_backward_workspace_bytes(batch_size, sequence_length, heads) / sizeof(float);
+}
+
+void mla_compressed_attention_backward_workspace_cuda(
+    __hip_bfloat16* query_latent_gradient, __hip_bfloat16* query_rope_gradient, __hip_bfloat16* kv_latent_gradient,
+    __hip_bfloat16* key_rope_gradient, const __hip_bfloat16* output_gradient, const __hip_bfloat16* output,
+    const float* logsumexp, const __hip_bfloat16* query_latent, const __hip_bfloat16* query_rope,
+    const __hip_bfloat16* kv_latent, const __hip_bfloat16* key_rope, float* workspace, std::size_t workspace_elements,
+    int batch_size, int sequence_length, int heads, int kv_rank, int rope_size, float scale, hipStream_t stream) {
+    check_shape(kv_rank, rope_size);
+    check_positive("MLA backward", batch_size, sequence_length, heads);
+    mla_absorbed_backward_dispatch(query_latent_gradient, query_rope_gradient, kv_latent_gradient, key_rope_gradient,
+                                   output_gradient, output, logsumexp, query_latent, query_rope, kv_latent, key_rope,
+                                   workspace, workspace_elements * sizeof(float), batch_size, sequence_length, heads,
+                                   scale, stream);
 }
 
 std::size_t mla_decode_workspace_elements(int batch_size, int heads, int splits, int kv_rank) {
@@ -269,6 +290,27 @@ extern "C" int dscuda_mla_backward(__hip_bfloat16* dquery, __hip_bfloat16* dquer
         dscuda::mla_compressed_attention_backward_cuda(dquery, dquery_rope, dlatent, dkey_rope, dout, output, lse,
                                                        query, query_rope, latent, key_rope, batch, sequence, heads,
                                                        rank, rope, scale, stream);
+    });
+}
+
+extern "C" std::size_t dscuda_mla_backward_workspace_elements(int batch, int sequence, int heads, int rank, int rope) {
+    std::size_t elements = 0;
+    guarded([&] { elements = dscuda::mla_backward_workspace_elements(batch, sequence, heads, rank, rope); });
+    return elements;
+}
+
+extern "C" int dscuda_mla_backward_workspace(__hip_bfloat16* dquery, __hip_bfloat16* dquery_rope, __hip_bfloat16* dlatent,
+                                             __hip_bfloat16* dkey_rope, const __hip_bfloat16* dout,
+                                             const __hip_bfloat16* output, const float* lse, const __hip_bfloat16* query,
+                                             const __hip_bfloat16* query_rope, const __hip_bfloat16* latent,
+                                             const __hip_bfloat16* key_rope, float* workspace,
+                                             std::size_t workspace_elements, int batch, int sequence, int heads, int rank,
+                                             int rope, float scale, hipStream_t stream) {
+    return guarded([&] {
+        dscuda::mla_compressed_attention_backward_workspace_cuda(dquery, dquery_rope, dlatent, dkey_rope, dout, output,
+                                                                 lse, query, query_rope, latent, key_rope, workspace,
+                                                                 workspace_elements, batch, sequence, heads, rank, rope,
+                                                                 scale, stream);
     });
 }
 

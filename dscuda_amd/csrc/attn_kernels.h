@@ -69,8 +69,18 @@ void mla_absorbed_backward_dispatch(__hip_bfloat16* query_latent_gradient, __hip
                                     const __hip_bfloat16* output_gradient, const __hip_bfloat16* output,
                                     const float* logsumexp, const __hip_bfloat16* query_latent,
                                     const __hip_bfloat16* query_rope, const __hip_bfloat16* kv_latent,
-                                    const __hip_bfloat16* key_rope, int batch_size, int sequence_length, int heads,
-                                    float scale, hipStream_t stream);
+                                    const __hip_bfloat16* key_rope, void* workspace, std::size_t workspace_bytes,
+                                    int batch_size, int sequence_length, int heads, float scale, hipStream_t stream);
+
+// Bytes of workspace with which the backward keeps dS for its query gradients; 0 where it does not use one.
+std::size_t mla_absorbed_backward_workspace_bytes(int batch_size, int sequence_length, int heads);
+
+// mla_absorbed_product.hip -- the query gradients from the dS blocks the key-gradient launch kept (16-byte aligned,
+// index_math::KeptGradients, key blocks of 32 * key_tiles keys).
+void mla_absorbed_query_product_launch(__hip_bfloat16* query_latent_gradient, __hip_bfloat16* query_rope_gradient,
+                                       const unsigned char* kept_gradients, const __hip_bfloat16* kv_latent,
+                                       const __hip_bfloat16* key_rope, int batch_size, int sequence_length, int heads,
+                                       int key_tiles, hipStream_t stream);
 
 // mla_absorbed_short.hip -- the launches after the row statistics for at most 512 tokens (delta of a row in the first
 // four bytes of its rope query gradient); the query gradients are 16-byte aligned.

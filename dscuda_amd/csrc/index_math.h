@@ -547,6 +547,36 @@ DSCUDA_HOST_DEVICE inline KeyVisits key_visits(int sequence_length, int heads, i
     return visits;
 }
 
+// Where the key-gradient kernels keep dS for the query-gradient product, when they have a workspace: a block of 2 KB
+// per (32-key tile, row tile) that a key block of 32 * key_tiles keys visits, in the order of the visits, so that the
+// blocks of neighbouring row tiles lie one behind the other.  Inside a block key k has bytes 64k .. 64k + 63: bf16 of
+// row 16r + 4q + e at 16q + 8r + 2e, which both sides move as whole 16-byte pieces of consecutive lanes.
+struct KeptGradients {
+    static constexpr int BLOCK_BYTES = 2048;
+    KeyVisits visits;
+    int key_tiles;
+
+    DSCUDA_HOST_DEVICE long long bytes() const { return visits.per_batch() * key_tiles * BLOCK_BYTES; }
+    // first row tile that visits the key block of `tile`
+    DSCUDA_HOST_DEVICE int first_row_tile(int tile) const { return visits.first_tile(tile / key_tiles); }
+    DSCUDA_HOST_DEVICE long long at(int tile, int row_tile) const {
+        const int block = tile / key_tiles;
+        const long long visit = visits.before(block) + row_tile - visits.first_tile(block);
+        return (visit * key_tiles + tile % key_tiles) * BLOCK_BYTES;
+    }
+};
+
+DSCUDA_HOST_DEVICE inline KeptGradients kept_gradients(int sequence_length, int heads, int key_tiles) {
+    return KeptGradients{key_visits(sequence_length, heads, key_tiles), key_tiles};
+}
+
+// Bytes that hold dS of one batch element for key blocks of either size.
+DSCUDA_HOST_DEVICE inline long long kept_gradient_bytes(int sequence_length, int heads) {
+    const long long narrow = kept_gradients(sequence_length, heads, 1).bytes();
+    const long long wide = kept_gradients(sequence_length, heads, 2).bytes();
+    return narrow > wide ? narrow : wide;
+}
+
 DSCUDA_HOST_DEVICE inline long long wide_range_begin(long long total, long long ranges, long long range) {
     return range * total / ranges;
 }
@@ -627,6 +657,55 @@ DSCUDA_HOST_DEVICE inline int key_interval_choice(int sequence_length, int heads
     }
 }
 
+// The same where dS is kept in a workspace, which has room for slots as well: the length whose items take the least
+// time, r rounds of the compute units of `length` + ITEM_OVERHEAD steps each (the keys, the first tile, the partial
+// result and its share of the reduction), over the shortest length whose items number at most r rounds, r = 1 .. 12.
+// Backward in us by rounds 1, 2, 3, 5, 7, 12: 2048 tokens x 128 heads 1786 1721 1744 1791 1862 2116, 4096 x 128 7260 6892
+// 6598 6397 6318 6519, 8000 x 16 3283 2942 2933 2927 2936 3009, 1024 x 128 535 554 594 683 804 1201, which is what the
+// sum predicts to 3 %; the ladder above: 1898, 6471, 605 (1024 x 128).
+// 0: so few visits a unit that ranges of 32-key blocks, which need no whole rounds, are the better cut (ranges / items:
+// 480 x 16 54 / 69, 200 x 32 43 / 65, 226 x 128 77 / 91; 1000 x 4 68 / 69, 4 x 512 x 8 78 / 73, 2 x 592 x 16 95 / 83,
+// 2048 x 4 137 / 117, 2845 x 4 x 3 583 / 385).
+constexpr int ITEM_OVERHEAD = 12;
+constexpr int MOST_ROUNDS = 12;
+constexpr int WORKSPACE_ROUNDS = 3;   // that a workspace has slots for; long inputs have more in the query gradients
+
+DSCUDA_HOST_DEVICE inline int key_interval_fit(int sequence_length, int heads, long long batch, long long slots,
+                                               int compute_units, int key_tiles) {
+    const long long visits = key_visits(sequence_length, heads, key_tiles).per_batch() * batch;
+    if (visits < (heads < 16 ? 5LL : 10LL) * compute_units) return 0;
+    const long long row_tiles = ((long long)sequence_length * heads + 31) / 32;
+    long long best = 0, best_cost = 0;
+    for (int rounds = 1; rounds <= MOST_ROUNDS; ++rounds) {
+        const long long most = (long long)rounds * compute_units < slots ? (long long)rounds * compute_units : slots;
+        long long length = (visits + most - 1) / most;
+        while (length < row_tiles && key_intervals(sequence_length, heads, (int)length, key_tiles).items() * batch > most) {
+            length += 1 + length / 64;
+        }
+        if (length > row_tiles) length = row_tiles;
+        if (length >= (1 << 24)) continue;
+        const long long items = key_intervals(sequence_length, heads, (int)length, key_tiles).items() * batch;
+        const long long cost = (items + compute_units - 1) / compute_units * (length + ITEM_OVERHEAD);
+        if (items <= slots && (best == 0 || cost < best_cost)) {
+            best = length;
+            best_cost = cost;
+        }
+    }
+    return (int)best;
+}
+
+// Bytes of slots a workspace should have room for, `batch` elements taken together: the items of WORKSPACE_ROUNDS rounds
+// of the 256 compute units, or a range per unit and the blocks that ranges may share.
+DSCUDA_HOST_DEVICE inline long long workspace_slot_bytes(int sequence_length, int heads, long long batch) {
+    constexpr long long UNITS = 256;
+    const KeyVisits narrow = key_visits(sequence_length, heads, 1);
+    const long long pair_visits = key_visits(sequence_length, heads, 2).per_batch() * batch;
+    const long long items = pair_visits < WORKSPACE_ROUNDS * UNITS ? pair_visits : WORKSPACE_ROUNDS * UNITS;
+    const long long visits = narrow.per_batch() * batch / 2;
+    const long long ranges = (visits < UNITS ? visits : UNITS) + narrow.key_blocks * batch;
+    return (2 * items > ranges ? 2 * items : ranges) * KEY_PARTIAL_BYTES;
+}
+
 // How many ranges the list is cut into when `scratch_bytes` are there for the slots: one per compute unit if the
 // slots allow.  0: every key block is one range and writes its result itself (too few slots for a cut whose
 // longest range is shorter than the longest key block, `row_tiles` visits).
@@ -665,6 +744,13 @@ DSCUDA_HOST_DEVICE inline bool short_backward(long long batch, int tokens, int h
     if (batch > (rows < 64 ? 12 : heads == 1 ? 16 : 32)) return false;
     if (heads <= 3) return batch * ((tokens + 31) / 32) <= 110;
     return heads < 16 || rows * batch * tokens <= (heads <= 20 ? 2000000 : 1600000);
+}
+
+// Which of them still do where a workspace could hold dS and the slots of ranges: one launch less, but key gradients that
+// read 64 bytes a row. Backward, P and dS kept / ranges (us): 300 x 4 30 / 32, 512 x 4 40 / 46, 250 x 8 33 / 38, 512 x 8 50 / 50;
+// 128 x 16 28 / 28, 64 x 32 28 / 25, 350 x 16 54 / 46, 480 x 16 77 / 54, 3 x 500 x 4 62 / 54, 8 x 338 x 3 63 / 49, 32 x 64 x 4 34 / 30.
+DSCUDA_HOST_DEVICE inline bool short_without_workspace(long long batch, int tokens, int heads) {
+    return heads < 16 && (long long)tokens * heads * batch <= 4096;
 }
 
 DSCUDA_HOST_DEVICE inline bool kept_in_rope(int token_block, int blocks) { return token_block == blocks - 1; }

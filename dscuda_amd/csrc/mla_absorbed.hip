@@ -39,6 +39,10 @@
 //                     token of those rows.  Every wave forms one quadrant of S^T and
 //                     dP^T of the tile, the quadrants of dS^T meet in LDS, and every
 //                     wave accumulates dQ^T for its own share of the 18 column blocks.
+// With a workspace the score waves of the key gradients keep dS there, and the query gradients are the product
+// dS [latent|rope] alone (mla_absorbed_product.hip); it also has slots for partial key gradients, so that calls whose
+// query gradients have room for few of them occupy the chip as well (4096 tokens x 4 heads: backward 638 -> 284 us with
+// both, 600 x 4 130 -> 49, 2048 x 128 2236 -> 1733).
 // Short sequences with few rows (index_math::short_backward), whose query-gradient buffers have room for few partial
 // results, take three other launches after the row statistics (mla_absorbed_short.hip).
 #include "attn_kernels.h"
@@ -556,6 +560,15 @@ __global__ __launch_bounds__(QUERY_THREADS) void mla_absorbed_query_gradient_ker
 
 // ---- key gradients -------------------------------------------------------------
 
+using index_math::KeptGradients;
+
+// The wave's tile requests have arrived; the two stores of dS that follow them in a wave that `keeps` it may still be
+// on their way (a store counts until it has reached the L2, which a step would otherwise wait for).
+__device__ __forceinline__ void wait_for_requests(bool keeps) {
+    asm volatile("" ::: "memory");   // the stores are issued before the wait
+    if (keeps) wait_vector_memory<2>(); else wait_vector_memory<0>();
+}
+
 struct KeyGradLayout {
     static constexpr int Q_LATENT = 0;                                   // [32 rows][512]
     static constexpr int DO_ROWS = Q_LATENT + Tile32<RANK>::BYTES;       // [32 rows][512]
@@ -596,8 +609,8 @@ __device__ __forceinline__ void key_gradient_walk(
     bf16_t* __restrict__ kv_latent_gradient, bf16_t* __restrict__ key_rope_gradient, float* __restrict__ partial_slots,
     const float* __restrict__ delta_of_rows, const bf16_t* __restrict__ output_gradient,
     const float* __restrict__ logsumexp, const bf16_t* __restrict__ query_latent, const bf16_t* __restrict__ query_rope,
-    const bf16_t* __restrict__ kv_latent, const bf16_t* __restrict__ key_rope, int batch_size, int sequence_length,
-    int heads, int ranges, int interval_length, float scale) {
+    const bf16_t* __restrict__ kv_latent, const bf16_t* __restrict__ key_rope, unsigned char* __restrict__ kept_gradients,
+    int batch_size, int sequence_length, int heads, int ranges, int interval_length, float scale) {
     using L = KeyGradLayout;
     using Wide = Tile32<RANK>;             // the latent query rows and the dO rows
     using Narrow = Tile32<ROPE>;           // the rope query rows
@@ -683,6 +696,7 @@ __device__ __forceinline__ void key_gradient_walk(
         const bf16_t* latent = kv_latent + (size_t)batch * T * RANK;
         const bf16_t* rope = key_rope + (size_t)batch * T * ROPE;
         const float* lse_batch = logsumexp + (size_t)batch * heads * T;
+        unsigned char* kept_segment = kept_gradients == nullptr ? nullptr : kept_gradients + position * KeptGradients::BLOCK_BYTES;
 
         // score waves: the keys as B operands (column = key 16*kh + l16); the value operand is the latent part
         bf16x8 kf[2][Q_STEPS];
@@ -778,7 +792,7 @@ __device__ __forceinline__ void key_gradient_walk(
 
         // scores of one tile: (rows x keys) quadrants of 16 x 16, lane holds key 16*kh + l16 and rows 4*quad .. +3 of
         // the wave's 16; the score and dP products take turns, every row fragment serves both key halves
-        auto score_tile = [&](const unsigned char* buffer, unsigned char* exchange) {
+        auto score_tile = [&](const unsigned char* buffer, unsigned char* exchange, unsigned char* kept) {
             const unsigned char* q_latent = buffer + L::Q_LATENT;
             const unsigned char* q_rope = buffer + L::Q_ROPE;
             const unsigned char* do_rows = buffer + L::DO_ROWS;
@@ -830,6 +844,10 @@ __device__ __forceinline__ void key_gradient_walk(
                 }
                 exchange_store(exchange, 16 * kh + l16, local, p);     // [key][row]
                 exchange_store(exchange + EXCHANGE_BYTES, 16 * kh + l16, local, ds);
+                if (kept != nullptr) {
+                    *reinterpret_cast<u32x2*>(kept + 64 * (16 * kh + l16) + 16 * quad + 8 * half) =
+                        u32x2{pack_bf16(ds[0], ds[1]), pack_bf16(ds[2], ds[3])};
+                }
             }
         };
 
@@ -887,13 +905,15 @@ __device__ __forceinline__ void key_gradient_walk(
             begin_requests(more ? tile + 1 : end_tile - 1, parity ^ 1);
             if constexpr (SCORES) {
                 if (tile < end_tile) {
-                    score_tile(lds + parity * L::BUFFER_BYTES, lds + L::EXCHANGE + parity * L::EXCHANGE_PAIR);
+                    score_tile(lds + parity * L::BUFFER_BYTES, lds + L::EXCHANGE + parity * L::EXCHANGE_PAIR,
+                               kept_segment == nullptr ? nullptr
+                                                       : kept_segment + (size_t)(tile - first_tile) * KeptGradients::BLOCK_BYTES);
                 }
             } else {
                 add_tile(lds + parity * L::BUFFER_BYTES, lds + L::EXCHANGE + (parity ^ 1) * L::EXCHANGE_PAIR,
                          tile > first_tile);
             }
-            wait_vector_memory<0>();
+            wait_for_requests(SCORES && kept_segment != nullptr);
             place_statistics(parity ^ 1);
             workgroup_barrier();   // tile t has been read, P and dS of it and tile t + 1 are in place
         }
@@ -935,16 +955,16 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_key_gradient_kernel(
     bf16_t* __restrict__ kv_latent_gradient, bf16_t* __restrict__ key_rope_gradient, float* __restrict__ partial_slots,
     const float* __restrict__ delta_of_rows, const bf16_t* __restrict__ output_gradient,
     const float* __restrict__ logsumexp, const bf16_t* __restrict__ query_latent, const bf16_t* __restrict__ query_rope,
-    const bf16_t* __restrict__ kv_latent, const bf16_t* __restrict__ key_rope, int batch_size, int sequence_length,
-    int heads, int ranges, int interval_length, float scale) {
+    const bf16_t* __restrict__ kv_latent, const bf16_t* __restrict__ key_rope, unsigned char* __restrict__ kept_gradients,
+    int batch_size, int sequence_length, int heads, int ranges, int interval_length, float scale) {
     if (threadIdx.x < THREADS / 2) {
         key_gradient_walk<true>(kv_latent_gradient, key_rope_gradient, partial_slots, delta_of_rows, output_gradient,
-                                logsumexp, query_latent, query_rope, kv_latent, key_rope, batch_size, sequence_length,
-                                heads, ranges, interval_length, scale);
+                                logsumexp, query_latent, query_rope, kv_latent, key_rope, kept_gradients, batch_size,
+                                sequence_length, heads, ranges, interval_length, scale);
     } else {
         key_gradient_walk<false>(kv_latent_gradient, key_rope_gradient, partial_slots, delta_of_rows, output_gradient,
-                                 logsumexp, query_latent, query_rope, kv_latent, key_rope, batch_size, sequence_length,
-                                 heads, ranges, interval_length, scale);
+                                 logsumexp, query_latent, query_rope, kv_latent, key_rope, kept_gradients, batch_size,
+                                 sequence_length, heads, ranges, interval_length, scale);
     }
 }
 
@@ -980,8 +1000,8 @@ __device__ __forceinline__ void key_pair_walk(
     bf16_t* __restrict__ kv_latent_gradient, bf16_t* __restrict__ key_rope_gradient, float* __restrict__ partial_slots,
     const float* __restrict__ delta_of_rows, const bf16_t* __restrict__ output_gradient,
     const float* __restrict__ logsumexp, const bf16_t* __restrict__ query_latent, const bf16_t* __restrict__ query_rope,
-    const bf16_t* __restrict__ kv_latent, const bf16_t* __restrict__ key_rope, int sequence_length, int heads,
-    int interval_length, float scale) {
+    const bf16_t* __restrict__ kv_latent, const bf16_t* __restrict__ key_rope, unsigned char* __restrict__ kept_gradients,
+    int sequence_length, int heads, int interval_length, float scale) {
     using L = KeyPairLayout;
     using Wide = Tile32<RANK>;
     using Narrow = Tile32<ROPE>;
@@ -1042,6 +1062,12 @@ __device__ __forceinline__ void key_pair_walk(
     const bf16_t* latent = kv_latent + (size_t)batch * T * RANK;
     const bf16_t* rope = key_rope + (size_t)batch * T * ROPE;
     const float* lse_batch = logsumexp + (size_t)batch * heads * T;
+
+    // dS of the wave's keys and the item's first row tile, if it is kept
+    unsigned char* kept_item = kept_gradients == nullptr
+        ? nullptr
+        : kept_gradients + ((batch * visits.per_batch() + visits.before(key_block) + first_tile - visits.first_tile(key_block)) * KEY_TILES +
+                            half) * KeptGradients::BLOCK_BYTES;
 
     // score waves: the wave's 32 keys as B operands (column = key 32*half + 16*kh + l16), and their rope sums
     bf16x8 kf[2][Q_STEPS];
@@ -1133,7 +1159,7 @@ __device__ __forceinline__ void key_pair_walk(
 
     // scores of one tile: (rows x keys) blocks of 16 x 16, lane holds key 32*half + 16*kh + l16 and rows 16*r + 4*quad .. +3;
     // the two halves of the rows one after the other, every row fragment serves both key blocks
-    auto score_tile = [&](const unsigned char* buffer, unsigned char* exchange) {
+    auto score_tile = [&](const unsigned char* buffer, unsigned char* exchange, unsigned char* kept) {
         const unsigned char* q_latent = buffer + L::Q_LATENT;
         const unsigned char* q_rope = buffer + L::Q_ROPE;
         const unsigned char* do_rows = buffer + L::DO_ROWS;
@@ -1184,6 +1210,7 @@ __device__ __forceinline__ void key_pair_walk(
                 rope_columns_of_rows[n][b] = transposed_fragment(q_rope, rope_columns.low[b], rope_columns.high[b], n * 16 * Narrow::ROW);
             }
         }
+        u32x2 packed_gradients[2][2];   // [key block][half of the rows]
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
             const int local = 16 * r + 4 * quad;
@@ -1204,6 +1231,7 @@ __device__ __forceinline__ void key_pair_walk(
                 // [key][row], the wave's 32 keys are one part of EXCHANGE_BYTES
                 exchange_store(exchange + half * EXCHANGE_BYTES, 16 * kh + l16, local, p);
                 exchange_store(exchange + L::EXCHANGE_PART + half * EXCHANGE_BYTES, 16 * kh + l16, local, ds);
+                packed_gradients[kh][r] = u32x2{pack_bf16(ds[0], ds[1]), pack_bf16(ds[2], ds[3])};
             }
         }
         // dK_rope += dS^T Q_rope for the wave's keys: their dS of all 32 rows were written by this wave
@@ -1213,6 +1241,14 @@ __device__ __forceinline__ void key_pair_walk(
 #pragma unroll
             for (int b = 0; b < ROPE / 32; ++b) {
                 rope_acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gradient, rope_columns_of_rows[n][b], rope_acc[b], 0, 0, 0);
+            }
+        }
+        if (kept != nullptr) {
+#pragma unroll
+            for (int kh = 0; kh < 2; ++kh) {
+                __builtin_nontemporal_store(u32x4{packed_gradients[kh][0].x, packed_gradients[kh][0].y, packed_gradients[kh][1].x,
+                                                  packed_gradients[kh][1].y},
+                                            reinterpret_cast<u32x4*>(kept + 1024 * kh + 16 * (4 * l16 + quad)));
             }
         }
     };
@@ -1275,12 +1311,14 @@ __device__ __forceinline__ void key_pair_walk(
         begin_requests(more ? tile + 1 : end_tile - 1, parity ^ 1);
         if constexpr (SCORES) {
             if (tile < end_tile) {
-                score_tile(lds + parity * L::BUFFER_BYTES, lds + L::EXCHANGE + parity * L::EXCHANGE_PAIR);
+                score_tile(lds + parity * L::BUFFER_BYTES, lds + L::EXCHANGE + parity * L::EXCHANGE_PAIR,
+                           kept_item == nullptr ? nullptr
+                                                : kept_item + (size_t)(tile - first_tile) * (KEY_TILES * KeptGradients::BLOCK_BYTES));
             }
         } else {
             add_tile(lds + parity * L::BUFFER_BYTES, lds + L::EXCHANGE + (parity ^ 1) * L::EXCHANGE_PAIR, tile > first_tile);
         }
-        wait_vector_memory<0>();
+        wait_for_requests(SCORES && kept_item != nullptr);
         place_statistics(parity ^ 1);
         workgroup_barrier();   // tile t has been read, P and dS of it and tile t + 1 are in place
     }
@@ -1332,14 +1370,16 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_key_pair_gradient_kernel
     bf16_t* __restrict__ kv_latent_gradient, bf16_t* __restrict__ key_rope_gradient, float* __restrict__ partial_slots,
     const float* __restrict__ delta_of_rows, const bf16_t* __restrict__ output_gradient,
     const float* __restrict__ logsumexp, const bf16_t* __restrict__ query_latent, const bf16_t* __restrict__ query_rope,
-    const bf16_t* __restrict__ kv_latent, const bf16_t* __restrict__ key_rope, int sequence_length, int heads,
-    int interval_length, float scale) {
+    const bf16_t* __restrict__ kv_latent, const bf16_t* __restrict__ key_rope, unsigned char* __restrict__ kept_gradients,
+    int sequence_length, int heads, int interval_length, float scale) {
     if (threadIdx.x < THREADS / 2) {
         key_pair_walk<true>(kv_latent_gradient, key_rope_gradient, partial_slots, delta_of_rows, output_gradient, logsumexp,
-                                 query_latent, query_rope, kv_latent, key_rope, sequence_length, heads, interval_length, scale);
+                       query_latent, query_rope, kv_latent, key_rope, kept_gradients, sequence_length, heads,
+                       interval_length, scale);
     } else {
         key_pair_walk<false>(kv_latent_gradient, key_rope_gradient, partial_slots, delta_of_rows, output_gradient, logsumexp,
-                                  query_latent, query_rope, kv_latent, key_rope, sequence_length, heads, interval_length, scale);
+                        query_latent, query_rope, kv_latent, key_rope, kept_gradients, sequence_length, heads,
+                        interval_length, scale);
     }
 }
 
@@ -1435,6 +1475,8 @@ void raise_lds_limit(Kernel kernel, int bytes) {
 
 constexpr long long LARGE_INPUT_BYTES = 64LL << 20;   // per batch element, against 32 MB of L2 and 256 MB behind it
 
+constexpr long long KEPT_BYTES_LIMIT = 4LL << 30;     // of dS in a workspace: 4096 tokens of 128 heads take 2.2 GB
+
 // mla_absorbed_backward_set_key_interval_tiles (> 0) forces the interval cut with that many row tiles per interval at
 // any size the slots allow; 0 gives the choice back to the dispatch below.
 std::atomic<int> forced_key_interval_tiles{0};
@@ -1453,34 +1495,29 @@ void mla_absorbed_backward_set_key_interval_tiles(int tiles) {
     forced_key_interval_tiles.store(tiles > 0 && tiles < (1 << 24) ? tiles : 0, std::memory_order_relaxed);
 }
 
-void mla_absorbed_backward_dispatch(bf16_t* query_latent_gradient, bf16_t* query_rope_gradient,
+namespace {
+
+// The whole batch, or as many batch elements as `kept_gradients` has room for (nullptr: dS is not kept).
+void backward_of_batch(bf16_t* query_latent_gradient, bf16_t* query_rope_gradient,
                                     bf16_t* kv_latent_gradient, bf16_t* key_rope_gradient,
                                     const bf16_t* output_gradient, const bf16_t* output, const float* logsumexp,
                                     const bf16_t* query_latent, const bf16_t* query_rope, const bf16_t* kv_latent,
-                                    const bf16_t* key_rope, int batch_size, int sequence_length, int heads, float scale,
-                                    hipStream_t stream) {
+                                    const bf16_t* key_rope, unsigned char* kept_gradients, float* partial_slots,
+                                    long long scratch_bytes, int batch_size, int sequence_length, int heads,
+                                    float scale, hipStream_t stream) {
     const long long rows = (long long)sequence_length * heads;
     const long long row_blocks = (rows + TILE - 1) / TILE;
-    if (row_blocks * batch_size > 0x7fffffffLL) {
-        throw std::invalid_argument("MLA backward: batch*tokens*heads exceeds the grid limit");
-    }
-    if (reinterpret_cast<uintptr_t>(query_latent_gradient) % 16 != 0 ||
-        reinterpret_cast<uintptr_t>(query_rope_gradient) % 16 != 0) {
-        throw std::invalid_argument("MLA backward: the query gradients must be aligned to 16 bytes");
-    }
     static hip_common::OncePerDevice prepared;
     prepared.run([] {
         raise_lds_limit(mla_absorbed_query_gradient_kernel, QueryGradLayout::LDS_BYTES);
         raise_lds_limit(mla_absorbed_key_gradient_kernel, KeyGradLayout::LDS_BYTES);
         raise_lds_limit(mla_absorbed_key_pair_gradient_kernel, KeyPairLayout::LDS_BYTES);
     });
-    // scratch memory until the last launch: delta in the rope query gradients, partial key gradients in the latent ones
+    // scratch memory until the last launch: delta in the rope query gradients
     float* delta = reinterpret_cast<float*>(query_rope_gradient);
-    float* partial_slots = reinterpret_cast<float*>(query_latent_gradient);
     const index_math::KeyVisits visits = index_math::key_visits(sequence_length, heads);
     long long blocks = (long long)visits.key_blocks * batch_size;
     const long long total = visits.per_batch() * batch_size;
-    const long long scratch_bytes = rows * batch_size * RANK * 2;
     // Rows that outgrow the caches (query and dO rows of a batch element, 2176 bytes per row): the interval cut
     // with key blocks of 64 keys (mla_absorbed_key_pair_gradient_kernel)
     constexpr int PAIR = KeyPairLayout::KEYS / TILE;
@@ -1488,20 +1525,23 @@ void mla_absorbed_backward_dispatch(bf16_t* query_latent_gradient, bf16_t* query
     int key_tiles = 1;
     long long grid = 0;
     const int forced = forced_interval_tiles();
-    if (forced > 0 || rows * (2 * RANK + ROPE) * 2 > LARGE_INPUT_BYTES) {
+    const bool keeps = kept_gradients != nullptr;
+    const int units = device_compute_units();
+    if (forced > 0 || keeps || rows * (2 * RANK + ROPE) * 2 > LARGE_INPUT_BYTES) {
         const long long slots = scratch_bytes / (PAIR * index_math::KEY_PARTIAL_BYTES);
         // (the choice walks the intervals of several lengths: remembered for the shape a thread asked about last)
         struct Choice {
             int sequence_length = -1, heads = -1, batch_size = -1, units = -1, forced = -1, tiles = 0;
-            long long items = 0;
+            bool keeps = false;
+            long long slots = 0, items = 0;
             int key_blocks = 0;
         };
         static thread_local Choice last;
-        const int units = device_compute_units();
         if (last.sequence_length != sequence_length || last.heads != heads || last.batch_size != batch_size ||
-            last.units != units || last.forced != forced) {
-            last = Choice{sequence_length, heads, batch_size, units, forced, 0, 0, 0};
+            last.units != units || last.forced != forced || last.keeps != keeps || last.slots != slots) {
+            last = Choice{sequence_length, heads, batch_size, units, forced, 0, keeps, slots, 0, 0};
             last.tiles = forced > 0 ? forced
+                         : keeps    ? index_math::key_interval_fit(sequence_length, heads, batch_size, slots, units, PAIR)
                                     : index_math::key_interval_choice(sequence_length, heads, batch_size, slots, units, PAIR);
             if (last.tiles > 0) {
                 const index_math::KeyIntervals chosen = index_math::key_intervals(sequence_length, heads, last.tiles, PAIR);
@@ -1528,7 +1568,7 @@ void mla_absorbed_backward_dispatch(bf16_t* query_latent_gradient, bf16_t* query
     hipLaunchKernelGGL(mla_absorbed_row_statistics_kernel, dim3((unsigned)(row_blocks * batch_size)), dim3(THREADS), 0,
                        stream, delta, output_gradient, output, rows * batch_size);
     HIP_CHECK(hipGetLastError());
-    if (forced == 0 && index_math::short_backward(batch_size, sequence_length, heads)) {
+    if (forced == 0 && !keeps && index_math::short_backward(batch_size, sequence_length, heads)) {
         mla_absorbed_short_backward_launch(query_latent_gradient, query_rope_gradient, kv_latent_gradient, key_rope_gradient,
                                            output_gradient, logsumexp, query_latent, query_rope, kv_latent, key_rope,
                                            batch_size, sequence_length, heads, scale, stream);
@@ -1537,13 +1577,13 @@ void mla_absorbed_backward_dispatch(bf16_t* query_latent_gradient, bf16_t* query
     if (interval_length > 0) {
         hipLaunchKernelGGL(mla_absorbed_key_pair_gradient_kernel, dim3((unsigned)grid), dim3(THREADS),
                            KeyPairLayout::LDS_BYTES, stream, kv_latent_gradient, key_rope_gradient, partial_slots, delta,
-                           output_gradient, logsumexp, query_latent, query_rope, kv_latent, key_rope, sequence_length,
-                           heads, interval_length, scale);
+                           output_gradient, logsumexp, query_latent, query_rope, kv_latent, key_rope, kept_gradients,
+                           sequence_length, heads, interval_length, scale);
     } else {
         hipLaunchKernelGGL(mla_absorbed_key_gradient_kernel, dim3((unsigned)grid), dim3(THREADS), KeyGradLayout::LDS_BYTES,
                            stream, kv_latent_gradient, key_rope_gradient, partial_slots, delta, output_gradient, logsumexp,
-                           query_latent, query_rope, kv_latent, key_rope, batch_size, sequence_length, heads, (int)ranges,
-                           0, scale);
+                           query_latent, query_rope, kv_latent, key_rope, kept_gradients, batch_size, sequence_length, heads,
+                           (int)ranges, 0, scale);
     }
     HIP_CHECK(hipGetLastError());
     if (ranges > 0 || interval_length > 0) {
@@ -1552,12 +1592,74 @@ void mla_absorbed_backward_dispatch(bf16_t* query_latent_gradient, bf16_t* query
                            heads, batch_size, (int)ranges, interval_length, key_tiles);
         HIP_CHECK(hipGetLastError());
     }
+    if (kept_gradients != nullptr) {
+        mla_absorbed_query_product_launch(query_latent_gradient, query_rope_gradient, kept_gradients, kv_latent, key_rope,
+                                          batch_size, sequence_length, heads, key_tiles, stream);
+        return;
+    }
     const long long query_blocks = (rows + QUERY_ROWS - 1) / QUERY_ROWS;
     hipLaunchKernelGGL(mla_absorbed_query_gradient_kernel, dim3((unsigned)(query_blocks * batch_size)), dim3(QUERY_THREADS),
                        QueryGradLayout::LDS_BYTES, stream, query_latent_gradient, query_rope_gradient, delta,
                        output_gradient, logsumexp, query_latent, query_rope, kv_latent, key_rope, sequence_length, heads,
                        (int)query_blocks, scale);
     HIP_CHECK(hipGetLastError());
+}
+
+}  // namespace
+
+std::size_t mla_absorbed_backward_workspace_bytes(int batch_size, int sequence_length, int heads) {
+    if (index_math::short_backward(batch_size, sequence_length, heads) &&
+        index_math::short_without_workspace(batch_size, sequence_length, heads)) {
+        return 0;
+    }
+    const long long element = index_math::kept_gradient_bytes(sequence_length, heads);
+    if (element > KEPT_BYTES_LIMIT) return 0;
+    const long long group = std::min<long long>(batch_size, KEPT_BYTES_LIMIT / element);
+    return (std::size_t)(element * group + index_math::workspace_slot_bytes(sequence_length, heads, group));
+}
+
+void mla_absorbed_backward_dispatch(bf16_t* query_latent_gradient, bf16_t* query_rope_gradient,
+                                    bf16_t* kv_latent_gradient, bf16_t* key_rope_gradient,
+                                    const bf16_t* output_gradient, const bf16_t* output, const float* logsumexp,
+                                    const bf16_t* query_latent, const bf16_t* query_rope, const bf16_t* kv_latent,
+                                    const bf16_t* key_rope, void* workspace, std::size_t workspace_bytes, int batch_size,
+                                    int sequence_length, int heads, float scale, hipStream_t stream) {
+    const long long rows = (long long)sequence_length * heads;
+    const long long row_blocks = (rows + TILE - 1) / TILE;
+    if (row_blocks * batch_size > 0x7fffffffLL) {
+        throw std::invalid_argument("MLA backward: batch*tokens*heads exceeds the grid limit");
+    }
+    if (reinterpret_cast<uintptr_t>(query_latent_gradient) % 16 != 0 ||
+        reinterpret_cast<uintptr_t>(query_rope_gradient) % 16 != 0) {
+        throw std::invalid_argument("MLA backward: the query gradients must be aligned to 16 bytes");
+    }
+    // batch elements whose dS the workspace holds
+    long long group = 0;
+    if (workspace != nullptr && mla_absorbed_backward_workspace_bytes(batch_size, sequence_length, heads) > 0) {
+        if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0) {
+            throw std::invalid_argument("MLA backward: the workspace must be aligned to 16 bytes");
+        }
+        group = std::min<long long>(batch_size, (long long)workspace_bytes / index_math::kept_gradient_bytes(sequence_length, heads));
+    }
+    unsigned char* kept = group > 0 ? static_cast<unsigned char*>(workspace) : nullptr;
+    if (group == 0) group = batch_size;
+    // partial key gradients: behind dS where there is more room than in the latent query gradients
+    const long long left = kept != nullptr ? (long long)workspace_bytes - group * index_math::kept_gradient_bytes(sequence_length, heads) : 0;
+    for (long long first = 0; first < batch_size; first += group) {
+        const long long row = first * rows;
+        const long long elements = std::min<long long>(group, batch_size - first);
+        long long scratch_bytes = elements * rows * RANK * 2;
+        float* partial_slots = reinterpret_cast<float*>(query_latent_gradient + row * RANK);
+        if (left > scratch_bytes) {
+            scratch_bytes = left;
+            partial_slots = reinterpret_cast<float*>(kept + group * index_math::kept_gradient_bytes(sequence_length, heads));
+        }
+        const long long token = first * sequence_length;
+        backward_of_batch(query_latent_gradient + row * RANK, query_rope_gradient + row * ROPE, kv_latent_gradient + token * RANK,
+                          key_rope_gradient + token * ROPE, output_gradient + row * RANK, output + row * RANK, logsumexp + row,
+                          query_latent + row * RANK, query_rope + row * ROPE, kv_latent + token * RANK, key_rope + token * ROPE,
+                          kept, partial_slots, scratch_bytes, (int)elements, sequence_length, heads, scale, stream);
+    }
 }
 
 }  // namespace dscuda

@@ -1,0 +1,247 @@
+// Query gradients of the absorbed MLA backward from dS that the key-gradient launch has kept:
+// dQ [rows, 576] = dS [rows, keys] [latent | rope], a plain causal product.
+//
+// mla_absorbed_query_gradient_kernel (mla_absorbed.hip) forms the scores and dP a second time, 1088 of its 1664
+// multiplications per (row, key) pair; with dS in memory (index_math::KeptGradients, T * rows bytes and a little)
+// this launch carries the other 576 and reads two bytes a pair instead.
+//
+// 2048 tokens x 128 heads: 815 us of query gradients there, 358 here, for 77 us more in the key gradients, whose score
+// waves store the 0.55 GB (1236 -> 1313); 2 x 592 x 16 35 -> 24.
+//
+// A workgroup of eight waves owns 64 * GROUP rows and walks the 32-key tiles they see, all of them through LDS stages
+// of [32 keys][512] + [32 keys][64] + dS.  Wave (r, v) = (w / 4, w % 4): row tiles GROUP * r .., latent column blocks
+// 4v .. 4v + 3 of each of them and one of the rope blocks.  Bound by the key tiles a compute unit draws from its L2
+// (36 KB a step, some 21 bytes a cycle against 1152 matrix cycles at GROUP = 2), hence 128 rows wherever that leaves
+// workgroups enough; 192 rows need more registers than there are.
+#include "attn_kernels.h"
+#include "hip_common.h"
+#include "index_math.h"
+#include "lds_tiles.h"
+
+#include <cstdint>
+
+namespace dscuda {
+namespace {
+
+constexpr int RANK = 512;
+constexpr int ROPE = 64;
+constexpr int TILE = 32;
+constexpr int THREADS = 512;
+
+template <int GROUP>
+struct ProductLayout {
+    static constexpr int ROWS = 64 * GROUP;
+    static constexpr int ROW_TILES = 2 * GROUP;
+    static constexpr int WIDE_ROW = 2 * RANK;
+    static constexpr int NARROW_ROW = 2 * ROPE;
+    static constexpr int ROPE_AT = TILE * WIDE_ROW;
+    static constexpr int DS_AT = ROPE_AT + TILE * NARROW_ROW;
+    static constexpr int STAGE_BYTES = DS_AT + ROW_TILES * index_math::KeptGradients::BLOCK_BYTES;
+    static constexpr int STAGES = GROUP == 1 ? 4 : 3;
+    static constexpr int OUT_PITCH = 2 * (RANK + ROPE) + 16;   // of a staged gradient row
+    static constexpr int OUT_BYTES = ROWS * OUT_PITCH;
+    static constexpr int LDS_BYTES = STAGES * STAGE_BYTES > OUT_BYTES ? STAGES * STAGE_BYTES : OUT_BYTES;
+    static_assert(LDS_BYTES <= 160 * 1024, "LDS of a compute unit");
+};
+
+template <int GROUP>
+__global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
+    bf16_t* __restrict__ query_latent_gradient, bf16_t* __restrict__ query_rope_gradient,
+    const unsigned char* __restrict__ kept_gradients, const bf16_t* __restrict__ kv_latent,
+    const bf16_t* __restrict__ key_rope, int batch_size, int sequence_length, int heads, int key_tiles, int row_blocks) {
+    using L = ProductLayout<GROUP>;
+    using Wide = index_math::TileReadMath<L::WIDE_ROW>;
+    using Narrow = index_math::TileReadMath<L::NARROW_ROW>;
+    constexpr int LATENT_BLOCKS = RANK / TILE / 4;   // 32-column blocks of a wave
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int lane = tid % 64;
+    const int lq = lane % 32;
+    const int g = lane / 32;
+    const int T = sequence_length;
+    const long long rows = (long long)T * heads;
+    const int batch = blockIdx.x % batch_size;
+    const int row_block = row_blocks - 1 - blockIdx.x / batch_size;   // latest rows (most keys) first
+    const long long row0 = (long long)row_block * L::ROWS;
+    const long long batch_row0 = (long long)batch * rows;
+    const unsigned char* latent = reinterpret_cast<const unsigned char*>(kv_latent + (size_t)batch * T * RANK);
+    const unsigned char* rope = reinterpret_cast<const unsigned char*>(key_rope + (size_t)batch * T * ROPE);
+    const int tiles = (int)((min(row0 + L::ROWS, rows) - 1) / heads) / TILE + 1;   // key tiles the rows see
+    const index_math::KeptGradients kept = index_math::kept_gradients(T, heads, key_tiles);
+    const unsigned char* kept_batch = kept_gradients + (size_t)batch * kept.bytes();
+    const int first_row_tile = row_block * L::ROW_TILES;
+
+    const int v = wave % 4;
+    const int wave_row_tile = GROUP * (wave / 4);   // of the workgroup's
+    const int rope_tile = GROUP == 1 ? 0 : v / 2;   // whose rope block v % 2 the wave sums; GROUP = 1: waves v < 2 only
+    const int rope_block = v % 2;
+
+    // A wave requests key rows 4*wave .. +3 of the wide tile, waves 0 .. 3 also eight rows of the narrow one, and 1 KB,
+    // half a row tile, of dS: every wave at GROUP = 2, waves 4 .. 7 at GROUP = 1.  Keys past the end repeat the last
+    // one (their dS is zero), row tiles past the end repeat the last one (their results are not stored), and a tile
+    // that does not see the keys yet reads what precedes its blocks and is left out below.
+    const unsigned lds_base = lds_offset_of(lds);
+    const int ds_part = GROUP == 1 ? wave - 4 : wave;
+    const int ds_row_tile = min(first_row_tile + max(ds_part, 0) / 2, kept.visits.row_tiles - 1);
+    auto request_tile = [&](int tile) {
+        const unsigned target = lds_base + tile % L::STAGES * L::STAGE_BYTES;
+        const int last = min(T - tile * TILE, TILE) - 1;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int key = 4 * wave + j;
+            direct_load_16_offset(latent + (size_t)tile * TILE * L::WIDE_ROW,
+                                  (unsigned)(min(key, last) * L::WIDE_ROW + 16 * (lane ^ index_math::tile_swizzle<L::WIDE_ROW>(key))),
+                                  target + key * L::WIDE_ROW);
+        }
+        if (wave < 4) {
+            const int key = 8 * wave + lane / 8;
+            direct_load_16_offset(rope + (size_t)tile * TILE * L::NARROW_ROW,
+                                  (unsigned)(min(key, last) * L::NARROW_ROW +
+                                             16 * ((lane % 8) ^ index_math::tile_swizzle<L::NARROW_ROW>(key))),
+                                  target + L::ROPE_AT + 8 * wave * L::NARROW_ROW);
+        }
+        if (GROUP > 1 || wave >= 4) {
+            direct_load_16_offset_streaming(kept_batch + kept.at(tile, ds_row_tile) + 1024 * (ds_part % 2), 16u * (unsigned)lane,
+                                            target + L::DS_AT + 1024 * ds_part);
+        }
+    };
+    // all but the newest `tiles_in_flight` tiles of the wave's requests have arrived
+    auto wait_for_all_but = [&](auto tiles_in_flight) {
+        constexpr int N = decltype(tiles_in_flight)::value;
+        if (GROUP > 1 && wave < 4) wait_vector_memory<6 * N>(); else wait_vector_memory<5 * N>();
+    };
+    constexpr int AHEAD = L::STAGES - 1;
+    for (int tile = 0; tile < min(tiles, AHEAD); ++tile) request_tile(tile);
+
+    unsigned wide_at[2][LATENT_BLOCKS], narrow_at[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int j = 0; j < LATENT_BLOCKS; ++j) wide_at[h][j] = Wide::transposed(h, j, lane) + 256 * v;
+        narrow_at[h] = L::ROPE_AT + Narrow::transposed(h, rope_block, lane);
+    }
+    // dS as it was kept: key k of a block in bytes 64k .., the transposing read takes four keys of 16 rows
+    const unsigned ds_at = L::DS_AT + wave_row_tile * index_math::KeptGradients::BLOCK_BYTES +
+                           64 * (4 * g + lane % 16 / 4) + 16 * (lane % 4) + 8 * (lane / 16 % 2);
+    f32x16 sum[GROUP][LATENT_BLOCKS], rope_sum;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        rope_sum[i] = 0.f;
+#pragma unroll
+        for (int t = 0; t < GROUP; ++t) {
+#pragma unroll
+            for (int j = 0; j < LATENT_BLOCKS; ++j) sum[t][j][i] = 0.f;
+        }
+    }
+    for (int tile = 0; tile < tiles; ++tile) {
+        const int behind = min(tiles - 1 - tile, AHEAD - 1);   // tiles that may stay in flight
+        if (behind == 0) {
+            wait_for_all_but(std::integral_constant<int, 0>{});
+        } else if (AHEAD == 2 || behind == 1) {
+            wait_for_all_but(std::integral_constant<int, 1>{});
+        } else {
+            wait_for_all_but(std::integral_constant<int, 2>{});
+        }
+        workgroup_barrier();   // the tile is there, and the stage of the tile before has been read
+        if (tile + AHEAD < tiles) request_tile(tile + AHEAD);
+        const unsigned char* stage = lds + tile % L::STAGES * L::STAGE_BYTES;
+        const int first_seen = kept.first_row_tile(tile);
+        unrolled<0, 2>([&](auto tag) {
+            constexpr int N = decltype(tag)::value;   // 16-key step
+            auto fragment = [&](unsigned low_at, unsigned high_at) {
+                const s16x4 low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((transposing_read_pointer)(stage + low_at));
+                const s16x4 high = __builtin_amdgcn_ds_read_tr16_b64_v4i16((transposing_read_pointer)(stage + high_at));
+                return __builtin_bit_cast(bf16x8, __builtin_shufflevector(low, high, 0, 1, 2, 3, 4, 5, 6, 7));
+            };
+            bf16x8 ds[GROUP];
+#pragma unroll
+            for (int t = 0; t < GROUP; ++t) {
+                const unsigned at = ds_at + t * index_math::KeptGradients::BLOCK_BYTES + 1024 * N;
+                ds[t] = fragment(at, at + 512);
+                if (first_row_tile + wave_row_tile + t < first_seen) ds[t] = __builtin_bit_cast(bf16x8, u32x4{0, 0, 0, 0});
+            }
+#pragma unroll
+            for (int j = 0; j < LATENT_BLOCKS; ++j) {
+                const bf16x8 columns = fragment(wide_at[0][j] + 16 * N * L::WIDE_ROW, wide_at[1][j] + 16 * N * L::WIDE_ROW);
+#pragma unroll
+                for (int t = 0; t < GROUP; ++t) {
+                    sum[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(columns, ds[t], sum[t][j], 0, 0, 0);
+                }
+            }
+            if (GROUP > 1 || v < 2) {
+                const bf16x8 columns = fragment(narrow_at[0] + 16 * N * L::NARROW_ROW, narrow_at[1] + 16 * N * L::NARROW_ROW);
+                bf16x8 own = ds[0];
+                if (GROUP > 1 && rope_tile == 1) own = ds[GROUP - 1];
+                rope_sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(columns, own, rope_sum, 0, 0, 0);
+            }
+        });
+    }
+
+    // A lane holds row lq of its row tiles and columns 32*block + 8*(i/4) + 4*g + i%4: rows through LDS, so that a store
+    // instruction writes whole lines
+    workgroup_barrier();
+    auto stage_block = [&](const f32x16& values, int row_tile, int block) {
+        unsigned char* staged = lds + (TILE * row_tile + lq) * L::OUT_PITCH + 2 * TILE * block + 8 * g;
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+            *reinterpret_cast<u32x2*>(staged + 16 * i4) =
+                u32x2{pack_bf16(values[4 * i4 + 0], values[4 * i4 + 1]), pack_bf16(values[4 * i4 + 2], values[4 * i4 + 3])};
+        }
+    };
+#pragma unroll
+    for (int t = 0; t < GROUP; ++t) {
+#pragma unroll
+        for (int j = 0; j < LATENT_BLOCKS; ++j) stage_block(sum[t][j], wave_row_tile + t, LATENT_BLOCKS * v + j);
+    }
+    if (GROUP > 1 || v < 2) stage_block(rope_sum, wave_row_tile + rope_tile, RANK / TILE + rope_block);
+    workgroup_barrier();
+    const int valid_rows = (int)min((long long)L::ROWS, rows - row0);
+    for (int out_row = wave; out_row < valid_rows; out_row += THREADS / 64) {
+        const size_t target = batch_row0 + row0 + out_row;
+        *reinterpret_cast<u32x4*>(query_latent_gradient + target * RANK + 8 * lane) =
+            *reinterpret_cast<const u32x4*>(lds + out_row * L::OUT_PITCH + 16 * lane);
+        if (lane < ROPE / 8) {
+            *reinterpret_cast<u32x4*>(query_rope_gradient + target * ROPE + 8 * lane) =
+                *reinterpret_cast<const u32x4*>(lds + out_row * L::OUT_PITCH + 2 * RANK + 16 * lane);
+        }
+    }
+}
+
+template <int GROUP>
+void launch(bf16_t* query_latent_gradient, bf16_t* query_rope_gradient, const unsigned char* kept_gradients,
+            const bf16_t* kv_latent, const bf16_t* key_rope, int batch_size, int sequence_length, int heads, int key_tiles,
+            hipStream_t stream) {
+    using L = ProductLayout<GROUP>;
+    static hip_common::OncePerDevice prepared;
+    prepared.run([] {
+        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(mla_absorbed_query_product_kernel<GROUP>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, L::LDS_BYTES));
+    });
+    const long long rows = (long long)sequence_length * heads;
+    const long long row_blocks = (rows + L::ROWS - 1) / L::ROWS;
+    hipLaunchKernelGGL(mla_absorbed_query_product_kernel<GROUP>, dim3((unsigned)(row_blocks * batch_size)), dim3(THREADS),
+                       L::LDS_BYTES, stream, query_latent_gradient, query_rope_gradient, kept_gradients, kv_latent, key_rope,
+                       batch_size, sequence_length, heads, key_tiles, (int)row_blocks);
+    HIP_CHECK(hipGetLastError());
+}
+
+}  // namespace
+
+void mla_absorbed_query_product_launch(bf16_t* query_latent_gradient, bf16_t* query_rope_gradient,
+                                       const unsigned char* kept_gradients, const bf16_t* kv_latent,
+                                       const bf16_t* key_rope, int batch_size, int sequence_length, int heads,
+                                       int key_tiles, hipStream_t stream) {
+    // 128 rows a workgroup where that is a workgroup per compute unit. The whole backward in us, 64 / 128 rows: 148 workgroups of
+    // 128 98 / 103, 226 82 / 81, 282 349 / 350, 304 118 / 114, 512 235 / 228, 1500 1995 / 1895; 33 81 / 87.
+    const long long rows = (long long)sequence_length * heads;
+    if ((rows + 127) / 128 * batch_size >= hip_common::compute_units_of_current_device()) {
+        launch<2>(query_latent_gradient, query_rope_gradient, kept_gradients, kv_latent, key_rope, batch_size,
+                  sequence_length, heads, key_tiles, stream);
+    } else {
+        launch<1>(query_latent_gradient, query_rope_gradient, kept_gradients, kv_latent, key_rope, batch_size,
+                  sequence_length, heads, key_tiles, stream);
+    }
+}
+
+}  // namespace dscuda

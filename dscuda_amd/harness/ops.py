@@ -31,6 +31,9 @@ class _Mla:
         self.lib = lib
         self.forward = bind(lib, "dscuda_mla_forward", [P] * 6 + [I] * 5 + [F, P])
         self.backward = bind(lib, "dscuda_mla_backward", [P] * 11 + [I] * 5 + [F, P])
+        self.backward_workspace_elements = bind(lib, "dscuda_mla_backward_workspace_elements", [I] * 5, ctypes.c_size_t)
+        self.backward_workspace = bind(
+            lib, "dscuda_mla_backward_workspace", [P] * 12 + [ctypes.c_size_t] + [I] * 5 + [F, P])
         self.decode = bind(lib, "dscuda_mla_decode", [P] * 7 + [I] * 7 + [F, P])
         self.decode_plan_elements = bind(lib, "dscuda_mla_decode_plan_elements", [I] * 4, ctypes.c_size_t)
         self.decode_plan = bind(lib, "dscuda_mla_decode_plan", [P] * 2 + [I] * 4 + [P])
@@ -152,16 +155,31 @@ def mla_forward(query_latent, query_rope, kv_latent, key_rope, scale, out=None, 
     return out, lse
 
 
-def mla_backward(dout, out, lse, query_latent, query_rope, kv_latent, key_rope, scale, grads=None):
-    """Absorbed MLA backward (dscuda_mla_backward) -> (dq_lat, dq_rope, dlatent, dk_rope)."""
+def mla_backward_workspace(batch, tokens, heads, rank=512, rope=64, device="cuda"):
+    """fp32 workspace of the absorbed backward (dscuda_mla_backward_workspace_elements): room for dS, two bytes per
+    visible (row, key) pair.  None where the call makes no use of one, or the memory is not there."""
+    elements = mla_library().backward_workspace_elements(batch, tokens, heads, rank, rope)
+    if not elements:
+        return None
+    try:
+        return torch.empty(elements, device=device, dtype=torch.float32)
+    except torch.OutOfMemoryError:
+        return None
+
+
+def mla_backward(dout, out, lse, query_latent, query_rope, kv_latent, key_rope, scale, grads=None, workspace=None):
+    """Absorbed MLA backward (dscuda_mla_backward_workspace) -> (dq_lat, dq_rope, dlatent, dk_rope)."""
     _require_cuda(dout, out, lse, query_latent, query_rope, kv_latent, key_rope)
     b, t, h, c = query_latent.shape
     r = query_rope.shape[-1]
     if grads is None:
         grads = tuple(torch.empty_like(x) for x in (query_latent, query_rope, kv_latent, key_rope))
+    if workspace is None:
+        workspace = mla_backward_workspace(b, t, h, c, r, query_latent.device)
     lib = mla_library()
-    checked(lib.lib, "mla", lib.backward(
-        *pointers((*grads, dout, out, lse, query_latent, query_rope, kv_latent, key_rope)),
+    kept = (None, 0) if workspace is None else (workspace.data_ptr(), workspace.numel() * workspace.element_size() // 4)
+    checked(lib.lib, "mla", lib.backward_workspace(
+        *pointers((*grads, dout, out, lse, query_latent, query_rope, kv_latent, key_rope)), *kept,
         b, t, h, c, r, scale, stream()))
     return grads
 

@@ -75,6 +75,41 @@ void mla_compressed_attention_backward_cuda(
     float scale,
     hipStream_t stream = nullptr);
 
+// The same with a workspace (additive, no counterpart in the reference): the key-gradient launch keeps dS there, two
+// bytes per (row, visible key) pair, so that the query gradients are one product instead of three, and partial key
+// gradients that the query-gradient buffers have no room for.  mla_backward_workspace_elements floats hold all that is
+// of use (at most 4 GiB of dS: batch elements are taken in groups; some 0.1 GB of partial results); 0 where a call
+// makes no use of one.  Any smaller size, 0 and nullptr included, is taken for the batch elements
+// that fit, or none.  16-byte aligned, needs no initialisation.
+std::size_t mla_backward_workspace_elements(
+    int batch_size,
+    int sequence_length,
+    int heads,
+    int kv_rank,
+    int rope_size);
+
+void mla_compressed_attention_backward_workspace_cuda(
+    __hip_bfloat16* query_latent_gradient,
+    __hip_bfloat16* query_rope_gradient,
+    __hip_bfloat16* kv_latent_gradient,
+    __hip_bfloat16* key_rope_gradient,
+    const __hip_bfloat16* output_gradient,
+    const __hip_bfloat16* output,
+    const float* logsumexp,
+    const __hip_bfloat16* query_latent,
+    const __hip_bfloat16* query_rope,
+    const __hip_bfloat16* kv_latent,
+    const __hip_bfloat16* key_rope,
+    float* workspace,
+    std::size_t workspace_elements,
+    int batch_size,
+    int sequence_length,
+    int heads,
+    int kv_rank,
+    int rope_size,
+    float scale,
+    hipStream_t stream = nullptr);
+
 // FP32 elements of decode workspace.  Replaces reference include/mla.h:57-61;
 // same formula, B*H*splits*(C+2), so buffers sized by either library fit.
 std::size_t mla_decode_workspace_elements(
@@ -355,6 +390,19 @@ int dscuda_mla_backward(  // mla_bridge.cu:33-51
     const __hip_bfloat16* dout, const __hip_bfloat16* output, const float* lse,
     const __hip_bfloat16* query, const __hip_bfloat16* query_rope,
     const __hip_bfloat16* latent, const __hip_bfloat16* key_rope,
+    int batch, int sequence, int heads, int rank, int rope, float scale,
+    hipStream_t stream);
+
+// additive (no counterpart in the reference): see the dscuda:: functions of the same names above
+std::size_t dscuda_mla_backward_workspace_elements(int batch, int sequence, int heads, int rank, int rope);
+
+int dscuda_mla_backward_workspace(
+    __hip_bfloat16* dquery, __hip_bfloat16* dquery_rope,
+    __hip_bfloat16* dlatent, __hip_bfloat16* dkey_rope,
+    const __hip_bfloat16* dout, const __hip_bfloat16* output, const float* lse,
+    const __hip_bfloat16* query, const __hip_bfloat16* query_rope,
+    const __hip_bfloat16* latent, const __hip_bfloat16* key_rope,
+    float* workspace, std::size_t workspace_elements,
     int batch, int sequence, int heads, int rank, int rope, float scale,
     hipStream_t stream);
 

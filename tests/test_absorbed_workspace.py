@@ -1,0 +1,78 @@
+"""The absorbed backward with a workspace (dS kept for the query gradients, slots for partial key gradients): its size
+on the host, and on the GPU the gradients with and without one at the edges of tiles, blocks and items."""
+
+import ctypes
+
+import pytest
+import torch
+
+from dscuda_amd.harness import configs
+from dscuda_amd.harness.common import I, bind, library
+from oracle import attention_oracle as oracle
+from parity import announce, assert_close_bf16
+
+
+def elements(batch, tokens, heads, rank=512):
+    return bind(library("mla"), "dscuda_mla_backward_workspace_elements", [I] * 5, ctypes.c_size_t)(
+        batch, tokens, heads, rank, 64)
+
+
+def kept_bytes(tokens, heads):
+    """dS of one batch element: 2 KB per 32 x 32 tile that a key block of 32 (or 64) keys visits."""
+    row_tiles = -(-tokens * heads // 32)
+    return max(sum(max(0, row_tiles - size * heads * block) for block in range(-(-tokens // (32 * size)))) * 2048 * size
+               for size in (1, 2))
+
+
+@pytest.mark.parametrize("batch,tokens,heads", [(1, 513, 8), (3, 700, 5), (1, 65, 128), (2, 4096, 16)])
+def test_size_holds_every_block_and_slot(batch, tokens, heads):
+    row_tiles = -(-tokens * heads // 32)
+    key_blocks = -(-tokens // 32)
+    visits = sum(max(0, row_tiles - heads * block) for block in range(key_blocks)) * batch
+    slots = min(256, visits // 2) + key_blocks * batch   # of ranges: [32 keys][576] floats each
+    assert elements(batch, tokens, heads) * 4 >= batch * kept_bytes(tokens, heads) + slots * 32 * 576 * 4
+
+
+def test_size_is_zero_or_bounded():
+    assert elements(1, 0, 8) == 0 and elements(1, 64, 8, rank=256) == 0
+    assert elements(1, 300, 4) == 0                       # P and dS are kept in the query gradients
+    assert elements(1, 16384, 128) == 0                   # dS of one batch element beyond 4 GiB: formed twice instead
+    assert 0 < elements(64, 4096, 32) * 4 <= (4 << 30) + (1 << 30)
+
+
+# rows that end inside a row tile, a 64- and a 128-row workgroup; key blocks of 64 cut at 1, 32, 33 keys; one head, and
+# more heads than a workgroup has rows; ranges of 32-key blocks and items of 64-key blocks; several batch elements
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,tokens,heads,interval_tiles", [
+    (1, 17, 128, 0), (2, 33, 40, 0), (1, 513, 3, 0), (1, 545, 8, 0), (3, 600, 4, 0), (1, 200, 33, 0), (2, 320, 16, 0),
+    (1, 1000, 1, 0), (1, 1025, 8, 0), (1, 130, 150, 0), (1, 1, 40, 0), (1, 187, 32, 0), (3, 9, 2, 0), (2, 700, 3, 0),
+    (1, 1000, 33, 0), (1, 513, 3, 7), (2, 97, 40, 50), (1, 65, 128, 100)])
+def test_gradients_with_and_without(cuda, batch, tokens, heads, interval_tiles):
+    from dscuda_amd.harness import ops
+    ql, qr, c, kr, scale = configs.mla_absorbed_inputs(batch, tokens, heads)
+    g = torch.Generator().manual_seed(6)
+    dout = (torch.randn(batch, tokens, heads, 512, generator=g) * (0.2 if heads < 16 else 0.05)).bfloat16()
+    mask = oracle.causal_mask(tokens)
+    out, lse = oracle.mla_forward(ql, qr, c, kr, scale, mask)
+    operands = [x.to(cuda) for x in (dout, out, lse, ql, qr, c, kr)]
+    announce("mla_backward, workspace", dict(B=batch, T=tokens, H=heads, tiles=interval_tiles))
+
+    def gradients(workspace):
+        grads = tuple(torch.full_like(x, float("nan")) for x in operands[3:])
+        return ops.mla_backward(*operands, scale, grads, workspace)
+
+    ops.mla_backward_set_key_interval_tiles(interval_tiles)
+    try:
+        runs = [gradients(torch.empty(0, device=cuda)), gradients(None)]
+        # dS of one batch element alone (the others after it, slots in the query gradients), and a guard behind it
+        one = kept_bytes(tokens, heads) // 4
+        buffer = torch.full((one + 1024,), float("nan"), device=cuda)
+        runs.append(gradients(buffer[:one]))
+        torch.cuda.synchronize()
+    finally:
+        ops.mla_backward_set_key_interval_tiles(0)
+    assert torch.isnan(buffer[one:]).all()
+    expected = oracle.mla_backward_unrounded(dout, out, lse, ql, qr, c, kr, scale, mask)
+    for run in runs:
+        for name, actual, reference in zip(("dq_latent", "dq_rope", "dlatent", "dk_rope"), run, expected):
+            assert_close_bf16(name, actual.cpu(), reference)
