@@ -747,10 +747,10 @@ DSCUDA_HOST_DEVICE inline bool short_backward(long long batch, int tokens, int h
 }
 
 // Which of them still do where a workspace could hold dS and the slots of ranges: one launch less, but key gradients that
-// read 64 bytes a row. Backward, P and dS kept / ranges (us): 300 x 4 30 / 32, 512 x 4 40 / 46, 250 x 8 33 / 38, 512 x 8 50 / 50;
-// 128 x 16 28 / 28, 64 x 32 28 / 25, 350 x 16 54 / 46, 480 x 16 77 / 54, 3 x 500 x 4 62 / 54, 8 x 338 x 3 63 / 49, 32 x 64 x 4 34 / 30.
+// read 64 bytes a row. Backward, P and dS kept / ranges (us): 100 x 8 24 / 28, 300 x 4 30 / 31, 512 x 4 40 / 43, 300 x 8 36 / 39;
+// 3 x 256 x 4 33 / 32, 512 x 6 46 / 45, 512 x 8 50 / 46, 64 x 32 28 / 24, 200 x 32 53 / 41, 480 x 16 77 / 53, 8 x 338 x 3 63 / 49.
 DSCUDA_HOST_DEVICE inline bool short_without_workspace(long long batch, int tokens, int heads) {
-    return heads < 16 && (long long)tokens * heads * batch <= 4096;
+    return heads < 16 && (long long)tokens * heads * batch <= 2500;
 }
 
 DSCUDA_HOST_DEVICE inline bool kept_in_rope(int token_block, int blocks) { return token_block == blocks - 1; }

@@ -12,7 +12,8 @@
 // of [32 keys][512] + [32 keys][64] + dS.  Wave (r, v) = (w / 4, w % 4): row tiles GROUP * r .., latent column blocks
 // 4v .. 4v + 3 of each of them and one of the rope blocks.  Bound by the key tiles a compute unit draws from its L2
 // (36 KB a step, some 21 bytes a cycle against 1152 matrix cycles at GROUP = 2), hence 128 rows wherever that leaves
-// workgroups enough; 192 rows need more registers than there are.
+// workgroups enough; 192 rows need more registers than there are.  With few rows a workgroup takes half of the columns
+// (PARTS = 2, 18 KB of keys a step and compute unit).
 #include "attn_kernels.h"
 #include "hip_common.h"
 #include "index_math.h"
@@ -28,31 +29,33 @@ constexpr int ROPE = 64;
 constexpr int TILE = 32;
 constexpr int THREADS = 512;
 
-template <int GROUP>
+template <int GROUP, int PARTS>
 struct ProductLayout {
+    static_assert(PARTS == 1 || GROUP == 1, "halves of the columns are for few rows");
     static constexpr int ROWS = 64 * GROUP;
     static constexpr int ROW_TILES = 2 * GROUP;
-    static constexpr int WIDE_ROW = 2 * RANK;
+    static constexpr int WIDE_ROW = 2 * RANK / PARTS;
     static constexpr int NARROW_ROW = 2 * ROPE;
     static constexpr int ROPE_AT = TILE * WIDE_ROW;
     static constexpr int DS_AT = ROPE_AT + TILE * NARROW_ROW;
     static constexpr int STAGE_BYTES = DS_AT + ROW_TILES * index_math::KeptGradients::BLOCK_BYTES;
     static constexpr int STAGES = GROUP == 1 ? 4 : 3;
-    static constexpr int OUT_PITCH = 2 * (RANK + ROPE) + 16;   // of a staged gradient row
+    static constexpr int OUT_ROPE = WIDE_ROW;                            // of a staged gradient row
+    static constexpr int OUT_PITCH = WIDE_ROW + 2 * ROPE / PARTS + 16;
     static constexpr int OUT_BYTES = ROWS * OUT_PITCH;
     static constexpr int LDS_BYTES = STAGES * STAGE_BYTES > OUT_BYTES ? STAGES * STAGE_BYTES : OUT_BYTES;
     static_assert(LDS_BYTES <= 160 * 1024, "LDS of a compute unit");
 };
 
-template <int GROUP>
+template <int GROUP, int PARTS>
 __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
     bf16_t* __restrict__ query_latent_gradient, bf16_t* __restrict__ query_rope_gradient,
     const unsigned char* __restrict__ kept_gradients, const bf16_t* __restrict__ kv_latent,
     const bf16_t* __restrict__ key_rope, int batch_size, int sequence_length, int heads, int key_tiles, int row_blocks) {
-    using L = ProductLayout<GROUP>;
+    using L = ProductLayout<GROUP, PARTS>;
     using Wide = index_math::TileReadMath<L::WIDE_ROW>;
     using Narrow = index_math::TileReadMath<L::NARROW_ROW>;
-    constexpr int LATENT_BLOCKS = RANK / TILE / 4;   // 32-column blocks of a wave
+    constexpr int LATENT_BLOCKS = RANK / TILE / 4 / PARTS;   // 32-column blocks of a wave
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -61,11 +64,12 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
     const int g = lane / 32;
     const int T = sequence_length;
     const long long rows = (long long)T * heads;
-    const int batch = blockIdx.x % batch_size;
-    const int row_block = row_blocks - 1 - blockIdx.x / batch_size;   // latest rows (most keys) first
+    const int column_part = blockIdx.x % PARTS;
+    const int batch = blockIdx.x / PARTS % batch_size;
+    const int row_block = row_blocks - 1 - blockIdx.x / PARTS / batch_size;   // latest rows (most keys) first
     const long long row0 = (long long)row_block * L::ROWS;
     const long long batch_row0 = (long long)batch * rows;
-    const unsigned char* latent = reinterpret_cast<const unsigned char*>(kv_latent + (size_t)batch * T * RANK);
+    const unsigned char* latent = reinterpret_cast<const unsigned char*>(kv_latent + (size_t)batch * T * RANK) + column_part * L::WIDE_ROW;
     const unsigned char* rope = reinterpret_cast<const unsigned char*>(key_rope + (size_t)batch * T * ROPE);
     const int tiles = (int)((min(row0 + L::ROWS, rows) - 1) / heads) / TILE + 1;   // key tiles the rows see
     const index_math::KeptGradients kept = index_math::kept_gradients(T, heads, key_tiles);
@@ -74,10 +78,11 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
 
     const int v = wave % 4;
     const int wave_row_tile = GROUP * (wave / 4);   // of the workgroup's
-    const int rope_tile = GROUP == 1 ? 0 : v / 2;   // whose rope block v % 2 the wave sums; GROUP = 1: waves v < 2 only
-    const int rope_block = v % 2;
+    const int rope_tile = GROUP == 1 ? 0 : v / 2;   // whose rope block the wave sums; GROUP = 1: not every wave has one
+    const int rope_block = PARTS == 1 ? v % 2 : column_part;
+    const bool sums_rope = GROUP > 1 || v < 2 / PARTS;
 
-    // A wave requests key rows 4*wave .. +3 of the wide tile, waves 0 .. 3 also eight rows of the narrow one, and 1 KB,
+    // A wave requests key rows 4*wave .. +3 of the wide tile (1 KB an instruction), waves 0 .. 3 also eight rows of the narrow one, and 1 KB,
     // half a row tile, of dS: every wave at GROUP = 2, waves 4 .. 7 at GROUP = 1.  Keys past the end repeat the last
     // one (their dS is zero), row tiles past the end repeat the last one (their results are not stored), and a tile
     // that does not see the keys yet reads what precedes its blocks and is left out below.
@@ -88,11 +93,12 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
         const unsigned target = lds_base + tile % L::STAGES * L::STAGE_BYTES;
         const int last = min(T - tile * TILE, TILE) - 1;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int key = 4 * wave + j;
-            direct_load_16_offset(latent + (size_t)tile * TILE * L::WIDE_ROW,
-                                  (unsigned)(min(key, last) * L::WIDE_ROW + 16 * (lane ^ index_math::tile_swizzle<L::WIDE_ROW>(key))),
-                                  target + key * L::WIDE_ROW);
+        for (int j = 0; j < 4 / PARTS; ++j) {
+            const int first = 4 * wave + PARTS * j;
+            const int key = first + lane / (64 / PARTS);
+            const int chunk = lane % (64 / PARTS) ^ index_math::tile_swizzle<L::WIDE_ROW>(key);
+            direct_load_16_offset(latent + (size_t)tile * TILE * (2 * RANK), (unsigned)(min(key, last) * (2 * RANK) + 16 * chunk),
+                                  target + first * L::WIDE_ROW);
         }
         if (wave < 4) {
             const int key = 8 * wave + lane / 8;
@@ -109,7 +115,7 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
     // all but the newest `tiles_in_flight` tiles of the wave's requests have arrived
     auto wait_for_all_but = [&](auto tiles_in_flight) {
         constexpr int N = decltype(tiles_in_flight)::value;
-        if (GROUP > 1 && wave < 4) wait_vector_memory<6 * N>(); else wait_vector_memory<5 * N>();
+        if (GROUP > 1 && wave < 4) wait_vector_memory<6 * N>(); else wait_vector_memory<(4 / PARTS + 1) * N>();
     };
     constexpr int AHEAD = L::STAGES - 1;
     for (int tile = 0; tile < min(tiles, AHEAD); ++tile) request_tile(tile);
@@ -118,7 +124,10 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
 #pragma unroll
-        for (int j = 0; j < LATENT_BLOCKS; ++j) wide_at[h][j] = Wide::transposed(h, j, lane) + 256 * v;
+        for (int j = 0; j < LATENT_BLOCKS; ++j) {
+            const int block = LATENT_BLOCKS * v + j;
+            wide_at[h][j] = Wide::transposed(h, block % Wide::TR, lane) + 64 * Wide::TR * (block / Wide::TR);
+        }
         narrow_at[h] = L::ROPE_AT + Narrow::transposed(h, rope_block, lane);
     }
     // dS as it was kept: key k of a block in bytes 64k .., the transposing read takes four keys of 16 rows
@@ -169,7 +178,7 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
                     sum[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(columns, ds[t], sum[t][j], 0, 0, 0);
                 }
             }
-            if (GROUP > 1 || v < 2) {
+            if (sums_rope) {
                 const bf16x8 columns = fragment(narrow_at[0] + 16 * N * L::NARROW_ROW, narrow_at[1] + 16 * N * L::NARROW_ROW);
                 bf16x8 own = ds[0];
                 if (GROUP > 1 && rope_tile == 1) own = ds[GROUP - 1];
@@ -181,8 +190,8 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
     // A lane holds row lq of its row tiles and columns 32*block + 8*(i/4) + 4*g + i%4: rows through LDS, so that a store
     // instruction writes whole lines
     workgroup_barrier();
-    auto stage_block = [&](const f32x16& values, int row_tile, int block) {
-        unsigned char* staged = lds + (TILE * row_tile + lq) * L::OUT_PITCH + 2 * TILE * block + 8 * g;
+    auto stage_block = [&](const f32x16& values, int row_tile, int byte) {
+        unsigned char* staged = lds + (TILE * row_tile + lq) * L::OUT_PITCH + byte + 8 * g;
 #pragma unroll
         for (int i4 = 0; i4 < 4; ++i4) {
             *reinterpret_cast<u32x2*>(staged + 16 * i4) =
@@ -192,35 +201,38 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
 #pragma unroll
     for (int t = 0; t < GROUP; ++t) {
 #pragma unroll
-        for (int j = 0; j < LATENT_BLOCKS; ++j) stage_block(sum[t][j], wave_row_tile + t, LATENT_BLOCKS * v + j);
+        for (int j = 0; j < LATENT_BLOCKS; ++j) stage_block(sum[t][j], wave_row_tile + t, 2 * TILE * (LATENT_BLOCKS * v + j));
     }
-    if (GROUP > 1 || v < 2) stage_block(rope_sum, wave_row_tile + rope_tile, RANK / TILE + rope_block);
+    if (sums_rope) stage_block(rope_sum, wave_row_tile + rope_tile, L::OUT_ROPE + (PARTS == 1 ? 2 * TILE * rope_block : 0));
     workgroup_barrier();
     const int valid_rows = (int)min((long long)L::ROWS, rows - row0);
-    for (int out_row = wave; out_row < valid_rows; out_row += THREADS / 64) {
+    constexpr int LANES = 64 / PARTS;   // of a row
+    for (int out_row = PARTS * wave + lane / LANES; out_row < valid_rows; out_row += PARTS * THREADS / 64) {
         const size_t target = batch_row0 + row0 + out_row;
-        *reinterpret_cast<u32x4*>(query_latent_gradient + target * RANK + 8 * lane) =
-            *reinterpret_cast<const u32x4*>(lds + out_row * L::OUT_PITCH + 16 * lane);
-        if (lane < ROPE / 8) {
-            *reinterpret_cast<u32x4*>(query_rope_gradient + target * ROPE + 8 * lane) =
-                *reinterpret_cast<const u32x4*>(lds + out_row * L::OUT_PITCH + 2 * RANK + 16 * lane);
+        const int part = lane % LANES;
+        const unsigned char* staged = lds + out_row * L::OUT_PITCH + 16 * part;
+        *reinterpret_cast<u32x4*>(query_latent_gradient + target * RANK + column_part * (RANK / PARTS) + 8 * part) =
+            *reinterpret_cast<const u32x4*>(staged);
+        if (part < ROPE / 8 / PARTS) {
+            *reinterpret_cast<u32x4*>(query_rope_gradient + target * ROPE + column_part * (ROPE / PARTS) + 8 * part) =
+                *reinterpret_cast<const u32x4*>(staged + L::OUT_ROPE);
         }
     }
 }
 
-template <int GROUP>
+template <int GROUP, int PARTS>
 void launch(bf16_t* query_latent_gradient, bf16_t* query_rope_gradient, const unsigned char* kept_gradients,
             const bf16_t* kv_latent, const bf16_t* key_rope, int batch_size, int sequence_length, int heads, int key_tiles,
             hipStream_t stream) {
-    using L = ProductLayout<GROUP>;
+    using L = ProductLayout<GROUP, PARTS>;
     static hip_common::OncePerDevice prepared;
     prepared.run([] {
-        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(mla_absorbed_query_product_kernel<GROUP>),
+        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(mla_absorbed_query_product_kernel<GROUP, PARTS>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, L::LDS_BYTES));
     });
     const long long rows = (long long)sequence_length * heads;
     const long long row_blocks = (rows + L::ROWS - 1) / L::ROWS;
-    hipLaunchKernelGGL(mla_absorbed_query_product_kernel<GROUP>, dim3((unsigned)(row_blocks * batch_size)), dim3(THREADS),
+    hipLaunchKernelGGL((mla_absorbed_query_product_kernel<GROUP, PARTS>), dim3((unsigned)(row_blocks * batch_size * PARTS)), dim3(THREADS),
                        L::LDS_BYTES, stream, query_latent_gradient, query_rope_gradient, kept_gradients, kv_latent, key_rope,
                        batch_size, sequence_length, heads, key_tiles, (int)row_blocks);
     HIP_CHECK(hipGetLastError());
@@ -234,13 +246,20 @@ void mla_absorbed_query_product_launch(bf16_t* query_latent_gradient, bf16_t* qu
                                        int key_tiles, hipStream_t stream) {
     // 128 rows a workgroup where that is a workgroup per compute unit. The whole backward in us, 64 / 128 rows: 148 workgroups of
     // 128 98 / 103, 226 82 / 81, 282 349 / 350, 304 118 / 114, 512 235 / 228, 1500 1995 / 1895; 33 81 / 87.
+    // Workgroups of 64 rows and half the columns where whole rows are no workgroup per compute unit, halves / whole rows: 38 workgroups
+    // of 64 rows 45 / 49, 63 63 / 68, 128 106 / 118, 150 64 / 67, 256 72 / 72; 296 87 / 83, 350 106 / 98.
     const long long rows = (long long)sequence_length * heads;
-    if ((rows + 127) / 128 * batch_size >= hip_common::compute_units_of_current_device()) {
-        launch<2>(query_latent_gradient, query_rope_gradient, kept_gradients, kv_latent, key_rope, batch_size,
-                  sequence_length, heads, key_tiles, stream);
+    const int units = hip_common::compute_units_of_current_device();
+    auto start = [&](auto launch_form) {
+        launch_form(query_latent_gradient, query_rope_gradient, kept_gradients, kv_latent, key_rope, batch_size, sequence_length,
+                    heads, key_tiles, stream);
+    };
+    if ((rows + 127) / 128 * batch_size >= units) {
+        start(launch<2, 1>);
+    } else if ((rows + 63) / 64 * batch_size > units) {
+        start(launch<1, 1>);
     } else {
-        launch<1>(query_latent_gradient, query_rope_gradient, kept_gradients, kv_latent, key_rope, batch_size,
-                  sequence_length, heads, key_tiles, stream);
+        start(launch<1, 2>);
     }
 }
 

@@ -46,7 +46,7 @@ def test_size_is_zero_or_bounded():
 @pytest.mark.parametrize("batch,tokens,heads,interval_tiles", [
     (1, 17, 128, 0), (2, 33, 40, 0), (1, 513, 3, 0), (1, 545, 8, 0), (3, 600, 4, 0), (1, 200, 33, 0), (2, 320, 16, 0),
     (1, 1000, 1, 0), (1, 1025, 8, 0), (1, 130, 150, 0), (1, 1, 40, 0), (1, 187, 32, 0), (3, 9, 2, 0), (2, 700, 3, 0),
-    (1, 1000, 33, 0), (1, 513, 3, 7), (2, 97, 40, 50), (1, 65, 128, 100)])
+    (1, 1000, 33, 0), (1, 512, 8, 0), (2, 530, 16, 0), (1, 513, 3, 7), (2, 97, 40, 50), (1, 65, 128, 100)])
 def test_gradients_with_and_without(cuda, batch, tokens, heads, interval_tiles):
     from dscuda_amd.harness import ops
     ql, qr, c, kr, scale = configs.mla_absorbed_inputs(batch, tokens, heads)
