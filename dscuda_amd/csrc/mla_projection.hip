@@ -268,11 +268,11 @@ __global__ __launch_bounds__(THREADS) void mla_unabsorb_output_kernel(bf16_t* __
 // tokens, and every load of a thread is in flight at once: one round trip to memory, eight MFMAs a wave.  16 tokens of
 // 16 heads: absorb 7.6 -> 3.2 us, un-absorb 6.6 -> 3.7.
 //
-// Every 32 tokens fetch the weight again, so the kernels above win once (token tiles) x heads is large.  Absorb at 256
-// tiles 8.0-8.2 against 9.3-11.6 us (64 tokens of 128 heads, 512 of 16), at 512 tiles 13.4 against 13.2-13.9.
-// Un-absorb, whose weight rows come as 32 bytes of 32 rows an instruction, at 128 tiles 5.1-5.8 against 6.7-9.7 us
+// Every 32 tokens fetch the weight again, so the kernels win once (token tiles) x heads is large.  Absorb by quarters,
+// below, against few tokens: equal up to 128 tiles, 7.9 / 9.2 us at 256 (1000 tokens of 8 heads; equal for 64 of 128), 9.1 / 12.8
+// at 512.  Un-absorb, whose weight rows come as 32 bytes of 32 rows an instruction, at 128 tiles 5.1-5.8 against 6.7-9.7 us
 // (16 tokens of 128 heads, 128 of 32), at 256 tiles 10.2-12.8 against 8.1-9.8.
-constexpr long long ABSORB_FEW_TILES = 256;
+constexpr long long ABSORB_FEW_TILES = 128;
 constexpr long long UNABSORB_FEW_TILES = 128;
 
 constexpr int SLICE = RANK / 4;                    // output columns of an absorb workgroup
@@ -401,6 +401,126 @@ __global__ __launch_bounds__(THREADS) void mla_unabsorb_output_few_kernel(bf16_t
     }
 }
 
+// ---- more tokens, results that the memory-side cache takes -----------------------------
+// q_latent = q_nope W_UK by quarters of the columns: a wave holds the quarter's weight in 128 registers and takes every
+// fourth token tile, and two workgroups share a compute unit, so that one's loads and stores go on while the other
+// multiplies or fetches its 32 KB of weight (mla_absorb_query_kernel keeps 128 KB in LDS, one workgroup of four waves
+// per compute unit, which fetches first and then streams).  blockIdx.x = (chunk of the tokens, head, quarter); the
+// quarters of a head, which read the same rows, go to one XCD.  Bound by the bytes written: 1024 tokens x 128 heads
+// 40.4 -> 33.5 us (5.5 TB/s), 1000 x 64 25.0 -> 19.7, 1000 x 16 12.8 -> 9.0, 250 x 64 12.0 -> 9.3.
+// Rows written as four times 256 bytes by workgroups of their own are slower once they go to memory: 2048 x 128
+// (268 MB) 80.7 -> 85, 4096 x 128 137 -> 154.
+constexpr long long SLICE_RESULT_BYTES = 160LL << 20;
+
+__global__ __launch_bounds__(THREADS, 2) void mla_absorb_query_slice_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
+                                                                            const bf16_t* __restrict__ weight,
+                                                                            long long tokens, long long tokens_per_workgroup,
+                                                                            int heads, Strides strides) {
+    constexpr int KSTEPS = HEAD / 16;
+    constexpr int BLOCKS = SLICE / 32;
+    constexpr int PIECES = HEAD * SLICE / 8 / THREADS;   // 16-byte pieces of the weight slice per thread
+    static_assert(4 * TILE * SLICE_PITCH == SLICE_BYTES, "the waves' output rows take the place of the weight");
+    constexpr int XCDS = 8;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[SLICE_BYTES];
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int lane = tid % 64;
+    const int lq = lane % 32;
+    const int g = lane / 32;
+    const unsigned items = gridDim.x / 4;
+    unsigned item, quarter;
+    if (items % XCDS == 0) {
+        quarter = blockIdx.x / XCDS % 4;
+        item = blockIdx.x / XCDS / 4 * XCDS + blockIdx.x % XCDS;
+    } else {
+        quarter = blockIdx.x % 4;
+        item = blockIdx.x / 4;
+    }
+    const int head = item % heads;
+    const long long chunk = item / heads;
+    const int column0 = quarter * SLICE;
+    const long long first = chunk * tokens_per_workgroup + TILE * wave;
+    const long long end = min((chunk + 1) * tokens_per_workgroup, tokens);
+    const bf16_t* x_head = x + head * strides.x_head;
+    auto row_of = [&](long long tile0) { return x_head + min(tile0 + lq, tokens - 1) * strides.x_token; };
+
+    u32x4 next_bits[KSTEPS], pieces[PIECES];
+    const bf16_t* slice = weight + head * strides.w_head + column0;
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) {
+        const int piece = tid + j * THREADS;
+        pieces[j] = *reinterpret_cast<const u32x4*>(slice + piece / (SLICE / 8) * RANK + 8 * (piece % (SLICE / 8)));
+    }
+    // rows past the end repeat the last one
+    fetch_token_row(next_bits, row_of(first), true, g);
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) {
+        const int piece = tid + j * THREADS;
+        *reinterpret_cast<u32x4*>(lds + piece / (SLICE / 8) * SLICE_PITCH + 16 * (piece % (SLICE / 8))) = pieces[j];
+    }
+    __syncthreads();
+    // operands as in mla_absorb_query_kernel
+    const int s = lane % 16;
+    const unsigned char* at = lds + (4 * g + s / 4) * SLICE_PITCH + 32 * (lane / 16 % 2) + 8 * (s % 4);
+    bf16x8 weights[KSTEPS][BLOCKS];
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks) {
+#pragma unroll
+        for (int b = 0; b < BLOCKS; ++b) {
+            const unsigned char* here = at + 16 * ks * SLICE_PITCH + 64 * b;
+            const s16x4 low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((transposing_read_pointer)here);
+            const s16x4 high = __builtin_amdgcn_ds_read_tr16_b64_v4i16((transposing_read_pointer)(here + 8 * SLICE_PITCH));
+            weights[ks][b] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(low, high, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+    }
+    __syncthreads();
+
+    unsigned char* out_rows = lds + wave * TILE * SLICE_PITCH;
+    bf16_t* y_head = y + head * strides.y_head + column0;
+    for (long long tile0 = first; tile0 < end; tile0 += 4 * TILE) {
+        bf16x8 xf[KSTEPS];
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ++ks) {
+            const auto first_pair = __builtin_amdgcn_permlane32_swap(next_bits[ks][0], next_bits[ks][2], false, false);
+            const auto second_pair = __builtin_amdgcn_permlane32_swap(next_bits[ks][1], next_bits[ks][3], false, false);
+            xf[ks] = __builtin_bit_cast(bf16x8, u32x4{first_pair[0], second_pair[0], first_pair[1], second_pair[1]});
+        }
+        if (tile0 + 4 * TILE < end) fetch_token_row(next_bits, row_of(tile0 + 4 * TILE), true, g);
+#pragma unroll
+        for (int pair = 0; pair < BLOCKS; pair += 2) {
+            f32x16 acc[2];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[0][i] = acc[1][i] = 0.f;
+#pragma unroll
+            for (int ks = 0; ks < KSTEPS; ++ks) {
+                acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(weights[ks][pair], xf[ks], acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(weights[ks][pair + 1], xf[ks], acc[1], 0, 0, 0);
+            }
+            // lane holds token lq and columns 32*block + 8*i4 + 4*g .. +3
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+#pragma unroll
+                for (int i4 = 0; i4 < 4; ++i4) {
+                    *reinterpret_cast<u32x2*>(out_rows + lq * SLICE_PITCH + 64 * (pair + b) + 16 * i4 + 8 * g) =
+                        u32x2{pack_bf16(acc[b][4 * i4 + 0], acc[b][4 * i4 + 1]), pack_bf16(acc[b][4 * i4 + 2], acc[b][4 * i4 + 3])};
+                }
+            }
+        }
+        __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): this wave's LDS writes have landed
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int row = 4 * j + lane / 16;   // 256 bytes of four rows an instruction
+            const u32x4 bits = *reinterpret_cast<const u32x4*>(out_rows + row * SLICE_PITCH + 16 * (lane % 16));
+            if (tile0 + row < end) {
+                *reinterpret_cast<u32x4*>(y_head + (tile0 + row) * strides.y_token + 8 * (lane % 16)) = bits;
+            }
+        }
+        __builtin_amdgcn_s_waitcnt(0xc07f);   // the reads are done before the next tile's rows take their place
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
 void check(bool condition, const char* message) {
     if (!condition) throw std::invalid_argument(message);
 }
@@ -409,24 +529,52 @@ int compute_units() {
     return hip_common::compute_units_of_current_device();
 }
 
-// The tokens of a head are cut into chunks, one workgroup each (multiples of the 128 tokens four waves take); every
+bool rows_apart(const bf16_t* y, const bf16_t* x, long long tokens, int heads, const Strides& strides, int x_width, int y_width) {
+    const long long offset = ((long long)reinterpret_cast<uintptr_t>(y) - (long long)reinterpret_cast<uintptr_t>(x)) / 2;
+    return index_math::rows_apart({strides.x_token, strides.x_head, x_width}, {strides.y_token, strides.y_head, y_width}, offset,
+                                  tokens, heads);
+}
+
+template <typename Kernel>
+void launch_few(Kernel kernel, bf16_t* y, const bf16_t* x, const bf16_t* weight, long long tokens, int heads,
+                const Strides& strides, hipStream_t stream) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(4 * heads), (unsigned)((tokens + TILE - 1) / TILE)), dim3(THREADS), 0, stream, y,
+                       x, weight, tokens, strides);
+    HIP_CHECK(hipGetLastError());
+}
+
+// Chunks that fill one to four rounds of two workgroups per compute unit, and of these the shortest schedule: rounds
+// times the cost of a workgroup, which fetches its quarter of the weight in the time of some 128 tokens.
+void launch_slices(bf16_t* y, const bf16_t* x, const bf16_t* weight, long long tokens, int heads, const Strides& strides,
+                   hipStream_t stream) {
+    constexpr long long STAGING_TOKENS = 4 * TILE;
+    constexpr long long GRANULE = 4 * TILE;
+    const long long slots = 2LL * std::max(1, compute_units());
+    long long per_workgroup = 0, best = -1;
+    for (long long rounds = 1; rounds <= 4; ++rounds) {
+        const long long chunks = std::max(1LL, rounds * slots / (4LL * heads));
+        const long long per_chunk = ((tokens + chunks - 1) / chunks + GRANULE - 1) / GRANULE * GRANULE;
+        const long long workgroups = 4LL * heads * ((tokens + per_chunk - 1) / per_chunk);
+        const long long cost = (workgroups + slots - 1) / slots * (STAGING_TOKENS + per_chunk);
+        if (best < 0 || cost < best) {
+            best = cost;
+            per_workgroup = per_chunk;
+        }
+    }
+    const long long chunks = (tokens + per_workgroup - 1) / per_workgroup;
+    check(4 * chunks * heads <= 0x7fffffffLL, "MLA projection: more tokens than the grid allows");
+    hipLaunchKernelGGL(mla_absorb_query_slice_kernel, dim3((unsigned)(4 * chunks * heads)), dim3(THREADS), 0, stream, y, x,
+                       weight, tokens, per_workgroup, heads, strides);
+    HIP_CHECK(hipGetLastError());
+}
+
+// Whole weights in LDS: the tokens of a head are cut into chunks, one workgroup each (multiples of the 128 tokens four waves take); every
 // workgroup stages the head's weight first, which costs it about as long as 128 tokens.  The number of chunks is
 // the one with the shortest schedule: rounds of workgroups over the compute units times the cost of a workgroup
 // (4096 tokens x 128 heads on 256 compute units: two chunks, one round, 138 / 171 us against 145 / 178 us with four).
-template <typename Kernel, typename FewKernel>
-void launch(Kernel kernel, FewKernel few_kernel, long long few_tiles, bf16_t* y, const bf16_t* x, const bf16_t* weight, long long tokens, int heads,
-            const Strides& strides, int x_width, int y_width, hipStream_t stream) {
-    check(heads <= 65535, "MLA projection: more heads than the grid allows");
-    const long long tiles = (tokens + TILE - 1) / TILE;
-    const long long offset = ((long long)reinterpret_cast<uintptr_t>(y) - (long long)reinterpret_cast<uintptr_t>(x)) / 2;
-    const bool apart = index_math::rows_apart({strides.x_token, strides.x_head, x_width}, {strides.y_token, strides.y_head, y_width},
-                                              offset, tokens, heads);
-    if (apart && tiles * heads <= few_tiles) {
-        hipLaunchKernelGGL(few_kernel, dim3((unsigned)(4 * heads), (unsigned)tiles), dim3(THREADS), 0, stream, y, x, weight,
-                           tokens, strides);
-        HIP_CHECK(hipGetLastError());
-        return;
-    }
+template <typename Kernel>
+void launch_whole(Kernel kernel, bf16_t* y, const bf16_t* x, const bf16_t* weight, long long tokens, int heads,
+                  const Strides& strides, hipStream_t stream) {
     constexpr long long STAGING_TOKENS = 4 * TILE;
     const long long units = std::max(1, compute_units());
     const long long most = (tokens + 4 * TILE - 1) / (4 * TILE);
@@ -472,13 +620,21 @@ void mla_absorb_query_dispatch(bf16_t* query_latent, const bf16_t* query_nope, c
     const Strides strides = {query_nope_token_stride, query_nope_head_stride, query_latent_token_stride,
                              query_latent_head_stride, weight_head_stride};
     validate(query_latent, query_nope, weight, tokens, heads, strides, HEAD, RANK);
+    check(heads <= 65535, "MLA projection: more heads than the grid allows");
+    const long long tiles = (tokens + TILE - 1) / TILE;
+    const bool apart = rows_apart(query_latent, query_nope, tokens, heads, strides, HEAD, RANK);
     static hip_common::OncePerDevice prepared;
     prepared.run([] {
         HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(mla_absorb_query_kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES));
     });
-    launch(mla_absorb_query_kernel, mla_absorb_query_few_kernel, ABSORB_FEW_TILES, query_latent, query_nope, weight, tokens, heads, strides, HEAD,
-           RANK, stream);
+    if (!apart || tokens * heads * (2LL * RANK) > SLICE_RESULT_BYTES) {
+        launch_whole(mla_absorb_query_kernel, query_latent, query_nope, weight, tokens, heads, strides, stream);
+    } else if (tiles * heads <= ABSORB_FEW_TILES) {
+        launch_few(mla_absorb_query_few_kernel, query_latent, query_nope, weight, tokens, heads, strides, stream);
+    } else {
+        launch_slices(query_latent, query_nope, weight, tokens, heads, strides, stream);
+    }
 }
 
 void mla_unabsorb_output_dispatch(bf16_t* output, const bf16_t* output_latent, const bf16_t* weight, long long tokens,
@@ -488,13 +644,19 @@ void mla_unabsorb_output_dispatch(bf16_t* output, const bf16_t* output_latent, c
     const Strides strides = {output_latent_token_stride, output_latent_head_stride, output_token_stride,
                              output_head_stride, weight_head_stride};
     validate(output, output_latent, weight, tokens, heads, strides, RANK, HEAD);
+    check(heads <= 65535, "MLA projection: more heads than the grid allows");
+    const long long tiles = (tokens + TILE - 1) / TILE;
+    const bool apart = rows_apart(output, output_latent, tokens, heads, strides, RANK, HEAD);
     static hip_common::OncePerDevice prepared;
     prepared.run([] {
         HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(mla_unabsorb_output_kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES));
     });
-    launch(mla_unabsorb_output_kernel, mla_unabsorb_output_few_kernel, UNABSORB_FEW_TILES, output, output_latent, weight, tokens, heads, strides,
-           RANK, HEAD, stream);
+    if (apart && tiles * heads <= UNABSORB_FEW_TILES) {
+        launch_few(mla_unabsorb_output_few_kernel, output, output_latent, weight, tokens, heads, strides, stream);
+        return;
+    }
+    launch_whole(mla_unabsorb_output_kernel, output, output_latent, weight, tokens, heads, strides, stream);
 }
 
 }  // namespace dscuda
