@@ -236,6 +236,22 @@ struct TileReadMath {
     }
 };
 
+// ---- absorbed prefill forward with few rows ------------------------------------------
+// 32 or 64 rows a workgroup (returned: 1, 2) where 64 rows are at most one round of the compute units.  64 rows take
+// longer a unit of 32 keys, 32 rows may take two rounds, whose second pays a workgroup's start and end again; the
+// sums (10 ns, from the times below) decide.  Forward in us, 32 / 64 rows: 100 tokens x 128 heads 14.5 / 12.1, 120 x 128
+// 15.5 / 12.9, 250 x 64 18.8 / 16.9, 200 x 64 16.1 / 15.2, 3 x 300 x 16 22.2 / 18.3, 8 x 250 x 8 23.5 / 17.2, 500 x 32
+// 25.5 / 24.4; 400 x 32 20.4 / 21.3, 300 x 32 15.6 / 17.8, 1000 x 16 38.6 / 39.4, 700 x 16 25.1 / 29.2, 2000 x 8 65 / 70.
+DSCUDA_HOST_DEVICE inline int narrow_forward_row_blocks(int sequence_length, int heads, long long batch, int compute_units) {
+    const long long blocks = ((long long)sequence_length * heads + 31) / 32 * batch;
+    if (blocks <= compute_units) return 1;
+    const long long keys = (sequence_length + 31LL) / 32;   // units of the longest walk
+    const long long longest = 700 + 80 * keys;
+    // the shortest walks of the first round and the longest of the second, one after the other
+    const long long second = 1300 + 160 * keys * (blocks - compute_units) / blocks;
+    return (longest > second ? longest : second) <= 900 + 94 * keys ? 1 : 2;
+}
+
 // ---- work order of the persistent forward kernel ------------------------------
 struct ForwardItem {
     int batch_head;
