@@ -97,7 +97,7 @@ def measure(device, event_time_ms, q, k, v, scale, out, lse, steps=40, warmup=15
         flops = pairs * 2 * (3 * 576 + 2 * 512)   # S, dP, dV (512), dQ and dK (576): the five products
         results["mla_absorbed_backward_T4096_H128"] = {"ms": ms, "tflops": flops / ms / 1e9,
                                                        "frac_of_bf16_peak": flops / ms / 1e9 / PEAK_BF16_TFLOPS, "flops": flops,
-                                                       "entry": "dscuda_mla_backward", "data": "synthetic, GPU generator"}
+                                                       "entry": "dscuda_mla_backward_workspace", "data": "synthetic, GPU generator"}
         del ql, qr, latent, kr, dout_a, aout, alse, agrads
     except Exception as error:
         results["mla_absorbed_T4096_H128"] = {"error": str(error)}
