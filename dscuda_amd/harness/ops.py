@@ -135,6 +135,8 @@ def mla_prefill_backward(dout, out, lse, query, key, value, scale, workspace=Non
     lib = mla_library()
     if workspace is None:
         workspace = mla_prefill_backward_workspace(b, s, h, dqk, dv, query.device)
+    else:
+        _require_cuda(workspace)
     if grads is None:
         grads = (torch.empty_like(query), torch.empty_like(key), torch.empty_like(value))
     checked(lib.lib, "mla", lib.prefill_backward(
@@ -176,6 +178,8 @@ def mla_backward(dout, out, lse, query_latent, query_rope, kv_latent, key_rope, 
         grads = tuple(torch.empty_like(x) for x in (query_latent, query_rope, kv_latent, key_rope))
     if workspace is None:
         workspace = mla_backward_workspace(b, t, h, c, r, query_latent.device)
+    else:
+        _require_cuda(workspace)
     lib = mla_library()
     kept = (None, 0) if workspace is None else (workspace.data_ptr(), workspace.numel() * workspace.element_size() // 4)
     checked(lib.lib, "mla", lib.backward_workspace(
@@ -201,6 +205,8 @@ def mla_decode(packed_query, paged_cache, block_table, lengths, scale, splits=8,
     device = packed_query.device
     if workspace is None:
         workspace = mla_decode_workspace(b, h, splits, rank, device)
+    else:
+        _require_cuda(workspace)
     out = torch.empty(b, 1, h, rank, device=device, dtype=torch.bfloat16) if out is None else out
     lse = torch.empty(b, h, 1, device=device, dtype=torch.float32) if lse is None else lse
     lib = mla_library()
@@ -241,6 +247,8 @@ def mla_decode_planned(packed_query, paged_cache, block_table, lengths, plan, sc
     device = packed_query.device
     if workspace is None:
         workspace = mla_decode_workspace(b, h, splits, rank, device)
+    else:
+        _require_cuda(workspace)
     out = torch.empty(b, 1, h, rank, device=device, dtype=torch.bfloat16) if out is None else out
     lse = torch.empty(b, h, 1, device=device, dtype=torch.float32) if lse is None else lse
     lib = mla_library()
@@ -343,6 +351,8 @@ def flash_backward(dout, out, lse, query, key, value, scale, workspace=None, gra
     lib = flash_library()
     if workspace is None:
         workspace = flash_backward_workspace(b, t, hq, hkv, d, query.device)
+    else:
+        _require_cuda(workspace)
     if grads is None:
         grads = (torch.empty_like(query), torch.empty_like(key), torch.empty_like(value))
     checked(lib.lib, "flash", lib.backward(
