@@ -1497,6 +1497,9 @@ void mla_absorbed_backward_set_key_interval_tiles(int tiles) {
 
 namespace {
 
+// more workgroups of 32 rows than a grid has
+bool exceeds_grid(int batch_size, long long rows) { return (rows + TILE - 1) / TILE > 0x7fffffffLL / batch_size; }
+
 // The whole batch, or as many batch elements as `kept_gradients` has room for (nullptr: dS is not kept).
 void backward_of_batch(bf16_t* query_latent_gradient, bf16_t* query_rope_gradient,
                                     bf16_t* kv_latent_gradient, bf16_t* key_rope_gradient,
@@ -1608,6 +1611,10 @@ void backward_of_batch(bf16_t* query_latent_gradient, bf16_t* query_rope_gradien
 }  // namespace
 
 std::size_t mla_absorbed_backward_workspace_bytes(int batch_size, int sequence_length, int heads) {
+    const long long rows = (long long)sequence_length * heads;
+    // a call that is refused, and dS (at least two bytes per pair of a row and half the keys) beyond the limit: the
+    // sizes below are formed in 64 bits
+    if (exceeds_grid(batch_size, rows) || heads > (1 << 30) || rows > KEPT_BYTES_LIMIT / sequence_length) return 0;
     if (index_math::short_backward(batch_size, sequence_length, heads) &&
         index_math::short_without_workspace(batch_size, sequence_length, heads)) {
         return 0;
@@ -1625,8 +1632,7 @@ void mla_absorbed_backward_dispatch(bf16_t* query_latent_gradient, bf16_t* query
                                     const bf16_t* key_rope, void* workspace, std::size_t workspace_bytes, int batch_size,
                                     int sequence_length, int heads, float scale, hipStream_t stream) {
     const long long rows = (long long)sequence_length * heads;
-    const long long row_blocks = (rows + TILE - 1) / TILE;
-    if (row_blocks * batch_size > 0x7fffffffLL) {
+    if (exceeds_grid(batch_size, rows)) {
         throw std::invalid_argument("MLA backward: batch*tokens*heads exceeds the grid limit");
     }
     if (reinterpret_cast<uintptr_t>(query_latent_gradient) % 16 != 0 ||

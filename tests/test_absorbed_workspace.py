@@ -2,6 +2,9 @@
 on the host, and on the GPU the gradients with and without one at the edges of tiles, blocks and items."""
 
 import ctypes
+import subprocess
+import sys
+from pathlib import Path
 
 import pytest
 import torch
@@ -38,6 +41,20 @@ def test_size_is_zero_or_bounded():
     assert elements(1, 300, 4) == 0                       # P and dS are kept in the query gradients
     assert elements(1, 16384, 128) == 0                   # dS of one batch element beyond 4 GiB: formed twice instead
     assert 0 < elements(64, 4096, 32) * 4 <= (4 << 30) + (1 << 30)
+
+
+@pytest.mark.parametrize("batch,tokens,heads", [
+    (1, 1 << 30, 1 << 30), (1, 2**31 - 1, 2**31 - 1), (2**31 - 1, 2**31 - 1, 2**31 - 1), (1, 2**31 - 1, 31),
+    (2**31 - 1, 1, 33), (1, 1, 2**31 - 1)])
+def test_size_of_calls_beyond_any_memory(batch, tokens, heads):
+    """Arithmetic that leaves 64 bits, or a grid that the call refuses: no size, and in a process of its own because a
+    division by a size of zero ends it."""
+    code = ("import ctypes\nfrom dscuda_amd.harness.common import I, bind, library\n"
+            "query = bind(library('mla'), 'dscuda_mla_backward_workspace_elements', [I] * 5, ctypes.c_size_t)\n"
+            f"print(query({batch}, {tokens}, {heads}, 512, 64))")
+    result = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300,
+                            cwd=Path(__file__).resolve().parents[1])
+    assert (result.returncode, result.stdout.strip()) == (0, "0"), (result.returncode, result.stdout, result.stderr[-500:])
 
 
 # rows that end inside a row tile, a 64- and a 128-row workgroup; key blocks of 64 cut at 1, 32, 33 keys; one head, and
