@@ -573,8 +573,6 @@ struct KeptGradients {
     int key_tiles;
 
     DSCUDA_HOST_DEVICE long long bytes() const { return visits.per_batch() * key_tiles * BLOCK_BYTES; }
-    // first row tile that visits the key block of `tile`
-    DSCUDA_HOST_DEVICE int first_row_tile(int tile) const { return visits.first_tile(tile / key_tiles); }
     DSCUDA_HOST_DEVICE long long at(int tile, int row_tile) const {
         const int block = tile / key_tiles;
         const long long visit = visits.before(block) + row_tile - visits.first_tile(block);

@@ -85,7 +85,7 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
     // A wave requests key rows 4*wave .. +3 of the wide tile (1 KB an instruction), waves 0 .. 3 also eight rows of the narrow one, and 1 KB,
     // half a row tile, of dS: every wave at GROUP = 2, waves 4 .. 7 at GROUP = 1.  Keys past the end repeat the last
     // one (their dS is zero), row tiles past the end repeat the last one (their results are not stored), and a tile
-    // that does not see the keys yet reads what precedes its blocks and is left out below.
+    // that does not see the keys yet may read what precedes its blocks and is left out below.
     const unsigned lds_base = lds_offset_of(lds);
     const int ds_part = GROUP == 1 ? wave - 4 : wave;
     const int ds_row_tile = min(first_row_tile + max(ds_part, 0) / 2, kept.visits.row_tiles - 1);
@@ -143,7 +143,10 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
             for (int j = 0; j < LATENT_BLOCKS; ++j) sum[t][j][i] = 0.f;
         }
     }
-    for (int tile = 0; tile < tiles; ++tile) {
+    // One key tile; the wave's row tiles from FIRST on see it.  Those before are left out, not multiplied by zeros: a key
+    // that is not finite would reach rows of earlier tokens.
+    auto step = [&](int tile, auto first_tag) {
+        constexpr int FIRST = decltype(first_tag)::value;
         const int behind = min(tiles - 1 - tile, AHEAD - 1);   // tiles that may stay in flight
         if (behind == 0) {
             wait_for_all_but(std::integral_constant<int, 0>{});
@@ -154,38 +157,48 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
         }
         workgroup_barrier();   // the tile is there, and the stage of the tile before has been read
         if (tile + AHEAD < tiles) request_tile(tile + AHEAD);
-        const unsigned char* stage = lds + tile % L::STAGES * L::STAGE_BYTES;
-        const int first_seen = kept.first_row_tile(tile);
-        unrolled<0, 2>([&](auto tag) {
-            constexpr int N = decltype(tag)::value;   // 16-key step
-            auto fragment = [&](unsigned low_at, unsigned high_at) {
-                const s16x4 low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((transposing_read_pointer)(stage + low_at));
-                const s16x4 high = __builtin_amdgcn_ds_read_tr16_b64_v4i16((transposing_read_pointer)(stage + high_at));
-                return __builtin_bit_cast(bf16x8, __builtin_shufflevector(low, high, 0, 1, 2, 3, 4, 5, 6, 7));
-            };
-            bf16x8 ds[GROUP];
+        if constexpr (FIRST < GROUP) {
+            const unsigned char* stage = lds + tile % L::STAGES * L::STAGE_BYTES;
+            unrolled<0, 2>([&](auto tag) {
+                constexpr int N = decltype(tag)::value;   // 16-key step
+                auto fragment = [&](unsigned low_at, unsigned high_at) {
+                    const s16x4 low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((transposing_read_pointer)(stage + low_at));
+                    const s16x4 high = __builtin_amdgcn_ds_read_tr16_b64_v4i16((transposing_read_pointer)(stage + high_at));
+                    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(low, high, 0, 1, 2, 3, 4, 5, 6, 7));
+                };
+                bf16x8 ds[GROUP];
 #pragma unroll
-            for (int t = 0; t < GROUP; ++t) {
-                const unsigned at = ds_at + t * index_math::KeptGradients::BLOCK_BYTES + 1024 * N;
-                ds[t] = fragment(at, at + 512);
-                if (first_row_tile + wave_row_tile + t < first_seen) ds[t] = __builtin_bit_cast(bf16x8, u32x4{0, 0, 0, 0});
-            }
-#pragma unroll
-            for (int j = 0; j < LATENT_BLOCKS; ++j) {
-                const bf16x8 columns = fragment(wide_at[0][j] + 16 * N * L::WIDE_ROW, wide_at[1][j] + 16 * N * L::WIDE_ROW);
-#pragma unroll
-                for (int t = 0; t < GROUP; ++t) {
-                    sum[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(columns, ds[t], sum[t][j], 0, 0, 0);
+                for (int t = FIRST; t < GROUP; ++t) {
+                    const unsigned at = ds_at + t * index_math::KeptGradients::BLOCK_BYTES + 1024 * N;
+                    ds[t] = fragment(at, at + 512);
                 }
-            }
-            if (sums_rope) {
-                const bf16x8 columns = fragment(narrow_at[0] + 16 * N * L::NARROW_ROW, narrow_at[1] + 16 * N * L::NARROW_ROW);
-                bf16x8 own = ds[0];
-                if (GROUP > 1 && rope_tile == 1) own = ds[GROUP - 1];
-                rope_sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(columns, own, rope_sum, 0, 0, 0);
-            }
-        });
+#pragma unroll
+                for (int j = 0; j < LATENT_BLOCKS; ++j) {
+                    const bf16x8 columns = fragment(wide_at[0][j] + 16 * N * L::WIDE_ROW, wide_at[1][j] + 16 * N * L::WIDE_ROW);
+#pragma unroll
+                    for (int t = FIRST; t < GROUP; ++t) {
+                        sum[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(columns, ds[t], sum[t][j], 0, 0, 0);
+                    }
+                }
+                if (sums_rope && rope_tile >= FIRST) {
+                    const bf16x8 columns = fragment(narrow_at[0] + 16 * N * L::NARROW_ROW, narrow_at[1] + 16 * N * L::NARROW_ROW);
+                    bf16x8 own = ds[FIRST];
+                    if (GROUP > 1 && rope_tile == 1) own = ds[GROUP - 1];
+                    rope_sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(columns, own, rope_sum, 0, 0, 0);
+                }
+            });
+        }
+    };
+    // key tile t is seen from row 32 * t * heads on, the first row of row tile t * heads
+    const int wave_tile = first_row_tile + wave_row_tile;
+    const int seen_by_all = min(wave_tile / heads + 1, tiles);
+    int tile = 0;
+    for (; tile < seen_by_all; ++tile) step(tile, std::integral_constant<int, 0>{});
+    if constexpr (GROUP == 2) {
+        const int seen_by_second = min((wave_tile + 1) / heads + 1, tiles);
+        for (; tile < seen_by_second; ++tile) step(tile, std::integral_constant<int, 1>{});
     }
+    for (; tile < tiles; ++tile) step(tile, std::integral_constant<int, GROUP>{});
 
     // A lane holds row lq of its row tiles and columns 32*block + 8*(i/4) + 4*g + i%4: rows through LDS, so that a store
     // instruction writes whole lines

@@ -93,3 +93,36 @@ def test_gradients_with_and_without(cuda, batch, tokens, heads, interval_tiles):
     for run in runs:
         for name, actual, reference in zip(("dq_latent", "dq_rope", "dlatent", "dk_rope"), run, expected):
             assert_close_bf16(name, actual.cpu(), reference)
+
+
+# 128 rows a workgroup (two row tiles a wave), 64 rows, 64 rows and half the columns; 64-key blocks by the library's own
+# choice and forced
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,tokens,heads,interval_tiles", [
+    (32, 1000, 1, 0), (16, 700, 3, 0), (20, 850, 1, 0), (2, 450, 3, 0), (32, 1000, 1, 9), (20, 850, 1, 9), (2, 450, 3, 9)])
+def test_keys_that_are_not_finite_stay_with_the_rows_that_see_their_tile(cuda, batch, tokens, heads, interval_tiles):
+    """A row that sees none of 32 keys gets the same query gradient whatever those keys hold."""
+    from dscuda_amd.harness import ops
+    g = torch.Generator(device=cuda).manual_seed(7)
+
+    def randn(*shape, factor=0.25):
+        return (torch.randn(shape, device=cuda, generator=g) * factor).bfloat16()
+
+    ql, qr = randn(batch, tokens, heads, 512), randn(batch, tokens, heads, 64)
+    latent, kr, dout = randn(batch, tokens, 512), randn(batch, tokens, 64), randn(batch, tokens, heads, 512, factor=0.1)
+    scale = configs.c_float(576 ** -0.5)
+    out, lse = ops.mla_forward(ql, qr, latent, kr, scale)
+    announce("mla_backward, keys not finite", dict(B=batch, T=tokens, H=heads, tiles=interval_tiles))
+    ops.mla_backward_set_key_interval_tiles(interval_tiles)
+    try:
+        assert ops.mla_backward_workspace(batch, tokens, heads, device=cuda) is not None
+        expected = ops.mla_backward(dout, out, lse, ql, qr, latent, kr, scale)[:2]
+        for key in (tokens // 64 * 32 + 9, tokens // 64 * 32 + 41):   # an even and an odd tile of keys
+            latent_changed, kr_changed = latent.clone(), kr.clone()
+            latent_changed[:, key], kr_changed[:, key] = float("inf"), float("nan")
+            actual = ops.mla_backward(dout, out, lse, ql, qr, latent_changed, kr_changed, scale)[:2]
+            for name, a, b in zip(("dq_latent", "dq_rope"), actual, expected):
+                assert torch.equal(a[:, :key // 32 * 32], b[:, :key // 32 * 32]), (name, key)
+                assert torch.isnan(a[:, key:].float()).all(), (name, key)
+    finally:
+        ops.mla_backward_set_key_interval_tiles(0)
