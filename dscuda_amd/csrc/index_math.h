@@ -687,7 +687,7 @@ constexpr int WORKSPACE_ROUNDS = 3;   // that a workspace has slots for; long in
 DSCUDA_HOST_DEVICE inline int key_interval_fit(int sequence_length, int heads, long long batch, long long slots,
                                                int compute_units, int key_tiles) {
     const long long visits = key_visits(sequence_length, heads, key_tiles).per_batch() * batch;
-    if (visits < (heads < 16 ? 5LL : 10LL) * compute_units) return 0;
+    if (slots <= 0 || visits < (heads < 16 ? 5LL : 10LL) * compute_units) return 0;
     const long long row_tiles = ((long long)sequence_length * heads + 31) / 32;
     long long best = 0, best_cost = 0;
     for (int rounds = 1; rounds <= MOST_ROUNDS; ++rounds) {

@@ -417,6 +417,25 @@ void check_key_interval_choice() {
     }
 }
 
+// where dS is kept: the items of the interval length the fit picks have a slot each, and no slots give no items
+void check_key_interval_fit() {
+    for (int heads : {1, 3, 8, 16, 128}) {
+        for (int tokens : {1, 64, 1000, 4096}) {
+            for (int batch : {1, 3, 300}) {
+                for (int units : {8, 256}) {
+                    EXPECT(key_interval_fit(tokens, heads, batch, 0, units, 2) == 0, "no slots, T=%d H=%d B=%d", tokens, heads, batch);
+                    for (long long slots : {1LL, 100LL, 768LL, 100000LL}) {
+                        const int length = key_interval_fit(tokens, heads, batch, slots, units, 2);
+                        if (length == 0) continue;
+                        const long long items = key_intervals(tokens, heads, length, 2).items() * batch;
+                        EXPECT(items <= slots, "items %lld, slots %lld, T=%d H=%d B=%d units %d", items, slots, tokens, heads, batch, units);
+                    }
+                }
+            }
+        }
+    }
+}
+
 // ---- decode: the ranges partition the list of positions, their lengths differ by at most one, every tile of every
 // sequence is computed by exactly one range, and (range, sequence) pairs that hold part of a sequence own distinct slots
 void check_decode_ranges() {
@@ -841,6 +860,7 @@ int main() {
     check_key_visits();
     check_key_intervals();
     check_key_interval_choice();
+    check_key_interval_fit();
     check_decode_ranges();
     check_decode_layout();
     check_rows_apart();
