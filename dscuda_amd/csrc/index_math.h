@@ -734,6 +734,35 @@ DSCUDA_HOST_DEVICE inline long long key_gradient_ranges(long long total, long lo
     return (longest < row_tiles || blocks > compute_units) ? ranges : 0;
 }
 
+// ---- absorbed backward where dS is kept: short walks ----------------------------------
+// A range that runs from one key block into the next ends one walk and begins another, and partial results take one launch
+// more (a range over the border costs some 6 us: 6 x 58 x 8 30, 6 x 64 x 8 26).  Ranges of two visits, which every call of at
+// most two a compute unit has, do not cross where the blocks' walks are even.
+DSCUDA_HOST_DEVICE inline bool ranges_stay_in_blocks(const KeyVisits& visits, long long batch, int compute_units) {
+    if (visits.per_batch() * batch > 2LL * compute_units) return false;
+    return visits.key_blocks * batch == 1 || (visits.row_tiles % 2 == 0 && (visits.key_blocks == 1 || visits.heads % 2 == 0));
+}
+
+// Whether a workgroup walks a key block from its first row tile to its last, writes its gradients itself and there is no
+// reduction, or the walks are cut into ranges.  In steps of a walk, fitted to 6100 shapes of up to 60000 rows (the choice
+// costs 0.3 % against the better of the two): beginning and end of a walk 7, the reduction 3.  Backward in us, cut /
+// whole: 512 x 1 token x 1 head 38 / 25, 2000 x 1 x 1 125 / 82, 128 x 5 x 16 37 / 30, 300 x 158 x 1 180 / 151, 64 x 49 x 5 40 / 36;
+// 1 x 142 x 40 36 / 227, 8 x 121 x 16 46 / 98, 16 x 21 x 16 31.0 / 29.6.
+constexpr int WALK_ENDS = 7;
+constexpr int REDUCTION_STEPS = 3;
+constexpr int SHORT_WALK = 12;   // row tiles up to which items of 64-key blocks are never the better cut (300 x 158 x 1 180)
+
+DSCUDA_HOST_DEVICE inline bool whole_key_walks(int sequence_length, int heads, long long batch, int compute_units) {
+    const KeyVisits visits = key_visits(sequence_length, heads);
+    const long long total = visits.per_batch() * batch, blocks = (long long)visits.key_blocks * batch;
+    const long long ranges = key_gradient_ranges(total, blocks, visits.row_tiles, (blocks + compute_units) * KEY_PARTIAL_BYTES, compute_units);
+    if (visits.row_tiles <= 2 || ranges == 0) return true;
+    const long long whole = blocks <= compute_units ? visits.row_tiles + WALK_ENDS
+                                                    : (total + WALK_ENDS * blocks) / compute_units + visits.row_tiles / 2;
+    const long long crossings = ranges_stay_in_blocks(visits, batch, compute_units) ? 0 : blocks > ranges ? blocks / ranges : 1;
+    return whole <= (total + ranges - 1) / ranges + WALK_ENDS * (1 + crossings) + REDUCTION_STEPS;
+}
+
 // ---- absorbed backward of short sequences: where P is kept ------------------------
 // Row `row` = token * heads + head of a batch element with `blocks` blocks of 32 tokens (the last one possibly short)
 // keeps dS of key block b (32 keys, 64 bytes) in chunk b of its own 16 chunks of the latent query gradient, b = 0 ..
@@ -760,11 +789,19 @@ DSCUDA_HOST_DEVICE inline bool short_backward(long long batch, int tokens, int h
     return heads < 16 || rows * batch * tokens <= (heads <= 20 ? 2000000 : 1600000);
 }
 
-// Which of them still do where a workspace could hold dS and the slots of ranges: one launch less, but key gradients that
-// read 64 bytes a row. Backward, P and dS kept / ranges (us): 100 x 8 24 / 28, 300 x 4 30 / 31, 512 x 4 40 / 43, 300 x 8 36 / 39;
-// 3 x 256 x 4 33 / 32, 512 x 6 46 / 45, 512 x 8 50 / 46, 64 x 32 28 / 24, 200 x 32 53 / 41, 480 x 16 77 / 53, 8 x 338 x 3 63 / 49.
+// Which of them still do where a workspace could hold dS: those of a few hundred visits whose key blocks are neither short
+// walks (whole_key_walks) nor cut into ranges that stay inside them.  Backward in us, P and dS kept / dS in a workspace:
+// 6 x 58 x 8 24 / 30, 3 x 121 x 8 27 / 34, 9 x 26 x 11 22 / 28, 1 x 49 x 17 23 / 27; 1 x 157 x 32 46 / 41;
+// taken by the workspace form: 2 x 219 x 20 53 / 43, 8 x 338 x 3 63 / 49, 512 x 8 50 / 46, 64 x 32 28 / 24, 32 x 64 x 4 34 / 29,
+// 12 x 2 x 17 20 / 15, 6 x 60 x 32 38 / 41, 9 x 168 x 4 39 / 43.
 DSCUDA_HOST_DEVICE inline bool short_without_workspace(long long batch, int tokens, int heads) {
-    return heads < 16 && (long long)tokens * heads * batch <= 2500;
+    const KeyVisits visits = key_visits(tokens, heads);
+    const long long blocks = (long long)visits.key_blocks * batch;
+    if (visits.row_tiles <= 2 || visits.per_batch() * batch > 512) return false;
+    if (ranges_stay_in_blocks(visits, batch, 256) && (heads > 4 || visits.row_tiles <= 5 || blocks > 16)) return false;
+    if (visits.row_tiles <= 5) return blocks <= 12 && heads <= 10;
+    if (visits.row_tiles <= 8) return blocks <= 20;
+    return visits.row_tiles > 12 || blocks <= 32;
 }
 
 DSCUDA_HOST_DEVICE inline bool kept_in_rope(int token_block, int blocks) { return token_block == blocks - 1; }

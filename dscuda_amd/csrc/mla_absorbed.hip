@@ -1530,7 +1530,7 @@ void backward_of_batch(bf16_t* query_latent_gradient, bf16_t* query_rope_gradien
     const int forced = forced_interval_tiles();
     const bool keeps = kept_gradients != nullptr;
     const int units = device_compute_units();
-    if (forced > 0 || keeps || rows * (2 * RANK + ROPE) * 2 > LARGE_INPUT_BYTES) {
+    if (forced > 0 || (keeps ? visits.row_tiles > index_math::SHORT_WALK : rows * (2 * RANK + ROPE) * 2 > LARGE_INPUT_BYTES)) {
         const long long slots = scratch_bytes / (PAIR * index_math::KEY_PARTIAL_BYTES);
         // (the choice walks the intervals of several lengths: remembered for the shape a thread asked about last)
         struct Choice {
@@ -1564,7 +1564,9 @@ void backward_of_batch(bf16_t* query_latent_gradient, bf16_t* query_rope_gradien
     }
     long long ranges = 0;
     if (interval_length == 0) {
-        ranges = index_math::key_gradient_ranges(total, blocks, visits.row_tiles, scratch_bytes, device_compute_units());
+        if (!keeps || !index_math::whole_key_walks(sequence_length, heads, batch_size, units)) {
+            ranges = index_math::key_gradient_ranges(total, blocks, visits.row_tiles, scratch_bytes, units);
+        }
         grid = ranges > 0 ? ranges : blocks;
     }
 

@@ -436,6 +436,42 @@ void check_key_interval_fit() {
     }
 }
 
+// where dS is kept: calls whose key blocks are walked whole, and short calls that stay without a workspace
+void check_kept_routes() {
+    struct { int batch, tokens, heads, whole; } walks[] = {
+        {512, 1, 1, 1}, {2000, 1, 1, 1}, {128, 5, 16, 1}, {300, 158, 1, 1}, {64, 49, 5, 1}, {1, 33, 2, 1}, {5000, 16, 16, 1},
+        {1, 142, 40, 0}, {8, 121, 16, 0}, {1, 513, 8, 0}, {1, 600, 4, 0}, {4, 96, 8, 0}, {1, 4096, 128, 0},
+    };
+    for (const auto& c : walks) {
+        EXPECT(whole_key_walks(c.tokens, c.heads, c.batch, 256) == (c.whole != 0), "whole walks B=%d T=%d H=%d", c.batch, c.tokens, c.heads);
+    }
+    struct { int batch, tokens, heads, without; } calls[] = {
+        {6, 58, 8, 1}, {3, 121, 8, 1}, {9, 26, 11, 1}, {1, 49, 17, 1}, {1, 300, 4, 1},
+        {2, 219, 20, 0}, {1, 187, 32, 0}, {8, 338, 3, 0}, {24, 35, 3, 0}, {1, 512, 8, 0}, {1, 64, 32, 0}, {32, 64, 4, 0}, {12, 2, 17, 0},
+    };
+    for (const auto& c : calls) {
+        EXPECT(short_backward(c.batch, c.tokens, c.heads), "short B=%d T=%d H=%d", c.batch, c.tokens, c.heads);
+        EXPECT(short_without_workspace(c.batch, c.tokens, c.heads) == (c.without != 0), "short without workspace B=%d T=%d H=%d", c.batch,
+               c.tokens, c.heads);
+    }
+    // what ranges_stay_in_blocks says of the ranges themselves: no range holds visits of two key blocks
+    for (int heads : {1, 2, 3, 8, 17}) {
+        for (int tokens = 1; tokens <= 130; ++tokens) {
+            for (int batch : {1, 2, 5, 40}) {
+                const KeyVisits visits = key_visits(tokens, heads);
+                const long long total = visits.per_batch() * batch, blocks = (long long)visits.key_blocks * batch;
+                const long long ranges = key_gradient_ranges(total, blocks, visits.row_tiles, 1LL << 40, 256);
+                if (ranges == 0 || !ranges_stay_in_blocks(visits, batch, 256)) continue;
+                for (long long block = 0; block < blocks; ++block) {
+                    const long long begin = block / visits.key_blocks * visits.per_batch() + visits.before((int)(block % visits.key_blocks));
+                    EXPECT(wide_range_begin(total, ranges, wide_range_of(total, ranges, begin)) == begin, "B=%d T=%d H=%d block %lld", batch,
+                           tokens, heads, block);
+                }
+            }
+        }
+    }
+}
+
 // ---- decode: the ranges partition the list of positions, their lengths differ by at most one, every tile of every
 // sequence is computed by exactly one range, and (range, sequence) pairs that hold part of a sequence own distinct slots
 void check_decode_ranges() {
@@ -861,6 +897,7 @@ int main() {
     check_key_intervals();
     check_key_interval_choice();
     check_key_interval_fit();
+    check_kept_routes();
     check_decode_ranges();
     check_decode_layout();
     check_rows_apart();
