@@ -682,7 +682,6 @@ DSCUDA_HOST_DEVICE inline int key_interval_choice(int sequence_length, int heads
 // 2048 x 4 137 / 117, 2845 x 4 x 3 583 / 385).
 constexpr int ITEM_OVERHEAD = 12;
 constexpr int MOST_ROUNDS = 12;
-constexpr int WORKSPACE_ROUNDS = 3;   // that a workspace has slots for; long inputs have more in the query gradients
 
 DSCUDA_HOST_DEVICE inline int key_interval_fit(int sequence_length, int heads, long long batch, long long slots,
                                                int compute_units, int key_tiles) {
@@ -706,18 +705,6 @@ DSCUDA_HOST_DEVICE inline int key_interval_fit(int sequence_length, int heads, l
         }
     }
     return (int)best;
-}
-
-// Bytes of slots a workspace should have room for, `batch` elements taken together: the items of WORKSPACE_ROUNDS rounds
-// of the 256 compute units, or a range per unit and the blocks that ranges may share.
-DSCUDA_HOST_DEVICE inline long long workspace_slot_bytes(int sequence_length, int heads, long long batch) {
-    constexpr long long UNITS = 256;
-    const KeyVisits narrow = key_visits(sequence_length, heads, 1);
-    const long long pair_visits = key_visits(sequence_length, heads, 2).per_batch() * batch;
-    const long long items = pair_visits < WORKSPACE_ROUNDS * UNITS ? pair_visits : WORKSPACE_ROUNDS * UNITS;
-    const long long visits = narrow.per_batch() * batch / 2;
-    const long long ranges = (visits < UNITS ? visits : UNITS) + narrow.key_blocks * batch;
-    return (2 * items > ranges ? 2 * items : ranges) * KEY_PARTIAL_BYTES;
 }
 
 // How many ranges the list is cut into when `scratch_bytes` are there for the slots: one per compute unit if the
@@ -761,6 +748,56 @@ DSCUDA_HOST_DEVICE inline bool whole_key_walks(int sequence_length, int heads, l
                                                     : (total + WALK_ENDS * blocks) / compute_units + visits.row_tiles / 2;
     const long long crossings = ranges_stay_in_blocks(visits, batch, compute_units) ? 0 : blocks > ranges ? blocks / ranges : 1;
     return whole <= (total + ranges - 1) / ranges + WALK_ENDS * (1 + crossings) + REDUCTION_STEPS;
+}
+
+// How the key gradients of a call are cut: items of 64-key blocks in intervals of `length` row tiles, or (length 0) ranges of
+// 32-key blocks, or (ranges 0) whole 32-key blocks, and the bytes of slots that takes.
+struct KeyCut {
+    int length;
+    long long items;
+    long long ranges;
+    long long slot_bytes;
+};
+constexpr int KEY_PAIR = 2;   // 32-key tiles of an item
+
+DSCUDA_HOST_DEVICE inline KeyCut key_cut_of_length(int sequence_length, int heads, long long batch, int length) {
+    const KeyIntervals intervals = key_intervals(sequence_length, heads, length, KEY_PAIR);
+    const long long items = intervals.items() * batch;
+    return KeyCut{length, items, 0, intervals.intervals > 1 ? items * KEY_PAIR * KEY_PARTIAL_BYTES : 0};   // one interval: no partial results
+}
+
+DSCUDA_HOST_DEVICE inline KeyCut key_cut_of_ranges(int sequence_length, int heads, long long batch, long long slot_bytes, int compute_units) {
+    const KeyVisits visits = key_visits(sequence_length, heads);
+    const long long blocks = (long long)visits.key_blocks * batch;
+    const long long ranges = key_gradient_ranges(visits.per_batch() * batch, blocks, visits.row_tiles, slot_bytes, compute_units);
+    return KeyCut{0, 0, ranges, ranges > 0 ? (ranges + blocks) * KEY_PARTIAL_BYTES : 0};
+}
+
+// Where dS is kept and there is room for `slot_bytes` of slots.
+DSCUDA_HOST_DEVICE inline KeyCut kept_cut(int sequence_length, int heads, long long batch, long long slot_bytes, int compute_units) {
+    const KeyVisits visits = key_visits(sequence_length, heads, KEY_PAIR);
+    if (visits.row_tiles > SHORT_WALK) {
+        // whole blocks, which take no slots, are as many items as there are blocks, and every cut of them is more
+        const long long blocks = (long long)visits.key_blocks * batch, slots = slot_bytes / (KEY_PAIR * KEY_PARTIAL_BYTES);
+        const int length = key_interval_fit(sequence_length, heads, batch, slots > blocks ? slots : blocks, compute_units, KEY_PAIR);
+        if (length > 0) return key_cut_of_length(sequence_length, heads, batch, length);
+    }
+    if (whole_key_walks(sequence_length, heads, batch, compute_units)) return KeyCut{0, 0, 0, 0};
+    return key_cut_of_ranges(sequence_length, heads, batch, slot_bytes, compute_units);
+}
+
+// The slots that a cut may ask of a workspace where the latent query gradients hold fewer: three rounds of items, more
+// than the blocks and ranges of any call that is cut into ranges.
+constexpr long long WORKSPACE_SLOT_BYTES = 3LL * 256 * KEY_PAIR * KEY_PARTIAL_BYTES;   // 113 MB
+
+DSCUDA_HOST_DEVICE inline long long query_gradient_bytes(int sequence_length, int heads, long long batch) {
+    return (long long)sequence_length * heads * batch * 1024;
+}
+
+// Slots to choose the cut of a call by that has a workspace of the size it asks for.
+DSCUDA_HOST_DEVICE inline long long slot_bytes_of_workspace(int sequence_length, int heads, long long batch) {
+    const long long scratch = query_gradient_bytes(sequence_length, heads, batch);
+    return scratch > WORKSPACE_SLOT_BYTES ? scratch : WORKSPACE_SLOT_BYTES;
 }
 
 // ---- absorbed backward of short sequences: where P is kept ------------------------

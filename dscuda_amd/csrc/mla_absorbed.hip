@@ -1500,14 +1500,50 @@ namespace {
 // more workgroups of 32 rows than a grid has
 bool exceeds_grid(int batch_size, long long rows) { return (rows + TILE - 1) / TILE > 0x7fffffffLL / batch_size; }
 
+static_assert(KeyPairLayout::KEYS == index_math::KEY_PAIR * TILE && RANK * 2 == 1024, "index_math::KeyCut, query_gradient_bytes");
+
+// The cut of the key gradients where there is room for `slot_bytes` of slots.  The choice walks the intervals of several
+// lengths: remembered for the shapes a thread asked about last (a call asks for its groups of batch elements, the last
+// of which may be smaller).
+index_math::KeyCut key_cut(int sequence_length, int heads, int batch_size, long long slot_bytes, int units, bool keeps) {
+    struct Choice {
+        int sequence_length = 0, heads = 0, batch_size = 0, units = 0;
+        bool keeps = false;
+        long long slot_bytes = 0;
+        index_math::KeyCut cut{};
+    };
+    static thread_local Choice chosen[4];
+    static thread_local unsigned next = 0;
+    for (const Choice& choice : chosen) {
+        if (choice.sequence_length == sequence_length && choice.heads == heads && choice.batch_size == batch_size &&
+            choice.units == units && choice.keeps == keeps && choice.slot_bytes == slot_bytes) {
+            return choice.cut;
+        }
+    }
+    index_math::KeyCut cut{};
+    if (keeps) {
+        cut = index_math::kept_cut(sequence_length, heads, batch_size, slot_bytes, units);
+    } else {
+        // Rows that outgrow the caches (query and dO rows of a batch element, 2176 bytes per row): the interval cut
+        // with key blocks of 64 keys (mla_absorbed_key_pair_gradient_kernel)
+        int length = 0;
+        if ((long long)sequence_length * heads * (2 * RANK + ROPE) * 2 > LARGE_INPUT_BYTES) {
+            length = index_math::key_interval_choice(sequence_length, heads, batch_size, slot_bytes / (index_math::KEY_PAIR * index_math::KEY_PARTIAL_BYTES),
+                                                     units, index_math::KEY_PAIR);
+        }
+        cut = length > 0 ? index_math::key_cut_of_length(sequence_length, heads, batch_size, length)
+                         : index_math::key_cut_of_ranges(sequence_length, heads, batch_size, slot_bytes, units);
+    }
+    chosen[next++ % 4] = Choice{sequence_length, heads, batch_size, units, keeps, slot_bytes, cut};
+    return cut;
+}
+
 // The whole batch, or as many batch elements as `kept_gradients` has room for (nullptr: dS is not kept).
-void backward_of_batch(bf16_t* query_latent_gradient, bf16_t* query_rope_gradient,
-                                    bf16_t* kv_latent_gradient, bf16_t* key_rope_gradient,
-                                    const bf16_t* output_gradient, const bf16_t* output, const float* logsumexp,
-                                    const bf16_t* query_latent, const bf16_t* query_rope, const bf16_t* kv_latent,
-                                    const bf16_t* key_rope, unsigned char* kept_gradients, float* partial_slots,
-                                    long long scratch_bytes, int batch_size, int sequence_length, int heads,
-                                    float scale, hipStream_t stream) {
+void backward_of_batch(bf16_t* query_latent_gradient, bf16_t* query_rope_gradient, bf16_t* kv_latent_gradient,
+                       bf16_t* key_rope_gradient, const bf16_t* output_gradient, const bf16_t* output, const float* logsumexp,
+                       const bf16_t* query_latent, const bf16_t* query_rope, const bf16_t* kv_latent, const bf16_t* key_rope,
+                       unsigned char* kept_gradients, float* partial_slots, const index_math::KeyCut& cut, int batch_size,
+                       int sequence_length, int heads, float scale, hipStream_t stream) {
     const long long rows = (long long)sequence_length * heads;
     const long long row_blocks = (rows + TILE - 1) / TILE;
     static hip_common::OncePerDevice prepared;
@@ -1518,57 +1554,13 @@ void backward_of_batch(bf16_t* query_latent_gradient, bf16_t* query_rope_gradien
     });
     // scratch memory until the last launch: delta in the rope query gradients
     float* delta = reinterpret_cast<float*>(query_rope_gradient);
-    const index_math::KeyVisits visits = index_math::key_visits(sequence_length, heads);
-    long long blocks = (long long)visits.key_blocks * batch_size;
-    const long long total = visits.per_batch() * batch_size;
-    // Rows that outgrow the caches (query and dO rows of a batch element, 2176 bytes per row): the interval cut
-    // with key blocks of 64 keys (mla_absorbed_key_pair_gradient_kernel)
-    constexpr int PAIR = KeyPairLayout::KEYS / TILE;
-    int interval_length = 0;
-    int key_tiles = 1;
-    long long grid = 0;
-    const int forced = forced_interval_tiles();
     const bool keeps = kept_gradients != nullptr;
-    const int units = device_compute_units();
-    if (forced > 0 || (keeps ? visits.row_tiles > index_math::SHORT_WALK : rows * (2 * RANK + ROPE) * 2 > LARGE_INPUT_BYTES)) {
-        const long long slots = scratch_bytes / (PAIR * index_math::KEY_PARTIAL_BYTES);
-        // (the choice walks the intervals of several lengths: remembered for the shape a thread asked about last)
-        struct Choice {
-            int sequence_length = -1, heads = -1, batch_size = -1, units = -1, forced = -1, tiles = 0;
-            bool keeps = false;
-            long long slots = 0, items = 0;
-            int key_blocks = 0;
-        };
-        static thread_local Choice last;
-        if (last.sequence_length != sequence_length || last.heads != heads || last.batch_size != batch_size ||
-            last.units != units || last.forced != forced || last.keeps != keeps || last.slots != slots) {
-            last = Choice{sequence_length, heads, batch_size, units, forced, 0, keeps, slots, 0, 0};
-            last.tiles = forced > 0 ? forced
-                         : keeps    ? index_math::key_interval_fit(sequence_length, heads, batch_size, slots, units, PAIR)
-                                    : index_math::key_interval_choice(sequence_length, heads, batch_size, slots, units, PAIR);
-            if (last.tiles > 0) {
-                const index_math::KeyIntervals chosen = index_math::key_intervals(sequence_length, heads, last.tiles, PAIR);
-                last.items = chosen.items() * batch_size;
-                last.key_blocks = chosen.key_blocks;
-            }
-        }
-        const int tiles = last.tiles;
-        const long long items = last.items;
-        // a slot for each item
-        if (tiles > 0 && items <= slots && items <= 0x7fffffffLL) {
-            interval_length = tiles;
-            key_tiles = PAIR;
-            grid = items;
-            blocks = (long long)last.key_blocks * batch_size;
-        }
-    }
-    long long ranges = 0;
-    if (interval_length == 0) {
-        if (!keeps || !index_math::whole_key_walks(sequence_length, heads, batch_size, units)) {
-            ranges = index_math::key_gradient_ranges(total, blocks, visits.row_tiles, scratch_bytes, units);
-        }
-        grid = ranges > 0 ? ranges : blocks;
-    }
+    const int forced = forced_interval_tiles();
+    const int interval_length = cut.length;
+    const long long ranges = cut.ranges;
+    const int key_tiles = interval_length > 0 ? index_math::KEY_PAIR : 1;
+    const long long blocks = (long long)index_math::key_visits(sequence_length, heads, key_tiles).key_blocks * batch_size;
+    const long long grid = interval_length > 0 ? cut.items : ranges > 0 ? ranges : blocks;
 
     hipLaunchKernelGGL(mla_absorbed_row_statistics_kernel, dim3((unsigned)(row_blocks * batch_size)), dim3(THREADS), 0,
                        stream, delta, output_gradient, output, rows * batch_size);
@@ -1610,6 +1602,10 @@ void backward_of_batch(bf16_t* query_latent_gradient, bf16_t* query_rope_gradien
     HIP_CHECK(hipGetLastError());
 }
 
+index_math::KeyCut workspace_cut(int sequence_length, int heads, int batch_size, int units) {
+    return key_cut(sequence_length, heads, batch_size, index_math::slot_bytes_of_workspace(sequence_length, heads, batch_size), units, true);
+}
+
 }  // namespace
 
 std::size_t mla_absorbed_backward_workspace_bytes(int batch_size, int sequence_length, int heads) {
@@ -1624,7 +1620,8 @@ std::size_t mla_absorbed_backward_workspace_bytes(int batch_size, int sequence_l
     const long long element = index_math::kept_gradient_bytes(sequence_length, heads);
     if (element > KEPT_BYTES_LIMIT) return 0;
     const long long group = std::min<long long>(batch_size, KEPT_BYTES_LIMIT / element);
-    return (std::size_t)(element * group + index_math::workspace_slot_bytes(sequence_length, heads, group));
+    const long long slots = workspace_cut(sequence_length, heads, (int)group, 256).slot_bytes;
+    return (std::size_t)(element * group + (slots > index_math::query_gradient_bytes(sequence_length, heads, group) ? slots : 0));
 }
 
 void mla_absorbed_backward_dispatch(bf16_t* query_latent_gradient, bf16_t* query_rope_gradient,
@@ -1651,22 +1648,30 @@ void mla_absorbed_backward_dispatch(bf16_t* query_latent_gradient, bf16_t* query
     }
     unsigned char* kept = group > 0 ? static_cast<unsigned char*>(workspace) : nullptr;
     if (group == 0) group = batch_size;
-    // partial key gradients: behind dS where there is more room than in the latent query gradients
-    const long long left = kept != nullptr ? (long long)workspace_bytes - group * index_math::kept_gradient_bytes(sequence_length, heads) : 0;
+    const long long kept_bytes = kept != nullptr ? group * index_math::kept_gradient_bytes(sequence_length, heads) : 0;
+    const long long left = kept != nullptr ? (long long)workspace_bytes - kept_bytes : 0;
+    const int units = device_compute_units();
+    const int forced = forced_interval_tiles();
     for (long long first = 0; first < batch_size; first += group) {
         const long long row = first * rows;
         const long long elements = std::min<long long>(group, batch_size - first);
-        long long scratch_bytes = elements * rows * RANK * 2;
-        float* partial_slots = reinterpret_cast<float*>(query_latent_gradient + row * RANK);
-        if (left > scratch_bytes) {
-            scratch_bytes = left;
-            partial_slots = reinterpret_cast<float*>(kept + group * index_math::kept_gradient_bytes(sequence_length, heads));
+        // partial key gradients: in the latent query gradients, behind dS where those have no room for them
+        const long long scratch_bytes = index_math::query_gradient_bytes(sequence_length, heads, elements);
+        const long long room = std::max(scratch_bytes, left);
+        index_math::KeyCut cut{};
+        if (forced > 0) cut = index_math::key_cut_of_length(sequence_length, heads, elements, forced);
+        if (cut.length == 0 || cut.items > room / (index_math::KEY_PAIR * index_math::KEY_PARTIAL_BYTES) || cut.items > 0x7fffffffLL) {
+            cut = kept != nullptr ? workspace_cut(sequence_length, heads, (int)elements, units)
+                                  : key_cut(sequence_length, heads, (int)elements, scratch_bytes, units, false);
+            if (cut.slot_bytes > room) cut = key_cut(sequence_length, heads, (int)elements, room, units, kept != nullptr);
         }
+        float* partial_slots = reinterpret_cast<float*>(query_latent_gradient + row * RANK);
+        if (cut.slot_bytes > scratch_bytes) partial_slots = reinterpret_cast<float*>(kept + kept_bytes);
         const long long token = first * sequence_length;
         backward_of_batch(query_latent_gradient + row * RANK, query_rope_gradient + row * ROPE, kv_latent_gradient + token * RANK,
                           key_rope_gradient + token * ROPE, output_gradient + row * RANK, output + row * RANK, logsumexp + row,
                           query_latent + row * RANK, query_rope + row * ROPE, kv_latent + token * RANK, key_rope + token * ROPE,
-                          kept, partial_slots, scratch_bytes, (int)elements, sequence_length, heads, scale, stream);
+                          kept, partial_slots, cut, (int)elements, sequence_length, heads, scale, stream);
     }
 }
 

@@ -27,6 +27,9 @@ extern "C" int backward_ranges(int batch, int tokens, int heads, int compute_uni
 extern "C" int walks_are_cut(int pairs, int tokens, int sharing) {
     return choose_walk_cut(pairs, (tokens + 127) / 128, (tokens + 63) / 64, sharing, 256).part_steps > 0;
 }
+extern "C" long long workspace_slots(int batch, int tokens, int heads) {   // of a call whose dS is kept, in bytes
+    return kept_cut(tokens, heads, batch, slot_bytes_of_workspace(tokens, heads, batch), 256).slot_bytes;
+}
 extern "C" int keeps_scores(int batch, int tokens, int heads) { return short_backward(batch, tokens, heads); }
 """
 
@@ -40,4 +43,6 @@ def rules():
     (directory / "rules.cpp").write_text(SOURCE)
     subprocess.run([compiler, "-std=c++17", "-shared", "-fPIC", f"-I{CSRC}", str(directory / "rules.cpp"), "-o",
                     str(directory / "rules.so")], check=True, timeout=120)
-    return ctypes.CDLL(str(directory / "rules.so"))
+    library = ctypes.CDLL(str(directory / "rules.so"))
+    library.workspace_slots.restype = ctypes.c_longlong
+    return library

@@ -472,6 +472,65 @@ void check_kept_routes() {
     }
 }
 
+// the cut of a call with a workspace of the size it asks for: a slot for each item or each range and block, none where
+// nothing is cut, and never more than the query gradients or WORKSPACE_SLOT_BYTES hold
+void check_kept_cut() {
+    struct { int batch, tokens, heads, length; long long items, ranges; } known[] = {
+        {300, 4096, 1, 128, 19200, 0}, {4096, 33, 16, 17, 4096, 0}, {1, 512, 8, 0, 0, 256}, {1, 513, 8, 0, 0, 256},
+        {512, 1, 1, 0, 0, 0}, {300, 158, 1, 0, 0, 0}, {400, 300, 1, 0, 0, 0}, {271, 352, 2, 22, 1626, 0},
+    };
+    for (const auto& c : known) {
+        const KeyCut cut = kept_cut(c.tokens, c.heads, c.batch, slot_bytes_of_workspace(c.tokens, c.heads, c.batch), 256);
+        EXPECT(cut.length == c.length && cut.items == c.items && cut.ranges == c.ranges, "B=%d T=%d H=%d: length %d, items %lld, ranges %lld",
+               c.batch, c.tokens, c.heads, cut.length, cut.items, cut.ranges);
+    }
+    for (int heads : {1, 2, 3, 8, 16, 40, 128}) {
+        for (int tokens : {1, 33, 64, 97, 300, 513, 1000, 4096}) {
+            for (int batch : {1, 3, 20, 200, 300, 4096}) {
+                if ((long long)batch * tokens * heads > 8000000) continue;
+                const long long room = slot_bytes_of_workspace(tokens, heads, batch);
+                for (long long bytes : {0LL, room / 7, room}) {
+                    const KeyCut cut = kept_cut(tokens, heads, batch, bytes, 256);
+                    EXPECT(cut.slot_bytes <= bytes, "B=%d T=%d H=%d: %lld bytes of slots of %lld", batch, tokens, heads, cut.slot_bytes, bytes);
+                    EXPECT(cut.length == 0 || (cut.items > 0 && cut.ranges == 0), "B=%d T=%d H=%d", batch, tokens, heads);
+                    if (cut.length > 0) {
+                        const bool whole = cut.length >= key_visits(tokens, heads).row_tiles;
+                        EXPECT(cut.slot_bytes == (whole ? 0 : cut.items * 2 * KEY_PARTIAL_BYTES), "B=%d T=%d H=%d", batch, tokens, heads);
+                    }
+                }
+                // all the slots that ranges can use are there
+                const KeyCut cut = kept_cut(tokens, heads, batch, room, 256), more = kept_cut(tokens, heads, batch, 1LL << 50, 256);
+                EXPECT(cut.length > 0 || more.length > 0 || cut.ranges == more.ranges, "B=%d T=%d H=%d: %lld ranges, %lld", batch, tokens, heads,
+                       cut.ranges, more.ranges);
+            }
+        }
+    }
+}
+
+// dS of a call: every (key tile, row tile) that a key block visits has a block of its own inside what the workspace holds
+void check_kept_gradients() {
+    for (int heads : {1, 3, 8, 40, 129}) {
+        for (int tokens : {1, 31, 33, 64, 65, 97, 300}) {
+            for (int key_tiles : {1, 2}) {
+                const KeptGradients kept = kept_gradients(tokens, heads, key_tiles);
+                EXPECT(kept.bytes() <= kept_gradient_bytes(tokens, heads), "T=%d H=%d", tokens, heads);
+                std::vector<int> seen(kept.bytes() / KeptGradients::BLOCK_BYTES, 0);
+                for (int tile = 0; tile < kept.visits.key_blocks * key_tiles; ++tile) {
+                    for (int row_tile = kept.visits.first_tile(tile / key_tiles); row_tile < kept.visits.row_tiles; ++row_tile) {
+                        const long long at = kept.at(tile, row_tile);
+                        const bool inside = at >= 0 && at % KeptGradients::BLOCK_BYTES == 0 && at + KeptGradients::BLOCK_BYTES <= kept.bytes();
+                        EXPECT(inside, "T=%d H=%d: tile %d, row tile %d at %lld", tokens, heads, tile, row_tile, at);
+                        if (inside) ++seen[at / KeptGradients::BLOCK_BYTES];
+                    }
+                    // a row tile that does not see the block yet reads inside the workspace as well
+                    EXPECT(kept.at(tile, 0) >= 0, "T=%d H=%d: tile %d", tokens, heads, tile);
+                }
+                for (int count : seen) EXPECT(count == 1, "T=%d H=%d key tiles %d: a block held %d times", tokens, heads, key_tiles, count);
+            }
+        }
+    }
+}
+
 // ---- decode: the ranges partition the list of positions, their lengths differ by at most one, every tile of every
 // sequence is computed by exactly one range, and (range, sequence) pairs that hold part of a sequence own distinct slots
 void check_decode_ranges() {
@@ -898,6 +957,8 @@ int main() {
     check_key_interval_choice();
     check_key_interval_fit();
     check_kept_routes();
+    check_kept_cut();
+    check_kept_gradients();
     check_decode_ranges();
     check_decode_layout();
     check_rows_apart();

@@ -11,6 +11,7 @@ import torch
 
 from dscuda_amd.harness import configs
 from dscuda_amd.harness.common import I, bind, library
+from dispatch_rules import rules
 from oracle import attention_oracle as oracle
 from parity import announce, assert_close_bf16
 
@@ -27,20 +28,23 @@ def kept_bytes(tokens, heads):
                for size in (1, 2))
 
 
-@pytest.mark.parametrize("batch,tokens,heads", [(1, 513, 8), (3, 700, 5), (1, 65, 128), (2, 4096, 16)])
-def test_size_holds_every_block_and_slot(batch, tokens, heads):
-    row_tiles = -(-tokens * heads // 32)
-    key_blocks = -(-tokens // 32)
-    visits = sum(max(0, row_tiles - heads * block) for block in range(key_blocks)) * batch
-    slots = min(256, visits // 2) + key_blocks * batch   # of ranges: [32 keys][576] floats each
-    assert elements(batch, tokens, heads) * 4 >= batch * kept_bytes(tokens, heads) + slots * 32 * 576 * 4
+@pytest.mark.parametrize("batch,tokens,heads", [
+    (1, 513, 8), (3, 700, 5), (1, 65, 128), (2, 4096, 16), (1, 512, 8), (1, 2048, 128), (1, 4096, 128), (240, 4096, 1),
+    (60, 4096, 4), (4096, 33, 16), (512, 1, 1), (20, 4096, 1), (271, 352, 2)])
+def test_size_holds_every_block_and_the_slots_that_are_used(batch, tokens, heads):
+    """dS, and slots for partial key gradients where the cut of the call needs more than the latent query gradients hold."""
+    slots = rules().workspace_slots(batch, tokens, heads)
+    room = elements(batch, tokens, heads) * 4 - batch * kept_bytes(tokens, heads)
+    assert room == (slots if slots > batch * tokens * heads * 1024 else 0)
+    assert room <= 114_000_000
 
 
 def test_size_is_zero_or_bounded():
     assert elements(1, 0, 8) == 0 and elements(1, 64, 8, rank=256) == 0
     assert elements(1, 300, 4) == 0                       # P and dS are kept in the query gradients
     assert elements(1, 16384, 128) == 0                   # dS of one batch element beyond 4 GiB: formed twice instead
-    assert 0 < elements(64, 4096, 32) * 4 <= (4 << 30) + (1 << 30)
+    for batch, tokens, heads in ((64, 4096, 32), (300, 4096, 1), (2000, 1500, 1), (64, 4096, 4), (100000, 33, 3)):
+        assert 0 < elements(batch, tokens, heads) * 4 <= (4 << 30) + 114_000_000, (batch, tokens, heads)
 
 
 @pytest.mark.parametrize("batch,tokens,heads", [
