@@ -794,6 +794,20 @@ DSCUDA_HOST_DEVICE inline long long query_gradient_bytes(int sequence_length, in
     return (long long)sequence_length * heads * batch * 1024;
 }
 
+// A batch in passes of at most `most` elements, as equal as they can be: pass p has elements first(p) .. first(p + 1) - 1.
+// (64 x 4096 tokens x 4 heads, whose dS allows 63 elements a pass: 17.0 ms with a last pass of one element, 15.5 in halves.)
+struct BatchPasses {
+    long long batch;
+    long long passes;
+
+    DSCUDA_HOST_DEVICE long long first(long long pass) const { return batch * pass / passes; }
+    DSCUDA_HOST_DEVICE long long largest() const { return (batch + passes - 1) / passes; }   // the others have one less, or as many
+};
+
+DSCUDA_HOST_DEVICE inline BatchPasses batch_passes(long long batch, long long most) {
+    return BatchPasses{batch, (batch + most - 1) / most};
+}
+
 // Slots to choose the cut of a call by that has a workspace of the size it asks for.
 DSCUDA_HOST_DEVICE inline long long slot_bytes_of_workspace(int sequence_length, int heads, long long batch) {
     const long long scratch = query_gradient_bytes(sequence_length, heads, batch);

@@ -1503,8 +1503,7 @@ bool exceeds_grid(int batch_size, long long rows) { return (rows + TILE - 1) / T
 static_assert(KeyPairLayout::KEYS == index_math::KEY_PAIR * TILE && RANK * 2 == 1024, "index_math::KeyCut, query_gradient_bytes");
 
 // The cut of the key gradients where there is room for `slot_bytes` of slots.  The choice walks the intervals of several
-// lengths: remembered for the shapes a thread asked about last (a call asks for its groups of batch elements, the last
-// of which may be smaller).
+// lengths: remembered for the shapes a thread asked about last (the passes of a call have two sizes).
 index_math::KeyCut key_cut(int sequence_length, int heads, int batch_size, long long slot_bytes, int units, bool keeps) {
     struct Choice {
         int sequence_length = 0, heads = 0, batch_size = 0, units = 0;
@@ -1606,22 +1605,41 @@ index_math::KeyCut workspace_cut(int sequence_length, int heads, int batch_size,
     return key_cut(sequence_length, heads, batch_size, index_math::slot_bytes_of_workspace(sequence_length, heads, batch_size), units, true);
 }
 
-}  // namespace
+// What a call asks of a workspace: room for dS of the largest pass over the batch, and slots.  No passes: it uses none.
+struct Workspace {
+    index_math::BatchPasses passes{0, 0};
+    long long element_bytes = 0;
+    long long slot_bytes = 0;
 
-std::size_t mla_absorbed_backward_workspace_bytes(int batch_size, int sequence_length, int heads) {
+    long long bytes() const { return passes.passes > 0 ? element_bytes * passes.largest() + slot_bytes : 0; }
+};
+
+Workspace workspace_of(int batch_size, int sequence_length, int heads) {
     const long long rows = (long long)sequence_length * heads;
     // a call that is refused, and dS (at least two bytes per pair of a row and half the keys) beyond the limit: the
     // sizes below are formed in 64 bits
-    if (exceeds_grid(batch_size, rows) || heads > (1 << 30) || rows > KEPT_BYTES_LIMIT / sequence_length) return 0;
+    if (exceeds_grid(batch_size, rows) || heads > (1 << 30) || rows > KEPT_BYTES_LIMIT / sequence_length) return {};
     if (index_math::short_backward(batch_size, sequence_length, heads) &&
         index_math::short_without_workspace(batch_size, sequence_length, heads)) {
-        return 0;
+        return {};
     }
-    const long long element = index_math::kept_gradient_bytes(sequence_length, heads);
-    if (element > KEPT_BYTES_LIMIT) return 0;
-    const long long group = std::min<long long>(batch_size, KEPT_BYTES_LIMIT / element);
-    const long long slots = workspace_cut(sequence_length, heads, (int)group, 256).slot_bytes;
-    return (std::size_t)(element * group + (slots > index_math::query_gradient_bytes(sequence_length, heads, group) ? slots : 0));
+    Workspace workspace;
+    workspace.element_bytes = index_math::kept_gradient_bytes(sequence_length, heads);
+    if (workspace.element_bytes > KEPT_BYTES_LIMIT) return {};
+    workspace.passes = index_math::batch_passes(batch_size, KEPT_BYTES_LIMIT / workspace.element_bytes);
+    for (const long long elements : {workspace.passes.largest(), batch_size / workspace.passes.passes}) {
+        const long long slots = workspace_cut(sequence_length, heads, (int)elements, 256).slot_bytes;
+        if (slots > index_math::query_gradient_bytes(sequence_length, heads, elements)) {
+            workspace.slot_bytes = std::max(workspace.slot_bytes, slots);
+        }
+    }
+    return workspace;
+}
+
+}  // namespace
+
+std::size_t mla_absorbed_backward_workspace_bytes(int batch_size, int sequence_length, int heads) {
+    return (std::size_t)workspace_of(batch_size, sequence_length, heads).bytes();
 }
 
 void mla_absorbed_backward_dispatch(bf16_t* query_latent_gradient, bf16_t* query_rope_gradient,
@@ -1638,23 +1656,24 @@ void mla_absorbed_backward_dispatch(bf16_t* query_latent_gradient, bf16_t* query
         reinterpret_cast<uintptr_t>(query_rope_gradient) % 16 != 0) {
         throw std::invalid_argument("MLA backward: the query gradients must be aligned to 16 bytes");
     }
-    // batch elements whose dS the workspace holds
-    long long group = 0;
-    if (workspace != nullptr && mla_absorbed_backward_workspace_bytes(batch_size, sequence_length, heads) > 0) {
+    const Workspace asked = workspace != nullptr ? workspace_of(batch_size, sequence_length, heads) : Workspace{};
+    long long most = 0;   // batch elements whose dS the workspace holds
+    if (asked.bytes() > 0) {
         if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0) {
             throw std::invalid_argument("MLA backward: the workspace must be aligned to 16 bytes");
         }
-        group = std::min<long long>(batch_size, (long long)workspace_bytes / index_math::kept_gradient_bytes(sequence_length, heads));
+        most = std::min<long long>(asked.passes.largest(), (long long)workspace_bytes / asked.element_bytes);
     }
-    unsigned char* kept = group > 0 ? static_cast<unsigned char*>(workspace) : nullptr;
-    if (group == 0) group = batch_size;
-    const long long kept_bytes = kept != nullptr ? group * index_math::kept_gradient_bytes(sequence_length, heads) : 0;
+    unsigned char* kept = most > 0 ? static_cast<unsigned char*>(workspace) : nullptr;
+    const index_math::BatchPasses passes = index_math::batch_passes(batch_size, most > 0 ? most : batch_size);
+    const long long kept_bytes = most > 0 ? passes.largest() * asked.element_bytes : 0;
     const long long left = kept != nullptr ? (long long)workspace_bytes - kept_bytes : 0;
     const int units = device_compute_units();
     const int forced = forced_interval_tiles();
-    for (long long first = 0; first < batch_size; first += group) {
+    for (long long pass = 0; pass < passes.passes; ++pass) {
+        const long long first = passes.first(pass);
         const long long row = first * rows;
-        const long long elements = std::min<long long>(group, batch_size - first);
+        const long long elements = passes.first(pass + 1) - first;
         // partial key gradients: in the latent query gradients, behind dS where those have no room for them
         const long long scratch_bytes = index_math::query_gradient_bytes(sequence_length, heads, elements);
         const long long room = std::max(scratch_bytes, left);

@@ -507,6 +507,21 @@ void check_kept_cut() {
     }
 }
 
+// passes over a batch: every element once, none more than allowed, sizes that differ by at most one
+void check_batch_passes() {
+    for (long long batch = 1; batch <= 200; ++batch) {
+        for (long long most = 1; most <= batch; ++most) {
+            const BatchPasses passes = batch_passes(batch, most);
+            EXPECT(passes.first(0) == 0 && passes.first(passes.passes) == batch, "batch %lld, most %lld", batch, most);
+            EXPECT(passes.largest() <= most && passes.passes == (batch + most - 1) / most, "batch %lld, most %lld", batch, most);
+            for (long long pass = 0; pass < passes.passes; ++pass) {
+                const long long size = passes.first(pass + 1) - passes.first(pass);
+                EXPECT(size <= passes.largest() && size >= batch / passes.passes, "batch %lld, most %lld: %lld elements", batch, most, size);
+            }
+        }
+    }
+}
+
 // dS of a call: every (key tile, row tile) that a key block visits has a block of its own inside what the workspace holds
 void check_kept_gradients() {
     for (int heads : {1, 3, 8, 40, 129}) {
@@ -959,6 +974,7 @@ int main() {
     check_kept_routes();
     check_kept_cut();
     check_kept_gradients();
+    check_batch_passes();
     check_decode_ranges();
     check_decode_layout();
     check_rows_apart();

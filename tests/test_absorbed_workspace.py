@@ -47,6 +47,14 @@ def test_size_is_zero_or_bounded():
         assert 0 < elements(batch, tokens, heads) * 4 <= (4 << 30) + 114_000_000, (batch, tokens, heads)
 
 
+@pytest.mark.parametrize("batch,tokens,heads,passes", [(64, 4096, 4, 2), (300, 4096, 1, 2), (2000, 1500, 1, 2), (65, 2048, 32, 3)])
+def test_batch_elements_are_taken_in_equal_passes(batch, tokens, heads, passes):
+    """dS beyond 4 GiB: no last pass of a few elements that leaves the chip idle (64 elements as 63 and one)."""
+    each = kept_bytes(tokens, heads)
+    assert -(-batch // ((4 << 30) // each)) == passes
+    assert 0 <= elements(batch, tokens, heads) * 4 - -(-batch // passes) * each <= 114_000_000
+
+
 @pytest.mark.parametrize("batch,tokens,heads", [
     (1, 1 << 30, 1 << 30), (1, 2**31 - 1, 2**31 - 1), (2**31 - 1, 2**31 - 1, 2**31 - 1), (1, 2**31 - 1, 31),
     (2**31 - 1, 1, 33), (1, 1, 2**31 - 1)])
