@@ -1628,9 +1628,8 @@ Workspace workspace_of(int batch_size, int sequence_length, int heads) {
     if (workspace.element_bytes > KEPT_BYTES_LIMIT) return {};
     workspace.passes = index_math::batch_passes(batch_size, KEPT_BYTES_LIMIT / workspace.element_bytes);
     for (const long long elements : {workspace.passes.largest(), batch_size / workspace.passes.passes}) {
-        const long long slots = workspace_cut(sequence_length, heads, (int)elements, 256).slot_bytes;
-        if (slots > index_math::query_gradient_bytes(sequence_length, heads, elements)) {
-            workspace.slot_bytes = std::max(workspace.slot_bytes, slots);
+        if (index_math::slots_in_workspace(sequence_length, heads, elements)) {
+            workspace.slot_bytes = std::max(workspace.slot_bytes, workspace_cut(sequence_length, heads, (int)elements, 256).slot_bytes);
         }
     }
     return workspace;
@@ -1674,7 +1673,7 @@ void mla_absorbed_backward_dispatch(bf16_t* query_latent_gradient, bf16_t* query
         const long long first = passes.first(pass);
         const long long row = first * rows;
         const long long elements = passes.first(pass + 1) - first;
-        // partial key gradients: in the latent query gradients, behind dS where those have no room for them
+        // partial key gradients: behind dS, or in the latent query gradients
         const long long scratch_bytes = index_math::query_gradient_bytes(sequence_length, heads, elements);
         const long long room = std::max(scratch_bytes, left);
         index_math::KeyCut cut{};
@@ -1685,7 +1684,10 @@ void mla_absorbed_backward_dispatch(bf16_t* query_latent_gradient, bf16_t* query
             if (cut.slot_bytes > room) cut = key_cut(sequence_length, heads, (int)elements, room, units, kept != nullptr);
         }
         float* partial_slots = reinterpret_cast<float*>(query_latent_gradient + row * RANK);
-        if (cut.slot_bytes > scratch_bytes) partial_slots = reinterpret_cast<float*>(kept + kept_bytes);
+        if (cut.slot_bytes > scratch_bytes ||
+            (kept != nullptr && cut.slot_bytes <= left && index_math::slots_in_workspace(sequence_length, heads, elements))) {
+            partial_slots = reinterpret_cast<float*>(kept + kept_bytes);
+        }
         const long long token = first * sequence_length;
         backward_of_batch(query_latent_gradient + row * RANK, query_rope_gradient + row * ROPE, kv_latent_gradient + token * RANK,
                           key_rope_gradient + token * ROPE, output_gradient + row * RANK, output + row * RANK, logsumexp + row,

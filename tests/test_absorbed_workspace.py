@@ -32,11 +32,11 @@ def kept_bytes(tokens, heads):
     (1, 513, 8), (3, 700, 5), (1, 65, 128), (2, 4096, 16), (1, 512, 8), (1, 2048, 128), (1, 4096, 128), (240, 4096, 1),
     (60, 4096, 4), (4096, 33, 16), (512, 1, 1), (20, 4096, 1), (271, 352, 2)])
 def test_size_holds_every_block_and_the_slots_that_are_used(batch, tokens, heads):
-    """dS, and slots for partial key gradients where the cut of the call needs more than the latent query gradients hold."""
+    """dS, and the slots that the call uses for partial key gradients, unless the latent query gradients hold any number."""
     slots = rules().workspace_slots(batch, tokens, heads)
     room = elements(batch, tokens, heads) * 4 - batch * kept_bytes(tokens, heads)
-    assert room == (slots if slots > batch * tokens * heads * 1024 else 0)
-    assert room <= 114_000_000
+    most = 3 * 256 * 64 * 576 * 4
+    assert room == (slots if batch * tokens * heads * 1024 < most else 0) and room <= most
 
 
 def test_size_is_zero_or_bounded():
