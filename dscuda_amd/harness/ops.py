@@ -157,11 +157,27 @@ def mla_forward(query_latent, query_rope, kv_latent, key_rope, scale, out=None, 
     return out, lse
 
 
+# bytes of a workspace from which on it is looked up whether they are there: 4 us (100 where the device has few left), in a
+# backward of 1 ms and more
+_LARGE_WORKSPACE = 256 << 20
+
+
+def _is_there(size, device):
+    """Whether `size` bytes are free on the device or in torch's cache.  An allocation that fails empties the cache first,
+    which a program short of memory would pay for on every call."""
+    free, _ = torch.cuda.mem_get_info(device)
+    if size <= free:
+        return True
+    stats = torch.cuda.memory_stats(device)
+    return size <= free + stats["reserved_bytes.all.current"] - stats["allocated_bytes.all.current"]
+
+
 def mla_backward_workspace(batch, tokens, heads, rank=512, rope=64, device="cuda"):
     """fp32 workspace of the absorbed backward (dscuda_mla_backward_workspace_elements): room for dS, two bytes per
-    visible (row, key) pair.  None where the call makes no use of one, or the memory is not there."""
+    visible (row, key) pair, at most 4 GiB, and at most 114 MB of partial key gradients.  None where the call makes no
+    use of one, or the memory is not there."""
     elements = mla_library().backward_workspace_elements(batch, tokens, heads, rank, rope)
-    if not elements:
+    if not elements or (4 * elements >= _LARGE_WORKSPACE and not _is_there(4 * elements, device)):
         return None
     try:
         return torch.empty(elements, device=device, dtype=torch.float32)
@@ -170,7 +186,12 @@ def mla_backward_workspace(batch, tokens, heads, rank=512, rope=64, device="cuda
 
 
 def mla_backward(dout, out, lse, query_latent, query_rope, kv_latent, key_rope, scale, grads=None, workspace=None):
-    """Absorbed MLA backward (dscuda_mla_backward_workspace) -> (dq_lat, dq_rope, dlatent, dk_rope)."""
+    """Absorbed MLA backward -> (dq_lat, dq_rope, dlatent, dk_rope).
+
+    Without a `workspace` the call allocates one of mla_backward_workspace (dscuda_mla_backward_workspace), up to 4 GiB, which
+    a captured graph keeps.  A program that calls this often passes one that it keeps; an empty tensor stands for none
+    (dscuda_mla_backward: nothing is allocated, and other kernels form scores and dP twice).  The last bits of the
+    gradients depend on the size of the workspace, and on nothing else but the inputs."""
     _require_cuda(dout, out, lse, query_latent, query_rope, kv_latent, key_rope)
     b, t, h, c = query_latent.shape
     r = query_rope.shape[-1]
@@ -181,10 +202,12 @@ def mla_backward(dout, out, lse, query_latent, query_rope, kv_latent, key_rope, 
     else:
         _require_cuda(workspace)
     lib = mla_library()
-    kept = (None, 0) if workspace is None else (workspace.data_ptr(), workspace.numel() * workspace.element_size() // 4)
-    checked(lib.lib, "mla", lib.backward_workspace(
-        *pointers((*grads, dout, out, lse, query_latent, query_rope, kv_latent, key_rope)), *kept,
-        b, t, h, c, r, scale, stream()))
+    operands = pointers((*grads, dout, out, lse, query_latent, query_rope, kv_latent, key_rope))
+    if workspace is None or workspace.numel() == 0:
+        checked(lib.lib, "mla", lib.backward(*operands, b, t, h, c, r, scale, stream()))
+    else:
+        checked(lib.lib, "mla", lib.backward_workspace(
+            *operands, workspace.data_ptr(), workspace.numel() * workspace.element_size() // 4, b, t, h, c, r, scale, stream()))
     return grads
 
 

@@ -77,3 +77,35 @@ def test_a_workspace_is_contiguous_gpu_memory(calls, call):
     call(operand(64, dtype=torch.float32))
     call(operand(0, dtype=torch.float32))
     assert len(calls) == 2
+
+
+def test_an_empty_workspace_stands_for_none(calls):
+    """The library's own backward without a workspace, and no question about the size of one."""
+    absorbed_backward(operand(0, dtype=torch.float32))
+    assert calls == ["backward"]
+    absorbed_backward(operand(64, dtype=torch.float32))
+    assert calls == ["backward", "backward_workspace"]
+
+
+def test_a_large_workspace_is_not_asked_for_where_the_memory_is_short(calls, monkeypatch):
+    """An allocation that fails gives all of torch's cached blocks back first: the call runs without, and nothing is tried."""
+    ops.mla_library().backward_workspace_elements = lambda *shape: 1 << 28   # 1 GiB
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device: (100 << 20, 288 << 30))
+    cached = [800 << 20]
+    monkeypatch.setattr(torch.cuda, "memory_stats", lambda device: {
+        "reserved_bytes.all.current": 10 << 30, "allocated_bytes.all.current": (10 << 30) - cached[0]})
+    tried = []
+    allocate = torch.empty
+
+    def empty(*shape, **options):
+        if shape == (1 << 28,):
+            tried.append(shape)
+            return operand(64, dtype=torch.float32)
+        return allocate(*shape, **options)
+
+    monkeypatch.setattr(torch, "empty", empty)
+    absorbed_backward(None)
+    assert calls == ["backward"] and not tried
+    cached[0] = 950 << 20   # the cache holds what is missing
+    absorbed_backward(None)
+    assert calls == ["backward", "backward_workspace"] and len(tried) == 1
