@@ -1,7 +1,7 @@
 """The reference's own prefill API (dscuda_mla_forward / dscuda_mla_backward) at the size the benchmark quotes,
 B=1, T=4096, H=128: the paths the library chooses by itself at that size (row blocks of the unit stream in the
-forward; the interval cut of the key gradients in the backward, taken when the rows outgrow the caches) against
-the fp32 oracle, which works through the heads in chunks and sums the shared key / latent gradients over them."""
+forward; the interval cut of the key gradients in the backward, taken when the rows outgrow the caches, without a
+workspace and with the one it asks for) against the fp32 oracle, which works through the heads in chunks and sums the shared key / latent gradients over them."""
 
 import pytest
 import torch
@@ -50,9 +50,11 @@ def test_absorbed_forward_and_backward_at_the_benched_size(cuda):
     assert_close_lse("LSE", lse, expected_lse)
     del out, lse
 
-    announce("mla_backward at the benched size", dict(B=1, T=TOKENS, H=HEADS))
-    grads = ops.mla_backward(dout.to(cuda), saved_out.to(cuda), expected_lse.to(cuda), *on_gpu, scale)
-    torch.cuda.synchronize()
     expected = (expected_dq, expected_dq_rope, expected_dlatent.float(), expected_dk_rope.float())
-    for name, actual, reference in zip(("dq_latent", "dq_rope", "dlatent", "dk_rope"), grads, expected):
-        assert_close_bf16(name, actual.cpu(), reference)
+    saved = (dout.to(cuda), saved_out.to(cuda), expected_lse.to(cuda))
+    for workspace in (torch.empty(0, device=cuda), None):   # dscuda_mla_backward, and the workspace the library asks for
+        announce("mla_backward at the benched size", dict(B=1, T=TOKENS, H=HEADS, workspace=workspace is None))
+        grads = ops.mla_backward(*saved, *on_gpu, scale, workspace=workspace)
+        torch.cuda.synchronize()
+        for name, actual, reference in zip(("dq_latent", "dq_rope", "dlatent", "dk_rope"), grads, expected):
+            assert_close_bf16(name, actual.cpu(), reference)

@@ -1,5 +1,6 @@
 """GPU parity of the absorbed backward of short sequences, which keeps P and dS in the query-gradient buffers
-(index_math::short_backward; the placement itself is enumerated in tests/host/index_math_test.cpp)."""
+(index_math::short_backward; the placement itself is enumerated in tests/host/index_math_test.cpp), and of the same calls
+with the workspace that the library asks for, which takes some of them to other kernels."""
 
 import pytest
 import torch
@@ -32,15 +33,16 @@ def test_absorbed_backward_of_short_sequences(cuda, batch, tokens, heads):
     out, lse = oracle.mla_forward(ql, qr, c, kr, scale, mask)
     announce("mla_backward, short", dict(B=batch, T=tokens, H=heads))
     operands = tuple(x.to(cuda) for x in (dout, out, lse, ql, qr, c, kr))
-    runs = []
-    for _ in range(2):
-        grads = tuple(torch.full_like(x, float("nan")) for x in operands[3:])   # scratch as well as results
-        runs.append(ops.mla_backward(*operands, scale, grads))
-    torch.cuda.synchronize()
     expected = oracle.mla_backward_unrounded(dout, out, lse, ql, qr, c, kr, scale, mask)
-    for name, first, second, reference in zip(("dq_latent", "dq_rope", "dlatent", "dk_rope"), *runs, expected):
-        assert torch.equal(first, second)
-        assert_close_bf16(name, first.cpu(), reference)
+    for workspace in (torch.empty(0, device=cuda), None):   # dscuda_mla_backward, and the workspace the library asks for
+        runs = []
+        for _ in range(2):
+            grads = tuple(torch.full_like(x, float("nan")) for x in operands[3:])   # scratch as well as results
+            runs.append(ops.mla_backward(*operands, scale, grads, workspace))
+        torch.cuda.synchronize()
+        for name, first, second, reference in zip(("dq_latent", "dq_rope", "dlatent", "dk_rope"), *runs, expected):
+            assert torch.equal(first, second)
+            assert_close_bf16(name, first.cpu(), reference)
 
 
 @pytest.mark.parametrize("batch,tokens,heads,kept", [
@@ -49,13 +51,15 @@ def test_absorbed_backward_of_short_sequences(cuda, batch, tokens, heads):
     (1, 1, 32, False), (13, 4, 8, False), (10, 353, 2, False), (2, 224, 20, False), (2, 160, 32, False),
 ])
 def test_which_calls_keep_their_scores(cuda, batch, tokens, heads, kept):
+    """Without a workspace; those that have one and still keep them are pinned in tests/host/index_math_test.cpp."""
     assert bool(rules().keeps_scores(batch, tokens, heads)) == kept
     test_absorbed_backward_of_short_sequences(cuda, batch, tokens, heads)
 
 
 @pytest.mark.parametrize("batch,tokens,heads", [(1, 1, 1), (3, 9, 2), (1, 513, 1), (2, 700, 3), (1, 1024, 2)])
 def test_absorbed_backward_of_whole_key_blocks(cuda, batch, tokens, heads):
-    """Calls whose query gradients have no room for partial results: a workgroup walks all rows of its key block."""
+    """Calls whose query gradients have no room for partial results: without a workspace a workgroup walks all rows of its
+    key block."""
     units = torch.cuda.get_device_properties(cuda).multi_processor_count
     assert not rules().keeps_scores(batch, tokens, heads) and rules().backward_ranges(batch, tokens, heads, units) == 0
     test_absorbed_backward_of_short_sequences(cuda, batch, tokens, heads)

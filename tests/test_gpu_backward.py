@@ -109,12 +109,13 @@ def _absorbed_case(cuda, batch, tokens, heads, seed, dout_factor):
     mask = oracle.causal_mask(tokens)
     out, lse = oracle.mla_forward(ql, qr, c, kr, scale, mask)
     announce("mla_backward", dict(B=batch, T=tokens, H=heads))
-    grads = ops.mla_backward(dout.to(cuda), out.to(cuda), lse.to(cuda), ql.to(cuda), qr.to(cuda), c.to(cuda),
-                             kr.to(cuda), scale)
-    torch.cuda.synchronize()
+    operands = [x.to(cuda) for x in (dout, out, lse, ql, qr, c, kr)]
     expected = oracle.mla_backward_unrounded(dout, out, lse, ql, qr, c, kr, scale, mask)
-    for name, actual, reference in zip(("dq_latent", "dq_rope", "dlatent", "dk_rope"), grads, expected):
-        assert_close_bf16(name, actual.cpu(), reference)
+    for workspace in (torch.empty(0, device=cuda), None):   # dscuda_mla_backward, and the workspace the library asks for
+        grads = ops.mla_backward(*operands, scale, workspace=workspace)
+        torch.cuda.synchronize()
+        for name, actual, reference in zip(("dq_latent", "dq_rope", "dlatent", "dk_rope"), grads, expected):
+            assert_close_bf16(name, actual.cpu(), reference)
 
 
 def test_absorbed_backward_closed_form_constant_fill(cuda):
@@ -166,7 +167,7 @@ def test_backward_in_chunks_of_pairs(cuda, batch, seq, heads, budget_pairs, expe
     (1, 256, 128, 256),   # 4 intervals, 20 items: key block 0 has four parts, the last two blocks one
     (2, 160, 128, 100),   # two batch elements, a short last interval, interval ends inside key blocks
     (1, 512, 8, 7),       # many short intervals
-    (2, 257, 4, 1000),    # one interval: every key block whole
+    (2, 257, 4, 1000),    # one interval: every key block whole (an item each, which the query gradients have room for)
     (1, 95, 3, 4),        # 285 rows: the last half tile of 16 rows holds 13
     (1, 50, 1, 1),        # 50 rows: the last row tile holds 18, its second half tile two; one key block, cut in two
     (3, 77, 5, 3),        # 385 rows: one row in the last tile, whose second half tile is past the end
@@ -183,8 +184,8 @@ def test_absorbed_backward_interval_cut(cuda, batch, tokens, heads, interval_til
 
 def test_absorbed_backward_interval_cut_chosen_by_the_library(cuda):
     """B=5, T=300, H=128: 38 400 rows of 2176 bytes per batch element are above the library's own bound for the
-    interval cut, and on 256 compute units it cuts into intervals of 24 row tiles (725 items; the choice itself is
-    pinned on the host, tests/host/index_math_test.cpp)."""
+    interval cut, and on 256 compute units it cuts into intervals of 24 row tiles without a workspace (725 items) and of 72
+    with one (255; the choices themselves are pinned on the host, tests/host/index_math_test.cpp)."""
     _absorbed_case(cuda, 5, 300, 128, seed=79, dout_factor=0.05)
 
 

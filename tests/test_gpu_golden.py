@@ -43,10 +43,12 @@ def test_mla_absorbed_fixture(cuda):
     torch.cuda.synchronize()
     assert_close_bf16("O", out, d["out"])
     assert_close_lse("LSE", lse, d["lse"])
-    grads = ops.mla_backward(d["dout"].to(cuda), d["saved_out"].to(cuda), d["lse"].to(cuda), *tensors, d["scale"])
-    torch.cuda.synchronize()
-    for actual, key in zip(grads, ("dql", "dqr", "dc", "dkr")):
-        assert_close_bf16(key, actual, d[key])
+    for workspace in (torch.empty(0, device=cuda), None):   # dscuda_mla_backward, and the workspace the library asks for
+        grads = ops.mla_backward(d["dout"].to(cuda), d["saved_out"].to(cuda), d["lse"].to(cuda), *tensors, d["scale"],
+                                 workspace=workspace)
+        torch.cuda.synchronize()
+        for actual, key in zip(grads, ("dql", "dqr", "dc", "dkr")):
+            assert_close_bf16(key, actual, d[key])
 
 
 def test_mla_decode_fixture(cuda):

@@ -101,9 +101,13 @@ def test_graph_mla_prefill_forward_and_backward(cuda):
     _replay_twice(cuda, make, call, check)
 
 
-def test_graph_mla_absorbed_forward_and_backward(cuda):
-    announce("graph capture: absorbed mla forward + backward")
-    batch, tokens, heads = 2, 65, 4
+# P and dS kept in the query gradients; with a workspace, which the captured call allocates, whole 32-key blocks, ranges and
+# items of 64 keys; the same without one
+@pytest.mark.parametrize("batch,tokens,heads,empty", [
+    (2, 65, 4, False), (40, 33, 3, False), (1, 513, 8, False), (2, 700, 5, False), (2, 65, 4, True), (2, 700, 5, True)])
+def test_graph_mla_absorbed_forward_and_backward(cuda, batch, tokens, heads, empty):
+    announce("graph capture: absorbed mla forward + backward", dict(B=batch, T=tokens, H=heads, empty=empty))
+    workspace = torch.empty(0, device=cuda) if empty else None
     scale = configs.c_float(576 ** -0.5)
     mask = oracle.causal_mask(tokens)
 
@@ -122,7 +126,7 @@ def test_graph_mla_absorbed_forward_and_backward(cuda):
             out = lse = None
             grads = tuple(torch.empty_like(t) for t in (ql, qr, c, kr))
         out, lse = ops.mla_forward(ql, qr, c, kr, scale, out, lse)
-        ops.mla_backward(dout, out, lse, ql, qr, c, kr, scale, grads)
+        ops.mla_backward(dout, out, lse, ql, qr, c, kr, scale, grads, workspace)
         return [out, lse, *grads]
 
     def check(cpu, got):
@@ -135,6 +139,28 @@ def test_graph_mla_absorbed_forward_and_backward(cuda):
             assert_close_bf16(name, actual, wanted)
 
     _replay_twice(cuda, make, call, check)
+
+
+def test_graph_absorbed_backward_with_a_large_workspace(cuda):
+    """From 256 MB on the operator looks up whether the memory is there, inside the capture too.  Replays against eager calls,
+    which the other tests hold against the oracle."""
+    batch, tokens, heads = 1, 2100, 64
+    assert ops.mla_backward_workspace(batch, tokens, heads, device=cuda).numel() * 4 >= ops._LARGE_WORKSPACE
+    announce("graph capture: absorbed mla backward, large workspace", dict(B=batch, T=tokens, H=heads))
+    scale = configs.c_float(576 ** -0.5)
+
+    def make(seed):
+        g = torch.Generator(device=cuda).manual_seed(110 + seed)
+        shapes = ((batch, tokens, heads, 512), (batch, tokens, heads, 64), (batch, tokens, 512), (batch, tokens, 64),
+                  (batch, tokens, heads, 512))
+        return [torch.randn(shape, device=cuda, generator=g).mul_(0.25).bfloat16() for shape in shapes]
+
+    def call(x, outputs):
+        ql, qr, c, kr, dout = x
+        out, lse = ops.mla_forward(ql, qr, c, kr, scale)
+        return list(ops.mla_backward(dout, out, lse, ql, qr, c, kr, scale, tuple(outputs) if outputs else None))
+
+    _replay_twice(cuda, make, call, lambda inputs, got: None)
 
 
 @pytest.mark.parametrize("splits", [1, 8])

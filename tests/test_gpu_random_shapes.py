@@ -84,11 +84,12 @@ def test_random_absorbed(cuda, case):
     assert_close_bf16("O", out, expected, max_abs=8e-3)     # the reference's own bars (benchmarks/mla.py)
     assert_close_lse("LSE", lse, expected_lse, tol=1e-4)
     saved = expected.bfloat16()
-    grads = ops.mla_backward(dout.to(cuda), saved.to(cuda), expected_lse.to(cuda), ql.to(cuda), qr.to(cuda),
-                             latent.to(cuda), kr.to(cuda), scale)
     references = oracle.mla_backward_unrounded(dout, saved, expected_lse, ql, qr, latent, kr, scale, mask)
-    for name, actual, reference in zip(("dq_latent", "dq_rope", "dlatent", "dk_rope"), grads, references):
-        assert_close_bf16(name, actual, reference)
+    for workspace in (torch.empty(0, device=cuda), None):   # dscuda_mla_backward, and the workspace the library asks for
+        grads = ops.mla_backward(dout.to(cuda), saved.to(cuda), expected_lse.to(cuda), ql.to(cuda), qr.to(cuda),
+                                 latent.to(cuda), kr.to(cuda), scale, workspace=workspace)
+        for name, actual, reference in zip(("dq_latent", "dq_rope", "dlatent", "dk_rope"), grads, references):
+            assert_close_bf16(name, actual, reference)
 
 
 @pytest.mark.parametrize("case", range(10))

@@ -25,15 +25,19 @@ def test_absorbed_prefill_is_reproducible(cuda, batch, tokens, heads):
     scale = configs.c_float(576 ** -0.5)
     announce("mla_forward / mla_backward twice", dict(B=batch, T=tokens, H=heads))
     out, lse = ops.mla_forward(ql, qr, latent, kr, scale)
-    first = [x.clone() for x in ops.mla_backward(dout, out, lse, ql, qr, latent, kr, scale)]
     out2, lse2 = ops.mla_forward(ql, qr, latent, kr, scale)
     assert torch.equal(out, out2) and torch.equal(lse, lse2)
-    grads = tuple(torch.full_like(x, 7.0) for x in first)   # the scratch use of the gradient buffers starts from other contents
-    for _ in range(2):
-        ops.mla_backward(dout, out, lse, ql, qr, latent, kr, scale, grads)
-        torch.cuda.synchronize()
-        for name, a, b in zip(("dq_latent", "dq_rope", "dlatent", "dk_rope"), first, grads):
-            assert torch.equal(a, b), name
+    kept = ops.mla_backward_workspace(batch, tokens, heads, device=cuda)
+    for workspace in (torch.empty(0, device=cuda), None if kept is None else kept.fill_(float("nan"))):
+        first = [x.clone() for x in ops.mla_backward(dout, out, lse, ql, qr, latent, kr, scale, workspace=workspace)]
+        grads = tuple(torch.full_like(x, 7.0) for x in first)   # the scratch use of the gradient buffers starts from other contents
+        for fill in (3.0, float("inf")):
+            if workspace is not None:
+                workspace.fill_(fill)
+            ops.mla_backward(dout, out, lse, ql, qr, latent, kr, scale, grads, workspace)
+            torch.cuda.synchronize()
+            for name, a, b in zip(("dq_latent", "dq_rope", "dlatent", "dk_rope"), first, grads):
+                assert torch.equal(a, b), name
 
 
 @pytest.mark.parametrize("batch,seq,heads", [(1, 1536, 16), (2, 449, 6)])
