@@ -252,6 +252,16 @@ DSCUDA_HOST_DEVICE inline int narrow_forward_row_blocks(int sequence_length, int
     return (longest > second ? longest : second) <= 900 + 94 * keys ? 1 : 2;
 }
 
+// How many 32-row blocks a workgroup of the absorbed prefill forward holds: 1 or 2 while 128 rows (0: four blocks, the
+// decode's kernel) leave compute units idle.  Whole layer of absorb, forward and un-absorb in us, 32 / 64 / 128 rows: 32 workgroups of 128
+// (512 tokens x 8 heads) 42 / 45 / 61, 128 of them 52 / 52 / 66, 243 of them 236 / 168 / 241, 256 108 / 84 / 103, 391
+// 113 / 95 / 92, 1024 374 / 284 / 268.
+DSCUDA_HOST_DEVICE inline int forward_row_blocks(int sequence_length, int heads, long long batch, int compute_units) {
+    const long long workgroups = ((long long)sequence_length * heads + 127) / 128 * batch;
+    if (2 * workgroups <= compute_units) return narrow_forward_row_blocks(sequence_length, heads, batch, compute_units);
+    return 4 * workgroups <= 5LL * compute_units ? 2 : 0;
+}
+
 // ---- work order of the persistent forward kernel ------------------------------
 struct ForwardItem {
     int batch_head;

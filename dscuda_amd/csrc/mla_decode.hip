@@ -933,12 +933,7 @@ void mla_absorbed_forward_dispatch(bf16_t* output, float* logsumexp, const bf16_
     if (row_blocks * batch_size > 0x7fffffffLL) {
         throw std::invalid_argument("MLA forward: batch*tokens*heads exceeds the grid limit");
     }
-    // 32 or 64 rows per workgroup while 128 rows leave compute units idle (whole layer of absorb, forward and
-    // un-absorb, 32 / 64 / 128 rows): 32 blocks (T = 512, H = 8) 42 / 45 / 61 us, 128 blocks 52 / 52 / 66, 243 blocks
-    // 236 / 168 / 241, 256 blocks 108 / 84 / 103, 391 blocks 113 / 95 / 92, 1024 blocks 374 / 284 / 268.
-    const long long blocks = row_blocks * batch_size;
-    const int narrow = 2 * blocks <= compute_units() ? index_math::narrow_forward_row_blocks(sequence_length, heads, batch_size, compute_units())
-                     : 4 * blocks <= 5LL * compute_units() ? 2 : 0;
+    const int narrow = index_math::forward_row_blocks(sequence_length, heads, batch_size, compute_units());
     if (narrow != 0) {
         mla_narrow_forward_launch(output, logsumexp, query_latent, query_rope, kv_latent, key_rope, batch_size,
                                   sequence_length, heads, narrow, scale, stream);

@@ -30,6 +30,10 @@ extern "C" int walks_are_cut(int pairs, int tokens, int sharing) {
 extern "C" long long workspace_slots(int batch, int tokens, int heads) {   // of a call whose dS is kept, in bytes
     return kept_cut(tokens, heads, batch, slot_bytes_of_workspace(tokens, heads, batch), 256).slot_bytes;
 }
+extern "C" int forward_rows(int batch, int tokens, int heads, int compute_units) {   // of a workgroup, absorbed prefill forward
+    const int blocks = forward_row_blocks(tokens, heads, batch, compute_units);
+    return blocks == 0 ? 128 : 32 * blocks;
+}
 extern "C" int keeps_scores(int batch, int tokens, int heads) { return short_backward(batch, tokens, heads); }
 """
 

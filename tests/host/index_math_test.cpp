@@ -507,6 +507,23 @@ void check_kept_cut() {
     }
 }
 
+// rows of a workgroup of the absorbed prefill forward: known cases at 256 compute units, and 32 rows wherever those are one round
+void check_forward_row_blocks() {
+    struct { int batch, tokens, heads, expected; } known[] = {
+        {1, 512, 8, 1}, {1, 64, 128, 1}, {1, 65, 128, 2}, {1, 433, 32, 1}, {1, 434, 32, 2}, {1, 140, 64, 1}, {1, 141, 64, 2}, {3, 300, 16, 2},
+        {1, 2000, 8, 1}, {300, 1, 40, 2}, {320, 3, 42, 2}, {321, 3, 42, 0}, {1, 1024, 128, 0},
+    };
+    for (const auto& c : known) {
+        const int blocks = forward_row_blocks(c.tokens, c.heads, c.batch, 256);
+        EXPECT(blocks == c.expected, "B=%d T=%d H=%d: %d blocks of 32 rows", c.batch, c.tokens, c.heads, blocks);
+    }
+    for (int heads : {1, 3, 16, 128}) {
+        for (int tokens = 1; tokens <= 300; ++tokens) {
+            if ((tokens * heads + 31) / 32 <= 256) EXPECT(forward_row_blocks(tokens, heads, 1, 256) == 1, "T=%d H=%d", tokens, heads);
+        }
+    }
+}
+
 // passes over a batch: every element once, none more than allowed, sizes that differ by at most one
 void check_batch_passes() {
     for (long long batch = 1; batch <= 200; ++batch) {
@@ -975,6 +992,7 @@ int main() {
     check_kept_cut();
     check_kept_gradients();
     check_batch_passes();
+    check_forward_row_blocks();
     check_decode_ranges();
     check_decode_layout();
     check_rows_apart();

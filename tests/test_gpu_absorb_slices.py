@@ -11,7 +11,7 @@ from parity import announce, assert_close_bf16
 pytestmark = pytest.mark.gpu
 
 
-# more than 256 (token tiles x heads); one row in the last tile, one tile in the last chunk; 8 | heads and not
+# more than 128 (token tiles x heads); one row in the last tile, one tile in the last chunk; 8 | heads and not
 @pytest.mark.parametrize("tokens,heads", [(65, 128), (129, 65), (257, 40), (2049, 7), (5000, 2), (4225, 3), (9000, 1), (1000, 17)])
 def test_absorb_query_by_quarters(cuda, tokens, heads):
     g = torch.Generator().manual_seed(61)
@@ -25,15 +25,18 @@ def test_absorb_query_by_quarters(cuda, tokens, heads):
     assert (packed[:, tokens:].float() == 7.0).all() and (packed[..., 512:].float() == 7.0).all()
 
 
-@pytest.mark.parametrize("tokens", [1280, 1281])
-def test_either_side_of_the_size_rule(cuda, tokens):
-    """160 MB of results: a head's rows are the same bits whichever kernel forms them."""
-    heads = 128
+# 160 MB of results and more: one round of chunks of many heads, many chunks of few
+@pytest.mark.parametrize("tokens,heads", [(1280, 128), (1281, 128), (20480, 8), (20481, 8), (163841, 1)])
+def test_either_side_of_the_size_rule(cuda, tokens, heads):
+    """A head's rows are the same bits whichever kernel forms them, in a buffer of rows with other columns behind them."""
     g = torch.Generator(device=cuda).manual_seed(67)
     weights = torch.randn(heads, 128, 512, device=cuda, generator=g).mul_(0.06).bfloat16()
     query = torch.randn(1, tokens, heads, 128, device=cuda, generator=g).mul_(0.5).bfloat16()
     announce("mla_absorb_query, size rule", dict(T=tokens, H=heads))
-    result = ops.mla_absorb_query(query, weights)
-    part = ops.mla_absorb_query(query[:, -64:].contiguous(), weights)
-    torch.cuda.synchronize()
-    assert torch.equal(result[:, -64:], part)
+    packed = torch.full((1, tokens + 1, heads, 576), 7.0, device=cuda, dtype=torch.bfloat16)
+    ops.mla_absorb_query(query, weights, out=packed[:, :tokens, :, :512])
+    for first in range(0, tokens, (tokens + 3) // 4):   # a quarter of the tokens: the kernel by quarters of the columns
+        part = ops.mla_absorb_query(query[:, first:first + (tokens + 3) // 4].contiguous(), weights)
+        torch.cuda.synchronize()
+        assert torch.equal(packed[:, first:min(first + (tokens + 3) // 4, tokens), :, :512], part)
+    assert (packed[:, tokens:] == 7.0).all() and (packed[..., 512:] == 7.0).all()
