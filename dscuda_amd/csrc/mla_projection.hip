@@ -268,9 +268,9 @@ __global__ __launch_bounds__(THREADS) void mla_unabsorb_output_kernel(bf16_t* __
 // tokens, and every load of a thread is in flight at once: one round trip to memory, eight MFMAs a wave.  16 tokens of
 // 16 heads: absorb 7.6 -> 3.2 us, un-absorb 6.6 -> 3.7.
 //
-// Every 32 tokens fetch the weight again, so the kernels win once (token tiles) x heads is large.  Absorb by quarters,
-// below, against few tokens: equal up to 128 tiles, 7.9 / 9.2 us at 256 (1000 tokens of 8 heads; equal for 64 of 128), 9.1 / 12.8
-// at 512.  Un-absorb, whose weight rows come as 32 bytes of 32 rows an instruction, at 128 tiles 5.1-5.8 against 6.7-9.7 us
+// Every 32 tokens fetch the weight again, so the kernels for more tokens win once (token tiles) x heads is large.  Absorb by
+// quarters, below, against few tokens: equal up to 128 tiles, 7.9 / 9.2 us at 256 (1000 tokens of 8 heads; equal for 64 of 128),
+// 9.1 / 12.8 at 512.  Un-absorb, whose weight rows come as 32 bytes of 32 rows an instruction, at 128 tiles 5.1-5.8 against 6.7-9.7 us
 // (16 tokens of 128 heads, 128 of 32), at 256 tiles 10.2-12.8 against 8.1-9.8.
 constexpr long long ABSORB_FEW_TILES = 128;
 constexpr long long UNABSORB_FEW_TILES = 128;
@@ -406,11 +406,13 @@ __global__ __launch_bounds__(THREADS) void mla_unabsorb_output_few_kernel(bf16_t
 // fourth token tile, and two workgroups share a compute unit, so that one's loads and stores go on while the other
 // multiplies or fetches its 32 KB of weight (mla_absorb_query_kernel keeps 128 KB in LDS, one workgroup of four waves
 // per compute unit, which fetches first and then streams).  blockIdx.x = (chunk of the tokens, head, quarter); the
-// quarters of a head, which read the same rows, go to one XCD.  Bound by the bytes written: 1024 tokens x 128 heads
-// 40.4 -> 33.5 us (5.5 TB/s), 1000 x 64 25.0 -> 19.7, 1000 x 16 12.8 -> 9.0, 250 x 64 12.0 -> 9.3.
-// Rows written as four times 256 bytes by workgroups of their own are slower once they go to memory: 2048 x 128
-// (268 MB) 80.7 -> 85, 4096 x 128 137 -> 154.
-constexpr long long SLICE_RESULT_BYTES = 160LL << 20;
+// quarters of a head, which read the same rows, go to one XCD.  Bound by the bytes written: into the
+// results of the call before, 1024 tokens x 128 heads 40.0 -> 32.1 us (168 MB of rows in and out, 5.2 TB/s), 1000 x 64 24.2 -> 19.0,
+// 1000 x 16 12.4 -> 8.6, 250 x 64 12.8 -> 8.6; into results of their own 42.9 -> 43.3 (3.9 TB/s), 25.6 -> 24.0, 13.4 -> 9.1, 13.5 -> 9.1.
+// Rows written as four times 256 bytes by workgroups of their own are slower once they go to memory.  Whole rows / quarters
+// into results of their own: 144 MB (1100 x 128) 46.8 / 46.6, 157 MB 46.8 / 49.9, 168 MB 48.7 / 51.9, 197 MB 54.4 / 59.3; into those
+// of the call before 157 MB 43.7 / 36.1, 197 MB 51.1 / 42.8, 223 MB 59.7 / 68.1, 268 MB 72.4 / 84.1.
+constexpr long long SLICE_RESULT_BYTES = 144LL << 20;
 
 __global__ __launch_bounds__(THREADS, 2) void mla_absorb_query_slice_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
                                                                             const bf16_t* __restrict__ weight,

@@ -25,8 +25,8 @@ def test_absorb_query_by_quarters(cuda, tokens, heads):
     assert (packed[:, tokens:].float() == 7.0).all() and (packed[..., 512:].float() == 7.0).all()
 
 
-# 160 MB of results and more: one round of chunks of many heads, many chunks of few
-@pytest.mark.parametrize("tokens,heads", [(1280, 128), (1281, 128), (20480, 8), (20481, 8), (163841, 1)])
+# 144 MiB of results and more: one round of chunks of many heads, many chunks of few
+@pytest.mark.parametrize("tokens,heads", [(1152, 128), (1153, 128), (18432, 8), (18433, 8), (147457, 1)])
 def test_either_side_of_the_size_rule(cuda, tokens, heads):
     """A head's rows are the same bits whichever kernel forms them, in a buffer of rows with other columns behind them."""
     g = torch.Generator(device=cuda).manual_seed(67)
