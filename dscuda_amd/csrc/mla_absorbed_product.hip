@@ -258,18 +258,23 @@ void mla_absorbed_query_product_launch(bf16_t* query_latent_gradient, bf16_t* qu
                                        const bf16_t* key_rope, int batch_size, int sequence_length, int heads,
                                        int key_tiles, hipStream_t stream) {
     // 128 rows a workgroup where that is a workgroup per compute unit. The whole backward in us, 64 / 128 rows: 148 workgroups of
-    // 128 98 / 103, 226 82 / 81, 282 349 / 350, 304 118 / 114, 512 235 / 228, 1500 1995 / 1895; 33 81 / 87.
+    // 128 98 / 103, 226 82 / 81, 282 349 / 350, 304 118 / 114, 512 235 / 228, 1500 1995 / 1895; 33 81 / 87;
+    // not for elements of at most 64 rows: 568 x 1 x 1 30.9 / 33.9, 1079 x 8 x 7 91 / 97.
     // Workgroups of 64 rows and half the columns where whole rows are no workgroup per compute unit, halves / whole rows: 38 workgroups
-    // of 64 rows 45 / 49, 63 63 / 68, 128 106 / 118, 150 64 / 67, 256 72 / 72; 296 87 / 83, 350 106 / 98.
+    // of 64 rows 45 / 49, 63 63 / 68, 128 106 / 118, 220 (2010 x 7) 130 / 143, 159 (3 x 279 x 12) 49 / 51; but where the halves are
+    // more than one round of them, short walks pay for a second start: 165 x 1 x 1 17.0 / 14.7, 57 x 21 x 11 32.5 / 30.1,
+    // 14 x 73 x 12 40.4 / 38.2, 47 x 133 x 1 30.7 / 29.6, 3 x 182 x 20 45.9 / 44.9; 3 x 204 x 14 41.2 / 42.0.
+    constexpr int SHORT_TOKENS = 192;
     const long long rows = (long long)sequence_length * heads;
     const int units = hip_common::compute_units_of_current_device();
     auto start = [&](auto launch_form) {
         launch_form(query_latent_gradient, query_rope_gradient, kept_gradients, kv_latent, key_rope, batch_size, sequence_length,
                     heads, key_tiles, stream);
     };
-    if ((rows + 127) / 128 * batch_size >= units) {
+    const long long workgroups = (rows + 63) / 64 * batch_size;   // of 64 rows
+    if (rows > 64 && (rows + 127) / 128 * batch_size >= units) {
         start(launch<2, 1>);
-    } else if ((rows + 63) / 64 * batch_size > units) {
+    } else if (workgroups > units || (2 * workgroups > units && sequence_length <= SHORT_TOKENS)) {
         start(launch<1, 1>);
     } else {
         start(launch<1, 2>);

@@ -71,12 +71,14 @@ def test_size_of_calls_beyond_any_memory(batch, tokens, heads):
 
 # rows that end inside a row tile, a 64- and a 128-row workgroup; key blocks of 64 cut at 1, 32, 33 keys; one head, and
 # more heads than a workgroup has rows; ranges of 32-key blocks and items of 64-key blocks; several batch elements; key
-# blocks walked whole, of one to twelve row tiles
+# blocks walked whole, of one to twelve row tiles; the query product's rows of a workgroup and halves of its columns by the
+# number of workgroups: 64 rows a batch element and one more, short walks and long ones
 @pytest.mark.gpu
 @pytest.mark.parametrize("batch,tokens,heads,interval_tiles", [
     (1, 17, 128, 0), (2, 33, 40, 0), (1, 513, 3, 0), (1, 545, 8, 0), (3, 600, 4, 0), (1, 200, 33, 0), (2, 320, 16, 0),
     (1, 1000, 1, 0), (1, 1025, 8, 0), (1, 130, 150, 0), (1, 1, 40, 0), (1, 187, 32, 0), (3, 9, 2, 0), (2, 700, 3, 0),
-    (1, 1000, 33, 0), (40, 33, 5, 0), (3, 64, 1, 0), (34, 126, 3, 0), (2, 2, 17, 0), (1, 512, 8, 0), (2, 530, 16, 0), (1, 513, 3, 7), (2, 97, 40, 50), (1, 65, 128, 100)])
+    (1, 1000, 33, 0), (40, 33, 5, 0), (3, 64, 1, 0), (34, 126, 3, 0), (2, 2, 17, 0), (1, 512, 8, 0), (2, 530, 16, 0), (1, 513, 3, 7), (2, 97, 40, 50), (1, 65, 128, 100),
+    (300, 3, 7, 0), (165, 2, 17, 0), (57, 21, 11, 0), (3, 193, 15, 0), (300, 5, 13, 0)])
 def test_gradients_with_and_without(cuda, batch, tokens, heads, interval_tiles):
     from dscuda_amd.harness import ops
     ql, qr, c, kr, scale = configs.mla_absorbed_inputs(batch, tokens, heads)
