@@ -41,8 +41,8 @@
 //                     wave accumulates dQ^T for its own share of the 18 column blocks.
 // With a workspace the score waves of the key gradients keep dS there, and the query gradients are the product
 // dS [latent|rope] alone (mla_absorbed_product.hip); it also has slots for partial key gradients, so that calls whose
-// query gradients have room for few of them occupy the chip as well (4096 tokens x 4 heads: backward 638 -> 284 us with
-// both, 600 x 4 130 -> 49, 2048 x 128 2236 -> 1733).
+// query gradients have room for few of them occupy the chip as well (4096 tokens x 4 heads: backward 632 -> 270 us with
+// both, 600 x 4 125 -> 44, 2048 x 128 2301 -> 1720).
 // Short sequences with few rows (index_math::short_backward), whose query-gradient buffers have room for few partial
 // results, take three other launches after the row statistics (mla_absorbed_short.hip).
 #include "attn_kernels.h"

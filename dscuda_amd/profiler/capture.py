@@ -120,7 +120,7 @@ def metric_cases(suite):
     add("mla_decode_B64_H128", "absorbed MLA decode B=64 H=128 lengths U[1024,8192] seed 3", "decode", 300, 100,
         DECODE_KERNELS)
     add("flash_forward_S512_H8_D64", "flash forward B=1 H=8 S=512 D=64", "flash", 300, 100, FORWARD_KERNELS)
-    add("mla_absorbed_T4096_H128", "absorbed MLA prefill forward + backward (dscuda_mla_forward / _backward) B=1 T=4096 H=128",
+    add("mla_absorbed_T4096_H128", "absorbed MLA prefill forward + backward (dscuda_mla_forward / _backward_workspace) B=1 T=4096 H=128",
         "absorbed", 6, 3, ABSORBED_KERNELS)
     add("mla_projection_T4096_H128", "W_UK absorb and W_UV un-absorb of 4096 tokens x 128 heads", "projection", 60, 20,
         PROJECTION_KERNELS)

@@ -78,7 +78,7 @@ void mla_compressed_attention_backward_cuda(
 // The same with a workspace (additive, no counterpart in the reference): the key-gradient launch keeps dS there, two
 // bytes per (row, visible key) pair, so that the query gradients are one product instead of three, and partial key
 // gradients that the query-gradient buffers have no room for.  mla_backward_workspace_elements floats hold all that is
-// of use (at most 4 GiB of dS: batch elements are taken in groups; at most 114 MB of partial results); 0 where a call
+// of use (at most 4 GiB of dS: the batch is taken in passes; at most 114 MB of partial results); 0 where a call
 // makes no use of one.  Any smaller size, 0 and nullptr included, is taken for the batch elements
 // that fit, or none.  16-byte aligned, needs no initialisation.
 std::size_t mla_backward_workspace_elements(
