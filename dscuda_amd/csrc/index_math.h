@@ -744,7 +744,7 @@ DSCUDA_HOST_DEVICE inline bool ranges_stay_in_blocks(const KeyVisits& visits, lo
 // reduction, or the walks are cut into ranges.  In steps of a walk, fitted to 6100 shapes of up to 60000 rows (the choice
 // costs 0.3 % against the better of the two): beginning and end of a walk 7, the reduction 3.  Backward in us, cut /
 // whole: 512 x 1 token x 1 head 38 / 25, 2000 x 1 x 1 125 / 82, 128 x 5 x 16 37 / 30, 300 x 158 x 1 180 / 151, 64 x 49 x 5 40 / 36;
-// 1 x 142 x 40 36 / 227, 8 x 121 x 16 46 / 98, 16 x 21 x 16 31.0 / 29.6.
+// 1 x 142 x 40 36 / 227, 8 x 121 x 16 46 / 98, 16 x 21 x 16 31.0 / 29.6, 3 x 11 x 36 23.3 / 27.7.
 constexpr int WALK_ENDS = 7;
 constexpr int REDUCTION_STEPS = 3;
 constexpr int SHORT_WALK = 12;   // row tiles up to which items of 64-key blocks are never the better cut (300 x 158 x 1 180)
@@ -757,7 +757,9 @@ DSCUDA_HOST_DEVICE inline bool whole_key_walks(int sequence_length, int heads, l
     const long long whole = blocks <= compute_units ? visits.row_tiles + WALK_ENDS
                                                     : (total + WALK_ENDS * blocks) / compute_units + visits.row_tiles / 2;
     const long long crossings = ranges_stay_in_blocks(visits, batch, compute_units) ? 0 : blocks > ranges ? blocks / ranges : 1;
-    return whole <= (total + ranges - 1) / ranges + WALK_ENDS * (1 + crossings) + REDUCTION_STEPS;
+    // (an odd list of visits in ranges of two has one of three, which crosses no border)
+    const long long longest = total == 2 * ranges + 1 ? 2 : (total + ranges - 1) / ranges;
+    return whole <= longest + WALK_ENDS * (1 + crossings) + REDUCTION_STEPS;
 }
 
 // How the key gradients of a call are cut: items of 64-key blocks in intervals of `length` row tiles, or (length 0) ranges of

@@ -440,7 +440,7 @@ void check_key_interval_fit() {
 void check_kept_routes() {
     struct { int batch, tokens, heads, whole; } walks[] = {
         {512, 1, 1, 1}, {2000, 1, 1, 1}, {128, 5, 16, 1}, {300, 158, 1, 1}, {64, 49, 5, 1}, {1, 33, 2, 1}, {5000, 16, 16, 1},
-        {1, 142, 40, 0}, {8, 121, 16, 0}, {1, 513, 8, 0}, {1, 600, 4, 0}, {4, 96, 8, 0}, {1, 4096, 128, 0},
+        {1, 142, 40, 0}, {8, 121, 16, 0}, {3, 11, 36, 0}, {8, 9, 43, 0}, {3, 6, 67, 0}, {4, 5, 39, 1}, {1, 513, 8, 0}, {1, 600, 4, 0}, {4, 96, 8, 0}, {1, 4096, 128, 0},
     };
     for (const auto& c : walks) {
         EXPECT(whole_key_walks(c.tokens, c.heads, c.batch, 256) == (c.whole != 0), "whole walks B=%d T=%d H=%d", c.batch, c.tokens, c.heads);
