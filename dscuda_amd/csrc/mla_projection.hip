@@ -413,6 +413,7 @@ __global__ __launch_bounds__(THREADS) void mla_unabsorb_output_few_kernel(bf16_t
 // into results of their own: 144 MB (1100 x 128) 46.8 / 46.6, 157 MB 46.8 / 49.9, 168 MB 48.7 / 51.9, 197 MB 54.4 / 59.3; into those
 // of the call before 157 MB 43.7 / 36.1, 197 MB 51.1 / 42.8, 223 MB 59.7 / 68.1, 268 MB 72.4 / 84.1.
 constexpr long long SLICE_RESULT_BYTES = 144LL << 20;
+constexpr int XCDS = 8;
 
 __global__ __launch_bounds__(THREADS, 2) void mla_absorb_query_slice_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
                                                                             const bf16_t* __restrict__ weight,
@@ -422,22 +423,16 @@ __global__ __launch_bounds__(THREADS, 2) void mla_absorb_query_slice_kernel(bf16
     constexpr int BLOCKS = SLICE / 32;
     constexpr int PIECES = HEAD * SLICE / 8 / THREADS;   // 16-byte pieces of the weight slice per thread
     static_assert(4 * TILE * SLICE_PITCH == SLICE_BYTES, "the waves' output rows take the place of the weight");
-    constexpr int XCDS = 8;
     __shared__ __attribute__((aligned(16))) unsigned char lds[SLICE_BYTES];
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const int lane = tid % 64;
     const int lq = lane % 32;
     const int g = lane / 32;
-    const unsigned items = gridDim.x / 4;
-    unsigned item, quarter;
-    if (items % XCDS == 0) {
-        quarter = blockIdx.x / XCDS % 4;
-        item = blockIdx.x / XCDS / 4 * XCDS + blockIdx.x % XCDS;
-    } else {
-        quarter = blockIdx.x % 4;
-        item = blockIdx.x / 4;
-    }
+    // groups of eight (chunk, head) one behind the other in blockIdx.x, the last of them filled up
+    const unsigned quarter = blockIdx.x / XCDS % 4;
+    const unsigned item = blockIdx.x / XCDS / 4 * XCDS + blockIdx.x % XCDS;
+    if (item / heads * tokens_per_workgroup >= tokens) return;
     const int head = item % heads;
     const long long chunk = item / heads;
     const int column0 = quarter * SLICE;
@@ -564,9 +559,10 @@ void launch_slices(bf16_t* y, const bf16_t* x, const bf16_t* weight, long long t
         }
     }
     const long long chunks = (tokens + per_workgroup - 1) / per_workgroup;
-    check(4 * chunks * heads <= 0x7fffffffLL, "MLA projection: more tokens than the grid allows");
-    hipLaunchKernelGGL(mla_absorb_query_slice_kernel, dim3((unsigned)(4 * chunks * heads)), dim3(THREADS), 0, stream, y, x,
-                       weight, tokens, per_workgroup, heads, strides);
+    const long long grid = 4 * XCDS * ((chunks * heads + XCDS - 1) / XCDS);
+    check(grid <= 0x7fffffffLL, "MLA projection: more tokens than the grid allows");
+    hipLaunchKernelGGL(mla_absorb_query_slice_kernel, dim3((unsigned)grid), dim3(THREADS), 0, stream, y, x, weight, tokens,
+                       per_workgroup, heads, strides);
     HIP_CHECK(hipGetLastError());
 }
 
