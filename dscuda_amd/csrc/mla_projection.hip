@@ -269,8 +269,9 @@ __global__ __launch_bounds__(THREADS) void mla_unabsorb_output_kernel(bf16_t* __
 // 16 heads: absorb 7.6 -> 3.2 us, un-absorb 6.6 -> 3.7.
 //
 // Every 32 tokens fetch the weight again, so the kernels for more tokens win once (token tiles) x heads is large.  Absorb by
-// quarters, below, against few tokens: equal up to 128 tiles, 7.9 / 9.2 us at 256 (1000 tokens of 8 heads; equal for 64 of 128),
-// 9.1 / 12.8 at 512.  Un-absorb, whose weight rows come as 32 bytes of 32 rows an instruction, at 128 tiles 5.1-5.8 against 6.7-9.7 us
+// quarters, below, against few tokens: equal up to 128 tiles, 6.2 / 7.5 us at 256 (128 tokens of 64 heads), 9.1 / 12.8 at 512.  One
+// tile a head fetches it once either way: 7 tokens of 140 heads 8.3 / 4.1, of 500 18.2 / 12.1, 32 of 256 11.7 / 9.3; two tiles, of
+// which four waves leave two idle there: 33 of 70 heads 6.0 / 5.2, 64 of 128 7.8 / 7.5, 33 of 250 (500 tiles) 11.9 / 12.9.  Un-absorb, whose weight rows come as 32 bytes of 32 rows an instruction, at 128 tiles 5.1-5.8 against 6.7-9.7 us
 // (16 tokens of 128 heads, 128 of 32), at 256 tiles 10.2-12.8 against 8.1-9.8.
 constexpr long long ABSORB_FEW_TILES = 128;
 constexpr long long UNABSORB_FEW_TILES = 128;
@@ -411,7 +412,11 @@ __global__ __launch_bounds__(THREADS) void mla_unabsorb_output_few_kernel(bf16_t
 // 1000 x 16 12.4 -> 8.6, 250 x 64 12.8 -> 8.6; into results of their own 42.9 -> 43.3 (3.9 TB/s), 25.6 -> 24.0, 13.4 -> 9.1, 13.5 -> 9.1.
 // Rows written as four times 256 bytes by workgroups of their own are slower once they go to memory.  Whole rows / quarters
 // into results of their own: 144 MB (1100 x 128) 46.8 / 46.6, 157 MB 46.8 / 49.9, 168 MB 48.7 / 51.9, 197 MB 54.4 / 59.3; into those
-// of the call before 157 MB 43.7 / 36.1, 197 MB 51.1 / 42.8, 223 MB 59.7 / 68.1, 268 MB 72.4 / 84.1.
+// of the call before 157 MB 43.7 / 36.1, 197 MB 51.1 / 42.8, 223 MB 59.7 / 68.1, 268 MB 72.4 / 84.1.  From 45 MB on calls of
+// their own are 0 to 10 % slower by quarters (2594 x 34 32.7 / 36.9; 5777 x 11 23.6 / 28.5), but not between the other operators of
+// a layer, absorb, forward and un-absorb: 512 x 128 107.9 / 103.2, 2500 x 32 289.6 / 282.6, 2000 x 64 367.8 / 364.2, 750 x 128 177.0 / 178.1.
+// Up to 128 tokens of so many heads that a workgroup of whole rows a head is a nearly full round, quarters are two rounds:
+// 33 x 250 10.5 / 12.4, 128 x 200 14.9 / 15.5.
 constexpr long long SLICE_RESULT_BYTES = 144LL << 20;
 constexpr int XCDS = 8;
 
@@ -626,10 +631,12 @@ void mla_absorb_query_dispatch(bf16_t* query_latent, const bf16_t* query_nope, c
         HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(mla_absorb_query_kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES));
     });
-    if (!apart || tokens * heads * (2LL * RANK) > SLICE_RESULT_BYTES) {
-        launch_whole(mla_absorb_query_kernel, query_latent, query_nope, weight, tokens, heads, strides, stream);
-    } else if (tiles * heads <= ABSORB_FEW_TILES) {
+    const long long units = compute_units();
+    const bool full_round = tokens <= 4 * TILE && heads <= units && 4LL * heads > 3 * units;   // whole rows, a workgroup a head
+    if (apart && (tiles == 1 || tiles * heads <= (tiles == 2 ? 2 : 1) * ABSORB_FEW_TILES)) {
         launch_few(mla_absorb_query_few_kernel, query_latent, query_nope, weight, tokens, heads, strides, stream);
+    } else if (!apart || full_round || tokens * heads * (2LL * RANK) > SLICE_RESULT_BYTES) {
+        launch_whole(mla_absorb_query_kernel, query_latent, query_nope, weight, tokens, heads, strides, stream);
     } else {
         launch_slices(query_latent, query_nope, weight, tokens, heads, strides, stream);
     }

@@ -50,10 +50,11 @@ def test_unabsorb_output(cuda, batch, seq, heads):
 
 
 @pytest.mark.parametrize("tokens,heads", [(32, 2), (33, 5), (64, 128), (65, 128), (32, 128), (33, 128), (512, 16), (513, 16),
-                                          (128, 32), (129, 32), (1, 128), (1, 129), (1, 257)])
+                                          (128, 32), (129, 32), (1, 128), (1, 129), (1, 257), (32, 300),
+                                          (33, 140), (64, 130), (128, 200), (33, 192), (33, 193), (96, 256), (96, 257)])
 def test_projections_on_either_side_of_the_token_rule(cuda, tokens, heads):
     """Whole and just exceeded token tiles at the largest (token tiles) x heads of the kernels for few tokens, 128, and at
-    twice that.  Weights are slices of wkv_b, rows slices of wider tensors."""
+    twice that; absorb: any heads of one tile, and whole rows where a workgroup a head is a nearly full round.  Weights are slices of wkv_b, rows slices of wider tensors."""
     wkv_b, g = _weights(heads, 53)
     device_weights = wkv_b.to(cuda)
     query = (torch.randn(1, tokens, heads, 192, generator=g) * 0.5).bfloat16()
