@@ -122,4 +122,10 @@ void mla_narrow_forward_launch(__hip_bfloat16* output, float* logsumexp, const _
                                const __hip_bfloat16* key_rope, int batch_size, int sequence_length, int heads,
                                int row_blocks, float scale, hipStream_t stream);
 
+// mla_wide.hip -- the forward with 128 rows per workgroup.
+void mla_wide_forward_launch(__hip_bfloat16* output, float* logsumexp, const __hip_bfloat16* query_latent,
+                             const __hip_bfloat16* query_rope, const __hip_bfloat16* kv_latent,
+                             const __hip_bfloat16* key_rope, int batch_size, int sequence_length, int heads, float scale,
+                             hipStream_t stream);
+
 }  // namespace dscuda

@@ -253,13 +253,19 @@ DSCUDA_HOST_DEVICE inline int narrow_forward_row_blocks(int sequence_length, int
 }
 
 // How many 32-row blocks a workgroup of the absorbed prefill forward holds: 1 or 2 while 128 rows (0: four blocks, the
-// decode's kernel) leave compute units idle.  Whole layer of absorb, forward and un-absorb in us, 32 / 64 / 128 rows: 32 workgroups of 128
-// (512 tokens x 8 heads) 42 / 45 / 61, 128 of them 52 / 52 / 66, 243 of them 236 / 168 / 241, 256 108 / 84 / 103, 391
-// 113 / 95 / 92, 1024 374 / 284 / 268.
+// kernels of mla_wide.hip) leave compute units idle.
+//   * up to half a round of 128-row workgroups: 32 or 64 rows (forward in us, 64 / 128 rows: 130 tokens x 128 heads 15.2 / 17.2)
+//   * up to one round, which 64 rows take in two: 128 rows for most of a round of walks of up to 384 keys (180 x 128
+//     19.3 / 18.5, 256 x 128 24.8 / 22.4, 8 x 125 x 32 23.8 / 17.1, 4 x 250 x 32 28.2 / 22.1, 350 x 80 25.9 / 25.7), 64 for longer
+//     ones, a unit of which takes them a third less (512 x 64 32.0 / 33.8, 1000 x 32 47.9 / 56.2, 2000 x 16 82 / 100)
+//   * beyond: 128 rows, whose second item needs no second start (258 x 128 31.0 / 23.4, 300 x 128 33.9 / 26.1, 1200 x 32 71 / 67,
+//     5 x 64 x 128 26.5 / 23.8), but for walks of one unit, of which they take two (300 x 1 x 40 13.4 / 17.1).
 DSCUDA_HOST_DEVICE inline int forward_row_blocks(int sequence_length, int heads, long long batch, int compute_units) {
     const long long workgroups = ((long long)sequence_length * heads + 127) / 128 * batch;
+    const int units = (sequence_length + 31) / 32;
     if (2 * workgroups <= compute_units) return narrow_forward_row_blocks(sequence_length, heads, batch, compute_units);
-    return 4 * workgroups <= 5LL * compute_units ? 2 : 0;
+    if (workgroups <= compute_units) return units <= 12 && 3 * workgroups > 2LL * compute_units ? 0 : 2;
+    return units == 1 && 4 * workgroups <= 5LL * compute_units ? 2 : 0;
 }
 
 // ---- work order of the persistent forward kernel ------------------------------

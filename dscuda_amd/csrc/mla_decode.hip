@@ -1,15 +1,13 @@
 // Absorbed-weight MLA over a shared 512+64 latent KV stream for gfx950:
-// single-token decode from a paged cache (split-KV + merge) and the causal
-// absorbed prefill forward.  Takes the place of the reference's
+// single-token decode from a paged cache (split-KV + merge), and which kernel
+// takes a prefill forward.  Takes the place of the reference's
 // mla_decode_split_kernel / mla_decode_combine_kernel
-// (kernels/attention/mla/sm89.cu:413-507) and mla_forward_kernel (:156-291);
-// the decomposition below is built around 64-lane MFMA waves and the 160 KB
+// (kernels/attention/mla/sm89.cu:413-507); the decomposition below is built around 64-lane MFMA waves and the 160 KB
 // LDS and shares nothing with their per-head scalar loops.
 //
 // Rows and units
-//   A workgroup (4 waves) owns 128 "rows" -- the heads of one sequence in
-//   decode, consecutive (token, head) pairs in prefill -- and walks the key
-//   stream in units of 32 tokens.  Every row of a workgroup reads the same
+//   A workgroup (4 waves) owns 128 "rows", heads of one sequence, and walks
+//   the key stream in units of 32 tokens.  Every row of a workgroup reads the same
 //   keys, so a 36 KB unit is fetched from HBM once and feeds 128 rows x
 //   (576 + 512) x 2 flop per token: the only way the 242 flop/byte of the
 //   H = 128 decode stays on the HBM roofline.  Each wave owns 32 rows: the
@@ -298,7 +296,7 @@ __device__ __forceinline__ void raise_reference(RowState& state, float& offset, 
 template <bool HAS_NEXT>
 __device__ __forceinline__ void unit_step(RowState& state, f32x16& scores, f32x16& next_scores,
                                           const bf16x8 (&qf)[KSTEPS], const UnitReads& reads,
-                                          const unsigned char* current, const unsigned char* next, int key0, int tokens,  // tokens: of the lane's row
+                                          const unsigned char* current, const unsigned char* next, int key0, int tokens,
                                           float c, const UnitSource& request, const FullUnitOffsets& offsets,
                                           const KeyStream& keys, int wave) {
     constexpr int SCORE_MFMAS = HAS_NEXT ? KSTEPS : 0;
@@ -363,7 +361,7 @@ __device__ __forceinline__ void unit_step(RowState& state, f32x16& scores, f32x1
     if constexpr (!HAS_NEXT) {
         unrolled<0, 33>(softmax_piece);   // the last unit: no score products to hide it behind
     }
-    if (request.enabled && !request.contiguous && !request.split) issue_unit(request, offsets, keys, wave);
+    if (request.enabled && !request.contiguous) issue_unit(request, offsets, keys, wave);
 
     unrolled<0, COUNT>([&](auto tag) {
         constexpr int I = decltype(tag)::value;
@@ -385,7 +383,6 @@ __device__ __forceinline__ void unit_step(RowState& state, f32x16& scores, f32x1
         // the requests go between the output MFMAs, which leave more issue slots free than the score MFMAs
         if constexpr (HAS_NEXT && I >= SCORE_MFMAS && (I - SCORE_MFMAS) % 3 == 1 && (I - SCORE_MFMAS) / 3 < UNIT_LOADS) {
             if (request.enabled && request.contiguous) issue_unit_load(request, offsets, wave, (I - SCORE_MFMAS) / 3, lane);
-            if (request.enabled && request.split) issue_split_load<(I - SCORE_MFMAS) / 3>(request, keys, wave, lane);
         }
         __builtin_amdgcn_sched_barrier(0);
     });
@@ -393,14 +390,11 @@ __device__ __forceinline__ void unit_step(RowState& state, f32x16& scores, f32x1
 
 // Walk tiles [tile_begin, tile_end) of one sequence of keys for the 128 rows of this workgroup
 // with the unit stream, from cleared accumulators (see raise_reference for what happens when a
-// row outruns its softmax reference).  Decode: the rows are the heads of one sequence, each sees
-// all `tokens` keys of the packed cache.  PREFILL: the rows are (token, head) pairs, a lane's row
-// sees the first `row_tokens` <= `tokens` keys (at least one), and the latent and rope parts of
-// the keys lie in tensors of their own.
-template <bool PREFILL>
+// row outruns its softmax reference).  The rows are heads of one sequence, each sees all `tokens`
+// keys of the packed cache.
 __device__ __forceinline__ void walk_units(RowState& state, const bf16_t* query_latent_row, const bf16_t* query_rope_row,
                                            bool valid, unsigned char* lds, const KeyStream& keys, int tile_begin,
-                                           int tile_end, int tokens, int row_tokens, float c, int tid, bool cold) {
+                                           int tile_end, int tokens, float c, int tid, bool cold) {
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const int last_token = tokens - 1;
     const int unit_begin = (BN / UNIT) * tile_begin;
@@ -415,13 +409,6 @@ __device__ __forceinline__ void walk_units(RowState& state, const bf16_t* query_
     load_query(qf, query_latent_row, query_rope_row, valid, (tid % 64) / 32);
     UnitCursor cursor;
     cursor.init(keys, unit_begin, last_token);
-    if constexpr (PREFILL) {
-        cursor.contiguous = false;   // latent and rope parts come from tensors of their own
-        // 32 rows of a unit times the row stride, in bytes, as a 32-bit lane offset
-        cursor.split = keys.block_table == nullptr && keys.latent_stride < ((size_t)1 << 24) &&
-                       keys.rope_stride < ((size_t)1 << 24);
-    }
-    const int visible = PREFILL ? row_tokens : tokens;   // keys the lane's row sees
     FullUnitOffsets offsets;
     offsets.init(wave, fresh_lane_id());
     issue_unit(cursor.next(lds, keys, last_token, wave, unit_end), offsets, keys, wave);
@@ -444,7 +431,7 @@ __device__ __forceinline__ void walk_units(RowState& state, const bf16_t* query_
     f32x16 scores_a, scores_b;
     unit_scores(scores_a, qf, slot_of(unit_begin), reads);
     {
-        mask_unit_scores(scores_a, unit_begin * UNIT, visible, fresh_lane_id() / 32);
+        mask_unit_scores(scores_a, unit_begin * UNIT, tokens, fresh_lane_id() / 32);
         float first_max = scores_a[0];
 #pragma unroll
         for (int i = 1; i < 16; ++i) first_max = fmaxf(first_max, scores_a[i]);
@@ -464,13 +451,13 @@ __device__ __forceinline__ void walk_units(RowState& state, const bf16_t* query_
     int unit = unit_begin;
     for (; unit + 1 < unit_end; ++unit) {
         synchronise(unit);
-        unit_step<true>(state, scores_a, scores_b, qf, reads, slot_of(unit), slot_of(unit + 1), unit * UNIT, visible, c,
+        unit_step<true>(state, scores_a, scores_b, qf, reads, slot_of(unit), slot_of(unit + 1), unit * UNIT, tokens, c,
                         cursor.next(lds, keys, last_token, wave, unit_end), offsets, keys, wave);
         // the next unit's scores take the place of this unit's (eight moves against a stream of 68 MFMAs)
         move_scores(scores_a, scores_b);
     }
     UnitSource nothing = {};
-    unit_step<false>(state, scores_a, scores_b, qf, reads, slot_of(unit), slot_of(unit), unit * UNIT, visible, c, nothing,
+    unit_step<false>(state, scores_a, scores_b, qf, reads, slot_of(unit), slot_of(unit), unit * UNIT, tokens, c, nothing,
                      offsets, keys, wave);
     workgroup_barrier();   // the slots are free: the caller stages its results through them
 }
@@ -623,7 +610,7 @@ __global__ __launch_bounds__(THREADS) void mla_decode_split_kernel(
         keys.rope_stride = WIDTH;
         keys.block_table = block_table + (size_t)sequence * pages_per_sequence;
         keys.page_size = page_size;
-        walk_units<false>(state, query_row, query_row + RANK, valid, lds, keys, tile_begin, tile_end, tokens, tokens, c, tid,
+        walk_units(state, query_row, query_row + RANK, valid, lds, keys, tile_begin, tile_end, tokens, c, tid,
                           position == range_begin);
         const float total_sum = half_wave_sum(state.row_sum);
 
@@ -784,61 +771,6 @@ __global__ __launch_bounds__(64) void mla_decode_merge_kernel(bf16_t* __restrict
     }
 }
 
-// ----------------------------------------------------------------------------
-// absorbed causal prefill forward
-// ----------------------------------------------------------------------------
-
-__global__ __launch_bounds__(THREADS) void mla_absorbed_forward_kernel(
-    bf16_t* __restrict__ output, float* __restrict__ logsumexp, const bf16_t* __restrict__ query_latent,
-    const bf16_t* __restrict__ query_rope, const bf16_t* __restrict__ kv_latent, const bf16_t* __restrict__ key_rope,
-    int sequence_length, int heads, int row_blocks, float scale) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    const int tid = threadIdx.x;
-    const int lane = tid % 64;
-    const int wave = tid / 64;
-    const int lq = lane % 32;
-    const int g = lane / 32;
-    const float c = uniform(scale * LOG2E);
-
-    // heaviest (latest) row blocks first
-    const int batch = blockIdx.x / row_blocks;
-    const int row_block = row_blocks - 1 - blockIdx.x % row_blocks;
-    const long long rows = (long long)sequence_length * heads;   // (token, head) pairs of one batch element
-    const long long row0 = (long long)row_block * ROWS;
-    const long long row = row0 + 32 * wave + lq;
-    const bool valid = row < rows;
-    const bool wave_active = row0 + 32 * wave < rows;
-    const int token = valid ? (int)(row / heads) : 0;
-    const int head = valid ? (int)(row % heads) : 0;
-    const long long global_row = (long long)batch * rows + (valid ? row : 0);
-
-    RowState state;
-
-    const long long last_row = min(rows, row0 + ROWS) - 1;
-    const int visible = (int)(last_row / heads) + 1;  // keys any row of this block may see
-    KeyStream keys;
-    keys.latent = kv_latent + (size_t)batch * sequence_length * RANK;
-    keys.rope = key_rope + (size_t)batch * sequence_length * ROPE;
-    keys.latent_stride = RANK;
-    keys.rope_stride = ROPE;
-    keys.block_table = nullptr;
-    keys.page_size = 0;
-    walk_units<true>(state, query_latent + global_row * RANK, query_rope + global_row * ROPE, valid, lds, keys, 0,
-                     tiles_of(visible), visible, valid ? token + 1 : visible, c, tid, true);
-
-    if (!wave_active) return;
-    const float total_sum = half_wave_sum(state.row_sum);
-    if (valid && g == 0) {
-        logsumexp[((size_t)batch * heads + head) * sequence_length + token] =
-            (state.reference + __builtin_amdgcn_logf(total_sum)) * LN2;
-    }
-    unsigned char* wave_lds = lds + wave * 32 * EPILOGUE_PITCH;
-    store_final(state, 1.0f / total_sum, wave_lds, lane, [&](int r) -> bf16_t* {
-        const long long rr = row0 + 32 * wave + r;
-        return rr < rows ? output + ((long long)batch * rows + rr) * RANK : nullptr;
-    });
-}
-
 constexpr int LDS_BYTES = UNIT_SLOTS * UNIT_BYTES;
 
 template <typename Kernel>
@@ -928,8 +860,7 @@ void mla_decode_dispatch(bf16_t* output, float* logsumexp, const bf16_t* query, 
 void mla_absorbed_forward_dispatch(bf16_t* output, float* logsumexp, const bf16_t* query_latent,
                                    const bf16_t* query_rope, const bf16_t* kv_latent, const bf16_t* key_rope,
                                    int batch_size, int sequence_length, int heads, float scale, hipStream_t stream) {
-    const long long rows = (long long)sequence_length * heads;
-    const long long row_blocks = (rows + ROWS - 1) / ROWS;
+    const long long row_blocks = ((long long)sequence_length * heads + ROWS - 1) / ROWS;
     if (row_blocks * batch_size > 0x7fffffffLL) {
         throw std::invalid_argument("MLA forward: batch*tokens*heads exceeds the grid limit");
     }
@@ -939,12 +870,8 @@ void mla_absorbed_forward_dispatch(bf16_t* output, float* logsumexp, const bf16_
                                   sequence_length, heads, narrow, scale, stream);
         return;
     }
-    static hip_common::OncePerDevice prepared;
-    prepared.run([] { allow_large_lds(mla_absorbed_forward_kernel); });
-    hipLaunchKernelGGL(mla_absorbed_forward_kernel, dim3((unsigned)(row_blocks * batch_size)), dim3(THREADS), LDS_BYTES,
-                       stream, output, logsumexp, query_latent, query_rope, kv_latent, key_rope, sequence_length, heads,
-                       (int)row_blocks, scale);
-    HIP_CHECK(hipGetLastError());
+    mla_wide_forward_launch(output, logsumexp, query_latent, query_rope, kv_latent, key_rope, batch_size, sequence_length,
+                            heads, scale, stream);
 }
 
 }  // namespace dscuda

@@ -1,0 +1,635 @@
+// Absorbed MLA attention, 128 query rows a workgroup: the causal prefill forward.  Takes the place of the reference's
+// mla_forward_kernel (kernels/attention/mla/sm89.cu:156-291); the decomposition below is built around 64-lane MFMA waves and the 160 KB LDS and
+// shares nothing with their per-head scalar loops.
+//
+// Rows and units
+//   A workgroup owns 128 rows, consecutive (token, head) pairs, and walks
+//   a stream of keys in units of 32.  Every row reads the same keys, so a unit is fetched once for 128 rows x (576 + 512)
+//   x 2 flop per key.
+//
+// Eight waves, two a SIMD
+//   scores     S^T (32 keys x 16 rows) = K Q^T: a wave has 16 rows, their 576 columns as operands in 72 registers
+//              (16x16x32 MFMA, two key halves, 18 steps), the exponentials of its scores, and leaves P as bf16 in LDS
+//   products   O^T (64 columns x 128 rows) += V^T P^T: a wave has 64 of the 512 columns of all rows, 128 registers
+//              (32x32x16 MFMA, 16 a unit); a V fragment is read once in the workgroup, P by all waves
+//   In a step the products of unit n and the scores of unit n + 1 go side by side: waves 0..3 take the products first,
+//   waves 4..7 (on the same SIMDs) the scores, so that one's exponentials run beside the other's MFMAs; one barrier ends
+//   the step.  With four waves of 32 rows each, 512 registers a wave and one wave a SIMD, a wave's scores, exponentials,
+//   LDS reads and products queue up behind each other: a step takes 3800 to 4100 cycles there and 3200 here, of which
+//   2176 are MFMAs (forward in us, four waves -> here, 128 heads: 1024 tokens 176 -> 140, 2048 583 -> 508, 4096 2110 -> 1880;
+//   3 x 700 x 33 87 -> 66, 40 x 130 x 16 57 -> 42, 7 x 257 x 128 167 -> 123).
+//
+// The stream runs on over the ends of items
+//   A workgroup takes several items (blocks of 128 rows), one a compute unit being all that the
+//   registers and the LDS hold.  Units are requested three steps ahead, the next item's among them; the query rows of the
+//   next item are asked for as the last scores of this one release their registers.  An item used to cost 12 to 20 us
+//   besides its units (a workgroup's start, query rows and first units, its rows on their way out), now some 7, of which
+//   the query rows take most: 147 KB at the 21 bytes a cycle that a compute unit draws.
+//
+// LDS
+//   Four slots of 32 latent rows, three of 32 rope rows (a unit's rope rows are only read for its scores, a step before
+//   its values), P of two units: 156 of 160 KB.  A latent row is one 1 KB request
+//   (global_load_lds, 16 bytes a lane): its address is a scalar, the swizzle of index_math::tile_swizzle a lane's constant.
+//   Bank conflicts: ds_read_b128 serves lanes 0-3, 12-15, 20-27 together, then 4-11, 16-19, 28-31, and the same of the
+//   upper half.  The 16x16x32 operand (row lane % 16, chunk lane / 16) meets itself there under the tiles' swizzle; with
+//   the four chunks of a step dealt to the lane groups in the order 0, 3, 1, 2 -- in the query rows as well, the sum over
+//   them is the same -- it does not: 1430 of 3100 LDS cycles a unit were conflicts (2048 tokens x 128 heads 575 -> 525 us).
+//
+// Softmax reference
+//   Exponentials are taken against a fixed reference, the maximum of the row's first unit plus 2^40.  A row whose scores
+//   outrun it by more than 2^80 (next to never) has its item walked a second time, against the maxima found.
+#include "attn_kernels.h"
+#include "hip_common.h"
+#include "index_math.h"
+#include "latent_stream.h"
+
+#include <algorithm>
+#include <cstdint>
+#include <stdexcept>
+
+namespace dscuda {
+namespace {
+
+constexpr int WIDE_WAVES = 8;
+constexpr int WIDE_THREADS = 64 * WIDE_WAVES;
+constexpr int WIDE_ROWS = index_math::DECODE_ROWS;
+constexpr int ROW_TILES = WIDE_ROWS / 32;                    // 4
+constexpr int WAVE_COLUMNS = RANK / WIDE_WAVES;              // 64 output columns of a wave
+constexpr int WAVE_BLOCKS = WAVE_COLUMNS / 32;               // 2
+constexpr int LATENT_BYTES = 2 * RANK;                       // of a latent row
+constexpr int ROPE_BYTES = 2 * ROPE;
+constexpr int LATENT_SLOT = UNIT * LATENT_BYTES;             // 32 KB
+constexpr int ROPE_SLOT = UNIT * ROPE_BYTES;                 // 4 KB
+constexpr int ROPE_SLOTS = UNIT_SLOTS - 1;
+constexpr int ROPE_AT = UNIT_SLOTS * LATENT_SLOT;
+constexpr int LATENT_STEPS = RANK / 32;                      // 16
+constexpr int SCORE_STEPS = WIDTH / 32;                      // 18
+constexpr int P_BYTES = UNIT * WIDE_ROWS * 2;                // 8 KB: [16 keys][32 rows][lane g][row][8 keys]
+constexpr int P_HALF = P_BYTES / 2;
+constexpr int P_AT = ROPE_AT + ROPE_SLOTS * ROPE_SLOT;
+constexpr int SUMS_AT = P_AT + 2 * P_BYTES;                  // [128] reciprocal sums of the rows
+constexpr int WIDE_LDS_BYTES = SUMS_AT + WIDE_ROWS * 4;
+static_assert(WIDE_LDS_BYTES <= 160 * 1024, "all there is");
+static_assert(LATENT_SLOT + ROPE_SLOT == UNIT_BYTES, "a unit");
+
+// Fragments read ahead of the MFMA that takes them (1024 / 2048 tokens x 128 heads: three 159 / 537 us, two 161 / 551,
+// four 160 / 542, six, which spill, 163 / 550).
+constexpr int KEY_RING = 3;
+// The 18 loads of the next query rows: 9 beside the last scores, 8 beside the last products, the last one behind them.
+// All beside the last scores, the waves stood at a full request queue for 6500 cycles (1024 x 128 147 -> 139 us).
+constexpr int QUERY_SCORES = 9;
+constexpr int QUERY_PRODUCTS = 17;
+
+constexpr float HEADROOM = 40.0f;
+constexpr float OUTRUN = 80.0f;
+
+typedef short wide_s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) wide_s16x4* wide_tr_pointer;
+
+using LatentReads = index_math::TileReadMath<LATENT_BYTES>;
+using RopeReads = index_math::TileReadMath<ROPE_BYTES>;
+
+// The order of the k-steps: of a row's 256-byte groups, the two lines of 128 bytes one after the other (steps of one line
+// are neighbours for the query loads; at most two chunk positions are live in the key reads).
+__device__ constexpr int step_of(int place) {
+    return place < LATENT_STEPS ? 4 * (place % 8 / 2) + 2 * (place / 8) + place % 2 : place;
+}
+
+// Chunk of a k-step that lane group q = lane / 16 of a 16x16x32 operand holds (see above).
+__device__ __forceinline__ int chunk_of_group(int q) {
+    return (q >> 1) ^ (3 * (q & 1));   // 0, 3, 1, 2
+}
+
+// over the lanes l, l ^ 16, l ^ 32, l ^ 48
+__device__ __forceinline__ float wide_quarter_max(float value) {
+    value = fmaxf(value, __shfl_xor(value, 16));
+    return half_wave_max(value);
+}
+
+__device__ __forceinline__ float wide_quarter_sum(float value) {
+    value += __shfl_xor(value, 16);
+    return half_wave_sum(value);
+}
+
+// ---- what a workgroup walks ---------------------------------------------------------------------------------------
+//
+// A Work is a kernel's argument.  It names the items of a workgroup, one after the other (Iterator), the rows of an item, and where the keys of its
+// units lie (Keys: first row of the unit at hand and the last row that holds a visible token, which those behind it
+// repeat).  An item has at least two units; one past its keys is masked as a whole.
+
+// A kernel's argument, read anew from the constant memory at every use: held in scalar registers from the kernel's start to
+// its end, its fields pushed what the loops use out into lanes of vector registers, and those into scratch.
+template <typename Work>
+struct Argument {
+    const __attribute__((address_space(4))) Work* place;
+
+    __device__ __forceinline__ Argument() {
+        place = (const __attribute__((address_space(4))) Work*)__builtin_amdgcn_kernarg_segment_ptr();   // the first argument
+    }
+    __device__ __forceinline__ const Work& operator*() const {
+        const __attribute__((address_space(4))) Work* fresh = place;
+        asm volatile("" : "+s"(fresh));
+        return *(const Work*)fresh;
+    }
+    __device__ __forceinline__ const Work* operator->() const { return &**this; }
+};
+
+// Prefill: 128 consecutive (token, head) pairs of a batch element.
+struct ForwardWork {
+    static constexpr int LATENT_STRIDE = 2 * RANK;   // bytes, of keys and query rows
+    static constexpr int ROPE_STRIDE = 2 * ROPE;
+
+    bf16_t* output;
+    float* logsumexp;
+    const bf16_t* query_latent;
+    const bf16_t* query_rope;
+    const bf16_t* kv_latent;
+    const bf16_t* key_rope;
+    int sequence_length;
+    int heads;
+    unsigned rows;                       // (token, head) pairs of a batch element
+    unsigned items;
+    unsigned row_blocks;
+    bool interleaved;                    // the batch elements' blocks are numbered together
+    index_math::FastDivision by_heads;
+    index_math::FastDivision by_order;   // batch elements (interleaved), row blocks of one
+    float c;
+
+    struct Place {};                     // what a workgroup knows of itself
+
+    struct Item {
+        int batch;
+        unsigned row0;
+        int tokens;                      // keys that any of its rows sees
+        int unit_begin;
+        int units;
+    };
+
+    // The heaviest blocks first, rounds there and back: a workgroup's items add up to the same for all.
+    struct Iterator {
+        int round;
+
+        __device__ __forceinline__ bool next(const ForwardWork& work, const Place&, Item& item) {
+            const unsigned place = round & 1 ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
+            const unsigned index = (unsigned)round * gridDim.x + place;
+            ++round;
+            if (index >= work.items) return false;
+            const unsigned quotient = index_math::divide(index, work.by_order);
+            const unsigned rest = index - quotient * work.by_order.divisor;
+            item.batch = (int)(work.interleaved ? rest : quotient);
+            item.row0 = (work.row_blocks - 1 - (work.interleaved ? quotient : rest)) * WIDE_ROWS;
+            const unsigned last_row = min(work.rows, item.row0 + WIDE_ROWS) - 1;
+            item.tokens = (int)index_math::divide(last_row, work.by_heads) + 1;
+            item.unit_begin = 0;
+            item.units = max((item.tokens + UNIT - 1) / UNIT, 2);
+            return true;
+        }
+    };
+
+    struct Keys {
+        const unsigned char* latent;
+        const unsigned char* rope_rows;
+        int limit;
+
+        __device__ __forceinline__ const unsigned char* rope() const { return rope_rows; }
+        __device__ __forceinline__ void open(const ForwardWork& work, const Item& item, unsigned char*, int) {
+            const size_t first = (size_t)item.batch * work.sequence_length;
+            latent = reinterpret_cast<const unsigned char*>(work.kv_latent + first * RANK);
+            rope_rows = reinterpret_cast<const unsigned char*>(work.key_rope + first * ROPE);
+            limit = item.tokens - 1;
+        }
+        __device__ __forceinline__ int look_up(const unsigned char*, int) const { return 0; }
+        __device__ __forceinline__ void next(int, unsigned char*, int) {
+            const int rows = min(limit, UNIT);   // fewer: no visible token behind them, the last row stands for the unit
+            latent += rows * LATENT_STRIDE;
+            rope_rows += rows * ROPE_STRIDE;
+            limit -= rows;
+        }
+    };
+
+    __device__ __forceinline__ unsigned valid_rows(const Place&, const Item& item) const {
+        return min(rows - item.row0, (unsigned)WIDE_ROWS);
+    }
+    __device__ __forceinline__ size_t query_row(const Place&, const Item& item, unsigned row) const {
+        return (size_t)item.batch * rows + item.row0 + row;
+    }
+    __device__ __forceinline__ const bf16_t* latent_row(const Place& place, const Item& item, unsigned row) const {
+        return query_latent + query_row(place, item, row) * RANK;
+    }
+    __device__ __forceinline__ const bf16_t* rope_row(const Place& place, const Item& item, unsigned row) const {
+        return query_rope + query_row(place, item, row) * ROPE;
+    }
+    __device__ __forceinline__ void store_logsumexp(const Place&, const Item& item, unsigned row, float value) const {
+        const unsigned token = index_math::divide(item.row0 + row, by_heads);
+        const unsigned head = item.row0 + row - token * heads;
+        logsumexp[((size_t)item.batch * heads + head) * sequence_length + token] = value;
+    }
+    // keys that a row of the item sees
+    __device__ __forceinline__ int visible(const Item& item, unsigned row) const {
+        return (int)index_math::divide(item.row0 + row, by_heads) + 1;
+    }
+};
+
+// The unit requested next; runs ahead of the products, over the ends of items.
+template <typename Work>
+struct WideCursor {
+    typename Work::Iterator items;
+    typename Work::Keys keys;
+    int left;   // units of the item from this one on; 0: no more items
+
+    __device__ __forceinline__ bool enabled() const { return left > 0; }
+    __device__ __forceinline__ void open(const Argument<Work>& work, const typename Work::Item& item, unsigned char* lds,
+                                         int wave) {
+        left = __builtin_amdgcn_readfirstlane(item.units);
+        keys.open(*work, item, lds, wave);
+    }
+    // (ahead: what keys.look_up returned)
+    __device__ __forceinline__ void advance(const Argument<Work>& work, const typename Work::Place& place, int ahead,
+                                            unsigned char* lds, int wave) {
+        if (left == 0) return;
+        if (--left > 0) {
+            keys.next(ahead, lds, wave);
+            return;
+        }
+        typename Work::Item item;
+        if (items.next(*work, place, item)) open(work, item, lds, wave);
+    }
+};
+
+// A workgroup's stream: the item at hand and those that `items` names after it.  LATE: waves 4..7, scores before products.
+template <typename Work, bool LATE>
+__device__ __forceinline__ void wide_stream(const typename Work::Place place, typename Work::Item item,
+                                            typename Work::Iterator items, unsigned char* lds, const int wave) {
+    using Item = typename Work::Item;
+    constexpr int REQUESTS = LATE ? 4 : 5;    // of a wave and unit
+    const unsigned lds0 = lds_offset_of(lds);
+    const Argument<Work> work;
+    const float c = work->c;
+
+    WideCursor<Work> cursor;
+    // request I (0..3 a latent row, 4 eight rope rows, of the early waves) of the cursor's unit, the stream's unit n
+    auto issue = [&](int n, auto tag) {
+        constexpr int I = decltype(tag)::value;
+        if (!cursor.enabled()) return;
+        auto load = [&](const unsigned char* base, unsigned offset, unsigned target) {
+            direct_load_16_offset(base, offset, target);
+        };
+        const int lane = fresh_lane_id();
+        if constexpr (I < 4) {
+            const int line = 4 * wave + I;
+            const unsigned target = lds0 + ((unsigned)n % UNIT_SLOTS) * LATENT_SLOT + line * LATENT_BYTES;
+            const unsigned chunk = 16 * (lane ^ (wave & 3)) ^ (64u * I);   // 16 * (lane ^ tile_swizzle(line))
+            load(cursor.keys.latent + min(line, cursor.keys.limit) * Work::LATENT_STRIDE, chunk, target);
+        } else if constexpr (!LATE) {
+            const int line = 8 * wave + lane / 8;
+            const unsigned chunk = 16 * ((lane % 8) ^ index_math::tile_swizzle<ROPE_BYTES>(line));
+            const unsigned target = lds0 + ROPE_AT + ((unsigned)n % ROPE_SLOTS) * ROPE_SLOT + wave * 1024;
+            load(cursor.keys.rope(), min(line, cursor.keys.limit) * Work::ROPE_STRIDE + chunk, target);
+        }
+    };
+    auto issue_all = [&](int n) {
+        const int ahead = cursor.keys.look_up(lds, wave);
+        unrolled<0, 5>([&](auto tag) { issue(n, tag); });
+        cursor.advance(work, place, ahead, lds, wave);
+    };
+
+    f32x16 out[ROW_TILES][WAVE_BLOCKS];   // 32 rows x 32 columns each
+    bf16x8 qf[SCORE_STEPS];
+    // of the lane's row 16 * wave + lane % 16
+    float reference, row_sum, highest;
+    const bf16_t* next_latent = nullptr;   // the lane's part of the query row that is loaded next
+    const bf16_t* next_rope = nullptr;
+    // (needed: there is a next item; otherwise the loads, which stay in the code, fetch a line each for all lanes)
+    auto find_query = [&](const Item& of, bool needed) {
+        const int lane = fresh_lane_id();
+        const int first = needed ? 8 * chunk_of_group(lane / 16) : 0;
+        // rows past the end repeat the last one, nothing of theirs is stored
+        const unsigned row = needed ? min((unsigned)(16 * wave + lane % 16), work->valid_rows(place, of) - 1) : 0;
+        next_latent = work->latent_row(place, of, row) + first;
+        next_rope = work->rope_row(place, of, row) + first;
+    };
+    auto load_query = [&](auto place) {
+        constexpr int S = step_of(decltype(place)::value);
+        qf[S] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(
+                                               S < LATENT_STEPS ? next_latent + 32 * S : next_rope + 32 * (S - LATENT_STEPS)));
+    };
+
+    // Offsets of the fragment reads in the slot at hand; the other chunks of a 256-byte group are one XOR away.
+    unsigned key_at, rope_at, value_at[2];
+    {
+        const int lane = fresh_lane_id();
+        const int operand = 16 * chunk_of_group(lane / 16) + lane % 16;
+        key_at = LatentReads::quadrant(0, operand);
+        rope_at = ROPE_AT + RopeReads::quadrant(0, operand);
+        // lanes 32..63 take the two key groups of their four rows in the other order, as P has them
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            value_at[h] = LatentReads::transposed(h ^ (lane / 32), 2 * (wave & 1), lane) + (wave >> 1) * 256;
+        }
+    }
+    auto latent_step = [&](int n) {   // from a unit's slot to the next one's
+        return (unsigned)n % UNIT_SLOTS == UNIT_SLOTS - 1 ? 0u - (UNIT_SLOTS - 1) * LATENT_SLOT : (unsigned)LATENT_SLOT;
+    };
+    auto rope_step = [&](int n) {
+        return (unsigned)n % ROPE_SLOTS == ROPE_SLOTS - 1 ? 0u - (ROPE_SLOTS - 1) * ROPE_SLOT : (unsigned)ROPE_SLOT;
+    };
+
+    int all_visible = 0;   // keys that all rows of the item see
+    f32x4 scores[2];
+    // Scores of the stream's unit n, unit `unit` of its item.  LAST: of its item; the query rows of the next one are asked
+    // for as those of this one have been used.
+    auto form_scores = [&](const Item& of, int n, int unit, auto last) {
+        // fragment F: key half F % 2 of the k-step in place F / 2
+        auto fragment = [&](auto tag) -> bf16x8 {
+            constexpr int F = decltype(tag)::value;
+            constexpr int S = step_of(F / 2);
+            if constexpr (S < LATENT_STEPS) {
+                return *reinterpret_cast<const bf16x8*>(lds + (key_at ^ (64 * (S % 4))) + (S / 4) * 256 + (F % 2) * 16 * LATENT_BYTES);
+            } else {
+                return *reinterpret_cast<const bf16x8*>(lds + (rope_at ^ (64 * (S % 2))) + (F % 2) * 16 * ROPE_BYTES);
+            }
+        };
+        constexpr int COUNT = 2 * SCORE_STEPS;
+        bf16x8 ring[KEY_RING];
+        unrolled<0, KEY_RING>([&](auto tag) { ring[decltype(tag)::value] = fragment(tag); });
+        scores[0] = scores[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // The chain of scores is what a step waits for: its MFMAs go first (531 against 550 us, 2048 tokens x 128 heads).
+        __builtin_amdgcn_s_setprio(1);
+        unrolled<0, COUNT>([&](auto tag) {
+            constexpr int F = decltype(tag)::value;
+            scores[F % 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ring[F % KEY_RING], qf[step_of(F / 2)], scores[F % 2], 0, 0, 0);
+            if constexpr (F + KEY_RING < COUNT) ring[F % KEY_RING] = fragment(std::integral_constant<int, F + KEY_RING>{});
+            if constexpr (decltype(last)::value && F % 2 == 1 && F / 2 < QUERY_SCORES) load_query(std::integral_constant<int, F / 2>{});
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        __builtin_amdgcn_s_setprio(0);
+        key_at += latent_step(n);
+        rope_at += rope_step(n);
+        const int first = (of.unit_begin + unit) * UNIT;
+        if (first + UNIT > all_visible) {
+            const int lane = fresh_lane_id();
+            const unsigned row = min((unsigned)(16 * wave + lane % 16), work->valid_rows(place, of) - 1);
+            const int hidden = work->visible(of, row) - first - 4 * (lane / 16);   // the lane's keys 16 * k + i from there on
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (16 * k + i >= hidden) scores[k][i] = -INFINITY;
+                }
+            }
+        }
+    };
+    auto lane_max = [&]() {
+        float value = fmaxf(scores[0][0], scores[1][0]);
+#pragma unroll
+        for (int i = 1; i < 4; ++i) value = fmaxf(value, fmaxf(scores[0][i], scores[1][i]));
+        return value;
+    };
+    auto write_probabilities = [&](int n) {
+        // Keys 4q .. 4q + 3 of a half: the 8 bytes q / 2 of lane group g = q % 2 of the product's operand, the other way
+        // round for g = 1, so that the two groups write to different banks.
+        const int lane = fresh_lane_id();
+        const unsigned to = P_AT + (n & 1) * P_BYTES + (wave / 2) * 1024 + (wave & 1) * 256 + (lane & 15) * 16 +
+                            ((lane >> 4) & 1) * 512 + (((lane >> 5) ^ (lane >> 4)) & 1) * 8;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            float p[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                p[i] = __builtin_amdgcn_exp2f(fmaf(scores[k][i], c, -reference));
+                row_sum += p[i];
+            }
+            const u32x2 packed = {pack_bf16(p[0], p[1]), pack_bf16(p[2], p[3])};
+            *reinterpret_cast<u32x2*>(lds + to + k * P_HALF) = packed;
+        }
+    };
+    auto score_phase = [&](const Item& of, int n, int unit, auto last) {
+        form_scores(of, n, unit, last);
+        highest = fmaxf(highest, lane_max());
+        write_probabilities(n);
+    };
+    // Products of the stream's unit n, and the requests of unit n + 3 into the slot that unit n - 1 has left.
+    auto output_phase = [&](int n, auto last) {
+        const int ahead = cursor.keys.look_up(lds, wave);
+        const unsigned p_at = P_AT + 16 * fresh_lane_id() + (n & 1) * P_BYTES;
+        auto value_fragment = [&](auto half, auto d) -> bf16x8 {
+            constexpr int AT = decltype(half)::value * 16 * LATENT_BYTES;
+            constexpr int D = decltype(d)::value;
+            const wide_s16x4 low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((wide_tr_pointer)(lds + (value_at[0] ^ (64 * D)) + AT));
+            const wide_s16x4 high = __builtin_amdgcn_ds_read_tr16_b64_v4i16((wide_tr_pointer)(lds + (value_at[1] ^ (64 * D)) + AT));
+            return __builtin_bit_cast(bf16x8, __builtin_shufflevector(low, high, 0, 1, 2, 3, 4, 5, 6, 7));
+        };
+        auto p_fragment = [&](int half, int b) -> bf16x8 {
+            return *reinterpret_cast<const bf16x8*>(lds + p_at + half * P_HALF + b * 1024);
+        };
+        using Zero = std::integral_constant<int, 0>;
+        using One = std::integral_constant<int, 1>;
+        bf16x8 vf[WAVE_BLOCKS], pf[ROW_TILES];
+        vf[0] = value_fragment(Zero{}, Zero{});
+#pragma unroll
+        for (int b = 0; b < ROW_TILES; ++b) pf[b] = p_fragment(0, b);
+        vf[1] = value_fragment(Zero{}, One{});
+        unrolled<0, 16>([&](auto tag) {
+            constexpr int M = decltype(tag)::value;
+            constexpr int HALF = M / 8, D = (M / 4) % 2, B = M % 4;
+            out[B][D] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[D], pf[B], out[B][D], 0, 0, 0);
+            if constexpr (HALF == 0 && D == 1) pf[B] = p_fragment(1, B);
+            if constexpr (M == 3) vf[0] = value_fragment(One{}, Zero{});
+            if constexpr (M == 7) vf[1] = value_fragment(One{}, One{});
+            if constexpr (M % 3 == 1 && M / 3 < 5) issue(n + 3, std::integral_constant<int, M / 3>{});
+            if constexpr (decltype(last)::value && M % 2 == 1 && QUERY_SCORES + M / 2 < QUERY_PRODUCTS) {
+                load_query(std::integral_constant<int, QUERY_SCORES + M / 2>{});
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        value_at[0] += latent_step(n);
+        value_at[1] += latent_step(n);
+        cursor.advance(work, place, ahead, lds, wave);
+    };
+
+    int n = 0;              // unit of the stream
+    bool restart = true;    // the stream starts (again) with the item at hand
+    bool again = false;     // the item is walked a second time, against the maxima of its rows
+    // Scores of an item's first unit, and the reference every exponential of its walk is taken against.
+    auto first_scores = [&](const Item& of, int at) {
+        all_visible = work->visible(of, 0);
+        form_scores(of, at, 0, std::false_type{});
+        reference = again ? wide_quarter_max(highest) * c : wide_quarter_max(lane_max()) * c + HEADROOM;
+        highest = lane_max();
+        row_sum = 0.f;
+        write_probabilities(at);
+    };
+    while (true) {
+        if (restart) {
+            // At the start of the kernel every workgroup asks at once and the answers come at the rate of the memory: what
+            // the first scores need is asked for first.
+            cursor.items = items;
+            cursor.open(work, item, lds, wave);
+            find_query(item, true);
+            unrolled<0, SCORE_STEPS>(load_query);
+            issue_all(n);
+            wait_vector_memory<0>();
+            workgroup_barrier();
+            issue_all(n + 1);
+            issue_all(n + 2);
+            first_scores(item, n);
+            wait_vector_memory<0>();
+            restart = false;
+        }
+        workgroup_barrier();   // the first probabilities are there
+#pragma unroll
+        for (int b = 0; b < ROW_TILES; ++b) {
+#pragma unroll
+            for (int d = 0; d < WAVE_BLOCKS; ++d) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) out[b][d][i] = 0.f;
+            }
+        }
+        const int units = __builtin_amdgcn_readfirstlane(item.units);
+        int unit = 0;
+        for (; unit + 2 < units; ++unit, ++n) {
+            const bool requested = cursor.enabled();
+            if (LATE) score_phase(item, n + 1, unit + 1, std::false_type{});
+            output_phase(n, std::false_type{});
+            if (!LATE) score_phase(item, n + 1, unit + 1, std::false_type{});
+            // unit n + 2 has landed; only this wave's share of unit n + 3 may still be on its way
+            if (requested) wait_vector_memory<REQUESTS>(); else wait_vector_memory<0>();
+            workgroup_barrier();
+        }
+        bool more;
+        {
+            typename Work::Iterator ahead = items;   // which stays: a second walk starts the stream from there
+            Item next = item;
+            more = ahead.next(*work, place, next);
+            find_query(next, more);
+        }
+        {
+            const bool requested = cursor.enabled();
+            if (LATE) score_phase(item, n + 1, unit + 1, std::true_type{});
+            output_phase(n, std::false_type{});
+            if (!LATE) score_phase(item, n + 1, unit + 1, std::true_type{});
+            if (requested) wait_vector_memory<REQUESTS + QUERY_SCORES>(); else wait_vector_memory<0>();
+            workgroup_barrier();
+            ++n;
+        }
+        float* inverses = reinterpret_cast<float*>(lds + SUMS_AT);
+        const float total = wide_quarter_sum(row_sum);
+        {
+            // (not twice: of scores beyond 2^24 the maximum itself is that far from its rounded product with c)
+            const bool outrun = !again && fmaf(wide_quarter_max(highest), c, -reference) > OUTRUN;
+            const int lane = fresh_lane_id();
+            if (lane < 16) inverses[16 * wave + lane] = outrun ? -1.0f : 1.0f / total;
+            const bool requested = cursor.enabled();
+            output_phase(n, std::true_type{});
+            // behind unit n + 2's requests: query rows (early waves: of both phases), the requests of unit n + 3
+            if (!requested) wait_vector_memory<0>();
+            else if (LATE) wait_vector_memory<REQUESTS + QUERY_PRODUCTS - QUERY_SCORES>();
+            else wait_vector_memory<REQUESTS + QUERY_PRODUCTS>();
+            workgroup_barrier();
+        }
+        unrolled<QUERY_PRODUCTS, SCORE_STEPS>(load_query);
+        const int lane = fresh_lane_id();
+        const int lq = lane % 32;
+        float inverse[ROW_TILES];
+#pragma unroll
+        for (int b = 0; b < ROW_TILES; ++b) inverse[b] = inverses[32 * b + lq];
+        const float least = fminf(fminf(inverse[0], inverse[1]), fminf(inverse[2], inverse[3]));
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(least < 0.f) != 0, 0)) {
+            wait_vector_memory<0>();
+            workgroup_barrier();   // what was on its way has arrived, everybody has read the verdict
+            again = restart = true;
+            ++n;
+            continue;
+        }
+        again = false;
+        const unsigned valid = work->valid_rows(place, item);
+        const unsigned own_row = 16 * wave + lane;   // of lanes 0..15
+        if (lane < 16 && own_row < valid) work->store_logsumexp(place, item, own_row, (reference + __builtin_amdgcn_logf(total)) * LN2);
+        // The rows leave through the slot of the last unit, a tile of 32 rows x the wave's 128 bytes at a time, eight
+        // whole lines an instruction, past the caches (1024 tokens x 128 heads 153 -> 143 us).
+        unsigned char* staged = lds + ((unsigned)n % UNIT_SLOTS) * LATENT_SLOT + wave * (32 * 2 * WAVE_COLUMNS);
+        bf16_t* rows = work->output + work->query_row(place, item, 0) * RANK + wave * WAVE_COLUMNS;
+        const int to = lq * 128 + 8 * (lane / 32), flip = (lq >> 1) & 7;
+        const int line8 = lane / 8, piece = lane % 8;
+#pragma unroll
+        for (int b = 0; b < ROW_TILES; ++b) {
+#pragma unroll
+            for (int d = 0; d < WAVE_BLOCKS; ++d) {
+#pragma unroll
+                for (int i4 = 0; i4 < 4; ++i4) {
+                    u32x2 packed;
+                    packed.x = pack_bf16(out[b][d][4 * i4 + 0] * inverse[b], out[b][d][4 * i4 + 1] * inverse[b]);
+                    packed.y = pack_bf16(out[b][d][4 * i4 + 2] * inverse[b], out[b][d][4 * i4 + 3] * inverse[b]);
+                    *reinterpret_cast<u32x2*>(staged + to + 16 * ((4 * d + i4) ^ flip)) = packed;
+                }
+            }
+            __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): this wave's LDS writes have landed
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int line = 8 * j + line8;
+                if ((unsigned)(32 * b + line) < valid) {
+                    const u32x4 bits = *reinterpret_cast<const u32x4*>(staged + line * 128 + 16 * (piece ^ ((line >> 1) & 7)));
+                    __builtin_nontemporal_store(bits, reinterpret_cast<u32x4*>(rows + (size_t)(32 * b + line) * RANK + 8 * piece));
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+        if (!more) break;
+        ++n;
+        items.next(*work, place, item);
+        first_scores(item, n);
+    }
+}
+
+__global__ __launch_bounds__(WIDE_THREADS) void mla_wide_forward_kernel(ForwardWork) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const Argument<ForwardWork> work;
+    ForwardWork::Item item;
+    ForwardWork::Iterator items = {0};
+    if (!items.next(*work, {}, item)) return;
+    if (wave >= 4) {
+        wide_stream<ForwardWork, true>({}, item, items, lds, wave);
+    } else {
+        wide_stream<ForwardWork, false>({}, item, items, lds, wave);
+    }
+}
+
+template <typename Kernel>
+void allow_wide_lds(Kernel kernel) {
+    HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  WIDE_LDS_BYTES));
+}
+
+}  // namespace
+
+void mla_wide_forward_launch(bf16_t* output, float* logsumexp, const bf16_t* query_latent, const bf16_t* query_rope,
+                             const bf16_t* kv_latent, const bf16_t* key_rope, int batch_size, int sequence_length,
+                             int heads, float scale, hipStream_t stream) {
+    static hip_common::OncePerDevice prepared;
+    prepared.run([] { allow_wide_lds(mla_wide_forward_kernel); });
+    ForwardWork work;
+    work.output = output;
+    work.logsumexp = logsumexp;
+    work.query_latent = query_latent;
+    work.query_rope = query_rope;
+    work.kv_latent = kv_latent;
+    work.key_rope = key_rope;
+    work.sequence_length = sequence_length;
+    work.heads = heads;
+    work.rows = (unsigned)((long long)sequence_length * heads);
+    work.row_blocks = (work.rows + WIDE_ROWS - 1) / WIDE_ROWS;
+    work.items = work.row_blocks * batch_size;
+    // Numbered together, the blocks of all batch elements go from heavy to light once, which the rounds even out; one batch
+    // element after the other keeps few keys live in the L2s.
+    work.interleaved = (long long)batch_size * sequence_length * 2 * WIDTH <= (3 << 20);
+    work.by_heads = index_math::fast_division((unsigned)heads);
+    work.by_order = index_math::fast_division(work.interleaved ? (unsigned)batch_size : work.row_blocks);
+    work.c = scale * LOG2E;
+    const unsigned workgroups = std::min(work.items, (unsigned)std::max(hip_common::compute_units_of_current_device(), 1));
+    hipLaunchKernelGGL(mla_wide_forward_kernel, dim3(workgroups), dim3(WIDE_THREADS), WIDE_LDS_BYTES, stream, work);
+    HIP_CHECK(hipGetLastError());
+}
+
+}  // namespace dscuda
