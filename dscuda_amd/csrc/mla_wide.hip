@@ -45,7 +45,6 @@
 
 #include <algorithm>
 #include <cstdint>
-#include <stdexcept>
 
 namespace dscuda {
 namespace {
@@ -545,8 +544,9 @@ __device__ __forceinline__ void wide_stream(const typename Work::Place place, ty
         const unsigned valid = work->valid_rows(place, item);
         const unsigned own_row = 16 * wave + lane;   // of lanes 0..15
         if (lane < 16 && own_row < valid) work->store_logsumexp(place, item, own_row, (reference + __builtin_amdgcn_logf(total)) * LN2);
-        // The rows leave through the slot of the last unit, a tile of 32 rows x the wave's 128 bytes at a time, eight
-        // whole lines an instruction, past the caches (1024 tokens x 128 heads 153 -> 143 us).
+        // The rows leave through the slot of the last unit, a tile of 32 rows x the wave's 128 bytes at a time, eight whole
+        // lines an instruction.  (With the hint for streams the kernel by itself is 10 us shorter at 1024 tokens x 128 heads,
+        // but the un-absorb that reads the rows 20 longer: the layer 245 against 234 us.)
         unsigned char* staged = lds + ((unsigned)n % UNIT_SLOTS) * LATENT_SLOT + wave * (32 * 2 * WAVE_COLUMNS);
         bf16_t* rows = work->output + work->query_row(place, item, 0) * RANK + wave * WAVE_COLUMNS;
         const int to = lq * 128 + 8 * (lane / 32), flip = (lq >> 1) & 7;
@@ -570,7 +570,7 @@ __device__ __forceinline__ void wide_stream(const typename Work::Place place, ty
                 const int line = 8 * j + line8;
                 if ((unsigned)(32 * b + line) < valid) {
                     const u32x4 bits = *reinterpret_cast<const u32x4*>(staged + line * 128 + 16 * (piece ^ ((line >> 1) & 7)));
-                    __builtin_nontemporal_store(bits, reinterpret_cast<u32x4*>(rows + (size_t)(32 * b + line) * RANK + 8 * piece));
+                    *reinterpret_cast<u32x4*>(rows + (size_t)(32 * b + line) * RANK + 8 * piece) = bits;
                 }
             }
             __builtin_amdgcn_wave_barrier();
