@@ -122,7 +122,13 @@ void mla_narrow_forward_launch(__hip_bfloat16* output, float* logsumexp, const _
                                const __hip_bfloat16* key_rope, int batch_size, int sequence_length, int heads,
                                int row_blocks, float scale, hipStream_t stream);
 
-// mla_wide.hip -- the forward with 128 rows per workgroup.
+// mla_wide.hip -- the same with 128 rows per workgroup; the decode for pages that hold whole units of 32 keys, without
+// the merge (`layout` is that of index_math::decode_layout).
+void mla_wide_decode_launch(__hip_bfloat16* output, float* logsumexp, const __hip_bfloat16* query,
+                            const __hip_bfloat16* paged_kv_cache, const int* block_table, const int* cache_lengths,
+                            float* workspace, int* plan, int batch_size, int heads, int page_size, int pages_per_sequence,
+                            const index_math::DecodeLayout& layout, bool own_plan, float scale, hipStream_t stream);
+
 void mla_wide_forward_launch(__hip_bfloat16* output, float* logsumexp, const __hip_bfloat16* query_latent,
                              const __hip_bfloat16* query_rope, const __hip_bfloat16* kv_latent,
                              const __hip_bfloat16* key_rope, int batch_size, int sequence_length, int heads, float scale,

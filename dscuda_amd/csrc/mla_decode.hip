@@ -839,16 +839,22 @@ void mla_decode_dispatch(bf16_t* output, float* logsumexp, const bf16_t* query, 
                                  stream);
         return;
     }
-    static hip_common::OncePerDevice prepared;
-    prepared.run([] { allow_large_lds(mla_decode_split_kernel); });
     // a plan built for the other form counts other ranges
     const bool recut = !own_plan && index_math::decode_form(batch_size, heads, splits, compute_units(), RANK).row_blocks != 0;
     const int padded_rows = (heads + 31) / 32 * 32;
-    const dim3 grid(layout.workgroups, layout.head_groups);
-    hipLaunchKernelGGL(mla_decode_split_kernel, grid, dim3(THREADS), LDS_BYTES, stream, output, logsumexp, query,
-                       paged_kv_cache, block_table, cache_lengths, workspace, plan, batch_size, heads, page_size,
-                       pages_per_sequence, layout.slot_floats, padded_rows, scale, own_plan, recut, cut_of(layout));
-    HIP_CHECK(hipGetLastError());
+    // pages that do not hold whole units are looked up key by key, which only the four-wave kernel does
+    if (page_size % UNIT == 0) {
+        mla_wide_decode_launch(output, logsumexp, query, paged_kv_cache, block_table, cache_lengths, workspace, plan,
+                               batch_size, heads, page_size, pages_per_sequence, layout, own_plan, scale, stream);
+    } else {
+        static hip_common::OncePerDevice prepared;
+        prepared.run([] { allow_large_lds(mla_decode_split_kernel); });
+        const dim3 grid(layout.workgroups, layout.head_groups);
+        hipLaunchKernelGGL(mla_decode_split_kernel, grid, dim3(THREADS), LDS_BYTES, stream, output, logsumexp, query,
+                           paged_kv_cache, block_table, cache_lengths, workspace, plan, batch_size, heads, page_size,
+                           pages_per_sequence, layout.slot_floats, padded_rows, scale, own_plan, recut, cut_of(layout));
+        HIP_CHECK(hipGetLastError());
+    }
     if (!layout.whole_sequences) {
         hipLaunchKernelGGL(mla_decode_merge_kernel, dim3(MERGE_SLICES * (padded_rows / 32), batch_size), dim3(64), 0,
                            stream, output, logsumexp, workspace, plan, heads, layout.slot_floats, padded_rows,

@@ -1,9 +1,10 @@
-// Absorbed MLA attention, 128 query rows a workgroup: the causal prefill forward.  Takes the place of the reference's
-// mla_forward_kernel (kernels/attention/mla/sm89.cu:156-291); the decomposition below is built around 64-lane MFMA waves and the 160 KB LDS and
+// Absorbed MLA attention, 128 query rows a workgroup: the causal prefill forward, and the decode over pages that hold whole
+// units.  Takes the place of the reference's mla_forward_kernel and mla_decode_split_kernel
+// (kernels/attention/mla/sm89.cu:156-291, 413-477); the decomposition below is built around 64-lane MFMA waves and the 160 KB LDS and
 // shares nothing with their per-head scalar loops.
 //
 // Rows and units
-//   A workgroup owns 128 rows, consecutive (token, head) pairs, and walks
+//   A workgroup owns 128 rows, consecutive (token, head) pairs (decode: heads of a sequence), and walks
 //   a stream of keys in units of 32.  Every row reads the same keys, so a unit is fetched once for 128 rows x (576 + 512)
 //   x 2 flop per key.
 //
@@ -20,7 +21,7 @@
 //   3 x 700 x 33 87 -> 66, 40 x 130 x 16 57 -> 42, 7 x 257 x 128 167 -> 123).
 //
 // The stream runs on over the ends of items
-//   A workgroup takes several items (blocks of 128 rows), one a compute unit being all that the
+//   A workgroup takes several items (blocks of 128 rows; decode: the segments of its range of the work list), one a compute unit being all that the
 //   registers and the LDS hold.  Units are requested three steps ahead, the next item's among them; the query rows of the
 //   next item are asked for as the last scores of this one release their registers.  An item used to cost 12 to 20 us
 //   besides its units (a workgroup's start, query rows and first units, its rows on their way out), now some 7, of which
@@ -34,6 +35,14 @@
 //   upper half.  The 16x16x32 operand (row lane % 16, chunk lane / 16) meets itself there under the tiles' swizzle; with
 //   the four chunks of a step dealt to the lane groups in the order 0, 3, 1, 2 -- in the query rows as well, the sum over
 //   them is the same -- it does not: 1430 of 3100 LDS cycles a unit were conflicts (2048 tokens x 128 heads 575 -> 525 us).
+//
+// What bounds the decode
+//   64 sequences of 1024..8192 tokens, 128 heads: 13 us until the loop (plan, block table, query rows and the first units of
+//   all workgroups at once), 44 units in 80 us, 6 us of parts stored.  1.83 us a unit are 4.9 TB/s and 1.25 PFLOP/s,
+//   what the power limit leaves: 1.55 with a zero cache and query, 1.43 with its rows in the L2s as well.  So the four waves
+//   of mla_decode_split_kernel come to the same there (119 / 119 us), and cutting the list by units or counting fewer
+//   positions for a segment gains nothing.  Short sequences, whose start and end count, are faster here: 64 x 200..1000
+//   tokens 39.4 -> 36.6 us, 64 x 100..200 31.3 -> 28.8, 64 x 512..4096 64.4 / 64.2, 32 x 1024..8192 72.9 / 73.2.
 //
 // Softmax reference
 //   Exponentials are taken against a fixed reference, the maximum of the row's first unit plus 2^40.  A row whose scores
@@ -137,6 +146,7 @@ struct Argument {
 struct ForwardWork {
     static constexpr int LATENT_STRIDE = 2 * RANK;   // bytes, of keys and query rows
     static constexpr int ROPE_STRIDE = 2 * ROPE;
+    static constexpr bool STREAMING = false;         // keys are read by many workgroups
 
     bf16_t* output;
     float* logsumexp;
@@ -191,14 +201,14 @@ struct ForwardWork {
         int limit;
 
         __device__ __forceinline__ const unsigned char* rope() const { return rope_rows; }
-        __device__ __forceinline__ void open(const ForwardWork& work, const Item& item, unsigned char*, int) {
+        __device__ __forceinline__ void open(const ForwardWork& work, const Item& item) {
             const size_t first = (size_t)item.batch * work.sequence_length;
             latent = reinterpret_cast<const unsigned char*>(work.kv_latent + first * RANK);
             rope_rows = reinterpret_cast<const unsigned char*>(work.key_rope + first * ROPE);
             limit = item.tokens - 1;
         }
-        __device__ __forceinline__ int look_up(const unsigned char*, int) const { return 0; }
-        __device__ __forceinline__ void next(int, unsigned char*, int) {
+        __device__ __forceinline__ int look_up() const { return 0; }
+        __device__ __forceinline__ void next(const ForwardWork&, int) {
             const int rows = min(limit, UNIT);   // fewer: no visible token behind them, the last row stands for the unit
             latent += rows * LATENT_STRIDE;
             rope_rows += rows * ROPE_STRIDE;
@@ -227,6 +237,171 @@ struct ForwardWork {
     __device__ __forceinline__ int visible(const Item& item, unsigned row) const {
         return (int)index_math::divide(item.row0 + row, by_heads) + 1;
     }
+    __device__ __forceinline__ static constexpr bool is_part(const Item&) { return false; }
+    __device__ __forceinline__ float* part_statistics(const Place&, const Item&) const { return nullptr; }
+    __device__ __forceinline__ unsigned char* part_rows(const Place&, const Item&) const { return nullptr; }
+};
+
+// What is the same for all lanes, by the scalar unit: its wait is that of the LDS reads, not of the requests on their way.
+__device__ __forceinline__ int scalar_load(const int* place) {
+    return *(const __attribute__((address_space(4))) int*)place;
+}
+
+// The lengths' plan that a workgroup works out for itself (latent_stream.h) lies behind the LDS of the walk.
+constexpr int OWN_PREFIX_AT = WIDE_LDS_BYTES;
+constexpr int OWN_LENGTHS_AT = OWN_PREFIX_AT + 4 * (SELF_PLAN_BATCH + 4);
+constexpr int OWN_TOTALS_AT = OWN_LENGTHS_AT + 4 * SELF_PLAN_BATCH;
+constexpr int OWN_RANGE_AT = OWN_TOTALS_AT + 4 * (2 * SELF_PLAN_BATCH / 64);   // end of the range, overhead of a sequence
+constexpr int DECODE_LDS_BYTES = OWN_RANGE_AT + 8;
+static_assert(DECODE_LDS_BYTES <= 160 * 1024, "all there is");
+
+__device__ __forceinline__ int own_value(int at, int index) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    return __builtin_amdgcn_readfirstlane(*reinterpret_cast<const int*>(lds + at + 4 * index));
+}
+
+// Decode: 128 heads of a sequence, the tiles of it that a range of the work list holds.  Pages hold whole units.
+struct DecodeWork {
+    static constexpr int LATENT_STRIDE = 2 * WIDTH;
+    static constexpr int ROPE_STRIDE = 2 * WIDTH;
+    static constexpr bool STREAMING = true;          // each head group reads the cache once
+
+    bf16_t* output;
+    float* logsumexp;
+    const bf16_t* query;
+    const bf16_t* cache;
+    const int* block_table;
+    const int* cache_lengths;
+    float* workspace;
+    int* plan;
+    int batch_size;
+    int heads;
+    int page_size;
+    int pages_per_sequence;
+    long long slot_floats;
+    int padded_rows;
+    bool own_plan;
+    DecodeCut cut;
+    float c;
+
+    struct Place {};                     // its range lies in the LDS: scalar registers are scarce
+
+    struct Item {
+        int sequence;
+        int tokens;
+        int unit_begin;
+        int units;
+        bool part;                       // of its sequence
+    };
+
+    struct Iterator {
+        int position;
+        int sequence;
+
+        __device__ __forceinline__ bool next(const DecodeWork& work, const Place&, Item& item) {
+            const int end = own_value(OWN_RANGE_AT, 0);
+            while (position < end) {
+                const int overhead = own_value(OWN_RANGE_AT, 1);
+                const int at = sequence++;
+                int before, after, tokens;
+                if (work.own_plan) {
+                    before = own_value(OWN_PREFIX_AT, at);
+                    after = own_value(OWN_PREFIX_AT, at + 1);
+                    tokens = own_value(OWN_LENGTHS_AT, at);
+                } else {
+                    const int* prefix = work.plan + index_math::plan_prefix_at() + at;
+                    before = scalar_load(prefix);
+                    after = scalar_load(prefix + 1);
+                    tokens = scalar_load(work.cache_lengths + at);
+                }
+                const int segment_end = min(end, after);
+                if (segment_end <= position) continue;   // a sequence without tiles
+                int tile_begin, tile_end;
+                index_math::tiles_in_positions(position, segment_end, before, overhead, tile_begin, tile_end);
+                position = segment_end;
+                item.sequence = at;
+                item.tokens = tokens;
+                item.unit_begin = (BN / UNIT) * tile_begin;
+                item.units = min((BN / UNIT) * tile_end, (tokens + UNIT - 1) / UNIT) - item.unit_begin;
+                item.part = tile_begin != 0 || tile_end != after - before - overhead;
+                if (item.units <= 0) continue;           // nothing but positions that stand for the sequence's overhead
+                item.units = max(item.units, 2);
+                return true;
+            }
+            return false;
+        }
+    };
+
+    struct Keys {
+        const unsigned char* latent;
+        const int* entry;                // of the block table, of the page behind the unit's
+        int limit;
+        int left;                        // units of the page from this one on
+
+        __device__ __forceinline__ const unsigned char* rope() const { return latent + 2 * RANK; }
+        __device__ __forceinline__ void open(const DecodeWork& work, const Item& item) {
+            const int key0 = item.unit_begin * UNIT;
+            const int page = __builtin_amdgcn_readfirstlane((unsigned)key0 / (unsigned)work.page_size);
+            const int inside = key0 - page * work.page_size;
+            entry = work.block_table + (size_t)item.sequence * work.pages_per_sequence + page;
+            const long long id = scalar_load(entry);
+            latent = reinterpret_cast<const unsigned char*>(work.cache + (id * work.page_size + inside) * WIDTH);
+            ++entry;
+            left = (work.page_size - inside) / UNIT;
+            limit = item.tokens - 1 - key0;
+        }
+        // The next unit's page, if that is another one: asked for ahead of the products, used behind them.  No entry past
+        // the last page with a visible token is read.
+        __device__ __forceinline__ int look_up() const { return left == 1 && limit >= UNIT ? scalar_load(entry) : 0; }
+        __device__ __forceinline__ void next(const DecodeWork& work, int ahead) {
+            if (limit < UNIT) {          // no visible token behind them, the last row stands for the unit
+                latent += limit * LATENT_STRIDE;
+                limit = 0;
+                return;
+            }
+            limit -= UNIT;
+            latent += UNIT * LATENT_STRIDE;
+            if (--left == 0) {
+                latent = reinterpret_cast<const unsigned char*>(work.cache + (long long)ahead * work.page_size * WIDTH);
+                left = work.page_size / UNIT;
+                ++entry;
+            }
+        }
+    };
+
+    // Workgroups go to the eight XCDs round-robin by linear id.  Neighbouring ranges are mostly parts of the same
+    // sequence and fetch the same query rows, so each XCD takes a run of consecutive ranges.
+    __device__ __forceinline__ static int workgroup() {
+        return gridDim.x % 8 == 0 ? (int)(blockIdx.x % 8) * (int)(gridDim.x / 8) + (int)(blockIdx.x / 8) : (int)blockIdx.x;
+    }
+    __device__ __forceinline__ static unsigned head0() { return blockIdx.y * WIDE_ROWS; }
+    __device__ __forceinline__ unsigned valid_rows(const Place&, const Item&) const {
+        return min((unsigned)heads - head0(), (unsigned)WIDE_ROWS);
+    }
+    __device__ __forceinline__ size_t query_row(const Place&, const Item& item, unsigned row) const {
+        return (size_t)item.sequence * heads + head0() + row;
+    }
+    __device__ __forceinline__ const bf16_t* latent_row(const Place& place, const Item& item, unsigned row) const {
+        return query + query_row(place, item, row) * WIDTH;
+    }
+    __device__ __forceinline__ const bf16_t* rope_row(const Place& place, const Item& item, unsigned row) const {
+        return query + query_row(place, item, row) * WIDTH + RANK;
+    }
+    __device__ __forceinline__ void store_logsumexp(const Place& place, const Item& item, unsigned row, float value) const {
+        logsumexp[query_row(place, item, row)] = value;
+    }
+    __device__ __forceinline__ int visible(const Item& item, unsigned) const { return item.tokens; }
+    __device__ __forceinline__ static bool is_part(const Item& item) { return item.part; }
+    // A part's slot: 32 KB for every 32 rows, in the order of the accumulators' registers, then (reference, sum) of a head.
+    __device__ __forceinline__ float* slot(const Place& place, const Item& item) const {
+        return workspace + ((long long)workgroup() + item.sequence) * slot_floats;
+    }
+    __device__ __forceinline__ float* part_statistics(const Place& place, const Item& item) const {
+        return slot(place, item) + (size_t)padded_rows * (RANK / 2) + 2 * head0();
+    }
+    __device__ __forceinline__ unsigned char* part_rows(const Place& place, const Item& item) const {
+        return reinterpret_cast<unsigned char*>(slot(place, item)) + (size_t)head0() * (2 * RANK);
+    }
 };
 
 // The unit requested next; runs ahead of the products, over the ends of items.
@@ -237,21 +412,19 @@ struct WideCursor {
     int left;   // units of the item from this one on; 0: no more items
 
     __device__ __forceinline__ bool enabled() const { return left > 0; }
-    __device__ __forceinline__ void open(const Argument<Work>& work, const typename Work::Item& item, unsigned char* lds,
-                                         int wave) {
+    __device__ __forceinline__ void open(const Argument<Work>& work, const typename Work::Item& item) {
         left = __builtin_amdgcn_readfirstlane(item.units);
-        keys.open(*work, item, lds, wave);
+        keys.open(*work, item);
     }
     // (ahead: what keys.look_up returned)
-    __device__ __forceinline__ void advance(const Argument<Work>& work, const typename Work::Place& place, int ahead,
-                                            unsigned char* lds, int wave) {
+    __device__ __forceinline__ void advance(const Argument<Work>& work, const typename Work::Place& place, int ahead) {
         if (left == 0) return;
         if (--left > 0) {
-            keys.next(ahead, lds, wave);
+            keys.next(*work, ahead);
             return;
         }
         typename Work::Item item;
-        if (items.next(*work, place, item)) open(work, item, lds, wave);
+        if (items.next(*work, place, item)) open(work, item);
     }
 };
 
@@ -271,7 +444,8 @@ __device__ __forceinline__ void wide_stream(const typename Work::Place place, ty
         constexpr int I = decltype(tag)::value;
         if (!cursor.enabled()) return;
         auto load = [&](const unsigned char* base, unsigned offset, unsigned target) {
-            direct_load_16_offset(base, offset, target);
+            if constexpr (Work::STREAMING) direct_load_16_offset_streaming(base, offset, target);
+            else direct_load_16_offset(base, offset, target);
         };
         const int lane = fresh_lane_id();
         if constexpr (I < 4) {
@@ -287,9 +461,9 @@ __device__ __forceinline__ void wide_stream(const typename Work::Place place, ty
         }
     };
     auto issue_all = [&](int n) {
-        const int ahead = cursor.keys.look_up(lds, wave);
+        const int ahead = cursor.keys.look_up();
         unrolled<0, 5>([&](auto tag) { issue(n, tag); });
-        cursor.advance(work, place, ahead, lds, wave);
+        cursor.advance(work, place, ahead);
     };
 
     f32x16 out[ROW_TILES][WAVE_BLOCKS];   // 32 rows x 32 columns each
@@ -409,7 +583,7 @@ __device__ __forceinline__ void wide_stream(const typename Work::Place place, ty
     };
     // Products of the stream's unit n, and the requests of unit n + 3 into the slot that unit n - 1 has left.
     auto output_phase = [&](int n, auto last) {
-        const int ahead = cursor.keys.look_up(lds, wave);
+        const int ahead = cursor.keys.look_up();
         const unsigned p_at = P_AT + 16 * fresh_lane_id() + (n & 1) * P_BYTES;
         auto value_fragment = [&](auto half, auto d) -> bf16x8 {
             constexpr int AT = decltype(half)::value * 16 * LATENT_BYTES;
@@ -443,7 +617,7 @@ __device__ __forceinline__ void wide_stream(const typename Work::Place place, ty
         });
         value_at[0] += latent_step(n);
         value_at[1] += latent_step(n);
-        cursor.advance(work, place, ahead, lds, wave);
+        cursor.advance(work, place, ahead);
     };
 
     int n = 0;              // unit of the stream
@@ -463,7 +637,7 @@ __device__ __forceinline__ void wide_stream(const typename Work::Place place, ty
             // At the start of the kernel every workgroup asks at once and the answers come at the rate of the memory: what
             // the first scores need is asked for first.
             cursor.items = items;
-            cursor.open(work, item, lds, wave);
+            cursor.open(work, item);
             find_query(item, true);
             unrolled<0, SCORE_STEPS>(load_query);
             issue_all(n);
@@ -543,6 +717,28 @@ __device__ __forceinline__ void wide_stream(const typename Work::Place place, ty
         again = false;
         const unsigned valid = work->valid_rows(place, item);
         const unsigned own_row = 16 * wave + lane;   // of lanes 0..15
+        if (work->is_part(item)) {
+            if (lane < 16 && own_row < valid) {
+                float* statistics = work->part_statistics(place, item) + 2 * own_row;
+                statistics[0] = reference;
+                statistics[1] = total;
+            }
+            // 16-byte piece j of a lane: registers 8 * (j % 2) .. + 7 of column block j / 2
+            unsigned char* pieces = work->part_rows(place, item) + wave * (2 * WAVE_BLOCKS * 1024) + 16 * lane;
+#pragma unroll
+            for (int b = 0; b < ROW_TILES; ++b) {
+                if (32u * b >= valid) break;
+#pragma unroll
+                for (int j = 0; j < 2 * WAVE_BLOCKS; ++j) {
+                    u32x4 packed;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        packed[k] = pack_bf16(out[b][j / 2][8 * (j % 2) + 2 * k], out[b][j / 2][8 * (j % 2) + 2 * k + 1]);
+                    }
+                    *reinterpret_cast<u32x4*>(pieces + b * (32 * 2 * RANK) + j * 1024) = packed;
+                }
+            }
+        } else {
         if (lane < 16 && own_row < valid) work->store_logsumexp(place, item, own_row, (reference + __builtin_amdgcn_logf(total)) * LN2);
         // The rows leave through the slot of the last unit, a tile of 32 rows x the wave's 128 bytes at a time, eight whole
         // lines an instruction.  (With the hint for streams the kernel by itself is 10 us shorter at 1024 tokens x 128 heads,
@@ -575,6 +771,7 @@ __device__ __forceinline__ void wide_stream(const typename Work::Place place, ty
             }
             __builtin_amdgcn_wave_barrier();
         }
+        }
         if (!more) break;
         ++n;
         items.next(*work, place, item);
@@ -596,10 +793,32 @@ __global__ __launch_bounds__(WIDE_THREADS) void mla_wide_forward_kernel(ForwardW
     }
 }
 
+// A workgroup's range of the work list (index_math.h).  Its parts of sequences go to slot workgroup + sequence of the workspace.
+__global__ __launch_bounds__(WIDE_THREADS) void mla_wide_decode_kernel(DecodeWork) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const Argument<DecodeWork> work;
+    const DecodeRange range = decode_range(
+        work->plan, work->cache_lengths, work->batch_size, work->own_plan, false, work->cut,
+        reinterpret_cast<int*>(lds + OWN_PREFIX_AT), reinterpret_cast<int*>(lds + OWN_LENGTHS_AT),
+        reinterpret_cast<int*>(lds + OWN_TOTALS_AT), threadIdx.x, WIDE_THREADS, DecodeWork::workgroup(), blockIdx.x == 0 && blockIdx.y == 0);
+    if (range.begin >= range.end) return;
+    int* own_range = reinterpret_cast<int*>(lds + OWN_RANGE_AT);
+    own_range[0] = range.end;     // the same from every wave, which reads what it wrote
+    own_range[1] = range.overhead;
+    DecodeWork::Iterator items = {__builtin_amdgcn_readfirstlane(range.begin), __builtin_amdgcn_readfirstlane(range.sequence)};
+    DecodeWork::Item item;
+    if (!items.next(*work, {}, item)) return;
+    if (wave >= 4) {
+        wide_stream<DecodeWork, true>({}, item, items, lds, wave);
+    } else {
+        wide_stream<DecodeWork, false>({}, item, items, lds, wave);
+    }
+}
+
 template <typename Kernel>
-void allow_wide_lds(Kernel kernel) {
-    HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  WIDE_LDS_BYTES));
+void allow_wide_lds(Kernel kernel, int bytes) {
+    HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
 }
 
 }  // namespace
@@ -608,7 +827,7 @@ void mla_wide_forward_launch(bf16_t* output, float* logsumexp, const bf16_t* que
                              const bf16_t* kv_latent, const bf16_t* key_rope, int batch_size, int sequence_length,
                              int heads, float scale, hipStream_t stream) {
     static hip_common::OncePerDevice prepared;
-    prepared.run([] { allow_wide_lds(mla_wide_forward_kernel); });
+    prepared.run([] { allow_wide_lds(mla_wide_forward_kernel, WIDE_LDS_BYTES); });
     ForwardWork work;
     work.output = output;
     work.logsumexp = logsumexp;
@@ -629,6 +848,35 @@ void mla_wide_forward_launch(bf16_t* output, float* logsumexp, const bf16_t* que
     work.c = scale * LOG2E;
     const unsigned workgroups = std::min(work.items, (unsigned)std::max(hip_common::compute_units_of_current_device(), 1));
     hipLaunchKernelGGL(mla_wide_forward_kernel, dim3(workgroups), dim3(WIDE_THREADS), WIDE_LDS_BYTES, stream, work);
+    HIP_CHECK(hipGetLastError());
+}
+
+void mla_wide_decode_launch(bf16_t* output, float* logsumexp, const bf16_t* query, const bf16_t* paged_kv_cache,
+                            const int* block_table, const int* cache_lengths, float* workspace, int* plan, int batch_size,
+                            int heads, int page_size, int pages_per_sequence, const index_math::DecodeLayout& layout,
+                            bool own_plan, float scale, hipStream_t stream) {
+    static hip_common::OncePerDevice prepared;
+    prepared.run([] { allow_wide_lds(mla_wide_decode_kernel, DECODE_LDS_BYTES); });
+    DecodeWork work;
+    work.output = output;
+    work.logsumexp = logsumexp;
+    work.query = query;
+    work.cache = paged_kv_cache;
+    work.block_table = block_table;
+    work.cache_lengths = cache_lengths;
+    work.workspace = workspace;
+    work.plan = plan;
+    work.batch_size = batch_size;
+    work.heads = heads;
+    work.page_size = page_size;
+    work.pages_per_sequence = pages_per_sequence;
+    work.slot_floats = layout.slot_floats;
+    work.padded_rows = (heads + 31) / 32 * 32;
+    work.own_plan = own_plan;
+    work.cut = DecodeCut{layout.workgroups, layout.whole_sequences, layout.reference_ranges, layout.wide_ranges};
+    work.c = scale * LOG2E;
+    hipLaunchKernelGGL(mla_wide_decode_kernel, dim3(layout.workgroups, layout.head_groups), dim3(WIDE_THREADS),
+                       DECODE_LDS_BYTES, stream, work);
     HIP_CHECK(hipGetLastError());
 }
 
