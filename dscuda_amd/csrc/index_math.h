@@ -513,13 +513,20 @@ DSCUDA_HOST_DEVICE inline int positions_of(int tiles, int overhead) { return til
 
 DSCUDA_HOST_DEVICE inline int ranges_of(int total, int workgroups) { return total < workgroups ? total : workgroups; }
 
+// Whether what the two functions below divide fits 32 bits (a 64-bit division is some 500 cycles of a kernel's start).
+DSCUDA_HOST_DEVICE inline bool products_fit(int total, int ranges) {
+    return (unsigned long long)(unsigned)total * (unsigned)ranges <= 0xffffffffull;
+}
+
 // First position of range `range` (0 .. ranges: the last one is the end of the list).
 DSCUDA_HOST_DEVICE inline int range_begin_of(int total, int ranges, int range) {
+    if (products_fit(total, ranges)) return (int)((unsigned)range * (unsigned)total / (unsigned)ranges);
     return (int)((long long)range * total / ranges);
 }
 
 // The range that holds position `position` (0 <= position < total).
 DSCUDA_HOST_DEVICE inline int range_of_position(int total, int ranges, int position) {
+    if (products_fit(total, ranges)) return (int)((((unsigned)position + 1) * (unsigned)ranges - 1) / (unsigned)total);
     return (int)((((long long)position + 1) * ranges - 1) / total);
 }
 

@@ -275,6 +275,7 @@ struct DecodeRange {
     int begin, end;      // positions of this workgroup's range; begin >= end: nothing to do
     int sequence;        // first sequence that reaches past `begin`
     bool wide;           // parts of cut sequences are kept in fp32
+    bool local;          // prefix and lengths lie in LDS
 };
 
 // How a call cuts its list (index_math::DecodeLayout).
@@ -319,6 +320,94 @@ __device__ __forceinline__ int wave_min(int value) {
     return value;
 }
 
+// Sum over the lanes up to this one.
+__device__ __forceinline__ int wave_prefix_sum(int value) {
+    auto add = [&](auto control, auto rows) {
+        value += __builtin_amdgcn_update_dpp(0, value, decltype(control)::value, decltype(rows)::value, 0xf, false);
+    };
+    using All = std::integral_constant<int, 0xf>;
+    add(std::integral_constant<int, 0x111>{}, All{});   // row_shr 1, 2, 4, 8: within 16 lanes
+    add(std::integral_constant<int, 0x112>{}, All{});
+    add(std::integral_constant<int, 0x114>{}, All{});
+    add(std::integral_constant<int, 0x118>{}, All{});
+    add(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});   // row_bcast 15, 31
+    add(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});
+    return value;
+}
+
+// decode_range for at most 64 sequences: every wave scans the batch in its own registers, lane = sequence, without a
+// barrier or a search in LDS, and the plan of a caller comes in one round trip with the lengths.  Stamps of a workgroup's
+// start: 3.5 us with the scan over a workgroup of 256, 1.0 so (of which a round trip to memory is 0.7).
+__device__ __forceinline__ DecodeRange small_decode_range(int* plan, const int* cache_lengths, int batch_size, bool own_plan,
+                                                          bool recut, const DecodeCut& cut, int* own_prefix, int* own_lengths,
+                                                          int tid, int workgroup, bool leave_plan) {
+    DecodeRange range;
+    const int lane = tid % 64;
+    const int length = cache_lengths[min(lane, batch_size - 1)];
+    int before, after, total, ranges;
+    bool whole_sequences;
+    if (own_plan) {
+        whole_sequences = cut.whole_sequences != 0;
+        range.overhead = whole_sequences ? 0 : index_math::SEGMENT_OVERHEAD;
+        const int positions = lane < batch_size ? index_math::positions_of(tiles_of(length), range.overhead) : 0;
+        after = wave_prefix_sum(positions);
+        before = after - positions;
+        total = __builtin_amdgcn_readlane(after, 63);
+        ranges = index_math::ranges_of(total, cut.workgroups);
+        range.wide = false;
+        if (cut.reference_ranges > 0 && total > 0) {   // as choose_ranges
+            const int reference = index_math::ranges_of(total, cut.reference_ranges);
+            const bool uncut = positions > 0 && !index_math::sequence_is_cut(total, reference, before, positions, range.overhead);
+            if (__builtin_amdgcn_ballot_w64(uncut) != 0) {
+                range.wide = cut.wide_ranges > 0;
+                ranges = range.wide ? index_math::ranges_of(total, cut.wide_ranges) : reference;
+            }
+        }
+        if (leave_plan && tid < 64) {
+            if (lane == 0) {
+                plan[PLAN_TOTAL] = total;
+                plan[PLAN_WORKGROUPS] = cut.workgroups;
+                plan[PLAN_OVERHEAD] = range.overhead;
+                plan[PLAN_MODE] = plan_mode(cut, range.wide);
+                plan[PLAN_RANGES] = ranges;
+                plan[index_math::plan_prefix_at()] = 0;
+            }
+            if (lane < batch_size) plan[index_math::plan_prefix_at() + lane + 1] = after;
+        }
+    } else {
+        const int* prefix = plan + index_math::plan_prefix_at();
+        before = prefix[min(lane, batch_size)];
+        after = prefix[min(lane + 1, batch_size)];
+        total = __builtin_amdgcn_readfirstlane(plan[PLAN_TOTAL]);
+        range.overhead = __builtin_amdgcn_readfirstlane(plan[PLAN_OVERHEAD]);
+        const int mode = __builtin_amdgcn_readfirstlane(plan[PLAN_MODE]);
+        ranges = __builtin_amdgcn_readfirstlane(plan[PLAN_RANGES]);
+        whole_sequences = mode == PLAN_WHOLE;
+        range.wide = mode == PLAN_WIDE_PARTS;
+        if (recut) ranges = index_math::ranges_of(total, cut.workgroups);
+    }
+    // the same from every wave, which reads what it wrote
+    own_prefix[lane] = before;
+    own_prefix[lane + 1] = after;
+    own_lengths[lane] = length;
+    range.prefix = own_prefix;
+    range.local = true;
+    range.sequence = 0;
+    if (whole_sequences) {
+        range.begin = __builtin_amdgcn_readlane(before, workgroup);
+        range.end = __builtin_amdgcn_readlane(after, workgroup);
+        range.sequence = workgroup;
+        return range;
+    }
+    range.begin = range.end = 0;
+    if (workgroup >= ranges) return range;
+    range.begin = __builtin_amdgcn_readfirstlane(index_math::range_begin_of(total, ranges, workgroup));
+    range.end = __builtin_amdgcn_readfirstlane(index_math::range_begin_of(total, ranges, workgroup + 1));
+    // sequences that end before the range
+    range.sequence = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < batch_size && after <= range.begin));
+    return range;
+}
+
 // The plan comes from memory (own_plan false: the caller's, or one mla_decode_plan_kernel has just built), or,
 // for a batch that one workgroup scans in one go, is worked out here by every workgroup for itself, which saves the
 // call a kernel launch; `leave_plan`: this workgroup then also writes what the merge kernel reads of it.  `recut`: the
@@ -328,7 +417,12 @@ __device__ __forceinline__ int wave_min(int value) {
 __device__ __forceinline__ DecodeRange decode_range(int* plan, const int* cache_lengths, int batch_size, bool own_plan,
                                                     bool recut, const DecodeCut& cut, int* own_prefix, int* own_lengths,
                                                     int* own_wave_totals, int tid, int threads, int workgroup, bool leave_plan) {
+    if (batch_size <= 64) {
+        return small_decode_range(plan, cache_lengths, batch_size, own_plan, recut, cut, own_prefix, own_lengths, tid, workgroup,
+                                  leave_plan);
+    }
     DecodeRange range;
+    range.local = own_plan;
     int total, ranges;
     bool whole_sequences;
     if (own_plan) {

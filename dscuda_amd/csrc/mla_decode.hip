@@ -599,7 +599,7 @@ __global__ __launch_bounds__(THREADS) void mla_decode_split_kernel(
             ++sequence;
             continue;
         }
-        const int tokens = own_plan ? __builtin_amdgcn_readfirstlane(own_lengths[sequence]) : cache_lengths[sequence];
+        const int tokens = range.local ? __builtin_amdgcn_readfirstlane(own_lengths[sequence]) : cache_lengths[sequence];
         const bool whole = tile_begin == 0 && tile_end == sequence_end - sequence_begin - overhead;
         const bf16_t* query_row = query + ((size_t)sequence * heads + row) * WIDTH;
 

@@ -421,8 +421,19 @@ __global__ __launch_bounds__(NARROW_THREADS) void mla_narrow_decode_kernel(
     int sequence = range.sequence;
     int position = range.begin;
     while (position < range.end) {
-        const int sequence_begin = __builtin_amdgcn_readfirstlane(range.prefix[sequence]);
-        const int sequence_end = __builtin_amdgcn_readfirstlane(range.prefix[sequence + 1]);
+        int sequence_begin, sequence_end, tokens;
+        if (range.local) {
+            sequence_begin = own_prefix[sequence];
+            sequence_end = own_prefix[sequence + 1];
+            tokens = own_lengths[sequence];
+        } else {
+            sequence_begin = range.prefix[sequence];
+            sequence_end = range.prefix[sequence + 1];
+            tokens = cache_lengths[sequence];
+        }
+        sequence_begin = __builtin_amdgcn_readfirstlane(sequence_begin);
+        sequence_end = __builtin_amdgcn_readfirstlane(sequence_end);
+        tokens = __builtin_amdgcn_readfirstlane(tokens);
         const int segment_end = min(range.end, sequence_end);
         if (segment_end <= position) {  // a sequence without tiles (length < 1) owns nothing
             ++sequence;
@@ -435,7 +446,6 @@ __global__ __launch_bounds__(NARROW_THREADS) void mla_narrow_decode_kernel(
             ++sequence;
             continue;
         }
-        const int tokens = __builtin_amdgcn_readfirstlane(own_plan ? own_lengths[sequence] : cache_lengths[sequence]);
         const bool whole = tile_begin == 0 && tile_end == sequence_end - sequence_begin - range.overhead;
 
         KeyStream keys;

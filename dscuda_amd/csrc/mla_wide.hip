@@ -304,7 +304,7 @@ struct DecodeWork {
                 const int overhead = own_value(OWN_RANGE_AT, 1);
                 const int at = sequence++;
                 int before, after, tokens;
-                if (work.own_plan) {
+                if (work.batch_size <= 64 || work.own_plan) {
                     before = own_value(OWN_PREFIX_AT, at);
                     after = own_value(OWN_PREFIX_AT, at + 1);
                     tokens = own_value(OWN_LENGTHS_AT, at);
