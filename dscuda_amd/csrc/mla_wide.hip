@@ -644,9 +644,10 @@ __device__ __forceinline__ void wide_stream(const typename Work::Place place, ty
             wait_vector_memory<0>();
             workgroup_barrier();
             issue_all(n + 1);
+            const bool third = cursor.enabled();
             issue_all(n + 2);
             first_scores(item, n);
-            wait_vector_memory<0>();
+            if (third) wait_vector_memory<REQUESTS>(); else wait_vector_memory<0>();   // unit n + 1 has landed
             restart = false;
         }
         workgroup_barrier();   // the first probabilities are there
@@ -798,8 +799,10 @@ __global__ __launch_bounds__(WIDE_THREADS) void mla_wide_decode_kernel(DecodeWor
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const Argument<DecodeWork> work;
+    DecodeCut cut = work->cut;
+    cut.reference_ranges = 0;   // decode_layout has none; the vote over them would take LDS in front of the slots
     const DecodeRange range = decode_range(
-        work->plan, work->cache_lengths, work->batch_size, work->own_plan, false, work->cut,
+        work->plan, work->cache_lengths, work->batch_size, work->own_plan, false, cut,
         reinterpret_cast<int*>(lds + OWN_PREFIX_AT), reinterpret_cast<int*>(lds + OWN_LENGTHS_AT),
         reinterpret_cast<int*>(lds + OWN_TOTALS_AT), threadIdx.x, WIDE_THREADS, DecodeWork::workgroup(), blockIdx.x == 0 && blockIdx.y == 0);
     if (range.begin >= range.end) return;
