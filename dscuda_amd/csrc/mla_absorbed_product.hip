@@ -8,12 +8,16 @@
 // 2048 tokens x 128 heads: 815 us of query gradients there, 358 here, for 77 us more in the key gradients, whose score
 // waves store the 0.55 GB (1236 -> 1313); 2 x 592 x 16 35 -> 24.
 //
-// A workgroup of eight waves owns 64 * GROUP rows and walks the 32-key tiles they see, all of them through LDS stages
-// of [32 keys][512] + [32 keys][64] + dS.  Wave (r, v) = (w / 4, w % 4): row tiles GROUP * r .., latent column blocks
-// 4v .. 4v + 3 of each of them and one of the rope blocks.  Bound by the key tiles a compute unit draws from its L2
-// (36 KB a step, some 21 bytes a cycle against 1152 matrix cycles at GROUP = 2), hence 128 rows wherever that leaves
-// workgroups enough; 192 rows need more registers than there are.  With few rows a workgroup takes half of the columns
-// (PARTS = 2, 18 KB of keys a step and compute unit).
+// A workgroup of eight waves walks the 32-key tiles its rows see, all of them through LDS stages of [32 keys][columns] + dS,
+// three tiles ahead.  A wave sums GROUP row tiles x LATENT_BLOCKS latent column blocks and, of some waves, a rope block.
+//   GROUP = 2   256 rows and half of the columns.  Bound by what a compute unit draws into LDS (some 21 bytes a cycle) and the
+//               power limit: 16 KB of latent rows, 4 of rope rows and 16 of dS a step of 1152 matrix cycles; the halves, which
+//               run side by side on one XCD, read dS from memory once.  With 128 rows and all columns (44 KB, three stages)
+//               and the requests in front of the fragments, forward and backward in us, -> here: 2048 x 128 2245 -> 2235 (2204 ->
+//               2201 and, requests apart, 2166 -> 2130 on other boxes), 4096 x 32 2102 -> 2080, 2048 x 16 346 -> 340,
+//               300 x 128 140.1 -> 137.8, 1024 x 128 680.8 / 681.5, 2 x 700 x 32 202.6 / 203.7.  All columns with the requests
+//               among the products are within 1 % of either.
+//   GROUP = 1   64 rows, all columns or (PARTS = 2) half of them, for few rows.
 #include "attn_kernels.h"
 #include "hip_common.h"
 #include "index_math.h"
@@ -28,18 +32,22 @@ constexpr int RANK = 512;
 constexpr int ROPE = 64;
 constexpr int TILE = 32;
 constexpr int THREADS = 512;
+constexpr int XCDS = 8;
 
 template <int GROUP, int PARTS>
 struct ProductLayout {
-    static_assert(PARTS == 1 || GROUP == 1, "halves of the columns are for few rows");
-    static constexpr int ROWS = 64 * GROUP;
-    static constexpr int ROW_TILES = 2 * GROUP;
+    static_assert(GROUP == 1 || PARTS == 2, "the accumulators of 256 rows take halves of the columns");
+    static constexpr int ROW_GROUPS = 2 * GROUP;
+    static constexpr int ROW_TILES = ROW_GROUPS * GROUP;
+    static constexpr int ROWS = TILE * ROW_TILES;
+    static constexpr int COLUMN_WAVES = THREADS / 64 / ROW_GROUPS;
+    static constexpr int DS_REQUESTS = GROUP == 1 ? 1 : ROW_TILES / 4;   // 1 KB requests of dS of a wave (GROUP = 1: of the later four)
     static constexpr int WIDE_ROW = 2 * RANK / PARTS;
     static constexpr int NARROW_ROW = 2 * ROPE;
     static constexpr int ROPE_AT = TILE * WIDE_ROW;
     static constexpr int DS_AT = ROPE_AT + TILE * NARROW_ROW;
     static constexpr int STAGE_BYTES = DS_AT + ROW_TILES * index_math::KeptGradients::BLOCK_BYTES;
-    static constexpr int STAGES = GROUP == 1 ? 4 : 3;
+    static constexpr int STAGES = 4;
     static constexpr int OUT_ROPE = WIDE_ROW;                            // of a staged gradient row
     static constexpr int OUT_PITCH = WIDE_ROW + 2 * ROPE / PARTS + 16;
     static constexpr int OUT_BYTES = ROWS * OUT_PITCH;
@@ -55,7 +63,7 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
     using L = ProductLayout<GROUP, PARTS>;
     using Wide = index_math::TileReadMath<L::WIDE_ROW>;
     using Narrow = index_math::TileReadMath<L::NARROW_ROW>;
-    constexpr int LATENT_BLOCKS = RANK / TILE / 4 / PARTS;   // 32-column blocks of a wave
+    constexpr int LATENT_BLOCKS = RANK / TILE / L::COLUMN_WAVES / PARTS;   // 32-column blocks of a wave
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -64,9 +72,12 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
     const int g = lane / 32;
     const int T = sequence_length;
     const long long rows = (long long)T * heads;
-    const int column_part = blockIdx.x % PARTS;
-    const int batch = blockIdx.x / PARTS % batch_size;
-    const int row_block = row_blocks - 1 - blockIdx.x / PARTS / batch_size;   // latest rows (most keys) first
+    // GROUP = 2: the halves of the columns, which read the same dS, run side by side on one XCD
+    const int column_part = GROUP == 2 ? blockIdx.x / XCDS % 2 : blockIdx.x % PARTS;
+    const unsigned item = GROUP == 2 ? blockIdx.x / (2 * XCDS) * XCDS + blockIdx.x % XCDS : blockIdx.x / PARTS;
+    const int batch = item % (unsigned)batch_size;
+    const int row_block = row_blocks - 1 - (int)(item / (unsigned)batch_size);   // latest rows (most keys) first
+    if (GROUP == 2 && row_block < 0) return;               // the last of the groups of XCDS items is filled up
     const long long row0 = (long long)row_block * L::ROWS;
     const long long batch_row0 = (long long)batch * rows;
     const unsigned char* latent = reinterpret_cast<const unsigned char*>(kv_latent + (size_t)batch * T * RANK) + column_part * L::WIDE_ROW;
@@ -76,46 +87,58 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
     const unsigned char* kept_batch = kept_gradients + (size_t)batch * kept.bytes();
     const int first_row_tile = row_block * L::ROW_TILES;
 
-    const int v = wave % 4;
-    const int wave_row_tile = GROUP * (wave / 4);   // of the workgroup's
-    const int rope_tile = GROUP == 1 ? 0 : v / 2;   // whose rope block the wave sums; GROUP = 1: not every wave has one
+    const int v = wave % L::COLUMN_WAVES;
+    const int wave_row_tile = GROUP * (wave / L::COLUMN_WAVES);   // of the workgroup's
+    const int rope_tile = GROUP == 1 ? 0 : v * PARTS / 2;   // whose rope block the wave sums; GROUP = 1: not every wave has one
     const int rope_block = PARTS == 1 ? v % 2 : column_part;
     const bool sums_rope = GROUP > 1 || v < 2 / PARTS;
 
-    // A wave requests key rows 4*wave .. +3 of the wide tile (1 KB an instruction), waves 0 .. 3 also eight rows of the narrow one, and 1 KB,
-    // half a row tile, of dS: every wave at GROUP = 2, waves 4 .. 7 at GROUP = 1.  Keys past the end repeat the last
+    // A wave requests key rows 4*wave .. +3 of the wide tile (1 KB an instruction), waves 0 .. 3 also eight rows of the narrow one, and 1 KB
+    // pieces, halves of a row tile, of dS: every wave at GROUP = 2, waves 4 .. 7 at GROUP = 1.  Keys past the end repeat the last
     // one (their dS is zero), row tiles past the end repeat the last one (their results are not stored), and a tile
     // that does not see the keys yet may read what precedes its blocks and is left out below.
     const unsigned lds_base = lds_offset_of(lds);
-    const int ds_part = GROUP == 1 ? wave - 4 : wave;
+    const int ds_part = GROUP == 1 ? wave - 4 : L::DS_REQUESTS * wave;   // the first
     const int ds_row_tile = min(first_row_tile + max(ds_part, 0) / 2, kept.visits.row_tiles - 1);
-    auto request_tile = [&](int tile) {
+    // request I (0 .. REQUESTS - 1) of a tile
+    constexpr int WIDE_REQUESTS = 4 / PARTS;
+    constexpr int REQUESTS = WIDE_REQUESTS + 1 + L::DS_REQUESTS;
+    auto request = [&](int tile, auto tag) {
+        constexpr int I = decltype(tag)::value;
         const unsigned target = lds_base + tile % L::STAGES * L::STAGE_BYTES;
-        const int last = min(T - tile * TILE, TILE) - 1;
-#pragma unroll
-        for (int j = 0; j < 4 / PARTS; ++j) {
-            const int first = 4 * wave + PARTS * j;
+        if constexpr (I < WIDE_REQUESTS) {
+            const int last = min(T - tile * TILE, TILE) - 1;
+            const int first = 4 * wave + PARTS * I;
             const int key = first + lane / (64 / PARTS);
             const int chunk = lane % (64 / PARTS) ^ index_math::tile_swizzle<L::WIDE_ROW>(key);
             direct_load_16_offset(latent + (size_t)tile * TILE * (2 * RANK), (unsigned)(min(key, last) * (2 * RANK) + 16 * chunk),
                                   target + first * L::WIDE_ROW);
+        } else if constexpr (I == WIDE_REQUESTS) {
+            if (wave < 4) {
+                const int last = min(T - tile * TILE, TILE) - 1;
+                const int key = 8 * wave + lane / 8;
+                direct_load_16_offset(rope + (size_t)tile * TILE * L::NARROW_ROW,
+                                      (unsigned)(min(key, last) * L::NARROW_ROW +
+                                                 16 * ((lane % 8) ^ index_math::tile_swizzle<L::NARROW_ROW>(key))),
+                                      target + L::ROPE_AT + 8 * wave * L::NARROW_ROW);
+            }
+        } else if (GROUP > 1 || wave >= 4) {
+            constexpr int PIECE = I - WIDE_REQUESTS - 1;
+            const unsigned char* source = kept_batch + kept.at(tile, ds_row_tile) + 1024 * (ds_part % 2 + PIECE);
+            const unsigned piece_target = target + L::DS_AT + 1024 * (ds_part + PIECE);
+            // of the halves of the columns one finds what the other has fetched
+            if constexpr (GROUP == 2) direct_load_16_offset(source, 16u * (unsigned)lane, piece_target);
+            else direct_load_16_offset_streaming(source, 16u * (unsigned)lane, piece_target);
         }
-        if (wave < 4) {
-            const int key = 8 * wave + lane / 8;
-            direct_load_16_offset(rope + (size_t)tile * TILE * L::NARROW_ROW,
-                                  (unsigned)(min(key, last) * L::NARROW_ROW +
-                                             16 * ((lane % 8) ^ index_math::tile_swizzle<L::NARROW_ROW>(key))),
-                                  target + L::ROPE_AT + 8 * wave * L::NARROW_ROW);
-        }
-        if (GROUP > 1 || wave >= 4) {
-            direct_load_16_offset_streaming(kept_batch + kept.at(tile, ds_row_tile) + 1024 * (ds_part % 2), 16u * (unsigned)lane,
-                                            target + L::DS_AT + 1024 * ds_part);
-        }
+    };
+    auto request_tile = [&](int tile) {
+        unrolled<0, REQUESTS>([&](auto tag) { request(tile, tag); });
     };
     // all but the newest `tiles_in_flight` tiles of the wave's requests have arrived
     auto wait_for_all_but = [&](auto tiles_in_flight) {
         constexpr int N = decltype(tiles_in_flight)::value;
-        if (GROUP > 1 && wave < 4) wait_vector_memory<6 * N>(); else wait_vector_memory<(4 / PARTS + 1) * N>();
+        constexpr int EACH = 4 / PARTS + L::DS_REQUESTS;
+        if (GROUP > 1 && wave < 4) wait_vector_memory<(EACH + 1) * N>(); else wait_vector_memory<EACH * N>();
     };
     constexpr int AHEAD = L::STAGES - 1;
     for (int tile = 0; tile < min(tiles, AHEAD); ++tile) request_tile(tile);
@@ -150,42 +173,65 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
         const int behind = min(tiles - 1 - tile, AHEAD - 1);   // tiles that may stay in flight
         if (behind == 0) {
             wait_for_all_but(std::integral_constant<int, 0>{});
-        } else if (AHEAD == 2 || behind == 1) {
+        } else if (behind == 1) {
             wait_for_all_but(std::integral_constant<int, 1>{});
         } else {
             wait_for_all_but(std::integral_constant<int, 2>{});
         }
         workgroup_barrier();   // the tile is there, and the stage of the tile before has been read
-        if (tile + AHEAD < tiles) request_tile(tile + AHEAD);
+        const bool more = tile + AHEAD < tiles;
+        // Few rows: the requests, a step's longest part, go first (1000 tokens x 8 heads 104.3 us, among the products 107.4).
+        constexpr bool SPREAD = GROUP == 2 && FIRST < GROUP;
+        if (!SPREAD && more) request_tile(tile + AHEAD);
         if constexpr (FIRST < GROUP) {
+            // one stream of products, its fragments read RING column blocks ahead
             const unsigned char* stage = lds + tile % L::STAGES * L::STAGE_BYTES;
-            unrolled<0, 2>([&](auto tag) {
-                constexpr int N = decltype(tag)::value;   // 16-key step
-                auto fragment = [&](unsigned low_at, unsigned high_at) {
-                    const s16x4 low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((transposing_read_pointer)(stage + low_at));
-                    const s16x4 high = __builtin_amdgcn_ds_read_tr16_b64_v4i16((transposing_read_pointer)(stage + high_at));
-                    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(low, high, 0, 1, 2, 3, 4, 5, 6, 7));
-                };
-                bf16x8 ds[GROUP];
+            auto fragment = [&](unsigned low_at, unsigned high_at) {
+                const s16x4 low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((transposing_read_pointer)(stage + low_at));
+                const s16x4 high = __builtin_amdgcn_ds_read_tr16_b64_v4i16((transposing_read_pointer)(stage + high_at));
+                return __builtin_bit_cast(bf16x8, __builtin_shufflevector(low, high, 0, 1, 2, 3, 4, 5, 6, 7));
+            };
+            constexpr int COUNT = 2 * LATENT_BLOCKS;   // column blocks of two 16-key steps
+            constexpr int RING = LATENT_BLOCKS < 3 ? LATENT_BLOCKS : 3;
+            bf16x8 ds[2][GROUP], ring[RING], narrow[2];
+            auto read_ds = [&](int n) {
 #pragma unroll
                 for (int t = FIRST; t < GROUP; ++t) {
-                    const unsigned at = ds_at + t * index_math::KeptGradients::BLOCK_BYTES + 1024 * N;
-                    ds[t] = fragment(at, at + 512);
+                    const unsigned at = ds_at + t * index_math::KeptGradients::BLOCK_BYTES + 1024 * n;
+                    ds[n][t] = fragment(at, at + 512);
                 }
+            };
+            auto read_columns = [&](auto tag) {
+                constexpr int I = decltype(tag)::value;
+                constexpr int N = I / LATENT_BLOCKS, J = I % LATENT_BLOCKS;
+                ring[I % RING] = fragment(wide_at[0][J] + 16 * N * L::WIDE_ROW, wide_at[1][J] + 16 * N * L::WIDE_ROW);
+            };
+            const bool own_rope = sums_rope && rope_tile >= FIRST;
+            read_ds(0);
+            unrolled<0, RING>(read_columns);
+            unrolled<0, COUNT>([&](auto tag) {
+                constexpr int I = decltype(tag)::value;
+                constexpr int N = I / LATENT_BLOCKS, J = I % LATENT_BLOCKS;
 #pragma unroll
-                for (int j = 0; j < LATENT_BLOCKS; ++j) {
-                    const bf16x8 columns = fragment(wide_at[0][j] + 16 * N * L::WIDE_ROW, wide_at[1][j] + 16 * N * L::WIDE_ROW);
-#pragma unroll
-                    for (int t = FIRST; t < GROUP; ++t) {
-                        sum[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(columns, ds[t], sum[t][j], 0, 0, 0);
+                for (int t = FIRST; t < GROUP; ++t) {
+                    sum[t][J] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[I % RING], ds[N][t], sum[t][J], 0, 0, 0);
+                }
+                if constexpr (I == LATENT_BLOCKS - RING) read_ds(1);
+                if constexpr (I + RING < COUNT) read_columns(std::integral_constant<int, I + RING>{});
+                if constexpr (J == LATENT_BLOCKS - 2 + LATENT_BLOCKS % 2) {
+                    if (own_rope) narrow[N] = fragment(narrow_at[0] + 16 * N * L::NARROW_ROW, narrow_at[1] + 16 * N * L::NARROW_ROW);
+                }
+                if (SPREAD && more) {
+                    unrolled<I * REQUESTS / COUNT, (I + 1) * REQUESTS / COUNT>([&](auto piece) { request(tile + AHEAD, piece); });
+                }
+                if constexpr (J == LATENT_BLOCKS - 1) {
+                    if (own_rope) {
+                        bf16x8 own = ds[N][FIRST];
+                        if (GROUP > 1 && rope_tile == 1) own = ds[N][GROUP - 1];
+                        rope_sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(narrow[N], own, rope_sum, 0, 0, 0);
                     }
                 }
-                if (sums_rope && rope_tile >= FIRST) {
-                    const bf16x8 columns = fragment(narrow_at[0] + 16 * N * L::NARROW_ROW, narrow_at[1] + 16 * N * L::NARROW_ROW);
-                    bf16x8 own = ds[FIRST];
-                    if (GROUP > 1 && rope_tile == 1) own = ds[GROUP - 1];
-                    rope_sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(columns, own, rope_sum, 0, 0, 0);
-                }
+                __builtin_amdgcn_sched_barrier(0);
             });
         }
     };
@@ -245,7 +291,9 @@ void launch(bf16_t* query_latent_gradient, bf16_t* query_rope_gradient, const un
     });
     const long long rows = (long long)sequence_length * heads;
     const long long row_blocks = (rows + L::ROWS - 1) / L::ROWS;
-    hipLaunchKernelGGL((mla_absorbed_query_product_kernel<GROUP, PARTS>), dim3((unsigned)(row_blocks * batch_size * PARTS)), dim3(THREADS),
+    const long long items = row_blocks * batch_size;
+    const long long workgroups = PARTS * (GROUP == 2 ? (items + XCDS - 1) / XCDS * XCDS : items);
+    hipLaunchKernelGGL((mla_absorbed_query_product_kernel<GROUP, PARTS>), dim3((unsigned)workgroups), dim3(THREADS),
                        L::LDS_BYTES, stream, query_latent_gradient, query_rope_gradient, kept_gradients, kv_latent, key_rope,
                        batch_size, sequence_length, heads, key_tiles, (int)row_blocks);
     HIP_CHECK(hipGetLastError());
@@ -257,7 +305,8 @@ void mla_absorbed_query_product_launch(bf16_t* query_latent_gradient, bf16_t* qu
                                        const unsigned char* kept_gradients, const bf16_t* kv_latent,
                                        const bf16_t* key_rope, int batch_size, int sequence_length, int heads,
                                        int key_tiles, hipStream_t stream) {
-    // 128 rows a workgroup where that is a workgroup per compute unit. The whole backward in us, 64 / 128 rows: 148 workgroups of
+    // 256 rows and half the columns where that is a workgroup per compute unit (the work of 128 whole rows, with which the
+    // line was measured).  The whole backward in us, 64 / 128 rows: 148 workgroups of
     // 128 98 / 103, 226 82 / 81, 282 349 / 350, 304 118 / 114, 512 235 / 228, 1500 1995 / 1895; 33 81 / 87;
     // not for elements of at most 64 rows: 568 x 1 x 1 30.9 / 33.9, 1079 x 8 x 7 91 / 97.
     // Workgroups of 64 rows and half the columns where whole rows are no workgroup per compute unit, halves / whole rows: 38 workgroups
@@ -273,7 +322,7 @@ void mla_absorbed_query_product_launch(bf16_t* query_latent_gradient, bf16_t* qu
     };
     const long long workgroups = (rows + 63) / 64 * batch_size;   // of 64 rows
     if (rows > 64 && (rows + 127) / 128 * batch_size >= units) {
-        start(launch<2, 1>);
+        start(launch<2, 2>);
     } else if (workgroups > units || (2 * workgroups > units && sequence_length <= SHORT_TOKENS)) {
         start(launch<1, 1>);
     } else {
