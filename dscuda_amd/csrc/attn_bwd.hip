@@ -100,9 +100,17 @@ __global__ __launch_bounds__(256) void attention_backward_statistics_kernel(
     if (row >= rows) {
         return;
     }
-    const long long h = row % heads;
-    const long long s = (row / heads) % padded;
-    const long long b = row / (heads * padded);
+    long long h, s, b;
+    if (rows <= 0xffffffffLL) {   // (64-bit divisions: 8 heads of 300 tokens, 192 / 128 columns, forward and backward 36.05 us, 35.8 so)
+        const unsigned token = (unsigned)row / (unsigned)heads;
+        h = (unsigned)row - token * (unsigned)heads;
+        b = token / (unsigned)padded;
+        s = token - (unsigned)b * (unsigned)padded;
+    } else {
+        h = row % heads;
+        s = (row / heads) % padded;
+        b = row / (heads * padded);
+    }
     float sum = 0.f;
     float lse2 = INFINITY;
     if (s < sequence_length) {
