@@ -27,6 +27,7 @@
 #include "attn_kernels.h"
 #include "hip_common.h"
 #include "index_math.h"
+#include "lds_tiles.h"
 
 #include <algorithm>
 #include <cstdint>
@@ -45,9 +46,6 @@ constexpr int PITCH = 2 * RANK + 16;            // bytes per weight row in LDS: 
 constexpr int TILE_BYTES = TILE * PITCH;
 constexpr int WEIGHT_BYTES = (HEAD / TILE) * TILE_BYTES;   // 133 120
 constexpr int AHEAD = 6;
-
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4* transposing_read_pointer;
 
 // W[h] ([128][512], `weight`) -> LDS, 16-byte pieces
 // (sixteen loads in flight per thread and round trip: one at a time, the 32 round trips of a thread's share were a
@@ -523,6 +521,95 @@ __global__ __launch_bounds__(THREADS, 2) void mla_absorb_query_slice_kernel(bf16
     }
 }
 
+// out = o_latent W_UV^T as a stream of token tiles: a wave holds 32 of the head's 128 weight rows in 128 registers, the four
+// waves of a workgroup read each tile of 32 tokens from LDS, whole rows of 1 KB brought there by global_load_lds two tiles
+// ahead, a workgroup a compute unit (its LDS admits a second one, for what does not come out even).  blockIdx.x =
+// chunk * heads + head.  Bound by the rows read.  mla_unabsorb_output_kernel, each of whose waves fetches a token's row 32
+// bytes at a time and keeps 128 KB of weight in LDS, -> here, us, inputs that are not in the caches: 1024 tokens x 128 heads
+// 41.1 -> 33.9 (185 MB, 5.5 TB/s), 4096 x 128 135 -> 125, 512 x 128 26.2 -> 19.9, 300 x 128 22.4 -> 14.5, 200 x 300 36 -> 27,
+// 1000 x 64 25.9 -> 20.1, 1000 x 16 10.9 -> 9.5, 700 x 8 9.9 -> 7.6, 4000 x 8 13.2 / 13.3.  Three or four tiles ahead: 34.3 / 34.5,
+// 122 / 123, 20.7 / 21.1, 15.5 / 16.2, 31 / 32, 20.7 / 21.4.
+constexpr int STREAM_TILE_BYTES = TILE * 2 * RANK;           // 32 KB
+constexpr int STREAM_SLOTS = 2;
+constexpr int STREAM_OUT_AT = STREAM_SLOTS * STREAM_TILE_BYTES;
+constexpr int STREAM_OUT_PITCH = 2 * HEAD + 16;
+constexpr int STREAM_LDS_BYTES = STREAM_OUT_AT + TILE * STREAM_OUT_PITCH;
+static_assert(2 * STREAM_LDS_BYTES <= 160 * 1024, "two workgroups fit a compute unit");
+
+__global__ __launch_bounds__(THREADS, 2) void mla_unabsorb_output_stream_kernel(bf16_t* __restrict__ y,
+                                                                                const bf16_t* __restrict__ x,
+                                                                                const bf16_t* __restrict__ weight,
+                                                                                long long tokens,
+                                                                                long long tokens_per_workgroup, int heads,
+                                                                                Strides strides) {
+    constexpr int KSTEPS = RANK / 16;
+    constexpr int ROWS = TILE / (THREADS / 64);    // of a tile that a wave requests, one an instruction
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int lane = tid % 64;
+    const int lq = lane % 32;
+    const int g = lane / 32;
+    const int head = blockIdx.x % heads;
+    const long long first = blockIdx.x / heads * tokens_per_workgroup;
+    const int tiles = (int)((min(tokens_per_workgroup, tokens - first) + TILE - 1) / TILE);
+    const bf16_t* x_head = x + head * strides.x_head;
+    const unsigned lds_base = lds_offset_of(lds);
+    auto request = [&](int tile) {
+        const long long token0 = first + (long long)tile * TILE;
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) {
+            const int row = ROWS * wave + i;
+            // rows past the end repeat the last one, nothing of theirs is stored
+            direct_load_16_offset(x_head + min(token0 + row, tokens - 1) * strides.x_token,
+                                  16u * (unsigned)(lane ^ index_math::tile_swizzle<2 * RANK>(row)),
+                                  lds_base + tile % STREAM_SLOTS * STREAM_TILE_BYTES + row * 2 * RANK);
+        }
+    };
+    u32x4 weights[KSTEPS];
+    fetch_token_row(weights, weight + head * strides.w_head + (TILE * wave + lq) * RANK, true, g);
+    for (int tile = 0; tile < min(tiles, STREAM_SLOTS); ++tile) request(tile);
+    TileReads<2 * RANK> reads;
+    reads.init(lane);
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks) asm volatile("" : "+v"(weights[ks]));   // here, not at every use
+    for (int tile = 0; tile < tiles; ++tile) {
+        // The tile has landed; the requests of the next one, the youngest of this wave, may be on their way.
+        if (tile + 1 < tiles) wait_vector_memory<ROWS>(); else wait_vector_memory<0>();
+        workgroup_barrier();
+        unsigned at[TileReads<2 * RANK>::NAT];
+        rebase(at, reads.natural, tile % STREAM_SLOTS * STREAM_TILE_BYTES);
+        f32x16 acc;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+        bf16x8 ring[AHEAD];
+        unrolled<0, AHEAD>([&](auto tag) { ring[decltype(tag)::value] = natural_fragment<2 * RANK, 0, decltype(tag)::value>(lds, at); });
+        unrolled<0, KSTEPS>([&](auto tag) {
+            constexpr int I = decltype(tag)::value;
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, weights[I]), ring[I % AHEAD], acc, 0, 0, 0);
+            if constexpr (I + AHEAD < KSTEPS) ring[I % AHEAD] = natural_fragment<2 * RANK, 0, I + AHEAD>(lds, at);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        // lane holds token lq and columns 32*wave + 8*i4 + 4*g .. +3: rows of 256 bytes through LDS
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+            *reinterpret_cast<u32x2*>(lds + STREAM_OUT_AT + lq * STREAM_OUT_PITCH + 64 * wave + 16 * i4 + 8 * g) =
+                u32x2{pack_bf16(acc[4 * i4 + 0], acc[4 * i4 + 1]), pack_bf16(acc[4 * i4 + 2], acc[4 * i4 + 3])};
+        }
+        workgroup_barrier();   // the rows are there, and everybody has read the tile
+        const long long token0 = first + (long long)tile * TILE;
+        bf16_t* y_tile = y + head * strides.y_head + token0 * strides.y_token;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int row = 8 * wave + 4 * j + lane / 16;   // 256 bytes of four rows an instruction
+            const u32x4 bits = *reinterpret_cast<const u32x4*>(lds + STREAM_OUT_AT + row * STREAM_OUT_PITCH + 16 * (lane % 16));
+            if (token0 + row < tokens) *reinterpret_cast<u32x4*>(y_tile + row * strides.y_token + 8 * (lane % 16)) = bits;
+        }
+        // behind the stores: the wait above then counts these requests alone
+        if (tile + STREAM_SLOTS < tiles) request(tile + STREAM_SLOTS);
+    }
+}
+
 void check(bool condition, const char* message) {
     if (!condition) throw std::invalid_argument(message);
 }
@@ -571,20 +658,19 @@ void launch_slices(bf16_t* y, const bf16_t* x, const bf16_t* weight, long long t
     HIP_CHECK(hipGetLastError());
 }
 
-// Whole weights in LDS: the tokens of a head are cut into chunks, one workgroup each (multiples of the 128 tokens four waves take); every
-// workgroup stages the head's weight first, which costs it about as long as 128 tokens.  The number of chunks is
+// The tokens of a head are cut into chunks, one workgroup each, multiples of `granule` tokens; every
+// workgroup fetches the head's weight first, which costs it about as long as 128 tokens.  The number of chunks is
 // the one with the shortest schedule: rounds of workgroups over the compute units times the cost of a workgroup
-// (4096 tokens x 128 heads on 256 compute units: two chunks, one round, 138 / 171 us against 145 / 178 us with four).
-template <typename Kernel>
-void launch_whole(Kernel kernel, bf16_t* y, const bf16_t* x, const bf16_t* weight, long long tokens, int heads,
-                  const Strides& strides, hipStream_t stream) {
+// (whole weights in LDS, 4096 tokens x 128 heads on 256 compute units: two chunks, one round, 138 / 171 us against 145 / 178
+// us with four; un-absorb as a stream, 1024 x 128: 256 workgroups 33.5 us, 128 45.5, 384 37.3, 512 36.0, 768 40.3).
+long long tokens_per_workgroup(long long tokens, int heads, long long granule) {
     constexpr long long STAGING_TOKENS = 4 * TILE;
     const long long units = std::max(1, compute_units());
-    const long long most = (tokens + 4 * TILE - 1) / (4 * TILE);
+    const long long most = (tokens + granule - 1) / granule;
     const long long limit = std::min(most, std::max(1LL, (4 * units + heads - 1) / heads));
     long long chunks = 1, best = -1;
     for (long long candidate = 1; candidate <= limit; ++candidate) {
-        const long long per_chunk = ((tokens + candidate - 1) / candidate + 4 * TILE - 1) / (4 * TILE) * (4 * TILE);
+        const long long per_chunk = ((tokens + candidate - 1) / candidate + granule - 1) / granule * granule;
         const long long workgroups = heads * ((tokens + per_chunk - 1) / per_chunk);
         const long long cost = (workgroups + units - 1) / units * (STAGING_TOKENS + per_chunk);
         if (best < 0 || cost < best) {
@@ -592,11 +678,32 @@ void launch_whole(Kernel kernel, bf16_t* y, const bf16_t* x, const bf16_t* weigh
             chunks = candidate;
         }
     }
-    long long per_workgroup = (tokens + chunks - 1) / chunks;
-    per_workgroup = (per_workgroup + 4 * TILE - 1) / (4 * TILE) * (4 * TILE);
+    return ((tokens + chunks - 1) / chunks + granule - 1) / granule * granule;
+}
+
+// Whole weights in LDS: chunks are multiples of the 128 tokens four waves take.
+template <typename Kernel>
+void launch_whole(Kernel kernel, bf16_t* y, const bf16_t* x, const bf16_t* weight, long long tokens, int heads,
+                  const Strides& strides, hipStream_t stream) {
+    const long long per_workgroup = tokens_per_workgroup(tokens, heads, 4 * TILE);
     const long long grid = (tokens + per_workgroup - 1) / per_workgroup;
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid, (unsigned)heads), dim3(THREADS), LDS_BYTES, stream, y, x, weight,
                        tokens, per_workgroup, strides);
+    HIP_CHECK(hipGetLastError());
+}
+
+void launch_stream(bf16_t* y, const bf16_t* x, const bf16_t* weight, long long tokens, int heads, const Strides& strides,
+                   hipStream_t stream) {
+    static hip_common::OncePerDevice prepared;
+    prepared.run([] {
+        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(mla_unabsorb_output_stream_kernel),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, STREAM_LDS_BYTES));
+    });
+    const long long per_workgroup = tokens_per_workgroup(tokens, heads, TILE);
+    const long long grid = (tokens + per_workgroup - 1) / per_workgroup * heads;
+    check(grid <= 0x7fffffffLL, "MLA projection: more tokens than the grid allows");
+    hipLaunchKernelGGL(mla_unabsorb_output_stream_kernel, dim3((unsigned)grid), dim3(THREADS), STREAM_LDS_BYTES, stream, y, x,
+                       weight, tokens, per_workgroup, heads, strides);
     HIP_CHECK(hipGetLastError());
 }
 
@@ -659,6 +766,10 @@ void mla_unabsorb_output_dispatch(bf16_t* output, const bf16_t* output_latent, c
     });
     if (apart && tiles * heads <= UNABSORB_FEW_TILES) {
         launch_few(mla_unabsorb_output_few_kernel, output, output_latent, weight, tokens, heads, strides, stream);
+        return;
+    }
+    if (apart) {
+        launch_stream(output, output_latent, weight, tokens, heads, strides, stream);
         return;
     }
     launch_whole(mla_unabsorb_output_kernel, output, output_latent, weight, tokens, heads, strides, stream);
