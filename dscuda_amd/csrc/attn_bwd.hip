@@ -87,8 +87,13 @@ __device__ __forceinline__ void clear(f32x16& value) {
 
 // ---- statistics ---------------------------------------------------------------
 
-// One group of DV / 8 lanes per (b, s, h) row of the sequence padded to whole query tiles.
-template <int DV>
+// One group of DV / 8 lanes per (b, s, h) row of the sequence padded to whole query tiles.  STREAMING: many rows of 128 columns, which
+// the next launches do not find in the caches anyway.  Forward and backward, us, 192 / 128 columns, read as usual / streamed: 1000
+// tokens x 16 heads (8 MB) 63.8 / 64.4, 1000 x 32 (16 MB) 87.8 / 87.8, 1500 x 32 148.3 / 146.5, 2000 x 32 228 / 224, 2 x 2000 x 32
+// 409 / 404, 3 x 3000 x 32 1233 / 1224, 4096 x 128 2821 / 2819; 64 columns 8 x 1024 x 32 on 8 306 / 312, 8192 x 16 on 4 809 / 813.
+constexpr long long STATISTICS_STREAM_BYTES = 24LL << 20;
+
+template <int DV, bool STREAMING>
 __global__ __launch_bounds__(256) void attention_backward_statistics_kernel(
     float* __restrict__ statistics, const bf16_t* __restrict__ output_gradient, const bf16_t* __restrict__ output,
     const float* __restrict__ logsumexp, int batch_size, int sequence_length, int heads, int query_tiles) {
@@ -115,8 +120,10 @@ __global__ __launch_bounds__(256) void attention_backward_statistics_kernel(
     float lse2 = INFINITY;
     if (s < sequence_length) {
         const long long source = ((b * sequence_length + s) * heads + h) * DV;
-        const u32x4 x = *reinterpret_cast<const u32x4*>(output_gradient + source + part * 8);
-        const u32x4 y = *reinterpret_cast<const u32x4*>(output + source + part * 8);
+        const u32x4* x_place = reinterpret_cast<const u32x4*>(output_gradient + source + part * 8);
+        const u32x4* y_place = reinterpret_cast<const u32x4*>(output + source + part * 8);
+        const u32x4 x = STREAMING ? __builtin_nontemporal_load(x_place) : *x_place;
+        const u32x4 y = STREAMING ? __builtin_nontemporal_load(y_place) : *y_place;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             sum += bf16_bits_to_float(x[j] & 0xffffu) * bf16_bits_to_float(y[j] & 0xffffu);
@@ -1061,8 +1068,14 @@ void launch_backward(bf16_t* query_gradient, bf16_t* key_gradient, bf16_t* value
         raise_lds_limit(attention_key_value_gradient_kernel<DQK, DV>, KC::LDS_BYTES);
         raise_lds_limit(attention_query_gradient_kernel<DQK, DV>, QC::LDS_BYTES);
     });
-    hipLaunchKernelGGL((attention_backward_statistics_kernel<DV>), dim3((unsigned)(padded_rows / STATISTICS_ROWS)),
-                       dim3(256), 0, stream, statistics, output_gradient, output, logsumexp, batch_size, sequence_length, heads,
+    auto statistics_kernel = attention_backward_statistics_kernel<DV, false>;
+    if constexpr (DV == 128) {
+        if ((long long)batch_size * sequence_length * heads * (4LL * DV) >= STATISTICS_STREAM_BYTES) {
+            statistics_kernel = attention_backward_statistics_kernel<DV, true>;
+        }
+    }
+    hipLaunchKernelGGL(statistics_kernel, dim3((unsigned)(padded_rows / STATISTICS_ROWS)), dim3(256), 0,
+                       stream, statistics, output_gradient, output, logsumexp, batch_size, sequence_length, heads,
                        shape.query_tiles);
     HIP_CHECK(hipGetLastError());
     for (long long first = 0; first < shape.pairs; first += shape.pairs_per_launch) {
