@@ -1,6 +1,8 @@
 // Absorbed-weight MLA over a shared 512+64 latent KV stream for gfx950:
 // single-token decode from a paged cache (split-KV + merge), and which kernel
-// takes a prefill forward.  Takes the place of the reference's
+// takes a call.  The split kernel of this file is for 128 heads a workgroup and
+// pages that hold no whole units of 32 keys; mla_wide.hip and mla_narrow.hip
+// have the others.  Takes the place of the reference's
 // mla_decode_split_kernel / mla_decode_combine_kernel
 // (kernels/attention/mla/sm89.cu:413-507); the decomposition below is built around 64-lane MFMA waves and the 160 KB
 // LDS and shares nothing with their per-head scalar loops.

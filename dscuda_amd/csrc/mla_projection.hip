@@ -10,7 +10,7 @@
 // wkv_b[:, -128:] after the attention).  BF16 in and out, FP32 accumulation on the
 // 32x32x16 MFMA.
 //
-// A head's weight (128 KB) is staged once per workgroup in LDS, row-major as 32-row tiles;
+// Whole weights: a head's weight (128 KB) is staged once per workgroup in LDS, row-major as 32-row tiles;
 // a wave then takes 32 tokens at a time, holds their input rows in registers straight from
 // memory (lane = token, as the operand whose column is the token) and forms the transposed
 // product y^T = W x^T; a lane ends up with one token and groups of four neighbouring output
@@ -21,6 +21,7 @@
 //              into the same order by one lane exchange per step.
 //   un-absorb: W_UV[h] is [d][c]; the contraction index c is the tile column: plain 16-byte
 //              row reads on both sides.
+// Which calls take it, and the kernels for few tokens, for quarters of the columns and for streams of token tiles: below.
 // Either way a token tile costs 128 MFMAs per wave against 8 + 32 KB (absorb) or 32 + 8 KB
 // of memory traffic: the kernels are bound by memory.
 

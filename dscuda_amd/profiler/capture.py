@@ -87,8 +87,8 @@ Case = collections.namedtuple("Case", "stem label command counter_command kernel
 # Parts of the names of the kernels that an operation may launch, whichever of them a shape takes
 FORWARD_KERNELS = ["attention_forward"]
 BACKWARD_KERNELS = ["attention_backward", "attention_key_value", "attention_query"]
-DECODE_KERNELS = ["mla_decode", "mla_narrow_decode", "mla_narrow_merge"]
-ABSORBED_KERNELS = ["mla_absorbed", "mla_narrow_forward", "mla_short"]
+DECODE_KERNELS = ["mla_decode", "mla_narrow_decode", "mla_narrow_merge", "mla_wide_decode"]
+ABSORBED_KERNELS = ["mla_absorbed", "mla_narrow_forward", "mla_short", "mla_wide_forward"]
 PROJECTION_KERNELS = ["mla_absorb_query", "mla_unabsorb_output"]
 ROPE_KERNELS = ["rope_apply"]
 
