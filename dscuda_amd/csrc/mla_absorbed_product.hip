@@ -17,6 +17,7 @@
 //               2201 and, requests apart, 2166 -> 2130 on other boxes), 4096 x 32 2102 -> 2080, 2048 x 16 346 -> 340,
 //               300 x 128 140.1 -> 137.8, 1024 x 128 680.8 / 681.5, 2 x 700 x 32 202.6 / 203.7.  All columns with the requests
 //               among the products are within 1 % of either.
+//               (PARTS = 1: 128 rows and all columns, the better one for much of dS.)
 //   GROUP = 1   64 rows, all columns or (PARTS = 2) half of them, for few rows.
 #include "attn_kernels.h"
 #include "hip_common.h"
@@ -36,8 +37,8 @@ constexpr int XCDS = 8;
 
 template <int GROUP, int PARTS>
 struct ProductLayout {
-    static_assert(GROUP == 1 || PARTS == 2, "the accumulators of 256 rows take halves of the columns");
-    static constexpr int ROW_GROUPS = 2 * GROUP;
+    static constexpr bool PAIRED = GROUP == 2 && PARTS == 2;       // halves of the columns side by side
+    static constexpr int ROW_GROUPS = PAIRED ? 4 : 2;
     static constexpr int ROW_TILES = ROW_GROUPS * GROUP;
     static constexpr int ROWS = TILE * ROW_TILES;
     static constexpr int COLUMN_WAVES = THREADS / 64 / ROW_GROUPS;
@@ -47,7 +48,7 @@ struct ProductLayout {
     static constexpr int ROPE_AT = TILE * WIDE_ROW;
     static constexpr int DS_AT = ROPE_AT + TILE * NARROW_ROW;
     static constexpr int STAGE_BYTES = DS_AT + ROW_TILES * index_math::KeptGradients::BLOCK_BYTES;
-    static constexpr int STAGES = 4;
+    static constexpr int STAGES = GROUP == 2 && PARTS == 1 ? 3 : 4;
     static constexpr int OUT_ROPE = WIDE_ROW;                            // of a staged gradient row
     static constexpr int OUT_PITCH = WIDE_ROW + 2 * ROPE / PARTS + 16;
     static constexpr int OUT_BYTES = ROWS * OUT_PITCH;
@@ -72,12 +73,12 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
     const int g = lane / 32;
     const int T = sequence_length;
     const long long rows = (long long)T * heads;
-    // GROUP = 2: the halves of the columns, which read the same dS, run side by side on one XCD
-    const int column_part = GROUP == 2 ? blockIdx.x / XCDS % 2 : blockIdx.x % PARTS;
-    const unsigned item = GROUP == 2 ? blockIdx.x / (2 * XCDS) * XCDS + blockIdx.x % XCDS : blockIdx.x / PARTS;
+    // PAIRED: the halves of the columns, which read the same dS, run side by side on one XCD
+    const int column_part = L::PAIRED ? blockIdx.x / XCDS % 2 : blockIdx.x % PARTS;
+    const unsigned item = L::PAIRED ? blockIdx.x / (2 * XCDS) * XCDS + blockIdx.x % XCDS : blockIdx.x / PARTS;
     const int batch = item % (unsigned)batch_size;
     const int row_block = row_blocks - 1 - (int)(item / (unsigned)batch_size);   // latest rows (most keys) first
-    if (GROUP == 2 && row_block < 0) return;               // the last of the groups of XCDS items is filled up
+    if (L::PAIRED && row_block < 0) return;               // the last of the groups of XCDS items is filled up
     const long long row0 = (long long)row_block * L::ROWS;
     const long long batch_row0 = (long long)batch * rows;
     const unsigned char* latent = reinterpret_cast<const unsigned char*>(kv_latent + (size_t)batch * T * RANK) + column_part * L::WIDE_ROW;
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
             const unsigned char* source = kept_batch + kept.at(tile, ds_row_tile) + 1024 * (ds_part % 2 + PIECE);
             const unsigned piece_target = target + L::DS_AT + 1024 * (ds_part + PIECE);
             // of the halves of the columns one finds what the other has fetched
-            if constexpr (GROUP == 2) direct_load_16_offset(source, 16u * (unsigned)lane, piece_target);
+            if constexpr (L::PAIRED) direct_load_16_offset(source, 16u * (unsigned)lane, piece_target);
             else direct_load_16_offset_streaming(source, 16u * (unsigned)lane, piece_target);
         }
     };
@@ -173,7 +174,7 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
         const int behind = min(tiles - 1 - tile, AHEAD - 1);   // tiles that may stay in flight
         if (behind == 0) {
             wait_for_all_but(std::integral_constant<int, 0>{});
-        } else if (behind == 1) {
+        } else if (AHEAD == 2 || behind == 1) {
             wait_for_all_but(std::integral_constant<int, 1>{});
         } else {
             wait_for_all_but(std::integral_constant<int, 2>{});
@@ -295,7 +296,7 @@ void launch(bf16_t* query_latent_gradient, bf16_t* query_rope_gradient, const un
     const long long rows = (long long)sequence_length * heads;
     const long long row_blocks = (rows + L::ROWS - 1) / L::ROWS;
     const long long items = row_blocks * batch_size;
-    const long long workgroups = PARTS * (GROUP == 2 ? (items + XCDS - 1) / XCDS * XCDS : items);
+    const long long workgroups = PARTS * (L::PAIRED ? (items + XCDS - 1) / XCDS * XCDS : items);
     hipLaunchKernelGGL((mla_absorbed_query_product_kernel<GROUP, PARTS>), dim3((unsigned)workgroups), dim3(THREADS),
                        L::LDS_BYTES, stream, query_latent_gradient, query_rope_gradient, kept_gradients, kv_latent, key_rope,
                        batch_size, sequence_length, heads, key_tiles, (int)row_blocks);
@@ -316,6 +317,10 @@ void mla_absorbed_query_product_launch(bf16_t* query_latent_gradient, bf16_t* qu
     // of 64 rows 45 / 49, 63 63 / 68, 128 106 / 118, 220 (2010 x 7) 130 / 143, 159 (3 x 279 x 12) 49 / 51; but where the halves are
     // more than one round of them, short walks pay for a second start: 165 x 1 x 1 17.0 / 14.7, 57 x 21 x 11 32.5 / 30.1,
     // 14 x 73 x 12 40.4 / 38.2, 47 x 133 x 1 30.7 / 29.6, 3 x 182 x 20 45.9 / 44.9; 3 x 204 x 14 41.2 / 42.0.
+    // 128 rows and all columns where dS is over 0.6 GB, which halves of the columns do not find in the caches as often: forward
+    // and backward in us, 256 rows / 128, 4096 tokens x 128 heads 8323 / 8277, 4096 x 64 4107 / 4099, 3000 x 128 4523 / 4508;
+    // 2048 x 128 and 4096 x 32 equal.
+    constexpr long long PAIRED_LIMIT = 600LL << 20;   // (row, key) pairs, half of them visible, two bytes each
     constexpr int SHORT_TOKENS = 192;
     const long long rows = (long long)sequence_length * heads;
     const int units = hip_common::compute_units_of_current_device();
@@ -325,7 +330,7 @@ void mla_absorbed_query_product_launch(bf16_t* query_latent_gradient, bf16_t* qu
     };
     const long long workgroups = (rows + 63) / 64 * batch_size;   // of 64 rows
     if (rows > 64 && (rows + 127) / 128 * batch_size >= units) {
-        start(launch<2, 2>);
+        if (rows * sequence_length * batch_size < PAIRED_LIMIT) start(launch<2, 2>); else start(launch<2, 1>);
     } else if (workgroups > units || (2 * workgroups > units && sequence_length <= SHORT_TOKENS)) {
         start(launch<1, 1>);
     } else {
