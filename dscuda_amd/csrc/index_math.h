@@ -943,6 +943,10 @@ DSCUDA_HOST_DEVICE inline long long plan_first_sequence_at(int batch) { return P
 DSCUDA_HOST_DEVICE inline long long plan_elements(int batch, int workgroups) {
     return plan_first_sequence_at(batch) + workgroups;
 }
+// Thread `thread` of `threads` copies its share of a plan's prefix, which has an entry more than there are sequences.
+DSCUDA_HOST_DEVICE inline void leave_prefix(int* plan, const int* prefix, int batch, int thread, int threads) {
+    for (int s = thread; s <= batch; s += threads) plan[plan_prefix_at() + s] = prefix[s];
+}
 // Size of a plan buffer that fits whatever device builds the plan: a call cuts its list into at
 // most one range per compute unit (the host clamps the count it asks the device for to
 // PLAN_MAX_WORKGROUPS), or runs one workgroup per sequence.

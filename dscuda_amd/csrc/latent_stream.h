@@ -471,7 +471,7 @@ __device__ __forceinline__ DecodeRange decode_range(int* plan, const int* cache_
                 plan[PLAN_MODE] = plan_mode(cut, range.wide);
                 plan[PLAN_RANGES] = ranges;
             }
-            if (tid <= batch_size) plan[index_math::plan_prefix_at() + tid] = own_prefix[tid];
+            index_math::leave_prefix(plan, own_prefix, batch_size, tid, threads);
         }
     } else {
         total = plan[PLAN_TOTAL];

@@ -738,6 +738,22 @@ void check_decode_layout() {
     EXPECT(moved > 0 && decode_form_of_call(20, 128, 32, 1, 256, RANK).row_blocks == 0, "pages of one token, 128 heads");
 }
 
+// ---- the plan a decode kernel leaves for its merge: every entry of the prefix, also where the batch is as large as the
+// workgroup of 256 or 512 threads, and nothing behind it
+void check_leave_prefix() {
+    for (int threads : {256, 512}) {
+        for (int batch : {1, 64, 65, 255, 256}) {
+            std::vector<int> prefix(batch + 1), plan(plan_elements(batch, 0) + 1, -7);
+            for (int s = 0; s <= batch; ++s) prefix[s] = 11 * s;
+            for (int thread = 0; thread < threads; ++thread) leave_prefix(plan.data(), prefix.data(), batch, thread, threads);
+            for (int s = 0; s <= batch; ++s) {
+                EXPECT(plan[plan_prefix_at() + s] == 11 * s, "B %d, %d threads: entry %d not left", batch, threads, s);
+            }
+            EXPECT(plan[plan_first_sequence_at(batch)] == -7 && plan[plan_prefix_at() - 1] == -7, "B %d, %d threads", batch, threads);
+        }
+    }
+}
+
 // ---- projections: rows_apart never calls rows that share an element apart, and sees what is apart in the usual layouts
 void check_rows_apart() {
     const long long strides[][2] = {{8, 8}, {24, 8}, {24, 12}, {30, 12}, {40, 8}};
@@ -995,6 +1011,7 @@ int main() {
     check_forward_row_blocks();
     check_decode_ranges();
     check_decode_layout();
+    check_leave_prefix();
     check_rows_apart();
     if (failures) {
         std::printf("%d check(s) failed\n", failures);

@@ -38,6 +38,8 @@ def _inputs(batch, heads, page_size, lengths, seed):
     (257, 65, 64, 8, [70, 5, 40]),   # a plan by a kernel of its own
     (64, 16, 64, 8, [200, 33, 1, 90]), (65, 16, 64, 8, [200, 33, 1, 90]), (40, 64, 64, 8, EDGES), (1, 128, 64, 8, [700]),
     (64, 16, 48, 2, [13, 400]), (25, 128, 48, 8, EDGES),
+    (255, 128, 48, 8, [70, 5, 40]), (256, 128, 48, 8, [70, 5, 40, 300]), (256, 128, 64, 8, [70, 5, 40, 300]),   # as many sequences as a
+    (256, 16, 48, 8, [70, 5, 40, 300]), (257, 128, 48, 8, [70, 5, 40, 300]),                                    # workgroup plans for
 ])
 def test_decode(cuda, batch, heads, page_size, splits, lengths):
     query, cache, paged, table, lengths_t = _inputs(batch, heads, page_size, lengths, seed=batch + heads)
@@ -47,7 +49,9 @@ def test_decode(cuda, batch, heads, page_size, splits, lengths):
     # a table entry past the last page with a visible token is never read: such entries hold what no pool has
     for row, length in enumerate(lengths_t.tolist()):
         on_gpu[2][row, (length + page_size - 1) // page_size:] = 0x3fffffff
-    out, lse = ops.mla_decode(*on_gpu, scale, splits=splits)
+    # an entry of the plan that the call does not write for itself stands for no sequence
+    workspace = ops.mla_decode_workspace(batch, heads, splits).zero_()
+    out, lse = ops.mla_decode(*on_gpu, scale, splits=splits, workspace=workspace)
     plan = ops.mla_decode_plan(on_gpu[3], heads, splits)
     planned, planned_lse = ops.mla_decode_planned(*on_gpu, plan, scale, splits=splits)
     torch.cuda.synchronize()
