@@ -391,6 +391,34 @@ DSCUDA_HOST_DEVICE inline unsigned divide(unsigned n, const FastDivision& by) {
     return (unsigned)(((((unsigned long long)n * by.multiplier) >> 32) + n) >> by.shift);
 }
 
+// Whether the 128-row forward numbers the row blocks of all batch elements together, from heavy to light, or one element
+// after the other, which keeps few keys live in the L2s.  A workgroup takes a block of every round of `workgroups`, rounds there
+// and back.  Numbered together the rounds even out; one element after the other they do only where elements fill rounds or rounds
+// hold whole elements, and there is an even number of them.  Everywhere else a workgroup gets the heavy blocks of several elements.
+// Forward in us, one after the other / together: 4 x 1957 x 16 372 / 241, 16 x 537 x 8 93 / 57, 8 x 1976 x 32 1323 / 994, 2 x 3000 x 32
+// 631 / 523, 16 x 484 x 128 723 / 701, 9 x 800 x 64 452 / 457; even ones: 64 x 256 x 64 556 / 590, 12 x 1024 x 64 893 / 923, 2 x 2048 x
+// 128 1031 / 1059, 40 x 1018 x 16 756 / 774.
+DSCUDA_HOST_DEVICE inline bool forward_interleaves(int sequence_length, long long batch, long long row_blocks, long long workgroups) {
+    if (batch * sequence_length * 2 * (512 + 64) <= (3 << 20)) return true;   // the keys of all fit an L2
+    const bool whole = row_blocks % workgroups == 0 || workgroups % row_blocks == 0;
+    return !whole || batch * row_blocks % (2 * workgroups) != 0;
+}
+
+// Item `index` of that order: the batch element and its row block, the heaviest first.  by_order: divides by the number of batch
+// elements (interleaved) or of row blocks.
+DSCUDA_HOST_DEVICE inline void forward_item(unsigned index, bool interleaved, const FastDivision& by_order, unsigned row_blocks,
+                                            unsigned& batch, unsigned& row_block) {
+    const unsigned quotient = divide(index, by_order);
+    const unsigned rest = index - quotient * by_order.divisor;
+    batch = interleaved ? rest : quotient;
+    row_block = row_blocks - 1 - (interleaved ? quotient : rest);
+}
+
+// Index of the item that `workgroup` takes in a round.
+DSCUDA_HOST_DEVICE inline unsigned forward_index(unsigned round, unsigned workgroup, unsigned workgroups) {
+    return round * workgroups + (round & 1 ? workgroups - 1 - workgroup : workgroup);
+}
+
 // Items (batch, query head, query block), numbered so that what runs at one time shares keys and ends together.
 // Workgroups go to the XCDs round-robin by linear id and every XCD has an L2 of its own, so the query heads that read
 // one key/value head stay on one XCD; with too few key/value heads for that, query heads are dealt to the XCDs one by

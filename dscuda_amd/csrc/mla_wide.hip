@@ -174,19 +174,18 @@ struct ForwardWork {
         int units;
     };
 
-    // The heaviest blocks first, rounds there and back: a workgroup's items add up to the same for all.
+    // The heaviest blocks first, rounds there and back (index_math::forward_interleaves).
     struct Iterator {
         int round;
 
         __device__ __forceinline__ bool next(const ForwardWork& work, const Place&, Item& item) {
-            const unsigned place = round & 1 ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
-            const unsigned index = (unsigned)round * gridDim.x + place;
+            const unsigned index = index_math::forward_index((unsigned)round, blockIdx.x, gridDim.x);
             ++round;
             if (index >= work.items) return false;
-            const unsigned quotient = index_math::divide(index, work.by_order);
-            const unsigned rest = index - quotient * work.by_order.divisor;
-            item.batch = (int)(work.interleaved ? rest : quotient);
-            item.row0 = (work.row_blocks - 1 - (work.interleaved ? quotient : rest)) * WIDE_ROWS;
+            unsigned batch, row_block;
+            index_math::forward_item(index, work.interleaved, work.by_order, work.row_blocks, batch, row_block);
+            item.batch = (int)batch;
+            item.row0 = row_block * WIDE_ROWS;
             const unsigned last_row = min(work.rows, item.row0 + WIDE_ROWS) - 1;
             item.tokens = (int)index_math::divide(last_row, work.by_heads) + 1;
             item.unit_begin = 0;
@@ -843,13 +842,11 @@ void mla_wide_forward_launch(bf16_t* output, float* logsumexp, const bf16_t* que
     work.rows = (unsigned)((long long)sequence_length * heads);
     work.row_blocks = (work.rows + WIDE_ROWS - 1) / WIDE_ROWS;
     work.items = work.row_blocks * batch_size;
-    // Numbered together, the blocks of all batch elements go from heavy to light once, which the rounds even out; one batch
-    // element after the other keeps few keys live in the L2s.
-    work.interleaved = (long long)batch_size * sequence_length * 2 * WIDTH <= (3 << 20);
+    const unsigned workgroups = std::min(work.items, (unsigned)std::max(hip_common::compute_units_of_current_device(), 1));
+    work.interleaved = index_math::forward_interleaves(sequence_length, batch_size, work.row_blocks, workgroups);
     work.by_heads = index_math::fast_division((unsigned)heads);
     work.by_order = index_math::fast_division(work.interleaved ? (unsigned)batch_size : work.row_blocks);
     work.c = scale * LOG2E;
-    const unsigned workgroups = std::min(work.items, (unsigned)std::max(hip_common::compute_units_of_current_device(), 1));
     hipLaunchKernelGGL(mla_wide_forward_kernel, dim3(workgroups), dim3(WIDE_THREADS), WIDE_LDS_BYTES, stream, work);
     HIP_CHECK(hipGetLastError());
 }

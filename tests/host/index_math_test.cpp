@@ -524,6 +524,41 @@ void check_forward_row_blocks() {
     }
 }
 
+// the items of the absorbed prefill forward with 128 rows: every one once, and no workgroup walks far more units of keys than the
+// mean (`slack`: a part of the heaviest item; the last rounds are not full)
+void check_forward_deal() {
+    const int units = 256;
+    for (const auto& c : std::vector<std::tuple<int, int, int>>{
+             {4, 1957, 16}, {4, 2152, 12}, {4, 4010, 16}, {8, 1976, 32}, {16, 537, 8}, {16, 270, 8}, {40, 1058, 4}, {2, 3000, 32},
+             {3, 3000, 32}, {7, 2000, 16}, {13, 2000, 8}, {4, 1329, 12}, {16, 3789, 2}, {9, 800, 64}, {1, 1024, 128}, {2, 700, 64},
+             {64, 256, 64}, {12, 1024, 64}, {2, 2048, 128}, {40, 1018, 16}, {3, 512, 64}, {5, 2048, 16}, {321, 5, 25}}) {
+        const int batch = std::get<0>(c), tokens = std::get<1>(c), heads = std::get<2>(c);
+        const long long rows = (long long)tokens * heads;
+        const unsigned blocks = (unsigned)((rows + 127) / 128), items = blocks * batch, workgroups = std::min(items, (unsigned)units);
+        const bool interleaved = forward_interleaves(tokens, batch, blocks, workgroups);
+        const FastDivision by_order = fast_division(interleaved ? batch : blocks);
+        std::vector<int> seen(items, 0);
+        double total = 0, most = 0, heaviest = (tokens + 31) / 32;
+        for (unsigned w = 0; w < workgroups; ++w) {
+            double load = 0;
+            for (unsigned round = 0;; ++round) {
+                const unsigned index = forward_index(round, w, workgroups);
+                if (index >= items) break;
+                unsigned element, block;
+                forward_item(index, interleaved, by_order, blocks, element, block);
+                EXPECT(element < (unsigned)batch && block < blocks, "B=%d T=%d H=%d item %u", batch, tokens, heads, index);
+                ++seen[element * blocks + block];
+                load += (double)((std::min(rows, (block + 1) * 128LL) - 1) / heads + 32) / 32;
+            }
+            total += load;
+            most = std::max(most, load);
+        }
+        for (unsigned i = 0; i < items; ++i) EXPECT(seen[i] == 1, "B=%d T=%d H=%d: item %u taken %d times", batch, tokens, heads, i, seen[i]);
+        EXPECT(most <= total / workgroups + 0.55 * heaviest + 1, "B=%d T=%d H=%d: %.0f units of keys, mean %.0f, heaviest item %.0f", batch, tokens,
+               heads, most, total / workgroups, heaviest);
+    }
+}
+
 // passes over a batch: every element once, none more than allowed, sizes that differ by at most one
 void check_batch_passes() {
     for (long long batch = 1; batch <= 200; ++batch) {
@@ -1009,6 +1044,7 @@ int main() {
     check_kept_gradients();
     check_batch_passes();
     check_forward_row_blocks();
+    check_forward_deal();
     check_decode_ranges();
     check_decode_layout();
     check_leave_prefix();

@@ -21,7 +21,8 @@ pytestmark = pytest.mark.gpu
     (7, 161, 40, 128),    # batch elements end inside a row block and a unit; two rounds
     (70, 40, 64, 128),    # 1400 items of two units
     (1, 515, 131, 128),   # three rounds, the last of 16 items
-    (2, 1500, 30, 128),   # one element after the other: their keys would not fit the L2s together
+    (2, 1500, 30, 128),   # keys of both elements together do not fit an L2; their blocks are numbered together all the same
+    (4, 1024, 32, 128),   # such keys, and elements that fill rounds: one element after the other
 ])
 def test_forward(cuda, batch, tokens, heads, rows):
     units = torch.cuda.get_device_properties(cuda).multi_processor_count
