@@ -258,14 +258,21 @@ DSCUDA_HOST_DEVICE inline int narrow_forward_row_blocks(int sequence_length, int
 //   * up to one round, which 64 rows take in two: 128 rows for most of a round of walks of up to 384 keys (180 x 128
 //     19.3 / 18.5, 256 x 128 24.8 / 22.4, 8 x 125 x 32 23.8 / 17.1, 4 x 250 x 32 28.2 / 22.1, 350 x 80 25.9 / 25.7), 64 for longer
 //     ones, a unit of which takes them a third less (512 x 64 32.0 / 33.8, 1000 x 32 47.9 / 56.2, 2000 x 16 82 / 100)
+//   * up to a round and a fifth, one or two batch elements: the longest walk decides, which 64 rows take faster, where it is long
+//     against the blocks of a second round (1 x 516 x 64, 258 workgroups, 40 / 37.5; 1 x 750 x 44, 258, 46.0 / 47.1; 1 x 2064 x 16,
+//     258, 92 / 105; 1 x 8256 x 4, 258, 313 / 382; 2 x 1100 x 16, 276, 59.8 / 62.5; 1 x 1200 x 32, 300, 71.5 / 69; 1 x 2400 x 16, 300,
+//     121 / 124; 1 x 5104 x 8, 319, 257 / 254); of more elements 64 rows get the heavy blocks late (3 x 2800 x 4, 264, 151 / 137,
+//     4 x 8200 x 1 443 / 380)
 //   * beyond: 128 rows, whose second item needs no second start (258 x 128 31.0 / 23.4, 300 x 128 33.9 / 26.1, 1200 x 32 71 / 67,
-//     5 x 64 x 128 26.5 / 23.8), but for walks of one unit, of which they take two (300 x 1 x 40 13.4 / 17.1).
+//     5 x 64 x 128 26.5 / 23.8, 1 x 5440 x 8, 340, 287 / 276), but for walks of one unit, of which they take two (300 x 1 x 40
+//     13.4 / 17.1).
 DSCUDA_HOST_DEVICE inline int forward_row_blocks(int sequence_length, int heads, long long batch, int compute_units) {
     const long long workgroups = ((long long)sequence_length * heads + 127) / 128 * batch;
     const int units = (sequence_length + 31) / 32;
     if (2 * workgroups <= compute_units) return narrow_forward_row_blocks(sequence_length, heads, batch, compute_units);
     if (workgroups <= compute_units) return units <= 12 && 3 * workgroups > 2LL * compute_units ? 0 : 2;
-    return units == 1 && 4 * workgroups <= 5LL * compute_units ? 2 : 0;
+    if (units == 1) return 4 * workgroups <= 5LL * compute_units ? 2 : 0;
+    return batch <= 2 && 5 * workgroups <= 6LL * compute_units && 2 * (units - 20) > workgroups - compute_units ? 2 : 0;
 }
 
 // ---- work order of the persistent forward kernel ------------------------------

@@ -512,6 +512,9 @@ void check_forward_row_blocks() {
     struct { int batch, tokens, heads, expected; } known[] = {
         {1, 512, 8, 1}, {1, 64, 128, 1}, {1, 65, 128, 2}, {1, 433, 32, 1}, {1, 434, 32, 2}, {1, 140, 64, 1}, {1, 141, 64, 2}, {3, 300, 16, 2},
         {1, 2000, 8, 1}, {300, 1, 40, 2}, {320, 3, 42, 2}, {321, 3, 42, 0}, {1, 1024, 128, 0},
+        // just over a round of 128 rows: long walks of one or two elements by 64, short ones and more elements by 128
+        {1, 2064, 16, 2}, {1, 4666, 8, 2}, {2, 4200, 4, 2}, {1, 516, 64, 0}, {1, 258, 128, 0}, {3, 2800, 4, 0}, {1, 4912, 8, 2}, {1, 4944, 8, 0},
+        {1, 672, 49, 0}, {1, 673, 49, 2},
     };
     for (const auto& c : known) {
         const int blocks = forward_row_blocks(c.tokens, c.heads, c.batch, 256);
