@@ -8,17 +8,17 @@
 // 2048 tokens x 128 heads: 815 us of query gradients there, 358 here, for 77 us more in the key gradients, whose score
 // waves store the 0.55 GB (1236 -> 1313); 2 x 592 x 16 35 -> 24.
 //
-// A workgroup of eight waves walks the 32-key tiles its rows see, all of them through LDS stages of [32 keys][columns] + dS,
-// three tiles ahead.  A wave sums GROUP row tiles x LATENT_BLOCKS latent column blocks and, of some waves, a rope block.
-//   GROUP = 2   256 rows and half of the columns.  Bound by what a compute unit draws into LDS (some 21 bytes a cycle) and the
-//               power limit: 16 KB of latent rows, 4 of rope rows and 16 of dS a step of 1152 matrix cycles; the halves, which
-//               run side by side on one XCD, read dS from memory once.  With 128 rows and all columns (44 KB, three stages)
-//               and the requests in front of the fragments, forward and backward in us, -> here: 2048 x 128 2245 -> 2235 (2204 ->
-//               2201 and, requests apart, 2166 -> 2130 on other boxes), 4096 x 32 2102 -> 2080, 2048 x 16 346 -> 340,
-//               300 x 128 140.1 -> 137.8, 1024 x 128 680.8 / 681.5, 2 x 700 x 32 202.6 / 203.7.  All columns with the requests
-//               among the products are within 1 % of either.
-//               (PARTS = 1: 128 rows and all columns, the better one for much of dS.)
-//   GROUP = 1   64 rows, all columns or (PARTS = 2) half of them, for few rows.
+// A workgroup of eight waves owns 64 * GROUP rows and walks the 32-key tiles they see, all of them through LDS stages
+// of [32 keys][512] + [32 keys][64] + dS.  Wave (r, v) = (w / 4, w % 4): row tiles GROUP * r .., latent column blocks
+// 4v .. 4v + 3 of each of them and one of the rope blocks.  Bound by the key tiles a compute unit draws from its L2
+// (36 KB a step, some 21 bytes a cycle against 1152 matrix cycles at GROUP = 2), hence 128 rows wherever that leaves
+// workgroups enough; 192 rows need more registers than there are.  With few rows a workgroup takes half of the columns
+// (PARTS = 2, 18 KB of keys a step and compute unit).
+// The fragments are read a few products ahead, at GROUP = 2 with a tile's requests spread among the products. The backward in us
+// with requests and fragments in front of the products instead, -> here (gradient rows with ordinary stores): 1000 tokens x 64
+// heads 251 / 252, 2048 x 16 247 -> 245, 4096 x 32 1577 -> 1566, 2048 x 128 1679 -> 1664. 256 rows and half of the columns a
+// workgroup, the halves side by side on an XCD, draw as many bytes and are not faster, here / there: 1000 x 64 235 / 248, 2048 x 16
+// 244 / 249, 4096 x 8 465 / 477, 1024 x 128 486 / 498, 2048 x 128 1658 / 1683; 8 x 300 x 32 157 / 156.
 #include "attn_kernels.h"
 #include "hip_common.h"
 #include "index_math.h"
@@ -33,22 +33,18 @@ constexpr int RANK = 512;
 constexpr int ROPE = 64;
 constexpr int TILE = 32;
 constexpr int THREADS = 512;
-constexpr int XCDS = 8;
 
 template <int GROUP, int PARTS>
 struct ProductLayout {
-    static constexpr bool PAIRED = GROUP == 2 && PARTS == 2;       // halves of the columns side by side
-    static constexpr int ROW_GROUPS = PAIRED ? 4 : 2;
-    static constexpr int ROW_TILES = ROW_GROUPS * GROUP;
-    static constexpr int ROWS = TILE * ROW_TILES;
-    static constexpr int COLUMN_WAVES = THREADS / 64 / ROW_GROUPS;
-    static constexpr int DS_REQUESTS = GROUP == 1 ? 1 : ROW_TILES / 4;   // 1 KB requests of dS of a wave (GROUP = 1: of the later four)
+    static_assert(PARTS == 1 || GROUP == 1, "halves of the columns are for few rows");
+    static constexpr int ROWS = 64 * GROUP;
+    static constexpr int ROW_TILES = 2 * GROUP;
     static constexpr int WIDE_ROW = 2 * RANK / PARTS;
     static constexpr int NARROW_ROW = 2 * ROPE;
     static constexpr int ROPE_AT = TILE * WIDE_ROW;
     static constexpr int DS_AT = ROPE_AT + TILE * NARROW_ROW;
     static constexpr int STAGE_BYTES = DS_AT + ROW_TILES * index_math::KeptGradients::BLOCK_BYTES;
-    static constexpr int STAGES = GROUP == 2 && PARTS == 1 ? 3 : 4;
+    static constexpr int STAGES = GROUP == 1 ? 4 : 3;
     static constexpr int OUT_ROPE = WIDE_ROW;                            // of a staged gradient row
     static constexpr int OUT_PITCH = WIDE_ROW + 2 * ROPE / PARTS + 16;
     static constexpr int OUT_BYTES = ROWS * OUT_PITCH;
@@ -64,7 +60,7 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
     using L = ProductLayout<GROUP, PARTS>;
     using Wide = index_math::TileReadMath<L::WIDE_ROW>;
     using Narrow = index_math::TileReadMath<L::NARROW_ROW>;
-    constexpr int LATENT_BLOCKS = RANK / TILE / L::COLUMN_WAVES / PARTS;   // 32-column blocks of a wave
+    constexpr int LATENT_BLOCKS = RANK / TILE / 4 / PARTS;   // 32-column blocks of a wave
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -73,12 +69,9 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
     const int g = lane / 32;
     const int T = sequence_length;
     const long long rows = (long long)T * heads;
-    // PAIRED: the halves of the columns, which read the same dS, run side by side on one XCD
-    const int column_part = L::PAIRED ? blockIdx.x / XCDS % 2 : blockIdx.x % PARTS;
-    const unsigned item = L::PAIRED ? blockIdx.x / (2 * XCDS) * XCDS + blockIdx.x % XCDS : blockIdx.x / PARTS;
-    const int batch = item % (unsigned)batch_size;
-    const int row_block = row_blocks - 1 - (int)(item / (unsigned)batch_size);   // latest rows (most keys) first
-    if (L::PAIRED && row_block < 0) return;               // the last of the groups of XCDS items is filled up
+    const int column_part = blockIdx.x % PARTS;
+    const int batch = blockIdx.x / PARTS % batch_size;
+    const int row_block = row_blocks - 1 - blockIdx.x / PARTS / batch_size;   // latest rows (most keys) first
     const long long row0 = (long long)row_block * L::ROWS;
     const long long batch_row0 = (long long)batch * rows;
     const unsigned char* latent = reinterpret_cast<const unsigned char*>(kv_latent + (size_t)batch * T * RANK) + column_part * L::WIDE_ROW;
@@ -88,22 +81,22 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
     const unsigned char* kept_batch = kept_gradients + (size_t)batch * kept.bytes();
     const int first_row_tile = row_block * L::ROW_TILES;
 
-    const int v = wave % L::COLUMN_WAVES;
-    const int wave_row_tile = GROUP * (wave / L::COLUMN_WAVES);   // of the workgroup's
-    const int rope_tile = GROUP == 1 ? 0 : v * PARTS / 2;   // whose rope block the wave sums; GROUP = 1: not every wave has one
+    const int v = wave % 4;
+    const int wave_row_tile = GROUP * (wave / 4);   // of the workgroup's
+    const int rope_tile = GROUP == 1 ? 0 : v / 2;   // whose rope block the wave sums; GROUP = 1: not every wave has one
     const int rope_block = PARTS == 1 ? v % 2 : column_part;
     const bool sums_rope = GROUP > 1 || v < 2 / PARTS;
 
-    // A wave requests key rows 4*wave .. +3 of the wide tile (1 KB an instruction), waves 0 .. 3 also eight rows of the narrow one, and 1 KB
-    // pieces, halves of a row tile, of dS: every wave at GROUP = 2, waves 4 .. 7 at GROUP = 1.  Keys past the end repeat the last
+    // A wave requests key rows 4*wave .. +3 of the wide tile (1 KB an instruction), waves 0 .. 3 also eight rows of the narrow one, and 1 KB,
+    // half a row tile, of dS: every wave at GROUP = 2, waves 4 .. 7 at GROUP = 1.  Keys past the end repeat the last
     // one (their dS is zero), row tiles past the end repeat the last one (their results are not stored), and a tile
     // that does not see the keys yet may read what precedes its blocks and is left out below.
     const unsigned lds_base = lds_offset_of(lds);
-    const int ds_part = GROUP == 1 ? wave - 4 : L::DS_REQUESTS * wave;   // the first
+    const int ds_part = GROUP == 1 ? wave - 4 : wave;
     const int ds_row_tile = min(first_row_tile + max(ds_part, 0) / 2, kept.visits.row_tiles - 1);
     // request I (0 .. REQUESTS - 1) of a tile
     constexpr int WIDE_REQUESTS = 4 / PARTS;
-    constexpr int REQUESTS = WIDE_REQUESTS + 1 + L::DS_REQUESTS;
+    constexpr int REQUESTS = WIDE_REQUESTS + 2;
     auto request = [&](int tile, auto tag) {
         constexpr int I = decltype(tag)::value;
         const unsigned target = lds_base + tile % L::STAGES * L::STAGE_BYTES;
@@ -124,12 +117,8 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
                                       target + L::ROPE_AT + 8 * wave * L::NARROW_ROW);
             }
         } else if (GROUP > 1 || wave >= 4) {
-            constexpr int PIECE = I - WIDE_REQUESTS - 1;
-            const unsigned char* source = kept_batch + kept.at(tile, ds_row_tile) + 1024 * (ds_part % 2 + PIECE);
-            const unsigned piece_target = target + L::DS_AT + 1024 * (ds_part + PIECE);
-            // of the halves of the columns one finds what the other has fetched
-            if constexpr (L::PAIRED) direct_load_16_offset(source, 16u * (unsigned)lane, piece_target);
-            else direct_load_16_offset_streaming(source, 16u * (unsigned)lane, piece_target);
+            direct_load_16_offset_streaming(kept_batch + kept.at(tile, ds_row_tile) + 1024 * (ds_part % 2), 16u * (unsigned)lane,
+                                            target + L::DS_AT + 1024 * ds_part);
         }
     };
     auto request_tile = [&](int tile) {
@@ -138,8 +127,7 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
     // all but the newest `tiles_in_flight` tiles of the wave's requests have arrived
     auto wait_for_all_but = [&](auto tiles_in_flight) {
         constexpr int N = decltype(tiles_in_flight)::value;
-        constexpr int EACH = 4 / PARTS + L::DS_REQUESTS;
-        if (GROUP > 1 && wave < 4) wait_vector_memory<(EACH + 1) * N>(); else wait_vector_memory<EACH * N>();
+        if (GROUP > 1 && wave < 4) wait_vector_memory<REQUESTS * N>(); else wait_vector_memory<(REQUESTS - 1) * N>();
     };
     constexpr int AHEAD = L::STAGES - 1;
     for (int tile = 0; tile < min(tiles, AHEAD); ++tile) request_tile(tile);
@@ -295,9 +283,7 @@ void launch(bf16_t* query_latent_gradient, bf16_t* query_rope_gradient, const un
     });
     const long long rows = (long long)sequence_length * heads;
     const long long row_blocks = (rows + L::ROWS - 1) / L::ROWS;
-    const long long items = row_blocks * batch_size;
-    const long long workgroups = PARTS * (L::PAIRED ? (items + XCDS - 1) / XCDS * XCDS : items);
-    hipLaunchKernelGGL((mla_absorbed_query_product_kernel<GROUP, PARTS>), dim3((unsigned)workgroups), dim3(THREADS),
+    hipLaunchKernelGGL((mla_absorbed_query_product_kernel<GROUP, PARTS>), dim3((unsigned)(row_blocks * batch_size * PARTS)), dim3(THREADS),
                        L::LDS_BYTES, stream, query_latent_gradient, query_rope_gradient, kept_gradients, kv_latent, key_rope,
                        batch_size, sequence_length, heads, key_tiles, (int)row_blocks);
     HIP_CHECK(hipGetLastError());
@@ -309,18 +295,13 @@ void mla_absorbed_query_product_launch(bf16_t* query_latent_gradient, bf16_t* qu
                                        const unsigned char* kept_gradients, const bf16_t* kv_latent,
                                        const bf16_t* key_rope, int batch_size, int sequence_length, int heads,
                                        int key_tiles, hipStream_t stream) {
-    // 256 rows and half the columns where that is a workgroup per compute unit (the work of 128 whole rows, with which the
-    // line was measured).  The whole backward in us, 64 / 128 rows: 148 workgroups of
+    // 128 rows a workgroup where that is a workgroup per compute unit. The whole backward in us, 64 / 128 rows: 148 workgroups of
     // 128 98 / 103, 226 82 / 81, 282 349 / 350, 304 118 / 114, 512 235 / 228, 1500 1995 / 1895; 33 81 / 87;
     // not for elements of at most 64 rows: 568 x 1 x 1 30.9 / 33.9, 1079 x 8 x 7 91 / 97.
     // Workgroups of 64 rows and half the columns where whole rows are no workgroup per compute unit, halves / whole rows: 38 workgroups
     // of 64 rows 45 / 49, 63 63 / 68, 128 106 / 118, 220 (2010 x 7) 130 / 143, 159 (3 x 279 x 12) 49 / 51; but where the halves are
     // more than one round of them, short walks pay for a second start: 165 x 1 x 1 17.0 / 14.7, 57 x 21 x 11 32.5 / 30.1,
     // 14 x 73 x 12 40.4 / 38.2, 47 x 133 x 1 30.7 / 29.6, 3 x 182 x 20 45.9 / 44.9; 3 x 204 x 14 41.2 / 42.0.
-    // 128 rows and all columns where dS is over 0.6 GB, which halves of the columns do not find in the caches as often: forward
-    // and backward in us, 256 rows / 128, 4096 tokens x 128 heads 8323 / 8277, 4096 x 64 4107 / 4099, 3000 x 128 4523 / 4508;
-    // 2048 x 128 and 4096 x 32 equal.
-    constexpr long long PAIRED_LIMIT = 600LL << 20;   // (row, key) pairs, half of them visible, two bytes each
     constexpr int SHORT_TOKENS = 192;
     const long long rows = (long long)sequence_length * heads;
     const int units = hip_common::compute_units_of_current_device();
@@ -330,7 +311,7 @@ void mla_absorbed_query_product_launch(bf16_t* query_latent_gradient, bf16_t* qu
     };
     const long long workgroups = (rows + 63) / 64 * batch_size;   // of 64 rows
     if (rows > 64 && (rows + 127) / 128 * batch_size >= units) {
-        if (rows * sequence_length * batch_size < PAIRED_LIMIT) start(launch<2, 2>); else start(launch<2, 1>);
+        start(launch<2, 1>);
     } else if (workgroups > units || (2 * workgroups > units && sequence_length <= SHORT_TOKENS)) {
         start(launch<1, 1>);
     } else {

@@ -1,6 +1,5 @@
-"""The absorbed backward's query product with 256 rows and half of the columns a workgroup (csrc/mla_absorbed_product.hip):
-items that fill the XCDs' groups of eight or do not, rows that end inside a row tile, a wave's pair of them or a workgroup,
-workgroups whose row tiles see different numbers of key tiles."""
+"""The absorbed backward's query product with 128 rows and all columns a workgroup (csrc/mla_absorbed_product.hip): rows that
+end inside a row tile, a wave's pair of them or a workgroup, workgroups whose row tiles see different numbers of key tiles."""
 
 import pytest
 import torch
@@ -10,8 +9,7 @@ from oracle import attention_oracle as oracle
 from parity import announce, assert_close_bf16
 
 
-# workgroups of 256 rows: 264 (every second of one row), 130 (the last of nine), 172 (four an element), 131, 131, 132; of 128 rows
-# and all columns: 1560 (dS of 0.65 GB)
+# workgroups of 128 rows: 396 (every third of one row), 259, 344, 262, 262, 264, 1560 (dS of 0.65 GB)
 @pytest.mark.gpu
 @pytest.mark.parametrize("batch,tokens,heads", [(132, 257, 1), (1, 1001, 33), (43, 1000, 1), (1, 515, 65), (131, 85, 3), (4, 840, 10),
                                                  (60, 3300, 1)])
