@@ -17,8 +17,9 @@
 // The fragments are read a few products ahead, at GROUP = 2 with a tile's requests spread among the products. The backward in us
 // with requests and fragments in front of the products instead, -> here (gradient rows with ordinary stores): 1000 tokens x 64
 // heads 251 / 252, 2048 x 16 247 -> 245, 4096 x 32 1577 -> 1566, 2048 x 128 1679 -> 1664. 256 rows and half of the columns a
-// workgroup, the halves side by side on an XCD, draw as many bytes and are not faster, here / there: 1000 x 64 235 / 248, 2048 x 16
-// 244 / 249, 4096 x 8 465 / 477, 1024 x 128 486 / 498, 2048 x 128 1658 / 1683; 8 x 300 x 32 157 / 156.
+// workgroup, the halves side by side on an XCD, draw as many bytes and are not faster, here / there, both with rows
+// past the caches: 1000 x 64 235 / 248, 2048 x 16 244 / 249, 4096 x 8 465 / 477, 1024 x 128 486 / 498, 2048 x 128 1658 / 1683;
+// 8 x 300 x 32 157 / 156.
 #include "attn_kernels.h"
 #include "hip_common.h"
 #include "index_math.h"
@@ -259,11 +260,10 @@ __global__ __launch_bounds__(THREADS) void mla_absorbed_query_product_kernel(
         const size_t target = batch_row0 + row0 + out_row;
         const int part = lane % LANES;
         const unsigned char* staged = lds + out_row * L::OUT_PITCH + 16 * part;
-        u32x4* place = reinterpret_cast<u32x4*>(query_latent_gradient + target * RANK + column_part * (RANK / PARTS) + 8 * part);
-        const u32x4 bits = *reinterpret_cast<const u32x4*>(staged);
-        // many rows: past the caches, which hold the key tiles (forward and backward 2 x 700 tokens x 32 heads 199.5 -> 197.0 us,
-        // 1500 x 128 1280 -> 1273, 2048 x 128 2168 -> 2163, 4096 x 32 2037 / 2040)
-        if (GROUP == 2) __builtin_nontemporal_store(bits, place); else *place = bits;
+        // (past the caches, backward and then a product that reads the rows, us, this / that: 300 tokens x 128 heads 122 / 125, 512 x 128
+        // 208 / 207, 1024 x 128 532 / 532, 4096 x 32 1593 / 1609, 3000 x 128 3492 / 3501, 1000 x 64 272 / 269, 40 x 85 x 64 335 / 340)
+        *reinterpret_cast<u32x4*>(query_latent_gradient + target * RANK + column_part * (RANK / PARTS) + 8 * part) =
+            *reinterpret_cast<const u32x4*>(staged);
         if (part < ROPE / 8 / PARTS) {
             *reinterpret_cast<u32x4*>(query_rope_gradient + target * ROPE + column_part * (ROPE / PARTS) + 8 * part) =
                 *reinterpret_cast<const u32x4*>(staged + L::OUT_ROPE);
