@@ -537,9 +537,11 @@ constexpr int STREAM_OUT_PITCH = 2 * HEAD + 16;
 constexpr int STREAM_LDS_BYTES = STREAM_OUT_AT + TILE * STREAM_OUT_PITCH;
 static_assert(2 * STREAM_LDS_BYTES <= 160 * 1024, "two workgroups fit a compute unit");
 
-// BYPASS: rows that fill the caches by themselves are read around them.  As usual / so: 4096 x 128 118.8 / 110 us, 1024 x 128
-// 33.7 / 33.2 and, behind the forward that wrote the rows, the layer 232 / 230.6; 1000 x 16 9.5 / 9.9, 2 x 300 x 32 40.7 / 41.0.
-constexpr long long BYPASS_BYTES = 128LL << 20;
+// BYPASS: rows that do not all survive in the caches behind the forward that wrote them are read around them.  Forward and
+// un-absorb, us, as usual / so: 600 tokens x 128 heads (79 MB) 108.5 / 109.2, 1200 x 64 (79) 149.2 / 150.1, 660 x 128 (87)
+// 123.2 / 122.5, 4 x 340 x 64 (89) 99.3 / 99.8, 700 x 128 (92) 133.9 / 131.0, 16 x 90 x 64 (94) 95.2 / 89.1, 768 x 128 (101) 151.3 / 145.9,
+// 3200 x 32 (105) 371.6 / 364.9, 1024 x 128 (134) 223.9 / 223.2, 2048 x 128 683 / 678.  4096 x 128 alone 125.5 / 117.6.
+constexpr long long BYPASS_BYTES = 84LL << 20;
 
 template <bool BYPASS>
 __global__ __launch_bounds__(THREADS, 2) void mla_unabsorb_output_stream_kernel(bf16_t* __restrict__ y,
