@@ -85,6 +85,20 @@ __device__ __forceinline__ void clear(f32x16& value) {
     for (int i = 0; i < 16; ++i) value[i] = 0.f;
 }
 
+// dQ, dK and dV that do not fit the caches together leave past them: the caller's next operators, the backward of the rotary
+// embedding and of the projections, find nothing of them there anyway.  Backward and these operators, us, in / past the caches:
+// 192 / 128 columns 1000 tokens x 16 heads (16 MB) 95.0 / 99.9, 1000 x 32 143.4 / 145.8, 1400 x 64 (92 MB) 358 / 361, 1500 x 64 (98)
+// 386 / 390, 1600 x 64 (105) 402 / 398, 4 x 850 x 32 (111) 311 / 299, 8 x 850 x 16 (111) 266 / 267, 1800 x 64 (118) 479 / 462, 2048 x 64
+// 576 / 560, 3000 x 128 1777 / 1751; 64 columns 8 x 1024 x 32 on 8 (50 MB) 289 / 293, 8 x 1408 x 32 on 8 (69) 420 / 421,
+// 3520 x 64 (87) 606 / 596, 4096 x 64 (101) 801 / 765; 128 columns 2 x 3008 x 32 on 8 (74) 583 / 572, 2048 x 64 (101) 407 / 404.
+constexpr long long GRADIENT_STREAM_BYTES = 96LL << 20;
+
+template <bool STREAM>   // (a branch at the stores instead: 300 tokens x 8 heads 27.6 -> 27.9 us)
+__device__ __forceinline__ void store_gradient(bf16_t* place, const u32x4& bits) {
+    if constexpr (STREAM) __builtin_nontemporal_store(bits, reinterpret_cast<u32x4*>(place));
+    else *reinterpret_cast<u32x4*>(place) = bits;
+}
+
 // ---- statistics ---------------------------------------------------------------
 
 // One group of DV / 8 lanes per (b, s, h) row of the sequence padded to whole query tiles.  STREAMING: many rows of 128 columns, which
@@ -218,7 +232,7 @@ struct KeyValueGradConfig {
     static_assert(LDS_BYTES <= 160 * 1024, "stages must fit the LDS");
 };
 
-template <int DQK, int DV>
+template <int DQK, int DV, bool STREAM>
 __global__ __launch_bounds__(KV_THREADS) void attention_key_value_gradient_kernel(
     bf16_t* __restrict__ key_gradient, bf16_t* __restrict__ value_gradient, unsigned char* __restrict__ ds_blocks,
     float* __restrict__ partial_sums, const float* __restrict__ statistics, const bf16_t* __restrict__ output_gradient,
@@ -511,9 +525,7 @@ __global__ __launch_bounds__(KV_THREADS) void attention_key_value_gradient_kerne
             const int chunk = position % (DV / 8);
             if (group_k0 + row < S) {
                 const u32x4 bits = *reinterpret_cast<const u32x4*>(dv_lds + row * C::DV_PITCH + 16 * chunk);
-                // whole lines that nothing reads next, here and for dK and dQ: past the caches (4096 tokens x 128 heads, 192 / 128
-                // columns, forward and backward 2856 -> 2835 us, 1500 x 64 265.5 -> 263.0)
-                __builtin_nontemporal_store(bits, reinterpret_cast<u32x4*>(dv_base + (size_t)(group_k0 + row) * v_stride + 8 * chunk));
+                store_gradient<STREAM>(dv_base + (size_t)(group_k0 + row) * v_stride + 8 * chunk, bits);
             }
         }
     } else {
@@ -647,7 +659,7 @@ __global__ __launch_bounds__(KV_THREADS) void attention_key_value_gradient_kerne
             const int chunk = position % (DQK / 8);
             if (group_k0 + row < S) {
                 const u32x4 bits = *reinterpret_cast<const u32x4*>(dk_lds + row * C::DK_PITCH + 16 * chunk);
-                __builtin_nontemporal_store(bits, reinterpret_cast<u32x4*>(dk_base + (size_t)(group_k0 + row) * qk_stride + 8 * chunk));
+                store_gradient<STREAM>(dk_base + (size_t)(group_k0 + row) * qk_stride + 8 * chunk, bits);
             }
         }
     }
@@ -738,7 +750,7 @@ __device__ __forceinline__ void add_partial_sums(const PartialSums& partial, int
     *reinterpret_cast<u32x2*>(target) = packed;
 }
 
-template <int DQK, int DV>
+template <int DQK, int DV, bool STREAM>
 __global__ __launch_bounds__(DQ_THREADS) void attention_query_gradient_kernel(
     bf16_t* __restrict__ query_gradient, const unsigned char* __restrict__ ds_blocks, const bf16_t* __restrict__ key,
     int sequence_length, int heads, int kv_heads, int query_blocks, int key_blocks, int query_tiles, int first_pair,
@@ -967,7 +979,7 @@ __global__ __launch_bounds__(DQ_THREADS) void attention_query_gradient_kernel(
             const int q_row = 2 * jb * QTILE + r;
             if (q_row < S) {
                 const u32x4 bits = *reinterpret_cast<const u32x4*>(lds + (size_t)r * ROW_PITCH + 16 * chunk);
-                __builtin_nontemporal_store(bits, reinterpret_cast<u32x4*>(dq_base + (size_t)q_row * q_stride + 8 * chunk));
+                store_gradient<STREAM>(dq_base + (size_t)q_row * q_stride + 8 * chunk, bits);
             }
         }
     }
@@ -1067,8 +1079,10 @@ void launch_backward(bf16_t* query_gradient, bf16_t* key_gradient, bf16_t* value
     float* partial_sums = workspace + shape.statistics_floats + shape.ds_floats;
     static hip_common::OncePerDevice prepared;
     prepared.run([] {
-        raise_lds_limit(attention_key_value_gradient_kernel<DQK, DV>, KC::LDS_BYTES);
-        raise_lds_limit(attention_query_gradient_kernel<DQK, DV>, QC::LDS_BYTES);
+        raise_lds_limit(attention_key_value_gradient_kernel<DQK, DV, false>, KC::LDS_BYTES);
+        raise_lds_limit(attention_key_value_gradient_kernel<DQK, DV, true>, KC::LDS_BYTES);
+        raise_lds_limit(attention_query_gradient_kernel<DQK, DV, false>, QC::LDS_BYTES);
+        raise_lds_limit(attention_query_gradient_kernel<DQK, DV, true>, QC::LDS_BYTES);
     });
     auto statistics_kernel = attention_backward_statistics_kernel<DV, false>;
     if constexpr (DV == 128) {
@@ -1080,9 +1094,15 @@ void launch_backward(bf16_t* query_gradient, bf16_t* key_gradient, bf16_t* value
                        stream, statistics, output_gradient, output, logsumexp, batch_size, sequence_length, heads,
                        shape.query_tiles);
     HIP_CHECK(hipGetLastError());
+    const long long gradient_bytes = 2LL * batch_size * sequence_length * ((long long)heads * DQK + (long long)kv_heads * (DQK + DV));
+    const bool stream_gradients = gradient_bytes >= GRADIENT_STREAM_BYTES;
+    const auto key_value_kernel = stream_gradients ? attention_key_value_gradient_kernel<DQK, DV, true>
+                                                   : attention_key_value_gradient_kernel<DQK, DV, false>;
+    const auto query_kernel = stream_gradients ? attention_query_gradient_kernel<DQK, DV, true>
+                                               : attention_query_gradient_kernel<DQK, DV, false>;
     for (long long first = 0; first < shape.pairs; first += shape.pairs_per_launch) {
         const long long count = std::min(shape.pairs_per_launch, shape.pairs - first);
-        hipLaunchKernelGGL((attention_key_value_gradient_kernel<DQK, DV>), dim3((unsigned)(count * shape.cut.items)),
+        hipLaunchKernelGGL(key_value_kernel, dim3((unsigned)(count * shape.cut.items)),
                            dim3(KV_THREADS), KC::LDS_BYTES, stream, key_gradient, value_gradient, ds_blocks, partial_sums,
                            statistics, output_gradient, query, key, value, sequence_length, heads, kv_heads,
                            shape.key_blocks, shape.query_tiles, (int)first, shape.cut.part_steps, shape.cut.items, scale);
@@ -1093,8 +1113,7 @@ void launch_backward(bf16_t* query_gradient, bf16_t* key_gradient, bf16_t* value
         const long long workgroups = count * shape.sharing * shape.query_blocks;
         const PartialSums partial = {partial_sums, key_gradient, value_gradient, shape.cut.items, shape.cut.cut_blocks,
                                      shape.cut.part_steps, (int)first};
-        hipLaunchKernelGGL((attention_query_gradient_kernel<DQK, DV>),
-                           dim3((unsigned)(workgroups + count * shape.cut.cut_blocks * PIECES)), dim3(DQ_THREADS),
+        hipLaunchKernelGGL(query_kernel, dim3((unsigned)(workgroups + count * shape.cut.cut_blocks * PIECES)), dim3(DQ_THREADS),
                            QC::LDS_BYTES, stream, query_gradient, ds_blocks, key, sequence_length, heads, kv_heads,
                            shape.query_blocks, shape.key_blocks, shape.query_tiles, (int)(first * shape.sharing),
                            (int)workgroups, scale, partial);
