@@ -45,9 +45,13 @@ def test_decode_row_blocks(cuda, batch, heads, splits):
     assert_close_lse("LSE", lse, expected_lse)
 
 
-@pytest.mark.parametrize("batch,heads", [(2, 40), (14, 64), (28, 128)])   # 32, 64 and 128 rows
-def test_decode_raised_reference(cuda, batch, heads):
+# 32, 64 and 128 rows; 128 rows over pages that hold no whole units of 32 keys, which have a kernel of their own
+@pytest.mark.parametrize("batch,heads,page_size,rows", [(2, 40, 64, 32), (14, 64, 64, 32), (24, 128, 64, 64),
+                                                        (28, 128, 64, 128), (28, 128, 48, 128), (28, 97, 16, 128)])
+def test_decode_raised_reference(cuda, batch, heads, page_size, rows):
     """Keys late in the stream aligned with one head of each row group: scores thousands above the first keys'."""
+    units = torch.cuda.get_device_properties(cuda).multi_processor_count
+    assert {0: 128, 1: 32, 2: 64}[rules().call_rows(batch, heads, 2, page_size, units)] == rows
     tokens = 420
     g = torch.Generator().manual_seed(31)
     query = torch.randn(batch, 1, heads, 576, generator=g).bfloat16()
@@ -55,8 +59,8 @@ def test_decode_raised_reference(cuda, batch, heads):
     for first, last, head, factor in [(70, 72, 0, 1.0), (200, 201, heads - 1, 2.0), (300, 340, heads // 2, 4.0)]:
         cache[:, first:last] = (query[:, 0, head:head + 1].float() * factor).bfloat16()
     lengths = torch.tensor([tokens - 11 * (b % 9) for b in range(batch)], dtype=torch.int32)
-    paged, table = configs.pack_cache(cache, 64)
-    announce("decode raised reference", dict(B=batch, H=heads))
+    paged, table = configs.pack_cache(cache, page_size)
+    announce("decode raised reference", dict(B=batch, H=heads, page=page_size))
     out, lse = ops.mla_decode(query.to(cuda), paged.to(cuda), table.to(cuda), lengths.to(cuda), 1.0, splits=2)
     expected, expected_lse = oracle.mla_decode_unrounded(query, cache, lengths, 1.0)
     assert expected_lse.max() > 500
