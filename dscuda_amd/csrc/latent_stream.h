@@ -92,6 +92,14 @@ struct UnitCursor {
         }
     }
 
+    // Pages that do not hold whole units: every key finds its own page when the unit is requested.
+    __device__ __forceinline__ void init_key_by_key(int first_unit) {
+        paged = true;
+        contiguous = split = false;
+        unit = __builtin_amdgcn_readfirstlane(first_unit);
+        page = within = units_per_page = first_page = last_page = ids = 0;
+    }
+
     __device__ __forceinline__ UnitSource next(unsigned char* lds, const KeyStream& keys, int last_token, int wave,
                                                int unit_end) {
         UnitSource source;
@@ -172,22 +180,10 @@ __device__ __forceinline__ void issue_split_load(const UnitSource& source, const
     direct_load_16(part + bytes, source.lds_base + I * 1024);
 }
 
-// All nine loads of a unit at once: the first units of a walk, and every unit of the
-// general form (per-lane page lookup, or latent and rope parts in tensors of their own).
-__device__ __forceinline__ void issue_unit(const UnitSource& source, const FullUnitOffsets& offsets, const KeyStream& keys,
-                                           int wave) {
+// All nine loads of a unit whose rows are found one by one: a page lookup per lane, or strides beyond those of `split`.
+__device__ __forceinline__ void issue_unit_key_by_key(const UnitSource& source, const KeyStream& keys, bool paged, int wave) {
     if (!source.enabled) return;
     const int lane = fresh_lane_id();
-    if (source.contiguous) {
-#pragma unroll
-        for (int i = 0; i < UNIT_LOADS; ++i) issue_unit_load(source, offsets, wave, i, lane);
-        return;
-    }
-    if (source.split) {
-        unrolled<0, UNIT_LOADS>([&](auto tag) { issue_split_load<decltype(tag)::value>(source, keys, wave, lane); });
-        return;
-    }
-    const bool paged = keys.block_table != nullptr;
 #pragma unroll 1
     for (int i = 0; i < UNIT_LOADS; ++i) {
         const int slot = 64 * i + lane;
@@ -203,6 +199,23 @@ __device__ __forceinline__ void issue_unit(const UnitSource& source, const FullU
                                                  : keys.rope + physical * keys.rope_stride + 8 * (chunk - RANK / 8);
         direct_load_16(address, source.lds_base + i * 1024);
     }
+}
+
+// All nine loads of a unit at once, of any form.
+__device__ __forceinline__ void issue_unit(const UnitSource& source, const FullUnitOffsets& offsets, const KeyStream& keys,
+                                           int wave) {
+    if (!source.enabled) return;
+    const int lane = fresh_lane_id();
+    if (source.contiguous) {
+#pragma unroll
+        for (int i = 0; i < UNIT_LOADS; ++i) issue_unit_load(source, offsets, wave, i, lane);
+        return;
+    }
+    if (source.split) {
+        unrolled<0, UNIT_LOADS>([&](auto tag) { issue_split_load<decltype(tag)::value>(source, keys, wave, lane); });
+        return;
+    }
+    issue_unit_key_by_key(source, keys, keys.block_table != nullptr, wave);
 }
 
 // Per-lane byte offsets of the fragment reads inside a unit (rows 0..31 of 1152 bytes).

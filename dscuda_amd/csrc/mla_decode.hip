@@ -25,7 +25,8 @@
 //
 // Global -> LDS without registers
 //   Units arrive by global_load_lds (16 bytes per lane, a wave instruction
-//   fills 1 KB of consecutive LDS).  With no padding possible inside that 1 KB
+//   fills 1 KB of consecutive LDS), each lane from the page of its own key: the
+//   round trips of these lookups bound the call.  With no padding possible inside that 1 KB
 //   the bank spread comes from a swizzle applied on the global side: the
 //   16-byte chunk c of row r lives at slot 72*r + (c ^ f(r)), f(r) = the three
 //   bits of r>>1 with bits 0 and 2 exchanged.  That makes both the 16-row
@@ -216,9 +217,10 @@ __device__ __forceinline__ void reset(RowState& state) {
 // the key stream is consumed in units of 32 keys and the work of consecutive units is
 // overlapped by hand:
 //
-//     step u:   S(u+1) = K(u+1) Q^T   36 MFMAs, with the softmax of S(u) -> P(u)
+//     step u:   the requests for unit u+3, whose rows are looked up page by page
+//               S(u+1) = K(u+1) Q^T   36 MFMAs, with the softmax of S(u) -> P(u)
 //                                     (exp2, sums, bf16 packing) issued between them
-//               O^T  += V(u)^T P(u)   32 MFMAs, with the requests for unit u+3 between them
+//               O^T  += V(u)^T P(u)   32 MFMAs
 //
 // one stream of 68 MFMAs per unit, each fed by one LDS fragment read through a small
 // register ring that runs a few MFMAs ahead.  The scores of two units are live at a
@@ -299,11 +301,9 @@ template <bool HAS_NEXT>
 __device__ __forceinline__ void unit_step(RowState& state, f32x16& scores, f32x16& next_scores,
                                           const bf16x8 (&qf)[KSTEPS], const UnitReads& reads,
                                           const unsigned char* current, const unsigned char* next, int key0, int tokens,
-                                          float c, const UnitSource& request, const FullUnitOffsets& offsets,
-                                          const KeyStream& keys, int wave) {
+                                          float c, const UnitSource& request, const KeyStream& keys, int wave) {
     constexpr int SCORE_MFMAS = HAS_NEXT ? KSTEPS : 0;
     constexpr int COUNT = SCORE_MFMAS + 2 * DBLOCKS;
-    const int lane = fresh_lane_id();
 
     // fragment I of the stream: the K fragments of the next unit, then the V fragments of this one
     auto fragment = [&](auto tag) -> bf16x8 {
@@ -317,7 +317,7 @@ __device__ __forceinline__ void unit_step(RowState& state, f32x16& scores, f32x1
     bf16x8 ring[STREAM_RING];
     unrolled<0, STREAM_RING>([&](auto tag) { ring[decltype(tag)::value] = fragment(tag); });
 
-    mask_unit_scores(scores, key0, tokens, lane / 32);
+    mask_unit_scores(scores, key0, tokens, fresh_lane_id() / 32);
 
     float unit_max;
     u32x4 probabilities[2];
@@ -363,7 +363,7 @@ __device__ __forceinline__ void unit_step(RowState& state, f32x16& scores, f32x1
     if constexpr (!HAS_NEXT) {
         unrolled<0, 33>(softmax_piece);   // the last unit: no score products to hide it behind
     }
-    if (request.enabled && !request.contiguous) issue_unit(request, offsets, keys, wave);
+    issue_unit_key_by_key(request, keys, true, wave);
 
     unrolled<0, COUNT>([&](auto tag) {
         constexpr int I = decltype(tag)::value;
@@ -382,10 +382,6 @@ __device__ __forceinline__ void unit_step(RowState& state, f32x16& scores, f32x1
         }
         if constexpr (I + STREAM_RING < COUNT) ring[I % STREAM_RING] = fragment(std::integral_constant<int, I + STREAM_RING>{});
         if constexpr (HAS_NEXT && I < 33) softmax_piece(tag);
-        // the requests go between the output MFMAs, which leave more issue slots free than the score MFMAs
-        if constexpr (HAS_NEXT && I >= SCORE_MFMAS && (I - SCORE_MFMAS) % 3 == 1 && (I - SCORE_MFMAS) / 3 < UNIT_LOADS) {
-            if (request.enabled && request.contiguous) issue_unit_load(request, offsets, wave, (I - SCORE_MFMAS) / 3, lane);
-        }
         __builtin_amdgcn_sched_barrier(0);
     });
 }
@@ -405,19 +401,16 @@ __device__ __forceinline__ void walk_units(RowState& state, const bf16_t* query_
     // The first three units and the query rows.  In the middle of a kernel one round trip brings them all.  At the
     // start of the kernel (`cold`) every workgroup asks at once and the answers come at the rate of the memory, not
     // of its latency: then only what the first scores need is asked for first, the rest once that has arrived.
-    // The query rows are asked for before the page ids of the cursor, whose wait then covers both round trips
-    // (the ids are needed before the first unit can be requested; the rows before its scores).
+    // The query rows are asked for before the first unit, whose page lookups then cover both round trips.
     bf16x8 qf[KSTEPS];
     load_query(qf, query_latent_row, query_rope_row, valid, (tid % 64) / 32);
     UnitCursor cursor;
-    cursor.init(keys, unit_begin, last_token);
-    FullUnitOffsets offsets;
-    offsets.init(wave, fresh_lane_id());
-    issue_unit(cursor.next(lds, keys, last_token, wave, unit_end), offsets, keys, wave);
+    cursor.init_key_by_key(unit_begin);
+    issue_unit_key_by_key(cursor.next(lds, keys, last_token, wave, unit_end), keys, true, wave);
     const UnitSource second = cursor.next(lds, keys, last_token, wave, unit_end);
     const UnitSource third = cursor.next(lds, keys, last_token, wave, unit_end);
-    if (!cold) issue_unit(second, offsets, keys, wave);
-    if (!cold) issue_unit(third, offsets, keys, wave);
+    if (!cold) issue_unit_key_by_key(second, keys, true, wave);
+    if (!cold) issue_unit_key_by_key(third, keys, true, wave);
     reset(state);
     UnitReads reads;
     reads.init(fresh_lane_id());
@@ -426,8 +419,8 @@ __device__ __forceinline__ void walk_units(RowState& state, const bf16_t* query_
     wait_vector_memory<0>();
     workgroup_barrier();
     if (cold) {
-        issue_unit(second, offsets, keys, wave);
-        issue_unit(third, offsets, keys, wave);
+        issue_unit_key_by_key(second, keys, true, wave);
+        issue_unit_key_by_key(third, keys, true, wave);
     }
     // scores of the first unit, and the reference every exponential of this walk is taken against
     f32x16 scores_a, scores_b;
@@ -454,13 +447,13 @@ __device__ __forceinline__ void walk_units(RowState& state, const bf16_t* query_
     for (; unit + 1 < unit_end; ++unit) {
         synchronise(unit);
         unit_step<true>(state, scores_a, scores_b, qf, reads, slot_of(unit), slot_of(unit + 1), unit * UNIT, tokens, c,
-                        cursor.next(lds, keys, last_token, wave, unit_end), offsets, keys, wave);
+                        cursor.next(lds, keys, last_token, wave, unit_end), keys, wave);
         // the next unit's scores take the place of this unit's (eight moves against a stream of 68 MFMAs)
         move_scores(scores_a, scores_b);
     }
     UnitSource nothing = {};
     unit_step<false>(state, scores_a, scores_b, qf, reads, slot_of(unit), slot_of(unit), unit * UNIT, tokens, c, nothing,
-                     offsets, keys, wave);
+                     keys, wave);
     workgroup_barrier();   // the slots are free: the caller stages its results through them
 }
 
@@ -841,14 +834,15 @@ void mla_decode_dispatch(bf16_t* output, float* logsumexp, const bf16_t* query, 
                                  stream);
         return;
     }
-    // a plan built for the other form counts other ranges
-    const bool recut = !own_plan && index_math::decode_form(batch_size, heads, splits, compute_units(), RANK).row_blocks != 0;
     const int padded_rows = (heads + 31) / 32 * 32;
-    // pages that do not hold whole units are looked up key by key, which only the four-wave kernel does
+    // A plan built for the other form counts other ranges.  Pages that hold whole units leave a call the form of its plan
+    // (decode_form_of_call); the others are looked up key by key, which of the 128-row kernels only the four-wave one does.
+    bool recut = false;
     if (page_size % UNIT == 0) {
         mla_wide_decode_launch(output, logsumexp, query, paged_kv_cache, block_table, cache_lengths, workspace, plan,
                                batch_size, heads, page_size, pages_per_sequence, layout, own_plan, scale, stream);
     } else {
+        recut = !own_plan && index_math::decode_form(batch_size, heads, splits, compute_units(), RANK).row_blocks != 0;
         static hip_common::OncePerDevice prepared;
         prepared.run([] { allow_large_lds(mla_decode_split_kernel); });
         const dim3 grid(layout.workgroups, layout.head_groups);
