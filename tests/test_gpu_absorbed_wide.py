@@ -64,9 +64,29 @@ def test_items_walked_again(cuda):
 
 
 def test_scores_too_large_for_their_own_rounding(cuda):
-    """Scores of 1e30: their distance from their rounded maximum is beyond any limit, a second walk is the last all the
-    same.  What comes out is not asserted."""
-    ql, qr, c, kr, _ = configs.mla_absorbed_inputs(1, 260, 128)
-    announce("mla_forward, huge scores", dict(T=260, H=128))
-    ops.mla_forward((ql * 1e15).to(cuda), qr.to(cuda), (c * 1e15).to(cuda), kr.to(cuda), 1.0)
+    """Scores of 1e30 in some rows of some items: their distance from their rounded maximum is beyond any limit, a second walk
+    is the last all the same.  What comes out for these rows is not asserted; all other rows, of the items walked twice and of
+    those before and after them, are as ever, and every row is written."""
+    tokens, heads = 400, 300
+    ql, qr, c, kr, scale = configs.mla_absorbed_inputs(1, tokens, heads)
+    huge = [(30, 0), (31, 299), (200, 7), (200, 130), (399, 150)]
+    for token, head in huge:
+        ql[0, token, head] *= 1e30
+    announce("mla_forward, huge scores", dict(T=tokens, H=heads))
+    on_gpu = [x.to(cuda) for x in (ql, qr, c, kr)]
+    untouched = -77.0
+    runs = []
+    for _ in range(2):
+        out, lse = torch.full_like(on_gpu[0], untouched), torch.full((1, heads, tokens), untouched, device=cuda)
+        ops.mla_forward(*on_gpu, scale, out=out, lse=lse)
+        runs.append((out.view(torch.int16), lse.view(torch.int32)))
     torch.cuda.synchronize()
+    assert torch.equal(runs[0][0], runs[1][0]) and torch.equal(runs[0][1], runs[1][1])
+    assert not (out == untouched).all(-1).any() and not (lse == untouched).any()
+    ordinary = torch.ones(1, tokens, heads, dtype=torch.bool)
+    for token, head in huge:
+        ordinary[0, token, head] = False
+        ql[0, token, head] = 0
+    expected, expected_lse = oracle.mla_forward_unrounded(ql, qr, c, kr, scale, oracle.causal_mask(tokens))
+    assert_close_bf16("O", out.cpu()[ordinary], expected[ordinary], max_abs=8e-3)
+    assert_close_lse("LSE", lse.cpu().transpose(1, 2)[ordinary], expected_lse.transpose(1, 2)[ordinary], tol=1e-4)

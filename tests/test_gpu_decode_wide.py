@@ -45,10 +45,11 @@ def test_decode(cuda, batch, heads, page_size, splits, lengths):
     query, cache, paged, table, lengths_t = _inputs(batch, heads, page_size, lengths, seed=batch + heads)
     scale = configs.c_float(576 ** -0.5)
     announce("mla_decode", dict(B=batch, H=heads, page=page_size, splits=splits))
-    on_gpu = [x.to(cuda) for x in (query, paged, table, lengths_t)]
-    # a table entry past the last page with a visible token is never read: such entries hold what no pool has
+    # a table entry past the last page with a visible token is never used: such entries name a page of NaNs
+    paged = torch.cat([paged, torch.full_like(paged[:1], float("nan"))])
     for row, length in enumerate(lengths_t.tolist()):
-        on_gpu[2][row, (length + page_size - 1) // page_size:] = 0x3fffffff
+        table[row, (length + page_size - 1) // page_size:] = paged.shape[0] - 1
+    on_gpu = [x.to(cuda) for x in (query, paged, table, lengths_t)]
     # an entry of the plan that the call does not write for itself stands for no sequence
     workspace = ops.mla_decode_workspace(batch, heads, splits).zero_()
     out, lse = ops.mla_decode(*on_gpu, scale, splits=splits, workspace=workspace)
