@@ -108,15 +108,19 @@ __device__ __forceinline__ int chunk_of_group(int q) {
     return (q >> 1) ^ (3 * (q & 1));   // 0, 3, 1, 2
 }
 
+// The value of lane l ^ 16, by a swizzle whose pattern is a constant (0x401f: exclusive or with 16 within 32 lanes): __shfl_xor
+// computes with the lane's number, which the decode then kept in scratch.
+__device__ __forceinline__ float of_lane_xor_16(float value) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, value), 0x401f));
+}
+
 // over the lanes l, l ^ 16, l ^ 32, l ^ 48
 __device__ __forceinline__ float wide_quarter_max(float value) {
-    value = fmaxf(value, __shfl_xor(value, 16));
-    return half_wave_max(value);
+    return half_wave_max(fmaxf(value, of_lane_xor_16(value)));
 }
 
 __device__ __forceinline__ float wide_quarter_sum(float value) {
-    value += __shfl_xor(value, 16);
-    return half_wave_sum(value);
+    return half_wave_sum(value + of_lane_xor_16(value));
 }
 
 // ---- what a workgroup walks ---------------------------------------------------------------------------------------

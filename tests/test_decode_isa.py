@@ -146,3 +146,19 @@ def test_no_access_to_score_accumulators_in_flight(tmp_path):
     report = "\n".join(f"{kernel} line {number}: `{line}` touches v[{low}:{high}] in flight"
                        for kernel, number, line, (low, high) in violations[:20])
     assert not violations, report
+
+
+def test_streams_of_requests_use_no_scratch(tmp_path):
+    """A reload from scratch waits for every request of the stream that is on its way (csrc/mla_wide.hip)."""
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not Path(hipcc).exists():
+        pytest.skip("no hipcc")
+    from dscuda_amd.build import COMMON_FLAGS, CSRC
+
+    target = tmp_path / "mla_wide.s"
+    flags = [flag for flag in COMMON_FLAGS if flag != "-fPIC"]
+    result = subprocess.run([hipcc, *flags, "--cuda-device-only", "-S", str(CSRC / "mla_wide.hip"), "-o", str(target)],
+                            capture_output=True, text=True, timeout=900)
+    assert result.returncode == 0, result.stderr[-3000:]
+    sizes = re.findall(r"\.private_segment_fixed_size:\s*(\d+)", target.read_text())
+    assert sizes == ["0", "0"]
