@@ -426,6 +426,12 @@ DSCUDA_HOST_DEVICE inline unsigned forward_index(unsigned round, unsigned workgr
     return round * workgroups + (round & 1 ? workgroups - 1 - workgroup : workgroup);
 }
 
+// The workgroup's index if every XCD took a run of consecutive ones; they go to the eight XCDs round-robin by linear id.
+DSCUDA_HOST_DEVICE inline unsigned run_index(unsigned workgroup, unsigned workgroups) {
+    const unsigned xcd = workgroup % 8, more = workgroups % 8;   // the first `more` XCDs have one more
+    return xcd * (workgroups / 8) + (xcd < more ? xcd : more) + workgroup / 8;
+}
+
 // Items (batch, query head, query block), numbered so that what runs at one time shares keys and ends together.
 // Workgroups go to the XCDs round-robin by linear id and every XCD has an L2 of its own, so the query heads that read
 // one key/value head stay on one XCD; with too few key/value heads for that, query heads are dealt to the XCDs one by

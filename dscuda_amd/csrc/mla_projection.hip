@@ -524,7 +524,7 @@ __global__ __launch_bounds__(THREADS, 2) void mla_absorb_query_slice_kernel(bf16
 
 // out = o_latent W_UV^T as a stream of token tiles: a wave holds 32 of the head's 128 weight rows in 128 registers, the four
 // waves of a workgroup read each tile of 32 tokens from LDS, whole rows of 1 KB brought there by global_load_lds two tiles
-// ahead, a workgroup a compute unit (its LDS admits a second one, for what does not come out even).  blockIdx.x =
+// ahead, a workgroup a compute unit (its LDS admits a second one, for what does not come out even).  Workgroup index =
 // chunk * heads + head.  Bound by the rows read.  mla_unabsorb_output_kernel, each of whose waves fetches a token's row 32
 // bytes at a time and keeps 128 KB of weight in LDS, -> here, us, inputs that are not in the caches: 1024 tokens x 128 heads
 // 41.1 -> 33.9 (185 MB, 5.5 TB/s), 4096 x 128 135 -> 125, 512 x 128 26.2 -> 19.9, 300 x 128 22.4 -> 14.5, 200 x 300 36 -> 27,
@@ -543,6 +543,13 @@ static_assert(2 * STREAM_LDS_BYTES <= 160 * 1024, "two workgroups fit a compute 
 // 3200 x 32 (105) 371.6 / 364.9, 1024 x 128 (134) 223.9 / 223.2, 2048 x 128 683 / 678.  4096 x 128 alone 125.5 / 117.6.
 constexpr long long BYPASS_BYTES = 84LL << 20;
 
+// Up to so many heads an XCD takes a run of indices, that is all heads of its tokens.  Dealt one by one, with 4, 8 or 16 heads an XCD
+// has the same one or two heads of all tokens, 1 KB of every 4 or 8.  us, whole weights in LDS / dealt / runs: 4000 tokens x 4 heads
+// 10.2 / 11.4 / 9.1, 8000 x 8 25.5 / 26.1 / 22.3, 16000 x 8 42.1 / 41.3 / 33.3, 2000 x 16 15.6 / 16.9 / 14.1, 8192 x 16 41.9 / 43.8 /
+// 34.0.  More heads share their weights in an L2 when dealt: 1000 x 24 13.3 / 11.3 / 11.6, 1000 x 48 23.7 / 17.6 / 18.3, 300 x 64 12.4 /
+// 10.3 / 12.0, 4096 x 128 135.7 / 117.8 / 126.3; 1000 x 32 equal, 4096 x 32 43.5 / 38.0 / 35.2.
+constexpr int RUN_HEADS = 16;
+
 template <bool BYPASS>
 __global__ __launch_bounds__(THREADS, 2) void mla_unabsorb_output_stream_kernel(bf16_t* __restrict__ y,
                                                                                 const bf16_t* __restrict__ x,
@@ -558,8 +565,9 @@ __global__ __launch_bounds__(THREADS, 2) void mla_unabsorb_output_stream_kernel(
     const int lane = tid % 64;
     const int lq = lane % 32;
     const int g = lane / 32;
-    const int head = blockIdx.x % heads;
-    const long long first = blockIdx.x / heads * tokens_per_workgroup;
+    const unsigned index = heads <= RUN_HEADS ? index_math::run_index(blockIdx.x, gridDim.x) : blockIdx.x;
+    const int head = index % (unsigned)heads;
+    const long long first = index / (unsigned)heads * tokens_per_workgroup;
     const int tiles = (int)((min(tokens_per_workgroup, tokens - first) + TILE - 1) / TILE);
     const bf16_t* x_head = x + head * strides.x_head;
     const unsigned lds_base = lds_offset_of(lds);

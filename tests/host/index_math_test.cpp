@@ -778,6 +778,19 @@ void check_decode_layout() {
 
 // ---- the plan a decode kernel leaves for its merge: every entry of the prefix, also where the batch is as large as the
 // workgroup of 256 or 512 threads, and nothing behind it
+void check_run_index() {
+    for (unsigned workgroups = 1; workgroups < 600; ++workgroups) {
+        std::vector<int> seen(workgroups, 0);
+        for (unsigned w = 0; w < workgroups; ++w) {
+            const unsigned index = run_index(w, workgroups);
+            EXPECT(index < workgroups, "%u of %u: %u", w, workgroups, index);
+            if (index >= workgroups) continue;
+            EXPECT(seen[index]++ == 0, "%u of %u: %u twice", w, workgroups, index);
+            if (w >= 8) EXPECT(index == run_index(w - 8, workgroups) + 1, "%u of %u", w, workgroups);
+        }
+    }
+}
+
 void check_leave_prefix() {
     for (int threads : {256, 512}) {
         for (int batch : {1, 64, 65, 255, 256}) {
@@ -1050,6 +1063,7 @@ int main() {
     check_forward_deal();
     check_decode_ranges();
     check_decode_layout();
+    check_run_index();
     check_leave_prefix();
     check_rows_apart();
     if (failures) {

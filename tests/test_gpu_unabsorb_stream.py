@@ -12,7 +12,8 @@ from parity import announce, assert_close_bf16
 # most a workgroup has: one tile; two, the last of one token; three; 33 tiles; chunks of two tiles and a last one of one;
 # two rounds of heads
 @pytest.mark.gpu
-@pytest.mark.parametrize("tokens,heads", [(32, 129), (33, 150), (96, 200), (65, 256), (1037, 200), (1000, 16), (1025, 33), (2049, 5), (70, 300), (129, 1)])
+@pytest.mark.parametrize("tokens,heads", [(32, 129), (33, 150), (96, 200), (65, 256), (1037, 200), (1000, 16), (1025, 33), (2049, 5), (70, 300), (129, 1),
+                                          (4001, 4), (3000, 3), (2200, 16), (2200, 17)])   # runs of an XCD, of unequal length; none
 def test_unabsorb_output(cuda, tokens, heads):
     g = torch.Generator().manual_seed(tokens + heads)
     wkv_b = (torch.randn(heads, 256, 512, generator=g) * 0.06).bfloat16()
