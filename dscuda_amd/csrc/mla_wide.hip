@@ -39,14 +39,18 @@
 // What bounds the decode
 //   64 sequences of 1024..8192 tokens, 128 heads: 13 us until the loop (plan, block table, query rows and the first units of
 //   all workgroups at once), 44 units in 80 us, 6 us of parts stored.  1.83 us a unit are 4.9 TB/s and 1.25 PFLOP/s,
-//   what the power limit leaves: 1.55 with a zero cache and query, 1.43 with its rows in the L2s as well.  So the four waves
-//   of mla_decode_split_kernel come to the same there (119 / 119 us), and cutting the list by units or counting fewer
-//   positions for a segment gains nothing.  Short sequences, whose start and end count, are faster here: 64 x 200..1000
-//   tokens 39.4 -> 36.6 us, 64 x 100..200 31.3 -> 28.8, 64 x 512..4096 64.4 / 64.2, 32 x 1024..8192 72.9 / 73.2.
+//   what the power limit leaves: 1.55 with a zero cache and query, 1.43 with its rows in the L2s as well.  So four waves
+//   (mla_decode_split_kernel when it took such pages) come to nearly the same there, and cutting the list by units or counting
+//   fewer positions for a segment gains nothing.  us, four waves / here, 128 heads: 64 x 1024..8192 tokens 116.9 / 116.3,
+//   32 x 1024..8192 76.3 / 74.4, 64 x 512..4096 66.7 / 65.6; short sequences, whose start and end count, 64 x 200..1000 37.6 / 35.0,
+//   64 x 100..200 30.1 / 27.1, 300 x 300..900 91.8 / 87.3; but 180 to 257 x 300..900, a sequence or two a workgroup, 75 / 76.6, and long
+//   sequences in one piece (one split) 64 x 1024..8192 243 / 249.
 //
 // Softmax reference
-//   Exponentials are taken against a fixed reference, the maximum of the row's first unit plus 2^40.  A row whose scores
-//   outrun it by more than 2^80 (next to never) has its item walked a second time, against the maxima found.
+//   Exponentials are taken against a fixed reference, the maximum of the row's first unit plus 40 in the log2 domain.  A row
+//   whose scores outrun that by more than 80 (120 above its first 32 keys: next to never) has its item walked a second time,
+//   against the maxima found.  That is what it costs: with such a row in every block of the later half 2048 tokens x 128 heads take
+//   916 us instead of 549; four waves, which scaled their sums in place, took 609 either way.
 #include "attn_kernels.h"
 #include "hip_common.h"
 #include "index_math.h"
