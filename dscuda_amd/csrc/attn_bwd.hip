@@ -91,6 +91,11 @@ __device__ __forceinline__ void clear(f32x16& value) {
 // 386 / 390, 1600 x 64 (105) 402 / 398, 4 x 850 x 32 (111) 311 / 299, 8 x 850 x 16 (111) 266 / 267, 1800 x 64 (118) 479 / 462, 2048 x 64
 // 576 / 560, 3000 x 128 1777 / 1751; 64 columns 8 x 1024 x 32 on 8 (50 MB) 289 / 293, 8 x 1408 x 32 on 8 (69) 420 / 421,
 // 3520 x 64 (87) 606 / 596, 4096 x 64 (101) 801 / 765; 128 columns 2 x 3008 x 32 on 8 (74) 583 / 572, 2048 x 64 (101) 407 / 404.
+// dK and dV of 192 / 128 columns leave past them at any size: the dQ pass comes between them and their readers, and it starts
+// earlier so.  The call / call and readers, in / past the caches: 3 x 240 tokens x 16 heads 27.0, 82.0 / 26.5, 81.9, 3 x 298 x 32
+// 44.5, 124.8 / 43.0, 123.6, 4 x 400 x 16 38.8, 96.5 / 37.5, 97.2, 1000 x 32 61.7, 142.5 / 60.8, 141.2.  Not those of the other
+// geometries, whose readers gain more than the call loses: 16 x 256 x 16 of 64 35.6, 70.3 / 34.8, 73.4, 2 x 1024 x 32 on 8 of 128 86.0,
+// 126.7 / 85.8, 131.6, 8 x 1024 x 32 on 8 of 64 241.1, 287.4 / 240.6, 290.3.
 constexpr long long GRADIENT_STREAM_BYTES = 96LL << 20;
 
 template <bool STREAM>   // (a branch at the stores instead: 300 tokens x 8 heads 27.6 -> 27.9 us)
@@ -1077,9 +1082,10 @@ void launch_backward(bf16_t* query_gradient, bf16_t* key_gradient, bf16_t* value
     float* statistics = workspace;
     unsigned char* ds_blocks = reinterpret_cast<unsigned char*>(workspace + shape.statistics_floats);
     float* partial_sums = workspace + shape.statistics_floats + shape.ds_floats;
+    constexpr bool ALWAYS = DQK != DV;   // dK and dV leave past the caches
     static hip_common::OncePerDevice prepared;
     prepared.run([] {
-        raise_lds_limit(attention_key_value_gradient_kernel<DQK, DV, false>, KC::LDS_BYTES);
+        if (!ALWAYS) raise_lds_limit(attention_key_value_gradient_kernel<DQK, DV, ALWAYS>, KC::LDS_BYTES);
         raise_lds_limit(attention_key_value_gradient_kernel<DQK, DV, true>, KC::LDS_BYTES);
         raise_lds_limit(attention_query_gradient_kernel<DQK, DV, false>, QC::LDS_BYTES);
         raise_lds_limit(attention_query_gradient_kernel<DQK, DV, true>, QC::LDS_BYTES);
@@ -1097,7 +1103,7 @@ void launch_backward(bf16_t* query_gradient, bf16_t* key_gradient, bf16_t* value
     const long long gradient_bytes = 2LL * batch_size * sequence_length * ((long long)heads * DQK + (long long)kv_heads * (DQK + DV));
     const bool stream_gradients = gradient_bytes >= GRADIENT_STREAM_BYTES;
     const auto key_value_kernel = stream_gradients ? attention_key_value_gradient_kernel<DQK, DV, true>
-                                                   : attention_key_value_gradient_kernel<DQK, DV, false>;
+                                                   : attention_key_value_gradient_kernel<DQK, DV, ALWAYS>;
     const auto query_kernel = stream_gradients ? attention_query_gradient_kernel<DQK, DV, true>
                                                : attention_query_gradient_kernel<DQK, DV, false>;
     for (long long first = 0; first < shape.pairs; first += shape.pairs_per_launch) {
