@@ -17,8 +17,8 @@
 //   waves 4..7 (on the same SIMDs) the scores, so that one's exponentials run beside the other's MFMAs; one barrier ends
 //   the step.  With four waves of 32 rows each, 512 registers a wave and one wave a SIMD, a wave's scores, exponentials,
 //   LDS reads and products queue up behind each other: a step takes 3800 to 4100 cycles there and 3200 here, of which
-//   2176 are MFMAs (forward in us, four waves -> here, 128 heads: 1024 tokens 176 -> 140, 2048 583 -> 508, 4096 2110 -> 1880;
-//   3 x 700 x 33 87 -> 66, 40 x 130 x 16 57 -> 42, 7 x 257 x 128 167 -> 123).
+//   2176 are MFMAs (forward in us, four waves -> here, 128 heads: 1024 tokens 176 -> 153, 2048 590 -> 519, 4096 2129 -> 1916;
+//   3 x 700 x 33 86 -> 66, 40 x 130 x 16 57 -> 39, 7 x 257 x 128 169 -> 139).
 //
 // The stream runs on over the ends of items
 //   A workgroup takes several items (blocks of 128 rows; decode: the segments of its range of the work list), one a compute unit being all that the
@@ -34,7 +34,7 @@
 //   Bank conflicts: ds_read_b128 serves lanes 0-3, 12-15, 20-27 together, then 4-11, 16-19, 28-31, and the same of the
 //   upper half.  The 16x16x32 operand (row lane % 16, chunk lane / 16) meets itself there under the tiles' swizzle; with
 //   the four chunks of a step dealt to the lane groups in the order 0, 3, 1, 2 -- in the query rows as well, the sum over
-//   them is the same -- it does not: 1430 of 3100 LDS cycles a unit were conflicts (2048 tokens x 128 heads 575 -> 525 us).
+//   them is the same -- it does not: 1430 of 3100 LDS cycles a unit were conflicts, 80 of 1710 are (2048 tokens x 128 heads 575 -> 525 us).
 //
 // What bounds the decode
 //   64 sequences of 1024..8192 tokens, 128 heads: 13 us until the loop (plan, block table, query rows and the first units of
