@@ -255,9 +255,12 @@ DSCUDA_HOST_DEVICE inline int narrow_forward_row_blocks(int sequence_length, int
 // How many 32-row blocks a workgroup of the absorbed prefill forward holds: 1 or 2 while 128 rows (0: four blocks, the
 // kernels of mla_wide.hip) leave compute units idle.
 //   * up to half a round of 128-row workgroups: 32 or 64 rows (forward in us, 64 / 128 rows: 130 tokens x 128 heads 15.2 / 17.2)
-//   * up to one round, which 64 rows take in two: 128 rows for most of a round of walks of up to 384 keys (180 x 128
-//     19.3 / 18.5, 256 x 128 24.8 / 22.4, 8 x 125 x 32 23.8 / 17.1, 4 x 250 x 32 28.2 / 22.1, 350 x 80 25.9 / 25.7), 64 for longer
-//     ones, a unit of which takes them a third less (512 x 64 32.0 / 33.8, 1000 x 32 47.9 / 56.2, 2000 x 16 82 / 100)
+//   * up to one round, which 64 rows take in two: 128 rows for most of a round of walks of up to 160 keys (128 x 172 18.2 / 17.3,
+//     2 x 123 x 98 18.3 / 17.4, 8 x 97 x 39 21.5 / 17.8), and up to 384 keys of many elements, whose heavy blocks 64 rows get late (3 x
+//     172 x 46 21.1 / 20.0, 4 x 225 x 36 27.4 / 23.9, 16 x 379 x 4 33.8 / 28.3); 64 for longer ones, a unit of which takes them a third
+//     less (512 x 64 32.0 / 33.8, 1000 x 32 47.9 / 56.2, 2000 x 16 82 / 100), and of one or two elements from 161 (192 x 126 19.8 / 20.5,
+//     251 x 87 20.6 / 22.8, 344 x 64 21.3 / 26.8, 2 x 353 x 37 25.3 / 28.4; nearly a round of up to 224 keys 161 x 193 22.5 / 21.6,
+//     256 x 114 24.7 / 24.2) or three from 225 (371 x 21 26.8 / 28.4, 236 x 34 23.7 / 23.0)
 //   * up to a round and a fifth, one or two batch elements: the longest walk decides, which 64 rows take faster, where it is long
 //     against the blocks of a second round (1 x 516 x 64, 258 workgroups, 40 / 37.5; 1 x 750 x 44, 258, 46.0 / 47.1; 1 x 2064 x 16,
 //     258, 92 / 105; 1 x 8256 x 4, 258, 313 / 382; 2 x 1100 x 16, 276, 59.8 / 62.5; 1 x 1200 x 32, 300, 71.5 / 69; 1 x 2400 x 16, 300,
@@ -270,7 +273,12 @@ DSCUDA_HOST_DEVICE inline int forward_row_blocks(int sequence_length, int heads,
     const long long workgroups = ((long long)sequence_length * heads + 127) / 128 * batch;
     const int units = (sequence_length + 31) / 32;
     if (2 * workgroups <= compute_units) return narrow_forward_row_blocks(sequence_length, heads, batch, compute_units);
-    if (workgroups <= compute_units) return units <= 12 && 3 * workgroups > 2LL * compute_units ? 0 : 2;
+    if (workgroups <= compute_units) {
+        if (units > 12 || 3 * workgroups <= 2LL * compute_units) return 2;
+        if (units <= 5) return 0;
+        if (batch <= 2) return units <= 7 && 8 * workgroups >= 7LL * compute_units ? 0 : 2;
+        return batch == 3 && units >= 8 && 4 * workgroups < 3LL * compute_units ? 2 : 0;
+    }
     if (units == 1) return 4 * workgroups <= 5LL * compute_units ? 2 : 0;
     return batch <= 2 && 5 * workgroups <= 6LL * compute_units && 2 * (units - 20) > workgroups - compute_units ? 2 : 0;
 }

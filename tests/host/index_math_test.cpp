@@ -515,6 +515,9 @@ void check_forward_row_blocks() {
         // just over a round of 128 rows: long walks of one or two elements by 64, short ones and more elements by 128
         {1, 2064, 16, 2}, {1, 4666, 8, 2}, {2, 4200, 4, 2}, {1, 516, 64, 0}, {1, 258, 128, 0}, {3, 2800, 4, 0}, {1, 4912, 8, 2}, {1, 4944, 8, 0},
         {1, 672, 49, 0}, {1, 673, 49, 2},
+        // most of a round of 128 rows: the walk's length decides, and how many elements have heavy blocks
+        {1, 160, 139, 0}, {1, 161, 139, 2}, {1, 224, 128, 0}, {1, 224, 127, 2}, {1, 256, 128, 2}, {1, 344, 64, 2}, {2, 353, 37, 2},
+        {3, 172, 46, 0}, {3, 225, 32, 2}, {3, 256, 34, 0}, {4, 225, 36, 0}, {16, 379, 4, 0}, {16, 385, 4, 2},
     };
     for (const auto& c : known) {
         const int blocks = forward_row_blocks(c.tokens, c.heads, c.batch, 256);

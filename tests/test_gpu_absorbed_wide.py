@@ -15,7 +15,8 @@ pytestmark = pytest.mark.gpu
 
 # 171 and 256 workgroups of 128 rows are two thirds and the whole of one round, 320 one and a quarter
 @pytest.mark.parametrize("batch,tokens,heads,rows", [
-    (1, 171, 128, 128), (1, 170, 128, 64), (1, 256, 128, 128), (2, 383, 42, 128), (2, 385, 42, 64), (1, 257, 128, 128),
+    (1, 171, 128, 64), (1, 170, 128, 64), (1, 256, 128, 64), (2, 383, 42, 64), (2, 385, 42, 64), (1, 257, 128, 128),
+    (1, 160, 139, 128), (1, 161, 139, 64), (1, 224, 146, 128), (4, 383, 21, 128), (3, 225, 32, 64), (3, 256, 34, 128),
     (1, 672, 49, 128), (1, 673, 49, 64),   # 258 workgroups, walks of 21 and 22 units
     (321, 5, 25, 128), (320, 5, 25, 64), (320, 33, 3, 128), (257, 1, 129, 128),
     (3, 97, 129, 128),    # a row block over two tokens, items of two, three and four units
