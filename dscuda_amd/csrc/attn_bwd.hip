@@ -96,7 +96,11 @@ __device__ __forceinline__ void clear(f32x16& value) {
 // 44.5, 124.8 / 43.0, 123.6, 4 x 400 x 16 38.8, 96.5 / 37.5, 97.2, 1000 x 32 61.7, 142.5 / 60.8, 141.2.  Not those of the other
 // geometries, whose readers gain more than the call loses: 16 x 256 x 16 of 64 35.6, 70.3 / 34.8, 73.4, 2 x 1024 x 32 on 8 of 128 86.0,
 // 126.7 / 85.8, 131.6, 8 x 1024 x 32 on 8 of 64 241.1, 287.4 / 240.6, 290.3.
+// dQ of these columns does so as well in short walks, whose readers come out even: 211 x 128 30.3, 267.6 / 29.4, 268.6, 2 x 250 x 64
+// 32.0, 147.9 / 30.9, 148.2, 2 x 444 x 64 71.3, 212.4 / 70.3, 212.8; longer ones gain, 4 x 500 x 32 79.6, 184.6 / 79.1, 186.3, 600 x 64
+// 60.0, 199.6 / 59.8, 201.5.
 constexpr long long GRADIENT_STREAM_BYTES = 96LL << 20;
+constexpr int SHORT_WALK = 480;   // tokens
 
 template <bool STREAM>   // (a branch at the stores instead: 300 tokens x 8 heads 27.6 -> 27.9 us)
 __device__ __forceinline__ void store_gradient(bf16_t* place, const u32x4& bits) {
@@ -1104,8 +1108,9 @@ void launch_backward(bf16_t* query_gradient, bf16_t* key_gradient, bf16_t* value
     const bool stream_gradients = gradient_bytes >= GRADIENT_STREAM_BYTES;
     const auto key_value_kernel = stream_gradients ? attention_key_value_gradient_kernel<DQK, DV, true>
                                                    : attention_key_value_gradient_kernel<DQK, DV, ALWAYS>;
-    const auto query_kernel = stream_gradients ? attention_query_gradient_kernel<DQK, DV, true>
-                                               : attention_query_gradient_kernel<DQK, DV, false>;
+    const auto query_kernel = stream_gradients || (ALWAYS && sequence_length < SHORT_WALK)
+                                  ? attention_query_gradient_kernel<DQK, DV, true>
+                                  : attention_query_gradient_kernel<DQK, DV, false>;
     for (long long first = 0; first < shape.pairs; first += shape.pairs_per_launch) {
         const long long count = std::min(shape.pairs_per_launch, shape.pairs - first);
         hipLaunchKernelGGL(key_value_kernel, dim3((unsigned)(count * shape.cut.items)),

@@ -1,5 +1,6 @@
 """GPU parity of the per-head backward on both sides of the size from which its gradient rows leave past the caches
-(csrc/attn_bwd.hip, GRADIENT_STREAM_BYTES): dQ, dK and dV of 96 MiB together or a little less."""
+(csrc/attn_bwd.hip, GRADIENT_STREAM_BYTES): dQ, dK and dV of 96 MiB together or a little less; and on both sides of the walks
+(SHORT_WALK) from which dQ of 192 / 128 columns stays in them."""
 
 import pytest
 import torch
@@ -17,6 +18,7 @@ LINE = 96 << 20
     (1535, 64, 64, 192, 128, False), (1537, 64, 64, 192, 128, True),   # last blocks of 127 keys and of one
     (2048, 64, 64, 128, 128, True), (1984, 64, 64, 128, 128, False),   # at the line itself
     (4096, 128, 16, 64, 64, False), (4928, 128, 16, 64, 64, True),
+    (479, 20, 20, 192, 128, False), (480, 20, 20, 192, 128, False),
 ])
 def test_gradients(cuda, seq, q_heads, kv_heads, dqk, dv, streamed):
     assert (2 * seq * (q_heads * dqk + kv_heads * (dqk + dv)) >= LINE) == streamed
